@@ -45,10 +45,12 @@ int i64h_device_check(void);
  *   bias (may be NULL; fp32 [N], batch stride bias_batch) is added to the sum before any epilogue but the three gate / up ones.
  * group_off (may be NULL; device int32 [batch + 1], ascending): batch b takes the rows [group_off[b], group_off[b + 1]) of a_rows
  *   (of A itself without a_rows) and of C instead of all M rows; M is then the most rows any batch may have (it sizes the launch,
- *   workgroups past a batch's rows leave at once), and the launch needs no count on the host.  Such launches take the 64 x 64 tile form,
- *   or with M <= 64 the fragment-streaming form.
+ *   workgroups past a batch's rows leave at once), and the launch needs no count on the host.  rows_total (0: unknown): a bound of
+ *   group_off[batch], which makes the launch smaller.
+ * a_height (0: unknown): the rows of A that a_rows may name; a launch with a_rows and without it takes the 64 x 64 tile form.
  * Any M, N, K >= 1; 16-byte loads are used where strides and addresses allow, element loads otherwise.
- * Launches with M <= I64H_SKINNY_ROWS take a weight-streaming form (one wave per output column group). */
+ * Launches with M <= I64H_SKINNY_ROWS take a weight-streaming form (one wave per output column group); the form of the others follows from
+ * their size (i64h_linear_block.hip). */
 #define I64H_EPI_STORE 0
 #define I64H_EPI_GELU_MUL 1
 #define I64H_EPI_MUL_SIGMOID 2
@@ -63,7 +65,7 @@ int i64h_device_check(void);
 #define I64H_EPI_DECAY 11
 #define I64H_EPI_ROW_SIGMOID 12
 #define I64H_EPI_IN_NORM 13
-#define I64H_SKINNY_ROWS 8
+#define I64H_SKINNY_ROWS 2
 typedef struct {
     const float* A;
     int64_t lda;
@@ -88,6 +90,7 @@ typedef struct {
     const float* row_scale;
     const float* in_norm_w;
     float in_eps;
+    int64_t rows_total, a_height;
 } i64h_linear;
 int i64h_linear_run(const i64h_linear* d, void* stream);
 

@@ -1,0 +1,117 @@
+"""The matrix-core tile forms of i64h_linear_run against 64-bit products of the same bf16 values: every form at sizes around its tiles' edges,
+ragged k, column offsets, gathered rows, rows dealt to experts, gate / up pairs, the normed input."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+FORMS = {"128x128": 1, "64x128": 2, "64x64": 3, "64x64/2": 4, "32x64/4": 5, "16x64/4": 6, "16x128/2 pair": 7, "by size": 0}
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return torch.device("cuda:0")
+
+
+@pytest.fixture
+def use_form():
+    from vllm_i64_amd import ops_dense as D
+    yield lambda name: D.call_dense("i64h_set_linear_skinny", 16 * FORMS[name] + 2 if FORMS[name] else 3)
+    D.call_dense("i64h_set_linear_skinny", 3)
+
+
+def bf16(t):
+    return t.to(torch.bfloat16)
+
+
+def close(got, ref, K):
+    """fp32 sums of exact products of order one over sqrt(K): a rounding of 2^-24 of the running sum per term at most."""
+    return torch.allclose(got.double().cpu(), ref, atol=K ** 0.5 * 2e-6, rtol=2e-5)
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("M,N,K", [(3, 4, 8), (17, 63, 72), (65, 129, 128), (130, 196, 1000), (129, 64, 64), (256, 260, 192)])
+def test_tiles_and_ends(dev, use_form, form, M, N, K):
+    from vllm_i64_amd import ops_dense as D
+    use_form(form)
+    g = torch.Generator().manual_seed(M + N + K)
+    a, w = torch.randn(M, K + 8, generator=g), bf16(torch.randn(2 * N, K, generator=g) / math.sqrt(K))
+    b = torch.randn(N, generator=g)
+    e = torch.randn(M, N + 3, generator=g)
+    A = bf16(a[:, 4:4 + K]).double()
+    ref, up = A @ w[:N].double().T, A @ w[N:].double().T
+    ad, wd = a.to(dev), w.to(dev)
+    out = torch.full((M, N + 5), 7.0, device=dev)
+    kw = dict(n=N, k=K, a_off=4, lda=K + 8)
+    D.linear(ad, wd, out, c_off=2, ldc=N + 5, **kw)
+    assert close(out[:, 2:2 + N], ref, K) and bool((out[:, :2] == 7).all()) and bool((out[:, 2 + N:] == 7).all())
+    out = torch.empty(M, N, device=dev)
+    D.linear(ad, wd, out, bias=b.to(dev), epilogue=D.EPI_ADD, e=e.to(dev), e_off=1, lde=N + 3, **kw)
+    assert close(out, ref + b.double() + e[:, 1:1 + N].double(), K)
+    s = torch.rand(M, generator=g) + 0.5
+    D.linear(ad, wd, out, epilogue=D.EPI_SILU_MUL, row_scale=s.to(dev), **kw)
+    z, u = ref * s[:, None].double(), up * s[:, None].double()
+    assert torch.allclose(out.double().cpu(), z * torch.sigmoid(z) * u, atol=1e-4, rtol=1e-4)
+    if K % 8 == 0 and M > 2:
+        nw = torch.rand(K, generator=g) + 0.5
+        D.linear(ad, wd, out, in_norm_w=nw.to(dev), in_eps=1e-6, **kw)
+        x = a[:, 4:4 + K]
+        f = 1.0 / torch.sqrt(x.double().pow(2).mean(-1, keepdim=True) + 1e-6)
+        assert close(out, (bf16(x * nw).double() @ w[:N].double().T) * f, K)
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("counts", [[5, 0, 70, 1], [0, 0, 0, 129], [64, 16, 128, 0], [1, 1, 1, 1]])
+def test_rows_dealt_to_experts(dev, use_form, form, counts):
+    """Gathered rows into a gate / up pair with a factor per row, and rows as they lie; empty batches; a larger bound than there are rows."""
+    from vllm_i64_amd import ops_dense as D
+    use_form(form)
+    E, N, K, n = len(counts), 72, 136, 150
+    g = torch.Generator().manual_seed(sum(counts))
+    off = torch.tensor([0] + counts).cumsum(0).to(torch.int32)
+    R = int(off[-1])
+    rows = torch.randint(0, n, (R + 9,), generator=g).to(torch.int32)
+    h, s = torch.randn(n, K, generator=g), torch.rand(R, generator=g) + 0.5
+    w = bf16(torch.randn(E, 2 * N, K, generator=g) / math.sqrt(K))
+    out = torch.full((R + 3, N), 7.0, device=dev)
+    D.linear(h.to(dev), w.to(dev), out, m=max(counts), n=N, k=K, a_rows=rows.to(dev), batch=E, w_batch=2 * N * K, group_off=off.to(dev), row_scale=s.to(dev),
+             epilogue=D.EPI_CLAMP_GLU, act_a=1.702, act_b=7.0)
+    A = bf16(h).double()[rows[:R].long()]
+    e_of = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    z = torch.einsum("rk,rnk->rn", A, w.double()[e_of]) * s[:, None].double()
+    u, v = z[:, :N].clamp(max=7.0), z[:, N:].clamp(-7.0, 7.0)
+    assert torch.allclose(out[:R].double().cpu(), u * torch.sigmoid(1.702 * u) * (v + 1), atol=1e-4, rtol=1e-4) and bool((out[R:] == 7).all())
+    wd = bf16(torch.randn(E, K, N, generator=g) / math.sqrt(N))
+    down = torch.full((R + 3, K), 7.0, device=dev)
+    D.linear(out[:R], wd.to(dev), down, m=max(counts), n=K, k=N, batch=E, w_batch=K * N, group_off=off.to(dev))
+    ref = torch.einsum("rn,rkn->rk", bf16(out[:R].cpu()).double(), wd.double()[e_of])
+    assert close(down[:R], ref, N) and bool((down[R:] == 7).all())
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("M", [5, 100])
+def test_batched_over_heads(dev, use_form, form, M):
+    from vllm_i64_amd import ops_dense as D
+    use_form(form)
+    H, n, k = 3, 40, 64
+    g = torch.Generator().manual_seed(M)
+    a, w = torch.randn(M, H * k, generator=g), bf16(torch.randn(H, n, k, generator=g) / 8)
+    out = torch.empty(M, H * n, device=dev)
+    D.linear(a.to(dev), w.to(dev), out, m=M, n=n, k=k, lda=H * k, ldc=H * n, batch=H, a_batch=k, w_batch=n * k, c_batch=n)
+    for h in range(H):
+        assert close(out[:, h * n:(h + 1) * n], bf16(a[:, h * k:(h + 1) * k]).double() @ w[h].double().T, k)
+
+
+def test_not_a_number_stays_in_its_row(dev, use_form):
+    """Rows past the end repeat the last one, chunks past k read as zeros: an infinity or NaN touches no other row."""
+    from vllm_i64_amd import ops_dense as D
+    a, w = torch.ones(66, 72), bf16(torch.ones(64, 72))
+    a[65, 71], a[3, 0] = math.nan, math.inf
+    for form in FORMS:
+        use_form(form)
+        out = torch.empty(66, 64, device=dev)
+        D.linear(a.to(dev), w.to(dev), out)
+        bad = ~torch.isfinite(out.cpu())
+        assert bool(bad[[3, 65]].all()) and int(bad.sum()) == 128 and bool((out.cpu()[:3] == 72).all())

@@ -242,7 +242,7 @@ class Linear(ctypes.Structure):
     """Mirror of i64h_linear (include/i64h_dense.h)."""
     _fields_ = [("A", _P), ("lda", _L), ("a_rows", _P), ("W", _P), ("C", _P), ("ldc", _L), ("M", _L), ("N", _I), ("K", _I), ("batch", _I),
                 ("a_batch", _L), ("w_batch", _L), ("c_batch", _L), ("exact", _I), ("epilogue", _I), ("E", _P), ("lde", _L), ("e_batch", _L),
-                ("softcap", _F), ("bias", _P), ("bias_batch", _L), ("scale", _F), ("act_a", _F), ("act_b", _F), ("group_off", _P), ("row_scale", _P), ("in_norm_w", _P), ("in_eps", _F)]
+                ("softcap", _F), ("bias", _P), ("bias_batch", _L), ("scale", _F), ("act_a", _F), ("act_b", _F), ("group_off", _P), ("row_scale", _P), ("in_norm_w", _P), ("in_eps", _F), ("rows_total", _L), ("a_height", _L)]
 
 
 class PostNorm(ctypes.Structure):

@@ -2,72 +2,19 @@
 //   linear_tile_kernel   : C = epilogue(A W^T), 64 x 64 tiles, four waves of 32 x 32, on v_mfma_f32_16x16x32_bf16 (A rounded to
 //                          bf16 while staged) or v_mfma_f32_16x16x4_f32 (W widened while staged: true 32-bit); batched over
 //                          blockIdx.z (per-head weights on column blocks of wider matrices); epilogues: gelu_tanh(gate) * up
-//                          on two accumulators, * sigmoid(E), logit soft cap and others; an RMS norm of its input on the way
-//   linear_tile128_kernel: bf16 form, 128 x 128 tiles (waves of 64 x 64); behind a knob, measured slower at the sizes tried
+//                          on two accumulators, * sigmoid(E), logit soft cap and others; an RMS norm of its input on the way.  The form
+//                          of true 32-bit products and of operands that 16-byte loads cannot read; every other launch of more than a
+//                          few rows is linear_block_kernel's (i64h_linear_block.hip)
 //   linear_skinny_kernel : the same product for at most I64H_SKINNY_ROWS rows (decode steps): the rows sit in LDS as bf16, every
 //                          wave streams four weight rows at a time with 16-byte loads and reduces over its lanes
-//   linear_rows64_kernel : at most 64 rows: 16 output columns per workgroup, the k steps dealt to its four waves, every operand read
-//                          from memory as a matrix-core fragment, partial tiles summed through LDS
+//   linear_rows16_kernel : at most 16 rows of a small product: 16 output columns per workgroup, the k steps dealt to its eight waves, every
+//                          operand read from memory as a matrix-core fragment, partial tiles summed through LDS
 //   embed_scaled_kernel  : bf16 table row * scale -> fp32
 //   gated_postnorm_kernel: alpha * x + sigmoid(gate) * y -> RMS norm in groups -> (optional) weighted sum over the outputs of
 //                          all earlier layers; one workgroup per row, the row held in LDS between the passes
 //   sample_rows_kernel   : greedy / temperature / top-k / top-p draw of one token per row
-#include "i64h_common.h"
-#include "i64h_dense.h"
+#include "i64h_dense_dev.h"
 #include <type_traits>
-
-typedef float dn_v4f __attribute__((ext_vector_type(4)));
-typedef __bf16 dn_v8bf __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ uint32_t dn_bf16_rne(float f) {  // round to nearest even, NaN stays NaN: the hardware conversion of this chip
-    return (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)f);
-}
-__device__ __forceinline__ float dn_bf16_to_f32(uint32_t h) { return __uint_as_float(h << 16); }
-__device__ __forceinline__ float dn_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
-__device__ __forceinline__ float dn_gelu_tanh(float z) {
-    const float inner = 0.7978845608028654f * (z + 0.044715f * z * z * z);
-    return 0.5f * z * (1.0f + tanhf(inner));
-}
-
-__device__ __forceinline__ float dn_gelu_erf(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
-
-// log(1 + e^z) with one logarithm: with u = 1 + x rounded, log(u) x / (u - 1) is log(1 + x) to a few units in the last place (Kahan's
-// correction of the rounding of u)
-__device__ __forceinline__ float dn_softplus(float z) {
-    const float x = expf(z), u = 1.0f + x, d = u - 1.0f;
-    const float l = d > 0.0f ? logf(u) * (x * __builtin_amdgcn_rcpf(d)) : x;
-    return z > 20.0f ? z : l;
-}
-
-__device__ __forceinline__ float dn_xielu(float z, float a, float b) {
-    return z > 0.0f ? a * z * z + 0.5f * z : b * (expm1f(z) - z) + 0.5f * z;
-}
-constexpr bool dn_dual(int epi) { return epi == I64H_EPI_GELU_MUL || epi == I64H_EPI_SILU_MUL || epi == I64H_EPI_CLAMP_GLU; }  // two accumulators: gate rows and up rows
-
-template <int EPI>
-__device__ __forceinline__ float dn_epilogue(const i64h_linear& p, float acc, float acc2, int64_t b, int64_t r, int c) {
-    if (dn_dual(EPI) && p.row_scale) {      // a factor on the input row
-        const float s = p.row_scale[r];
-        acc *= s, acc2 *= s;
-    }
-    if (EPI == I64H_EPI_GELU_MUL) return dn_gelu_tanh(acc) * acc2;
-    if (EPI == I64H_EPI_SILU_MUL) return acc * dn_sigmoid(acc) * acc2;
-    if (EPI == I64H_EPI_CLAMP_GLU) {
-        const float u = fminf(acc, p.act_b), w = fminf(fmaxf(acc2, -p.act_b), p.act_b);
-        return u * dn_sigmoid(p.act_a * u) * (w + 1.0f);
-    }
-    if (p.bias) acc += p.bias[b * p.bias_batch + c];
-    if (EPI == I64H_EPI_XIELU) return dn_xielu(acc, p.act_a, p.act_b);
-    if (EPI == I64H_EPI_RELU_SQ) return acc > 0.0f ? acc * acc : 0.0f;
-    if (EPI == I64H_EPI_GELU_ERF) return dn_gelu_erf(acc);
-    if (EPI == I64H_EPI_SCALE) return acc * p.scale;
-    if (EPI == I64H_EPI_MUL_SIGMOID) return acc * dn_sigmoid(p.E[b * p.e_batch + r * p.lde + c]);
-    if (EPI == I64H_EPI_ROW_SIGMOID) return acc * dn_sigmoid(p.E[b * p.e_batch + r * p.lde]);
-    if (EPI == I64H_EPI_SOFTCAP) return p.softcap * tanhf(acc / p.softcap);
-    if (EPI == I64H_EPI_ADD) return acc + p.E[b * p.e_batch + r * p.lde + c];
-    if (EPI == I64H_EPI_DECAY) return expf(-p.E[b * p.e_batch + r * p.lde + c] * dn_softplus(acc));
-    return acc;
-}
 
 // ---------------------------------------------------------------------------------------------------------------------------
 template <bool EXACT, int EPI>
@@ -238,128 +185,9 @@ __global__ __launch_bounds__(256) void linear_tile_kernel(const i64h_linear p, c
 
 
 // ---------------------------------------------------------------------------------------------------------------------------
-// The bf16 form for launches with many tiles: 128 x 128 per workgroup, four waves of 64 x 64 (16 matrix instructions per wave and
-// 32-wide k step against 8 fragment reads - four times the 64 x 64 kernel's ratio), the same staging scheme.
-template <int EPI>
-__global__ __launch_bounds__(256) void linear_tile128_kernel(const i64h_linear p, const int vecA, const int vecW) {
-    constexpr bool DUAL = dn_dual(EPI);
-    constexpr int LD = 40;
-    __shared__ __attribute__((aligned(16))) uint16_t sA[2][128][LD];
-    __shared__ __attribute__((aligned(16))) uint16_t sB[2][128][LD];
-    __shared__ __attribute__((aligned(16))) uint16_t sB2[DUAL ? 2 : 1][DUAL ? 128 : 1][LD];
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int wm = wid >> 1, wn = wid & 1;
-    const int64_t b = blockIdx.z;
-    const int64_t m0 = (int64_t)blockIdx.y * 128;
-    const int n0 = blockIdx.x * 128;
-    const int M = (int)min((int64_t)128, p.M - m0);
-    const int N = p.N, K = p.K;
-    const int lr = tid >> 2, lc = (tid & 3) * 8;
-    bool aok[2], bok[2];
-    const float* pa[2];
-    const uint16_t* pw[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int rr = lr + 64 * h;
-        aok[h] = rr < M;
-        bok[h] = n0 + rr < N;
-        const int64_t arow = aok[h] ? (p.a_rows ? (int64_t)p.a_rows[m0 + rr] : m0 + rr) : 0;
-        pa[h] = p.A + b * p.a_batch + arow * p.lda;
-        pw[h] = (const uint16_t*)p.W + b * p.w_batch + (int64_t)(bok[h] ? n0 + rr : 0) * K;
-    }
-    const int64_t w2 = (int64_t)N * K;
-    float ra[2][8];
-    uint16_t rb[2][8], rb2[2][8];
-    auto gload = [&](int k0) {
-        const int k = k0 + lc;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            if (aok[h] && vecA && k + 8 <= K) {
-                const float4 u = *(const float4*)(pa[h] + k), v = *(const float4*)(pa[h] + k + 4);
-                ra[h][0] = u.x; ra[h][1] = u.y; ra[h][2] = u.z; ra[h][3] = u.w; ra[h][4] = v.x; ra[h][5] = v.y; ra[h][6] = v.z; ra[h][7] = v.w;
-            } else {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) ra[h][i] = (aok[h] && k + i < K) ? pa[h][k + i] : 0.0f;
-            }
-            if (bok[h] && vecW && k + 8 <= K) {
-                *(uint4*)rb[h] = *(const uint4*)(pw[h] + k);
-                if (DUAL) *(uint4*)rb2[h] = *(const uint4*)(pw[h] + w2 + k);
-            } else {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    rb[h][i] = (bok[h] && k + i < K) ? pw[h][k + i] : (uint16_t)0;
-                    if (DUAL) rb2[h][i] = (bok[h] && k + i < K) ? pw[h][w2 + k + i] : (uint16_t)0;
-                }
-            }
-        }
-    };
-    auto lstore = [&](int buf) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            uint32_t w[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) w[i] = dn_bf16_rne(ra[h][2 * i]) | (dn_bf16_rne(ra[h][2 * i + 1]) << 16);
-            *(uint4*)&sA[buf][lr + 64 * h][lc] = make_uint4(w[0], w[1], w[2], w[3]);
-            *(uint4*)&sB[buf][lr + 64 * h][lc] = *(const uint4*)rb[h];
-            if (DUAL) *(uint4*)&sB2[buf][lr + 64 * h][lc] = *(const uint4*)rb2[h];
-        }
-    };
-    dn_v4f acc[4][4], acc2[DUAL ? 4 : 1][DUAL ? 4 : 1];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            acc[i][j] = dn_v4f{0, 0, 0, 0};
-            if (DUAL) acc2[DUAL ? i : 0][DUAL ? j : 0] = dn_v4f{0, 0, 0, 0};
-        }
-    const int fr = lane & 15, fk = lane >> 4;
-    gload(0);
-    lstore(0);
-    __syncthreads();
-    const int KT = (K + 31) / 32;
-    for (int kt = 0; kt < KT; ++kt) {
-        const int cur = kt & 1;
-        if (kt + 1 < KT) gload((kt + 1) * 32);
-        dn_v8bf a[4], bb[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) a[i] = *(const dn_v8bf*)&sA[cur][wm * 64 + i * 16 + fr][fk * 8];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) bb[j] = *(const dn_v8bf*)&sB[cur][wn * 64 + j * 16 + fr][fk * 8];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], bb[j], acc[i][j], 0, 0, 0);
-        if (DUAL) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) bb[j] = *(const dn_v8bf*)&sB2[cur][wn * 64 + j * 16 + fr][fk * 8];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc2[DUAL ? i : 0][DUAL ? j : 0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], bb[j], acc2[DUAL ? i : 0][DUAL ? j : 0], 0, 0, 0);
-        }
-        if (kt + 1 < KT) lstore(cur ^ 1);
-        __syncthreads();
-    }
-    float* C = p.C + b * p.c_batch;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int reg = 0; reg < 4; ++reg) {
-            const int rl = wm * 64 + i * 16 + fk * 4 + reg;
-            if (rl >= M) continue;
-            const int64_t r = m0 + rl;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int c = n0 + wn * 64 + j * 16 + fr;
-                if (c < N) C[r * p.ldc + c] = dn_epilogue<EPI>(p, acc[i][j][reg], DUAL ? acc2[DUAL ? i : 0][DUAL ? j : 0][reg] : 0.0f, b, r, c);
-            }
-        }
-}
-
-// ---------------------------------------------------------------------------------------------------------------------------
-// M <= 8 rows.  The rows are rounded to bf16 into LDS once per workgroup (M * K halves); a wave takes CPW = 4 weight rows at a
-// time, every lane 8 consecutive k of each per iteration (one 16-byte load per weight row), products in fp32.
+// One or two rows.  They are rounded to bf16 into LDS once per workgroup (M * K halves); a wave takes CPW = 4 weight rows at a time, every lane
+// 8 consecutive k of each per iteration (one 16-byte load per weight row), products in fp32.  The products are what bounds it: 1024 x 1024
+// in a replayed graph 4.2 us at one row, 5.0 at two, 6.4 at four, 8.4 at seven; on the matrix cores 5.4 us at any of them.
 template <int EPI>
 __global__ __launch_bounds__(256) void linear_skinny_kernel(const i64h_linear p, const int cols_per_block) {
     constexpr bool DUAL = dn_dual(EPI);
@@ -456,60 +284,45 @@ __global__ __launch_bounds__(256) void linear_skinny_kernel(const i64h_linear p,
 
 
 // ---------------------------------------------------------------------------------------------------------------------------
-// At most 64 rows (decode steps, small batches), bf16 form.  A workgroup owns 16 output columns; its four or eight waves deal the
-// 32-wide k steps among them, each with up to four 16-row blocks of A against the one weight fragment, all operands read straight from memory
-// as matrix-core fragments (no staging, no barrier inside the loop); the four partial tiles meet in LDS, then the epilogue.
-// Many small workgroups fill the chip where a launch has few 64-column tiles, and the weights stream exactly once.
-template <int EPI, int NW>
-__global__ __launch_bounds__(64 * NW) void linear_rows64_kernel(const i64h_linear p) {
-    constexpr bool DUAL = dn_dual(EPI);
-    constexpr bool INN = EPI == I64H_EPI_IN_NORM;
-    __shared__ float red[DUAL ? 2 : 1][NW][64][17];
-    __shared__ float sRow[INN ? NW : 1][64];
-    float ssq[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+// At most 16 rows of a small product, bf16 form.  A workgroup owns 16 output columns; its eight waves deal the 32-wide k steps among them,
+// all operands read straight from memory as matrix-core fragments (no staging, no barrier inside the loop); the partial tiles meet
+// in LDS, then the epilogue.  Its launch is one round of loads and one reduction: 7 x 1024 x 1024 5.4 us in a replayed graph against 5.9 us of
+// the 16 x 64 tiles of linear_block_kernel, 7 x 1024 x 128 3.2 against 4.1 us.
+template <int EPI>
+__global__ __launch_bounds__(512) void linear_rows16_kernel(const i64h_linear p) {
+    constexpr bool DUAL = dn_dual(EPI), INN = EPI == I64H_EPI_IN_NORM;
+    constexpr int NW = 8, U = 2;
+    __shared__ float red[DUAL ? 2 : 1][NW][16][17];
+    __shared__ float sRow[INN ? NW : 1][16];
+    float ssq = 0.0f;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int n = lane & 15, kg = lane >> 4;
     const int64_t b = blockIdx.z;
     const int n0 = blockIdx.x * 16;
-    int M = (int)p.M;
     const int N = p.N, K = p.K;
+    int M = (int)p.M;
     int64_t g0 = 0;      // this batch's first row among all rows, where the rows are dealt to the batches by group_off
     if (p.group_off) {
         g0 = p.group_off[b];
         M = min(M, p.group_off[b + 1] - (int)g0);
         if (M <= 0) return;
     }
-    const int mblocks = (M + 15) / 16;
-    const bool cok = n0 + n < N;
+    const bool cok = n0 + n < N, rok = n < M;
     const uint16_t* pw = (const uint16_t*)p.W + b * p.w_batch + (int64_t)(cok ? n0 + n : 0) * K;
     const uint16_t* pw2 = pw + (int64_t)N * K;
-    const float* pa[4];
-    bool rok[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = i * 16 + n;
-        rok[i] = m < M;
-        const int64_t arow = rok[i] ? (p.a_rows ? (int64_t)p.a_rows[g0 + m] : g0 + m) : 0;
-        pa[i] = p.A + b * p.a_batch + arow * p.lda;
-    }
-    dn_v4f acc[4], acc2[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        acc[i] = dn_v4f{0, 0, 0, 0};
-        acc2[i] = dn_v4f{0, 0, 0, 0};
-    }
+    const int64_t arow = rok ? (p.a_rows ? (int64_t)p.a_rows[g0 + n] : g0 + n) : 0;
+    const float* pa = p.A + b * p.a_batch + arow * p.lda;
+    dn_v4f acc = {0, 0, 0, 0}, acc2 = {0, 0, 0, 0};
     const int KT = (K + 31) / 32;
-    // U k steps per turn: the loads of all of them are requested before the first matrix instruction (four per turn measured slower:
-    // 21 against 17 us on the gate / up launch of 64 rows - the registers cost a wave per SIMD)
-    constexpr int U = 2;
-    for (int kt = wv; kt < KT; kt += U * NW) {
+    for (int kt = wv; kt < KT; kt += U * NW) {      // the loads of U steps are requested before the first matrix instruction
         uint4 wf[U], wf2[U];
-        float4 au[U][4], av[U][4], nu[INN ? U : 1], nv[INN ? U : 1];
+        float4 au[U], av[U], nu[INN ? U : 1], nv[INN ? U : 1];
 #pragma unroll
         for (int h = 0; h < U; ++h) {
             const int k = (kt + h * NW) * 32 + kg * 8;
             const bool kin = kt + h * NW < KT && k < K;
             wf[h] = wf2[h] = make_uint4(0, 0, 0, 0);
+            au[h] = av[h] = make_float4(0, 0, 0, 0);
             if (INN) {
                 nu[INN ? h : 0] = kin ? *(const float4*)(p.in_norm_w + k) : make_float4(0, 0, 0, 0);
                 nv[INN ? h : 0] = kin ? *(const float4*)(p.in_norm_w + k + 4) : make_float4(0, 0, 0, 0);
@@ -518,69 +331,52 @@ __global__ __launch_bounds__(64 * NW) void linear_rows64_kernel(const i64h_linea
                 wf[h] = *(const uint4*)(pw + k);
                 if (DUAL) wf2[h] = *(const uint4*)(pw2 + k);
             }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                au[h][i] = av[h][i] = make_float4(0, 0, 0, 0);
-                if (i < mblocks && rok[i] && kin) {
-                    au[h][i] = *(const float4*)(pa[i] + k);
-                    av[h][i] = *(const float4*)(pa[i] + k + 4);
-                }
+            if (rok && kin) {
+                au[h] = *(const float4*)(pa + k);
+                av[h] = *(const float4*)(pa + k + 4);
             }
         }
 #pragma unroll
-        for (int h = 0; h < U; ++h)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (i < mblocks) {
-                    float4 u = au[h][i], v = av[h][i];
-                    if (INN) {
-                        ssq[i] = fmaf(u.x, u.x, fmaf(u.y, u.y, fmaf(u.z, u.z, fmaf(u.w, u.w, ssq[i]))));
-                        ssq[i] = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ssq[i]))));
-                        u.x *= nu[INN ? h : 0].x, u.y *= nu[INN ? h : 0].y, u.z *= nu[INN ? h : 0].z, u.w *= nu[INN ? h : 0].w;
-                        v.x *= nv[INN ? h : 0].x, v.y *= nv[INN ? h : 0].y, v.z *= nv[INN ? h : 0].z, v.w *= nv[INN ? h : 0].w;
-                    }
-                    const uint4 af = make_uint4(dn_bf16_rne(u.x) | (dn_bf16_rne(u.y) << 16), dn_bf16_rne(u.z) | (dn_bf16_rne(u.w) << 16),
-                                                dn_bf16_rne(v.x) | (dn_bf16_rne(v.y) << 16), dn_bf16_rne(v.z) | (dn_bf16_rne(v.w) << 16));
-                    acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_v8bf, af), __builtin_bit_cast(dn_v8bf, wf[h]), acc[i], 0, 0, 0);
-                    if (DUAL) acc2[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_v8bf, af), __builtin_bit_cast(dn_v8bf, wf2[h]), acc2[i], 0, 0, 0);
-                }
+        for (int h = 0; h < U; ++h) {
+            float4 u = au[h], v = av[h];
+            if (INN) {
+                ssq = fmaf(u.x, u.x, fmaf(u.y, u.y, fmaf(u.z, u.z, fmaf(u.w, u.w, ssq))));
+                ssq = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ssq))));
+                u.x *= nu[INN ? h : 0].x, u.y *= nu[INN ? h : 0].y, u.z *= nu[INN ? h : 0].z, u.w *= nu[INN ? h : 0].w;
+                v.x *= nv[INN ? h : 0].x, v.y *= nv[INN ? h : 0].y, v.z *= nv[INN ? h : 0].z, v.w *= nv[INN ? h : 0].w;
             }
+            const uint4 af = make_uint4(dn_bf16_pair(u.x, u.y), dn_bf16_pair(u.z, u.w), dn_bf16_pair(v.x, v.y), dn_bf16_pair(v.z, v.w));
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_v8bf, af), __builtin_bit_cast(dn_v8bf, wf[h]), acc, 0, 0, 0);
+            if (DUAL) acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_v8bf, af), __builtin_bit_cast(dn_v8bf, wf2[h]), acc2, 0, 0, 0);
+        }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            red[0][wv][i * 16 + kg * 4 + g][n] = acc[i][g];
-            if (DUAL) red[DUAL ? 1 : 0][wv][i * 16 + kg * 4 + g][n] = acc2[i][g];
-        }
-    if (INN) {      // lanes n, n + 16, n + 32, n + 48 hold shares of row n of a block
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float q = ssq[i];
-            q += __shfl_xor(q, 16);
-            q += __shfl_xor(q, 32);
-            if (kg == 0) sRow[INN ? wv : 0][i * 16 + n] = q;
-        }
+    for (int g = 0; g < 4; ++g) {
+        red[0][wv][kg * 4 + g][n] = acc[g];
+        if (DUAL) red[DUAL ? 1 : 0][wv][kg * 4 + g][n] = acc2[g];
+    }
+    if (INN) {      // lanes n, n + 16, n + 32, n + 48 hold shares of row n
+        ssq += __shfl_xor(ssq, 16);
+        ssq += __shfl_xor(ssq, 32);
+        if (kg == 0) sRow[INN ? wv : 0][n] = ssq;
     }
     __syncthreads();
     float* C = p.C + b * p.c_batch;
-    for (int e = tid; e < 64 * 16; e += 64 * NW) {
-        const int m = e >> 4, c = e & 15;
-        if (m >= M || n0 + c >= N) continue;
-        float s = 0.0f, s2 = 0.0f;
+    const int m = tid >> 4, c = tid & 15;
+    if (m >= M || n0 + c >= N) return;
+    float s = 0.0f, s2 = 0.0f;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            s += red[0][w][m][c];
-            if (DUAL) s2 += red[DUAL ? 1 : 0][w][m][c];
-        }
-        if (INN) {
-            float q = 0.0f;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) q += sRow[INN ? w : 0][m];
-            s *= 1.0f / sqrtf(q / (float)K + p.in_eps);
-        }
-        C[(g0 + m) * p.ldc + n0 + c] = dn_epilogue<EPI>(p, s, s2, b, g0 + m, n0 + c);
+    for (int w = 0; w < NW; ++w) {
+        s += red[0][w][m][c];
+        if (DUAL) s2 += red[DUAL ? 1 : 0][w][m][c];
     }
+    if (INN) {
+        float q = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) q += sRow[INN ? w : 0][m];
+        s *= 1.0f / sqrtf(q / (float)K + p.in_eps);
+    }
+    C[(g0 + m) * p.ldc + n0 + c] = dn_epilogue<EPI>(p, s, s2, b, g0 + m, n0 + c);
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
@@ -791,19 +587,18 @@ static void launch_tile(const i64h_linear& d, dim3 grid, hipStream_t s, int vecA
     }
 }
 
-// the large tile is off by default: at 4096 rows and 1024 to 8192 columns (256 to 1024 tiles) it measured 1.3 to 1.8 times SLOWER than
-// the 64 x 64 kernel - one workgroup per CU leaves nothing to run while it waits at its barriers
-static int g_skinny = 1, g_rows64 = 1, g_tile128 = 0;
+static int g_skinny = 1, g_rows16 = 1, g_block = 1, g_form = -1;
 
 extern "C" {
 
-// tuning / test knob, bit 0: launches of at most 8 rows on the weight-streaming kernel; bit 1: launches of at most 64 rows on the
-// fragment-streaming kernel; bit 2: launches of 256 or more 128 x 128 tiles on the large-tile kernel (default 3; 0 = every launch on
-// the 64 x 64 tile kernel)
+// tuning / test knob, bit 0: launches of at most I64H_SKINNY_ROWS rows on the weight-streaming kernel; bit 1: small launches of at most 16 rows on
+// the fragment-streaming kernel; bits 4 and up: one more than the form of linear_block_kernel to take whatever the size (default 3;
+// 0 = every launch on the 64 x 64 tile kernel)
 int i64h_set_linear_skinny(int32_t on) {
     g_skinny = on & 1;
-    g_rows64 = (on >> 1) & 1;
-    g_tile128 = (on >> 2) & 1;
+    g_rows16 = (on >> 1) & 1;
+    g_block = on != 0;
+    g_form = (on >> 4) - 1;
     return 0;
 }
 
@@ -849,46 +644,22 @@ int i64h_linear_run(const i64h_linear* dp, void* stream) {
         I64H_CHECK_LAUNCH();
         return 0;
     }
-    if (g_rows64 && !d.exact && d.M <= 64 && vecA && vecW) {
+    // (the weights of a larger product take longer than its launch: linear_block_kernel has more of them on their way at a time.  Rows dealt
+    // to experts: with one or two tokens so few experts have rows that 16-column workgroups are needed to spread their weights over the CUs)
+    if (g_rows16 && !d.exact && d.M <= 16 && vecA && vecW &&
+        (d.group_off ? d.rows_total > 0 && d.rows_total <= 4 : !dn_dual(d.epilogue) && d.K <= 1024 && (int64_t)d.N * d.batch <= 4096)) {
         const dim3 grid((unsigned)((d.N + 15) / 16), 1, (unsigned)d.batch);
+#define DN_ROWS16(E) case E: hipLaunchKernelGGL((linear_rows16_kernel<E>), grid, dim3(512), 0, s, d); break;
         switch (d.epilogue) {
-            // eight waves share the k steps where one accumulator is kept (the gate / up pair needs twice the LDS: four)
-            case I64H_EPI_GELU_MUL: hipLaunchKernelGGL((linear_rows64_kernel<I64H_EPI_GELU_MUL, 4>), grid, dim3(256), 0, s, d); break;
-            case I64H_EPI_SILU_MUL: hipLaunchKernelGGL((linear_rows64_kernel<I64H_EPI_SILU_MUL, 4>), grid, dim3(256), 0, s, d); break;
-            case I64H_EPI_CLAMP_GLU: hipLaunchKernelGGL((linear_rows64_kernel<I64H_EPI_CLAMP_GLU, 4>), grid, dim3(256), 0, s, d); break;
-            case I64H_EPI_MUL_SIGMOID: hipLaunchKernelGGL((linear_rows64_kernel<I64H_EPI_MUL_SIGMOID, 8>), grid, dim3(512), 0, s, d); break;
-            case I64H_EPI_SOFTCAP: hipLaunchKernelGGL((linear_rows64_kernel<I64H_EPI_SOFTCAP, 8>), grid, dim3(512), 0, s, d); break;
-            case I64H_EPI_GELU_ERF: hipLaunchKernelGGL((linear_rows64_kernel<I64H_EPI_GELU_ERF, 8>), grid, dim3(512), 0, s, d); break;
-            case I64H_EPI_XIELU: hipLaunchKernelGGL((linear_rows64_kernel<I64H_EPI_XIELU, 8>), grid, dim3(512), 0, s, d); break;
-            case I64H_EPI_RELU_SQ: hipLaunchKernelGGL((linear_rows64_kernel<I64H_EPI_RELU_SQ, 8>), grid, dim3(512), 0, s, d); break;
-            case I64H_EPI_ADD: hipLaunchKernelGGL((linear_rows64_kernel<I64H_EPI_ADD, 8>), grid, dim3(512), 0, s, d); break;
-            case I64H_EPI_DECAY: hipLaunchKernelGGL((linear_rows64_kernel<I64H_EPI_DECAY, 8>), grid, dim3(512), 0, s, d); break;
-            case I64H_EPI_ROW_SIGMOID: hipLaunchKernelGGL((linear_rows64_kernel<I64H_EPI_ROW_SIGMOID, 8>), grid, dim3(512), 0, s, d); break;
-            case I64H_EPI_IN_NORM: hipLaunchKernelGGL((linear_rows64_kernel<I64H_EPI_IN_NORM, 8>), grid, dim3(512), 0, s, d); break;
-            case I64H_EPI_SCALE: hipLaunchKernelGGL((linear_rows64_kernel<I64H_EPI_SCALE, 8>), grid, dim3(512), 0, s, d); break;
-            default: hipLaunchKernelGGL((linear_rows64_kernel<I64H_EPI_STORE, 8>), grid, dim3(512), 0, s, d); break;
+            DN_ROWS16(I64H_EPI_GELU_MUL) DN_ROWS16(I64H_EPI_SILU_MUL) DN_ROWS16(I64H_EPI_CLAMP_GLU) DN_ROWS16(I64H_EPI_MUL_SIGMOID) DN_ROWS16(I64H_EPI_SOFTCAP) DN_ROWS16(I64H_EPI_GELU_ERF) DN_ROWS16(I64H_EPI_XIELU) DN_ROWS16(I64H_EPI_RELU_SQ)
+            DN_ROWS16(I64H_EPI_ADD) DN_ROWS16(I64H_EPI_DECAY) DN_ROWS16(I64H_EPI_ROW_SIGMOID) DN_ROWS16(I64H_EPI_IN_NORM) DN_ROWS16(I64H_EPI_SCALE)
+            default: hipLaunchKernelGGL((linear_rows16_kernel<I64H_EPI_STORE>), grid, dim3(512), 0, s, d); break;
         }
+#undef DN_ROWS16
         I64H_CHECK_LAUNCH();
         return 0;
     }
-    const int64_t tiles128 = ((d.N + 127) / 128) * ((d.M + 127) / 128) * (int64_t)d.batch;
-    if (g_tile128 && !d.group_off && !d.exact && d.epilogue != I64H_EPI_IN_NORM && tiles128 >= 256) {     // at least a workgroup per CU: the large tile pays
-        const dim3 grid((unsigned)((d.N + 127) / 128), (unsigned)((d.M + 127) / 128), (unsigned)d.batch);
-        switch (d.epilogue) {
-            case I64H_EPI_GELU_MUL: hipLaunchKernelGGL((linear_tile128_kernel<I64H_EPI_GELU_MUL>), grid, dim3(256), 0, s, d, vecA, vecW); break;
-            case I64H_EPI_SILU_MUL: hipLaunchKernelGGL((linear_tile128_kernel<I64H_EPI_SILU_MUL>), grid, dim3(256), 0, s, d, vecA, vecW); break;
-            case I64H_EPI_CLAMP_GLU: hipLaunchKernelGGL((linear_tile128_kernel<I64H_EPI_CLAMP_GLU>), grid, dim3(256), 0, s, d, vecA, vecW); break;
-            case I64H_EPI_MUL_SIGMOID: hipLaunchKernelGGL((linear_tile128_kernel<I64H_EPI_MUL_SIGMOID>), grid, dim3(256), 0, s, d, vecA, vecW); break;
-            case I64H_EPI_SOFTCAP: hipLaunchKernelGGL((linear_tile128_kernel<I64H_EPI_SOFTCAP>), grid, dim3(256), 0, s, d, vecA, vecW); break;
-            case I64H_EPI_GELU_ERF: hipLaunchKernelGGL((linear_tile128_kernel<I64H_EPI_GELU_ERF>), grid, dim3(256), 0, s, d, vecA, vecW); break;
-            case I64H_EPI_XIELU: hipLaunchKernelGGL((linear_tile128_kernel<I64H_EPI_XIELU>), grid, dim3(256), 0, s, d, vecA, vecW); break;
-            case I64H_EPI_RELU_SQ: hipLaunchKernelGGL((linear_tile128_kernel<I64H_EPI_RELU_SQ>), grid, dim3(256), 0, s, d, vecA, vecW); break;
-            case I64H_EPI_ADD: hipLaunchKernelGGL((linear_tile128_kernel<I64H_EPI_ADD>), grid, dim3(256), 0, s, d, vecA, vecW); break;
-            case I64H_EPI_DECAY: hipLaunchKernelGGL((linear_tile128_kernel<I64H_EPI_DECAY>), grid, dim3(256), 0, s, d, vecA, vecW); break;
-            case I64H_EPI_ROW_SIGMOID: hipLaunchKernelGGL((linear_tile128_kernel<I64H_EPI_ROW_SIGMOID>), grid, dim3(256), 0, s, d, vecA, vecW); break;
-            case I64H_EPI_SCALE: hipLaunchKernelGGL((linear_tile128_kernel<I64H_EPI_SCALE>), grid, dim3(256), 0, s, d, vecA, vecW); break;
-            default: hipLaunchKernelGGL((linear_tile128_kernel<I64H_EPI_STORE>), grid, dim3(256), 0, s, d, vecA, vecW); break;
-        }
+    if (g_block && !d.exact && vecA && vecW && dn_linear_block(d, g_form, s)) {
         I64H_CHECK_LAUNCH();
         return 0;
     }

@@ -1,0 +1,337 @@
+// C = epilogue(A W^T) on v_mfma_f32_16x16x32_bf16, A fp32 (rounded to bf16 while it is staged), W bf16 [N, K]: BM x BN tiles staged
+// through LDS, four waves a tile and KG groups of four waves that share a tile's k steps.
+//
+// What bounds it.  Large launches: the step from memory to LDS - A is read as 32-bit values and rounded on the way, so a 128 x 128 tile moves
+// 48 KiB a step for 512 cycles of matrix instructions; hence 128 x 128 before anything smaller, two steps of registers on their way, the
+// next step's LDS writes between this step's matrix instructions (2956 x 11008 x 2048: 247 us with one step ahead, 224 with two, 199 with the
+// writes interleaved; the 64 x 64 kernel with 32-wide steps that this one replaces: 360 us, 370 TFLOP/s against 670).  Small launches: the
+// latency of a load per step, hence groups that share the steps, their sums added in LDS in a fixed order (64 x 2048 x 2048: 19.6 us with
+// fragments straight from memory before, 15.1 with a group a tile, 8.3 with 16 x 64 tiles and four; 64 x 32000 x 2048, whose 131 MB take 28 us at
+// the rate of a large copy: 133 -> 31 us).
+#include "i64h_dense_dev.h"
+#include <type_traits>
+
+// 16-byte loads through a buffer descriptor: a 32-bit offset per lane, the step's offset in a scalar register, and offsets past the end read
+// as zeros - a ragged end needs no branch and nothing is done to the registers behind the load
+typedef uint32_t dn_v4u __attribute__((ext_vector_type(4)));
+constexpr uint32_t DN_BUF_END = 0xfffffff0u;       // from here on: zeros
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t dn_buffer(const void* base) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)DN_BUF_END, 0x00020000);
+}
+__device__ __forceinline__ dn_v4u dn_load16(__amdgpu_buffer_rsrc_t r, uint32_t lane_bytes, uint32_t step_bytes) {
+    return __builtin_amdgcn_raw_buffer_load_b128(r, lane_bytes, step_bytes, 0);
+}
+
+template <int EPI, int BM, int BN, int KG>
+__global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kernel(const i64h_linear p, const int n_tiles, const int m_tiles, const int vecC) {
+    constexpr bool DUAL = dn_dual(EPI), INN = EPI == I64H_EPI_IN_NORM;
+    constexpr int BK = 64, NWM = BM >= 64 ? 2 : 1, NWN = 4 / NWM;      // waves of a group over rows and columns
+    constexpr int WM = BM / NWM, WN = BN / NWN, FM = WM / 16, FN = WN / 16;
+    static_assert(FM > 0 && FN > (DUAL ? 1 : 0), "");
+    constexpr int PA = (BM + 31) / 32, PB = BN / 32;       // staging passes: 32 rows of 64 values, 8 values a thread
+    constexpr int COLS = DUAL ? BN / 2 : BN;               // output columns of a tile
+    constexpr int PLANE = (BM + BN) * BK;
+    // [buffer][group][A rows, W rows]; (variables of their own, so that the writes of one step may be scheduled between the reads of the other)
+    __shared__ __attribute__((aligned(16))) uint16_t s0[KG * PLANE], s1[KG * PLANE];
+    __shared__ float sRow[INN ? KG : 1][INN ? BM : 1];
+    const int grp = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+    const int tid = threadIdx.x & 255, lane = tid & 63, wid = tid >> 6, wm = wid / NWN, wn = wid % NWN;
+    const int N = p.N, K = p.K;
+    // the tile of this workgroup: workgroups go to the 8 XCDs in turn, so that every XCD gets a run of neighbouring tiles (its L2 then serves
+    // their common rows and columns); within the run, columns of eight row tiles
+    int64_t b = blockIdx.z, g0 = 0, rows = p.M;
+    int mt, nt, R = m_tiles;
+    {
+        // rows dealt to batches: lane l counts the tiles of batch 64 c + l, the lanes up to it their sum (one round of loads, not a chain of them)
+        const int batches = p.group_off ? p.batch : 0;
+        auto count = [&](int c) {
+            const int e = c + lane;
+            int t = e < batches ? (p.group_off[e + 1] - p.group_off[e] + BM - 1) / BM : 0;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int up = __shfl_up(t, d);
+                t += lane >= d ? up : 0;
+            }
+            return t;
+        };
+        if (p.group_off) {
+            R = 0;
+            for (int c = 0; c < batches; c += 64) R += __builtin_amdgcn_readlane(count(c), 63);
+        }
+        const int T = R * n_tiles, id = blockIdx.x;
+        if (id >= T) return;
+        const int q = T >> 3, r = T & 7, x = id & 7;
+        const int t = x * q + min(x, r) + (id >> 3);
+        const int per = 8 * n_tiles, g = t / per, first = g * 8, width = min(8, R - first), in = t - g * per;
+        mt = first + in % width;
+        nt = in / width;
+        for (int c = 0; c < batches; c += 64) {
+            const int upto = count(c), all = __builtin_amdgcn_readlane(upto, 63);
+            if (mt >= all) {
+                mt -= all;
+                continue;
+            }
+            const int e = __ffsll((unsigned long long)__ballot(upto > mt)) - 1;
+            if (e > 0) mt -= __builtin_amdgcn_readlane(upto, e - 1);
+            b = c + e;
+            g0 = p.group_off[b];
+            rows = p.group_off[b + 1] - g0;
+            break;
+        }
+    }
+    const int n0 = nt * COLS;
+    const int64_t m0 = g0 + (int64_t)mt * BM;
+    const int M = (int)min((int64_t)BM, rows - (int64_t)mt * BM);
+    const int lr = tid >> 3, lc = tid & 7;                 // staging: row within a pass, chunk of eight k
+    // (rows past the end repeat the last one and are not stored)
+    const __amdgpu_buffer_rsrc_t bufA = dn_buffer(p.A + b * p.a_batch + (p.a_rows ? 0 : m0 * p.lda)), bufW = dn_buffer((const uint16_t*)p.W + b * p.w_batch);
+    uint32_t oa[PA], ow[PB];
+#pragma unroll
+    for (int i = 0; i < PA; ++i) {
+        const int r = min(i * 32 + lr, M - 1);
+        oa[i] = (uint32_t)((p.a_rows ? p.a_rows[m0 + r] : r) * p.lda + lc * 8) * 4u;
+    }
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+        const int r = i * 32 + lr;
+        // gate and up rows of the same columns go to the same wave: its first half of fragments, its second half
+        const int c = DUAL ? (r / WN) * (WN / 2) + r % (WN / 2) : r;
+        ow[i] = (uint32_t)((int64_t)(min(n0 + c, N - 1) + (DUAL && r % WN >= WN / 2 ? N : 0)) * K + lc * 8) * 2u;
+    }
+    dn_v4u ra[2][PA][2], rb[2][PB], rn[2][2];      // two steps on their way
+    float ssq[PA];
+#pragma unroll
+    for (int i = 0; i < PA; ++i) ssq[i] = 0.0f;
+    // this group's steps: KT of them from k_base on, the last group's past the end of K reading zeros
+    const int KT = ((K + BK - 1) / BK + KG - 1) / KG, k_base = grp * KT * BK, k_end = KG > 1 ? min(K, k_base + KT * BK) : K;
+    auto gload = [&](int kt, auto set) {
+        constexpr int S = decltype(set)::value;
+        const int k0 = k_base + kt * BK;
+        const uint32_t past = k0 + lc * 8 >= k_end ? DN_BUF_END : 0u;      // (K is a multiple of eight)
+#pragma unroll
+        for (int i = 0; i < PA; ++i) {
+            ra[S][i][0] = dn_load16(bufA, oa[i] | past, k0 * 4);
+            ra[S][i][1] = dn_load16(bufA, (oa[i] + 16) | past, k0 * 4);
+        }
+#pragma unroll
+        for (int i = 0; i < PB; ++i) rb[S][i] = dn_load16(bufW, ow[i] | past, k0 * 2);
+        if (INN) {
+            const float* nw = p.in_norm_w + (past ? 0 : k0 + lc * 8);
+            rn[S][0] = *(const dn_v4u*)nw;
+            rn[S][1] = *(const dn_v4u*)(nw + 4);
+        }
+    };
+    // 128-byte rows; a row's chunks are stored exclusive-or its number, so that the 16 rows of a fragment read lie in different banks
+    auto lstore = [&](auto set) {      // into the buffer of the same number
+        constexpr int S = decltype(set)::value;
+        uint16_t* sm = (S ? s1 : s0) + grp * PLANE;
+#pragma unroll
+        for (int i = 0; i < PA; ++i) {
+            dn_v4f u = __builtin_bit_cast(dn_v4f, ra[S][i][0]), v = __builtin_bit_cast(dn_v4f, ra[S][i][1]);
+            if (INN) {      // the row's squares as they come, the norm's weights on what is staged
+                const dn_v4f nu = __builtin_bit_cast(dn_v4f, rn[S][0]), nv = __builtin_bit_cast(dn_v4f, rn[S][1]);
+#pragma unroll
+                for (int g = 0; g < 4; ++g) ssq[i] = fmaf(u[g], u[g], ssq[i]);
+#pragma unroll
+                for (int g = 0; g < 4; ++g) ssq[i] = fmaf(v[g], v[g], ssq[i]);
+#pragma unroll
+                for (int g = 0; g < 4; ++g) u[g] *= nu[g], v[g] *= nv[g];
+            }
+            const int r = i * 32 + lr;
+            if (BM >= 32 || lr < BM)
+                *(dn_v4u*)&sm[r * BK + ((lc ^ (r & 7)) << 3)] = dn_v4u{dn_bf16_pair(u[0], u[1]), dn_bf16_pair(u[2], u[3]), dn_bf16_pair(v[0], v[1]), dn_bf16_pair(v[2], v[3])};
+        }
+#pragma unroll
+        for (int i = 0; i < PB; ++i) {
+            const int r = i * 32 + lr;
+            *(dn_v4u*)&sm[(BM + r) * BK + ((lc ^ (r & 7)) << 3)] = rb[S][i];
+        }
+    };
+    dn_v4f acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = dn_v4f{0, 0, 0, 0};
+    const int fr = lane & 15, fk = lane >> 4;
+    auto multiply = [&](auto set) {
+        constexpr int S = decltype(set)::value;
+        const uint16_t* sm = (S ? s1 : s0) + grp * PLANE;
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            const int ch = ((kk * 4 + fk) ^ (fr & 7)) << 3;
+            dn_v8bf a[FM], w[FN];
+#pragma unroll
+            for (int i = 0; i < FM; ++i) a[i] = *(const dn_v8bf*)&sm[(wm * WM + i * 16 + fr) * BK + ch];
+#pragma unroll
+            for (int j = 0; j < FN; ++j) w[j] = *(const dn_v8bf*)&sm[(BM + wn * WN + j * 16 + fr) * BK + ch];
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j], a[i], acc[i][j], 0, 0, 0);
+        }
+    };
+    // the next tile's writes and the loads behind it between the matrix instructions; small tiles are faster as the compiler orders them
+    auto interleave = [&]() {
+        if (BN < 128 || BM < 64) return;
+        constexpr int MF = 2 * FM * FN, DR = 2 * (FM + FN), DW = PA + PB, VM = 2 * PA + PB;
+        __builtin_amdgcn_sched_group_barrier(0x100, DR / 2, 0);
+#pragma unroll
+        for (int g = 0; g < 8; ++g) {
+            __builtin_amdgcn_sched_group_barrier(0x008, MF / 8, 0);
+            if (g < 4) __builtin_amdgcn_sched_group_barrier(0x100, DR / 8, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+            __builtin_amdgcn_sched_group_barrier(0x200, DW / 8 > 0 ? DW / 8 : 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x020, (VM + 7) / 8, 0);
+        }
+    };
+    constexpr std::integral_constant<int, 0> S0{};
+    constexpr std::integral_constant<int, 1> S1{};
+    // a step's operands are requested two steps ahead (a workgroup alone on its CU waits for them otherwise), past the end as zeros
+    gload(0, S0);
+    gload(1, S1);
+    lstore(S0);
+    __syncthreads();
+    for (int kt = 0; kt + 1 < KT; kt += 2) {
+        gload(kt + 2, S0);
+        multiply(S0);
+        lstore(S1);
+        interleave();
+        __syncthreads();
+        gload(kt + 3, S1);
+        multiply(S1);
+        lstore(S0);
+        interleave();
+        __syncthreads();
+    }
+    if (KT & 1) multiply(S0);
+    if (INN) {      // eight neighbouring lanes hold a row's shares
+#pragma unroll
+        for (int i = 0; i < PA; ++i) {
+            float q = ssq[i];
+            q += __shfl_xor(q, 1);
+            q += __shfl_xor(q, 2);
+            q += __shfl_xor(q, 4);
+            if (lc == 0 && (BM >= 32 || lr < BM)) sRow[INN ? grp : 0][INN ? i * 32 + lr : 0] = q;
+        }
+        if (KG == 1) __syncthreads();
+    }
+    if (KG > 1) {      // the groups' sums meet in LDS, added in the groups' order by the first one
+        constexpr int TILE = 4 * 64 * FM * FN;      // fragments of four values
+        static_assert((KG - 1) * TILE * 16 <= 2 * KG * PLANE * 2, "");
+        constexpr int HALF = (KG * PLANE * 2) / (TILE * 16);      // tiles that fit the first buffer
+        __syncthreads();
+        dn_v4f* dst = grp - 1 < HALF ? (dn_v4f*)s0 + (grp - 1) * TILE : (dn_v4f*)s1 + (grp - 1 - HALF) * TILE;
+        if (grp > 0) {
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j) dst[(i * FN + j) * 256 + tid] = acc[i][j];
+        }
+        __syncthreads();
+        if (grp > 0) return;
+#pragma unroll
+        for (int g = 0; g < KG - 1; ++g) {
+            const dn_v4f* src = g < HALF ? (const dn_v4f*)s0 + g * TILE : (const dn_v4f*)s1 + (g - HALF) * TILE;
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j) acc[i][j] += src[(i * FN + j) * 256 + tid];
+        }
+    }
+    // the weights are the left operand: a lane holds four neighbouring columns of a row
+    float* C = p.C + b * p.c_batch;
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+        const int rl = wm * WM + i * 16 + fr;
+        if (rl >= M) continue;
+        const int64_t r = m0 + rl;
+        float f = 1.0f;
+        if (INN) {
+            float q = 0.0f;
+#pragma unroll
+            for (int g = 0; g < KG; ++g) q += sRow[INN ? g : 0][INN ? rl : 0];
+            f = 1.0f / sqrtf(q / (float)K + p.in_eps);
+        }
+#pragma unroll
+        for (int j = 0; j < (DUAL ? FN / 2 : FN); ++j) {
+            const int c = n0 + wn * (COLS / NWN) + j * 16 + fk * 4;
+            auto out = [&](int g) { return dn_epilogue<EPI>(p, INN ? acc[i][j][g] * f : acc[i][j][g], DUAL ? acc[i][DUAL ? j + FN / 2 : j][g] : 0.0f, b, r, c + g); };
+            float* dst = C + r * p.ldc + c;
+            if (vecC && c + 4 <= N) {
+                *(float4*)dst = make_float4(out(0), out(1), out(2), out(3));
+            } else {
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    if (c + g < N) dst[g] = out(g);
+            }
+        }
+    }
+}
+
+enum { PLAIN = 1, PAIR = 2 };      // the epilogues that a form is built for: all but the gate / up pairs, those, both
+template <int BM, int BN, int KG, int FOR = PLAIN | PAIR>
+static void launch(const i64h_linear& d, hipStream_t s) {
+    const int cols = dn_dual(d.epilogue) ? BN / 2 : BN;
+    const int nt = (d.N + cols - 1) / cols;
+    int64_t mt = (d.M + BM - 1) / BM;
+    if (d.group_off) {      // at most one partly filled row tile per batch beside the full ones
+        const int64_t most = mt * d.batch;
+        mt = d.rows_total > 0 ? (most < d.rows_total / BM + d.batch ? most : d.rows_total / BM + d.batch) : most;
+    }
+    const int vecC = (uintptr_t)d.C % 16 == 0 && d.ldc % 4 == 0 && d.c_batch % 4 == 0;
+    const dim3 grid((unsigned)(mt * nt), 1, d.group_off ? 1u : (unsigned)d.batch);
+#define DN_BLOCK(E) case E: if constexpr (FOR & (dn_dual(E) ? PAIR : PLAIN)) hipLaunchKernelGGL((linear_block_kernel<E, BM, BN, KG>), grid, dim3(256 * KG), 0, s, d, nt, (int)mt, vecC); break;
+    switch (d.epilogue) {
+        DN_BLOCK(I64H_EPI_GELU_MUL) DN_BLOCK(I64H_EPI_SILU_MUL) DN_BLOCK(I64H_EPI_CLAMP_GLU) DN_BLOCK(I64H_EPI_MUL_SIGMOID) DN_BLOCK(I64H_EPI_SOFTCAP)
+        DN_BLOCK(I64H_EPI_GELU_ERF) DN_BLOCK(I64H_EPI_XIELU) DN_BLOCK(I64H_EPI_RELU_SQ) DN_BLOCK(I64H_EPI_ADD) DN_BLOCK(I64H_EPI_DECAY) DN_BLOCK(I64H_EPI_ROW_SIGMOID)
+        DN_BLOCK(I64H_EPI_IN_NORM) DN_BLOCK(I64H_EPI_SCALE)
+        default: if constexpr (FOR & PLAIN) hipLaunchKernelGGL((linear_block_kernel<I64H_EPI_STORE, BM, BN, KG>), grid, dim3(256 * KG), 0, s, d, nt, (int)mt, vecC); break;
+    }
+#undef DN_BLOCK
+}
+
+// Workgroups of a launch in BM x BN tiles (all columns of a gate / up pair count twice).
+static int64_t tiles(const i64h_linear& d, int BM, int BN) {
+    int64_t mt = (d.M + BM - 1) / BM * d.batch;
+    if (d.group_off && d.rows_total > 0 && d.rows_total / BM + d.batch < mt) mt = d.rows_total / BM + d.batch;
+    const int64_t cols = dn_dual(d.epilogue) ? 2 * (int64_t)d.N : d.N;
+    return mt * ((cols + BN - 1) / BN);
+}
+
+bool dn_linear_block(const i64h_linear& d, int form, hipStream_t s) {
+    const bool dual = dn_dual(d.epilogue);
+    // the buffer descriptors' 32-bit offsets: rows of a tile, or whatever a_rows may name; all of a batch's weights
+    const int64_t span = (d.a_rows ? d.a_height : 128) * d.lda * 4;
+    if ((d.a_rows && d.a_height <= 0) || span >= (int64_t)DN_BUF_END - 64 || (int64_t)d.N * (dual ? 4 : 2) * d.K >= (int64_t)DN_BUF_END - 64) return false;
+    if (tiles(d, 16, 64) > 0x7fffffff) return false;
+    if (form < 0) {
+        // Large tiles as long as (nearly) every CU gets one: their operands are read least often.  Below that, a tile's k steps follow each
+        // other at the latency of a load and what counts is how few of them a workgroup has and how many CUs work: four groups a tile
+        // while its workgroups (one a CU, LDS) run in one round, two groups while there is a CU for each.  Microseconds in replayed graphs:
+        //   rows x columns x k       128x128  64x128   64x64  64x64/2  32x64/4  16x64/4
+        //   4096 x 5760 x 1024           98     110     133
+        //   2000 x 1024 x 1024         18.8    13.7    13.6     14.4     24.0     34.8
+        //    512 x 6464 x 2048         31.2    30.7    39.7     40.4     59.2     83.7
+        //    512 x 2048 x 2048         28.3    21.3    16.8     13.9     18.2     27.2
+        //    512 x 1024 x 1024         15.7    12.5     9.4      8.5      7.3     10.5
+        //     64 x 11392 x 2048                        16.3     13.5     18.6     21.1
+        //     64 x 2048 x 2048                         15.1     12.3      9.6      8.3
+        const bool longer = d.K > 128;
+        if (longer && tiles(d, 128, 128) >= 200) form = 0;
+        else if (longer && tiles(d, 64, 128) >= 250) form = 1;
+        else if (dual ? tiles(d, 16, 128) <= 256 : tiles(d, 16, 64) <= 256) form = dual ? 6 : 5;
+        else if (!dual && d.K >= 512 && tiles(d, 32, 64) <= 256) form = 4;
+        else if (d.K >= 512 && tiles(d, 64, 64) <= 256) form = 3;
+        else form = 2;
+    }
+    switch (form) {
+        case 0: launch<128, 128, 1>(d, s); break;
+        case 1: launch<64, 128, 1>(d, s); break;
+        case 3: launch<64, 64, 2>(d, s); break;
+        case 4: if (!dual) { launch<32, 64, 4, PLAIN>(d, s); break; } [[fallthrough]];
+        case 5: if (!dual) { launch<16, 64, 4, PLAIN>(d, s); break; } [[fallthrough]];
+        case 6: if (dual) { launch<16, 128, 2, PAIR>(d, s); break; } [[fallthrough]];      // 64 columns of a gate / up pair: 64 x 1792 x 2048 15.0 us, 64x64/2 17.5
+        default: launch<64, 64, 1>(d, s); break;
+    }
+    return true;
+}
