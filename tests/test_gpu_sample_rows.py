@@ -1,0 +1,65 @@
+"""The token draw against 64-bit softmax sums: vocabulary sizes around what a workgroup holds, every route (listed candidates, keys in registers, keys read
+again), ties, masked and non-finite logits."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def draw(x, T, k, p, u):
+    from vllm_i64_amd import ops_dense as D
+    n = x.shape[0]
+    dev = torch.device("cuda:0")
+    f = lambda v, dt: torch.full((n,), v, dtype=dt, device=dev)
+    return D.sample_rows(x.to(dev), temperature=f(T, torch.float32), top_k=f(k, torch.int32), top_p=f(p, torch.float32), u=u.to(dev)).cpu()
+
+
+def check(x, T, k, p, u, got):
+    """Every drawn token is kept, and u lies within fp32 rounding of the token's stretch of the running sum."""
+    V = x.shape[1]
+    for row, uu, tok in zip(x.double(), u.double(), got.tolist()):
+        w = torch.exp((row - row.max()) / float(torch.tensor(T)))
+        keep = torch.ones(V, dtype=torch.bool) if k <= 0 or k >= V else row >= row.topk(k).values[-1]
+        if p < 1:
+            order = row.masked_fill(~keep, -math.inf).argsort(descending=True)
+            mass = torch.cumsum(torch.where(keep, w, 0.0)[order], 0)
+            edge = row[order[min(int((mass < float(torch.tensor(p)) * mass[-1] * (1 - 1e-5)).sum()), V - 1)]]
+            slack = row[order[min(int((mass < float(torch.tensor(p)) * mass[-1] * (1 + 1e-5)).sum()), V - 1)]]
+            assert row[tok] >= slack
+            keep &= row >= edge
+        assert keep[tok] or p < 1
+        cum = torch.cumsum(torch.where(keep, w, 0.0), 0)
+        lo, hi = (cum[tok] - w[tok]) / cum[-1], cum[tok] / cum[-1]
+        assert lo - 1e-4 <= uu <= hi + 1e-4, (V, k, p, float(uu), tok)
+
+
+@pytest.mark.parametrize("V", [1, 5, 301, 1024, 4096, 4099, 32000, 32768, 32769, 50257])
+@pytest.mark.parametrize("k", [0, 1, 50, 512, 513, 40000])
+@pytest.mark.parametrize("p", [1.0, 0.9, 0.3])
+def test_draw(V, k, p):
+    g = torch.Generator().manual_seed(V + k)
+    x = 2 * torch.randn(7, V, generator=g)
+    u = torch.tensor([0.0, 0.1, 0.37, 0.5, 0.77, 0.95, 0.9999])
+    check(x, 0.8, k, p, u, draw(x, 0.8, k, p, u))
+
+
+@pytest.mark.parametrize("V", [300, 8192, 40000])
+@pytest.mark.parametrize("k", [0, 3, 600])
+def test_ties_masks_and_non_finite(V, k):
+    u = torch.tensor([0.0, 0.26, 0.51, 0.99])
+    same = torch.zeros(4, V)
+    got = draw(same, 1.0, k, 1.0, u)      # (values equal to the k-th are all kept)
+    assert torch.all((got - u.double() * V).abs() <= 2)
+    x = torch.full((4, V), -math.inf)
+    x[:, [7, 9, V - 1]] = torch.tensor([1.0, 1.0, 1.0])
+    assert draw(x, 1.0, k, 1.0, torch.tensor([0.1, 0.5, 0.9, 0.33])).tolist() == [7, 9, V - 1, 7]
+    assert draw(x, 1.0, k, 0.0, u).tolist() == [7] * 4      # no mass asked for: the first of the largest
+    assert draw(torch.full((4, V), -math.inf), 1.0, k, 0.9, u).tolist() == [0] * 4
+    x = torch.randn(4, V)
+    x[:, 11] = math.inf
+    assert draw(x, 1.0, k, 0.9, u).tolist() == [11] * 4
+    x[:, 11], x[:, 5], x[:, 20] = 50.0, math.nan, 50.0
+    assert draw(x, 1.0, k, 1.0, u).tolist() == [11] * 4      # a sum that is no number: the first of the largest
+    assert draw(x, 0.0, k, 1.0, u).tolist() == [11] * 4      # greedy

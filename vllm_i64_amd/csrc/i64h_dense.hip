@@ -469,101 +469,276 @@ __global__ __launch_bounds__(256) void gated_postnorm_kernel(const i64h_postnorm
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
-// One workgroup per row.  Thresholds are found by bisection over the bits of the order-preserving integer image of a float:
+// One workgroup of 16 waves per row.  Thresholds are found by bisection over the bits of the order-preserving integer image of a float:
 // top-k: the largest key with at least k values at or above it; top-p: the largest key whose values at or above it hold at
-// least p of the mass.  The draw walks the kept values in index order (each thread a contiguous range).
-__device__ __forceinline__ float block_sum(float v, float* red) {
-    v = wave_sum(v);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    return red[0] + red[1] + red[2] + red[3];
-}
+// least p of the mass.  The draw takes the first kept value, in index order, behind which the running sum exceeds u of the total.
+//
+// What bounds it is the chain of dependent block-wide sums, one per bit, so each is made short.  With top-k of at most 512 the row is read
+// once: the k-th largest of the threads' maxima is a bound that at least k values reach and few others do, those (at most 1024, sorted by
+// index) lie one to a thread from there on.  Without top-k the row's keys stay in registers (NV float4 per thread; NV = 0: read again,
+// vocabularies beyond 32768).  64 rows of 32000, top-k 50 and top-p 0.95: 1280 us with four
+// waves that read the row again for every bit, 34 us now.
+constexpr int SR_WAVES = 16, SR_THREADS = 64 * SR_WAVES, SR_LIST = SR_THREADS, SR_TOPK = 512;
 
-__global__ __launch_bounds__(256) void sample_rows_kernel(const float* __restrict__ logits, int64_t* __restrict__ out, int V,
-                                                          const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
-                                                          const float* __restrict__ top_p, const float* __restrict__ u) {
-    __shared__ float red[4];
-    __shared__ float smax[256];
-    __shared__ int sidx[256];
-    __shared__ float part[257];
-    __shared__ int chosen;
-    const int tid = threadIdx.x;
+template <int NV>
+__global__ __launch_bounds__(SR_THREADS) void sample_rows_kernel(const float* __restrict__ logits, int64_t* __restrict__ out, int V, const int vec,
+                                                                 const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
+                                                                 const float* __restrict__ top_p, const float* __restrict__ u) {
+    __shared__ float redf[2][SR_WAVES];
+    __shared__ int redi[2][SR_WAVES], bestc[SR_WAVES];
+    __shared__ float bestv[SR_WAVES];
+    __shared__ uint32_t lkey[SR_LIST], skey[SR_LIST];
+    __shared__ int lidx[SR_LIST], sidx[SR_LIST];
+    __shared__ int listed, chosen;
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int64_t r = blockIdx.x;
     const float* x = logits + r * V;
-    const float T = temperature ? temperature[r] : 0.0f;
-    // the maximum and its first index
+    int turn = 0;      // the sums alternate between two buffers: one barrier each
+    auto sum_i = [&](int v) {      // v: a wave's share, the same in all of its lanes
+        if (lane == 0) redi[turn & 1][wid] = v;
+        __syncthreads();
+        int s = 0;
+#pragma unroll
+        for (int w = 0; w < SR_WAVES; ++w) s += redi[turn & 1][w];
+        ++turn;
+        return s;
+    };
+    auto sum_f = [&](float v) {      // v: a thread's share
+        v = wave_sum(v);
+        if (lane == 0) redf[turn & 1][wid] = v;
+        __syncthreads();
+        float s = 0.0f;
+#pragma unroll
+        for (int w = 0; w < SR_WAVES; ++w) s += redf[turn & 1][w];
+        ++turn;
+        return s;
+    };
+    auto wave_count = [&](bool b) { return __popcll(__ballot(b)); };
+    constexpr int STEP = 4 * SR_THREADS;
+    const int chunks = (V + STEP - 1) / STEP;
+    auto load4 = [&](int i, uint32_t* k) {      // the keys of four neighbouring values; past the end 0, which no number has
+        const int c = i * STEP + tid * 4;
+        if (vec && c + 4 <= V) {
+            const float4 v = *(const float4*)(x + c);
+            k[0] = f32_to_ordered(v.x), k[1] = f32_to_ordered(v.y), k[2] = f32_to_ordered(v.z), k[3] = f32_to_ordered(v.w);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) k[j] = c + j < V ? f32_to_ordered(x[c + j]) : 0u;
+        }
+    };
+    uint32_t key[NV > 0 ? NV : 1][4];
     float best = -INFINITY;
     int bi = V;
-    for (int c = tid; c < V; c += 256) {
-        const float v = x[c];
-        if (v > best || (v == best && c < bi)) { best = v; bi = c; }
-    }
-    smax[tid] = best;
-    sidx[tid] = bi;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (tid < s) {
-            const float v = smax[tid + s];
-            const int i = sidx[tid + s];
-            if (v > smax[tid] || (v == smax[tid] && i < sidx[tid])) { smax[tid] = v; sidx[tid] = i; }
+    uint32_t kmax = 0;
+    auto look = [&](int i, const uint32_t* k) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float v = ordered_to_f32(k[j]);
+            const int c = i * STEP + tid * 4 + j;
+            if (c < V && (v > best || (v == best && c < bi))) best = v, bi = c;
+            kmax = max(kmax, k[j]);
         }
-        __syncthreads();
+    };
+    if (NV > 0) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) load4(i, key[i]);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) look(i, key[i]);
+    } else {
+        for (int i = 0; i < chunks; ++i) {
+            load4(i, key[0]);
+            look(i, key[0]);
+        }
     }
-    const float mx = smax[0];
+    uint32_t rmax = kmax;      // the largest key of the row, and the maximum and its first index
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        const float v = __shfl_xor(best, d);
+        const int c = __shfl_xor(bi, d);
+        if (v > best || (v == best && c < bi)) best = v, bi = c;
+        rmax = max(rmax, (uint32_t)__shfl_xor((int)rmax, d));
+    }
+    if (lane == 0) bestv[wid] = best, bestc[wid] = bi, skey[wid] = rmax;
+    if (tid == 0) listed = 0, chosen = V;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < SR_WAVES; ++w) {
+        const float v = bestv[w];
+        const int c = bestc[w];
+        if (v > best || (v == best && c < bi)) best = v, bi = c;
+        rmax = max(rmax, skey[w]);
+    }
+    const int arg = bi < V ? bi : 0;
+    const float T = temperature ? temperature[r] : 0.0f;
     if (!(T > 0.0f)) {
-        if (tid == 0) out[r] = sidx[0] < V ? sidx[0] : 0;
+        if (tid == 0) out[r] = arg;
         return;
     }
-    const float invT = 1.0f / T;
-    uint32_t thr = 0;  // keep values whose key is >= thr
+    const float invT = 1.0f / T, mx = best, pp = top_p ? top_p[r] : 1.0f, uu = u ? u[r] : 0.5f;
     const int k = top_k ? top_k[r] : 0;
-    if (k > 0 && k < V) {
+    auto weight = [&](uint32_t q) { return expf((ordered_to_f32(q) - mx) * invT); };
+    // the largest key that `enough` holds for, bit by bit; keys above every value of the row hold nothing
+    auto bisect = [&](auto enough) {
+        uint32_t thr = 0;
         for (int bit = 31; bit >= 0; --bit) {
             const uint32_t cand = thr | (1u << bit);
-            float cnt = 0.0f;
-            for (int c = tid; c < V; c += 256) cnt += f32_to_ordered(x[c]) >= cand ? 1.0f : 0.0f;
-            if (block_sum(cnt, red) >= (float)k) thr = cand;
+            if (cand > rmax) continue;
+            const int e = enough(cand);
+            if (e) thr = cand;
+            if (e > 1) break;      // exactly what was asked for: lower bits exclude nothing more
+        }
+        return thr;
+    };
+    if (k > 0 && k < V && k <= SR_TOPK) {
+        const uint32_t bound = bisect([&](uint32_t cand) {
+            const int n = sum_i(wave_count(kmax >= cand));
+            return n == k ? 2 : (n > k ? 1 : 0);
+        });
+        auto list4 = [&](int i, const uint32_t* q) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (q[j] >= bound && i * STEP + tid * 4 + j < V) {
+                    const int at = atomicAdd(&listed, 1);
+                    if (at < SR_LIST) lkey[at] = q[j], lidx[at] = i * STEP + tid * 4 + j;
+                }
+        };
+        if (NV > 0) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) list4(i, key[i]);
+        } else {
+            for (int i = 0; i < chunks; ++i) {
+                load4(i, key[0]);
+                list4(i, key[0]);
+            }
+        }
+        __syncthreads();
+        const int n = listed;
+        if (n <= SR_LIST) {
+            if (tid < n) {
+                const int c = lidx[tid];
+                int at = 0;
+                for (int j = 0; j < n; ++j) at += lidx[j] < c ? 1 : 0;
+                skey[at] = lkey[tid];
+                sidx[at] = c;
+            }
+            __syncthreads();
+            const uint32_t q = tid < n ? skey[tid] : 0u;
+            uint32_t thr = bisect([&](uint32_t cand) {
+                const int m = sum_i(wave_count(q >= cand));
+                return m == k ? 2 : (m > k ? 1 : 0);
+            });
+            const bool mine = tid < n;
+            const float w = mine ? weight(q) : 0.0f;
+            if (pp < 1.0f) {
+                const float need = pp * sum_f(mine && q >= thr ? w : 0.0f);
+                if (!(need > 0.0f)) {      // nothing is asked for (or the sum is no number): the most likely token
+                    if (tid == 0) out[r] = arg;
+                    return;
+                }
+                const uint32_t t2 = bisect([&](uint32_t cand) { return sum_f(mine && q >= max(cand, thr) ? w : 0.0f) >= need ? 1 : 0; });
+                thr = max(thr, t2);
+            }
+            // running sums in index order: within the wave, then over the waves in front
+            float run = mine && q >= thr ? w : 0.0f;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const float up = __shfl_up(run, d);
+                run += lane >= d ? up : 0.0f;
+            }
+            if (lane == 63) redf[turn & 1][wid] = run;
+            __syncthreads();
+            float before = 0.0f, total = 0.0f;
+#pragma unroll
+            for (int v = 0; v < SR_WAVES; ++v) {
+                if (v == wid) before = total;
+                total += redf[turn & 1][v];
+            }
+            if (mine && q >= thr && before + run > uu * total) atomicMin(&chosen, sidx[tid]);
+            __syncthreads();
+            if (tid == 0) out[r] = chosen < V ? chosen : arg;  // rounding at the far end of the walk: the most likely token
+            return;
         }
     }
-    const float pp = top_p ? top_p[r] : 1.0f;
+    // the row as a whole
+    auto each = [&](auto f) {      // f(chunk, four keys)
+        if (NV > 0) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) f(i, key[i]);
+        } else {
+            for (int i = 0; i < chunks; ++i) {
+                load4(i, key[0]);
+                f(i, key[0]);
+            }
+        }
+    };
+    uint32_t thr = 0;
+    if (k > 0 && k < V)
+        thr = bisect([&](uint32_t cand) {
+            int n = 0;
+            each([&](int, const uint32_t* q) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) n += wave_count(q[j] >= cand);
+            });
+            n = sum_i(n);
+            return n == k ? 2 : (n > k ? 1 : 0);
+        });
+    thr = max(thr, 1u);      // (0: the places past the end)
+    auto mass = [&](uint32_t cut) {
+        float s = 0.0f;
+        each([&](int, const uint32_t* q) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s += q[j] >= cut ? weight(q[j]) : 0.0f;
+        });
+        return sum_f(s);
+    };
     if (pp < 1.0f) {
-        float z = 0.0f;
-        for (int c = tid; c < V; c += 256) z += f32_to_ordered(x[c]) >= thr ? expf((x[c] - mx) * invT) : 0.0f;
-        const float need = pp * block_sum(z, red);
-        uint32_t t2 = 0;
-        for (int bit = 31; bit >= 0; --bit) {
-            const uint32_t cand = t2 | (1u << bit), cut = cand > thr ? cand : thr;
-            float s = 0.0f;
-            for (int c = tid; c < V; c += 256) s += f32_to_ordered(x[c]) >= cut ? expf((x[c] - mx) * invT) : 0.0f;
-            if (block_sum(s, red) >= need) t2 = cand;
+        const float need = pp * mass(thr);
+        if (!(need > 0.0f)) {
+            if (tid == 0) out[r] = arg;
+            return;
         }
-        thr = t2 > thr ? t2 : thr;
+        const uint32_t t2 = bisect([&](uint32_t cand) { return mass(max(cand, thr)) >= need ? 1 : 0; });
+        thr = max(thr, t2);
     }
-    // draw
-    const int per = (V + 255) / 256, lo = tid * per, hi = min(V, lo + per);
-    float s = 0.0f;
-    for (int c = lo; c < hi; ++c) s += f32_to_ordered(x[c]) >= thr ? expf((x[c] - mx) * invT) : 0.0f;
-    part[tid + 1] = s;
-    if (tid == 0) { part[0] = 0.0f; chosen = -1; }
-    __syncthreads();
-    if (tid == 0)
-        for (int i = 1; i <= 256; ++i) part[i] += part[i - 1];
-    __syncthreads();
-    const float target = (u ? u[r] : 0.5f) * part[256];
-    if (hi > lo && target >= part[tid] && target < part[tid + 1]) {
-        float a = part[tid];
-        int pick = -1;
-        for (int c = lo; c < hi; ++c) {
-            if (f32_to_ordered(x[c]) < thr) continue;
-            a += expf((x[c] - mx) * invT);
-            pick = c;
-            if (a > target) break;
+    const float target = uu * mass(thr);
+    // 4096 values at a time until the running sum passes the target, then inside that stretch
+    float base = 0.0f;
+    bool open = true;
+    each([&](int i, const uint32_t* q) {
+        if (!open || i >= chunks) return;
+        float w[4], s = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = q[j] >= thr ? weight(q[j]) : 0.0f, s += w[j];
+        float run = s;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const float up = __shfl_up(run, d);
+            run += lane >= d ? up : 0.0f;
         }
-        if (pick >= 0) chosen = pick;
-    }
+        if (lane == 63) redf[turn & 1][wid] = run;
+        __syncthreads();
+        float before = 0.0f, total = 0.0f;
+#pragma unroll
+        for (int v = 0; v < SR_WAVES; ++v) {
+            if (v == wid) before = total;
+            total += redf[turn & 1][v];
+        }
+        ++turn;
+        if (base + total > target) {
+            float a = base + (before + (run - s));
+            int pick = V;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                a += w[j];
+                if (pick == V && q[j] >= thr && a > target) pick = i * STEP + tid * 4 + j;
+            }
+            if (pick < V) atomicMin(&chosen, pick);
+            open = false;
+        }
+        base += total;
+    });
     __syncthreads();
-    if (tid == 0) out[r] = chosen >= 0 ? chosen : sidx[0];  // rounding at the far end of the walk: the most likely token
+    if (tid == 0) out[r] = chosen < V ? chosen : arg;
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
@@ -698,7 +873,12 @@ int i64h_sample_rows(const float* logits, int64_t* out, int64_t rows, int32_t V,
                      const float* top_p, const float* u, void* stream) {
     I64H_CHECK_ARG(rows >= 0 && V > 0 && logits && out, "sample_rows: bad arguments");
     if (rows == 0) return 0;
-    hipLaunchKernelGGL(sample_rows_kernel, dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream, logits, out, (int)V, temperature, top_k, top_p, u);
+    const int vec = (uintptr_t)logits % 16 == 0 && V % 4 == 0;
+    hipStream_t s = (hipStream_t)stream;
+    if (V <= 8 * 4 * SR_THREADS)
+        hipLaunchKernelGGL((sample_rows_kernel<8>), dim3((unsigned)rows), dim3(SR_THREADS), 0, s, logits, out, (int)V, vec, temperature, top_k, top_p, u);
+    else
+        hipLaunchKernelGGL((sample_rows_kernel<0>), dim3((unsigned)rows), dim3(SR_THREADS), 0, s, logits, out, (int)V, vec, temperature, top_k, top_p, u);
     I64H_CHECK_LAUNCH();
     return 0;
 }
