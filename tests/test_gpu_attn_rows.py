@@ -1,0 +1,91 @@
+"""The matrix-core attention of prompt portions against 64-bit attention over the same bf16 rows: every number of heads that shares a workgroup, key widths
+that are no multiple of a step, pages of any size, tiles that hold rows of several sequences, cached tokens in front, windows, kept
+first positions, sinks, soft cap."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return torch.device("cuda:0")
+
+
+def pages(lens, past, block, g):
+    need = [(n + p + block - 1) // block for n, p in zip(lens, past)]
+    order = torch.randperm(sum(need), generator=g).to(torch.int32)
+    bt, at = torch.zeros(len(lens), max(need), dtype=torch.int32), 0
+    for i, k in enumerate(need):
+        bt[i, :k] = order[at:at + k]
+        at += k
+    pos = torch.cat([torch.arange(p, p + n, dtype=torch.int32) for n, p in zip(lens, past)])
+    slots = torch.cat([torch.full((n,), i, dtype=torch.int32) for i, n in enumerate(lens)])
+    return bt, pos, slots, sum(need)
+
+
+def reference(q, keys, values, pos, scale, window, keep, cap, sink):
+    """q [n, H, d], keys [H, T, d], values [H, T, v]: one sequence, 64 bits."""
+    s = torch.einsum("nhd,htd->hnt", q.double(), keys.double()) * scale
+    if cap:
+        s = cap * torch.tanh(s / cap)
+    j = torch.arange(keys.shape[1])[None, :]
+    i = pos[:, None].long()
+    see = (j <= i) if not window else (j <= i) & ((i - j < window) | (j < keep))
+    s = torch.cat([s.masked_fill(~see, -math.inf), sink.double().view(-1, 1, 1).expand(-1, s.shape[1], 1)], -1)
+    return torch.einsum("hnt,htv->nhv", torch.softmax(s, -1)[..., :-1], values.double())
+
+
+LENS = [([1, 15, 16, 17, 40], [0, 3, 0, 31, 0]), ([70], [0]), ([33, 2], [64, 5])]
+
+
+@pytest.mark.parametrize("lens,past", LENS)
+@pytest.mark.parametrize("H,G,dim,vdim", [(4, 1, 64, 64), (2, 1, 32, 32), (3, 1, 64, 16), (8, 2, 24, 48), (6, 2, 128, 128), (12, 3, 8, 64)])
+@pytest.mark.parametrize("block,window,keep,cap", [(16, 0, 0, 0.0), (16, 20, 3, 0.0), (6, 33, 40, 0.0), (16, 0, 0, 2.0)])
+def test_keys_and_values(dev, lens, past, H, G, dim, vdim, block, window, keep, cap):
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator().manual_seed(H + dim + window)
+    bt, pos, slots, blocks = pages(lens, past, block, g)
+    n, w = int(pos.numel()), vdim + dim
+    cache = torch.randn(blocks, block, G * w, generator=g).bfloat16()
+    q = torch.randn(n, H, w, generator=g)
+    q[:, :, :vdim] = 0
+    sink = torch.randn(H, generator=g)
+    out = torch.full((n, H * vdim), 7.0, device=dev)
+    D.kattn(q.to(dev), cache.to(dev), None, bt.to(dev), slots.to(dev), pos.to(dev), chunk=0, bias=None, sink=True, heads=H, kv_heads=G, dim=dim, vdim=vdim, out=out, n=n, mode=3,
+            window=window, keep_first=keep, softcap=cap, sink_w=sink.to(dev))
+    # the prep kernel's scale is in the query: the launch has none of its own
+    at = 0
+    for i, (m, p) in enumerate(zip(lens, past)):
+        j = torch.arange(m + p)
+        rows = cache[bt[i].long()[j // block], j % block].view(m + p, G, w).repeat_interleave(H // G, 1).transpose(0, 1)
+        ref = reference(q[at:at + m, :, vdim:], rows[..., vdim:], rows[..., :vdim], pos[at:at + m], 1.0, window, keep, cap, sink)
+        got = out[at:at + m].view(m, H, vdim).double().cpu()
+        # two bf16 terms of query and weight: 2^-16 relative each, scores of up to sqrt(dim) * 4
+        assert torch.allclose(got, ref, atol=2e-3, rtol=1e-3), float((got - ref).abs().max())
+        at += m
+
+
+@pytest.mark.parametrize("lens,past", LENS)
+@pytest.mark.parametrize("H,r,e", [(4, 256, 32), (5, 256, 64), (8, 32, 8), (16, 128, 0), (2, 64, 64), (4, 144, 24)])
+@pytest.mark.parametrize("window", [0, 25])
+def test_latent_rows(dev, lens, past, H, r, e, window):
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator().manual_seed(H + r + e)
+    bt, pos, slots, blocks = pages(lens, past, 16, g)
+    n = int(pos.numel())
+    cache = torch.randn(blocks, 16, r + e, generator=g).bfloat16()
+    q = torch.randn(n, H, r + e, generator=g)
+    sink = torch.randn(H, generator=g)
+    out = torch.full((n * H * r,), 7.0, device=dev)
+    D.latent_attn(q.to(dev).flatten(), cache.to(dev), bt.to(dev), slots.to(dev), pos.to(dev), window=window, scale=0.1, heads=H, kv_rank=r, rot_dim=e, out=out, n=n, mode=3, sink=sink.to(dev))
+    at = 0
+    for i, (m, p) in enumerate(zip(lens, past)):
+        j = torch.arange(m + p)
+        rows = cache[bt[i].long()[j // 16], j % 16].expand(H, -1, -1)
+        ref = reference(q[at:at + m], rows, rows[..., :r], pos[at:at + m], 0.1, window, 0, 0.0, sink)
+        got = out.view(n, H, r)[at:at + m].double().cpu()
+        assert torch.allclose(got, ref, atol=5e-4, rtol=5e-4), float((got - ref).abs().max())
+        at += m

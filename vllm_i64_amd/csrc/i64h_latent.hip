@@ -5,8 +5,9 @@
 // q'_latent . latent_j + q_rot . key_rot_j and all heads read the same cached rows.
 //   latent_prep_kernel     : RMS norm of the latent, rotation of the shared key part and of every head's rotated query part,
 //                            cache write - one workgroup per token
-//   latent_attn_mfma_kernel: bf16 caches of aligned widths - 16 query vectors per wave (a token's heads, or a head's consecutive rows)
-//                            on the bf16 matrix cores, see below
+//   latent_attn_rows_kernel: bf16 caches of aligned widths, portions of prompts - four waves of 16 rows that share 32 keys at a time through LDS
+//   latent_attn_mfma_decode_kernel (latent_attn_mfma_kernel): rows that are one per sequence - a token's heads, 16 query vectors per wave;
+//                            both on the bf16 matrix cores, see below
 //   latent_attn_row_kernel : any width and cache type, true fp32 products: one wave per (token, head): 64 keys at a time, one key per lane for the scores (fp32 dot over the
 //                            cached row), online softmax over the wave, weighted row sum with the columns spread over the lanes
 #include "i64h_common.h"
@@ -153,10 +154,8 @@ __global__ __launch_bounds__(256) void latent_attn_row_kernel(const i64h_latent_
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
-// Matrix-core form (bf16 cache).  One wave per task of 16 query vectors that walk the same cached rows:
-//   head tiles: the (up to) 16 heads of a group of one token  - decode rows, one token per sequence;
-//   row tiles : 16 consecutive rows of the step for one head   - portions of prompts; rows of a tile that belong to different
-//               sequences are handled run by run (a run's keys are masked for every other row).
+// Matrix-core form (bf16 cache) of rows that are one per sequence.  One wave per task of 16 query vectors that walk the same cached rows:
+// the (up to) 16 heads of a group of one token.  (Behind the decode-form knob; the arrangement that such launches take is below it.)
 // Per tile of 32 keys: scores S[16, 32] = Q K^T on v_mfma_f32_16x16x32_bf16 with the cached rows read straight from memory as B
 // fragments (8 consecutive values of one key per lane) and the scaled query carried as TWO bf16 terms (hi + lo, 16 mantissa bits),
 // masking and the online softmax in fp32 on the accumulator layout, the weights again as two bf16 terms through LDS into the
@@ -176,10 +175,10 @@ __device__ __forceinline__ void lt_split(float x, uint32_t& hi, uint32_t& lo) {
     lo = lt_rne(x - __uint_as_float(hi << 16));
 }
 
-// KD, NB: 32-wide steps over a cached row and 16-column blocks of the output that the instance holds registers for (rows of at most
+// KD, NB: 32-wide steps over a cached row and 16-column blocks of the output that an instance holds registers for (rows of at most
 // 32 KD values, kv_rank <= 16 NB): the widest instance keeps two waves per SIMD, narrow rows leave room for more.
 template <int KD, int NB>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, KD > 4 ? 2 : 8))) void latent_attn_mfma_kernel(const i64h_latent_attn_args p, const int row_tiles, const int splits) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, KD > 4 ? 2 : 8))) void latent_attn_mfma_kernel(const i64h_latent_attn_args p, const int splits) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int lane = threadIdx.x, n = lane & 15, kg = lane >> 4;
     const int r = p.kv_rank, D = r + p.rot_dim, H = p.heads, bs = p.block_size, win = p.window;
@@ -195,14 +194,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, KD > 4 ? 
     const int G = p.kv_groups > 1 ? p.kv_groups : 1, rep = H / G, tpg = (rep + 15) / 16;
     const int hgroups = G * tpg;
     const int rstride = p.row_stride > 0 ? p.row_stride : D;
-    const int coff = (row_tiles ? (int)(task % H) / rep : (int)(task % hgroups) / tpg) * D;
-    const int hbase = row_tiles ? (int)(task % H) : ((int)(task % hgroups) / tpg) * rep + ((int)(task % hgroups) % tpg) * 16;
+    const int coff = (int)(task % hgroups) / tpg * D;
+    const int hbase = ((int)(task % hgroups) / tpg) * rep + ((int)(task % hgroups) % tpg) * 16;
     auto row_of = [&](int m, int64_t& tok, int& head) -> bool {
-        if (row_tiles) {     // the heads of a row tile are neighbours in the launch: they walk the same cached rows at the same time
-            tok = (task / H) * 16 + m;
-            head = hbase;
-            return tok < p.n;
-        }
         tok = task / hgroups;
         head = hbase + m;
         return ((int)(task % hgroups) % tpg) * 16 + m < rep;
@@ -248,7 +242,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, KD > 4 ? 
     for (int g = 0; g < 4; ++g) {
         const int pp = info[kg * 4 + g];
         lor[g] = p.chunk > 0 ? (max(pp, 0) / p.chunk) * p.chunk : (win > 0 ? max(0, pp - win + 1) : 0);
-        hrow[g] = min(row_tiles ? hbase : hbase + kg * 4 + g, H - 1);
+        hrow[g] = min(hbase + kg * 4 + g, H - 1);
         mrow[g] = sink ? (p.sink_w ? p.sink_w[hrow[g]] * 1.4426950408889634f : 0.0f) : -INFINITY;
         lrow[g] = sink ? 1.0f : 0.0f;
     }
@@ -574,6 +568,253 @@ __global__ __launch_bounds__(64) void latent_attn_mfma_decode_kernel(const i64h_
     }
 }
 
+// Portions of prompts: consecutive rows that share their sequences' cached rows.  A workgroup is four waves, each 16 rows of one head; the heads
+// of a workgroup belong to one key head (HW of them; 4 / HW blocks of 16 rows), so that all four waves read the same 32 keys, staged
+// in LDS once: row by row for the scores, the value columns transposed (a thread takes 4 keys x 8 columns) for the second product.
+// Products are taken transposed, S^T = K Q^T and out^T = V^T P^T: a lane then holds one row's scores (its maximum needs two exchanges, its
+// weights are the second product's operand as they lie, with the keys of the two 16-key blocks interleaved) and four neighbouring columns of
+// that row's result.  The next tile is requested before this one's products and stored behind them into the other buffer, the rows of
+// the one after that are looked up.  Query and weights are two bf16 terms each, as in the kernel above; sums, maxima and masks fp32.
+//
+// Bound by LDS and its latency: per 32 keys of 256 + 32 values a workgroup reads 136 KiB of fragments for 68 matrix instructions a wave, and
+// the registers of two waves per SIMD leave few reads on their way (one wave per SIMD with all it wants: 194 us where two take 130).
+// 8 prompts of 512 tokens, 16 heads over one cached row of 288: 304 -> 130 us against the form before (a wave per workgroup that read every
+// fragment from memory itself and transposed it two bytes at a time), 16 heads of 64 over 4 key heads 120 -> 48 us, 32 heads of 64 over 8 key heads
+// on prompts of 1531, 257, 64, 3 and 1101 tokens 285 -> 82 us, one prompt of 77 tokens 29 -> 20 and 17 -> 11 us.
+// KD: 32-wide steps over the columns that take part in the scores, NB: 16-column blocks of the result, EXTRA: key scales, a soft cap or a bias.
+template <int KD, int NB, bool EXTRA>
+__global__ __launch_bounds__(256, 2) void latent_attn_rows_kernel(const i64h_latent_attn_args p, const int hw) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, n = lane & 15, kg = lane >> 4;
+    const int r = p.kv_rank, D = r + p.rot_dim, H = p.heads, bs = p.block_size, win = p.window, koff = p.key_off & ~31;
+    const int keep = p.chunk <= 0 && win > 0 ? p.keep_first : 0;
+    const int kld = D - koff + 8;             // halves per key row in LDS: the columns that take part in the scores
+    const int plane = 32 * kld + r * LT_VLD;
+    uint16_t* const buf0 = (uint16_t*)smem;   // twice: keys [32][kld], values transposed [r][LT_VLD]
+    int* const info = (int*)(buf0 + 2 * plane);      // [64] positions, [64] slots (-1: no such row)
+    const int G = p.kv_groups > 1 ? p.kv_groups : 1, rep = H / G;
+    const int rstride = p.row_stride > 0 ? p.row_stride : D;
+    const int hgroups = H / hw, rows = 16 * (4 / hw), row_tiles = (int)((p.n + rows - 1) / rows);
+    const int task = blockIdx.x, hg = task % hgroups, rt = row_tiles - 1 - task / hgroups;      // (the longest contexts first)
+    const int head = hg * hw + wid % hw, coff = hg * hw / rep * D, wr = wid / hw * 16;
+    const int64_t row0 = (int64_t)rt * rows;
+    if (tid < rows) {
+        const bool ok = row0 + tid < p.n;
+        info[tid] = ok ? p.positions[row0 + tid] : -1;
+        info[64 + tid] = ok ? p.slot_ids[row0 + tid] : -1;
+    }
+    const int64_t tok = row0 + wr + n;
+    const bool valid = tok < p.n;
+    // the query of row n times scale * log2(e) (the softmax runs on powers of two), columns koff + ks * 32 + kg * 8 .. + 7, as two bf16 terms;
+    // zeros past the end, where the key reads repeat the first columns: no step and no block of columns has a branch of its own
+    uint4 Qh[KD], Ql[KD];
+    {
+        const float* q = p.Q + ((valid ? tok : row0) * H + head) * D;
+        const float qs = p.scale * 1.4426950408889634f;
+#pragma unroll
+        for (int ks = 0; ks < KD; ++ks) {
+            const int d0 = koff + ks * 32 + kg * 8;
+            Qh[ks] = Ql[ks] = make_uint4(0, 0, 0, 0);
+            if (valid && d0 < D) {
+                const float4 a = *(const float4*)(q + d0), b = *(const float4*)(q + d0 + 4);
+                const float v[8] = {a.x * qs, a.y * qs, a.z * qs, a.w * qs, b.x * qs, b.y * qs, b.z * qs, b.w * qs};
+                uint32_t h[8], l[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) lt_split(v[i], h[i], l[i]);
+                Qh[ks] = make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16));
+                Ql[ks] = make_uint4(l[0] | (l[1] << 16), l[2] | (l[3] << 16), l[4] | (l[5] << 16), l[6] | (l[7] << 16));
+            }
+        }
+    }
+    lt_v4f acc[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[nb] = lt_v4f{0, 0, 0, 0};
+    // (the weight sum of a row is kept in four shares, one per group of keys: the sink belongs to one of them)
+    float m = p.sink ? (p.sink_w ? p.sink_w[head] * 1.4426950408889634f : 0.0f) : -INFINITY, l = p.sink && kg == 0 ? 1.0f : 0.0f;
+    const float capl = p.softcap * 1.4426950408889634f;
+    const uint16_t* const cache = (const uint16_t*)p.cache + coff;
+    auto first_seen = [&](int pos) { return p.chunk > 0 ? pos / p.chunk * p.chunk : (win > 0 ? max(0, pos - win + 1) : 0); };
+    // staging: this thread's four keys and its (at most two) groups of eight columns
+    constexpr int PASS = NB > 8 ? 2 : 1;
+    const int kq = tid & 7, cg = tid >> 3;
+    const int groups = D >> 3;
+    uint4 st[PASS][4];
+    int64_t src[4];
+    __syncthreads();
+    int s0 = 0;
+    while (s0 < rows) {
+        const int sl = info[64 + s0];
+        if (sl < 0) {
+            ++s0;
+            continue;
+        }
+        int s1 = s0 + 1;
+        while (s1 < rows && info[64 + s1] == sl) ++s1;
+        int lo = 0x7fffffff, hi = -1;                      // the keys of the run; the same for this wave's rows of it
+        int wlo = 0x7fffffff, whi = -1, wall = 0x7fffffff, wfrom = 0;
+        for (int i = s0; i < s1; ++i) {
+            const int pp = info[i], f = first_seen(max(pp, 0));
+            hi = max(hi, pp), lo = min(lo, f);
+            if (i >= wr && i < wr + 16) wlo = min(wlo, f), whi = max(whi, pp), wall = min(wall, pp), wfrom = max(wfrom, f);
+        }
+        if (wr < s0 || wr + 16 > s1) wall = -1;            // rows of another run: every tile is masked
+        const int pos = wr + n >= s0 && wr + n < s1 ? info[wr + n] : -1, from = first_seen(max(pos, 0));
+        const int32_t* bt = p.block_table + (int64_t)sl * p.max_blocks_per_seq;
+        // tiles of 32 keys: those of the kept first positions that lie in front of the window's first tile, then the window's
+        const int t0 = lo >> 5, kt = min((keep + 31) >> 5, t0), tiles = hi < 0 ? 0 : kt + (hi >> 5) - t0 + 1;
+        auto key_base = [&](int tile) { return (tile < kt ? tile : t0 + tile - kt) * 32; };
+        auto look_up = [&](int tile) {
+            const int j0 = key_base(min(tile, tiles - 1)) + kq * 4;
+            if ((bs & 3) == 0) {      // four neighbours of one page
+                const int f = min(j0, hi), pg = f / bs;
+                const int64_t base = (int64_t)bt[pg] * bs - pg * bs;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) src[i] = (base + min(j0 + i, hi)) * rstride;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int j = min(j0 + i, hi);
+                    src[i] = ((int64_t)bt[j / bs] * bs + j % bs) * rstride;
+                }
+            }
+        };
+        auto request = [&]() {
+#pragma unroll
+            for (int q = 0; q < PASS; ++q)
+                if (cg + 32 * q < groups)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) st[q][i] = *(const uint4*)(cache + src[i] + (cg + 32 * q) * 8);
+        };
+        auto store = [&](int b) {
+            uint16_t* K = buf0 + b * plane;
+            uint16_t* V = K + 32 * kld;
+#pragma unroll
+            for (int q = 0; q < PASS; ++q) {
+                const int c0 = (cg + 32 * q) * 8;
+                if (c0 >= D) continue;
+                if (c0 >= koff)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) *(uint4*)&K[(kq * 4 + i) * kld + c0 - koff] = st[q][i];
+                if (c0 < r) {
+                    // columns c0 + c of keys 4 kq .. + 3; a row of V holds the 32 keys as the second product's lanes take them:
+                    // [key group kg][16-key block][4 keys]
+                    const int at = (kq & 3) * 8 + (kq >> 2) * 4;
+                    const uint32_t a[4][4] = {{st[q][0].x, st[q][0].y, st[q][0].z, st[q][0].w}, {st[q][1].x, st[q][1].y, st[q][1].z, st[q][1].w},
+                                              {st[q][2].x, st[q][2].y, st[q][2].z, st[q][2].w}, {st[q][3].x, st[q][3].y, st[q][3].z, st[q][3].w}};
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) {
+                        const uint32_t sel = c & 1 ? 0x07060302u : 0x05040100u;
+                        *(uint2*)&V[(c0 + c) * LT_VLD + at] = make_uint2(__builtin_amdgcn_perm(a[1][c >> 1], a[0][c >> 1], sel), __builtin_amdgcn_perm(a[3][c >> 1], a[2][c >> 1], sel));
+                    }
+                }
+            }
+        };
+        if (tiles > 0) {
+            look_up(0);
+            request();
+            look_up(1);
+            store(0);
+        }
+        __syncthreads();
+        for (int tile = 0; tile < tiles; ++tile) {
+            const int kb = key_base(tile);
+            if (tile + 1 < tiles) {
+                request();
+                look_up(tile + 2);
+            }
+            const uint16_t* K = buf0 + (tile & 1) * plane;
+            const uint16_t* V = K + 32 * kld;
+            if (kb <= whi && (kb + 31 >= wlo || kb < keep)) {      // (something that a row of this wave sees)
+                lt_v4f S[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+                for (int ks = 0; ks < KD; ++ks) {
+                    const int d0 = ks * 32 + kg * 8;
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) {
+                        const lt_v8bf kf = __builtin_bit_cast(lt_v8bf, *(const uint4*)&K[(16 * b + n) * kld + (d0 < D - koff ? d0 : 0)]);
+                        S[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, __builtin_bit_cast(lt_v8bf, Qh[ks]), S[b], 0, 0, 0);
+                        S[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, __builtin_bit_cast(lt_v8bf, Ql[ks]), S[b], 0, 0, 0);
+                    }
+                }
+                if (EXTRA) {
+#pragma unroll
+                    for (int b = 0; b < 2; ++b)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            const int j = kb + 16 * b + kg * 4 + g, jc = min(j, hi);
+                            if (p.kscale) S[b][g] *= p.kscale[(int64_t)bt[jc / bs] * bs + jc % bs];
+                            if (capl > 0.0f) S[b][g] = capl * tanhf(S[b][g] / capl);
+                            if (p.bias) S[b][g] += 1.4426950408889634f * p.bias[(int64_t)min(max(pos - j, 0), p.bias_rows - 1) * H + head];
+                        }
+                }
+                if (kb + 31 > wall || kb < wfrom) {
+#pragma unroll
+                    for (int b = 0; b < 2; ++b)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            const int j = kb + 16 * b + kg * 4 + g;
+                            S[b][g] = j <= pos && (j >= from || j < keep) ? S[b][g] : -INFINITY;
+                        }
+                }
+                float mx = fmaxf(fmaxf(fmaxf(S[0][0], S[0][1]), fmaxf(S[0][2], S[0][3])), fmaxf(fmaxf(S[1][0], S[1][1]), fmaxf(S[1][2], S[1][3])));
+                mx = fmaxf(mx, __shfl_xor(mx, 16));
+                mx = fmaxf(mx, __shfl_xor(mx, 32));
+                const float mn = fmaxf(m, mx), ms = mn == -INFINITY ? 0.0f : mn;
+                const float al = __builtin_amdgcn_exp2f(m - ms);
+                m = mn;
+                float w[2][4], sum = 0.0f;
+                uint32_t ph[4], pl[4];
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        w[b][g] = __builtin_amdgcn_exp2f(S[b][g] - ms);
+                        sum += w[b][g];
+                    }
+#pragma unroll
+                    for (int g = 0; g < 4; g += 2) {
+                        uint32_t h0, l0, h1, l1;
+                        lt_split(w[b][g], h0, l0);
+                        lt_split(w[b][g + 1], h1, l1);
+                        ph[b * 2 + g / 2] = h0 | (h1 << 16);
+                        pl[b * 2 + g / 2] = l0 | (l1 << 16);
+                    }
+                }
+                l = l * al + sum;
+                if (__ballot(al != 1.0f)) {
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) acc[nb][g] *= al;
+                }
+                const lt_v8bf Ph = __builtin_bit_cast(lt_v8bf, make_uint4(ph[0], ph[1], ph[2], ph[3])), Pl = __builtin_bit_cast(lt_v8bf, make_uint4(pl[0], pl[1], pl[2], pl[3]));
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) {
+                    const lt_v8bf vf = __builtin_bit_cast(lt_v8bf, *(const uint4*)&V[min(nb * 16 + n, r - 1) * LT_VLD + kg * 8]);
+                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, Ph, acc[nb], 0, 0, 0);
+                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, Pl, acc[nb], 0, 0, 0);
+                }
+            }
+            if (tile + 1 < tiles) store((tile + 1) & 1);
+            __syncthreads();
+        }
+        s0 = s1;
+    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (!valid) return;
+    float* o = p.out + (tok * H + head) * r;
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+        if (nb * 16 < r) {
+            const float4 v = make_float4(acc[nb][0] * inv, acc[nb][1] * inv, acc[nb][2] * inv, acc[nb][3] * inv);
+            float* dst = o + nb * 16 + kg * 4;
+            if (((uintptr_t)p.out & 15) == 0) *(float4*)dst = v;
+            else dst[0] = v.x, dst[1] = v.y, dst[2] = v.z, dst[3] = v.w;
+        }
+}
+
 // the shares of a token's keys, merged: one wave per (token, head); lane s holds share s's maximum and weight sum (at most 64
 // shares), then every lane sums its columns over the shares, eight loads in flight at a time
 __global__ __launch_bounds__(64) void latent_attn_merge_kernel(const i64h_latent_attn_args p, const int splits) {
@@ -662,10 +903,25 @@ int i64h_latent_attn(const i64h_latent_attn_args* dp, void* stream) {
         const dim3 grid((unsigned)tasks, (unsigned)splits);
         hipStream_t st = (hipStream_t)stream;
         const int size = (D <= 64 && d.kv_rank <= 64) ? 0 : ((D <= 128 && d.kv_rank <= 128) ? 1 : 2);     // the narrowest instance that holds the rows
-        if (row_tiles || !g_decode_form) {
-            if (size == 0) hipLaunchKernelGGL((latent_attn_mfma_kernel<2, 4>), grid, dim3(64), bytes, st, d, row_tiles, splits);
-            else if (size == 1) hipLaunchKernelGGL((latent_attn_mfma_kernel<4, 8>), grid, dim3(64), bytes, st, d, row_tiles, splits);
-            else hipLaunchKernelGGL((latent_attn_mfma_kernel<LT_KD, LT_NB>), grid, dim3(64), bytes, st, d, row_tiles, splits);
+        if (row_tiles) {
+            const int rep = d.heads / G, hw = rep % 4 == 0 ? 4 : (rep % 2 == 0 ? 2 : 1), rows = 16 * (4 / hw);
+            const int64_t wgs = (d.n + rows - 1) / rows * (d.heads / hw);
+            const size_t lds = ((size_t)32 * (D - (d.key_off & ~31) + 8) + (size_t)d.kv_rank * LT_VLD) * 4 + 128 * 4;
+            const bool extra = d.kscale || d.bias || d.softcap > 0.0f;
+#define LT_ROWS(KD, NB) do { \
+                if (extra) hipLaunchKernelGGL((latent_attn_rows_kernel<KD, NB, true>), dim3((unsigned)wgs), dim3(256), lds, st, d, hw); \
+                else hipLaunchKernelGGL((latent_attn_rows_kernel<KD, NB, false>), dim3((unsigned)wgs), dim3(256), lds, st, d, hw); \
+            } while (0)
+            const int steps = (D - (d.key_off & ~31) + 31) / 32;
+            if (steps <= 2 && d.kv_rank <= 64) LT_ROWS(2, 4);
+            else if (steps <= 4 && d.kv_rank <= 128) LT_ROWS(4, 8);
+            else if (steps <= 9) LT_ROWS(9, LT_NB);
+            else LT_ROWS(LT_KD, LT_NB);
+#undef LT_ROWS
+        } else if (!g_decode_form) {
+            if (size == 0) hipLaunchKernelGGL((latent_attn_mfma_kernel<2, 4>), grid, dim3(64), bytes, st, d, splits);
+            else if (size == 1) hipLaunchKernelGGL((latent_attn_mfma_kernel<4, 8>), grid, dim3(64), bytes, st, d, splits);
+            else hipLaunchKernelGGL((latent_attn_mfma_kernel<LT_KD, LT_NB>), grid, dim3(64), bytes, st, d, splits);
         } else {
             if (size == 0) hipLaunchKernelGGL((latent_attn_mfma_decode_kernel<2, 4>), grid, dim3(64), bytes, st, d, splits);
             else if (size == 1) hipLaunchKernelGGL((latent_attn_mfma_decode_kernel<4, 8>), grid, dim3(64), bytes, st, d, splits);
