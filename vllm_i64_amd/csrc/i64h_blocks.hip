@@ -70,6 +70,40 @@ template <int KPT>
 __device__ __forceinline__ int gd_channel(int nlane, int k) {
     return KPT >= 4 ? 4 * (nlane + 16 * (k >> 2)) + (k & 3) : nlane * KPT + k;
 }
+// A token's part in a column's state and what it reads, shared by both kernels: a lane's sums run in two chains (even and odd channels), whose
+// instructions follow each other without waiting.
+template <int KPT, bool CHD>
+__device__ __forceinline__ float gd_delta(float (&S)[KPT], const float* f, const float* k, const float* q, float v, float beta) {
+    float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+    for (int i = 0; i < KPT; ++i) {
+        S[i] *= f[CHD ? i : 0];
+        if (i & 1) s1 = fmaf(S[i], k[i], s1);
+        else s0 = fmaf(S[i], k[i], s0);
+    }
+    const float d = beta * (v - group_sum(s0 + s1, 16));
+    float o0 = 0.0f, o1 = 0.0f;
+#pragma unroll
+    for (int i = 0; i < KPT; ++i) {
+        S[i] = fmaf(k[i], d, S[i]);
+        if (i & 1) o1 = fmaf(S[i], q[i], o1);
+        else o0 = fmaf(S[i], q[i], o0);
+    }
+    return group_sum(o0 + o1, 16);
+}
+template <int KPT, bool CHD, bool FORGET>
+__device__ __forceinline__ float gd_linear(float (&S)[KPT], const float* f, const float* k, const float* q, float v) {
+    float o0 = 0.0f, o1 = 0.0f;
+#pragma unroll
+    for (int i = 0; i < KPT; ++i) {
+        const float fi = f[CHD ? i : 0];
+        S[i] = fmaf(fi, S[i], (FORGET ? 1.0f - fi : k[FORGET ? 0 : i]) * v);
+        if (i & 1) o1 = fmaf(S[i], q[i], o1);
+        else o0 = fmaf(S[i], q[i], o0);
+    }
+    return group_sum(o0 + o1, 16);
+}
+
 template <int KPT, int CPT, bool CHD, int TG, int RULE>
 __global__ __launch_bounds__(256) void gdn_scan_kernel(const i64h_gdn_args p, const int ctiles, const int vec) {
     const int N = p.dim, P = p.vdim;
@@ -143,30 +177,9 @@ __global__ __launch_bounds__(256) void gdn_scan_kernel(const i64h_gdn_args p, co
         if (t >= r1) return;
 #pragma unroll
         for (int j = 0; j < CPT; ++j) {
-            float part = 0.0f;
-            if constexpr (RULE == GD_DELTA) {
-                float seen = 0.0f;
-#pragma unroll
-                for (int k = 0; k < KPT; ++k) {
-                    S[j][k] *= u.f[CHD ? k : 0];
-                    seen = fmaf(S[j][k], u.k[k], seen);
-                }
-                seen = group_sum(seen, 16);
-                const float d = u.beta * (u.v[j] - seen);
-#pragma unroll
-                for (int k = 0; k < KPT; ++k) {
-                    S[j][k] = fmaf(u.k[k], d, S[j][k]);
-                    part = fmaf(S[j][k], u.q[k], part);
-                }
-            } else {
-#pragma unroll
-                for (int k = 0; k < KPT; ++k) {
-                    const float kk = RULE == GD_FORGET ? 1.0f - u.f[CHD ? k : 0] : u.k[RULE == GD_FORGET ? 0 : k];
-                    S[j][k] = fmaf(u.f[CHD ? k : 0], S[j][k], kk * u.v[j]);
-                    part = fmaf(S[j][k], u.q[k], part);
-                }
-            }
-            part = group_sum(part, 16);
+            float part;
+            if constexpr (RULE == GD_DELTA) part = gd_delta<KPT, CHD>(S[j], u.f, u.k, u.q, u.v[j], u.beta);
+            else part = gd_linear<KPT, CHD, RULE == GD_FORGET>(S[j], u.f, u.k, u.q, u.v[j]);
             if (nlane == 0 && cbase + j < P) p.out[t * p.ldo + a * P + cbase + j] = RULE == GD_DELTA ? part : part * p.q_scale;
         }
     };
@@ -202,6 +215,9 @@ __global__ __launch_bounds__(256) void gdn_scan_kernel(const i64h_gdn_args p, co
 // gdn_tile_kernel: the same recurrence, bit for bit, for runs of many rows.  What every wave of a workgroup reads of a token (query, key,
 // decays) is loaded once per workgroup, TT tokens at a time, into one of two LDS tiles while the other one is computed: the loads of a
 // tile have the arithmetic of a whole tile to arrive, and the waves read 16 bytes per lane from LDS one token ahead.  Needs 16-byte rows.
+// What bounds it is the chain from token to token - decay, row sum, correction - and the reads of the tile: the 16 tokens of a tile are one
+// stretch of code without a branch, so that a token's read-out runs beside the next one's sums, its result waiting in a lane until
+// the tile's end; 16 heads of 128, one run of 1531 rows: 339 -> 246 us (218 -> 160 ns a token), linear attention 283 -> 216 us.
 template <int KPT, int CPT, bool CHD, int RULE>
 __global__ __launch_bounds__(256) void gdn_tile_kernel(const i64h_gdn_args p, const int ctiles) {
     static_assert(KPT % 4 == 0, "whole 16-byte slices per lane");
@@ -294,51 +310,9 @@ __global__ __launch_bounds__(256) void gdn_tile_kernel(const i64h_gdn_args p, co
         u.beta = sG[b][i][0];
         if (!CHD) u.f[0] = sG[b][i][1];
     };
-    auto step = [&](int64_t t, const Tok& u) {
-        float seen[CPT], part[CPT], d[CPT];
-        if constexpr (RULE != GD_DELTA) {
-#pragma unroll
-            for (int j = 0; j < CPT; ++j) {
-                part[j] = 0.0f;
-#pragma unroll
-                for (int k = 0; k < KPT; ++k) {
-                    const float kk = RULE == GD_FORGET ? 1.0f - u.f[CHD ? k : 0] : u.k[RULE == GD_FORGET ? 0 : k];
-                    S[j][k] = fmaf(u.f[CHD ? k : 0], S[j][k], kk * u.v[j]);
-                    part[j] = fmaf(S[j][k], u.q[k], part[j]);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < CPT; ++j) {
-                const float o = group_sum(part[j], 16);
-                if (nlane == 0 && cbase + j < P) p.out[t * p.ldo + a * P + cbase + j] = o * p.q_scale;
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < CPT; ++j) {
-                seen[j] = 0.0f;
-#pragma unroll
-                for (int k = 0; k < KPT; ++k) {
-                    S[j][k] *= u.f[CHD ? k : 0];
-                    seen[j] = fmaf(S[j][k], u.k[k], seen[j]);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < CPT; ++j) d[j] = u.beta * (u.v[j] - group_sum(seen[j], 16));
-#pragma unroll
-            for (int j = 0; j < CPT; ++j) {
-                part[j] = 0.0f;
-#pragma unroll
-                for (int k = 0; k < KPT; ++k) {
-                    S[j][k] = fmaf(u.k[k], d[j], S[j][k]);
-                    part[j] = fmaf(S[j][k], u.q[k], part[j]);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < CPT; ++j) {
-                const float o = group_sum(part[j], 16);
-                if (nlane == 0 && cbase + j < P) p.out[t * p.ldo + a * P + cbase + j] = o;
-            }
-        }
+    auto step = [&](int j, const Tok& u) {
+        if constexpr (RULE == GD_DELTA) return gd_delta<KPT, CHD>(S[j], u.f, u.k, u.q, u.v[j], u.beta);
+        else return gd_linear<KPT, CHD, RULE == GD_FORGET>(S[j], u.f, u.k, u.q, u.v[j]) * p.q_scale;
     };
     gload(r0);
     lstore(0);
@@ -350,12 +324,39 @@ __global__ __launch_bounds__(256) void gdn_tile_kernel(const i64h_gdn_args p, co
         if (more) gload(t0 + TT);
         Tok A, B;
         fetch(b, 0, A);
-        for (int i = 0; i < cnt; i += 2) {
-            fetch(b, i + 1, B);            // (a tile has TT rows, an even number: zeros past the run's end)
-            step(t0 + i, A);
-            if (i + 1 < cnt) {
-                if (i + 2 < cnt) fetch(b, i + 2, A);
-                step(t0 + i + 1, B);
+        if (cnt == TT) {
+            // a whole tile without a branch: a token's read-out runs beside the next token's decay and sums.  All 16 lanes of a row end with
+            // a token's result: lane i keeps that of token i, stored once a tile
+            float o[CPT];
+#pragma unroll
+            for (int j = 0; j < CPT; ++j) o[j] = 0.0f;
+#pragma unroll
+            for (int i = 0; i < TT; i += 2) {
+                fetch(b, i + 1, B);
+#pragma unroll
+                for (int j = 0; j < CPT; ++j) {
+                    const float part = step(j, A);
+                    o[j] = nlane == i ? part : o[j];
+                }
+                if (i + 2 < TT) fetch(b, i + 2, A);
+#pragma unroll
+                for (int j = 0; j < CPT; ++j) {
+                    const float part = step(j, B);
+                    o[j] = nlane == i + 1 ? part : o[j];
+                }
+            }
+            if (nlane < TT)
+#pragma unroll
+                for (int j = 0; j < CPT; ++j)
+                    if (cbase + j < P) p.out[(t0 + nlane) * p.ldo + a * P + cbase + j] = o[j];
+        } else {
+            for (int i = 0; i < cnt; ++i) {
+                if (i > 0) fetch(b, i, A);
+#pragma unroll
+                for (int j = 0; j < CPT; ++j) {
+                    const float part = step(j, A);
+                    if (nlane == 0 && cbase + j < P) p.out[(t0 + i) * p.ldo + a * P + cbase + j] = part;
+                }
             }
         }
         if (more) lstore(b ^ 1);
@@ -639,12 +640,15 @@ static int gdn_launch(const i64h_gdn_args& d, void* stream) {
     };
     const int kround = kpt <= 4 ? 4 : (kpt <= 8 ? 8 : 16);
     if (g_gdn_form != 1 && vec_ok(kround) && (g_gdn_form > 1 || d.n >= 8 * (int64_t)d.nseg)) {
-        // one value column per lane while that is at most two workgroups per CU, two (fewer reads of the tile) beyond
-        const int cpt = g_gdn_form > 1 ? (g_gdn_form == 4 ? 4 : g_gdn_form - 1) : ((int64_t)d.heads * ((d.vdim + 15) / 16) * d.nseg <= 512 ? 1 : 2);
+        // One value column per lane: a token then takes the longest run least time, and it is the longest run that the launch waits for (16
+        // heads of 128, runs of 1531, 257, 64, 3 and 1101 rows: 275 us, two columns 449; 27 single rows beside 229 and 256: 67 and 99).  Two
+        // columns (fewer reads of the tile) only where many workgroups wait for a CU and the runs are long (32 runs of 128 rows: 212 and 215 us,
+        // linear attention 163 and 177; 8 of 512: 210 and 222).
+        const int cpt = g_gdn_form > 1 ? (g_gdn_form == 4 ? 4 : g_gdn_form - 1) : ((int64_t)d.heads * ((d.vdim + 15) / 16) * d.nseg >= 1024 && d.n >= 64 * (int64_t)d.nseg ? 2 : 1);
         const int ctiles = (d.vdim + 16 * cpt - 1) / (16 * cpt);
         const dim3 grid((unsigned)(d.heads * ctiles), (unsigned)d.nseg);
         auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, (hipStream_t)stream, d, ctiles); };
-#define GDN_TILE(C, CHD)                                            \
+#define GDN_TILE(C, CHD)                                             \
     if (kround == 4) launch(gdn_tile_kernel<4, C, CHD, RULE>);      \
     else if (kround == 8) launch(gdn_tile_kernel<8, C, CHD, RULE>); \
     else launch(gdn_tile_kernel<16, C, CHD, RULE>);
