@@ -7,7 +7,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-FORMS = {"128x128": 1, "64x128": 2, "64x64": 3, "64x64/2": 4, "32x64/4": 5, "16x64/4": 6, "16x128/2 pair": 7, "by size": 0}
+FORMS = {"128x128": 1, "64x128 (32x64 in 32 bits)": 2, "64x64": 3, "64x64/2": 4, "32x64/4": 5, "16x64/4": 6, "16x128/2 pair": 7, "32x128/2": 8, "by size": 0}
 
 
 @pytest.fixture(scope="module")
@@ -31,20 +31,22 @@ def close(got, ref, K):
     return torch.allclose(got.double().cpu(), ref, atol=K ** 0.5 * 2e-6, rtol=2e-5)
 
 
+@pytest.mark.parametrize("exact", [False, True])
 @pytest.mark.parametrize("form", FORMS)
 @pytest.mark.parametrize("M,N,K", [(3, 4, 8), (17, 63, 72), (65, 129, 128), (130, 196, 1000), (129, 64, 64), (256, 260, 192)])
-def test_tiles_and_ends(dev, use_form, form, M, N, K):
+def test_tiles_and_ends(dev, use_form, form, M, N, K, exact):
     from vllm_i64_amd import ops_dense as D
     use_form(form)
     g = torch.Generator().manual_seed(M + N + K)
     a, w = torch.randn(M, K + 8, generator=g), bf16(torch.randn(2 * N, K, generator=g) / math.sqrt(K))
     b = torch.randn(N, generator=g)
     e = torch.randn(M, N + 3, generator=g)
-    A = bf16(a[:, 4:4 + K]).double()
+    rounded = (lambda t: t.double()) if exact else (lambda t: bf16(t).double())
+    A = rounded(a[:, 4:4 + K])
     ref, up = A @ w[:N].double().T, A @ w[N:].double().T
     ad, wd = a.to(dev), w.to(dev)
     out = torch.full((M, N + 5), 7.0, device=dev)
-    kw = dict(n=N, k=K, a_off=4, lda=K + 8)
+    kw = dict(n=N, k=K, a_off=4, lda=K + 8, exact=exact)
     D.linear(ad, wd, out, c_off=2, ldc=N + 5, **kw)
     assert close(out[:, 2:2 + N], ref, K) and bool((out[:, :2] == 7).all()) and bool((out[:, 2 + N:] == 7).all())
     out = torch.empty(M, N, device=dev)
@@ -59,15 +61,17 @@ def test_tiles_and_ends(dev, use_form, form, M, N, K):
         D.linear(ad, wd, out, in_norm_w=nw.to(dev), in_eps=1e-6, **kw)
         x = a[:, 4:4 + K]
         f = 1.0 / torch.sqrt(x.double().pow(2).mean(-1, keepdim=True) + 1e-6)
-        assert close(out, (bf16(x * nw).double() @ w[:N].double().T) * f, K)
+        assert close(out, (rounded(x * nw) @ w[:N].double().T) * f, K)
 
 
+@pytest.mark.parametrize("exact", [False, True])
 @pytest.mark.parametrize("form", FORMS)
 @pytest.mark.parametrize("counts", [[5, 0, 70, 1], [0, 0, 0, 129], [64, 16, 128, 0], [1, 1, 1, 1]])
-def test_rows_dealt_to_experts(dev, use_form, form, counts):
+def test_rows_dealt_to_experts(dev, use_form, form, counts, exact):
     """Gathered rows into a gate / up pair with a factor per row, and rows as they lie; empty batches; a larger bound than there are rows."""
     from vllm_i64_amd import ops_dense as D
     use_form(form)
+    rounded = (lambda t: t.double()) if exact else (lambda t: bf16(t).double())
     E, N, K, n = len(counts), 72, 136, 150
     g = torch.Generator().manual_seed(sum(counts))
     off = torch.tensor([0] + counts).cumsum(0).to(torch.int32)
@@ -77,16 +81,16 @@ def test_rows_dealt_to_experts(dev, use_form, form, counts):
     w = bf16(torch.randn(E, 2 * N, K, generator=g) / math.sqrt(K))
     out = torch.full((R + 3, N), 7.0, device=dev)
     D.linear(h.to(dev), w.to(dev), out, m=max(counts), n=N, k=K, a_rows=rows.to(dev), batch=E, w_batch=2 * N * K, group_off=off.to(dev), row_scale=s.to(dev),
-             epilogue=D.EPI_CLAMP_GLU, act_a=1.702, act_b=7.0)
-    A = bf16(h).double()[rows[:R].long()]
+             epilogue=D.EPI_CLAMP_GLU, act_a=1.702, act_b=7.0, exact=exact)
+    A = rounded(h)[rows[:R].long()]
     e_of = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
     z = torch.einsum("rk,rnk->rn", A, w.double()[e_of]) * s[:, None].double()
     u, v = z[:, :N].clamp(max=7.0), z[:, N:].clamp(-7.0, 7.0)
     assert torch.allclose(out[:R].double().cpu(), u * torch.sigmoid(1.702 * u) * (v + 1), atol=1e-4, rtol=1e-4) and bool((out[R:] == 7).all())
     wd = bf16(torch.randn(E, K, N, generator=g) / math.sqrt(N))
     down = torch.full((R + 3, K), 7.0, device=dev)
-    D.linear(out[:R], wd.to(dev), down, m=max(counts), n=K, k=N, batch=E, w_batch=K * N, group_off=off.to(dev))
-    ref = torch.einsum("rn,rkn->rk", bf16(out[:R].cpu()).double(), wd.double()[e_of])
+    D.linear(out[:R], wd.to(dev), down, m=max(counts), n=K, k=N, batch=E, w_batch=K * N, group_off=off.to(dev), exact=exact)
+    ref = torch.einsum("rn,rkn->rk", rounded(out[:R].cpu()), wd.double()[e_of])
     assert close(down[:R], ref, N) and bool((down[R:] == 7).all())
 
 

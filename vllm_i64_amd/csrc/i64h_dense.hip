@@ -3,8 +3,8 @@
 //                          bf16 while staged) or v_mfma_f32_16x16x4_f32 (W widened while staged: true 32-bit); batched over
 //                          blockIdx.z (per-head weights on column blocks of wider matrices); epilogues: gelu_tanh(gate) * up
 //                          on two accumulators, * sigmoid(E), logit soft cap and others; an RMS norm of its input on the way.  The form
-//                          of true 32-bit products and of operands that 16-byte loads cannot read; every other launch of more than a
-//                          few rows is linear_block_kernel's (i64h_linear_block.hip)
+//                          of operands that 16-byte loads cannot read; every other launch of more than a few rows is
+//                          linear_block_kernel's (i64h_linear_block.hip)
 //   linear_skinny_kernel : the same product for at most I64H_SKINNY_ROWS rows (decode steps): the rows sit in LDS as bf16, every
 //                          wave streams four weight rows at a time with 16-byte loads and reduces over its lanes
 //   linear_rows16_kernel : at most 16 rows of a small product: 16 output columns per workgroup, the k steps dealt to its eight waves, every
@@ -834,7 +834,7 @@ int i64h_linear_run(const i64h_linear* dp, void* stream) {
         I64H_CHECK_LAUNCH();
         return 0;
     }
-    if (g_block && !d.exact && vecA && vecW && dn_linear_block(d, g_form, s)) {
+    if (g_block && vecA && vecW && dn_linear_block(d, g_form, s)) {
         I64H_CHECK_LAUNCH();
         return 0;
     }

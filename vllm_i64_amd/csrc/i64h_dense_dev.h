@@ -63,7 +63,7 @@ __device__ __forceinline__ float dn_epilogue(const i64h_linear& p, float acc, fl
     return acc;
 }
 
-// the matrix-core tile form of i64h_linear_run (i64h_linear_block.hip): bf16 products, operands readable 16 bytes at a time.
+// the matrix-core tile forms of i64h_linear_run (i64h_linear_block.hip): operands readable 16 bytes at a time.
 // form: -1 chosen by size, else the number of a tile form (tests, measurements).  False: the launch does not fit this form.
 bool dn_linear_block(const i64h_linear& d, int form, hipStream_t s);
 

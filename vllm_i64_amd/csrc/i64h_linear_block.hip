@@ -1,4 +1,4 @@
-// C = epilogue(A W^T) on v_mfma_f32_16x16x32_bf16, A fp32 (rounded to bf16 while it is staged), W bf16 [N, K]: BM x BN tiles staged
+// C = epilogue(A W^T), A fp32, W bf16 [N, K], on v_mfma_f32_16x16x32_bf16 (A rounded to bf16 while it is staged) or with true 32-bit products: BM x BN tiles staged
 // through LDS, four waves a tile and KG groups of four waves that share a tile's k steps.
 //
 // What bounds it.  Large launches: the step from memory to LDS - A is read as 32-bit values and rounded on the way, so a 128 x 128 tile moves
@@ -14,6 +14,7 @@
 // 16-byte loads through a buffer descriptor: a 32-bit offset per lane, the step's offset in a scalar register, and offsets past the end read
 // as zeros - a ragged end needs no branch and nothing is done to the registers behind the load
 typedef uint32_t dn_v4u __attribute__((ext_vector_type(4)));
+typedef uint32_t dn_v2u __attribute__((ext_vector_type(2)));
 constexpr uint32_t DN_BUF_END = 0xfffffff0u;       // from here on: zeros
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t dn_buffer(const void* base) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)DN_BUF_END, 0x00020000);
@@ -22,15 +23,17 @@ __device__ __forceinline__ dn_v4u dn_load16(__amdgpu_buffer_rsrc_t r, uint32_t l
     return __builtin_amdgcn_raw_buffer_load_b128(r, lane_bytes, step_bytes, 0);
 }
 
-template <int EPI, int BM, int BN, int KG>
+// EX: 32-bit products on v_mfma_f32_16x16x4_f32, W widened while it is staged.  A staged row is 128 bytes either way: steps of 64 or of 32 values.
+template <int EPI, int BM, int BN, int KG, bool EX>
 __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kernel(const i64h_linear p, const int n_tiles, const int m_tiles, const int vecC) {
     constexpr bool DUAL = dn_dual(EPI), INN = EPI == I64H_EPI_IN_NORM;
-    constexpr int BK = 64, NWM = BM >= 64 ? 2 : 1, NWN = 4 / NWM;      // waves of a group over rows and columns
+    constexpr int BK = EX ? 32 : 64, CH = BK / 8;      // values of a step, of a 16-byte chunk
+    constexpr int NWM = BM >= 64 ? 2 : 1, NWN = 4 / NWM;      // waves of a group over rows and columns
     constexpr int WM = BM / NWM, WN = BN / NWN, FM = WM / 16, FN = WN / 16;
     static_assert(FM > 0 && FN > (DUAL ? 1 : 0), "");
     constexpr int PA = (BM + 31) / 32, PB = BN / 32;       // staging passes: 32 rows of 64 values, 8 values a thread
     constexpr int COLS = DUAL ? BN / 2 : BN;               // output columns of a tile
-    constexpr int PLANE = (BM + BN) * BK;
+    constexpr int PLANE = (BM + BN) * 64;                  // (in 16-bit units)
     // [buffer][group][A rows, W rows]; (variables of their own, so that the writes of one step may be scheduled between the reads of the other)
     __shared__ __attribute__((aligned(16))) uint16_t s0[KG * PLANE], s1[KG * PLANE];
     __shared__ float sRow[INN ? KG : 1][INN ? BM : 1];
@@ -89,14 +92,14 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
 #pragma unroll
     for (int i = 0; i < PA; ++i) {
         const int r = min(i * 32 + lr, M - 1);
-        oa[i] = (uint32_t)((p.a_rows ? p.a_rows[m0 + r] : r) * p.lda + lc * 8) * 4u;
+        oa[i] = (uint32_t)((p.a_rows ? p.a_rows[m0 + r] : r) * p.lda + lc * CH) * 4u;
     }
 #pragma unroll
     for (int i = 0; i < PB; ++i) {
         const int r = i * 32 + lr;
         // gate and up rows of the same columns go to the same wave: its first half of fragments, its second half
         const int c = DUAL ? (r / WN) * (WN / 2) + r % (WN / 2) : r;
-        ow[i] = (uint32_t)((int64_t)(min(n0 + c, N - 1) + (DUAL && r % WN >= WN / 2 ? N : 0)) * K + lc * 8) * 2u;
+        ow[i] = (uint32_t)((int64_t)(min(n0 + c, N - 1) + (DUAL && r % WN >= WN / 2 ? N : 0)) * K + lc * CH) * 2u;
     }
     dn_v4u ra[2][PA][2], rb[2][PB], rn[2][2];      // two steps on their way
     float ssq[PA];
@@ -107,18 +110,21 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
     auto gload = [&](int kt, auto set) {
         constexpr int S = decltype(set)::value;
         const int k0 = k_base + kt * BK;
-        const uint32_t past = k0 + lc * 8 >= k_end ? DN_BUF_END : 0u;      // (K is a multiple of eight)
+        const uint32_t past = k0 + lc * CH >= k_end ? DN_BUF_END : 0u;      // (K is a multiple of eight)
 #pragma unroll
         for (int i = 0; i < PA; ++i) {
             ra[S][i][0] = dn_load16(bufA, oa[i] | past, k0 * 4);
-            ra[S][i][1] = dn_load16(bufA, (oa[i] + 16) | past, k0 * 4);
+            if (!EX) ra[S][i][1] = dn_load16(bufA, (oa[i] + 16) | past, k0 * 4);
         }
 #pragma unroll
-        for (int i = 0; i < PB; ++i) rb[S][i] = dn_load16(bufW, ow[i] | past, k0 * 2);
+        for (int i = 0; i < PB; ++i) {
+            if (EX) rb[S][i].xy = __builtin_bit_cast(dn_v2u, __builtin_amdgcn_raw_buffer_load_b64(bufW, ow[i] | past, k0 * 2, 0));
+            else rb[S][i] = dn_load16(bufW, ow[i] | past, k0 * 2);
+        }
         if (INN) {
-            const float* nw = p.in_norm_w + (past ? 0 : k0 + lc * 8);
+            const float* nw = p.in_norm_w + (past ? 0 : k0 + lc * CH);
             rn[S][0] = *(const dn_v4u*)nw;
-            rn[S][1] = *(const dn_v4u*)(nw + 4);
+            if (!EX) rn[S][1] = *(const dn_v4u*)(nw + 4);
         }
     };
     // 128-byte rows; a row's chunks are stored exclusive-or its number, so that the 16 rows of a fragment read lie in different banks
@@ -127,24 +133,26 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
         uint16_t* sm = (S ? s1 : s0) + grp * PLANE;
 #pragma unroll
         for (int i = 0; i < PA; ++i) {
-            dn_v4f u = __builtin_bit_cast(dn_v4f, ra[S][i][0]), v = __builtin_bit_cast(dn_v4f, ra[S][i][1]);
+            dn_v4f u = __builtin_bit_cast(dn_v4f, ra[S][i][0]), v = __builtin_bit_cast(dn_v4f, ra[S][i][EX ? 0 : 1]);
             if (INN) {      // the row's squares as they come, the norm's weights on what is staged
-                const dn_v4f nu = __builtin_bit_cast(dn_v4f, rn[S][0]), nv = __builtin_bit_cast(dn_v4f, rn[S][1]);
+                const dn_v4f nu = __builtin_bit_cast(dn_v4f, rn[S][0]), nv = __builtin_bit_cast(dn_v4f, rn[S][EX ? 0 : 1]);
 #pragma unroll
                 for (int g = 0; g < 4; ++g) ssq[i] = fmaf(u[g], u[g], ssq[i]);
+                if (!EX)
 #pragma unroll
-                for (int g = 0; g < 4; ++g) ssq[i] = fmaf(v[g], v[g], ssq[i]);
+                    for (int g = 0; g < 4; ++g) ssq[i] = fmaf(v[g], v[g], ssq[i]);
 #pragma unroll
                 for (int g = 0; g < 4; ++g) u[g] *= nu[g], v[g] *= nv[g];
             }
             const int r = i * 32 + lr;
-            if (BM >= 32 || lr < BM)
-                *(dn_v4u*)&sm[r * BK + ((lc ^ (r & 7)) << 3)] = dn_v4u{dn_bf16_pair(u[0], u[1]), dn_bf16_pair(u[2], u[3]), dn_bf16_pair(v[0], v[1]), dn_bf16_pair(v[2], v[3])};
+            const dn_v4u w = EX ? __builtin_bit_cast(dn_v4u, u) : dn_v4u{dn_bf16_pair(u[0], u[1]), dn_bf16_pair(u[2], u[3]), dn_bf16_pair(v[0], v[1]), dn_bf16_pair(v[2], v[3])};
+            if (BM >= 32 || lr < BM) *(dn_v4u*)&sm[r * 64 + ((lc ^ (r & 7)) << 3)] = w;
         }
 #pragma unroll
         for (int i = 0; i < PB; ++i) {
             const int r = i * 32 + lr;
-            *(dn_v4u*)&sm[(BM + r) * BK + ((lc ^ (r & 7)) << 3)] = rb[S][i];
+            const dn_v4u x = rb[S][i];
+            *(dn_v4u*)&sm[(BM + r) * 64 + ((lc ^ (r & 7)) << 3)] = EX ? dn_v4u{x[0] << 16, x[0] & 0xffff0000u, x[1] << 16, x[1] & 0xffff0000u} : x;
         }
     };
     dn_v4f acc[FM][FN];
@@ -159,20 +167,28 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
             const int ch = ((kk * 4 + fk) ^ (fr & 7)) << 3;
-            dn_v8bf a[FM], w[FN];
+            dn_v4u a[FM], w[FN];
 #pragma unroll
-            for (int i = 0; i < FM; ++i) a[i] = *(const dn_v8bf*)&sm[(wm * WM + i * 16 + fr) * BK + ch];
+            for (int i = 0; i < FM; ++i) a[i] = *(const dn_v4u*)&sm[(wm * WM + i * 16 + fr) * 64 + ch];
 #pragma unroll
-            for (int j = 0; j < FN; ++j) w[j] = *(const dn_v8bf*)&sm[(BM + wn * WN + j * 16 + fr) * BK + ch];
+            for (int j = 0; j < FN; ++j) w[j] = *(const dn_v4u*)&sm[(BM + wn * WN + j * 16 + fr) * 64 + ch];
 #pragma unroll
             for (int i = 0; i < FM; ++i)
 #pragma unroll
-                for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j], a[i], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < FN; ++j) {
+                    if constexpr (EX) {      // (a lane's four neighbouring k go to four products: the same permutation on both sides)
+                        const dn_v4f wf = __builtin_bit_cast(dn_v4f, w[j]), af = __builtin_bit_cast(dn_v4f, a[i]);
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[g], af[g], acc[i][j], 0, 0, 0);
+                    } else {
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_v8bf, w[j]), __builtin_bit_cast(dn_v8bf, a[i]), acc[i][j], 0, 0, 0);
+                    }
+                }
         }
     };
     // the next tile's writes and the loads behind it between the matrix instructions; small tiles are faster as the compiler orders them
     auto interleave = [&]() {
-        if (BN < 128 || BM < 64) return;
+        if (EX || BN < 128 || BM < 64) return;
         constexpr int MF = 2 * FM * FN, DR = 2 * (FM + FN), DW = PA + PB, VM = 2 * PA + PB;
         __builtin_amdgcn_sched_group_barrier(0x100, DR / 2, 0);
 #pragma unroll
@@ -180,7 +196,7 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
             __builtin_amdgcn_sched_group_barrier(0x008, MF / 8, 0);
             if (g < 4) __builtin_amdgcn_sched_group_barrier(0x100, DR / 8, 0);
             __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
-            __builtin_amdgcn_sched_group_barrier(0x200, DW / 8 > 0 ? DW / 8 : 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x200, (DW + 7) / 8, 0);
             __builtin_amdgcn_sched_group_barrier(0x020, (VM + 7) / 8, 0);
         }
     };
@@ -269,7 +285,7 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
 }
 
 enum { PLAIN = 1, PAIR = 2 };      // the epilogues that a form is built for: all but the gate / up pairs, those, both
-template <int BM, int BN, int KG, int FOR = PLAIN | PAIR>
+template <int BM, int BN, int KG, int FOR = PLAIN | PAIR, bool EX = false>
 static void launch(const i64h_linear& d, hipStream_t s) {
     const int cols = dn_dual(d.epilogue) ? BN / 2 : BN;
     const int nt = (d.N + cols - 1) / cols;
@@ -280,12 +296,12 @@ static void launch(const i64h_linear& d, hipStream_t s) {
     }
     const int vecC = (uintptr_t)d.C % 16 == 0 && d.ldc % 4 == 0 && d.c_batch % 4 == 0;
     const dim3 grid((unsigned)(mt * nt), 1, d.group_off ? 1u : (unsigned)d.batch);
-#define DN_BLOCK(E) case E: if constexpr (FOR & (dn_dual(E) ? PAIR : PLAIN)) hipLaunchKernelGGL((linear_block_kernel<E, BM, BN, KG>), grid, dim3(256 * KG), 0, s, d, nt, (int)mt, vecC); break;
+#define DN_BLOCK(E) case E: if constexpr (FOR & (dn_dual(E) ? PAIR : PLAIN)) hipLaunchKernelGGL((linear_block_kernel<E, BM, BN, KG, EX>), grid, dim3(256 * KG), 0, s, d, nt, (int)mt, vecC); break;
     switch (d.epilogue) {
         DN_BLOCK(I64H_EPI_GELU_MUL) DN_BLOCK(I64H_EPI_SILU_MUL) DN_BLOCK(I64H_EPI_CLAMP_GLU) DN_BLOCK(I64H_EPI_MUL_SIGMOID) DN_BLOCK(I64H_EPI_SOFTCAP)
         DN_BLOCK(I64H_EPI_GELU_ERF) DN_BLOCK(I64H_EPI_XIELU) DN_BLOCK(I64H_EPI_RELU_SQ) DN_BLOCK(I64H_EPI_ADD) DN_BLOCK(I64H_EPI_DECAY) DN_BLOCK(I64H_EPI_ROW_SIGMOID)
         DN_BLOCK(I64H_EPI_IN_NORM) DN_BLOCK(I64H_EPI_SCALE)
-        default: if constexpr (FOR & PLAIN) hipLaunchKernelGGL((linear_block_kernel<I64H_EPI_STORE, BM, BN, KG>), grid, dim3(256 * KG), 0, s, d, nt, (int)mt, vecC); break;
+        default: if constexpr (FOR & PLAIN) hipLaunchKernelGGL((linear_block_kernel<I64H_EPI_STORE, BM, BN, KG, EX>), grid, dim3(256 * KG), 0, s, d, nt, (int)mt, vecC); break;
     }
 #undef DN_BLOCK
 }
@@ -304,6 +320,36 @@ bool dn_linear_block(const i64h_linear& d, int form, hipStream_t s) {
     const int64_t span = (d.a_rows ? d.a_height : 128) * d.lda * 4;
     if ((d.a_rows && d.a_height <= 0) || span >= (int64_t)DN_BUF_END - 64 || (int64_t)d.N * (dual ? 4 : 2) * d.K >= (int64_t)DN_BUF_END - 64) return false;
     if (tiles(d, 16, 64) > 0x7fffffff) return false;
+    // rows that share a batch's weights: taller tiles would only repeat the last one
+    const int64_t tall = d.group_off && d.rows_total > 0 ? (d.rows_total + d.batch - 1) / d.batch : d.M;
+    if (d.exact) {
+        // Bound by the matrix instructions, a sixteenth of the bf16 rate: what counts is that every CU works, then that few values are staged per
+        // product.  Microseconds in replayed graphs, in front the 64 x 64 tile kernel with 32-wide steps:
+        //   rows x columns x k                 before   64x64  64x64/2  32x64  32x64/4  16x64/4  16x128/2 (a gate / up pair)
+        //   4096 x 1024 x 1024                    83      69       71     74       98       96
+        //    376 x 5760 x 1024                    66      54       54     49       62       56
+        //    376 x 1024 x 2752                    99      58       49     40       30       33
+        //     40 x 1024 x 1024                    35      23       20     16       14       10
+        //      3 x 32000 x 1024                   54      39       36     25       26       16
+        //    376 x 2752 x 1024, pair              91      54       55                                  59
+        //  8 x 10 x 896 x 1024, pair              66      26       22                                  17
+        if (form < 0) {
+            if (dual) form = tiles(d, 16, 128) <= 256 ? 6 : (d.K >= 512 && tiles(d, 64, 64) <= 256 ? 3 : 2);
+            else if (tall <= 16 || tiles(d, 16, 64) <= 256) form = 5;
+            else if (tiles(d, 32, 64) <= 256) form = 4;
+            else if (d.K >= 512 && tiles(d, 64, 64) <= 256) form = 3;
+            else form = tiles(d, 32, 64) < 1500 ? 1 : 2;
+        }
+        switch (form) {
+            case 1: if (!dual) { launch<32, 64, 1, PLAIN, true>(d, s); break; } [[fallthrough]];
+            case 3: launch<64, 64, 2, PLAIN | PAIR, true>(d, s); break;
+            case 4: if (!dual) { launch<32, 64, 4, PLAIN, true>(d, s); break; } [[fallthrough]];
+            case 5: if (!dual) { launch<16, 64, 4, PLAIN, true>(d, s); break; } [[fallthrough]];
+            case 6: if (dual) { launch<16, 128, 2, PAIR, true>(d, s); break; } [[fallthrough]];
+            default: launch<64, 64, 1, PLAIN | PAIR, true>(d, s); break;
+        }
+        return true;
+    }
     if (form < 0) {
         // Large tiles as long as (nearly) every CU gets one: their operands are read least often.  Below that, a tile's k steps follow each
         // other at the latency of a load and what counts is how few of them a workgroup has and how many CUs work: four groups a tile
@@ -316,17 +362,21 @@ bool dn_linear_block(const i64h_linear& d, int form, hipStream_t s) {
         //    512 x 1024 x 1024         15.7    12.5     9.4      8.5      7.3     10.5
         //     64 x 11392 x 2048                        16.3     13.5     18.6     21.1
         //     64 x 2048 x 2048                         15.1     12.3      9.6      8.3
+        // Few rows under weights that take longer than everything else: 32 x 128 tiles, two groups (8 experts of 16 rows x 3584 x 2048: 24.4 us, in 128
+        // x 128 tiles 33, in 64 x 64 30; 7 x 32000 x 1024 12.7, 64x64 13.4).
         const bool longer = d.K > 128;
-        if (longer && tiles(d, 128, 128) >= 200) form = 0;
-        else if (longer && tiles(d, 64, 128) >= 250) form = 1;
+        if (longer && tall > 64 && tiles(d, 128, 128) >= 200) form = 0;
+        else if (longer && tall > 32 && tiles(d, 64, 128) >= 250) form = 1;
         else if (dual ? tiles(d, 16, 128) <= 256 : tiles(d, 16, 64) <= 256) form = dual ? 6 : 5;
         else if (!dual && d.K >= 512 && tiles(d, 32, 64) <= 256) form = 4;
+        else if (d.K >= 512 && tall <= 32) form = 7;
         else if (d.K >= 512 && tiles(d, 64, 64) <= 256) form = 3;
         else form = 2;
     }
     switch (form) {
         case 0: launch<128, 128, 1>(d, s); break;
         case 1: launch<64, 128, 1>(d, s); break;
+        case 7: launch<32, 128, 2>(d, s); break;
         case 3: launch<64, 64, 2>(d, s); break;
         case 4: if (!dual) { launch<32, 64, 4, PLAIN>(d, s); break; } [[fallthrough]];
         case 5: if (!dual) { launch<16, 64, 4, PLAIN>(d, s); break; } [[fallthrough]];
