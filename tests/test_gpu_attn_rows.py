@@ -1,4 +1,4 @@
-"""The matrix-core attention of prompt portions against 64-bit attention over the same bf16 rows: every number of heads that shares a workgroup, key widths
+"""The matrix-core attention of prompt portions (bf16 and 32-bit caches) against 64-bit attention over the same rows: every number of heads that shares a workgroup, key widths
 that are no multiple of a step, pages of any size, tiles that hold rows of several sequences, cached tokens in front, windows, kept
 first positions, sinks, soft cap."""
 import math
@@ -41,15 +41,16 @@ def reference(q, keys, values, pos, scale, window, keep, cap, sink):
 LENS = [([1, 15, 16, 17, 40], [0, 3, 0, 31, 0]), ([70], [0]), ([33, 2], [64, 5])]
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("lens,past", LENS)
 @pytest.mark.parametrize("H,G,dim,vdim", [(4, 1, 64, 64), (2, 1, 32, 32), (3, 1, 64, 16), (8, 2, 24, 48), (6, 2, 128, 128), (12, 3, 8, 64)])
 @pytest.mark.parametrize("block,window,keep,cap", [(16, 0, 0, 0.0), (16, 20, 3, 0.0), (6, 33, 40, 0.0), (16, 0, 0, 2.0)])
-def test_keys_and_values(dev, lens, past, H, G, dim, vdim, block, window, keep, cap):
+def test_keys_and_values(dev, lens, past, H, G, dim, vdim, block, window, keep, cap, dtype):
     from vllm_i64_amd import ops_dense as D
     g = torch.Generator().manual_seed(H + dim + window)
     bt, pos, slots, blocks = pages(lens, past, block, g)
     n, w = int(pos.numel()), vdim + dim
-    cache = torch.randn(blocks, block, G * w, generator=g).bfloat16()
+    cache = torch.randn(blocks, block, G * w, generator=g).to(dtype)
     q = torch.randn(n, H, w, generator=g)
     q[:, :, :vdim] = 0
     sink = torch.randn(H, generator=g)
@@ -63,20 +64,22 @@ def test_keys_and_values(dev, lens, past, H, G, dim, vdim, block, window, keep, 
         rows = cache[bt[i].long()[j // block], j % block].view(m + p, G, w).repeat_interleave(H // G, 1).transpose(0, 1)
         ref = reference(q[at:at + m, :, vdim:], rows[..., vdim:], rows[..., :vdim], pos[at:at + m], 1.0, window, keep, cap, sink)
         got = out[at:at + m].view(m, H, vdim).double().cpu()
-        # two bf16 terms of query and weight: 2^-16 relative each, scores of up to sqrt(dim) * 4
-        assert torch.allclose(got, ref, atol=2e-3, rtol=1e-3), float((got - ref).abs().max())
+        # two bf16 terms of query and weight: 2^-16 relative each, scores of up to sqrt(dim) * 4; 32-bit products: 2^-24 times the score
+        tol = 1e-3 if dtype == torch.bfloat16 else 2e-5
+        assert torch.allclose(got, ref, atol=2 * tol, rtol=tol), float((got - ref).abs().max())
         at += m
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("lens,past", LENS)
 @pytest.mark.parametrize("H,r,e", [(4, 256, 32), (5, 256, 64), (8, 32, 8), (16, 128, 0), (2, 64, 64), (4, 144, 24)])
 @pytest.mark.parametrize("window", [0, 25])
-def test_latent_rows(dev, lens, past, H, r, e, window):
+def test_latent_rows(dev, lens, past, H, r, e, window, dtype):
     from vllm_i64_amd import ops_dense as D
     g = torch.Generator().manual_seed(H + r + e)
     bt, pos, slots, blocks = pages(lens, past, 16, g)
     n = int(pos.numel())
-    cache = torch.randn(blocks, 16, r + e, generator=g).bfloat16()
+    cache = torch.randn(blocks, 16, r + e, generator=g).to(dtype)
     q = torch.randn(n, H, r + e, generator=g)
     sink = torch.randn(H, generator=g)
     out = torch.full((n * H * r,), 7.0, device=dev)
@@ -87,5 +90,6 @@ def test_latent_rows(dev, lens, past, H, r, e, window):
         rows = cache[bt[i].long()[j // 16], j % 16].expand(H, -1, -1)
         ref = reference(q[at:at + m], rows, rows[..., :r], pos[at:at + m], 0.1, window, 0, 0.0, sink)
         got = out.view(n, H, r)[at:at + m].double().cpu()
-        assert torch.allclose(got, ref, atol=5e-4, rtol=5e-4), float((got - ref).abs().max())
+        tol = 5e-4 if dtype == torch.bfloat16 else 1e-5
+        assert torch.allclose(got, ref, atol=tol, rtol=tol), float((got - ref).abs().max())
         at += m

@@ -5,7 +5,8 @@
 // q'_latent . latent_j + q_rot . key_rot_j and all heads read the same cached rows.
 //   latent_prep_kernel     : RMS norm of the latent, rotation of the shared key part and of every head's rotated query part,
 //                            cache write - one workgroup per token
-//   latent_attn_rows_kernel: bf16 caches of aligned widths, portions of prompts - four waves of 16 rows that share 32 keys at a time through LDS
+//   latent_attn_rows_kernel: bf16 caches of aligned widths, portions of prompts - four waves of 16 rows that share 32 keys at a time through LDS;
+//                            latent_attn_rows_f32_kernel: the same for 32-bit caches, 32-bit products
 //   latent_attn_mfma_decode_kernel (latent_attn_mfma_kernel): rows that are one per sequence - a token's heads, 16 query vectors per wave;
 //                            both on the bf16 matrix cores, see below
 //   latent_attn_row_kernel : any width and cache type, true fp32 products: one wave per (token, head): 64 keys at a time, one key per lane for the scores (fp32 dot over the
@@ -815,6 +816,212 @@ __global__ __launch_bounds__(256, 2) void latent_attn_rows_kernel(const i64h_lat
         }
 }
 
+// The same for caches of 32-bit rows, with 32-bit products: keys and transposed values once in LDS (twice would be a workgroup per CU), the next tile
+// waiting in registers.  Bound by the matrix instructions at their 32-bit rate (272 a wave and 32 keys of 256 + 32 values).  16 heads over one
+// cached row of 288, prompts of 300, 75 and 1 tokens: 315 -> 93 us against latent_attn_row_kernel, which reads every key again for each query (the
+// widest rows with a SIMD's registers to themselves: 109 us at two waves, whose spills cost more).
+#define LT_FLD 36  // values per row of the transposed tile (32 keys + 4)
+template <int KC, int NB, bool EXTRA>
+__global__ __launch_bounds__(256, NB > 8 ? 1 : 2) void latent_attn_rows_f32_kernel(const i64h_latent_attn_args p, const int hw) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, n = lane & 15, kg = lane >> 4;
+    const int r = p.kv_rank, D = r + p.rot_dim, H = p.heads, bs = p.block_size, win = p.window, koff = p.key_off & ~15;
+    const int keep = p.chunk <= 0 && win > 0 ? p.keep_first : 0;
+    const int kld = D - koff + 4;             // values per key row in LDS: the columns that take part in the scores
+    float* const K = (float*)smem;            // keys [32][kld], values transposed [r][LT_FLD]
+    float* const V = K + 32 * kld;
+    int* const info = (int*)(V + r * LT_FLD);      // [64] positions, [64] slots (-1: no such row)
+    const int G = p.kv_groups > 1 ? p.kv_groups : 1, rep = H / G;
+    const int rstride = p.row_stride > 0 ? p.row_stride : D;
+    const int hgroups = H / hw, rows = 16 * (4 / hw), row_tiles = (int)((p.n + rows - 1) / rows);
+    const int task = blockIdx.x, hg = task % hgroups, rt = row_tiles - 1 - task / hgroups;      // (the longest contexts first)
+    const int head = hg * hw + wid % hw, coff = hg * hw / rep * D, wr = wid / hw * 16;
+    const int64_t row0 = (int64_t)rt * rows;
+    if (tid < rows) {
+        const bool ok = row0 + tid < p.n;
+        info[tid] = ok ? p.positions[row0 + tid] : -1;
+        info[64 + tid] = ok ? p.slot_ids[row0 + tid] : -1;
+    }
+    const int64_t tok = row0 + wr + n;
+    const bool valid = tok < p.n;
+    // the query of row n times scale * log2(e), columns koff + c * 16 + kg * 4 .. + 3; zeros past the end, where the key reads repeat the first columns
+    lt_v4f Q[KC];
+    {
+        const float* q = p.Q + ((valid ? tok : row0) * H + head) * D;
+        const float qs = p.scale * 1.4426950408889634f;
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+            const int d0 = koff + c * 16 + kg * 4;
+            Q[c] = lt_v4f{0, 0, 0, 0};
+            if (valid && d0 < D) Q[c] = *(const lt_v4f*)(q + d0) * qs;
+        }
+    }
+    lt_v4f acc[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[nb] = lt_v4f{0, 0, 0, 0};
+    // (the weight sum of a row is kept in four shares, one per group of keys: the sink belongs to one of them)
+    float m = p.sink ? (p.sink_w ? p.sink_w[head] * 1.4426950408889634f : 0.0f) : -INFINITY, l = p.sink && kg == 0 ? 1.0f : 0.0f;
+    const float capl = p.softcap * 1.4426950408889634f;
+    const float* const cache = (const float*)p.cache + coff;
+    auto first_seen = [&](int pos) { return p.chunk > 0 ? pos / p.chunk * p.chunk : (win > 0 ? max(0, pos - win + 1) : 0); };
+    // staging: this thread's four keys and its (at most three) groups of four columns
+    constexpr int PASS = NB > 8 ? 3 : 2;
+    const int kq = tid & 7, cg = tid >> 3;
+    const int groups = D >> 2;
+    lt_v4f st[PASS][4];
+    int64_t src[4];
+    __syncthreads();
+    int s0 = 0;
+    while (s0 < rows) {
+        const int sl = info[64 + s0];
+        if (sl < 0) {
+            ++s0;
+            continue;
+        }
+        int s1 = s0 + 1;
+        while (s1 < rows && info[64 + s1] == sl) ++s1;
+        int lo = 0x7fffffff, hi = -1;                      // the keys of the run; the same for this wave's rows of it
+        int wlo = 0x7fffffff, whi = -1, wall = 0x7fffffff, wfrom = 0;
+        for (int i = s0; i < s1; ++i) {
+            const int pp = info[i], f = first_seen(max(pp, 0));
+            hi = max(hi, pp), lo = min(lo, f);
+            if (i >= wr && i < wr + 16) wlo = min(wlo, f), whi = max(whi, pp), wall = min(wall, pp), wfrom = max(wfrom, f);
+        }
+        if (wr < s0 || wr + 16 > s1) wall = -1;            // rows of another run: every tile is masked
+        const int pos = wr + n >= s0 && wr + n < s1 ? info[wr + n] : -1, from = first_seen(max(pos, 0));
+        const int32_t* bt = p.block_table + (int64_t)sl * p.max_blocks_per_seq;
+        // tiles of 32 keys: those of the kept first positions that lie in front of the window's first tile, then the window's
+        const int t0 = lo >> 5, kt = min((keep + 31) >> 5, t0), tiles = hi < 0 ? 0 : kt + (hi >> 5) - t0 + 1;
+        auto key_base = [&](int tile) { return (tile < kt ? tile : t0 + tile - kt) * 32; };
+        auto look_up = [&](int tile) {
+            const int j0 = key_base(min(tile, tiles - 1)) + kq * 4;
+            if ((bs & 3) == 0) {      // four neighbours of one page
+                const int f = min(j0, hi), pg = f / bs;
+                const int64_t base = (int64_t)bt[pg] * bs - pg * bs;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) src[i] = (base + min(j0 + i, hi)) * rstride;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int j = min(j0 + i, hi);
+                    src[i] = ((int64_t)bt[j / bs] * bs + j % bs) * rstride;
+                }
+            }
+        };
+        auto request = [&]() {
+#pragma unroll
+            for (int q = 0; q < PASS; ++q)
+                if (cg + 32 * q < groups)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) st[q][i] = *(const lt_v4f*)(cache + src[i] + (cg + 32 * q) * 4);
+        };
+        auto store = [&]() {
+#pragma unroll
+            for (int q = 0; q < PASS; ++q) {
+                const int c0 = (cg + 32 * q) * 4;
+                if (c0 >= D) continue;
+                if (c0 >= koff)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) *(lt_v4f*)&K[(kq * 4 + i) * kld + c0 - koff] = st[q][i];
+                if (c0 < r)      // columns c0 + c of keys 4 kq .. + 3
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) *(lt_v4f*)&V[(c0 + c) * LT_FLD + kq * 4] = lt_v4f{st[q][0][c], st[q][1][c], st[q][2][c], st[q][3][c]};
+            }
+        };
+        if (tiles > 0) {
+            look_up(0);
+            request();
+            look_up(1);
+        }
+        for (int tile = 0; tile < tiles; ++tile) {
+            const int kb = key_base(tile);
+            __syncthreads();      // (the tile before has been read)
+            store();
+            __syncthreads();
+            if (tile + 1 < tiles) {
+                request();
+                look_up(tile + 2);
+            }
+            if (kb <= whi && (kb + 31 >= wlo || kb < keep)) {      // (something that a row of this wave sees)
+                lt_v4f S[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+                for (int c = 0; c < KC; ++c) {
+                    const int d0 = c * 16 + kg * 4;
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) {      // (a lane's four neighbouring columns go to four products)
+                        const lt_v4f kf = *(const lt_v4f*)&K[(16 * b + n) * kld + (d0 < D - koff ? d0 : 0)];
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) S[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[g], Q[c][g], S[b], 0, 0, 0);
+                    }
+                }
+                if (EXTRA) {
+#pragma unroll
+                    for (int b = 0; b < 2; ++b)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            const int j = kb + 16 * b + kg * 4 + g, jc = min(j, hi);
+                            if (p.kscale) S[b][g] *= p.kscale[(int64_t)bt[jc / bs] * bs + jc % bs];
+                            if (capl > 0.0f) S[b][g] = capl * tanhf(S[b][g] / capl);
+                            if (p.bias) S[b][g] += 1.4426950408889634f * p.bias[(int64_t)min(max(pos - j, 0), p.bias_rows - 1) * H + head];
+                        }
+                }
+                if (kb + 31 > wall || kb < wfrom) {
+#pragma unroll
+                    for (int b = 0; b < 2; ++b)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            const int j = kb + 16 * b + kg * 4 + g;
+                            S[b][g] = j <= pos && (j >= from || j < keep) ? S[b][g] : -INFINITY;
+                        }
+                }
+                float mx = fmaxf(fmaxf(fmaxf(S[0][0], S[0][1]), fmaxf(S[0][2], S[0][3])), fmaxf(fmaxf(S[1][0], S[1][1]), fmaxf(S[1][2], S[1][3])));
+                mx = fmaxf(mx, __shfl_xor(mx, 16));
+                mx = fmaxf(mx, __shfl_xor(mx, 32));
+                const float mn = fmaxf(m, mx), ms = mn == -INFINITY ? 0.0f : mn;
+                const float al = exp2f(m - ms);
+                m = mn;
+                float w[2][4], sum = 0.0f;
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        w[b][g] = exp2f(S[b][g] - ms);
+                        sum += w[b][g];
+                    }
+                l = l * al + sum;
+                if (__ballot(al != 1.0f)) {
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) acc[nb][g] *= al;
+                }
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) {
+                        const lt_v4f vf = *(const lt_v4f*)&V[min(nb * 16 + n, r - 1) * LT_FLD + b * 16 + kg * 4];
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[g], w[b][g], acc[nb], 0, 0, 0);
+                    }
+            }
+        }
+        s0 = s1;
+    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (!valid) return;
+    float* o = p.out + (tok * H + head) * r;
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+        if (nb * 16 < r) {
+            const float4 v = make_float4(acc[nb][0] * inv, acc[nb][1] * inv, acc[nb][2] * inv, acc[nb][3] * inv);
+            float* dst = o + nb * 16 + kg * 4;
+            if (((uintptr_t)p.out & 15) == 0) *(float4*)dst = v;
+            else dst[0] = v.x, dst[1] = v.y, dst[2] = v.z, dst[3] = v.w;
+        }
+}
+
 // the shares of a token's keys, merged: one wave per (token, head); lane s holds share s's maximum and weight sum (at most 64
 // shares), then every lane sums its columns over the shares, eight loads in flight at a time
 __global__ __launch_bounds__(64) void latent_attn_merge_kernel(const i64h_latent_attn_args p, const int splits) {
@@ -888,7 +1095,9 @@ int i64h_latent_attn(const i64h_latent_attn_args* dp, void* stream) {
     const int D = d.kv_rank + d.rot_dim;
     const bool mfma_ok = d.cache_dtype == 2 && D % 8 == 0 && d.kv_rank % 16 == 0 && d.kv_rank <= 16 * LT_NB && D <= 32 * LT_KD &&
                          (uintptr_t)d.Q % 16 == 0 && (uintptr_t)d.cache % 16 == 0 && d.row_stride % 8 == 0;
-    I64H_CHECK_ARG(mfma_ok || (d.kv_groups <= 1 && d.row_stride <= 0 && d.chunk <= 0 && !d.kscale && !d.bias),
+    const bool rows_f32 = d.mode == 3 && d.cache_dtype == 0 && D % 4 == 0 && d.kv_rank % 16 == 0 && d.kv_rank <= 256 && D <= 320 && (uintptr_t)d.Q % 16 == 0 &&
+                          (uintptr_t)d.cache % 16 == 0 && d.row_stride % 4 == 0;
+    I64H_CHECK_ARG(mfma_ok || rows_f32 || (d.kv_groups <= 1 && d.row_stride <= 0 && d.chunk <= 0 && !d.kscale && !d.bias),
                    "latent_attn: key heads, chunks, key scales and bias are built for the matrix-core form only");
     I64H_CHECK_ARG(!d.sink_w || d.sink, "latent_attn: sink scores without the sink");
     I64H_CHECK_ARG(d.keep_first >= 0, "latent_attn: %d kept positions", d.keep_first);
@@ -932,6 +1141,27 @@ int i64h_latent_attn(const i64h_latent_attn_args* dp, void* stream) {
             hipLaunchKernelGGL(latent_attn_merge_kernel, dim3((unsigned)tasks, 16), dim3(64), 0, (hipStream_t)stream, d, splits);
             I64H_CHECK_LAUNCH();
         }
+        return 0;
+    }
+    if (rows_f32) {
+        const int G = d.kv_groups > 1 ? d.kv_groups : 1;
+        I64H_CHECK_ARG(d.heads % G == 0, "latent_attn: %d heads over %d key heads", d.heads, G);
+        const int rep = d.heads / G, hw = rep % 4 == 0 ? 4 : (rep % 2 == 0 ? 2 : 1), rows = 16 * (4 / hw);
+        const int64_t wgs = (d.n + rows - 1) / rows * (d.heads / hw);
+        I64H_CHECK_ARG(wgs < (1ll << 31), "latent_attn: too many tiles");
+        const int kcols = D - (d.key_off & ~15), chunks = (kcols + 15) / 16;
+        const size_t bytes = ((size_t)32 * (kcols + 4) + (size_t)d.kv_rank * LT_FLD) * 4 + 128 * 4;
+        const bool extra = d.kscale || d.bias || d.softcap > 0.0f;
+#define LT_ROWS(KC, NB) do { \
+            if (extra) hipLaunchKernelGGL((latent_attn_rows_f32_kernel<KC, NB, true>), dim3((unsigned)wgs), dim3(256), bytes, (hipStream_t)stream, d, hw); \
+            else hipLaunchKernelGGL((latent_attn_rows_f32_kernel<KC, NB, false>), dim3((unsigned)wgs), dim3(256), bytes, (hipStream_t)stream, d, hw); \
+        } while (0)
+        if (chunks <= 4 && d.kv_rank <= 64) LT_ROWS(4, 4);
+        else if (chunks <= 8 && d.kv_rank <= 128) LT_ROWS(8, 8);
+        else if (chunks <= 18) LT_ROWS(18, 16);
+        else LT_ROWS(20, 16);
+#undef LT_ROWS
+        I64H_CHECK_LAUNCH();
         return 0;
     }
     const size_t lds = (size_t)(4 * D + 512) * 4;
