@@ -93,3 +93,48 @@ def test_latent_rows(dev, lens, past, H, r, e, window, dtype):
         tol = 5e-4 if dtype == torch.bfloat16 else 1e-5
         assert torch.allclose(got, ref, atol=tol, rtol=tol), float((got - ref).abs().max())
         at += m
+
+
+@pytest.mark.parametrize("bad", [math.inf, math.nan])
+@pytest.mark.parametrize("H,G,dim,vdim,window,keep", [(4, 1, 32, 64, 0, 0), (2, 1, 32, 32, 9, 2), (3, 1, 32, 256, 0, 0)])
+def test_unseen_values_of_32_bits(dev, H, G, dim, vdim, window, keep, bad):
+    """A key that a row does not see adds nothing to the row, also where its value is no finite number."""
+    from vllm_i64_amd import ops_dense as D
+    lens, past, at_key = [40, 30, 5], [0, 3, 0], [33, 4, 2]
+    g = torch.Generator().manual_seed(H + vdim)
+    bt, pos, slots, blocks = pages(lens, past, 16, g)
+    n, w = int(pos.numel()), vdim + dim
+    cache = torch.randn(blocks, 16, G * w, generator=g)
+    for i, j in enumerate(at_key):
+        cache[bt[i, j // 16], j % 16, i] = bad
+    q = torch.randn(n, H, w, generator=g)
+    q[:, :, :vdim] = 0
+    out = torch.full((n, H * vdim), 7.0, device=dev)
+    D.kattn(q.to(dev), cache.to(dev), None, bt.to(dev), slots.to(dev), pos.to(dev), chunk=0, bias=None, sink=False, heads=H, kv_heads=G, dim=dim, vdim=vdim, out=out, n=n, mode=3,
+            window=window, keep_first=keep)
+    at = 0
+    for i, (m, p) in enumerate(zip(lens, past)):
+        j = torch.arange(m + p)
+        rows = cache[bt[i].long()[j // 16], j % 16].expand(H, -1, -1)
+        values = rows[..., :vdim].clone()
+        values[:, at_key[i], i] = 0.0
+        ref = reference(q[at:at + m, :, vdim:], rows[..., vdim:], values, pos[at:at + m], 1.0, window, keep, 0.0, torch.full((H,), -math.inf))
+        got = out[at:at + m].view(m, H, vdim).double().cpu()
+        d = pos[at:at + m].long() - at_key[i]
+        sees = (d >= 0) & ((d < window) | (at_key[i] < keep)) if window else d >= 0
+        assert bool((~torch.isfinite(got[sees][..., i])).all())
+        ref[sees, :, i] = 0.0
+        got[sees, :, i] = 0.0
+        assert torch.allclose(got, ref, atol=4e-5, rtol=2e-5), float((got - ref).abs().max())
+        at += m
+
+
+def test_options_of_key_heads_stay_refused_over_32_bits(dev):
+    from vllm_i64_amd import _lib
+    from vllm_i64_amd import ops_dense as D
+    f, i = torch.zeros(4096, device=dev), torch.zeros(64, dtype=torch.int32, device=dev)
+    for option in ({"kv_groups": 2}, {"row_stride": 64}, {"chunk": 16}, {"kscale": D.ptr(f)}, {"bias": D.ptr(f), "bias_rows": 4}):
+        d = _lib.LatentAttn(Q=D.ptr(f), cache=D.ptr(f), cache_dtype=0, block_table=D.ptr(i), max_blocks_per_seq=1, block_size=16, slot_ids=D.ptr(i), positions=D.ptr(i), scale=1.0,
+                            out=D.ptr(f), n=1, heads=2, kv_rank=32, rot_dim=0, mode=3, **option)
+        with pytest.raises(_lib.I64HError, match="matrix-core form only"):
+            D.call_dense("i64h_latent_attn", D._ref(d), D._stream())

@@ -20,6 +20,10 @@
 #include "i64h_common.h"
 #include "i64h_dense.h"
 
+// i64h_latent.hip
+bool latent_rows_f32_ok(const i64h_latent_attn_args& d);
+int latent_rows_f32_run(const i64h_latent_attn_args& d, void* stream);
+
 __device__ __forceinline__ float hy_bf16(const void* p, int64_t i) { return __uint_as_float((uint32_t)((const uint16_t*)p)[i] << 16); }
 __device__ __forceinline__ float hy_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
 __device__ __forceinline__ float hy_silu(float x) { return x / (1.0f + expf(-x)); }
@@ -992,6 +996,7 @@ int i64h_kattn(const i64h_kattn_args* dp, void* stream) {
         a.row_stride = d.kv_heads * gs, a.kv_groups = d.kv_heads, a.chunk = d.chunk, a.kscale = d.kscale, a.bias = d.bias, a.bias_rows = d.bias_rows;
         a.sink = d.sink, a.sink_w = d.sink_w, a.softcap = d.softcap;
         a.key_off = d.vdim > 0 ? d.vdim : 0;
+        if (latent_rows_f32_ok(a)) return latent_rows_f32_run(a, stream);
         return i64h_latent_attn(&a, stream);
     }
     const int64_t items = d.n * d.heads;

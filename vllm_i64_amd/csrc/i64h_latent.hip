@@ -6,7 +6,7 @@
 //   latent_prep_kernel     : RMS norm of the latent, rotation of the shared key part and of every head's rotated query part,
 //                            cache write - one workgroup per token
 //   latent_attn_rows_kernel: bf16 caches of aligned widths, portions of prompts - four waves of 16 rows that share 32 keys at a time through LDS;
-//                            latent_attn_rows_f32_kernel: the same for 32-bit caches, 32-bit products
+//                            latent_attn_rows_f32_kernel: the same for 32-bit caches, 32-bit products (latent_row_f32 where a value is no finite number)
 //   latent_attn_mfma_decode_kernel (latent_attn_mfma_kernel): rows that are one per sequence - a token's heads, 16 query vectors per wave;
 //                            both on the bf16 matrix cores, see below
 //   latent_attn_row_kernel : any width and cache type, true fp32 products: one wave per (token, head): 64 keys at a time, one key per lane for the scores (fp32 dot over the
@@ -816,9 +816,52 @@ __global__ __launch_bounds__(256, 2) void latent_attn_rows_kernel(const i64h_lat
         }
 }
 
+// one row and head by one wave, 32-bit cache: a key per lane for the scores, the columns (at most 256) spread over the lanes for the sum
+__device__ __forceinline__ void latent_row_f32(const i64h_latent_attn_args& p, const int64_t t, const int h) {
+    const int lane = threadIdx.x & 63, r = p.kv_rank, D = r + p.rot_dim, bs = p.block_size, win = p.window;
+    const int G = p.kv_groups > 1 ? p.kv_groups : 1, rstride = p.row_stride > 0 ? p.row_stride : D;
+    const float* const cache = (const float*)p.cache + h / (p.heads / G) * D;
+    const float* const q = p.Q + (t * p.heads + h) * D;
+    const int pos = p.positions[t], from = p.chunk > 0 ? pos / p.chunk * p.chunk : (win > 0 ? max(0, pos - win + 1) : 0);
+    const int kept = p.chunk <= 0 && win > 0 ? min(p.keep_first, from) : 0, total = kept + pos - from + 1;
+    const int32_t* const bt = p.block_table + (int64_t)p.slot_ids[t] * p.max_blocks_per_seq;
+    auto key_of = [&](int i) { return i < kept ? i : from + i - kept; };      // the visible keys in order
+    auto row_of = [&](int i) {
+        const int j = key_of(i);
+        return cache + ((int64_t)bt[j / bs] * bs + j % bs) * rstride;
+    };
+    float m = p.sink ? (p.sink_w ? p.sink_w[h] : 0.0f) : -INFINITY, l = p.sink ? 1.0f : 0.0f, acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i0 = 0; i0 < total; i0 += 64) {
+        const int i = min(i0 + lane, total - 1), j = key_of(i);
+        const float* const kr = row_of(i);
+        float s = 0.0f;
+        for (int d = p.key_off; d < D; ++d) s = fmaf(q[d] * p.scale, kr[d], s);
+        if (p.kscale) s *= p.kscale[(int64_t)bt[j / bs] * bs + j % bs];
+        if (p.softcap > 0.0f) s = p.softcap * tanhf(s / p.softcap);
+        if (p.bias) s += p.bias[(int64_t)min(pos - j, p.bias_rows - 1) * p.heads + h];
+        if (i0 + lane >= total) s = -INFINITY;
+        const float mn = fmaxf(m, wave_max(s)), al = expf(m - mn), w = i0 + lane < total ? expf(s - mn) : 0.0f;
+        l = l * al + wave_sum(w);
+        m = mn;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[c] *= al;
+        for (int k = 0; k < min(64, total - i0); ++k) {
+            const float wk = __shfl(w, k);
+            const float* const v = row_of(i0 + k);
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (lane + 64 * c < r) acc[c] = fmaf(wk, v[lane + 64 * c], acc[c]);
+        }
+    }
+    float* const o = p.out + (t * p.heads + h) * r;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        if (lane + 64 * c < r) o[lane + 64 * c] = acc[c] / l;
+}
+
 // The same for caches of 32-bit rows, with 32-bit products: keys and transposed values once in LDS (twice would be a workgroup per CU), the next tile
 // waiting in registers.  Bound by the matrix instructions at their 32-bit rate (272 a wave and 32 keys of 256 + 32 values).  16 heads over one
-// cached row of 288, prompts of 300, 75 and 1 tokens: 315 -> 93 us against latent_attn_row_kernel, which reads every key again for each query (the
+// cached row of 288, prompts of 300, 75 and 1 tokens: 315 -> 96 us against latent_attn_row_kernel, which reads every key again for each query (the
 // widest rows with a SIMD's registers to themselves: 109 us at two waves, whose spills cost more).
 #define LT_FLD 36  // values per row of the transposed tile (32 keys + 4)
 template <int KC, int NB, bool EXTRA>
@@ -827,10 +870,11 @@ __global__ __launch_bounds__(256, NB > 8 ? 1 : 2) void latent_attn_rows_f32_kern
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, n = lane & 15, kg = lane >> 4;
     const int r = p.kv_rank, D = r + p.rot_dim, H = p.heads, bs = p.block_size, win = p.window, koff = p.key_off & ~15;
     const int keep = p.chunk <= 0 && win > 0 ? p.keep_first : 0;
-    const int kld = D - koff + 4;             // values per key row in LDS: the columns that take part in the scores
+    const int kld = D - koff + 4;             // values per key row in LDS: the columns that take part in the scores, and four zeros
     float* const K = (float*)smem;            // keys [32][kld], values transposed [r][LT_FLD]
     float* const V = K + 32 * kld;
     int* const info = (int*)(V + r * LT_FLD);      // [64] positions, [64] slots (-1: no such row)
+    int* const odd = info + 128;                   // a value of a tile that some row sees a part of is no finite number
     const int G = p.kv_groups > 1 ? p.kv_groups : 1, rep = H / G;
     const int rstride = p.row_stride > 0 ? p.row_stride : D;
     const int hgroups = H / hw, rows = 16 * (4 / hw), row_tiles = (int)((p.n + rows - 1) / rows);
@@ -844,7 +888,9 @@ __global__ __launch_bounds__(256, NB > 8 ? 1 : 2) void latent_attn_rows_f32_kern
     }
     const int64_t tok = row0 + wr + n;
     const bool valid = tok < p.n;
-    // the query of row n times scale * log2(e), columns koff + c * 16 + kg * 4 .. + 3; zeros past the end, where the key reads repeat the first columns
+    if (tid < 32) *(lt_v4f*)&K[tid * kld + D - koff] = lt_v4f{0, 0, 0, 0};
+    if (tid == 0) *odd = 0;
+    // the query of row n times scale * log2(e), columns koff + c * 16 + kg * 4 .. + 3; zeros past the end, as in the keys
     lt_v4f Q[KC];
     {
         const float* q = p.Q + ((valid ? tok : row0) * H + head) * D;
@@ -880,14 +926,15 @@ __global__ __launch_bounds__(256, NB > 8 ? 1 : 2) void latent_attn_rows_f32_kern
         }
         int s1 = s0 + 1;
         while (s1 < rows && info[64 + s1] == sl) ++s1;
-        int lo = 0x7fffffff, hi = -1;                      // the keys of the run; the same for this wave's rows of it
+        int lo = 0x7fffffff, hi = -1, all = 0x7fffffff, last = 0;      // the keys of the run; the same for this wave's rows of it
         int wlo = 0x7fffffff, whi = -1, wall = 0x7fffffff, wfrom = 0;
         for (int i = s0; i < s1; ++i) {
             const int pp = info[i], f = first_seen(max(pp, 0));
-            hi = max(hi, pp), lo = min(lo, f);
+            hi = max(hi, pp), lo = min(lo, f), all = min(all, pp), last = max(last, f);
             if (i >= wr && i < wr + 16) wlo = min(wlo, f), whi = max(whi, pp), wall = min(wall, pp), wfrom = max(wfrom, f);
         }
         if (wr < s0 || wr + 16 > s1) wall = -1;            // rows of another run: every tile is masked
+        if (s0 > 0 || s1 < rows) all = -1;
         const int pos = wr + n >= s0 && wr + n < s1 ? info[wr + n] : -1, from = first_seen(max(pos, 0));
         const int32_t* bt = p.block_table + (int64_t)sl * p.max_blocks_per_seq;
         // tiles of 32 keys: those of the kept first positions that lie in front of the window's first tile, then the window's
@@ -915,14 +962,28 @@ __global__ __launch_bounds__(256, NB > 8 ? 1 : 2) void latent_attn_rows_f32_kern
 #pragma unroll
                     for (int i = 0; i < 4; ++i) st[q][i] = *(const lt_v4f*)(cache + src[i] + (cg + 32 * q) * 4);
         };
-        auto store = [&]() {
+        auto store = [&](bool partial) {
 #pragma unroll
             for (int q = 0; q < PASS; ++q) {
                 const int c0 = (cg + 32 * q) * 4;
-                if (c0 >= D) continue;
-                if (c0 >= koff)
+                if (c0 < D && c0 >= koff)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) *(lt_v4f*)&K[(kq * 4 + i) * kld + c0 - koff] = st[q][i];
+            }
+            if (partial) {      // a sum of zeros unless a value is infinite or no number
+                float z = 0.0f;
+#pragma unroll
+                for (int q = 0; q < PASS; ++q)
+                    if ((cg + 32 * q) * 4 < r)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+#pragma unroll
+                            for (int c = 0; c < 4; ++c) z = fmaf(st[q][i][c], 0.0f, z);
+                if (z != 0.0f) *odd = 1;
+            }
+#pragma unroll
+            for (int q = 0; q < PASS; ++q) {
+                const int c0 = (cg + 32 * q) * 4;
                 if (c0 < r)      // columns c0 + c of keys 4 kq .. + 3
 #pragma unroll
                     for (int c = 0; c < 4; ++c) *(lt_v4f*)&V[(c0 + c) * LT_FLD + kq * 4] = lt_v4f{st[q][0][c], st[q][1][c], st[q][2][c], st[q][3][c]};
@@ -936,7 +997,7 @@ __global__ __launch_bounds__(256, NB > 8 ? 1 : 2) void latent_attn_rows_f32_kern
         for (int tile = 0; tile < tiles; ++tile) {
             const int kb = key_base(tile);
             __syncthreads();      // (the tile before has been read)
-            store();
+            store(kb + 31 > all || kb < last);      // (true: a row does not see every key)
             __syncthreads();
             if (tile + 1 < tiles) {
                 request();
@@ -949,7 +1010,7 @@ __global__ __launch_bounds__(256, NB > 8 ? 1 : 2) void latent_attn_rows_f32_kern
                     const int d0 = c * 16 + kg * 4;
 #pragma unroll
                     for (int b = 0; b < 2; ++b) {      // (a lane's four neighbouring columns go to four products)
-                        const lt_v4f kf = *(const lt_v4f*)&K[(16 * b + n) * kld + (d0 < D - koff ? d0 : 0)];
+                        const lt_v4f kf = *(const lt_v4f*)&K[(16 * b + n) * kld + min(d0, D - koff)];
 #pragma unroll
                         for (int g = 0; g < 4; ++g) S[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[g], Q[c][g], S[b], 0, 0, 0);
                     }
@@ -1007,6 +1068,11 @@ __global__ __launch_bounds__(256, NB > 8 ? 1 : 2) void latent_attn_rows_f32_kern
         }
         s0 = s1;
     }
+    __syncthreads();
+    if (*odd) {      // zero times such a value is no zero: these rows key by key, each the keys that it sees
+        for (int64_t t = row0 + wr; t < min(row0 + wr + 16, p.n); ++t) latent_row_f32(p, t, head);
+        return;
+    }
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
     if (!valid) return;
@@ -1057,6 +1123,36 @@ __global__ __launch_bounds__(64) void latent_attn_merge_kernel(const i64h_latent
     }
 }
 
+// portions of prompts over 32-bit caches (i64h_latent_attn, and i64h_kattn with its key heads, chunks, key scales and bias)
+bool latent_rows_f32_ok(const i64h_latent_attn_args& d) {
+    const int D = d.kv_rank + d.rot_dim;
+    return d.mode == 3 && d.cache_dtype == 0 && D % 4 == 0 && d.kv_rank % 16 == 0 && d.kv_rank <= 256 && D <= 320 && (uintptr_t)d.Q % 16 == 0 &&
+           (uintptr_t)d.cache % 16 == 0 && d.row_stride % 4 == 0;
+}
+
+int latent_rows_f32_run(const i64h_latent_attn_args& d, void* stream) {
+    const int D = d.kv_rank + d.rot_dim;
+    const int G = d.kv_groups > 1 ? d.kv_groups : 1;
+    I64H_CHECK_ARG(d.heads % G == 0, "latent_attn: %d heads over %d key heads", d.heads, G);
+    const int rep = d.heads / G, hw = rep % 4 == 0 ? 4 : (rep % 2 == 0 ? 2 : 1), rows = 16 * (4 / hw);
+    const int64_t wgs = (d.n + rows - 1) / rows * (d.heads / hw);
+    I64H_CHECK_ARG(wgs < (1ll << 31), "latent_attn: too many tiles");
+    const int kcols = D - (d.key_off & ~15), chunks = (kcols + 15) / 16;
+    const size_t bytes = ((size_t)32 * (kcols + 4) + (size_t)d.kv_rank * LT_FLD) * 4 + 129 * 4;
+    const bool extra = d.kscale || d.bias || d.softcap > 0.0f;
+#define LT_ROWS(KC, NB) do { \
+        if (extra) hipLaunchKernelGGL((latent_attn_rows_f32_kernel<KC, NB, true>), dim3((unsigned)wgs), dim3(256), bytes, (hipStream_t)stream, d, hw); \
+        else hipLaunchKernelGGL((latent_attn_rows_f32_kernel<KC, NB, false>), dim3((unsigned)wgs), dim3(256), bytes, (hipStream_t)stream, d, hw); \
+    } while (0)
+    if (chunks <= 4 && d.kv_rank <= 64) LT_ROWS(4, 4);
+    else if (chunks <= 8 && d.kv_rank <= 128) LT_ROWS(8, 8);
+    else if (chunks <= 18) LT_ROWS(18, 16);
+    else LT_ROWS(20, 16);
+#undef LT_ROWS
+    I64H_CHECK_LAUNCH();
+    return 0;
+}
+
 extern "C" {
 
 int i64h_latent_prep(const i64h_latent_prep_args* dp, void* stream) {
@@ -1095,9 +1191,7 @@ int i64h_latent_attn(const i64h_latent_attn_args* dp, void* stream) {
     const int D = d.kv_rank + d.rot_dim;
     const bool mfma_ok = d.cache_dtype == 2 && D % 8 == 0 && d.kv_rank % 16 == 0 && d.kv_rank <= 16 * LT_NB && D <= 32 * LT_KD &&
                          (uintptr_t)d.Q % 16 == 0 && (uintptr_t)d.cache % 16 == 0 && d.row_stride % 8 == 0;
-    const bool rows_f32 = d.mode == 3 && d.cache_dtype == 0 && D % 4 == 0 && d.kv_rank % 16 == 0 && d.kv_rank <= 256 && D <= 320 && (uintptr_t)d.Q % 16 == 0 &&
-                          (uintptr_t)d.cache % 16 == 0 && d.row_stride % 4 == 0;
-    I64H_CHECK_ARG(mfma_ok || rows_f32 || (d.kv_groups <= 1 && d.row_stride <= 0 && d.chunk <= 0 && !d.kscale && !d.bias),
+    I64H_CHECK_ARG(mfma_ok || (d.kv_groups <= 1 && d.row_stride <= 0 && d.chunk <= 0 && !d.kscale && !d.bias),
                    "latent_attn: key heads, chunks, key scales and bias are built for the matrix-core form only");
     I64H_CHECK_ARG(!d.sink_w || d.sink, "latent_attn: sink scores without the sink");
     I64H_CHECK_ARG(d.keep_first >= 0, "latent_attn: %d kept positions", d.keep_first);
@@ -1143,27 +1237,7 @@ int i64h_latent_attn(const i64h_latent_attn_args* dp, void* stream) {
         }
         return 0;
     }
-    if (rows_f32) {
-        const int G = d.kv_groups > 1 ? d.kv_groups : 1;
-        I64H_CHECK_ARG(d.heads % G == 0, "latent_attn: %d heads over %d key heads", d.heads, G);
-        const int rep = d.heads / G, hw = rep % 4 == 0 ? 4 : (rep % 2 == 0 ? 2 : 1), rows = 16 * (4 / hw);
-        const int64_t wgs = (d.n + rows - 1) / rows * (d.heads / hw);
-        I64H_CHECK_ARG(wgs < (1ll << 31), "latent_attn: too many tiles");
-        const int kcols = D - (d.key_off & ~15), chunks = (kcols + 15) / 16;
-        const size_t bytes = ((size_t)32 * (kcols + 4) + (size_t)d.kv_rank * LT_FLD) * 4 + 128 * 4;
-        const bool extra = d.kscale || d.bias || d.softcap > 0.0f;
-#define LT_ROWS(KC, NB) do { \
-            if (extra) hipLaunchKernelGGL((latent_attn_rows_f32_kernel<KC, NB, true>), dim3((unsigned)wgs), dim3(256), bytes, (hipStream_t)stream, d, hw); \
-            else hipLaunchKernelGGL((latent_attn_rows_f32_kernel<KC, NB, false>), dim3((unsigned)wgs), dim3(256), bytes, (hipStream_t)stream, d, hw); \
-        } while (0)
-        if (chunks <= 4 && d.kv_rank <= 64) LT_ROWS(4, 4);
-        else if (chunks <= 8 && d.kv_rank <= 128) LT_ROWS(8, 8);
-        else if (chunks <= 18) LT_ROWS(18, 16);
-        else LT_ROWS(20, 16);
-#undef LT_ROWS
-        I64H_CHECK_LAUNCH();
-        return 0;
-    }
+    if (latent_rows_f32_ok(d)) return latent_rows_f32_run(d, stream);
     const size_t lds = (size_t)(4 * D + 512) * 4;
     I64H_CHECK_ARG(lds <= 64 * 1024, "latent_attn: cached rows of %d values do not fit", D);
     hipLaunchKernelGGL(latent_attn_row_kernel, dim3((unsigned)d.n, (unsigned)((d.heads + 3) / 4)), dim3(256), lds, (hipStream_t)stream, d);
