@@ -63,3 +63,5 @@ def test_ties_masks_and_non_finite(V, k):
     x[:, 11], x[:, 5], x[:, 20] = 50.0, math.nan, 50.0
     assert draw(x, 1.0, k, 1.0, u).tolist() == [11] * 4      # a sum that is no number: the first of the largest
     assert draw(x, 0.0, k, 1.0, u).tolist() == [11] * 4      # greedy
+    y = torch.randn(4, V)
+    assert draw(y, 1.0, k, 0.9, torch.full((4,), -0.5)).tolist() == y.argmax(1).tolist()      # a draw below zero: the most likely token

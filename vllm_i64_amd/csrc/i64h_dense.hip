@@ -570,7 +570,7 @@ __global__ __launch_bounds__(SR_THREADS) void sample_rows_kernel(const float* __
     }
     const int arg = bi < V ? bi : 0;
     const float T = temperature ? temperature[r] : 0.0f;
-    if (!(T > 0.0f)) {
+    if (!(T > 0.0f) || (u && u[r] < 0.0f)) {
         if (tid == 0) out[r] = arg;
         return;
     }
