@@ -383,11 +383,15 @@ __device__ __forceinline__ int bl_wave_argmax(float v, int idx, float& best) {
 }
 
 #define RT_MAX_TOP 32
-#define RT_SPLIT_ROWS 512      // launches of at most so many rows give every row a workgroup
-// SPLIT: a workgroup per row - its four waves share the columns of the router's products, the first one goes on with their sums (few
-// rows: one wave's chain of loads is what a launch would wait for).
+// SPLIT: a workgroup per row - four waves share the columns of the router's products, four such groups (or one) the entries, eight at a time, the first
+// wave goes on with their sums (few rows: one wave's chain of loads is what a launch would wait for).
+// One group | four, rows of 2048: 16 entries 64 rows 10.4 | 8.0 us, 256 rows 10.5 | 8.3, 512 rows 10.9 | 12.0; 64 entries 28.4 | 13.8, 28.6 | 14.5,
+// 29.1 | 19.0.  Without SPLIT 1024 rows of 16 entries take 25 us and of 64 entries 87, with it 33.
+#define RT_WIDE_ROWS 256       // launches of at most so many rows have the four groups; all of more than RT_MANY entries do
+#define RT_MANY 32
+#define RT_SPLIT_ROWS 512      // launches of at most so many rows are split; twice as many over more than RT_MANY entries
 template <bool SPLIT>
-__global__ __launch_bounds__(256) void route_topk_kernel(const i64h_route_args p) {
+__global__ __launch_bounds__(SPLIT ? 1024 : 256) void route_topk_kernel(const i64h_route_args p) {
     extern __shared__ float rt_lds[];   // per wave: [E] scores, [E] choice values, [groups] group flags; SPLIT: once, and [4][E + 1] partial products
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const int64_t t = SPLIT ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wid;
@@ -404,10 +408,10 @@ __global__ __launch_bounds__(256) void route_topk_kernel(const i64h_route_args p
         const int K = p.K;
         const bool vec = (K & 3) == 0 && (p.ldh & 3) == 0 && ((uintptr_t)p.h & 15) == 0 && ((uintptr_t)p.W & 7) == 0;
         const int rows = p.gate_out ? E + 1 : E;
-        for (int e0 = 0; e0 < rows; e0 += 8) {
+        for (int e0 = SPLIT ? wid / 4 * 8 : 0; e0 < rows; e0 += SPLIT ? blockDim.x / 32 : 8) {
             float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
             if (vec) {
-                for (int k = (SPLIT ? threadIdx.x : lane) * 4; k < K; k += SPLIT ? 1024 : 256) {
+                for (int k = (SPLIT ? threadIdx.x & 255 : lane) * 4; k < K; k += SPLIT ? 1024 : 256) {
                     const float4 x = *(const float4*)(h + k);
 #pragma unroll
                     for (int j = 0; j < 8; ++j) {
@@ -421,7 +425,7 @@ __global__ __launch_bounds__(256) void route_topk_kernel(const i64h_route_args p
                     }
                 }
             } else {
-                for (int k = SPLIT ? threadIdx.x : lane; k < K; k += SPLIT ? 256 : 64) {
+                for (int k = SPLIT ? threadIdx.x & 255 : lane; k < K; k += SPLIT ? 256 : 64) {
                     const float x = h[k];
 #pragma unroll
                     for (int j = 0; j < 8; ++j)
@@ -432,7 +436,7 @@ __global__ __launch_bounds__(256) void route_topk_kernel(const i64h_route_args p
             for (int j = 0; j < 8; ++j) {
                 const float v = wave_sum(acc[j]);
                 if (SPLIT) {
-                    if (lane == 0 && e0 + j < rows) part[wid * rows + e0 + j] = v;
+                    if (lane == 0 && e0 + j < rows) part[(wid & 3) * rows + e0 + j] = v;
                     continue;
                 }
                 if (lane == 0 && e0 + j < E) ch[e0 + j] = p.bias ? v + p.bias[e0 + j] : v;
@@ -569,18 +573,31 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const i64h_moe_plan_args
     }
 }
 
+// A thread's loads of four choices are on their way together (as one after the other, each behind its row's number: 7.9 us for 64 rows of
+// 2048, 4 choices and a shared part, 3.6 so; 4096 rows 37 -> 29); VEC columns at a time.
+template <int VEC>
 __global__ __launch_bounds__(256) void moe_combine_kernel(const i64h_moe_combine_args p) {
+    typedef float vec __attribute__((ext_vector_type(VEC)));
     const int64_t t = blockIdx.x;
     const int W = p.W;
-    for (int c = threadIdx.x; c < W; c += 256) {
-        float a = 0.0f;
-        for (int k = 0; k < p.top; ++k) {
-            const int r = p.pair_row[t * p.top + k];
-            const float v = r >= 0 ? p.Y[(int64_t)r * W + c] : p.h[t * W + c];
-            a += p.wgt ? p.wgt[t * p.top + k] * v : v;
+    for (int c = threadIdx.x * VEC; c < W; c += 256 * VEC) {
+        vec a = 0.0f, sh = 0.0f;
+        if (p.shared) sh = *(const vec*)(p.shared + t * W + c);
+        for (int k0 = 0; k0 < p.top; k0 += 4) {
+            vec v[4];
+            float w[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int k = min(k0 + i, p.top - 1), r = p.pair_row[t * p.top + k];
+                v[i] = *(const vec*)(r >= 0 ? p.Y + (int64_t)r * W + c : p.h + t * W + c);
+                w[i] = p.wgt ? p.wgt[t * p.top + k] : 1.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (k0 + i < p.top) a += w[i] * v[i];
         }
-        if (p.shared) a += p.shared_gate ? p.shared_gate[t] * p.shared[t * W + c] : p.shared[t * W + c];
-        p.out[t * W + c] = a;
+        if (p.shared) a += p.shared_gate ? p.shared_gate[t] * sh : sh;
+        *(vec*)(p.out + t * W + c) = a;
     }
 }
 
@@ -728,8 +745,9 @@ int i64h_route_topk(const i64h_route_args* dp, void* stream) {
     I64H_CHECK_ARG(d.idx && d.wgt && ((d.logits && d.ld >= d.E) || (d.W && d.h && d.K > 0 && d.ldh >= d.K)), "route_topk: null operand or row stride below the row");
     if (d.n == 0) return 0;
     const size_t own = (size_t)(2 * d.E + (d.groups > 1 ? d.groups : 1));
-    if (d.W && d.n <= RT_SPLIT_ROWS)
-        hipLaunchKernelGGL(route_topk_kernel<true>, dim3((unsigned)d.n), dim3(256), (own + 4 * (size_t)(d.E + 1)) * 4, (hipStream_t)stream, d);
+    const int many = d.E > RT_MANY;
+    if (d.W && d.n <= (RT_SPLIT_ROWS << many))
+        hipLaunchKernelGGL(route_topk_kernel<true>, dim3((unsigned)d.n), dim3(many || d.n <= RT_WIDE_ROWS ? 1024 : 256), (own + 4 * (size_t)(d.E + 1)) * 4, (hipStream_t)stream, d);
     else
         hipLaunchKernelGGL(route_topk_kernel<false>, dim3((unsigned)((d.n + 3) / 4)), dim3(256), 4 * own * 4, (hipStream_t)stream, d);
     I64H_CHECK_LAUNCH();
@@ -754,7 +772,9 @@ int i64h_moe_combine(const i64h_moe_combine_args* dp, void* stream) {
     I64H_CHECK_ARG(d.top > 0 && d.W > 0 && d.n >= 0, "moe_combine: top %d, width %d", d.top, d.W);
     I64H_CHECK_ARG(d.Y && d.pair_row && d.h && d.out, "moe_combine: null operand");
     if (d.n == 0) return 0;
-    hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)d.n), dim3(256), 0, (hipStream_t)stream, d);
+    const bool vec = d.W % 4 == 0 && (((uintptr_t)d.Y | (uintptr_t)d.h | (uintptr_t)d.shared | (uintptr_t)d.out) & 15) == 0;
+    if (vec) hipLaunchKernelGGL(moe_combine_kernel<4>, dim3((unsigned)d.n), dim3(256), 0, (hipStream_t)stream, d);
+    else hipLaunchKernelGGL(moe_combine_kernel<1>, dim3((unsigned)d.n), dim3(256), 0, (hipStream_t)stream, d);
     I64H_CHECK_LAUNCH();
     return 0;
 }

@@ -447,32 +447,44 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(const i64h_ssm_scan_args 
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void gate_norm_kernel(const i64h_gate_norm_args p) {
-    extern __shared__ float sv[];   // [width] gated values, [groups] root mean squares
+// VEC columns at a time and, for few rows, more waves (one column a thread and four waves: 6.5 us for 64 rows of 2048, 3.6 now; 4096 rows
+// 26.4 -> 22.5, where 96 MiB travel).
+template <int NT, int VEC>
+__global__ __launch_bounds__(NT) void gate_norm_kernel(const i64h_gate_norm_args p) {
+    extern __shared__ __attribute__((aligned(16))) float gv[];   // [width] gated values, [groups] root mean squares
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int64_t m = blockIdx.x;
-    const int W = p.width;
-    for (int c = tid; c < W; c += 256) {
-        float v = p.y[m * p.ldy + c];
-        if (p.z && !p.gate_after) v *= p.gate_act ? hy_sigmoid(p.z[m * p.ldz + c]) : hy_silu(p.z[m * p.ldz + c]);
-        sv[c] = v;
+    const int W = p.width, gs = W / p.groups, wl = p.w_len > 0 ? p.w_len : W;
+    typedef float vec __attribute__((ext_vector_type(VEC)));
+    const float* const y = p.y + m * p.ldy;
+    const float* const z = p.z ? p.z + m * p.ldz : nullptr;
+    auto gate = [&](vec v, vec g) {
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) v[i] *= p.gate_act ? hy_sigmoid(g[i]) : hy_silu(g[i]);
+        return v;
+    };
+#pragma unroll 2
+    for (int c = tid * VEC; c < W; c += NT * VEC) {
+        vec v = *(const vec*)(y + c);
+        if (z && !p.gate_after) v = gate(v, *(const vec*)(z + c));
+        *(vec*)(gv + c) = v;
     }
     __syncthreads();
-    const int gs = W / p.groups;
-    for (int g = wid; g < p.groups; g += 4) {
+    for (int g = wid; g < p.groups; g += NT / 64) {
         float s = 0.0f;
         for (int c = lane; c < gs; c += 64) {
-            const float v = sv[g * gs + c];
+            const float v = gv[g * gs + c];
             s += v * v;
         }
         s = wave_sum(s);
-        if (lane == 0) sv[W + g] = sqrtf(s / (float)gs + p.eps);
+        if (lane == 0) gv[W + g] = sqrtf(s / (float)gs + p.eps);
     }
     __syncthreads();
-    for (int c = tid; c < W; c += 256) {
-        float v = sv[c] / sv[W + c / gs] * p.w[p.w_len > 0 ? c % p.w_len : c];
-        if (p.z && p.gate_after) v *= p.gate_act ? hy_sigmoid(p.z[m * p.ldz + c]) : hy_silu(p.z[m * p.ldz + c]);
-        p.out[m * p.ldo + c] = v;
+#pragma unroll 2
+    for (int c = tid * VEC; c < W; c += NT * VEC) {      // (VEC divides a group and the weights' period)
+        vec v = *(const vec*)(gv + c) / gv[W + c / gs] * *(const vec*)(p.w + c % wl);
+        if (z && p.gate_after) v = gate(v, *(const vec*)(z + c));
+        *(vec*)(p.out + m * p.ldo + c) = v;
     }
 }
 
@@ -674,7 +686,7 @@ __device__ __forceinline__ void rot_pair(int d, int dims, int interleaved, int& 
 // pass norms and rotates out of LDS straight into the query rows and the cached row.
 template <int NT>
 __global__ __launch_bounds__(NT) void rot_prep_kernel(const i64h_rot_prep_args p) {
-    extern __shared__ float sv[];   // [heads * dim + kv_heads * dim] raw queries and keys, [heads + kv_heads] 1 / rms per head, 8 for
+    extern __shared__ float sv[];   // [heads * dim + kv_heads * dim] raw queries and keys, [heads + kv_heads] 1 / rms per head, two per wave for
                                     // reductions, [rot_dims] cosines and sines of the row's angles, [vdim] those of the values' angles
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int64_t t = blockIdx.x;
@@ -683,7 +695,7 @@ __global__ __launch_bounds__(NT) void rot_prep_kernel(const i64h_rot_prep_args p
     const int half = p.rot_dims >> 1, vhalf = p.v_freq ? vd >> 1 : 0;
     float* inv = sv + nq + nk;
     float* red = inv + p.heads + p.kv_heads;
-    float* rcs = red + 8;           // [half] cosines, [half] sines: every head turns by the same angles
+    float* rcs = red + 2 * (NT / 64);           // [half] cosines, [half] sines: every head turns by the same angles
     float* vcs = rcs + 2 * half;    // [vhalf] cosines, [vhalf] sines
     const float* q = p.P + t * p.ldp + p.q_off;
     const float* k = p.P + t * p.ldp + p.k_off;
@@ -691,13 +703,14 @@ __global__ __launch_bounds__(NT) void rot_prep_kernel(const i64h_rot_prep_args p
     const int pos = p.positions[t];
     const float fpos = (float)pos;
     float a = 0.0f, b = 0.0f;
+#pragma unroll 4
     for (int c = tid; c < nq + nk; c += NT) {
         const float x = c < nq ? q[c] : k[c - nq];
         sv[c] = x;
         if (c < nq) a += x * x;
         else b += x * x;
     }
-    for (int i = tid; i < half + vhalf; i += NT) {
+    for (int i = NT - 1 - tid; i < half + vhalf; i += NT) {      // (the last waves have least of the row)
         float sn, cs;
         if (i < half) {
             sincosf(fpos * p.inv_freq[i], &sn, &cs);
@@ -711,11 +724,11 @@ __global__ __launch_bounds__(NT) void rot_prep_kernel(const i64h_rot_prep_args p
     if (p.q_norm_w && !p.norm_heads) {   // (both sums through one exchange)
         a = wave_sum(a), b = wave_sum(b);
         __syncthreads();
-        if (lane == 0) red[wid] = a, red[4 + wid] = b;
+        if (lane == 0) red[wid] = a, red[NT / 64 + wid] = b;
         __syncthreads();
         float sa = 0.0f, sb = 0.0f;
 #pragma unroll
-        for (int w = 0; w < NT / 64; ++w) sa += red[w], sb += red[4 + w];
+        for (int w = 0; w < NT / 64; ++w) sa += red[w], sb += red[NT / 64 + w];
         qr = 1.0f / sqrtf(sa / (float)nq + p.eps);
         kr = 1.0f / sqrtf(sb / (float)nk + p.eps);
     }
@@ -810,6 +823,11 @@ __global__ __launch_bounds__(256) void rot_post_kernel(const i64h_rot_post_args 
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
+// Launches of at most so many rows give a row's workgroup more waves: it is one workgroup's chain of loads and sums that they wait for.  rot_prep (32 + 8
+// heads of 64 + 64, rotated values | 16 + 4 heads), 4 | 16 waves a row: 64 rows 16.5 | 8.7 and 9.2 | 6.3 us, 256 rows 17.1 | 9.5 and 9.4 | 6.8,
+// 512 rows 18.7 | 16.7 and 10.2 | 11.4.
+#define HY_WIDE_ROWS 256
+
 extern "C" {
 
 int i64h_embed_bigram(const i64h_embed_bigram_args* dp, void* stream) {
@@ -938,7 +956,12 @@ int i64h_gate_norm(const i64h_gate_norm_args* dp, void* stream) {
     const size_t lds = ((size_t)d.width + d.groups) * 4;
     I64H_CHECK_ARG(lds <= 64 * 1024, "gate_norm: a row of %d values does not fit the kernel's LDS buffer", d.width);
     if (d.n == 0) return 0;
-    hipLaunchKernelGGL(gate_norm_kernel, dim3((unsigned)d.n), dim3(256), lds, (hipStream_t)stream, d);
+    const bool vec = (d.width / d.groups) % 4 == 0 && d.w_len % 4 == 0 && (d.ldy | d.ldo | (d.z ? d.ldz : 0)) % 4 == 0 &&
+                     (((uintptr_t)d.y | (uintptr_t)d.z | (uintptr_t)d.w | (uintptr_t)d.out) & 15) == 0;
+    const bool wide = d.n <= HY_WIDE_ROWS;
+    auto launch = [&](auto kern, int nt) { hipLaunchKernelGGL(kern, dim3((unsigned)d.n), dim3(nt), lds, (hipStream_t)stream, d); };
+    if (vec) wide ? launch(gate_norm_kernel<512, 4>, 512) : launch(gate_norm_kernel<256, 4>, 256);
+    else wide ? launch(gate_norm_kernel<1024, 1>, 1024) : launch(gate_norm_kernel<256, 1>, 256);
     I64H_CHECK_LAUNCH();
     return 0;
 }
@@ -1034,7 +1057,10 @@ int i64h_rot_prep(const i64h_rot_prep_args* dp, void* stream) {
     const size_t lds = ((size_t)(d.heads + d.kv_heads) * (d.dim + 1) + 8 + d.rot_dims + (d.v_freq ? d.vdim : 0)) * 4;
     I64H_CHECK_ARG(lds <= 64 * 1024, "rot_prep: %d + %d heads of %d values do not fit the kernel's LDS buffer", d.heads, d.kv_heads, d.dim);
     if (d.n == 0) return 0;
-    hipLaunchKernelGGL(rot_prep_kernel<256>, dim3((unsigned)d.n), dim3(256), lds, (hipStream_t)stream, d);
+    if (d.n <= HY_WIDE_ROWS && lds + 24 * 4 <= 64 * 1024)
+        hipLaunchKernelGGL(rot_prep_kernel<1024>, dim3((unsigned)d.n), dim3(1024), lds + 24 * 4, (hipStream_t)stream, d);
+    else
+        hipLaunchKernelGGL(rot_prep_kernel<256>, dim3((unsigned)d.n), dim3(256), lds, (hipStream_t)stream, d);
     I64H_CHECK_LAUNCH();
     return 0;
 }
