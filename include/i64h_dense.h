@@ -163,10 +163,11 @@ int i64h_latent_prep(const i64h_latent_prep_args* d, void* stream);
  * 0 <= p - j < window (window <= 0: every j <= p) and, under a window, the first keep_first positions j < keep_first (<= p);  s_j = scale * Q[t, h, :] . row_j;  ordinary softmax over the visible j;
  * out[t, h, :kv_rank] = sum_j w_j * row_j[:kv_rank].  Scores, weights and sums in fp32.  out fp32 [n, heads, kv_rank].
  * With sink the denominator also holds exp(sink_w[h]) (exp(0) without sink_w): a term without a key and without a value, not scaled.
- * mode 1: one wave per (row, head), fp32 products, any sizes and cache type (of the options below it knows the sink).  Modes 0 / 2 / 3 take the matrix-core form when the cache
- * is bf16, kv_rank % 16 == 0 and <= 256, (kv_rank + rot_dim) % 8 == 0 and <= 320 (the row form otherwise): 2 (and 0) one wave per token
- * and group of 16 heads (rows that are one per sequence), 3 one wave per 16 consecutive rows and head (portions of prompts; rows of
- * different sequences in one tile are handled run by run). */
+ * mode 1: one wave per (row, head), fp32 products, any sizes and cache type (of the options below it knows the sink, the soft cap and the kept positions).
+ * Modes 0 / 2 / 3 take the matrix-core forms when the cache is bf16, kv_rank % 16 == 0 and <= 256, (kv_rank + rot_dim) % 8 == 0 and <= 320 (the row
+ * form otherwise): 2 (and 0) one wave per token and group of 16 heads (rows that are one per sequence), 3 four waves of 16 consecutive rows and
+ * a head each that share a key head's tiles (portions of prompts; rows of different sequences in one tile are handled run by run).  Mode 3 over a
+ * 32-bit cache of such sizes ((kv_rank + rot_dim) % 4 == 0) is the same on 32-bit matrix products. */
 typedef struct {
     const float* Q;
     const void* cache;
@@ -197,7 +198,7 @@ typedef struct {
     float softcap;       /* > 0: a score s (after scale and key scale, before any bias) becomes softcap * tanh(s / softcap) */
     int32_t keep_first;  /* with a window: the first positions of a sequence that stay visible to everyone */
 } i64h_latent_attn_args;
-int i64h_set_latent_attn_decode_form(int32_t on); /* tuning / test knob: 1 (default) = mode 2 launches run the kernel that requests a tile's fragments a tile ahead; 0 = the general matrix-core kernel; same results up to summation order */
+int i64h_set_latent_attn_decode_form(int32_t on); /* tuning / test knob: 1 (default) = mode 2 launches run the kernel that requests a tile's fragments a tile ahead; 0 = a plainer kernel with the same tiles; same results up to summation order */
 int64_t i64h_latent_attn_workspace_floats(int64_t n, int32_t heads, int32_t kv_rank, int32_t splits);
 int i64h_latent_attn(const i64h_latent_attn_args* d, void* stream);
 
