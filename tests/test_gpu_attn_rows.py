@@ -138,3 +138,22 @@ def test_options_of_key_heads_stay_refused_over_32_bits(dev):
                             out=D.ptr(f), n=1, heads=2, kv_rank=32, rot_dim=0, mode=3, **option)
         with pytest.raises(_lib.I64HError, match="matrix-core form only"):
             D.call_dense("i64h_latent_attn", D._ref(d), D._stream())
+
+
+def test_a_score_of_minus_infinity_is_a_weight_of_zero(dev):
+    """An infinite first column of a key meets negative queries only: the columns past a key's end, which a step of the products takes along, add nothing to its score.  (32-bit products: two bf16 terms of a query may differ in sign, and then meet an infinity as both.)"""
+    from vllm_i64_amd import ops_dense as D
+    H, dim, vdim, n = 4, 24, 48, 20
+    g = torch.Generator().manual_seed(5)
+    bt, pos, slots, blocks = pages([n], [0], 16, g)
+    cache = torch.randn(blocks, 16, vdim + dim, generator=g)
+    cache[bt[0, 0], 3, vdim] = math.inf
+    q = torch.randn(n, H, vdim + dim, generator=g)
+    q[:, :, :vdim] = 0
+    q[:, :, vdim] = -q[:, :, vdim].abs() - 0.1
+    out = torch.empty(n, H * vdim, device=dev)
+    D.kattn(q.to(dev), cache.to(dev), None, bt.to(dev), slots.to(dev), pos.to(dev), chunk=0, bias=None, sink=False, heads=H, kv_heads=1, dim=dim, vdim=vdim, out=out, n=n, mode=3)
+    j = torch.arange(n)
+    rows = cache[bt[0].long()[j // 16], j % 16].expand(H, -1, -1)
+    ref = reference(q[:, :, vdim:], rows[..., vdim:], rows[..., :vdim], pos, 1.0, 0, 0, 0.0, torch.full((H,), -math.inf))
+    assert torch.allclose(out.view(n, H, vdim).double().cpu(), ref, atol=4e-5, rtol=2e-5)
