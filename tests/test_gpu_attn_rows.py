@@ -157,3 +157,24 @@ def test_a_score_of_minus_infinity_is_a_weight_of_zero(dev):
     rows = cache[bt[0].long()[j // 16], j % 16].expand(H, -1, -1)
     ref = reference(q[:, :, vdim:], rows[..., vdim:], rows[..., :vdim], pos, 1.0, 0, 0, 0.0, torch.full((H,), -math.inf))
     assert torch.allclose(out.view(n, H, vdim).double().cpu(), ref, atol=4e-5, rtol=2e-5)
+
+
+@pytest.mark.parametrize("dim,vdim", [(24, 64), (40, 32), (8, 256)])
+def test_an_infinite_first_column_of_a_bf16_key(dev, dim, vdim):
+    """A step of the products takes columns past a key's end along, as zeros: beside an infinite first column they would make a score of minus infinity
+    no number.  (The first column's queries are such that both of their bf16 terms, after the factor log2(e), are negative.)"""
+    from vllm_i64_amd import ops_dense as D
+    H, n = 4, 20
+    g = torch.Generator().manual_seed(5)
+    bt, pos, slots, blocks = pages([n], [0], 16, g)
+    cache = torch.randn(blocks, 16, vdim + dim, generator=g).to(torch.bfloat16)
+    cache[bt[0, 0], 3, vdim] = math.inf
+    q = torch.randn(n, H, vdim + dim, generator=g)
+    q[:, :, :vdim] = 0
+    q[:, :, vdim] = -(1.0 + 2.0 ** -10) / math.log2(math.e)
+    out = torch.empty(n, H * vdim, device=dev)
+    D.kattn(q.to(dev), cache.to(dev), None, bt.to(dev), slots.to(dev), pos.to(dev), chunk=0, bias=None, sink=False, heads=H, kv_heads=1, dim=dim, vdim=vdim, out=out, n=n, mode=3)
+    j = torch.arange(n)
+    rows = cache[bt[0].long()[j // 16], j % 16].expand(H, -1, -1)
+    ref = reference(q[:, :, vdim:], rows[..., vdim:], rows[..., :vdim], pos, 1.0, 0, 0, 0.0, torch.full((H,), -math.inf))
+    assert torch.allclose(out.view(n, H, vdim).double().cpu(), ref, atol=2e-3, rtol=1e-3)

@@ -589,7 +589,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_rows_kernel(const i64h_lat
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, n = lane & 15, kg = lane >> 4;
     const int r = p.kv_rank, D = r + p.rot_dim, H = p.heads, bs = p.block_size, win = p.window, koff = p.key_off & ~31;
     const int keep = p.chunk <= 0 && win > 0 ? p.keep_first : 0;
-    const int kld = D - koff + 8;             // halves per key row in LDS: the columns that take part in the scores
+    const int kld = D - koff + 8;             // halves per key row in LDS: the columns that take part in the scores, and eight zeros
     const int plane = 32 * kld + r * LT_VLD;
     uint16_t* const buf0 = (uint16_t*)smem;   // twice: keys [32][kld], values transposed [r][LT_VLD]
     int* const info = (int*)(buf0 + 2 * plane);      // [64] positions, [64] slots (-1: no such row)
@@ -606,8 +606,9 @@ __global__ __launch_bounds__(256, 2) void latent_attn_rows_kernel(const i64h_lat
     }
     const int64_t tok = row0 + wr + n;
     const bool valid = tok < p.n;
+    if (tid < 64) *(uint4*)&buf0[(tid >> 5) * plane + (tid & 31) * kld + D - koff] = make_uint4(0, 0, 0, 0);
     // the query of row n times scale * log2(e) (the softmax runs on powers of two), columns koff + ks * 32 + kg * 8 .. + 7, as two bf16 terms;
-    // zeros past the end, where the key reads repeat the first columns: no step and no block of columns has a branch of its own
+    // zeros past the end, as in the keys: no step and no block of columns has a branch of its own
     uint4 Qh[KD], Ql[KD];
     {
         const float* q = p.Q + ((valid ? tok : row0) * H + head) * D;
@@ -732,7 +733,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_rows_kernel(const i64h_lat
                     const int d0 = ks * 32 + kg * 8;
 #pragma unroll
                     for (int b = 0; b < 2; ++b) {
-                        const lt_v8bf kf = __builtin_bit_cast(lt_v8bf, *(const uint4*)&K[(16 * b + n) * kld + (d0 < D - koff ? d0 : 0)]);
+                        const lt_v8bf kf = __builtin_bit_cast(lt_v8bf, *(const uint4*)&K[(16 * b + n) * kld + min(d0, D - koff)]);
                         S[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, __builtin_bit_cast(lt_v8bf, Qh[ks]), S[b], 0, 0, 0);
                         S[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, __builtin_bit_cast(lt_v8bf, Ql[ks]), S[b], 0, 0, 0);
                     }
