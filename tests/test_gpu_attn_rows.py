@@ -178,3 +178,30 @@ def test_an_infinite_first_column_of_a_bf16_key(dev, dim, vdim):
     rows = cache[bt[0].long()[j // 16], j % 16].expand(H, -1, -1)
     ref = reference(q[:, :, vdim:], rows[..., vdim:], rows[..., :vdim], pos, 1.0, 0, 0, 0.0, torch.full((H,), -math.inf))
     assert torch.allclose(out.view(n, H, vdim).double().cpu(), ref, atol=2e-3, rtol=1e-3)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32])
+def test_rows_without_a_sequence(dev, dtype):
+    """Rows whose slot is -1 see no key, also where rows are summed key by key because a value of their tile is no finite number: the sink alone, zeros."""
+    from vllm_i64_amd import ops_dense as D
+    H, dim, vdim, n = 4, 32, 64, 24
+    g = torch.Generator().manual_seed(7)
+    bt, pos, slots, blocks = pages([n], [0], 16, g)
+    cache = torch.randn(blocks, 16, vdim + dim, generator=g).to(dtype)
+    q = torch.randn(n, H, vdim + dim, generator=g)
+    q[:, :, :vdim] = 0
+    slots[[2, 5, 20]] = -1
+    cache[bt[0, 0], 9, 7] = math.inf
+    out = torch.empty(n, H * vdim, device=dev)
+    D.kattn(q.to(dev), cache.to(dev), None, bt.to(dev), slots.to(dev), pos.to(dev), chunk=0, bias=None, sink=True, heads=H, kv_heads=1, dim=dim, vdim=vdim, out=out, n=n, mode=3)
+    rows = cache[bt[0].long()[torch.arange(n) // 16], torch.arange(n) % 16].expand(H, -1, -1)
+    values = rows[..., :vdim].clone()
+    values[:, 9, 7] = 0.0
+    ref = reference(q[:, :, vdim:], rows[..., vdim:], values, pos, 1.0, 0, 0, 0.0, torch.zeros(H))
+    ref[slots < 0] = 0.0
+    got = out.view(n, H, vdim).double().cpu()
+    sees = (pos >= 9) & (slots >= 0)
+    assert bool((~torch.isfinite(got[sees][..., 7])).all())
+    got[sees, :, 7] = ref[sees, :, 7] = 0.0
+    tol = 1e-3 if dtype == torch.bfloat16 else 2e-5
+    assert torch.allclose(got, ref, atol=2 * tol, rtol=tol), float((got - ref).abs().max())

@@ -823,9 +823,9 @@ __device__ __forceinline__ void latent_row_f32(const i64h_latent_attn_args& p, c
     const int G = p.kv_groups > 1 ? p.kv_groups : 1, rstride = p.row_stride > 0 ? p.row_stride : D;
     const float* const cache = (const float*)p.cache + h / (p.heads / G) * D;
     const float* const q = p.Q + (t * p.heads + h) * D;
-    const int pos = p.positions[t], from = p.chunk > 0 ? pos / p.chunk * p.chunk : (win > 0 ? max(0, pos - win + 1) : 0);
-    const int kept = p.chunk <= 0 && win > 0 ? min(p.keep_first, from) : 0, total = kept + pos - from + 1;
-    const int32_t* const bt = p.block_table + (int64_t)p.slot_ids[t] * p.max_blocks_per_seq;
+    const int pos = p.positions[t], slot = p.slot_ids[t], from = p.chunk > 0 ? pos / p.chunk * p.chunk : (win > 0 ? max(0, pos - win + 1) : 0);
+    const int kept = p.chunk <= 0 && win > 0 ? min(p.keep_first, from) : 0, total = slot < 0 ? 0 : kept + pos - from + 1;      // (no slot: no keys)
+    const int32_t* const bt = p.block_table + (int64_t)slot * p.max_blocks_per_seq;
     auto key_of = [&](int i) { return i < kept ? i : from + i - kept; };      // the visible keys in order
     auto row_of = [&](int i) {
         const int j = key_of(i);
