@@ -6,7 +6,7 @@
 //   latent_prep_kernel     : RMS norm of the latent, rotation of the shared key part and of every head's rotated query part,
 //                            cache write - one workgroup per token
 //   latent_attn_rows_kernel: bf16 caches of aligned widths, portions of prompts - four waves of 16 rows that share 32 keys at a time through LDS;
-//                            latent_attn_rows_f32_kernel: the same for 32-bit caches, 32-bit products (latent_row_f32 where a value is no finite number)
+//                            latent_attn_rows_f32_kernel: the same for 32-bit caches, 32-bit products (latent_row in both where a value is no finite number
 //   latent_attn_mfma_decode_kernel (latent_attn_mfma_kernel): rows that are one per sequence - a token's heads, 16 query vectors per wave;
 //                            both on the bf16 matrix cores, see below
 //   latent_attn_row_kernel : any width and cache type, true fp32 products: one wave per (token, head): 64 keys at a time, one key per lane for the scores (fp32 dot over the
@@ -569,6 +569,56 @@ __global__ __launch_bounds__(64) void latent_attn_mfma_decode_kernel(const i64h_
     }
 }
 
+// One row and head by one wave, over the keys that it sees only: a key per lane for the scores, the columns (at most 256) spread over the lanes for the
+// sum, 32-bit products.  The kernels of prompt portions below multiply a tile's values for all rows of a wave, with weights of zero for keys that
+// a row does not see (later ones, another sequence's).  Zero times an infinity is no number, and a sum stays no number from there on: such rows go here.
+template <typename T>
+__device__ __forceinline__ void latent_row(const i64h_latent_attn_args& p, const int64_t t, const int h) {
+    const int lane = threadIdx.x & 63, r = p.kv_rank, D = r + p.rot_dim, bs = p.block_size, win = p.window;
+    const int G = p.kv_groups > 1 ? p.kv_groups : 1, rstride = p.row_stride > 0 ? p.row_stride : D;
+    const T* const cache = (const T*)p.cache + h / (p.heads / G) * D;
+    auto value = [](T x) {
+        if constexpr (sizeof(T) == 2) return __uint_as_float((uint32_t)x << 16);
+        else return x;
+    };
+    const float* const q = p.Q + (t * p.heads + h) * D;
+    const int pos = p.positions[t], slot = p.slot_ids[t], from = p.chunk > 0 ? pos / p.chunk * p.chunk : (win > 0 ? max(0, pos - win + 1) : 0);
+    const int kept = p.chunk <= 0 && win > 0 ? min(p.keep_first, from) : 0, total = slot < 0 ? 0 : kept + pos - from + 1;      // (no slot: no keys)
+    const int32_t* const bt = p.block_table + (int64_t)slot * p.max_blocks_per_seq;
+    auto key_of = [&](int i) { return i < kept ? i : from + i - kept; };      // the visible keys in order
+    auto row_of = [&](int i) {
+        const int j = key_of(i);
+        return cache + ((int64_t)bt[j / bs] * bs + j % bs) * rstride;
+    };
+    float m = p.sink ? (p.sink_w ? p.sink_w[h] : 0.0f) : -INFINITY, l = p.sink ? 1.0f : 0.0f, acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i0 = 0; i0 < total; i0 += 64) {
+        const int i = min(i0 + lane, total - 1), j = key_of(i);
+        const T* const kr = row_of(i);
+        float s = 0.0f;
+        for (int d = p.key_off; d < D; ++d) s = fmaf(q[d] * p.scale, value(kr[d]), s);
+        if (p.kscale) s *= p.kscale[(int64_t)bt[j / bs] * bs + j % bs];
+        if (p.softcap > 0.0f) s = p.softcap * tanhf(s / p.softcap);
+        if (p.bias) s += p.bias[(int64_t)min(pos - j, p.bias_rows - 1) * p.heads + h];
+        if (i0 + lane >= total) s = -INFINITY;
+        const float mn = fmaxf(m, wave_max(s)), al = expf(m - mn), w = i0 + lane < total ? expf(s - mn) : 0.0f;
+        l = l * al + wave_sum(w);
+        m = mn;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[c] *= al;
+        for (int k = 0; k < min(64, total - i0); ++k) {
+            const float wk = __shfl(w, k);
+            const T* const v = row_of(i0 + k);
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (lane + 64 * c < r) acc[c] = fmaf(wk, value(v[lane + 64 * c]), acc[c]);
+        }
+    }
+    float* const o = p.out + (t * p.heads + h) * r;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        if (lane + 64 * c < r) o[lane + 64 * c] = acc[c] / l;
+}
+
 // Portions of prompts: consecutive rows that share their sequences' cached rows.  A workgroup is four waves, each 16 rows of one head; the heads
 // of a workgroup belong to one key head (HW of them; 4 / HW blocks of 16 rows), so that all four waves read the same 32 keys, staged
 // in LDS once: row by row for the scores, the value columns transposed (a thread takes 4 keys x 8 columns) for the second product.
@@ -582,11 +632,13 @@ __global__ __launch_bounds__(64) void latent_attn_mfma_decode_kernel(const i64h_
 // 8 prompts of 512 tokens, 16 heads over one cached row of 288: 304 -> 130 us against the form before (a wave per workgroup that read every
 // fragment from memory itself and transposed it two bytes at a time), 16 heads of 64 over 4 key heads 120 -> 48 us, 32 heads of 64 over 8 key heads
 // on prompts of 1531, 257, 64, 3 and 1101 tokens 285 -> 82 us, one prompt of 77 tokens 29 -> 20 and 17 -> 11 us.
+// Which rows latent_row sums again is seen at the end, from sums that are no number: nothing between the products (the first of these prompts
+// 135 us beside 133 without it; the wave's number in a scalar register pays for its registers).
 // KD: 32-wide steps over the columns that take part in the scores, NB: 16-column blocks of the result, EXTRA: key scales, a soft cap or a bias.
 template <int KD, int NB, bool EXTRA>
 __global__ __launch_bounds__(256, 2) void latent_attn_rows_kernel(const i64h_latent_attn_args p, const int hw) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, n = lane & 15, kg = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, kg = lane >> 4;
     const int r = p.kv_rank, D = r + p.rot_dim, H = p.heads, bs = p.block_size, win = p.window, koff = p.key_off & ~31;
     const int keep = p.chunk <= 0 && win > 0 ? p.keep_first : 0;
     const int kld = D - koff + 8;             // halves per key row in LDS: the columns that take part in the scores, and eight zeros
@@ -645,7 +697,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_rows_kernel(const i64h_lat
     __syncthreads();
     int s0 = 0;
     while (s0 < rows) {
-        const int sl = info[64 + s0];
+        const int sl = __builtin_amdgcn_readfirstlane(info[64 + s0]);
         if (sl < 0) {
             ++s0;
             continue;
@@ -804,7 +856,15 @@ __global__ __launch_bounds__(256, 2) void latent_attn_rows_kernel(const i64h_lat
     }
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
-    if (!valid) return;
+    bool nan = false;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) nan |= acc[nb][g] != acc[nb][g];
+    const uint64_t lanes = __ballot(valid && nan);
+    const uint32_t by_key = (uint32_t)(lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) & 0xffffu;      // rows of this wave
+    for (uint32_t left = by_key; left; left &= left - 1) latent_row<uint16_t>(p, row0 + wr + __ffs((int)left) - 1, head);
+    if (!valid || (by_key >> n & 1)) return;
     float* o = p.out + (tok * H + head) * r;
     const float inv = 1.0f / l;
 #pragma unroll
@@ -815,49 +875,6 @@ __global__ __launch_bounds__(256, 2) void latent_attn_rows_kernel(const i64h_lat
             if (((uintptr_t)p.out & 15) == 0) *(float4*)dst = v;
             else dst[0] = v.x, dst[1] = v.y, dst[2] = v.z, dst[3] = v.w;
         }
-}
-
-// one row and head by one wave, 32-bit cache: a key per lane for the scores, the columns (at most 256) spread over the lanes for the sum
-__device__ __forceinline__ void latent_row_f32(const i64h_latent_attn_args& p, const int64_t t, const int h) {
-    const int lane = threadIdx.x & 63, r = p.kv_rank, D = r + p.rot_dim, bs = p.block_size, win = p.window;
-    const int G = p.kv_groups > 1 ? p.kv_groups : 1, rstride = p.row_stride > 0 ? p.row_stride : D;
-    const float* const cache = (const float*)p.cache + h / (p.heads / G) * D;
-    const float* const q = p.Q + (t * p.heads + h) * D;
-    const int pos = p.positions[t], slot = p.slot_ids[t], from = p.chunk > 0 ? pos / p.chunk * p.chunk : (win > 0 ? max(0, pos - win + 1) : 0);
-    const int kept = p.chunk <= 0 && win > 0 ? min(p.keep_first, from) : 0, total = slot < 0 ? 0 : kept + pos - from + 1;      // (no slot: no keys)
-    const int32_t* const bt = p.block_table + (int64_t)slot * p.max_blocks_per_seq;
-    auto key_of = [&](int i) { return i < kept ? i : from + i - kept; };      // the visible keys in order
-    auto row_of = [&](int i) {
-        const int j = key_of(i);
-        return cache + ((int64_t)bt[j / bs] * bs + j % bs) * rstride;
-    };
-    float m = p.sink ? (p.sink_w ? p.sink_w[h] : 0.0f) : -INFINITY, l = p.sink ? 1.0f : 0.0f, acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int i0 = 0; i0 < total; i0 += 64) {
-        const int i = min(i0 + lane, total - 1), j = key_of(i);
-        const float* const kr = row_of(i);
-        float s = 0.0f;
-        for (int d = p.key_off; d < D; ++d) s = fmaf(q[d] * p.scale, kr[d], s);
-        if (p.kscale) s *= p.kscale[(int64_t)bt[j / bs] * bs + j % bs];
-        if (p.softcap > 0.0f) s = p.softcap * tanhf(s / p.softcap);
-        if (p.bias) s += p.bias[(int64_t)min(pos - j, p.bias_rows - 1) * p.heads + h];
-        if (i0 + lane >= total) s = -INFINITY;
-        const float mn = fmaxf(m, wave_max(s)), al = expf(m - mn), w = i0 + lane < total ? expf(s - mn) : 0.0f;
-        l = l * al + wave_sum(w);
-        m = mn;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[c] *= al;
-        for (int k = 0; k < min(64, total - i0); ++k) {
-            const float wk = __shfl(w, k);
-            const float* const v = row_of(i0 + k);
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-                if (lane + 64 * c < r) acc[c] = fmaf(wk, v[lane + 64 * c], acc[c]);
-        }
-    }
-    float* const o = p.out + (t * p.heads + h) * r;
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-        if (lane + 64 * c < r) o[lane + 64 * c] = acc[c] / l;
 }
 
 // The same for caches of 32-bit rows, with 32-bit products: keys and transposed values once in LDS (twice would be a workgroup per CU), the next tile
@@ -1071,7 +1088,7 @@ __global__ __launch_bounds__(256, NB > 8 ? 1 : 2) void latent_attn_rows_f32_kern
     }
     __syncthreads();
     if (*odd) {      // zero times such a value is no zero: these rows key by key, each the keys that it sees
-        for (int64_t t = row0 + wr; t < min(row0 + wr + 16, p.n); ++t) latent_row_f32(p, t, head);
+        for (int64_t t = row0 + wr; t < min(row0 + wr + 16, p.n); ++t) latent_row<float>(p, t, head);
         return;
     }
     l += __shfl_xor(l, 16);
