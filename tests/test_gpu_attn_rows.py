@@ -220,3 +220,32 @@ def test_rows_without_a_sequence(dev, dtype):
     got[sees, :, 7] = ref[sees, :, 7] = 0.0
     tol = 1e-3 if dtype == torch.bfloat16 else 2e-5
     assert torch.allclose(got, ref, atol=2 * tol, rtol=tol), float((got - ref).abs().max())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_scores_of_minus_infinity_beside_a_value_that_is_no_number(dev, dtype):
+    """Rows that are summed key by key, because a later key's value in their tile is no finite number, while a distance bias of minus infinity hides all
+    but their last keys: the first 64 scores are minus infinity, weights of zero."""
+    from vllm_i64_amd import ops_dense as D
+    H, dim, vdim, n, past, reach = 4, 32, 64, 16, 144, 5
+    g = torch.Generator().manual_seed(6)
+    bt, pos, slots, blocks = pages([n], [past], 16, g)
+    cache = torch.randn(blocks, 16, vdim + dim, generator=g).to(dtype)
+    last = past + n - 1
+    cache[bt[0, last // 16], last % 16, 7] = math.nan      # seen by the last row only
+    q = torch.randn(n, H, vdim + dim, generator=g)
+    q[:, :, :vdim] = 0
+    bias = torch.randn(reach + 1, H, generator=g)
+    bias[reach:] = -math.inf      # (the table's last row stands for all distances behind it)
+    out = torch.empty(n, H * vdim, device=dev)
+    D.kattn(q.to(dev), cache.to(dev), None, bt.to(dev), slots.to(dev), pos.to(dev), chunk=0, bias=bias.to(dev), sink=False, heads=H, kv_heads=1, dim=dim, vdim=vdim, out=out, n=n, mode=3)
+    j = torch.arange(past + n)
+    rows = cache[bt[0].long()[j // 16], j % 16].double()
+    s = torch.einsum("nhd,td->hnt", q[:, :, vdim:].double(), rows[:, vdim:])
+    d = pos[:, None].long() - j[None, :]
+    s = (s + bias.double()[d.clamp(0, reach)].permute(2, 0, 1)).masked_fill(d < 0, -math.inf)
+    ref = torch.einsum("hnt,tv->nhv", torch.softmax(s, -1)[:, :-1], rows[:, :vdim].nan_to_num())
+    got = out.view(n, H, vdim).double().cpu()
+    assert bool(got[-1, :, 7].isnan().all())
+    tol = 1e-3 if dtype == torch.bfloat16 else 2e-5
+    assert torch.allclose(got[:-1], ref, atol=2 * tol, rtol=tol), float((got[:-1] - ref).abs().max())

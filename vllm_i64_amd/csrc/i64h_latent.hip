@@ -600,7 +600,7 @@ __device__ __forceinline__ void latent_row(const i64h_latent_attn_args& p, const
         if (p.softcap > 0.0f) s = p.softcap * tanhf(s / p.softcap);
         if (p.bias) s += p.bias[(int64_t)min(pos - j, p.bias_rows - 1) * p.heads + h];
         if (i0 + lane >= total) s = -INFINITY;
-        const float mn = fmaxf(m, wave_max(s)), al = expf(m - mn), w = i0 + lane < total ? expf(s - mn) : 0.0f;
+        const float mn = fmaxf(m, wave_max(s)), ms = mn == -INFINITY ? 0.0f : mn, al = expf(m - ms), w = i0 + lane < total ? expf(s - ms) : 0.0f;
         l = l * al + wave_sum(w);
         m = mn;
 #pragma unroll
