@@ -119,3 +119,24 @@ def test_not_a_number_stays_in_its_row(dev, use_form):
         D.linear(a.to(dev), w.to(dev), out)
         bad = ~torch.isfinite(out.cpu())
         assert bool(bad[[3, 65]].all()) and int(bad.sum()) == 128 and bool((out.cpu()[:3] == 72).all())
+
+
+@pytest.mark.parametrize("exact", [False, True])
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("m", [2, 16, 40])
+def test_no_more_rows_of_a_batch_than_the_launch_says(dev, use_form, form, m, exact):
+    """Rows that a batch has beyond m are left alone, and those of the batches behind it are found all the same."""
+    from vllm_i64_amd import ops_dense as D
+    use_form(form)
+    counts, N, K = [70, 3, 0, 45], 72, 136
+    g = torch.Generator().manual_seed(m)
+    off = torch.tensor([0] + counts).cumsum(0).to(torch.int32)
+    R = int(off[-1])
+    a, w = torch.randn(R, K, generator=g), bf16(torch.randn(len(counts), N, K, generator=g) / math.sqrt(K))
+    out = torch.full((R, N), 7.0, device=dev)
+    D.linear(a.to(dev), w.to(dev), out, m=m, n=N, k=K, batch=len(counts), w_batch=N * K, group_off=off.to(dev), exact=exact)
+    got = out.cpu()
+    for e, c in enumerate(counts):
+        rows, o = min(c, m), int(off[e])
+        A = a[o:o + rows].double() if exact else bf16(a[o:o + rows]).double()
+        assert close(got[o:o + rows], A @ w[e].double().T, K) and bool((got[o + rows:o + c] == 7).all()), e

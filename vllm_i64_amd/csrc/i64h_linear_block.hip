@@ -49,7 +49,7 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
         const int batches = p.group_off ? p.batch : 0;
         auto count = [&](int c) {
             const int e = c + lane;
-            int t = e < batches ? (p.group_off[e + 1] - p.group_off[e] + BM - 1) / BM : 0;
+            int t = e < batches ? (min(p.group_off[e + 1] - p.group_off[e], (int)p.M) + BM - 1) / BM : 0;
 #pragma unroll
             for (int d = 1; d < 64; d <<= 1) {
                 const int up = __shfl_up(t, d);
@@ -78,7 +78,7 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
             if (e > 0) mt -= __builtin_amdgcn_readlane(upto, e - 1);
             b = c + e;
             g0 = p.group_off[b];
-            rows = p.group_off[b + 1] - g0;
+            rows = min(p.M, p.group_off[b + 1] - g0);
             break;
         }
     }
