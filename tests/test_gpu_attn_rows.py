@@ -38,7 +38,8 @@ def reference(q, keys, values, pos, scale, window, keep, cap, sink):
     return torch.einsum("hnt,htv->nhv", torch.softmax(s, -1)[..., :-1], values.double())
 
 
-LENS = [([1, 15, 16, 17, 40], [0, 3, 0, 31, 0]), ([70], [0]), ([33, 2], [64, 5])]
+# (the last one: more portions in a tile of 64 rows than workgroups that they are dealt to)
+LENS = [([1, 15, 16, 17, 40], [0, 3, 0, 31, 0]), ([70], [0]), ([33, 2], [64, 5]), ([2, 1] * 40 + [70], [3, 40] * 40 + [0])]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
