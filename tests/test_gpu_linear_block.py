@@ -140,3 +140,22 @@ def test_no_more_rows_of_a_batch_than_the_launch_says(dev, use_form, form, m, ex
         rows, o = min(c, m), int(off[e])
         A = a[o:o + rows].double() if exact else bf16(a[o:o + rows]).double()
         assert close(got[o:o + rows], A @ w[e].double().T, K) and bool((got[o + rows:o + c] == 7).all()), e
+
+
+@pytest.mark.parametrize("M", [3, 64, 100])
+def test_a_weight_of_more_than_4_gib(dev, use_form, M):
+    """A tile's weights are addressed from the tile's first row: every column of a product whose weight does not fit 32-bit offsets."""
+    from vllm_i64_amd import ops_dense as D
+    use_form("by size")
+    N, K = 262400, 8192
+    g = torch.Generator().manual_seed(M)
+    a, row = torch.randn(M, K, generator=g), bf16(torch.randn(K, generator=g) / math.sqrt(K))
+    f = bf16(torch.arange(N) % 61 - 30)      # (row n of the weight: one row times a whole number)
+    w = torch.empty(N, K, dtype=torch.bfloat16, device=dev)
+    torch.mul(f.to(dev)[:, None], row.to(dev)[None, :], out=w)
+    out = torch.empty(M, N, device=dev)
+    D.linear(a.to(dev), w, out)
+    cols = torch.cat([torch.arange(0, N, 997), torch.arange(N - 70, N)])
+    ref = bf16(a).double() @ w[cols.to(dev)].cpu().double().T
+    # (terms up to 30 times those of `close`)
+    assert torch.allclose(out[:, cols.to(dev)].double().cpu(), ref, atol=30 * K ** 0.5 * 2e-6, rtol=2e-5)

@@ -87,7 +87,7 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
     const int M = (int)min((int64_t)BM, rows - (int64_t)mt * BM);
     const int lr = tid >> 3, lc = tid & 7;                 // staging: row within a pass, chunk of eight k
     // (rows past the end repeat the last one and are not stored)
-    const __amdgpu_buffer_rsrc_t bufA = dn_buffer(p.A + b * p.a_batch + (p.a_rows ? 0 : m0 * p.lda)), bufW = dn_buffer((const uint16_t*)p.W + b * p.w_batch);
+    const __amdgpu_buffer_rsrc_t bufA = dn_buffer(p.A + b * p.a_batch + (p.a_rows ? 0 : m0 * p.lda)), bufW = dn_buffer((const uint16_t*)p.W + b * p.w_batch + (int64_t)n0 * K);
     uint32_t oa[PA], ow[PB];
 #pragma unroll
     for (int i = 0; i < PA; ++i) {
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
         const int r = i * 32 + lr;
         // gate and up rows of the same columns go to the same wave: its first half of fragments, its second half
         const int c = DUAL ? (r / WN) * (WN / 2) + r % (WN / 2) : r;
-        ow[i] = (uint32_t)((int64_t)(min(n0 + c, N - 1) + (DUAL && r % WN >= WN / 2 ? N : 0)) * K + lc * CH) * 2u;
+        ow[i] = (uint32_t)((int64_t)(min(c, N - 1 - n0) + (DUAL && r % WN >= WN / 2 ? N : 0)) * K + lc * CH) * 2u;
     }
     dn_v4u ra[2][PA][2], rb[2][PB], rn[2][2];      // two steps on their way
     float ssq[PA];
@@ -316,9 +316,9 @@ static int64_t tiles(const i64h_linear& d, int BM, int BN) {
 
 bool dn_linear_block(const i64h_linear& d, int form, hipStream_t s) {
     const bool dual = dn_dual(d.epilogue);
-    // the buffer descriptors' 32-bit offsets: rows of a tile, or whatever a_rows may name; all of a batch's weights
+    // the buffer descriptors' 32-bit offsets: rows of a tile, or whatever a_rows may name; the weights of a tile, of a pair from gate to up
     const int64_t span = (d.a_rows ? d.a_height : 128) * d.lda * 4;
-    if ((d.a_rows && d.a_height <= 0) || span >= (int64_t)DN_BUF_END - 64 || (int64_t)d.N * (dual ? 4 : 2) * d.K >= (int64_t)DN_BUF_END - 64) return false;
+    if ((d.a_rows && d.a_height <= 0) || span >= (int64_t)DN_BUF_END - 64 || ((dual ? (int64_t)d.N : 0) + 128) * 2 * d.K >= (int64_t)DN_BUF_END - 64) return false;
     if (tiles(d, 16, 64) > 0x7fffffff) return false;
     // rows that share a batch's weights: taller tiles would only repeat the last one
     const int64_t tall = d.group_off && d.rows_total > 0 ? (d.rows_total + d.batch - 1) / d.batch : d.M;
