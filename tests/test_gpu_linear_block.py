@@ -159,3 +159,36 @@ def test_a_weight_of_more_than_4_gib(dev, use_form, M):
     ref = bf16(a).double() @ w[cols.to(dev)].cpu().double().T
     # (terms up to 30 times those of `close`)
     assert torch.allclose(out[:, cols.to(dev)].double().cpu(), ref, atol=30 * K ** 0.5 * 2e-6, rtol=2e-5)
+
+
+# sizes that take a large form by their rule: 128 x 128 tiles (at least 200), 64 x 128 (at least 250, and fewer than 200 of the former), the 64 x 64 tile kernel (short
+# k and many tiles, or k up to 32), 64-column tiles for narrow batches of many rows
+LARGE = {"128x128": (1700, 1990, 136, 1), "64x128": (1000, 1996, 200, 1), "short k": (1500, 1990, 128, 1), "k 24": (70, 1000, 24, 1), "narrow": (1100, 60, 264, 16)}
+
+
+@pytest.mark.parametrize("exact", [False, True])
+@pytest.mark.parametrize("epilogue", ["plain", "pair", "normed"])
+@pytest.mark.parametrize("size", LARGE)
+def test_large_forms_by_size(dev, use_form, size, epilogue, exact):
+    from vllm_i64_amd import ops_dense as D
+    use_form("by size")
+    M, N, K, H = LARGE[size]
+    if H > 1 and epilogue != "plain":
+        pytest.skip("batches of heads are plain products")
+    g = torch.Generator().manual_seed(M + N)
+    a, nw = torch.randn(M, H * K, generator=g), torch.rand(K, generator=g) + 0.5
+    w = bf16(torch.randn(H, (2 if epilogue == "pair" else 1) * N, K, generator=g) / math.sqrt(K))
+    out = torch.empty(M, H * N, device=dev)
+    kw = {"plain": {}, "pair": {"epilogue": D.EPI_SILU_MUL}, "normed": {"in_norm_w": nw.to(dev), "in_eps": 1e-6}}[epilogue]
+    D.linear(a.to(dev), w.to(dev), out, m=M, n=N, k=K, lda=H * K, ldc=H * N, batch=H, a_batch=K, w_batch=w[0].numel(), c_batch=N, exact=exact, **kw)
+    for h in range(H):
+        x = a[:, h * K:(h + 1) * K]
+        x = x * nw if epilogue == "normed" else x
+        ref = (x if exact else bf16(x)).double() @ w[h].double().T
+        got = out[:, h * N:(h + 1) * N]
+        if epilogue == "pair":
+            ref = ref[:, :N] * torch.sigmoid(ref[:, :N]) * ref[:, N:]
+            assert torch.allclose(got.double().cpu(), ref, atol=1e-4, rtol=1e-4)
+        else:
+            ref = ref / torch.sqrt(a.double().pow(2).mean(-1, keepdim=True) + 1e-6) if epilogue == "normed" else ref
+            assert close(got, ref, K)

@@ -322,6 +322,11 @@ bool dn_linear_block(const i64h_linear& d, int form, hipStream_t s) {
     if (tiles(d, 16, 64) > 0x7fffffff) return false;
     // rows that share a batch's weights: taller tiles would only repeat the last one
     const int64_t tall = d.group_off && d.rows_total > 0 ? (d.rows_total + d.batch - 1) / d.batch : d.M;
+    // Short k and many tiles: two steps of registers and LDS on their way are little use, and the plainer kernel's smaller workgroups overlap their loads and
+    // stores better.  Microseconds, here | there: 12000 x 4096 x 64 62 | 35, x 128 80 | 48, 4096 x 1024 x 128 11.1 | 9.7, 1000 x 4096 x 64 10.0 | 7.8, 320 x 4096 x 128 6.6 | 6.4, 1000 x
+    // 1024 x 128 5.2 | 5.7 (a gate / up pair: 2048 x 4096 x 128 25.3 | 23.3, 1000 x 4096 15.2 | 13.5, 1000 x 1024 6.2 | 8.4); 32-bit products 4096 x 1024 x 64 12.9 | 11.4,
+    // x 32 10.2 | 8.6, 512 x 1024 x 32 5.7 | 4.9.
+    auto short_k = [&](int64_t many, int k) { return (d.K <= 32 && !dual) || (d.K <= k && tiles(d, 64, 64) >= many); };
     if (d.exact) {
         // Bound by the matrix instructions, a sixteenth of the bf16 rate: what counts is that every CU works, then that few values are staged per
         // product.  Microseconds in replayed graphs, in front the 64 x 64 tile kernel with 32-wide steps:
@@ -334,6 +339,7 @@ bool dn_linear_block(const i64h_linear& d, int form, hipStream_t s) {
         //    376 x 2752 x 1024, pair              91      54       55                                  59
         //  8 x 10 x 896 x 1024, pair              66      26       22                                  17
         if (form < 0) {
+            if (!dual && short_k(1000, 64)) return false;
             if (dual) form = tiles(d, 16, 128) <= 256 ? 6 : (d.K >= 512 && tiles(d, 64, 64) <= 256 ? 3 : 2);
             else if (tall <= 16 || tiles(d, 16, 64) <= 256) form = 5;
             else if (tiles(d, 32, 64) <= 256) form = 4;
@@ -364,12 +370,13 @@ bool dn_linear_block(const i64h_linear& d, int form, hipStream_t s) {
         //     64 x 2048 x 2048                         15.1     12.3      9.6      8.3
         // Few rows under weights that take longer than everything else: 32 x 128 tiles, two groups (8 experts of 16 rows x 3584 x 2048: 24.4 us, in 128
         // x 128 tiles 33, in 64 x 64 30; 7 x 32000 x 1024 12.7, 64x64 13.4).
-        const bool longer = d.K > 128;
-        if (longer && tall > 64 && tiles(d, 128, 128) >= 200) form = 0;
-        else if (longer && tall > 32 && tiles(d, 64, 128) >= 250) form = 1;
+        const bool longer = d.K > 128, wide = (dual ? 2 * (int64_t)d.N : d.N) > 64;      // (half of a 128-column tile would be idle)
+        if (short_k(dual ? 2000 : 700, 128)) return false;
+        if (longer && wide && tall > 64 && tiles(d, 128, 128) >= 200) form = 0;
+        else if (longer && wide && tall > 32 && tiles(d, 64, 128) >= 250) form = 1;
         else if (dual ? tiles(d, 16, 128) <= 256 : tiles(d, 16, 64) <= 256) form = dual ? 6 : 5;
         else if (!dual && d.K >= 512 && tiles(d, 32, 64) <= 256) form = 4;
-        else if (d.K >= 512 && tall <= 32) form = 7;
+        else if (d.K >= 512 && wide && tall <= 32) form = 7;
         else if (d.K >= 512 && tiles(d, 64, 64) <= 256) form = 3;
         else form = 2;
     }
