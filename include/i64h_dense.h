@@ -47,10 +47,11 @@ int i64h_device_check(void);
  *   (of A itself without a_rows) and of C instead of all M rows; M is then the most rows any batch may have (it sizes the launch,
  *   workgroups past a batch's rows leave at once), and the launch needs no count on the host.  rows_total (0: unknown): a bound of
  *   group_off[batch], which makes the launch smaller.
- * a_height (0: unknown): the rows of A that a_rows may name; a launch with a_rows and without it takes the 64 x 64 tile form.
+ * a_height (0: unknown): the rows of A that a_rows may name; a launch with a_rows and without it takes the fragment-streaming form up to eight rows,
+ * the 64 x 64 tile form beyond.
  * Any M, N, K >= 1; 16-byte loads are used where strides and addresses allow, element loads otherwise.
  * Launches with M <= I64H_SKINNY_ROWS take a weight-streaming form (one wave per output column group); the form of the others follows from
- * their size (i64h_linear_block.hip). */
+ * their size (i64h_dense.hip for few rows, i64h_linear_block.hip). */
 #define I64H_EPI_STORE 0
 #define I64H_EPI_GELU_MUL 1
 #define I64H_EPI_MUL_SIGMOID 2

@@ -7,7 +7,8 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-FORMS = {"128x128": 1, "64x128 (32x64 in 32 bits)": 2, "64x64": 3, "64x64/2": 4, "32x64/4": 5, "16x64/4": 6, "16x128/2 pair": 7, "32x128/2": 8, "by size": 0}
+# (one more than the form of the block kernel; "rows": the fragment-streaming kernel for at most 64 rows, the block kernel by size beyond)
+FORMS = {"128x128": 1, "64x128 (32x64 in 32 bits)": 2, "64x64": 3, "64x64/2": 4, "32x64/4": 5, "16x64/4": 6, "16x128/2 pair": 7, "32x128/2": 8, "by size": 0, "rows": -1}
 
 
 @pytest.fixture(scope="module")
@@ -18,7 +19,7 @@ def dev():
 @pytest.fixture
 def use_form():
     from vllm_i64_amd import ops_dense as D
-    yield lambda name: D.call_dense("i64h_set_linear_skinny", 16 * FORMS[name] + 2 if FORMS[name] else 3)
+    yield lambda name: D.call_dense("i64h_set_linear_skinny", {-1: 4, 0: 3}.get(FORMS[name], 16 * FORMS[name]))
     D.call_dense("i64h_set_linear_skinny", 3)
 
 
@@ -192,3 +193,18 @@ def test_large_forms_by_size(dev, use_form, size, epilogue, exact):
         else:
             ref = ref / torch.sqrt(a.double().pow(2).mean(-1, keepdim=True) + 1e-6) if epilogue == "normed" else ref
             assert close(got, ref, K)
+
+
+@pytest.mark.parametrize("M", [3, 8, 9, 64])
+def test_gathered_rows_of_a_matrix_of_unknown_height(dev, use_form, M):
+    """A caller that does not say how many rows the list may name: 64-bit addresses."""
+    from vllm_i64_amd import _lib
+    from vllm_i64_amd import ops_dense as D
+    use_form("by size")
+    n, N, K = 300, 5000, 264
+    g = torch.Generator().manual_seed(M)
+    a, w, rows = torch.randn(n, K, generator=g), bf16(torch.randn(N, K, generator=g) / math.sqrt(K)), torch.randint(0, n, (M,), generator=g).to(torch.int32)
+    ad, wd, rd, out = a.to(dev), w.to(dev), rows.to(dev), torch.empty(M, N, device=dev)
+    d = _lib.Linear(A=D.ptr(ad), lda=K, a_rows=D.ptr(rd), W=D.ptr(wd), C=D.ptr(out), ldc=N, M=M, N=N, K=K, batch=1)
+    D.call_dense("i64h_linear_run", D._ref(d), D._stream())
+    assert close(out, bf16(a[rows.long()]).double() @ w.double().T, K)

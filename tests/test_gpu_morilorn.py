@@ -92,7 +92,7 @@ def test_linear_plain_and_epilogues(dev, exact, M, N, K):
     ad, wd, ed = a.to(dev), w.to(dev), e.to(dev)
     A = a[:, 2:2 + K].double() if exact else bf16(a[:, 2:2 + K]).double()
     tol = 1e-5 if exact else 2e-5   # both forms sum exact products in fp32
-    for skinny in (7, 1, 0):     # every kernel where it applies; rows <= 8 on their own kernel only; everything on the 64 x 64 tile kernel
+    for skinny in (7, 1, 0):     # one or two rows, and up to 64, on their own kernels; one or two only; everything on the 64 x 64 tile kernel
         D.call_dense("i64h_set_linear_skinny", skinny)
         out = torch.full((M, N + 4), 7.0, device=dev)
         D.linear(ad, wd, out, n=N, k=K, a_off=2, lda=K + 5, c_off=1, ldc=N + 4, exact=exact)
