@@ -65,3 +65,20 @@ def test_ties_masks_and_non_finite(V, k):
     assert draw(x, 0.0, k, 1.0, u).tolist() == [11] * 4      # greedy
     y = torch.randn(4, V)
     assert draw(y, 1.0, k, 0.9, torch.full((4,), -0.5)).tolist() == y.argmax(1).tolist()      # a draw below zero: the most likely token
+
+
+@pytest.mark.parametrize("V", [300, 40000])
+@pytest.mark.parametrize("k,p", [(0, 1.0), (0, 0.9), (600, 1.0)])
+@pytest.mark.parametrize("bits", [0x7fc00000, -0x400000, -1])
+def test_every_nan_counts(V, k, p, bits):
+    """Quiet NaNs of either sign, all bits set among them (the smallest value of the order that the kernel bisects in): kept, the sum is no number and the
+    first of the largest is drawn; top-k leaves a NaN with the sign bit out, as the smallest value, if there are enough others."""
+    x = torch.randn(4, V, generator=torch.Generator().manual_seed(V))
+    x.view(torch.int32)[:, 20] = bits
+    if 0 < k < V and bits < 0:
+        u = torch.tensor([0.0, 0.26, 0.51, 0.99])
+        clean = x.clone()
+        clean[:, 20] = -math.inf
+        check(clean, 1.0, k, p, u, draw(x, 1.0, k, p, u))
+    else:
+        assert draw(x, 1.0, k, p, torch.tensor([0.1, 0.5, 0.9, 0.33])).tolist() == x.nan_to_num(-1e9).argmax(1).tolist()

@@ -554,7 +554,7 @@ __global__ __launch_bounds__(SR_THREADS) void sample_rows_kernel(const float* __
     uint32_t key[NV > 0 ? NV : 1][4];
     float best = -INFINITY;
     int bi = V;
-    uint32_t kmax = 0;
+    uint32_t kmax = 0, kmin = ~0u;
     auto look = [&](int i, const uint32_t* k) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -563,6 +563,10 @@ __global__ __launch_bounds__(SR_THREADS) void sample_rows_kernel(const float* __
             if (c < V && (v > best || (v == best && c < bi))) best = v, bi = c;
             kmax = max(kmax, k[j]);
         }
+        if (i < V / STEP) kmin = min(min(min(k[0], k[1]), min(k[2], k[3])), kmin);
+        else
+#pragma unroll
+            for (int j = 0; j < 4; ++j) kmin = i * STEP + tid * 4 + j < V ? min(kmin, k[j]) : kmin;
     };
     if (NV > 0) {
 #pragma unroll
@@ -707,6 +711,10 @@ __global__ __launch_bounds__(SR_THREADS) void sample_rows_kernel(const float* __
             n = sum_i(n);
             return n == k ? 2 : (n > k ? 1 : 0);
         });
+    if (thr == 0u && sum_i(wave_count(kmin == 0u)) > 0) {      // the NaN of all bits set is kept: the sum is no number
+        if (tid == 0) out[r] = arg;
+        return;
+    }
     thr = max(thr, 1u);      // (0: the places past the end)
     auto mass = [&](uint32_t cut) {
         float s = 0.0f;
