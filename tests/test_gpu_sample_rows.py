@@ -82,3 +82,12 @@ def test_every_nan_counts(V, k, p, bits):
         check(clean, 1.0, k, p, u, draw(x, 1.0, k, p, u))
     else:
         assert draw(x, 1.0, k, p, torch.tensor([0.1, 0.5, 0.9, 0.33])).tolist() == x.nan_to_num(-1e9).argmax(1).tolist()
+
+
+@pytest.mark.parametrize("V", [130, 4095, 4096, 4097])
+@pytest.mark.parametrize("k", [128, 129])
+def test_draw_of_short_rows(V, k):
+    """Around the longest row of the four-wave form and the largest top-k that it lists."""
+    x = 2 * torch.randn(5, V, generator=torch.Generator().manual_seed(V + k))
+    u = torch.tensor([0.0, 0.1, 0.5, 0.95, 0.9999])
+    check(x, 0.8, k, 0.9, u, draw(x, 0.8, k, 0.9, u))

@@ -494,21 +494,21 @@ __global__ __launch_bounds__(256) void gated_postnorm_kernel(const i64h_postnorm
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
-// One workgroup of 16 waves per row.  Thresholds are found by bisection over the bits of the order-preserving integer image of a float:
+// One workgroup per row.  Thresholds are found by bisection over the bits of the order-preserving integer image of a float:
 // top-k: the largest key with at least k values at or above it; top-p: the largest key whose values at or above it hold at
 // least p of the mass.  The draw takes the first kept value, in index order, behind which the running sum exceeds u of the total.
 //
-// What bounds it is the chain of dependent block-wide sums, one per bit, so each is made short.  With top-k of at most 512 the row is read
-// once: the k-th largest of the threads' maxima is a bound that at least k values reach and few others do, those (at most 1024, sorted by
-// index) lie one to a thread from there on.  Without top-k the row's keys stay in registers (NV float4 per thread; NV = 0: read again,
+// What bounds it is the chain of dependent block-wide sums, one per bit, so each is made short.  With top-k of at most half as many as there are
+// threads the row is read once: the k-th largest of the threads' maxima is a bound that at least k values reach and few others do, those (at most one
+// a thread, sorted by index) lie one to a thread from there on.  Without top-k the row's keys stay in registers (NV float4 per thread; NV = 0: read again,
 // vocabularies beyond 32768).  64 rows of 32000, top-k 50 and top-p 0.95: 1280 us with four
-// waves that read the row again for every bit, 34 us now.
-constexpr int SR_WAVES = 16, SR_THREADS = 64 * SR_WAVES, SR_LIST = SR_THREADS, SR_TOPK = 512;
-
-template <int NV>
-__global__ __launch_bounds__(SR_THREADS) void sample_rows_kernel(const float* __restrict__ logits, int64_t* __restrict__ out, int V, const int vec,
+// waves that read the row again for every bit, 35 us with sixteen.  Up to 4096 values four waves have the shorter sums: 64 rows of 1000 drawn without
+// top-k 11 us, sixteen waves 16, rows of 4000 13 and 17.
+template <int NV, int SR_WAVES>
+__global__ __launch_bounds__(64 * SR_WAVES) void sample_rows_kernel(const float* __restrict__ logits, int64_t* __restrict__ out, int V, const int vec,
                                                                  const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
                                                                  const float* __restrict__ top_p, const float* __restrict__ u) {
+    constexpr int SR_THREADS = 64 * SR_WAVES, SR_LIST = SR_THREADS, SR_TOPK = SR_LIST / 2;
     __shared__ float redf[2][SR_WAVES];
     __shared__ int redi[2][SR_WAVES], bestc[SR_WAVES];
     __shared__ float bestv[SR_WAVES];
@@ -939,10 +939,10 @@ int i64h_sample_rows(const float* logits, int64_t* out, int64_t rows, int32_t V,
     if (rows == 0) return 0;
     const int vec = (uintptr_t)logits % 16 == 0 && V % 4 == 0;
     hipStream_t s = (hipStream_t)stream;
-    if (V <= 8 * 4 * SR_THREADS)
-        hipLaunchKernelGGL((sample_rows_kernel<8>), dim3((unsigned)rows), dim3(SR_THREADS), 0, s, logits, out, (int)V, vec, temperature, top_k, top_p, u);
-    else
-        hipLaunchKernelGGL((sample_rows_kernel<0>), dim3((unsigned)rows), dim3(SR_THREADS), 0, s, logits, out, (int)V, vec, temperature, top_k, top_p, u);
+    auto launch = [&](auto kern, int threads) { hipLaunchKernelGGL(kern, dim3((unsigned)rows), dim3(threads), 0, s, logits, out, (int)V, vec, temperature, top_k, top_p, u); };
+    if (V <= 4096) launch(sample_rows_kernel<4, 4>, 256);
+    else if (V <= 32768) launch(sample_rows_kernel<8, 16>, 1024);
+    else launch(sample_rows_kernel<0, 16>, 1024);
     I64H_CHECK_LAUNCH();
     return 0;
 }
