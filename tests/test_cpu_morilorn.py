@@ -146,3 +146,17 @@ def test_scores_and_values_through_latent_space_equal_the_written_out_form():
         assert torch.allclose(s, s2)
         wgt = torch.softmax(s, -1)
         assert torch.allclose(wgt @ val[:, h], (wgt @ c) @ uv[h * v:(h + 1) * v].T)
+
+
+def test_gathered_rows_count_a_last_row_that_ends_with_the_buffer(monkeypatch):
+    """The height that a Linear over gathered rows states bounds the offsets of its loads: a last row shorter than the row stride is one of the rows."""
+    from vllm_i64_amd import ops_dense as D
+    seen = []
+    monkeypatch.setattr(D, "_chk", lambda *a: None)
+    monkeypatch.setattr(D, "_stream", lambda: 0)
+    monkeypatch.setattr(D, "ptr", lambda t: 0)
+    monkeypatch.setattr(D, "call_dense", lambda name, d, stream: seen.append(d._obj.a_height))
+    w, rows, out = torch.zeros(4, 8, dtype=torch.bfloat16), torch.tensor([2, 0], dtype=torch.int32), torch.zeros(2, 4)
+    for size in (48, 45, 42, 32):      # three rows of stride 16, the last one whole, cut, just k values long; two rows
+        D.linear(torch.zeros(size), w, out, n=4, k=8, a_off=2, lda=16, a_rows=rows)
+    assert seen == [3, 3, 3, 2]

@@ -76,7 +76,7 @@ def linear(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, m: Optional[i
                     bias=ptr(bias), bias_batch=int(bias_batch), scale=float(scale), act_a=float(act_a), act_b=float(act_b), group_off=ptr(group_off),
                     row_scale=ptr(row_scale), in_norm_w=ptr(in_norm_w), in_eps=float(in_eps),
                     rows_total=min((a_rows.numel() if a_rows is not None else a.numel() // lda), out.numel() // ldc) if group_off is not None else 0,
-                    a_height=a.numel() // lda if a_rows is not None else 0)
+                    a_height=-(-a.numel() // lda) if a_rows is not None else 0)
     call_dense("i64h_linear_run", _ref(d), _stream())
     return out
 
