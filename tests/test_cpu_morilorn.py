@@ -155,7 +155,8 @@ def test_gathered_rows_count_a_last_row_that_ends_with_the_buffer(monkeypatch):
     monkeypatch.setattr(D, "_chk", lambda *a: None)
     monkeypatch.setattr(D, "_stream", lambda: 0)
     monkeypatch.setattr(D, "ptr", lambda t: 0)
-    monkeypatch.setattr(D, "call_dense", lambda name, d, stream: seen.append(d._obj.a_height))
+    monkeypatch.setattr(D, "_ref", lambda d: d)
+    monkeypatch.setattr(D, "call_dense", lambda name, d, stream: seen.append(d.a_height))
     w, rows, out = torch.zeros(4, 8, dtype=torch.bfloat16), torch.tensor([2, 0], dtype=torch.int32), torch.zeros(2, 4)
     for size in (48, 45, 42, 32):      # three rows of stride 16, the last one whole, cut, just k values long; two rows
         D.linear(torch.zeros(size), w, out, n=4, k=8, a_off=2, lda=16, a_rows=rows)
