@@ -199,7 +199,7 @@ typedef struct {
     float softcap;       /* > 0: a score s (after scale and key scale, before any bias) becomes softcap * tanh(s / softcap) */
     int32_t keep_first;  /* with a window: the first positions of a sequence that stay visible to everyone */
 } i64h_latent_attn_args;
-int i64h_set_latent_attn_decode_form(int32_t on); /* tuning / test knob: 1 (default) = mode 2 launches run the kernel that requests a tile's fragments a tile ahead; 0 = a plainer kernel with the same tiles; same results up to summation order */
+int i64h_set_latent_attn_decode_form(int32_t on); /* tuning / test knob: 1 (default) = mode 0 / 2 launches over bf16 caches of fitting sizes take the matrix-core form; 0 = all of them take the row form */
 int64_t i64h_latent_attn_workspace_floats(int64_t n, int32_t heads, int32_t kv_rank, int32_t splits);
 int i64h_latent_attn(const i64h_latent_attn_args* d, void* stream);
 
@@ -419,9 +419,10 @@ typedef struct {
     float* out;
     int64_t n;
     int32_t heads, kv_heads, dim;
-    int32_t mode;        /* 1: one wave per (row, head), fp32 products, any sizes and cache type; otherwise, where the cache is bf16 and dim % 16 == 0
-                            and <= 256, the matrix-core kernel of the latent attention: 3 a wave per 16 consecutive rows and head (portions of
-                            prompts), 0 / 2 a wave per token and 16 query heads of one key head (rows that are one per sequence) */
+    int32_t mode;        /* 1: one wave per (row, head), fp32 products, any sizes and cache type; otherwise, where the cache is bf16 and the values of a key
+                          * head (vdim, or dim without it) % 16 == 0 and <= 256, the whole row part % 8 == 0 and <= 320: 2 (and 0) one wave per token and 16
+                          * heads of a key head, 3 four waves of 16 consecutive rows and a head each that share a key head's tiles (portions of prompts);
+                          * 3 over a 32-bit cache of such sizes (% 4) the same on 32-bit matrix products */
     int32_t splits;      /* mode 0 / 2: every token's keys are dealt to this many waves and merged by a second launch */
     float* workspace;    /* i64h_kattn_workspace_floats(n, heads, kv_heads, dim, splits) floats when splits > 1 */
     int32_t vdim;        /* > 0: keys and values are separate (see i64h_kv_prep): a cached row holds per key head [vdim values | dim key values], Q is

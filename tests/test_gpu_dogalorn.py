@@ -414,7 +414,7 @@ def test_key_attention_matrix_core_form(dev, H, G, d, chunk, block, cut_sizes):
     from vllm_i64_amd import ops_dense as D
     from vllm_i64_amd.dogalorn import distance_bias_table
     bias = distance_bias_table(w["rel"], 30.0).to(dev)
-    # single rows: the kernel that requests its tiles ahead (1), and the general kernel with a token's heads per wave (0)
+    # single rows: the matrix-core form (1), and a wave per row and head (0)
     for single_row_form in ((1, 0) if 1 in cut_sizes else (1,)):
         D.call_dense("i64h_set_latent_attn_decode_form", single_row_form)
         try:

@@ -311,7 +311,7 @@ def test_latent_attn_keys_dealt_to_several_waves(dev, H, r, e):
     pos = torch.tensor([t - 1 for t in lens], dtype=torch.int32)
     for window in (0, 100):
         ref = torch.cat([_ref_attn(Q[i:i + 1], rows_of[i], [lens[i] - 1], window, 0.4, r) for i in range(4)])
-        for form in (1, 0):      # the kernel that requests its fragments a tile ahead, and the general matrix-core kernel
+        for form in (1, 0):      # the matrix-core form, and a wave per row and head
             D.call_dense("i64h_set_latent_attn_decode_form", form)
             for splits in (1, 2, 5, 64):
                 out = torch.empty(4, H, r, device=dev)

@@ -6,9 +6,8 @@
 //   latent_prep_kernel     : RMS norm of the latent, rotation of the shared key part and of every head's rotated query part,
 //                            cache write - one workgroup per token
 //   latent_attn_rows_kernel: bf16 caches of aligned widths, portions of prompts - four waves of 16 rows that share 32 keys at a time through LDS;
-//                            latent_attn_rows_f32_kernel: the same for 32-bit caches, 32-bit products (latent_row in both where a value is no finite number
-//   latent_attn_mfma_decode_kernel (latent_attn_mfma_kernel): rows that are one per sequence - a token's heads, 16 query vectors per wave;
-//                            both on the bf16 matrix cores, see below
+//                            latent_attn_rows_f32_kernel: the same for 32-bit caches, 32-bit products (latent_row in both where a value is no finite number)
+//   latent_attn_mfma_decode_kernel: the same caches, rows that are one per sequence - a token's heads, 16 query vectors per wave
 //   latent_attn_row_kernel : any width and cache type, true fp32 products: one wave per (token, head): 64 keys at a time, one key per lane for the scores (fp32 dot over the
 //                            cached row), online softmax over the wave, weighted row sum with the columns spread over the lanes
 #include "i64h_common.h"
@@ -155,13 +154,6 @@ __global__ __launch_bounds__(256) void latent_attn_row_kernel(const i64h_latent_
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
-// Matrix-core form (bf16 cache) of rows that are one per sequence.  One wave per task of 16 query vectors that walk the same cached rows:
-// the (up to) 16 heads of a group of one token.  (Behind the decode-form knob; the arrangement that such launches take is below it.)
-// Per tile of 32 keys: scores S[16, 32] = Q K^T on v_mfma_f32_16x16x32_bf16 with the cached rows read straight from memory as B
-// fragments (8 consecutive values of one key per lane) and the scaled query carried as TWO bf16 terms (hi + lo, 16 mantissa bits),
-// masking and the online softmax in fp32 on the accumulator layout, the weights again as two bf16 terms through LDS into the
-// A layout, the tile's latent columns transposed through LDS (4 keys x 8 columns per lane and pass, 8-byte writes) into the B
-// layout of the second product, out[16, kv_rank] += P V in fp32.  Every product of two bf16 values is exact in fp32.
 #define LT_KD 10   // 32-wide steps over a cached row: kv_rank + rot_dim <= 320
 #define LT_NB 16   // 16-column blocks of the output: kv_rank <= 256
 #define LT_VLD 40  // halves per row of the transposed tile and of the weight planes (32 keys + 8: 16-byte aligned, conflict-poor)
@@ -176,211 +168,19 @@ __device__ __forceinline__ void lt_split(float x, uint32_t& hi, uint32_t& lo) {
     lo = lt_rne(x - __uint_as_float(hi << 16));
 }
 
-// KD, NB: 32-wide steps over a cached row and 16-column blocks of the output that an instance holds registers for (rows of at most
-// 32 KD values, kv_rank <= 16 NB): the widest instance keeps two waves per SIMD, narrow rows leave room for more.
-template <int KD, int NB>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, KD > 4 ? 2 : 8))) void latent_attn_mfma_kernel(const i64h_latent_attn_args p, const int splits) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    const int lane = threadIdx.x, n = lane & 15, kg = lane >> 4;
-    const int r = p.kv_rank, D = r + p.rot_dim, H = p.heads, bs = p.block_size, win = p.window;
-    const int keep = p.chunk <= 0 && win > 0 ? p.keep_first : 0;
-    uint16_t* Vt = (uint16_t*)smem;           // [r][LT_VLD]
-    uint16_t* Ph = Vt + r * LT_VLD;           // [16][LT_VLD]
-    uint16_t* Pl = Ph + 16 * LT_VLD;
-    int* info = (int*)(Pl + 16 * LT_VLD);     // [16] positions, [16] slots (-1: no such row), [32] cache rows of the tile's keys
-    int* rowoff = info + 32;
-    const int64_t task = blockIdx.x;
-    const int split = blockIdx.y;
-    // key heads side by side in a cached row (key-valued attention): a head tile takes 16 of the rep query heads of ONE key head
-    const int G = p.kv_groups > 1 ? p.kv_groups : 1, rep = H / G, tpg = (rep + 15) / 16;
-    const int hgroups = G * tpg;
-    const int rstride = p.row_stride > 0 ? p.row_stride : D;
-    const int coff = (int)(task % hgroups) / tpg * D;
-    const int hbase = ((int)(task % hgroups) / tpg) * rep + ((int)(task % hgroups) % tpg) * 16;
-    auto row_of = [&](int m, int64_t& tok, int& head) -> bool {
-        tok = task / hgroups;
-        head = hbase + m;
-        return ((int)(task % hgroups) % tpg) * 16 + m < rep;
-    };
-    int64_t tok_n;
-    int head_n;
-    const bool valid_n = row_of(n, tok_n, head_n);
-    if (lane < 16) {
-        info[lane] = valid_n ? p.positions[tok_n] : -1;
-        info[16 + lane] = valid_n ? p.slot_ids[tok_n] : -1;
-    }
-    // the query of row n times scale * log2(e) (the softmax runs on powers of two), columns ks * 32 + kg * 8 .. + 7, as two bf16 terms
-    uint4 Qh[KD], Ql[KD];
-    {
-        const float* q = p.Q + (tok_n * H + head_n) * D;
-        const float qs = p.scale * 1.4426950408889634f;
-#pragma unroll
-        for (int ks = 0; ks < KD; ++ks) {
-            const int d0 = ks * 32 + kg * 8;
-            uint32_t h[8], l[8];
-            if (valid_n && d0 < D) {
-                const float4 a = *(const float4*)(q + d0), b = *(const float4*)(q + d0 + 4);
-                const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-                for (int i = 0; i < 8; ++i) lt_split(v[i] * qs, h[i], l[i]);
-            } else {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) h[i] = l[i] = 0;
-            }
-            Qh[ks] = make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16));
-            Ql[ks] = make_uint4(l[0] | (l[1] << 16), l[2] | (l[3] << 16), l[4] | (l[5] << 16), l[6] | (l[7] << 16));
-        }
-    }
-    lt_v4f acc[NB];
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) acc[nb] = lt_v4f{0, 0, 0, 0};
-    float mrow[4], lrow[4];
-    int lor[4], hrow[4];   // per row of the tile: the first position it sees, its head (for the bias table)
-    const bool sink = p.sink && split == 0;     // the extra score of zero counts once: in the first share of the keys
-    __syncthreads();
-    const float capl = p.softcap * 1.4426950408889634f;     // the cap in the units of the scores (powers of two)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        const int pp = info[kg * 4 + g];
-        lor[g] = p.chunk > 0 ? (max(pp, 0) / p.chunk) * p.chunk : (win > 0 ? max(0, pp - win + 1) : 0);
-        hrow[g] = min(hbase + kg * 4 + g, H - 1);
-        mrow[g] = sink ? (p.sink_w ? p.sink_w[hrow[g]] * 1.4426950408889634f : 0.0f) : -INFINITY;
-        lrow[g] = sink ? 1.0f : 0.0f;
-    }
-    const uint16_t* cache = (const uint16_t*)p.cache;
-    int s0 = 0;
-    while (s0 < 16) {
-        const int sl = info[16 + s0];
-        if (sl < 0) {
-            ++s0;
-            continue;
-        }
-        int s1 = s0 + 1;
-        while (s1 < 16 && info[16 + s1] == sl) ++s1;
-        int lo = 0x7fffffff, hi = -1;
-        for (int i = s0; i < s1; ++i) {
-            const int pp = info[i];
-            hi = max(hi, pp);
-            lo = min(lo, p.chunk > 0 ? (pp / p.chunk) * p.chunk : (win > 0 ? max(0, pp - win + 1) : 0));
-        }
-        const int32_t* bt = p.block_table + (int64_t)sl * p.max_blocks_per_seq;
-        // tiles of 32 keys: those of the kept first positions that lie in front of the window's first tile, then the window's
-        const int t0 = lo >> 5, kt = min((keep + 31) >> 5, t0), tiles = kt + (hi >> 5) - t0 + 1;
-        for (int tile = split; tile < tiles; tile += splits) {
-            const int kb = (tile < kt ? tile : t0 + tile - kt) * 32;
-            if (lane < 32) {
-                const int jc = min(kb + lane, hi);
-                rowoff[lane] = bt[jc / bs] * bs + jc % bs;
-            }
-            __syncthreads();
-            lt_v4f S[2];
-            float ksc[2] = {1.0f, 1.0f};
-            if (p.kscale) {
-                ksc[0] = p.kscale[rowoff[n]];
-                ksc[1] = p.kscale[rowoff[16 + n]];
-            }
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                S[b] = lt_v4f{0, 0, 0, 0};
-                const uint16_t* rowp = cache + (int64_t)rowoff[16 * b + n] * rstride + coff;
-#pragma unroll
-                for (int ks = 0; ks < KD; ++ks) {
-                    if (ks * 32 < D) {
-                        const int d0 = ks * 32 + kg * 8;
-                        const uint4 kf = d0 < D ? *(const uint4*)(rowp + d0) : make_uint4(0, 0, 0, 0);
-                        if ((ks + 1) * 32 > p.key_off) {     // (a step of value-only columns: the query is zero there)
-                            S[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lt_v8bf, Qh[ks]), __builtin_bit_cast(lt_v8bf, kf), S[b], 0, 0, 0);
-                            S[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lt_v8bf, Ql[ks]), __builtin_bit_cast(lt_v8bf, kf), S[b], 0, 0, 0);
-                        }
-                        if (d0 < r) {   // the same registers, transposed, are the second product's operand: column d0 + c of key 16 b + n
-                            const uint32_t kw[4] = {kf.x, kf.y, kf.z, kf.w};
-#pragma unroll
-                            for (int c = 0; c < 8; ++c) Vt[(d0 + c) * LT_VLD + 16 * b + n] = (uint16_t)(kw[c >> 1] >> (16 * (c & 1)));
-                        }
-                    }
-                }
-            }
-            float al[4];
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int rr = kg * 4 + g;
-                const int pr = info[rr];
-                const bool in_run = rr >= s0 && rr < s1;
-                float sv[2];
-#pragma unroll
-                for (int b = 0; b < 2; ++b) {
-                    const int j = kb + 16 * b + n;
-                    const bool vis = in_run && j <= pr && (j >= lor[g] || j < keep);
-                    float sc = S[b][g] * ksc[b];
-                    if (capl > 0.0f) sc = capl * tanhf(sc / capl);
-                    if (p.bias) sc += 1.4426950408889634f * p.bias[(int64_t)min(max(pr - j, 0), p.bias_rows - 1) * H + hrow[g]];
-                    sv[b] = vis ? sc : -INFINITY;
-                }
-                const float mx = row16_max(fmaxf(sv[0], sv[1]));
-                const float mn = fmaxf(mrow[g], mx);
-                const float ms = mn == -INFINITY ? 0.0f : mn;
-                al[g] = __builtin_amdgcn_exp2f(mrow[g] - ms);
-                const float p0 = __builtin_amdgcn_exp2f(sv[0] - ms), p1 = __builtin_amdgcn_exp2f(sv[1] - ms);
-                lrow[g] = lrow[g] * al[g] + group_sum(p0 + p1, 16);
-                mrow[g] = mn;
-                uint32_t h0, l0, h1, l1;
-                lt_split(p0, h0, l0);
-                lt_split(p1, h1, l1);
-                Ph[rr * LT_VLD + n] = (uint16_t)h0;
-                Pl[rr * LT_VLD + n] = (uint16_t)l0;
-                Ph[rr * LT_VLD + 16 + n] = (uint16_t)h1;
-                Pl[rr * LT_VLD + 16 + n] = (uint16_t)l1;
-            }
-            __syncthreads();
-            const uint4 pah = *(const uint4*)&Ph[n * LT_VLD + kg * 8], pal = *(const uint4*)&Pl[n * LT_VLD + kg * 8];
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                if (nb * 16 < r) {
-                    const uint4 vf = *(const uint4*)&Vt[(nb * 16 + n) * LT_VLD + kg * 8];
-#pragma unroll
-                    for (int g = 0; g < 4; ++g) acc[nb][g] *= al[g];
-                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lt_v8bf, pah), __builtin_bit_cast(lt_v8bf, vf), acc[nb], 0, 0, 0);
-                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lt_v8bf, pal), __builtin_bit_cast(lt_v8bf, vf), acc[nb], 0, 0, 0);
-                }
-            }
-            __syncthreads();
-        }
-        s0 = s1;
-    }
-    if (splits > 1) {
-        // partial result of this share of the keys: [16 rows][kv_rank unnormalised sums | maximum (log2 units) | sum of weights]
-        float* w = p.workspace + ((int64_t)task * splits + split) * 16 * (r + 2);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            float* o = w + (kg * 4 + g) * (r + 2);
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-                if (nb * 16 < r) o[nb * 16 + n] = acc[nb][g];
-            if (n == 0) {
-                o[r] = mrow[g];
-                o[r + 1] = lrow[g];
-            }
-        }
-        return;
-    }
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        int64_t tok;
-        int head;
-        if (!row_of(kg * 4 + g, tok, head)) continue;
-        float* o = p.out + (tok * H + head) * r;
-        const float inv = 1.0f / lrow[g];
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-            if (nb * 16 < r) o[nb * 16 + n] = acc[nb][g] * inv;
-    }
-}
-
-// The same products for rows that are one per sequence (every wave: one token, 16 heads, a share of the keys), arranged around the
-// memory latency that dominates such launches: a tile's 18 fragment loads are requested together, the NEXT tile's are requested as
-// soon as this tile's scores and transposed columns are done - under its softmax and second product - and the cache rows of the tile
+// Matrix-core form (bf16 cache) of rows that are one per sequence.  One wave per task of 16 query vectors that walk the same cached rows: the (up to) 16
+// heads of a group of one token, a share of its keys.
+// Per tile of 32 keys: scores S[16, 32] = Q K^T on v_mfma_f32_16x16x32_bf16 with the cached rows read straight from memory as B
+// fragments (8 consecutive values of one key per lane) and the scaled query carried as TWO bf16 terms (hi + lo, 16 mantissa bits),
+// masking and the online softmax in fp32 on the accumulator layout, the weights again as two bf16 terms through LDS into the
+// A layout, the tile's latent columns transposed through LDS (8 two-byte writes per fragment) into the B
+// layout of the second product, out[16, kv_rank] += P V in fp32.  Every product of two bf16 values is exact in fp32.
+// Arranged around the memory latency that dominates such launches: a tile's 18 fragment loads are requested together, the NEXT tile's are
+// requested as soon as this tile's scores and transposed columns are done - under its softmax and second product - and the cache rows of the tile
 // after that are looked up a tile ahead.  The workgroup is one wave, so LDS traffic needs program order only (no barrier, whose
 // fence would wait for the loads in flight).  Registers: a whole SIMD's (one wave per SIMD is all such a launch has anyway).
+// KD, NB: 32-wide steps over a cached row and 16-column blocks of the output that an instance holds registers for (rows of at most
+// 32 KD values, kv_rank <= 16 NB).
 template <int KD, int NB>
 __global__ __launch_bounds__(64) void latent_attn_mfma_decode_kernel(const i64h_latent_attn_args p, const int splits) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -1195,6 +995,9 @@ int latent_rows_f32_run(const i64h_latent_attn_args& d, void* stream) {
     return 0;
 }
 
+static int g_decode_form = 1;
+bool latent_decode_form() { return g_decode_form; }
+
 extern "C" {
 
 int i64h_latent_prep(const i64h_latent_prep_args* dp, void* stream) {
@@ -1210,8 +1013,7 @@ int i64h_latent_prep(const i64h_latent_prep_args* dp, void* stream) {
     return 0;
 }
 
-static int g_decode_form = 1;
-int i64h_set_latent_attn_decode_form(int32_t on) {  // tuning / test knob: 0 = rows that are one per sequence on the general matrix-core kernel
+int i64h_set_latent_attn_decode_form(int32_t on) {  // tuning / test knob: 0 = rows that are one per sequence by a wave per row and head, 32-bit products
     g_decode_form = on;
     return 0;
 }
@@ -1232,7 +1034,7 @@ int i64h_latent_attn(const i64h_latent_attn_args* dp, void* stream) {
     if (d.n == 0) return 0;
     const int D = d.kv_rank + d.rot_dim;
     const bool mfma_ok = d.cache_dtype == 2 && D % 8 == 0 && d.kv_rank % 16 == 0 && d.kv_rank <= 16 * LT_NB && D <= 32 * LT_KD &&
-                         (uintptr_t)d.Q % 16 == 0 && (uintptr_t)d.cache % 16 == 0 && d.row_stride % 8 == 0;
+                         (uintptr_t)d.Q % 16 == 0 && (uintptr_t)d.cache % 16 == 0 && d.row_stride % 8 == 0 && (d.mode == 3 || g_decode_form);
     I64H_CHECK_ARG(mfma_ok || (d.kv_groups <= 1 && d.row_stride <= 0 && d.chunk <= 0 && !d.kscale && !d.bias),
                    "latent_attn: key heads, chunks, key scales and bias are built for the matrix-core form only");
     I64H_CHECK_ARG(!d.sink_w || d.sink, "latent_attn: sink scores without the sink");
@@ -1263,10 +1065,6 @@ int i64h_latent_attn(const i64h_latent_attn_args* dp, void* stream) {
             else if (steps <= 9) LT_ROWS(9, LT_NB);
             else LT_ROWS(LT_KD, LT_NB);
 #undef LT_ROWS
-        } else if (!g_decode_form) {
-            if (size == 0) hipLaunchKernelGGL((latent_attn_mfma_kernel<2, 4>), grid, dim3(64), bytes, st, d, splits);
-            else if (size == 1) hipLaunchKernelGGL((latent_attn_mfma_kernel<4, 8>), grid, dim3(64), bytes, st, d, splits);
-            else hipLaunchKernelGGL((latent_attn_mfma_kernel<LT_KD, LT_NB>), grid, dim3(64), bytes, st, d, splits);
         } else {
             if (size == 0) hipLaunchKernelGGL((latent_attn_mfma_decode_kernel<2, 4>), grid, dim3(64), bytes, st, d, splits);
             else if (size == 1) hipLaunchKernelGGL((latent_attn_mfma_decode_kernel<4, 8>), grid, dim3(64), bytes, st, d, splits);
