@@ -217,7 +217,7 @@ __global__ __launch_bounds__(256) void gdn_scan_kernel(const i64h_gdn_args p, co
 // tile have the arithmetic of a whole tile to arrive, and the waves read 16 bytes per lane from LDS one token ahead.  Needs 16-byte rows.
 // What bounds it is the chain from token to token - decay, row sum, correction - and the reads of the tile: the 16 tokens of a tile are one
 // stretch of code without a branch, so that a token's read-out runs beside the next one's sums, its result waiting in a lane until
-// the tile's end; 16 heads of 128, one run of 1531 rows: 339 -> 246 us (218 -> 160 ns a token), linear attention 283 -> 216 us.
+// the tile's end; 16 heads of 128, one run of 1531 rows: 334 -> 245 us (218 -> 160 ns a token), linear attention, 1500 rows, 278 -> 213 us.
 template <int KPT, int CPT, bool CHD, int RULE>
 __global__ __launch_bounds__(256) void gdn_tile_kernel(const i64h_gdn_args p, const int ctiles) {
     static_assert(KPT % 4 == 0, "whole 16-byte slices per lane");
@@ -658,9 +658,10 @@ static int gdn_launch(const i64h_gdn_args& d, void* stream) {
     const int kround = kpt <= 4 ? 4 : (kpt <= 8 ? 8 : 16);
     if (g_gdn_form != 1 && vec_ok(kround) && (g_gdn_form > 1 || d.n >= 8 * (int64_t)d.nseg)) {
         // One value column per lane: a token then takes the longest run least time, and it is the longest run that the launch waits for (16
-        // heads of 128, runs of 1531, 257, 64, 3 and 1101 rows: 275 us, two columns 449; 27 single rows beside 229 and 256: 67 and 99).  Two
-        // columns (fewer reads of the tile) only where many workgroups wait for a CU and the runs are long (32 runs of 128 rows: 212 and 215 us,
-        // linear attention 163 and 177; 8 of 512: 210 and 222).
+        // heads of 128, runs of 1531, 257, 64, 3 and 1101 rows: 264 us, two columns 448; 27 single rows beside 229 and 256: 68 and 100).  Two
+        // columns (fewer reads of the tile) only where many workgroups wait for a CU and the runs are long (8 runs of 512 rows: 220 and 199 us, 32 of 128
+        // 212 and 203, 64 of 64 rows and 32 heads 419 and 389).  Short runs in such numbers would rather have two (64 of 17: 70 and 66), but are not to be
+        // told from single rows beside a prompt by their count.
         const int cpt = g_gdn_form > 1 ? (g_gdn_form == 4 ? 4 : g_gdn_form - 1) : ((int64_t)d.heads * ((d.vdim + 15) / 16) * d.nseg >= 1024 && d.n >= 64 * (int64_t)d.nseg ? 2 : 1);
         const int ctiles = (d.vdim + 16 * cpt - 1) / (16 * cpt);
         const dim3 grid((unsigned)(d.heads * ctiles), (unsigned)d.nseg);
