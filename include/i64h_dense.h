@@ -49,6 +49,10 @@ int i64h_device_check(void);
  *   group_off[batch], which makes the launch smaller.
  * a_height (0: unknown): the rows of A that a_rows may name; a launch with a_rows and without it takes the fragment-streaming form up to eight rows,
  * the 64 x 64 tile form beyond.
+ * A16 (may be NULL; exact = 0): A's rows rounded to bf16 by whoever wrote them, strides as A's; they are read in A's place and A may be NULL.  Such a
+ * launch needs K a multiple of 64, 16-byte aligned rows (lda, a_batch, w_batch multiples of eight) and
+ * I64H_EPI_STORE, I64H_EPI_SCALE, I64H_EPI_ADD or one of the gate / up epilogues; its products are those of A.
+ * C16 (may be NULL; with A16): the results rounded to bf16, strides as C's, beside C or (C = NULL) in its place.
  * Any M, N, K >= 1; 16-byte loads are used where strides and addresses allow, element loads otherwise.
  * Launches with M <= I64H_SKINNY_ROWS take a weight-streaming form (one wave per output column group); the form of the others follows from
  * their size (i64h_dense.hip for few rows, i64h_linear_block.hip). */
@@ -92,6 +96,8 @@ typedef struct {
     const float* in_norm_w;
     float in_eps;
     int64_t rows_total, a_height;
+    const void* A16;
+    void* C16;
 } i64h_linear;
 int i64h_linear_run(const i64h_linear* d, void* stream);
 
@@ -245,7 +251,8 @@ int i64h_embed_bigram(const i64h_embed_bigram_args* d, void* stream);
  *   read  (h != NULL):  u = sum_s in_w[s] * x_s  (in_w == NULL: the plain sum);  h = u / sqrt(mean(u^2) + eps) * norm_w[c % norm_w_len],
  *                       or with h_center the centred norm (u - mean) / sqrt(mean((u - mean)^2) + eps) * norm_w;  norm_b (may be NULL, [W])
  *                       is added behind the weight
- * rows (may be NULL, read only launches): h[m] is computed from row rows[m] of the streams (the rows whose logits are wanted). */
+ * rows (may be NULL, read only launches): h[m] is computed from row rows[m] of the streams (the rows whose logits are wanted).
+ * h16 (may be NULL): the rows of h rounded to bf16 [n, W] (or [m_rows, W]), beside h or (h = NULL) in its place. */
 typedef struct {
     float* streams;
     int32_t S;
@@ -272,6 +279,7 @@ typedef struct {
     int32_t h_center;
     const float* norm_b;
     const float* y_scale;
+    void* h16;
 } i64h_streams_args;
 int i64h_streams_step(const i64h_streams_args* d, void* stream);
 int i64h_set_residual_form(int32_t on); /* tuning / test knob: 1 (default) = one stream and results without norms of their own take the kernel that keeps the row in registers (16-byte rows) */
@@ -331,7 +339,8 @@ int i64h_ssm_scan(const i64h_ssm_scan_args* d, void* stream);
 /* out[t, :] = rms_groups(y[t, :] * silu(z[t, :])) * w: the `width` columns in `groups` equal consecutive parts, each divided by
  * sqrt(mean(part^2) + eps).  z == NULL: no gate.  gate_after: out = rms_groups(y) * w * silu(z), the gate behind the norm.
  * gate_act 1: sigmoid(z) in the place of silu(z).
- * w_len (0: width) values of w, repeated over the columns (a head norm whose weights all heads share). */
+ * w_len (0: width) values of w, repeated over the columns (a head norm whose weights all heads share).
+ * out16 (may be NULL): the rows rounded to bf16, row stride ldo, beside out or (out = NULL) in its place. */
 typedef struct {
     const float* y;
     int64_t ldy;
@@ -346,6 +355,7 @@ typedef struct {
     int32_t gate_after;
     int32_t w_len;
     int32_t gate_act;
+    void* out16;
 } i64h_gate_norm_args;
 int i64h_gate_norm(const i64h_gate_norm_args* d, void* stream);
 

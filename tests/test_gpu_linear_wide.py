@@ -1,0 +1,132 @@
+"""Linears whose input rows come in bf16 against 64-bit products of the same values: every tile form around its tiles' edges, one to five steps of k,
+gathered rows, rows dealt to batches, gate / up pairs, results in bf16."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+FORMS = {"by size": 3, "256x256": 16, "256x128": 32, "192x128": 48, "128x128": 64, "64x128": 80, "64x64": 96}
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return torch.device("cuda:0")
+
+
+@pytest.fixture(params=FORMS)
+def form(request):
+    from vllm_i64_amd import ops_dense as D
+    D.call_dense("i64h_set_linear_skinny", FORMS[request.param])
+    yield request.param
+    D.call_dense("i64h_set_linear_skinny", 3)
+
+
+def close(got, ref, K):
+    """fp32 sums of exact products of order one over sqrt(K): a rounding of 2^-24 of the running sum per term at most."""
+    return torch.allclose(got.double().cpu(), ref, atol=K ** 0.5 * 2e-6, rtol=2e-5)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 4, 64), (63, 63, 128), (65, 132, 192), (129, 64, 256), (193, 260, 320), (257, 129, 576)])
+def test_tiles_and_ends(dev, form, M, N, K):
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randn(M, K + 16, generator=g).bfloat16()
+    w, b, e = (torch.randn(2 * N, K, generator=g) / math.sqrt(K)).bfloat16(), torch.randn(N, generator=g), torch.randn(M, N, generator=g)
+    A = a[:, 8:8 + K].double()
+    ref, up = A @ w[:N].double().T, A @ w[N:].double().T
+    ad, wd = a.to(dev), w.to(dev)
+    kw = dict(a16=ad, n=N, k=K, a_off=8, lda=K + 16)
+    out, out16 = torch.full((M, N + 3), 7.0, device=dev), torch.full((M, N + 3), 7.0, device=dev, dtype=torch.bfloat16)
+    D.linear(None, wd, out, out16=out16, c_off=1, ldc=N + 3, **kw)
+    assert close(out[:, 1:1 + N], ref, K) and torch.equal(out16, out.bfloat16()) and bool((out[:, 0] == 7).all()) and bool((out[:, 1 + N:] == 7).all())
+    y = torch.empty(M, N, device=dev)
+    D.linear(None, wd, y, bias=b.to(dev), epilogue=D.EPI_ADD, e=e.to(dev), lde=N, **kw)
+    assert close(y, ref + b.double() + e.double(), K)
+    y16 = torch.empty(M, N, device=dev, dtype=torch.bfloat16)
+    D.linear(None, wd, None, out16=y16, epilogue=D.EPI_SCALE, scale=0.5, **kw)
+    assert torch.allclose(y16.double().cpu(), 0.5 * ref, atol=1e-5, rtol=2.0 ** -8)      # (one rounding to eight bits)
+    s = torch.rand(M, generator=g) + 0.5
+    D.linear(None, wd, y, epilogue=D.EPI_SILU_MUL, row_scale=s.to(dev), **kw)
+    z, u = ref * s[:, None].double(), up * s[:, None].double()
+    assert torch.allclose(y.double().cpu(), z * torch.sigmoid(z) * u, atol=1e-4, rtol=1e-4)
+
+
+def test_same_as_rows_rounded_while_staged(dev, form):
+    """The sums run over k in one order in every form: the bits of a 128 x 128 tile that rounds its rows itself."""
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator().manual_seed(3)
+    a, w = torch.randn(300, 448, generator=g).to(dev), (torch.randn(200, 448, generator=g) / 20).bfloat16().to(dev)
+    out, ref = torch.empty(300, 200, device=dev), torch.empty(300, 200, device=dev)
+    D.linear(None, w, out, a16=a.bfloat16())
+    D.call_dense("i64h_set_linear_skinny", 16)
+    D.linear(a, w, ref)
+    assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("counts", [[5, 0, 70, 1], [0, 0, 0, 259], [64, 16, 128, 0], [1, 1, 1, 1]])
+def test_rows_dealt_to_experts(dev, form, counts):
+    """Gathered rows into a gate / up pair with a factor per row, its bf16 results as they lie into the next; empty batches; a larger bound than there are rows."""
+    from vllm_i64_amd import ops_dense as D
+    E, N, K, n = len(counts), 128, 192, 150
+    g = torch.Generator().manual_seed(sum(counts))
+    off = torch.tensor([0] + counts).cumsum(0).to(torch.int32)
+    R = int(off[-1])
+    rows = torch.randint(0, n, (R + 9,), generator=g).to(torch.int32)
+    h, s = torch.randn(n, K, generator=g).bfloat16(), torch.rand(R, generator=g) + 0.5
+    w = (torch.randn(E, 2 * N, K, generator=g) / math.sqrt(K)).bfloat16()
+    act = torch.full((R + 3, N), 7.0, device=dev, dtype=torch.bfloat16)
+    D.linear(None, w.to(dev), None, a16=h.to(dev), out16=act, m=max(counts), n=N, k=K, a_rows=rows.to(dev), batch=E, w_batch=2 * N * K, group_off=off.to(dev), row_scale=s.to(dev),
+             epilogue=D.EPI_CLAMP_GLU, act_a=1.702, act_b=7.0)
+    e_of = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    z = torch.matmul(w.double()[e_of], h.double()[rows[:R].long()].unsqueeze(-1)).squeeze(-1) * s[:, None].double()
+    u, v = z[:, :N].clamp(max=7.0), z[:, N:].clamp(-7.0, 7.0)
+    assert torch.allclose(act[:R].double().cpu(), u * torch.sigmoid(1.702 * u) * (v + 1), atol=2e-4, rtol=2.0 ** -8) and bool((act[R:] == 7).all())
+    wd = (torch.randn(E, K, N, generator=g) / math.sqrt(N)).bfloat16()
+    down = torch.full((R + 3, K), 7.0, device=dev)
+    D.linear(None, wd.to(dev), down, a16=act[:R], m=max(counts), n=K, k=N, batch=E, w_batch=K * N, group_off=off.to(dev))
+    ref = torch.matmul(wd.double()[e_of], act[:R].double().cpu().unsqueeze(-1)).squeeze(-1)
+    assert close(down[:R], ref, N) and bool((down[R:] == 7).all())
+
+
+def test_not_a_number_stays_in_its_row(dev, form):
+    from vllm_i64_amd import ops_dense as D
+    a, w = torch.ones(66, 128).bfloat16(), torch.ones(64, 128).bfloat16()
+    a[65, 127], a[3, 0] = math.nan, math.inf
+    out = torch.empty(66, 64, device=dev)
+    D.linear(None, w.to(dev), out, a16=a.to(dev))
+    rest = [r for r in range(66) if r not in (3, 65)]
+    assert bool((out[rest] == 128).all()) and bool(out[65].isnan().all()) and bool(out[3].isinf().all())
+
+
+def test_refused(dev):
+    from vllm_i64_amd import ops_dense as D
+    a16, w, out = torch.ones(66, 96, device=dev).bfloat16(), torch.ones(64, 96, device=dev).bfloat16(), torch.empty(66, 64, device=dev)
+    with pytest.raises(D._lib.I64HError):      # k no multiple of 64
+        D.linear(None, w, out, a16=a16)
+    a16, w = torch.ones(66, 128, device=dev).bfloat16(), torch.ones(64, 128, device=dev).bfloat16()
+    for kw in (dict(exact=True), dict(epilogue=D.EPI_RELU_SQ), dict(in_norm_w=torch.ones(128, device=dev), in_eps=1e-6)):
+        with pytest.raises(D._lib.I64HError):
+            D.linear(None, w, out, a16=a16, **kw)
+    with pytest.raises(D._lib.I64HError):      # a result in bf16 belongs to rows in bf16
+        D.linear(a16.float(), w, out, out16=torch.empty(66, 64, device=dev).bfloat16())
+
+
+def test_producers_round_once(dev):
+    """The normed rows of the residual kernel (both forms) and of the gate norm, in bf16 beside fp32 and alone: the fp32 rows rounded."""
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator(device=dev).manual_seed(1)
+    for W, S in ((96, 1), (1023, 1), (2048, 1), (64, 3)):
+        x, w = torch.randn(S, 5, W, generator=g, device=dev), torch.rand(W, generator=g, device=dev)
+        h, h16, alone = torch.empty(5, W, device=dev), *(torch.empty(5, W, device=dev, dtype=torch.bfloat16) for _ in range(2))
+        D.streams_step(x, norm_w=w, eps=1e-6, h=h, h16=h16)
+        D.streams_step(x, norm_w=w, eps=1e-6, h16=alone)
+        assert torch.equal(h16, h.bfloat16()) and torch.equal(alone, h16)
+    for width, n in ((128, 5), (130, 5), (512, 300)):
+        y, z, w = (torch.randn(n, width, generator=g, device=dev) for _ in range(3))
+        o, o16, alone = torch.empty(n, width, device=dev), *(torch.empty(n, width, device=dev, dtype=torch.bfloat16) for _ in range(2))
+        kw = dict(groups=2, eps=1e-6, z=z, ldz=width, n=n, gate_after=True)
+        D.gate_norm(y, w[0].contiguous(), o, out16=o16, **kw)
+        D.gate_norm(y, w[0].contiguous(), None, out16=alone, **kw)
+        assert torch.equal(o16, o.bfloat16()) and torch.equal(alone, o16)

@@ -242,7 +242,7 @@ class Linear(ctypes.Structure):
     """Mirror of i64h_linear (include/i64h_dense.h)."""
     _fields_ = [("A", _P), ("lda", _L), ("a_rows", _P), ("W", _P), ("C", _P), ("ldc", _L), ("M", _L), ("N", _I), ("K", _I), ("batch", _I),
                 ("a_batch", _L), ("w_batch", _L), ("c_batch", _L), ("exact", _I), ("epilogue", _I), ("E", _P), ("lde", _L), ("e_batch", _L),
-                ("softcap", _F), ("bias", _P), ("bias_batch", _L), ("scale", _F), ("act_a", _F), ("act_b", _F), ("group_off", _P), ("row_scale", _P), ("in_norm_w", _P), ("in_eps", _F), ("rows_total", _L), ("a_height", _L)]
+                ("softcap", _F), ("bias", _P), ("bias_batch", _L), ("scale", _F), ("act_a", _F), ("act_b", _F), ("group_off", _P), ("row_scale", _P), ("in_norm_w", _P), ("in_eps", _F), ("rows_total", _L), ("a_height", _L), ("A16", _P), ("C16", _P)]
 
 
 class PostNorm(ctypes.Structure):
@@ -277,7 +277,7 @@ class Streams(ctypes.Structure):
     """Mirror of i64h_streams_args (include/i64h_dense.h)."""
     _fields_ = [("streams", _P), ("S", _I), ("n", _L), ("W", _I), ("y", _P), ("ldy", _L), ("y2", _P), ("ldy2", _L), ("yn_w", _P), ("y2n_w", _P),
                 ("y_eps", _F), ("mix", _P), ("out_w", _P), ("in_w", _P), ("norm_w", _P), ("norm_w_len", _I), ("eps", _F), ("h", _P), ("rows", _P),
-                ("m_rows", _L), ("post_w", _P), ("post_center", _I), ("h_center", _I), ("norm_b", _P), ("y_scale", _P)]
+                ("m_rows", _L), ("post_w", _P), ("post_center", _I), ("h_center", _I), ("norm_b", _P), ("y_scale", _P), ("h16", _P)]
 
 
 class CausalConv(ctypes.Structure):
@@ -296,7 +296,7 @@ class SsmScan(ctypes.Structure):
 class GateNorm(ctypes.Structure):
     """Mirror of i64h_gate_norm_args (include/i64h_dense.h)."""
     _fields_ = [("y", _P), ("ldy", _L), ("z", _P), ("ldz", _L), ("w", _P), ("width", _I), ("groups", _I), ("eps", _F), ("out", _P), ("ldo", _L), ("n", _L),
-                ("gate_after", _I), ("w_len", _I), ("gate_act", _I)]
+                ("gate_after", _I), ("w_len", _I), ("gate_act", _I), ("out16", _P)]
 
 
 class MinGruScan(ctypes.Structure):

@@ -848,7 +848,7 @@ int i64h_linear_run(const i64h_linear* dp, void* stream) {
     I64H_CHECK_ARG(dp != nullptr, "linear: no descriptor");
     const i64h_linear& d = *dp;
     I64H_CHECK_ARG(d.M >= 0 && d.N > 0 && d.K > 0 && d.batch > 0, "linear: bad sizes M=%lld N=%d K=%d batch=%d", (long long)d.M, d.N, d.K, d.batch);
-    I64H_CHECK_ARG(d.A && d.W && d.C, "linear: null operand");
+    I64H_CHECK_ARG((d.A || d.A16) && d.W && (d.C || (d.A16 && d.C16)), "linear: null operand");
     I64H_CHECK_ARG(d.epilogue >= 0 && d.epilogue <= I64H_EPI_IN_NORM, "linear: epilogue %d", d.epilogue);
     I64H_CHECK_ARG((d.epilogue != I64H_EPI_MUL_SIGMOID && d.epilogue != I64H_EPI_ADD && d.epilogue != I64H_EPI_DECAY && d.epilogue != I64H_EPI_ROW_SIGMOID) || d.E, "linear: epilogue %d needs E", d.epilogue);
     I64H_CHECK_ARG(d.epilogue != I64H_EPI_CLAMP_GLU || d.act_b > 0.0f, "linear: bound %g of the clamped gate / up epilogue", (double)d.act_b);
@@ -858,6 +858,17 @@ int i64h_linear_run(const i64h_linear* dp, void* stream) {
     I64H_CHECK_ARG(dn_dual(d.epilogue) || !d.row_scale, "linear: row factors belong to the gate / up epilogues");
     I64H_CHECK_ARG(d.lda >= d.K || d.M <= 1, "linear: lda %lld < K %d", (long long)d.lda, d.K);
     I64H_CHECK_ARG(d.batch <= 65535 && (d.M + 63) / 64 <= 65535, "linear: grid too large");
+    I64H_CHECK_ARG(d.A16 || !d.C16, "linear: results in bf16 belong to input rows in bf16");
+    if (d.A16) {
+        I64H_CHECK_ARG(!d.exact && (dn_dual(d.epilogue) || d.epilogue == I64H_EPI_STORE || d.epilogue == I64H_EPI_SCALE || d.epilogue == I64H_EPI_ADD),
+                       "linear: input rows in bf16 with epilogue %d or 32-bit products", d.epilogue);
+        I64H_CHECK_ARG(d.K % 64 == 0 && d.lda % 8 == 0 && d.a_batch % 8 == 0 && d.w_batch % 8 == 0 && ((uintptr_t)d.A16 | (uintptr_t)d.W) % 16 == 0,
+                       "linear: input rows in bf16 need K a multiple of 64 (%d) and rows at 16 bytes", d.K);
+        if (d.M == 0) return 0;
+        I64H_CHECK_ARG(dn_linear_wide(d, g_form, (hipStream_t)stream), "linear: input rows in bf16 beyond 32-bit offsets");
+        I64H_CHECK_LAUNCH();
+        return 0;
+    }
     if (d.M == 0) return 0;
     const int vecA = (uintptr_t)d.A % 16 == 0 && d.lda % 4 == 0 && d.a_batch % 4 == 0 && (uintptr_t)d.in_norm_w % 16 == 0;
     const int vecW = (uintptr_t)d.W % 16 == 0 && d.K % 8 == 0 && d.w_batch % 8 == 0;

@@ -63,8 +63,76 @@ __device__ __forceinline__ float dn_epilogue(const i64h_linear& p, float acc, fl
     return acc;
 }
 
+// 16-byte loads through a buffer descriptor: a 32-bit offset per lane, the step's offset in a scalar register, and offsets past the end read
+// as zeros - a ragged end needs no branch and nothing is done to the registers behind the load
+typedef uint32_t dn_v4u __attribute__((ext_vector_type(4)));
+typedef uint32_t dn_v2u __attribute__((ext_vector_type(2)));
+constexpr uint32_t DN_BUF_END = 0xfffffff0u;       // from here on: zeros
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t dn_buffer(const void* base) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)DN_BUF_END, 0x00020000);
+}
+__device__ __forceinline__ dn_v4u dn_load16(__amdgpu_buffer_rsrc_t r, uint32_t lane_bytes, uint32_t step_bytes) {
+    return __builtin_amdgcn_raw_buffer_load_b128(r, lane_bytes, step_bytes, 0);
+}
+
+// The tile of a workgroup.  Workgroups go to the 8 XCDs in turn, so that every XCD gets a run of neighbouring tiles (its L2 then serves their common
+// rows and columns); within the run, columns of eight row tiles.
+struct dn_tile {
+    int64_t b, g0, rows;      // batch, its first row, its rows
+    int mt, nt;
+    bool any;
+};
+template <int BM>
+__device__ __forceinline__ dn_tile dn_find_tile(const i64h_linear& p, int n_tiles, int m_tiles, int lane) {
+    dn_tile o{(int64_t)blockIdx.z, 0, p.M, 0, 0, true};
+    int R = m_tiles;
+    // rows dealt to batches: lane l counts the tiles of batch 64 c + l, the lanes up to it their sum (one round of loads, not a chain of them)
+    const int batches = p.group_off ? p.batch : 0;
+    auto count = [&](int c) {
+        const int e = c + lane;
+        int t = e < batches ? (min(p.group_off[e + 1] - p.group_off[e], (int)p.M) + BM - 1) / BM : 0;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int up = __shfl_up(t, d);
+            t += lane >= d ? up : 0;
+        }
+        return t;
+    };
+    if (p.group_off) {
+        R = 0;
+        for (int c = 0; c < batches; c += 64) R += __builtin_amdgcn_readlane(count(c), 63);
+    }
+    const int T = R * n_tiles, id = blockIdx.x;
+    if (id >= T) {
+        o.any = false;
+        return o;
+    }
+    const int q = T >> 3, r = T & 7, x = id & 7;
+    const int t = x * q + min(x, r) + (id >> 3);
+    const int per = 8 * n_tiles, g = t / per, first = g * 8, width = min(8, R - first), in = t - g * per;
+    o.mt = first + in % width;
+    o.nt = in / width;
+    for (int c = 0; c < batches; c += 64) {
+        const int upto = count(c), all = __builtin_amdgcn_readlane(upto, 63);
+        if (o.mt >= all) {
+            o.mt -= all;
+            continue;
+        }
+        const int e = __ffsll((unsigned long long)__ballot(upto > o.mt)) - 1;
+        if (e > 0) o.mt -= __builtin_amdgcn_readlane(upto, e - 1);
+        o.b = c + e;
+        o.g0 = p.group_off[o.b];
+        o.rows = min(p.M, p.group_off[o.b + 1] - o.g0);
+        break;
+    }
+    return o;
+}
+
 // the matrix-core tile forms of i64h_linear_run (i64h_linear_block.hip): operands readable 16 bytes at a time.
 // form: -1 chosen by size, else the number of a tile form (tests, measurements).  False: the launch does not fit this form.
 bool dn_linear_block(const i64h_linear& d, int form, hipStream_t s);
+
+// launches whose input rows come in bf16 (i64h_linear_wide.hip).  form as above.  False: the launch does not fit.
+bool dn_linear_wide(const i64h_linear& d, int form, hipStream_t s);
 
 #endif

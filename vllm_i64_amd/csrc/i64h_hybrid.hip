@@ -17,8 +17,7 @@
 //   rot_prep_kernel       : the same with whole-row or per-head query / key norms, rotation of a part of every head in either pair layout
 //                           and values turned by their own position; rot_post_kernel turns a head's sum back and applies a gate per head
 // A row continues the row before it iff slot and position say so; state is taken as empty at position 0.  All arithmetic fp32.
-#include "i64h_common.h"
-#include "i64h_dense.h"
+#include "i64h_dense_dev.h"
 
 // i64h_latent.hip
 bool latent_decode_form();
@@ -160,7 +159,7 @@ __global__ __launch_bounds__(256) void streams_kernel(const i64h_streams_args p)
 #pragma unroll
             for (int t = 0; t < HY_MAX_STREAMS; ++t) x[t] = nx[t];
         }
-        if (p.h) {
+        if (p.h || p.h16) {
             float u = 0.0f;
 #pragma unroll
             for (int s = 0; s < HY_MAX_STREAMS; ++s)
@@ -170,7 +169,7 @@ __global__ __launch_bounds__(256) void streams_kernel(const i64h_streams_args p)
             su += u;
         }
     }
-    if (!p.h) return;
+    if (!p.h && !p.h16) return;
     float mean = 0.0f;
     if (p.h_center) {        // the centred norm: the squared deviations from the mean, summed in a pass of their own
         mean = hy_block_sum(su, red) / (float)W;
@@ -184,7 +183,9 @@ __global__ __launch_bounds__(256) void streams_kernel(const i64h_streams_args p)
     const float den = sqrtf(ss / (float)W + p.eps);
     for (int c = tid; c < W; c += 256) {
         const float v = (sv[c] - mean) / den * p.norm_w[p.norm_w_len == 1 ? 0 : c];
-        p.h[m * W + c] = p.norm_b ? v + p.norm_b[c] : v;
+        const float o = p.norm_b ? v + p.norm_b[c] : v;
+        if (p.h) p.h[m * W + c] = o;
+        if (p.h16) ((uint16_t*)p.h16)[m * W + c] = (uint16_t)dn_bf16_rne(o);
     }
 }
 
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(256) void residual_kernel(const i64h_streams_args p
 #pragma unroll
         for (int k = 0; k < 4; ++k) ss += v[i][k] * v[i][k], su += v[i][k];
     }
-    if (!p.h) return;
+    if (!p.h && !p.h16) return;
     float mean = 0.0f;
     if (p.h_center) {
         mean = hy_block_sum(su, red) / (float)W;
@@ -249,7 +250,8 @@ __global__ __launch_bounds__(256) void residual_kernel(const i64h_streams_args p
             const float4 b = *(const float4*)(p.norm_b + c);
             o.x += b.x, o.y += b.y, o.z += b.z, o.w += b.w;
         }
-        *(float4*)(p.h + m * W + c) = o;
+        if (p.h) *(float4*)(p.h + m * W + c) = o;
+        if (p.h16) *(uint2*)((uint16_t*)p.h16 + m * W + c) = make_uint2(dn_bf16_pair(o.x, o.y), dn_bf16_pair(o.z, o.w));
     }
 }
 
@@ -485,7 +487,12 @@ __global__ __launch_bounds__(NT) void gate_norm_kernel(const i64h_gate_norm_args
     for (int c = tid * VEC; c < W; c += NT * VEC) {      // (VEC divides a group and the weights' period)
         vec v = *(const vec*)(gv + c) / gv[W + c / gs] * *(const vec*)(p.w + c % wl);
         if (z && p.gate_after) v = gate(v, *(const vec*)(z + c));
-        *(vec*)(p.out + m * p.ldo + c) = v;
+        if (p.out) *(vec*)(p.out + m * p.ldo + c) = v;
+        if (p.out16) {
+            uint16_t* o = (uint16_t*)p.out16 + m * p.ldo + c;
+            if constexpr (VEC == 4) *(uint2*)o = make_uint2(dn_bf16_pair(v[0], v[1]), dn_bf16_pair(v[2], v[3]));
+            else *o = (uint16_t)dn_bf16_rne(v[0]);
+        }
     }
 }
 
@@ -858,18 +865,18 @@ int i64h_streams_step(const i64h_streams_args* dp, void* stream) {
     I64H_CHECK_ARG(dp != nullptr, "streams: no descriptor");
     const i64h_streams_args& d = *dp;
     I64H_CHECK_ARG(d.S >= 1 && d.S <= HY_MAX_STREAMS && d.W > 0 && d.n >= 0, "streams: %d streams (at most %d), width %d", d.S, HY_MAX_STREAMS, d.W);
-    I64H_CHECK_ARG(d.streams && (d.y || d.h), "streams: nothing to do");
+    I64H_CHECK_ARG(d.streams && (d.y || d.h || d.h16), "streams: nothing to do");
     I64H_CHECK_ARG(!d.y || d.out_w, "streams: the write needs out_w");
     I64H_CHECK_ARG(!d.y2 || (d.y && !d.yn_w == !d.y2n_w), "streams: two results take both norm weights or none");
-    I64H_CHECK_ARG(!d.h || (d.norm_w && (d.norm_w_len == 1 || d.norm_w_len == d.W)), "streams: the read needs a norm weight of 1 or W values");
+    I64H_CHECK_ARG(!(d.h || d.h16) || (d.norm_w && (d.norm_w_len == 1 || d.norm_w_len == d.W)), "streams: the read needs a norm weight of 1 or W values");
     I64H_CHECK_ARG(!d.rows || !d.y, "streams: gathered rows are read only");
     const int64_t rows = d.rows ? d.m_rows : d.n;
     const size_t lds = ((size_t)d.W + 4) * 4;
     I64H_CHECK_ARG(lds <= 64 * 1024, "streams: a row of %d values does not fit the kernel's LDS buffer", d.W);
     if (rows == 0) return 0;
-    const uintptr_t at = (uintptr_t)d.streams | (uintptr_t)d.y | (uintptr_t)d.y2 | (uintptr_t)d.y_scale | (uintptr_t)d.norm_w | (uintptr_t)d.norm_b | (uintptr_t)d.h;
+    const uintptr_t at = (uintptr_t)d.streams | (uintptr_t)d.y | (uintptr_t)d.y2 | (uintptr_t)d.y_scale | (uintptr_t)d.norm_w | (uintptr_t)d.norm_b | (uintptr_t)d.h | (uintptr_t)d.h16;
     if (g_residual_form && d.S == 1 && !d.mix && !d.in_w && !d.yn_w && !d.post_w && d.W % 4 == 0 && d.W <= 8 * 1024 && at % 16 == 0 && (!d.y || d.ldy % 4 == 0) &&
-        (!d.y2 || d.ldy2 % 4 == 0) && (!d.h || d.norm_w_len == d.W)) {
+        (!d.y2 || d.ldy2 % 4 == 0) && (!(d.h || d.h16) || d.norm_w_len == d.W)) {
         const dim3 grid((unsigned)rows);
         if (d.W <= 1024) hipLaunchKernelGGL(residual_kernel<1>, grid, dim3(256), 0, (hipStream_t)stream, d);
         else if (d.W <= 2048) hipLaunchKernelGGL(residual_kernel<2>, grid, dim3(256), 0, (hipStream_t)stream, d);
@@ -953,12 +960,12 @@ int i64h_gate_norm(const i64h_gate_norm_args* dp, void* stream) {
     I64H_CHECK_ARG(dp != nullptr, "gate_norm: no descriptor");
     const i64h_gate_norm_args& d = *dp;
     I64H_CHECK_ARG(d.width > 0 && d.groups > 0 && d.width % d.groups == 0, "gate_norm: width %d does not split into %d groups", d.width, d.groups);
-    I64H_CHECK_ARG(d.y && d.w && d.out, "gate_norm: null operand");
+    I64H_CHECK_ARG(d.y && d.w && (d.out || d.out16), "gate_norm: null operand");
     const size_t lds = ((size_t)d.width + d.groups) * 4;
     I64H_CHECK_ARG(lds <= 64 * 1024, "gate_norm: a row of %d values does not fit the kernel's LDS buffer", d.width);
     if (d.n == 0) return 0;
     const bool vec = (d.width / d.groups) % 4 == 0 && d.w_len % 4 == 0 && (d.ldy | d.ldo | (d.z ? d.ldz : 0)) % 4 == 0 &&
-                     (((uintptr_t)d.y | (uintptr_t)d.z | (uintptr_t)d.w | (uintptr_t)d.out) & 15) == 0;
+                     (((uintptr_t)d.y | (uintptr_t)d.z | (uintptr_t)d.w | (uintptr_t)d.out | (uintptr_t)d.out16) & 15) == 0;
     const bool wide = d.n <= HY_WIDE_ROWS;
     auto launch = [&](auto kern, int nt) { hipLaunchKernelGGL(kern, dim3((unsigned)d.n), dim3(nt), lds, (hipStream_t)stream, d); };
     if (vec) wide ? launch(gate_norm_kernel<512, 4>, 512) : launch(gate_norm_kernel<256, 4>, 256);

@@ -11,18 +11,6 @@
 #include "i64h_dense_dev.h"
 #include <type_traits>
 
-// 16-byte loads through a buffer descriptor: a 32-bit offset per lane, the step's offset in a scalar register, and offsets past the end read
-// as zeros - a ragged end needs no branch and nothing is done to the registers behind the load
-typedef uint32_t dn_v4u __attribute__((ext_vector_type(4)));
-typedef uint32_t dn_v2u __attribute__((ext_vector_type(2)));
-constexpr uint32_t DN_BUF_END = 0xfffffff0u;       // from here on: zeros
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t dn_buffer(const void* base) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)DN_BUF_END, 0x00020000);
-}
-__device__ __forceinline__ dn_v4u dn_load16(__amdgpu_buffer_rsrc_t r, uint32_t lane_bytes, uint32_t step_bytes) {
-    return __builtin_amdgcn_raw_buffer_load_b128(r, lane_bytes, step_bytes, 0);
-}
-
 // EX: 32-bit products on v_mfma_f32_16x16x4_f32, W widened while it is staged.  A staged row is 128 bytes either way: steps of 64 or of 32 values.
 template <int EPI, int BM, int BN, int KG, bool EX>
 __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kernel(const i64h_linear p, const int n_tiles, const int m_tiles, const int vecC) {
@@ -40,48 +28,10 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
     const int grp = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
     const int tid = threadIdx.x & 255, lane = tid & 63, wid = tid >> 6, wm = wid / NWN, wn = wid % NWN;
     const int N = p.N, K = p.K;
-    // the tile of this workgroup: workgroups go to the 8 XCDs in turn, so that every XCD gets a run of neighbouring tiles (its L2 then serves
-    // their common rows and columns); within the run, columns of eight row tiles
-    int64_t b = blockIdx.z, g0 = 0, rows = p.M;
-    int mt, nt, R = m_tiles;
-    {
-        // rows dealt to batches: lane l counts the tiles of batch 64 c + l, the lanes up to it their sum (one round of loads, not a chain of them)
-        const int batches = p.group_off ? p.batch : 0;
-        auto count = [&](int c) {
-            const int e = c + lane;
-            int t = e < batches ? (min(p.group_off[e + 1] - p.group_off[e], (int)p.M) + BM - 1) / BM : 0;
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const int up = __shfl_up(t, d);
-                t += lane >= d ? up : 0;
-            }
-            return t;
-        };
-        if (p.group_off) {
-            R = 0;
-            for (int c = 0; c < batches; c += 64) R += __builtin_amdgcn_readlane(count(c), 63);
-        }
-        const int T = R * n_tiles, id = blockIdx.x;
-        if (id >= T) return;
-        const int q = T >> 3, r = T & 7, x = id & 7;
-        const int t = x * q + min(x, r) + (id >> 3);
-        const int per = 8 * n_tiles, g = t / per, first = g * 8, width = min(8, R - first), in = t - g * per;
-        mt = first + in % width;
-        nt = in / width;
-        for (int c = 0; c < batches; c += 64) {
-            const int upto = count(c), all = __builtin_amdgcn_readlane(upto, 63);
-            if (mt >= all) {
-                mt -= all;
-                continue;
-            }
-            const int e = __ffsll((unsigned long long)__ballot(upto > mt)) - 1;
-            if (e > 0) mt -= __builtin_amdgcn_readlane(upto, e - 1);
-            b = c + e;
-            g0 = p.group_off[b];
-            rows = min(p.M, p.group_off[b + 1] - g0);
-            break;
-        }
-    }
+    const dn_tile t = dn_find_tile<BM>(p, n_tiles, m_tiles, lane);
+    if (!t.any) return;
+    const int64_t b = t.b, g0 = t.g0, rows = t.rows;
+    const int mt = t.mt, nt = t.nt;
     const int n0 = nt * COLS;
     const int64_t m0 = g0 + (int64_t)mt * BM;
     const int M = (int)min((int64_t)BM, rows - (int64_t)mt * BM);

@@ -1,0 +1,269 @@
+// C = epilogue(A W^T) with both operands in bf16 (i64h_linear's A16): the products of linear_block_kernel on rows that their producer rounded once
+// instead of every tile that reads them, summed in the order of k.
+//
+// What bounds it.  Large launches: the matrix instructions and, at k of 1024, a round's stores.  The kernel that rounds while it stages moved 48 KiB
+// a step of a 128 x 128 tile through registers; here 32 KiB go from memory to LDS by themselves, a wave's registers hold fragments alone and the
+// reads of one half step lie under the products of the other.  Small launches: the latency of a step, hence three or four steps on their way where a
+// stage is small enough (512 x 2048 x 5504 in 64 x 64 tiles: 41.8 us with two stages, 24.7 with three, 21.6 with four).  Microseconds in replayed
+// graphs, the weights of eight launches in turn:
+//   rows x columns x k            rounded while staged   256x256  256x128  192x128  128x128  64x128  64x64
+//   4096 x 5760 x 1024                  92                  62       56       54       55      69      82
+//   4096 x 1024 x 1024                  20                  28       18       18       16      15      17
+//   4096 x 2752 x 1024, pair            77                  60       52       50       53      59      70
+//   2956 x 8352 x 2048                 168                 109      111      112      115     135     156
+//   2956 x 5504 x 2048, pair           197                 154      140      133      147     166     196
+//   2956 x 2048 x 5504                 123                 114       66       75       72      84     102
+//   8 batches, 5912 x 2048 x 1792       95                  55       63       75       71      78      90
+//    512 x 5504 x 2048, pair            50                  54       32       40       39      42      48
+//    512 x 2048 x 2048                  13.5                41       23       25       22      13       9.4
+//    200 x 5760 x 1024                  13.3                26       15       16       14       9.4     9.9
+//     77 x 1024 x 1024                   5.9                21       13       12       10       7.3     5.6
+// Wider shares of a tile for a wave cost LDS reads the least (a 64 x 64 share reads as many bytes of LDS a cycle as the products take), so the large
+// tiles win as soon as their rounds fill the chip.
+#include "i64h_dense_dev.h"
+#include <cmath>
+#include <type_traits>
+
+// 16 bytes a lane from memory to LDS without registers between: the wave's 1024 bytes land one lane after the other
+__device__ __forceinline__ void dn_load_lds(__amdgpu_buffer_rsrc_t r, uint16_t* lds, uint32_t lane_bytes, uint32_t step_bytes) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, lane_bytes, step_bytes, 0, 0);
+}
+
+template <bool DUAL, int BM, int BN, int NWM, int NWN, int NS, int PER_CU>
+__global__ __launch_bounds__(64 * NWM * NWN, PER_CU * NWM * NWN / 4) void linear_wide_kernel(const i64h_linear p, const int n_tiles, const int m_tiles, const int vecC) {
+    constexpr int NW = NWM * NWN, WM = BM / NWM, WN = BN / NWN, FM = WM / 16, FN = WN / 16;
+    constexpr int COLS = DUAL ? BN / 2 : BN;               // output columns of a tile
+    constexpr int LA = BM / 8 / NW, LB = BN / 8 / NW;      // loads of a wave a step: eight rows of 64 values each
+    static_assert(LA > 0 && LB > 0 && FN > (DUAL ? 1 : 0), "");
+    // (variables of their own: the compiler then knows which loads a read of one has to wait for)
+    constexpr int STAGE = (BM + BN) * 64;
+    static_assert(NS >= 2 && NS <= 4, "");
+    __shared__ __attribute__((aligned(1024))) uint16_t s0[STAGE], s1[STAGE], s2[NS > 2 ? STAGE : 8], s3[NS > 3 ? STAGE : 8];
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wid / NWN, wn = wid % NWN;
+    const int N = p.N, K = p.K;
+    const dn_tile t = dn_find_tile<BM>(p, n_tiles, m_tiles, lane);
+    if (!t.any) return;
+    const int64_t b = t.b;
+    const int n0 = t.nt * COLS;
+    const int64_t m0 = t.g0 + (int64_t)t.mt * BM;
+    const int M = (int)min((int64_t)BM, t.rows - (int64_t)t.mt * BM);
+    const uint16_t *baseA = (const uint16_t*)p.A16 + b * p.a_batch + (p.a_rows ? 0 : m0 * p.lda), *baseW = (const uint16_t*)p.W + b * p.w_batch + (int64_t)n0 * K;
+    // 128-byte rows in LDS; the lane that fills chunk c of row r brings chunk c ^ (r & 7), so that the 16 rows of a fragment read lie in different banks
+    const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 16;
+    uint32_t oa[LA], ow[LB];
+#pragma unroll
+    for (int i = 0; i < LA; ++i) {      // (rows past the end repeat the last one and are not stored)
+        const int r = min((i * NW + wid) * 8 + lr, M - 1);
+        oa[i] = (uint32_t)((p.a_rows ? p.a_rows[m0 + r] : r) * p.lda) * 2u + lc;
+    }
+#pragma unroll
+    for (int i = 0; i < LB; ++i) {
+        const int r = (i * NW + wid) * 8 + lr;
+        // gate and up rows of the same columns go to the same wave: its first half of fragments, its second half
+        const int c = DUAL ? (r / WN) * (WN / 2) + r % (WN / 2) : r;
+        ow[i] = (uint32_t)((int64_t)(min(c, N - 1 - n0) + (DUAL && r % WN >= WN / 2 ? N : 0)) * K) * 2u + lc;
+    }
+    constexpr std::integral_constant<int, 0> S0{};
+    constexpr std::integral_constant<int, 1> S1{};
+    constexpr std::integral_constant<int, 2> S2{};
+    constexpr std::integral_constant<int, 3> S3{};
+    auto stage = [&](auto set) -> uint16_t* {
+        constexpr int S = decltype(set)::value;
+        return S == 0 ? s0 : S == 1 ? s1 : S == 2 ? s2 : s3;
+    };
+    const int KT = K / 64;
+    // (a step past the end asks for nothing: a buffer of no bytes)
+    auto load = [&](int kt, auto set) {
+        uint16_t* sm = stage(set);
+        const uint32_t bytes = kt < KT ? DN_BUF_END : 0u;
+        const __amdgpu_buffer_rsrc_t bufA = __builtin_amdgcn_make_buffer_rsrc((void*)baseA, 0, (int)bytes, 0x00020000), bufW = __builtin_amdgcn_make_buffer_rsrc((void*)baseW, 0, (int)bytes, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < LA; ++i) dn_load_lds(bufA, sm + (i * NW + wid) * 512, oa[i], kt * 128);
+#pragma unroll
+        for (int i = 0; i < LB; ++i) dn_load_lds(bufW, sm + BM * 64 + (i * NW + wid) * 512, ow[i], kt * 128);
+    };
+    dn_v4f acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = dn_v4f{0, 0, 0, 0};
+    const int fr = lane & 15, fk = lane >> 4;
+    dn_v4u a[2][FM], w[2][FN];      // the fragments of a step's two halves
+    auto fragments = [&](auto set, auto half) {
+        constexpr int H = decltype(half)::value;
+        const uint16_t* sm = stage(set);
+        const int ch = ((H * 4 + fk) ^ (fr & 7)) << 3;
+#pragma unroll
+        for (int i = 0; i < FM; ++i) a[H][i] = *(const dn_v4u*)&sm[(wm * WM + i * 16 + fr) * 64 + ch];
+#pragma unroll
+        for (int j = 0; j < FN; ++j) w[H][j] = *(const dn_v4u*)&sm[(BM + wn * WN + j * 16 + fr) * 64 + ch];
+    };
+    auto multiply = [&](auto half) {
+        constexpr int H = decltype(half)::value;
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_v8bf, w[H][j]), __builtin_bit_cast(dn_v8bf, a[H][i]), acc[i][j], 0, 0, 0);
+    };
+    // this wave's loads of the step after this one are in LDS and its fragments in registers; then everybody's
+    auto meet = [&]() {
+        constexpr int LEFT = (NS - 2) * (LA + LB);      // loads of later steps
+        static_assert(LEFT < 64, "");
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0070 | (LEFT & 15) | (LEFT >> 4) << 14);      // vmcnt LEFT, lgkmcnt 0
+        asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // reads (and loads) from the first product on, one between two products
+    auto interleave = [&](auto loads) {
+        constexpr int MF = FM * FN, DR = FM + FN, VM = decltype(loads)::value ? LA + LB : 0;
+#pragma unroll
+        for (int g = 0; g < DR; ++g) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (g < VM) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+            if (MF >= 2 * DR) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, MF, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    load(0, S0);
+    load(1, S1);
+    if constexpr (NS > 2) load(2, S2);
+    if constexpr (NS > 3) load(3, S3);
+    {
+        constexpr int LEFT = (NS - 1) * (LA + LB);
+        __builtin_amdgcn_s_waitcnt(0x0f70 | (LEFT & 15) | (LEFT >> 4) << 14);
+        asm volatile("s_barrier" ::: "memory");
+    }
+    fragments(S0, S0);
+    // The second half's fragments are read under the first half's products.  Behind them the step's buffer is free: the loads of the step NS further on
+    // go there, and the next step's first fragments are read under the second half's products.
+    // (Without a branch in the loop: where paths meet the compiler waits for whatever either may have on its way.)
+    auto step = [&](int kt, auto cur, auto nxt) {
+        fragments(cur, S1);
+        multiply(S0);
+        interleave(S0);
+        meet();
+        load(kt + NS, cur);
+        fragments(nxt, S0);
+        multiply(S1);
+        interleave(S1);
+    };
+    int kt = 0;
+    for (; kt + NS <= KT; kt += NS) {
+        if constexpr (NS == 2) {
+            step(kt, S0, S1);
+            step(kt + 1, S1, S0);
+        } else if constexpr (NS == 3) {
+            step(kt, S0, S1);
+            step(kt + 1, S1, S2);
+            step(kt + 2, S2, S0);
+        } else {
+            step(kt, S0, S1);
+            step(kt + 1, S1, S2);
+            step(kt + 2, S2, S3);
+            step(kt + 3, S3, S0);
+        }
+    }
+    if (kt < KT) step(kt, S0, S1);
+    if constexpr (NS > 2)
+        if (kt + 1 < KT) step(kt + 1, S1, S2);
+    if constexpr (NS > 3)
+        if (kt + 2 < KT) step(kt + 2, S2, S3);
+    __builtin_amdgcn_s_waitcnt(0x0f70);      // (nothing is on its way into LDS when the workgroup ends)
+    // the weights are the left operand: a lane holds four neighbouring columns of a row
+    auto finish = [&](auto epi, auto vec) {      // (vec: a lane's four columns at a time)
+        constexpr int EPI = decltype(epi)::value;
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            const int rl = wm * WM + i * 16 + fr;
+            if (rl >= M) continue;
+            const int64_t r = m0 + rl, row = b * p.c_batch + r * p.ldc;
+#pragma unroll
+            for (int j = 0; j < (DUAL ? FN / 2 : FN); ++j) {
+                const int c = n0 + wn * (COLS / NWN) + j * 16 + fk * 4;
+                auto out = [&](int g) { return dn_epilogue<EPI>(p, acc[i][j][g], DUAL ? acc[i][DUAL ? j + FN / 2 : j][g] : 0.0f, b, r, c + g); };
+                if constexpr (decltype(vec)::value) {
+                    if (c >= N) continue;
+                    const float4 v = make_float4(out(0), out(1), out(2), out(3));
+                    if (p.C16) *(uint2*)((uint16_t*)p.C16 + row + c) = make_uint2(dn_bf16_pair(v.x, v.y), dn_bf16_pair(v.z, v.w));
+                    if (p.C) *(float4*)(p.C + row + c) = v;
+                } else {
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        if (c + g >= N) continue;
+                        const float v = out(g);
+                        if (p.C16) ((uint16_t*)p.C16)[row + c + g] = (uint16_t)dn_bf16_rne(v);
+                        if (p.C) p.C[row + c + g] = v;
+                    }
+                }
+            }
+        }
+    };
+#define DN_FINISH(E) case E: if (vecC) finish(std::integral_constant<int, E>{}, S1); else finish(std::integral_constant<int, E>{}, S0); break;
+    if constexpr (DUAL) {
+        switch (p.epilogue) { DN_FINISH(I64H_EPI_CLAMP_GLU) DN_FINISH(I64H_EPI_GELU_MUL) DN_FINISH(I64H_EPI_SILU_MUL) }
+    } else {
+        switch (p.epilogue) { DN_FINISH(I64H_EPI_SCALE) DN_FINISH(I64H_EPI_ADD) DN_FINISH(I64H_EPI_STORE) }
+    }
+#undef DN_FINISH
+}
+
+template <int BM, int BN, int NWM, int NWN, int NS, int PER_CU>
+static void launch(const i64h_linear& d, hipStream_t s) {
+    const bool dual = dn_dual(d.epilogue);
+    const int cols = dual ? BN / 2 : BN;
+    const int nt = (d.N + cols - 1) / cols;
+    int64_t mt = (d.M + BM - 1) / BM;
+    if (d.group_off) {      // at most one partly filled row tile per batch beside the full ones
+        const int64_t most = mt * d.batch;
+        mt = d.rows_total > 0 ? (most < d.rows_total / BM + d.batch ? most : d.rows_total / BM + d.batch) : most;
+    }
+    const int vecC = ((uintptr_t)d.C | (uintptr_t)d.C16) % 16 == 0 && d.ldc % 4 == 0 && d.c_batch % 4 == 0 && d.N % 4 == 0;
+    const dim3 grid((unsigned)(mt * nt), 1, d.group_off ? 1u : (unsigned)d.batch);
+    if (dual) hipLaunchKernelGGL((linear_wide_kernel<true, BM, BN, NWM, NWN, NS, PER_CU>), grid, dim3(64 * NWM * NWN), 0, s, d, nt, (int)mt, vecC);
+    else hipLaunchKernelGGL((linear_wide_kernel<false, BM, BN, NWM, NWN, NS, PER_CU>), grid, dim3(64 * NWM * NWN), 0, s, d, nt, (int)mt, vecC);
+}
+
+// The form of a launch by what it costs: its workgroups' rounds on the 256 CUs times a round's microseconds, fitted to the measurements above (weights
+// that come from memory: a step is not shorter than the microsecond that its loads take, divided by the steps on their way).
+struct dn_wide_form {
+    int BM, BN;
+    bool alone;           // one workgroup a CU: every round ends with its stores, in the open; two a CU: the one's stores lie under the other's products
+    float first, step;    // a step of 64 k: of a workgroup alone on its CU, of a round (of two workgroups a CU)
+    float end;            // a round's stores
+};
+
+bool dn_linear_wide(const i64h_linear& d, int form, hipStream_t s) {
+    const bool dual = dn_dual(d.epilogue);
+    const int64_t span = (d.a_rows ? d.a_height : 256) * d.lda * 2;
+    if ((d.a_rows && d.a_height <= 0) || span >= (int64_t)DN_BUF_END - 64 || ((dual ? (int64_t)d.N : 0) + 256) * 2 * d.K >= (int64_t)DN_BUF_END - 64) return false;
+    const int64_t cols = dual ? 2 * (int64_t)d.N : d.N;
+    if ((d.M + 63) / 64 * d.batch * ((cols + 63) / 64) > 0x7fffffff) return false;
+    static const dn_wide_form forms[] = {{256, 256, true, 1.3f, 1.3f, 12.0f}, {256, 128, true, 0.72f, 0.72f, 7.0f}, {192, 128, false, 1.0f, 1.7f, 0.0f},
+                                         {128, 128, false, 1.0f, 1.2f, 0.0f}, {64, 128, false, 0.5f, 0.75f, 0.0f}, {64, 64, false, 0.33f, 0.4f, 0.0f}};
+    constexpr int FORMS = sizeof(forms) / sizeof(forms[0]);
+    if (form < 0) {
+        float best = 0.0f;
+        for (int i = 0; i < FORMS; ++i) {
+            const dn_wide_form& f = forms[i];
+            int64_t mt = (d.M + f.BM - 1) / f.BM * d.batch;
+            // rows dealt to batches: half a tile more than the rows fill, on average
+            if (d.group_off && d.rows_total > 0 && d.rows_total / f.BM + (d.batch + 1) / 2 < mt) mt = d.rows_total / f.BM + (d.batch + 1) / 2;
+            const float q = (float)(mt * ((cols + f.BN - 1) / f.BN)) / 256.0f;
+            const float step = f.alone ? ceilf(q) * f.step : fmaxf(f.first, fmaxf(0.5f * q, q > 1.0f ? 0.75f : 0.0f) * f.step);
+            const float cost = (float)(d.K / 64) * step + (f.alone ? ceilf(q) * f.end : 0.0f);
+            if (i == 0 || cost < best) best = cost, form = i;
+        }
+    }
+    switch (form) {
+        case 0: launch<256, 256, 2, 4, 2, 1>(d, s); break;
+        case 1: launch<256, 128, 4, 2, 3, 1>(d, s); break;
+        case 2: launch<192, 128, 2, 2, 2, 2>(d, s); break;
+        case 3: launch<128, 128, 2, 2, 2, 2>(d, s); break;
+        case 4: launch<64, 128, 2, 2, 3, 2>(d, s); break;
+        default: launch<64, 64, 2, 2, 4, 2>(d, s); break;
+    }
+    return true;
+}

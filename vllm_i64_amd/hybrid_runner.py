@@ -53,6 +53,18 @@ class HybridRunner:
         if self.side is not None:
             torch.cuda.current_stream().wait_stream(self.side)
 
+    # ---- rows that only Linears read: their producer rounds them to bf16 once where enough rows share a tile ----
+    WIDE_ROWS = 64      # more rows than this
+
+    def _wide(self, n: int, *widths: int) -> bool:
+        """Whether Linears over rows of these widths read them in bf16 (the values their tiles would round to: results are the same)."""
+        return not self.exact and n > self.WIDE_ROWS and all(w % 64 == 0 for w in widths)
+
+    @staticmethod
+    def _as16(t: torch.Tensor, n: int, width: int) -> torch.Tensor:
+        """The memory of a buffer of fp32 rows as rows in bf16."""
+        return t.view(torch.bfloat16)[: n * width].view(n, width)
+
     # ---- tensors by name and shape, in the two forms the kernels read ----
     def _bf(self, t: torch.Tensor) -> torch.Tensor:
         return t.to(device=self.device, dtype=torch.bfloat16).contiguous()
@@ -195,8 +207,8 @@ class HybridRunner:
                        gate=P if a.head_gate else None, gate_off=d.get("g_off", 0), ldg=P.shape[-1], n=n)
         self._out(O, d["o"], out, scale)
 
-    def _out(self, a, w, out, scale: float = 1.0) -> None:
-        D.linear(a, w, out, exact=self.exact, epilogue=D.EPI_STORE if scale == 1.0 else D.EPI_SCALE, scale=scale)
+    def _out(self, a, w, out, scale: float = 1.0, a16=None) -> None:
+        D.linear(a, w, out, a16=a16, exact=self.exact, epilogue=D.EPI_STORE if scale == 1.0 else D.EPI_SCALE, scale=scale)
 
     # ---- latent attention: one cached row per token that all heads share ----
     def _load_latent(self, p: str, m, need, d: dict) -> list:
@@ -258,11 +270,12 @@ class HybridRunner:
         rv = r.heads * r.vdim
         F = B.f[: n * r.heads * r.dim].view(n, r.heads * r.dim)
         D.linear(P, d["a2"], F, m=n, a_off=d["a1_off"], exact=self.exact, bias=d["a2_b"], epilogue=D.EPI_DECAY, e=d["a_rate"])
-        R, Rn = B.r[: n * rv].view(n, rv), B.rn[: n * rv].view(n, rv)
+        wide = self._wide(n, rv)
+        R, Rn, Rn16 = B.r[: n * rv].view(n, rv), None if wide else B.rn[: n * rv].view(n, rv), self._as16(B.rn, n, rv) if wide else None
         D.gla_scan(P, f=F, q_off=d["rq_off"], k_off=d["rk_off"], f_off=0, v_off=d["rv_off"], heads=r.heads, dim=r.dim, vdim=r.vdim, seg_start=seg, nseg=nseg,
                    positions=positions, slot_ids=slot_ids, state=kvc.state[l]["gla"], out=R, n=n, q_scale=r.dim ** -0.5)
-        D.gate_norm(R, d["r_norm"], Rn, groups=r.heads, eps=self.cfg.norm_eps, z=P, z_off=d["rg_off"], ldz=P.shape[-1], n=n, gate_after=True, width=rv)
-        self._out(Rn, d["o_right"], out, scale)
+        D.gate_norm(R, d["r_norm"], Rn, groups=r.heads, eps=self.cfg.norm_eps, z=P, z_off=d["rg_off"], ldz=P.shape[-1], n=n, gate_after=True, width=rv, out16=Rn16)
+        self._out(Rn, d["o_right"], out, scale, Rn16)
 
     # ---- gated delta rule ----
     def _gated_delta(self, B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, single: bool, out) -> None:
@@ -287,9 +300,10 @@ class HybridRunner:
             D.linear(P, d["g2"], Z, m=n, a_off=d["g1_off"], exact=ex)
         R = B.b[: n * rv].view(n, rv)
         D.gdn_scan(X, G, f=F, seg_start=seg, nseg=nseg, positions=positions, slot_ids=slot_ids, state=st["gdn"], out=R, **cols)
-        Rn = B.c[: n * rv].view(n, rv)
-        D.gate_norm(R, d["r_norm"], Rn, groups=r.heads, eps=self.cfg.norm_eps, z=Z, z_off=z_off, ldz=ldz, n=n, gate_after=True, width=rv, sigmoid=r.gate == "sigmoid")
-        D.linear(Rn, d["o_right"], out, exact=ex)
+        wide = self._wide(n, rv)
+        Rn, Rn16 = None if wide else B.c[: n * rv].view(n, rv), self._as16(B.c, n, rv) if wide else None
+        D.gate_norm(R, d["r_norm"], Rn, groups=r.heads, eps=self.cfg.norm_eps, z=Z, z_off=z_off, ldz=ldz, n=n, gate_after=True, width=rv, sigmoid=r.gate == "sigmoid", out16=Rn16)
+        D.linear(Rn, d["o_right"], out, a16=Rn16, exact=ex)
 
     # ---- mixture of experts ----
     def _load_moe(self, p: str, f, need, d: dict) -> None:
@@ -340,14 +354,21 @@ class HybridRunner:
         d["ff_gate_up"] = self._bf(torch.cat([need(p + "gate", (f.ff, W)), need(p + "up", (f.ff, W))], 0))
         d["ff_down"] = self._bf(need(p + "down", (W, f.ff)))
 
-    def _dense_glu(self, B, d, n, h, out) -> None:
-        f = d["mlp"]
-        act = B.act[: n * f.ff].view(n, f.ff)
-        D.linear(h, d["ff_gate_up"], act, exact=self.exact, **self._glu(f.limit, f.glu_alpha))
-        D.linear(act, d["ff_down"], out, exact=self.exact)
+    def _act(self, buf, n: int, width: int, h16):
+        """A feed-forward's inner rows: (fp32, bf16), one of them None."""
+        if h16 is not None and width % 64 == 0:
+            return None, self._as16(buf, n, width)
+        return buf[: n * width].view(n, width), None
 
-    def _moe_ff(self, B, d, n, h, out, shared_out, record: Optional[dict] = None, tag: str = "", beside: bool = False) -> None:
-        """out <- the mixture of d["mlp"] on h fp32 [n, width]; shared_out [n, width] receives the shared expert's rows on the way (beside: on
+    def _dense_glu(self, B, d, n, h, out, h16=None) -> None:
+        """h16: the input rows in bf16, read in h's place."""
+        f = d["mlp"]
+        act, act16 = self._act(B.act, n, f.ff, h16)
+        D.linear(h, d["ff_gate_up"], act, a16=h16, out16=act16, exact=self.exact, **self._glu(f.limit, f.glu_alpha))
+        D.linear(act, d["ff_down"], out, a16=act16, exact=self.exact)
+
+    def _moe_ff(self, B, d, n, h, out, shared_out, record: Optional[dict] = None, tag: str = "", beside: bool = False, h16=None) -> None:
+        """out <- the mixture of d["mlp"] on h fp32 [n, width] (h16: its rows in bf16, which the experts read); shared_out [n, width] receives the shared expert's rows on the way (beside: on
         the side stream, while the routed experts run)."""
         f, ex, W = d["mlp"], self.exact, self.cfg.width
         E, top = f.experts, f.top
@@ -355,9 +376,9 @@ class HybridRunner:
         shared = None
         if f.shared_ff:
             with self._beside() if beside else nullcontext():
-                sact = B.sact[: n * f.shared_ff].view(n, f.shared_ff)
-                D.linear(h, d["s_gate_up"], sact, exact=ex, **self._glu(f.shared_limit, f.glu_alpha))
-                shared = D.linear(sact, d["s_down"], shared_out, exact=ex)
+                sact, sact16 = self._act(B.sact, n, f.shared_ff, h16)
+                D.linear(h, d["s_gate_up"], sact, a16=h16, out16=sact16, exact=ex, **self._glu(f.shared_limit, f.glu_alpha))
+                shared = D.linear(sact, d["s_down"], shared_out, a16=sact16, exact=ex)
         # the router's products in 32 bits in both modes (a choice between experts is not rounding's to make), inside the choice's launch
         D.route_topk(None, h=h, w=d["router"], entries=f.entries, correction=d.get("correction"), groups=f.groups, keep=f.keep, top=top, scale=f.scale,
                      idx=B.idx, wgt=B.wgt, n=n, bias=d["router_b"], chosen_softmax=f.chosen_softmax, gate_out=gate, sigmoid_scores=f.sigmoid_scores, raw_weights=f.raw_weights)
@@ -366,9 +387,9 @@ class HybridRunner:
         pair_wgt = B.pair_wgt if f.weigh_input else None      # the weight multiplies what the expert reads, not what it returns
         D.moe_plan(B.idx, n=n, top=top, experts=E, group_off=B.group_off, pair_token=B.pair_token, pair_row=B.pair_row, wgt=B.wgt, pair_wgt=pair_wgt)
         # the (token, expert) pairs lie grouped by expert: one launch runs every expert over its own rows, the counts stay on the device
-        act = B.act[: n * top * f.ff].view(n * top, f.ff)
-        D.linear(h, d["gate_up"], act, m=n, a_rows=B.pair_token, batch=E, w_batch=2 * f.ff * W, exact=ex, group_off=B.group_off, row_scale=pair_wgt, **self._glu(f.limit, f.glu_alpha))
-        D.linear(act, d["e_down"], B.ey, m=n, batch=E, w_batch=W * f.ff, exact=ex, group_off=B.group_off)
+        act, act16 = self._act(B.act, n * top, f.ff, h16)
+        D.linear(h, d["gate_up"], act, a16=h16, out16=act16, m=n, a_rows=B.pair_token, batch=E, w_batch=2 * f.ff * W, exact=ex, group_off=B.group_off, row_scale=pair_wgt, **self._glu(f.limit, f.glu_alpha))
+        D.linear(act, d["e_down"], B.ey, a16=act16, m=n, batch=E, w_batch=W * f.ff, exact=ex, group_off=B.group_off)
         if shared is not None and beside:
             self._meet()
         D.moe_combine(B.ey, B.pair_row, None if f.weigh_input else B.wgt, h, shared, out, n=n, top=top, width=W, shared_gate=gate)

@@ -21,31 +21,47 @@ def _ref(s):
     return ctypes.addressof(s)
 
 
-def linear(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, m: Optional[int] = None, n: Optional[int] = None, k: Optional[int] = None,
+def linear(a: Optional[torch.Tensor], w: torch.Tensor, out: Optional[torch.Tensor], *, m: Optional[int] = None, n: Optional[int] = None, k: Optional[int] = None,
            a_off: int = 0, lda: Optional[int] = None, a_rows: Optional[torch.Tensor] = None, c_off: int = 0, ldc: Optional[int] = None,
            batch: int = 1, a_batch: int = 0, w_batch: int = 0, c_batch: int = 0, exact: bool = False, epilogue: int = EPI_STORE,
            e: Optional[torch.Tensor] = None, e_off: int = 0, lde: int = 0, e_batch: int = 0, softcap: float = 0.0,
            bias: Optional[torch.Tensor] = None, bias_batch: int = 0, scale: float = 1.0, act_a: float = 0.0, act_b: float = 0.0,
            group_off: Optional[torch.Tensor] = None, row_scale: Optional[torch.Tensor] = None,
-           in_norm_w: Optional[torch.Tensor] = None, in_eps: float = 0.0) -> torch.Tensor:
+           in_norm_w: Optional[torch.Tensor] = None, in_eps: float = 0.0, a16: Optional[torch.Tensor] = None,
+           out16: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out[b][:, c_off + b * c_batch : + n] = epilogue(a[b][rows, a_off + b * a_batch : + k] @ w[b]^T): see i64h_linear.  a, out and e are
     fp32 matrices addressed by (column offset, row stride; e with lde = 0 is one row for all); w is bf16 [n, k] (the gate / up epilogues: [2n, k], gate rows first), or a
     stack [batch, n, k] with w_batch = n * k.  bias fp32 [n] (per batch: bias_batch apart) is added before the epilogue.  group_off int32
     [batch + 1] on the device: batch b takes the rows [group_off[b], group_off[b + 1]) of a_rows (or a) and out; m is then the most rows a
     batch may have, and a_rows / a / out must hold group_off[batch] rows (the caller's business: the counts stay on the device).
     row_scale fp32, one factor per row of out (the gate / up epilogues): the input row times that factor.
-    in_norm_w fp32 [k] with in_eps: the input rows are RMS-normed first (plain result: the epilogue is then EPI_IN_NORM)."""
-    _chk(a, torch.float32, "a"), _chk(w, torch.bfloat16, "w"), _chk(out, torch.float32, "out")
+    in_norm_w fp32 [k] with in_eps: the input rows are RMS-normed first (plain result: the epilogue is then EPI_IN_NORM).
+    a16 bf16 (k a multiple of 64; the plain, scaled, adding and gate / up epilogues): the rows of a, rounded by whoever wrote them, in a's place.
+    out16 bf16 (with a16): receives the result rounded, beside out or (out None) in its place."""
+    if a16 is None:
+        if a is None or out is None or out16 is not None:
+            raise _lib.I64HError("linear: no input rows, or a result in bf16 without input rows in bf16")
+        _chk(a, torch.float32, "a"), _chk(w, torch.bfloat16, "w"), _chk(out, torch.float32, "out")
+        o = out
+    else:
+        _chk(a16, torch.bfloat16, "a16"), _chk(w, torch.bfloat16, "w")
+        a, o = a16, out if out is not None else out16
+        if out is not None:
+            _chk(out, torch.float32, "out")
+        if out16 is not None:
+            _chk(out16, torch.bfloat16, "out16")
+            if out is not None and (out16.numel() != out.numel() or out16.shape[-1] != out.shape[-1]):
+                raise _lib.I64HError("linear: out16 is not laid out as out")
     if a_rows is not None:
         _chk(a_rows, torch.int32, "a_rows")
     N = int(n if n is not None else w.shape[-2] // (2 if epilogue in _DUAL else 1))
     K = int(k if k is not None else w.shape[-1])
     M = int(m if m is not None else (a_rows.numel() if a_rows is not None else a.shape[0]))
     lda = int(lda if lda is not None else a.shape[-1])
-    ldc = int(ldc if ldc is not None else out.shape[-1])
+    ldc = int(ldc if ldc is not None else o.shape[-1])
     if w.shape[-1] != K or a_off + (batch - 1) * a_batch + K > lda or c_off + (batch - 1) * c_batch + N > ldc:
         raise _lib.I64HError(f"linear: K {K} / N {N} do not fit a (row stride {lda}), w {tuple(w.shape)} or out (row stride {ldc})")
-    if out.numel() < (M - 1) * ldc + c_off + (batch - 1) * c_batch + N or (a_rows is None and a.numel() < (M - 1) * lda + a_off + (batch - 1) * a_batch + K):
+    if o.numel() < (M - 1) * ldc + c_off + (batch - 1) * c_batch + N or (a_rows is None and a.numel() < (M - 1) * lda + a_off + (batch - 1) * a_batch + K):
         raise _lib.I64HError("linear: operand smaller than the launch reads or writes")
     if w.numel() < (batch - 1) * w_batch + N * K * (2 if epilogue in _DUAL else 1):
         raise _lib.I64HError("linear: weight smaller than the launch reads")
@@ -70,15 +86,16 @@ def linear(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, m: Optional[i
         _chk(group_off, torch.int32, "group_off")
         if group_off.numel() < batch + 1:
             raise _lib.I64HError("linear: group_off needs batch + 1 entries")
-    d = _lib.Linear(A=ptr(a) + 4 * a_off, lda=lda, a_rows=ptr(a_rows), W=ptr(w), C=ptr(out) + 4 * c_off, ldc=ldc, M=M, N=N, K=K, batch=batch,
+    d = _lib.Linear(A=ptr(a) + 4 * a_off if a16 is None else 0, lda=lda, a_rows=ptr(a_rows), W=ptr(w), C=ptr(out) + 4 * c_off if out is not None else 0, ldc=ldc, M=M, N=N, K=K, batch=batch,
                     a_batch=a_batch, w_batch=w_batch, c_batch=c_batch, exact=int(exact), epilogue=epilogue,
                     E=(ptr(e) + 4 * e_off) if e is not None else 0, lde=lde, e_batch=e_batch, softcap=float(softcap),
                     bias=ptr(bias), bias_batch=int(bias_batch), scale=float(scale), act_a=float(act_a), act_b=float(act_b), group_off=ptr(group_off),
                     row_scale=ptr(row_scale), in_norm_w=ptr(in_norm_w), in_eps=float(in_eps),
-                    rows_total=min((a_rows.numel() if a_rows is not None else a.numel() // lda), out.numel() // ldc) if group_off is not None else 0,
-                    a_height=-(-a.numel() // lda) if a_rows is not None else 0)
+                    rows_total=min((a_rows.numel() if a_rows is not None else a.numel() // lda), o.numel() // ldc) if group_off is not None else 0,
+                    a_height=-(-a.numel() // lda) if a_rows is not None else 0, A16=ptr(a16) + 2 * a_off if a16 is not None else 0,
+                    C16=ptr(out16) + 2 * c_off if out16 is not None else 0)
     call_dense("i64h_linear_run", _ref(d), _stream())
-    return out
+    return o
 
 
 def embed_scaled(ids: torch.Tensor, table: torch.Tensor, scale: float, out: torch.Tensor) -> torch.Tensor:
@@ -217,10 +234,12 @@ def streams_step(streams: torch.Tensor, *, y: Optional[torch.Tensor] = None, y2:
                  y2n_w: Optional[torch.Tensor] = None, y_eps: float = 0.0, mix: Optional[torch.Tensor] = None, out_w: Optional[torch.Tensor] = None,
                  in_w: Optional[torch.Tensor] = None, norm_w: Optional[torch.Tensor] = None, eps: float = 0.0, h: Optional[torch.Tensor] = None,
                  rows: Optional[torch.Tensor] = None, post_w: Optional[torch.Tensor] = None, post_center: bool = False,
-                 h_center: bool = False, norm_b: Optional[torch.Tensor] = None, y_scale: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+                 h_center: bool = False, norm_b: Optional[torch.Tensor] = None, y_scale: Optional[torch.Tensor] = None,
+                 h16: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """See i64h_streams_step.  streams fp32 [S, n, W], updated in place when y is given; h fp32 [n, W] (or [rows, W]).  post_w fp32 [W]: a
     norm over the result as a whole (centred with post_center) before it is added; h_center: the read's norm is centred; norm_b: added behind
-    the read's norm weight.  y2 without norm weights is simply added to y.  y_scale fp32 [W]: a factor per column on what is added."""
+    the read's norm weight.  y2 without norm weights is simply added to y.  y_scale fp32 [W]: a factor per column on what is added.
+    h16 bf16 [n, W]: the rows of h rounded, beside h or (h None) in its place."""
     _chk(streams, torch.float32, "streams")
     S, n, W = streams.shape
     for t, name in ((y, "y"), (y2, "y2"), (yn_w, "yn_w"), (y2n_w, "y2n_w"), (mix, "mix"), (out_w, "out_w"), (in_w, "in_w"), (norm_w, "norm_w"), (h, "h"),
@@ -242,10 +261,14 @@ def streams_step(streams: torch.Tensor, *, y: Optional[torch.Tensor] = None, y2:
         m_rows = rows.numel()
     if h is not None and h.numel() < m_rows * W:
         raise _lib.I64HError("streams_step: h smaller than the rows it receives")
+    if h16 is not None:
+        _chk(h16, torch.bfloat16, "h16")
+        if h16.numel() < m_rows * W:
+            raise _lib.I64HError("streams_step: h16 smaller than the rows it receives")
     d = _lib.Streams(streams=ptr(streams), S=S, n=n, W=W, y=ptr(y), ldy=W, y2=ptr(y2), ldy2=W, yn_w=ptr(yn_w), y2n_w=ptr(y2n_w), y_eps=float(y_eps),
                      mix=ptr(mix), out_w=ptr(out_w), in_w=ptr(in_w), norm_w=ptr(norm_w), norm_w_len=norm_w.numel() if norm_w is not None else 0,
                      eps=float(eps), h=ptr(h), rows=ptr(rows), m_rows=m_rows, post_w=ptr(post_w), post_center=int(bool(post_center)), h_center=int(bool(h_center)),
-                     norm_b=ptr(norm_b), y_scale=ptr(y_scale))
+                     norm_b=ptr(norm_b), y_scale=ptr(y_scale), h16=ptr(h16))
     call_dense("i64h_streams_step", _ref(d), _stream())
     return h
 
@@ -303,24 +326,30 @@ def ssm_scan(xbc: torch.Tensor, dt: torch.Tensor, *, dt_off: int, lddt: int, dt_
     return y
 
 
-def gate_norm(y: torch.Tensor, w: torch.Tensor, out: torch.Tensor, *, groups: int, eps: float, z: Optional[torch.Tensor] = None, z_off: int = 0,
-              ldz: int = 0, n: Optional[int] = None, gate_after: bool = False, width: Optional[int] = None, sigmoid: bool = False) -> torch.Tensor:
+def gate_norm(y: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor], *, groups: int, eps: float, z: Optional[torch.Tensor] = None, z_off: int = 0,
+              ldz: int = 0, n: Optional[int] = None, gate_after: bool = False, width: Optional[int] = None, sigmoid: bool = False,
+              out16: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """out = rms_groups(y * silu(z)) * w: see i64h_gate_norm.  y, out fp32 [n, width]; z the columns [z_off, + width) of a matrix of row stride ldz.
-    gate_after: out = rms_groups(y) * w * silu(z).  sigmoid: the gate is sigmoid(z).  width (default: w's length): the row's width, w then repeats over it."""
-    _chk(y, torch.float32, "y"), _chk(w, torch.float32, "w"), _chk(out, torch.float32, "out")
+    gate_after: out = rms_groups(y) * w * silu(z).  sigmoid: the gate is sigmoid(z).  width (default: w's length): the row's width, w then repeats over it.
+    out16 bf16: receives the rows rounded, beside out or (out None) in its place."""
+    _chk(y, torch.float32, "y"), _chk(w, torch.float32, "w")
+    if out is not None or out16 is None:
+        _chk(out, torch.float32, "out")
     w_len = w.numel()
     width = int(width if width is not None else w_len)
     if width % w_len:
         raise _lib.I64HError("gate_norm: the weights do not repeat evenly over the row")
     rows = int(n if n is not None else y.numel() // width)
-    if y.numel() < rows * width or out.numel() < rows * width:
+    if out16 is not None:
+        _chk(out16, torch.bfloat16, "out16")
+    if min(t.numel() for t in (y, out, out16) if t is not None) < rows * width:
         raise _lib.I64HError("gate_norm: operand smaller than the launch reads or writes")
     if z is not None:
         _chk(z, torch.float32, "z")
         if z.numel() < (rows - 1) * ldz + z_off + width:
             raise _lib.I64HError("gate_norm: gate smaller than the launch reads")
     d = _lib.GateNorm(y=ptr(y), ldy=width, z=(ptr(z) + 4 * z_off) if z is not None else 0, ldz=ldz, w=ptr(w), width=width, groups=groups, eps=float(eps),
-                      out=ptr(out), ldo=width, n=rows, gate_after=int(bool(gate_after)), w_len=w_len if w_len != width else 0, gate_act=int(bool(sigmoid)))
+                      out=ptr(out), ldo=width, n=rows, gate_after=int(bool(gate_after)), w_len=w_len if w_len != width else 0, gate_act=int(bool(sigmoid)), out16=ptr(out16))
     call_dense("i64h_gate_norm", _ref(d), _stream())
     return out
 

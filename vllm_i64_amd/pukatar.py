@@ -40,6 +40,7 @@ class _StepBuffers:
         self.e = torch.empty(1, n, W, **f32)                    # embedding rows
         self.x0 = torch.empty(n, W, **f32) if model.cfg.loop is not None else None    # the embedding output's part of what a pass starts from
         self.h = torch.empty(n, W, **f32)                       # the normed input of the current layer
+        self.h16 = torch.empty(n, W, dtype=torch.bfloat16, device=model.device) if model._wide(n, W) else None      # ... in bf16
         self.y = torch.empty(n, W, **f32)                       # the mixer's result
         self.y2 = torch.empty(n, W, **f32)                      # the feed-forward's
         self.y3 = torch.empty(n if model.max_shared else 0, W, **f32)
@@ -132,11 +133,11 @@ class PukatarModel(HybridRunner):
             self._load_moe(p + "mlp.", ff, need, d)
         return d
 
-    def _feed_forward(self, B, d, n, record, r) -> None:
+    def _feed_forward(self, B, d, n, record, r, h16=None) -> None:
         if d["mlp"].kind == "dense":
-            self._dense_glu(B, d, n, B.h, B.y2)
+            self._dense_glu(B, d, n, B.h, B.y2, h16)
         else:
-            self._moe_ff(B, d, n, B.h, B.y2, B.y3, record, f"r{r}")
+            self._moe_ff(B, d, n, B.h, B.y2, B.y3, record, f"r{r}", h16=h16)
 
     @torch.no_grad()
     def forward(self, token_ids: torch.Tensor, positions: torch.Tensor, slot_ids: torch.Tensor, ctx_len: Optional[torch.Tensor] = None,
@@ -164,6 +165,10 @@ class PukatarModel(HybridRunner):
         # every row the only row of its sequence (a decode step): the convolutions then store their carried inputs in the launch that reads them
         single = bool(rows_are_slots) or (tokens_per_seq is not None and all(int(t) <= 1 for t in tokens_per_seq))
         read = lambda norm, h, **kw: dict(norm_w=norm[0], norm_b=norm[1], eps=eps, h=h, h_center=True, **kw)
+
+        def normed(d):      # a layer's input: in bf16 alone where no router reads it
+            moe = d["mlp"] is not None and d["mlp"].kind == "moe"
+            return read(d["norm1"], B.h if moe or B.h16 is None else None, h16=B.h16)
         D.embed_scaled(token_ids, self.embed, 1.0, B.e)
         cur = 0
         D.streams_step(B.e, **read(self.embed_norm, B.x[0]))
@@ -175,13 +180,13 @@ class PukatarModel(HybridRunner):
                 D.linear(B.x[cur][0], self.loop_x, B.x[1 - cur][0], exact=ex, bias=self.loop_step[t], epilogue=D.EPI_ADD, e=B.x0, lde=cfg.width)
                 cur = 1 - cur
             if r == 0 or t is not None:      # (elsewhere the launch that wrote the residual has normed it)
-                D.streams_step(B.x[cur], **read(d["norm1"], B.h))
+                D.streams_step(B.x[cur], **normed(d))
             # mixer and feed-forward read the same input and meet at the residual: they run side by side
             if d["mlp"] is not None:
                 with self._beside():
-                    self._feed_forward(B, d, n, record, r)
+                    self._feed_forward(B, d, n, record, r, B.h16)
             P = B.p[: n * d["ld"]].view(n, d["ld"])
-            D.linear(B.h, d["w_in"], P, exact=ex)
+            D.linear(B.h, d["w_in"], P, a16=B.h16, exact=ex)
             if d["type"] == "attention":
                 self._rotary_attention(B, d, d["m"], P, r, n, positions, slot_ids, kvc, runs, hint, B.y)
             else:
@@ -191,7 +196,7 @@ class PukatarModel(HybridRunner):
                 write["y2"] = B.y2
                 self._meet()
             if r + 1 < len(self.layer_runs) and self.layer_runs[r + 1][1] is None:
-                write.update(read(self.layers[self.layer_runs[r + 1][0]]["norm1"], B.h))
+                write.update(normed(self.layers[self.layer_runs[r + 1][0]]))
             D.streams_step(B.x[cur], **write)
             if record is not None:
                 record[f"r{r}.x"] = B.x[cur][0].clone()

@@ -38,6 +38,7 @@ class _StepBuffers:
         W = model.cfg.width
         self.xe = torch.empty(2 if model.repeats else 1, n, W, **f32)      # the residual; the embedding output, where a further pass adds it
         self.h = torch.empty(n, W, **f32)                       # the normed input of the current sublayer
+        self.h16 = torch.empty(n, W, dtype=torch.bfloat16, device=model.device) if model._wide(n, W) else None      # ... in bf16
         self.y = torch.empty(n, W, **f32)                       # a sublayer's result
         self.y2 = torch.empty(n, W, **f32)                      # that of the right one of two side-by-side mixers / the shared expert's
         self.p = torch.empty(n * model.max_proj, **f32)         # everything projected from the mixer's input
@@ -126,11 +127,11 @@ class VepelixModel(HybridRunner):
         return d
 
     # ---- sublayers: the input is B.h, the result lands in B.y (and B.y2, to be added) ----
-    def _mixer(self, B, d, r, n, positions, slot_ids, kvc, seg, nseg, runs, hint) -> dict:
-        """Returns the operands of the residual's write."""
+    def _mixer(self, B, d, r, n, positions, slot_ids, kvc, seg, nseg, runs, hint, h16=None) -> dict:
+        """Returns the operands of the residual's write.  h16: the input rows in bf16, read in B.h's place."""
         m = d["m"]
         P = B.p[: n * d["ld"]].view(n, d["ld"])
-        D.linear(B.h, d["w_in"], P, exact=self.exact)
+        D.linear(B.h, d["w_in"], P, a16=h16, exact=self.exact)
         if d["type"] == "latent_attention":
             self._latent_attention(B, d, m, P, r, n, positions, slot_ids, kvc, runs, hint, B.y)
             return dict(y=B.y)
@@ -140,11 +141,11 @@ class VepelixModel(HybridRunner):
         self._meet()
         return dict(y=B.y, y2=B.y2)
 
-    def _feed_forward(self, B, d, n, record, r) -> None:
+    def _feed_forward(self, B, d, n, record, r, h16=None) -> None:
         if d["mlp"].kind == "dense":
-            self._dense_glu(B, d, n, B.h, B.y)
+            self._dense_glu(B, d, n, B.h, B.y, h16)
         else:
-            self._moe_ff(B, d, n, B.h, B.y, B.y2, record, f"r{r}", beside=True)
+            self._moe_ff(B, d, n, B.h, B.y, B.y2, record, f"r{r}", beside=True, h16=h16)
 
     @torch.no_grad()
     def forward(self, token_ids: torch.Tensor, positions: torch.Tensor, slot_ids: torch.Tensor, ctx_len: Optional[torch.Tensor] = None,
@@ -169,23 +170,25 @@ class VepelixModel(HybridRunner):
         else:
             runs = [(0, n, bool(rows_are_slots))]
         read = lambda w, h, **kw: dict(norm_w=w, eps=cfg.norm_eps, h=h, **kw)
+        h_mix = dict(h=B.h if B.h16 is None else None, h16=B.h16)      # a mixer reads rows in bf16 alone, so does a dense feed-forward
+        normed = lambda w: dict(norm_w=w, eps=cfg.norm_eps, **h_mix)
         D.embed_bigram(token_ids, positions, slot_ids, self.embed, B.xe)      # (a plane each for the residual and the embedding output)
         x = B.xe[0:1]
         for r, (l, t) in enumerate(self.layer_runs):
             d = self.layers[l]
             if r == 0:
-                D.streams_step(x, **read(d["norm1"], B.h))
+                D.streams_step(x, **normed(d["norm1"]))
             elif t:
-                D.streams_step(x, y=B.xe[1], out_w=self.ones1, **read(d["norm1"], B.h))
+                D.streams_step(x, y=B.xe[1], out_w=self.ones1, **normed(d["norm1"]))
             # (elsewhere the launch that wrote the residual has normed it)
-            write = self._mixer(B, d, r, n, positions, slot_ids, kvc, seg, nseg, runs, int(max_ctx_hint))
+            write = self._mixer(B, d, r, n, positions, slot_ids, kvc, seg, nseg, runs, int(max_ctx_hint), B.h16)
             write.update(out_w=self.ones1, y_scale=d["ls1"])
             if d["mlp"] is not None:
-                D.streams_step(x, **write, **read(d["norm2"], B.h))
-                self._feed_forward(B, d, n, record, r)
+                D.streams_step(x, **write, **(normed(d["norm2"]) if d["mlp"].kind == "dense" else read(d["norm2"], B.h, h16=B.h16)))
+                self._feed_forward(B, d, n, record, r, B.h16)
                 write = dict(y=B.y, out_w=self.ones1, y_scale=d["ls2"])
             if r + 1 < len(self.layer_runs) and not self.layer_runs[r + 1][1]:
-                write.update(read(self.layers[self.layer_runs[r + 1][0]]["norm1"], B.h))
+                write.update(normed(self.layers[self.layer_runs[r + 1][0]]["norm1"]))
             D.streams_step(x, **write)
             if record is not None:
                 record[f"r{r}.x"] = B.xe[0].clone()
