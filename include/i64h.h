@@ -318,6 +318,33 @@ typedef struct i64h_fp8_rows_desc {
     float norm_eps;
 } i64h_fp8_rows_desc;
 int i64h_gemm_fp8_rows_pair(const i64h_fp8_rows_desc* a, const i64h_fp8_rows_desc* b, int32_t epilogue, void* stream);
+/* The same products and sums (bit for bit) on rows quantized beforehand, for launches of a few hundred rows: A e4m3fn codes [*, K] with a_scale [*], 64 x
+ * 64 tiles.  K a multiple of 64, N of 16 (epilogue 1: 32), operands 16-byte aligned; other fields as i64h_fp8_rows_desc, B row-major.  Up to two problems of one
+ * epilogue in a launch (b may be NULL). */
+typedef struct i64h_fp8_codes_desc {
+    const uint8_t* A;               /* e4m3fn [*, K] */
+    const float* a_scale;           /* [*] */
+    const int32_t* a_src_row;
+    int32_t a_src_mod;
+    const uint8_t* B;
+    const float* b_scale;
+    const int32_t* group_offsets;
+    int32_t num_groups;
+    int64_t M;
+    int32_t N, K;
+    float* C;
+    const int32_t* c_row_map;
+    const float* c_add;
+} i64h_fp8_codes_desc;
+int i64h_gemm_fp8_codes_pair(const i64h_fp8_codes_desc* a, const i64h_fp8_codes_desc* b, int32_t epilogue, void* stream);
+/* ... with QK norm, rotary and the paged-KV write behind it: i64h_gemm_fp8_rows_qkv_rope_kv on codes (C is not used). */
+int i64h_gemm_fp8_codes_qkv_rope_kv(const i64h_fp8_codes_desc* d, const float* q_norm_w, const float* k_norm_w, float qk_eps, const float* rope_tab,
+                                    const int32_t* positions, const int32_t* slot_ids, const int32_t* block_table, int32_t max_blocks_per_seq, float* q_out,
+                                    void* k_cache, void* v_cache, int32_t kv_dtype, int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
+                                    int32_t block_size, void* stream);
+/* i64h_quantize_fp8_rows of two matrices in one launch (rows1 = 0: one); K multiples of four, 16-byte aligned rows. */
+int i64h_quantize_fp8_rows_pair(const float* x0, int64_t rows0, int32_t K0, uint8_t* q0, float* scale0, const float* x1, int64_t rows1, int32_t K1,
+                                uint8_t* q1, float* scale1, void* stream);
 /* Decode-sized fused form for e4m3 weights: qkv projection (one problem of i64h_gemm_fp8_rows_pair, epilogue 0: one group, no row
  * maps, 256 <= K) + per-head QK RMSNorm + rotate-half RoPE + paged-KV write in one launch (arguments as i64h_qk_norm_rope_kv;
  * head_dim 64, N = (heads + 2 kv heads) * 64; d->C is not written).  No counterpart in the reference: it stands for the pair

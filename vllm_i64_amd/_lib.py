@@ -47,6 +47,9 @@ SIGNATURES: Dict[str, str] = {
     "i64h_gemm_fp8_rows": "ppipppiliippip",
     "i64h_gemm_fp8_rows_pair": "ppip",
     "i64h_gemm_fp8_rows_qkv_rope_kv": "pppfpppp" + "ipppiiiiip",
+    "i64h_gemm_fp8_codes_pair": "ppip",
+    "i64h_gemm_fp8_codes_qkv_rope_kv": "pppfpppp" + "ipppiiiiip",
+    "i64h_quantize_fp8_rows_pair": "plipppli" + "ppp",
     "i64h_gemm_f32_grouped": "pppippiliippip",
     "i64h_gemm_w4_grouped": "pppppipiliippip",
     "i64h_gemm_h16_grouped": "pppipiliippip",
@@ -139,6 +142,12 @@ class Fp8RowsDesc(ctypes.Structure):
     """Mirror of i64h_fp8_rows_desc (include/i64h.h)."""
     _fields_ = [("A", _P), ("a_src_row", _P), ("a_src_mod", _I), ("B", _P), ("b_scale", _P), ("group_offsets", _P), ("num_groups", _I),
                 ("M", _L), ("N", _I), ("K", _I), ("C", _P), ("c_row_map", _P), ("b_frags", _I), ("c_add", _P), ("norm_w", _P), ("norm_eps", _F)]
+
+
+class Fp8CodesDesc(ctypes.Structure):
+    """Mirror of i64h_fp8_codes_desc (include/i64h.h)."""
+    _fields_ = [("A", _P), ("a_scale", _P), ("a_src_row", _P), ("a_src_mod", _I), ("B", _P), ("b_scale", _P), ("group_offsets", _P), ("num_groups", _I),
+                ("M", _L), ("N", _I), ("K", _I), ("C", _P), ("c_row_map", _P), ("c_add", _P)]
 
 
 class MoeLayer(ctypes.Structure):

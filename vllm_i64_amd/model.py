@@ -349,6 +349,12 @@ class I64MoEModel:
     # e4m3 runner: routed rows of a decode-sized step (ms/step at 256 | 512 | 1024: 200 sequences 4.97 | 3.48 | 3.48, 256 sequences
     # 5.75 | 4.41 | 4.40, 512 sequences 6.15 | 6.14 | 5.48)
     FP8_FUSE_MAX_ROWS = int(os.environ.get("I64H_FP8_FUSE_MAX_ROWS", "1024"))
+    # ... and from this many rows on the rows are quantized once and the products run in 64 x 64 tiles (us a step of two layers, without | with: mixture of
+    # experts 128 rows 193 | 241 - the host's launches -, 231 238 | 236, 512 341 | 255, 900 353 | 280, 4000 808 | 711, 12000 1627 | 1567, 16384 2002 | 2130; dense
+    # 128 199 | 204, 231 245 | 205, 512 341 | 237, 900 509 | 260, 4000 766 | 676, 12000 1680 | 1602, 16384 2158 | 2200)
+    FP8_TILE_ROWS = int(os.environ.get("I64H_FP8_TILE_ROWS", "160"))
+    FP8_TILE_ROWS_MOE = int(os.environ.get("I64H_FP8_TILE_ROWS_MOE", "240"))
+    FP8_TILE_MAX_ROWS = int(os.environ.get("I64H_FP8_TILE_MAX_ROWS", "12288"))
     EP_FUSE_MAX_ROWS = 1024  # the same for the pooled expert rows of the expert-parallel runner (8 ranks x 64 sequences x top-2)
     # expert-parallel runner, steps with more pooled expert rows than that (prefill chunks): dispatch every (route, token) row to the
     # rank that owns its expert and return the result by variable-split all-to-alls (each rank quantizes and multiplies only the rows of
@@ -793,6 +799,52 @@ class I64MoEModel:
         else:
             ops.fused_residual_norm(hbuf, self.final_norm, eps, normed=B.normed, h_out=B.h, lm_workspace=lm_ws)
 
+    def _fp8_tiles(self, n: int) -> bool:
+        """Whether the e4m3 Linears of a step of n rows run on rows quantized once, in 64 x 64 tiles (see FP8_TILE_ROWS); same bits as the step that
+        quantizes in front of every launch's tiles."""
+        cfg = self.cfg
+        if not ((self.FP8_TILE_ROWS_MOE if cfg.is_moe else self.FP8_TILE_ROWS) <= n <= self.FP8_TILE_MAX_ROWS and self.FP8_FUSE_NORM and cfg.head_dim == 64 and cfg.hidden_size <= 1024 and cfg.hidden_size % 64 == 0):
+            return False
+        inner = [cfg.expert_inter] + ([cfg.shared_intermediate_size] if cfg.shared_intermediate_size else []) if cfg.is_moe else [cfg.intermediate_size]
+        return all(k > 0 and k % 64 == 0 for k in inner) and all((W["q_norm"] is None) == (W["k_norm"] is None) for W in self.layers)
+
+    def _layers_fp8_tiles(self, B, n, positions, slot_ids, ctx_len, kvc, rows_are_slots, splits) -> None:
+        """The decoder layers of such a step.  B.xa / B.xs hold the first layer's normed rows quantized; leaves B.normed (the final norm's rows)."""
+        cfg, H, eps = self.cfg, self.cfg.hidden_size, self.cfg.rms_eps
+        desc = ops.fp8_codes_desc
+        attn2d = B.attn.view(n, H)
+        S = cfg.shared_intermediate_size if cfg.is_moe else 0
+        for l, W in enumerate(self.layers):
+            Wq, Wo = W["qkv"], W["o"]
+            ops.gemm_fp8_codes_qkv_rope_kv(desc(B.xa, B.xs, Wq.w_q, Wq.w_s, None), W["q_norm"], W["k_norm"], 1e-6, self.rope, positions, slot_ids, kvc.block_table,
+                                           kvc.k[l], kvc.v[l], B.q, cfg.num_heads, cfg.num_kv_heads, cfg.head_dim)
+            self._attention(B, kvc, l, ctx_len, None if rows_are_slots else slot_ids, splits)
+            ops.quantize_fp8_rows_pair(attn2d, B.xa, B.xs)
+            ops.gemm_fp8_codes_pair(desc(B.xa, B.xs, Wo.w_q, Wo.w_s, B.h, c_add=B.h))
+            ops.fused_residual_norm_fp8(B.h, W["ln2"], eps, B.xa, B.xs, h_out=B.h)
+            nxt = self.layers[l + 1]["ln1"] if l + 1 < cfg.num_layers else self.final_norm
+            if cfg.is_moe:
+                plan, R = B.plan, B.plan.rows
+                Wg, Wd, Xg, Xd = W.get("sh_gu"), W.get("sh_dn"), W["exp_gu"], W["exp_dn"]
+                routed = desc(B.xa, B.xs, Xg.w_q, Xg.w_s, B.e_inter, m=R, a_src_row=plan.perm[l], a_src_mod=n, group_offsets=plan.expert_offsets[l])
+                # (the shared expert's tiles first: the surplus tiles of the grouped problem's upper bound end the launch)
+                first = (desc(B.xa, B.xs, Wg.w_q, Wg.w_s, B.sh_inter), routed) if S else (routed,)
+                ops.gemm_fp8_codes_pair(*first, epilogue=ops.EPI_SWIGLU)
+                ops.quantize_fp8_rows_pair(B.e_inter, B.eia, B.eis, *((B.sh_inter, B.sha, B.shs) if S else ()))
+                routed = desc(B.eia, B.eis, Xd.w_q, Xd.w_s, B.e_out, m=R, group_offsets=plan.expert_offsets[l], c_row_map=plan.perm[l])
+                ops.gemm_fp8_codes_pair(*((desc(B.sha, B.shs, Wd.w_q, Wd.w_s, B.sh_out), routed) if S else (routed,)))
+                mk = dict(moe_rows=B.e_out, moe_inv=None, moe_shared=B.sh_out if S else None, route_weights=cfg.route_weights,
+                          routed_scale=W["routed_scale"], shared_scale=W["shared_scale"], h_out=B.h)
+            else:
+                ops.gemm_fp8_codes_pair(desc(B.xa, B.xs, W["gu"].w_q, W["gu"].w_s, B.d_inter), epilogue=ops.EPI_SWIGLU)
+                ops.quantize_fp8_rows_pair(B.d_inter, B.da, B.ds)
+                ops.gemm_fp8_codes_pair(desc(B.da, B.ds, W["dn"].w_q, W["dn"].w_s, B.h, c_add=B.h))
+                mk = dict(h_out=B.h)
+            if l + 1 < cfg.num_layers:
+                ops.fused_residual_norm_fp8(B.h, nxt, eps, B.xa, B.xs, **mk)
+            else:
+                ops.fused_residual_norm(B.h, nxt, eps, normed=B.normed, **mk)
+
     def _forward_fp8(self, token_ids, positions, slot_ids, ctx_len, logit_rows, kvc, record, max_ctx_hint, rows_are_slots, tokens_per_seq=None):
         """The forward with every Linear an fp8_linear (vllm_i64/core/fp8.py:137-194, its torch._scaled_mm branch): activations are
         quantized per token, so no call-wide statistics exist and the expert rows need no per-bucket treatment - one
@@ -813,7 +865,8 @@ class I64MoEModel:
         small = n * max(1, cfg.top_k if cfg.is_moe else 1) <= self.FP8_FUSE_MAX_ROWS
         # prefill-sized chunks (see FP8_FUSE_NORM): the norm quantizes the normalised rows itself (a row's scale needs only that
         # row), the fp32 rows are not stored; decode-sized steps quantize inside their GEMMs; recording runs keep the fp32 rows
-        nq = self.FP8_FUSE_NORM and not small and record is None and H <= 1024 and H % 4 == 0
+        tiles = record is None and self._fp8_tiles(n)
+        nq = (self.FP8_FUSE_NORM and not small and record is None and H <= 1024 and H % 4 == 0) or tiles
         qkr_ok = lambda W: (self.FP8_FUSE_QKV and small and not nq and record is None and cfg.head_dim == 64 and ops.fp8_rows_ok(H)
                             and H >= 256 and (W["q_norm"] is None) == (W["k_norm"] is None))
         # decode-sized steps: no norm launches in front of the qkv / gate_up calls, no residual launches behind o / down (see
@@ -842,7 +895,9 @@ class I64MoEModel:
                 wf = Wp.frags(epi == ops.EPI_SWIGLU)   # prefill-sized call: the operand-stationary kernel on the weight's fragment pack
             return ops.gemm_fp8(xq, xs, Wp.w_q, Wp.w_s, out, w_frags=wf, **kw)
 
-        for l, W in enumerate(self.layers):
+        if tiles:
+            self._layers_fp8_tiles(B, n, positions, slot_ids, ctx_len, kvc, rows_are_slots, splits)
+        for l, W in enumerate(self.layers) if not tiles else ():
             if record is not None:
                 record[f"l{l}.in"] = B.h.clone()
             if qkr_ok(W):

@@ -367,6 +367,43 @@ def gemm_fp8_rows_qkv_rope_kv(desc, q_norm_w, k_norm_w, qk_eps, rope_tab, positi
     return q_out
 
 
+def fp8_codes_desc(a: torch.Tensor, a_scale: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor, out: Optional[torch.Tensor], *, m: Optional[int] = None,
+                   a_src_row=None, a_src_mod: int = 0, group_offsets=None, c_row_map=None, c_add=None):
+    """One problem of gemm_fp8_codes_pair: e4m3 rows a with their scales, e4m3 weights w [(G,) N, K]; other arguments as fp8_rows_desc."""
+    _chk(a, None, "a"), _chk(a_scale, torch.float32, "a_scale"), _chk(w, None, "w")
+    G, N, K = w.shape if w.dim() == 3 else (1, *w.shape)
+    M = m if m is not None else a.shape[0]
+    if a.element_size() != 1 or w.element_size() != 1 or a.shape[1] != K or a_scale.numel() < a.shape[0] or (a_src_row is None and a.shape[0] < M) or (a_src_row is not None and a.shape[0] < a_src_mod):
+        raise _lib.I64HError("fp8_codes_desc: operand rows do not fit the sizes")
+    return _lib.Fp8CodesDesc(ptr(a), ptr(a_scale), ptr(a_src_row), a_src_mod, ptr(w), ptr(w_scale), ptr(group_offsets), G, M, N, K, ptr(out), ptr(c_row_map), ptr(c_add))
+
+
+def gemm_fp8_codes_pair(a_desc, b_desc=None, epilogue: int = EPI_STORE):
+    """Up to two e4m3 products of one epilogue on rows quantized beforehand (see i64h_gemm_fp8_codes_pair)."""
+    call("i64h_gemm_fp8_codes_pair", ctypes.addressof(a_desc), ctypes.addressof(b_desc) if b_desc is not None else 0, epilogue, _stream())
+
+
+def gemm_fp8_codes_qkv_rope_kv(desc, q_norm_w, k_norm_w, qk_eps, rope_tab, positions, slot_ids, block_table, k_cache, v_cache, q_out,
+                               num_heads: int, num_kv_heads: int, head_dim: int):
+    """gemm_fp8_rows_qkv_rope_kv on rows quantized beforehand (desc: one problem of gemm_fp8_codes_pair, no result tensor)."""
+    call("i64h_gemm_fp8_codes_qkv_rope_kv", ctypes.addressof(desc), ptr(q_norm_w), ptr(k_norm_w), float(qk_eps), ptr(rope_tab),
+         ptr(positions), ptr(slot_ids), ptr(block_table), block_table.shape[1], ptr(q_out), ptr(k_cache), ptr(v_cache),
+         KV_DTYPE_CODE[k_cache.dtype], num_heads, num_kv_heads, head_dim, k_cache.shape[1], _stream())
+    return q_out
+
+
+def quantize_fp8_rows_pair(x0: torch.Tensor, q0: torch.Tensor, s0: torch.Tensor, x1: Optional[torch.Tensor] = None, q1: Optional[torch.Tensor] = None,
+                           s1: Optional[torch.Tensor] = None) -> None:
+    """quantize_fp8_rows of one or two matrices in one launch (row lengths multiples of four)."""
+    for x, q, s in ((x0, q0, s0), (x1, q1, s1)):
+        if x is not None:
+            _chk(x, torch.float32, "x"), _chk(q, None, "q"), _chk(s, torch.float32, "scale")
+            if q.element_size() != 1 or q.numel() < x.numel() or s.numel() < x.shape[0]:
+                raise _lib.I64HError("quantize_fp8_rows_pair: outputs smaller than the rows")
+    call("i64h_quantize_fp8_rows_pair", ptr(x0), x0.shape[0], x0.shape[1], ptr(q0), ptr(s0), ptr(x1), x1.shape[0] if x1 is not None else 0,
+         x1.shape[1] if x1 is not None else 0, ptr(q1), ptr(s1), _stream())
+
+
 def fp8_rows_ok(k: int) -> bool:
     return k % 64 == 0 and k <= 8192
 
