@@ -91,3 +91,26 @@ def test_draw_of_short_rows(V, k):
     x = 2 * torch.randn(5, V, generator=torch.Generator().manual_seed(V + k))
     u = torch.tensor([0.0, 0.1, 0.5, 0.95, 0.9999])
     check(x, 0.8, k, 0.9, u, draw(x, 0.8, k, 0.9, u))
+
+
+@pytest.mark.parametrize("V", [100, 5000, 40000])
+@pytest.mark.parametrize("k", [1, 50, 64, 65, 100, 128, 129])
+@pytest.mark.parametrize("p", [1.0, 0.9, 0.05])
+def test_few_candidates_of_few_values(V, k, p):
+    """Lists around one and two a lane of a wave, with the k-th value tied and with top-p's bound inside a run of equal values."""
+    g = torch.Generator().manual_seed(V + k)
+    x = (torch.randn(6, V, generator=g) * 4).round() / 4
+    x[1] = torch.randn(V, generator=g) * 0.01
+    x[2] = -0.0
+    x[3] = -x[3].abs()
+    u = torch.tensor([0.0, 0.1, 0.37, 0.5, 0.95, 0.9999])
+    check(x, 0.8, k, p, u, draw(x, 0.8, k, p, u))
+
+
+def test_first_of_the_largest():
+    for V in (5, 3000, 40000):
+        x = torch.full((5, V), -math.inf)
+        x[0, 0], x[1], x[2, 2:4] = math.nan, math.nan, torch.tensor([-0.0, 0.0])
+        x[3, 3:] = -1.0
+        want = [1, 0, 2, 3, 0]
+        assert draw(x, 0.0, 0, 1.0, torch.zeros(5)).tolist() == want

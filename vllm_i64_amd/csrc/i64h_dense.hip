@@ -498,23 +498,23 @@ __global__ __launch_bounds__(256) void gated_postnorm_kernel(const i64h_postnorm
 // top-k: the largest key with at least k values at or above it; top-p: the largest key whose values at or above it hold at
 // least p of the mass.  The draw takes the first kept value, in index order, behind which the running sum exceeds u of the total.
 //
-// What bounds it is the chain of dependent block-wide sums, one per bit, so each is made short.  With top-k of at most half as many as there are
-// threads the row is read once: the k-th largest of the threads' maxima is a bound that at least k values reach and few others do, those (at most one
-// a thread, sorted by index) lie one to a thread from there on.  Without top-k the row's keys stay in registers (NV float4 per thread; NV = 0: read again,
-// vocabularies beyond 32768).  64 rows of 32000, top-k 50 and top-p 0.95: 1280 us with four
-// waves that read the row again for every bit, 35 us with sixteen.  Up to 4096 values four waves have the shorter sums: 64 rows of 1000 drawn without
-// top-k 11 us, sixteen waves 16, rows of 4000 13 and 17.
+// What bounds it is the chain of dependent sums, one per bit, so each is made short.  With top-k of at most half as many as there are threads the row
+// is read once: a bound that at least k of the threads' maxima reach and few others do is found by one wave that holds them all, the values above it
+// (at most one a thread, sorted by index) lie one to a thread from there on - and up to 128 of them in one wave, whose sums need no barrier.  Without
+// top-k the row's keys stay in registers (NV float4 per thread; NV = 0: read again, vocabularies beyond 32768).  64 rows of 32000, top-k 50 and
+// top-p 0.95: 1280 us with four waves that read the row again for every bit, 33 us with sixteen and a barrier a bit, 15.7 with one wave's sums.  Up to 4096
+// values four waves have the shorter sums: 64 rows of 1000 drawn without top-k 11 us, sixteen waves 16, rows of 4000 13 and 17.
 template <int NV, int SR_WAVES>
 __global__ __launch_bounds__(64 * SR_WAVES) void sample_rows_kernel(const float* __restrict__ logits, int64_t* __restrict__ out, int V, const int vec,
                                                                  const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
                                                                  const float* __restrict__ top_p, const float* __restrict__ u) {
     constexpr int SR_THREADS = 64 * SR_WAVES, SR_LIST = SR_THREADS, SR_TOPK = SR_LIST / 2;
     __shared__ float redf[2][SR_WAVES];
-    __shared__ int redi[2][SR_WAVES], bestc[SR_WAVES];
-    __shared__ float bestv[SR_WAVES];
-    __shared__ uint32_t lkey[SR_LIST], skey[SR_LIST];
+    __shared__ int redi[2][SR_WAVES];
+    __shared__ uint32_t lkey[SR_LIST], skey[SR_LIST], svalue[128];
     __shared__ int lidx[SR_LIST], sidx[SR_LIST];
-    __shared__ int listed, chosen;
+    __shared__ int listed, chosen, sarg;
+    __shared__ uint32_t sbound;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int64_t r = blockIdx.x;
     const float* x = logits + r * V;
@@ -552,21 +552,15 @@ __global__ __launch_bounds__(64 * SR_WAVES) void sample_rows_kernel(const float*
         }
     };
     uint32_t key[NV > 0 ? NV : 1][4];
-    float best = -INFINITY;
-    int bi = V;
-    uint32_t kmax = 0, kmin = ~0u;
+    // the largest number (kbest: its key, of what is no NaN; 0: none) and the largest key; where the first value that large lies is looked up behind them
+    constexpr uint32_t KINF = 0xff800000u, KNINF = 0x007fffffu;      // the keys of the infinities: beyond them lie the NaNs
+    uint32_t kmax = 0, kbest = 0;
     auto look = [&](int i, const uint32_t* k) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const float v = ordered_to_f32(k[j]);
-            const int c = i * STEP + tid * 4 + j;
-            if (c < V && (v > best || (v == best && c < bi))) best = v, bi = c;
             kmax = max(kmax, k[j]);
+            kbest = max(kbest, k[j] <= KINF ? k[j] : 0u);
         }
-        if (i < V / STEP) kmin = min(min(min(k[0], k[1]), min(k[2], k[3])), kmin);
-        else
-#pragma unroll
-            for (int j = 0; j < 4; ++j) kmin = i * STEP + tid * 4 + j < V ? min(kmin, k[j]) : kmin;
     };
     if (NV > 0) {
 #pragma unroll
@@ -579,25 +573,47 @@ __global__ __launch_bounds__(64 * SR_WAVES) void sample_rows_kernel(const float*
             look(i, key[0]);
         }
     }
-    uint32_t rmax = kmax;      // the largest key of the row, and the maximum and its first index
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) {
-        const float v = __shfl_xor(best, d);
-        const int c = __shfl_xor(bi, d);
-        if (v > best || (v == best && c < bi)) best = v, bi = c;
-        rmax = max(rmax, (uint32_t)__shfl_xor((int)rmax, d));
-    }
-    if (lane == 0) bestv[wid] = best, bestc[wid] = bi, skey[wid] = rmax;
-    if (tid == 0) listed = 0, chosen = V;
+    auto max16 = [](uint32_t v) {      // over sixteen neighbouring lanes
+        v = max(v, __float_as_uint(I64H_DPPF(__uint_as_float(v), 0x128)));
+        v = max(v, __float_as_uint(I64H_DPPF(__uint_as_float(v), 0x124)));
+        v = max(v, __float_as_uint(I64H_DPPF(__uint_as_float(v), 0x4E)));
+        return max(v, __float_as_uint(I64H_DPPF(__uint_as_float(v), 0xB1)));
+    };
+    auto max64 = [&](uint32_t v) {
+        v = max16(v);
+        const uint32_t a = max((uint32_t)__builtin_amdgcn_readlane((int)v, 0), (uint32_t)__builtin_amdgcn_readlane((int)v, 16));
+        const uint32_t b = max((uint32_t)__builtin_amdgcn_readlane((int)v, 32), (uint32_t)__builtin_amdgcn_readlane((int)v, 48));
+        return max(a, b);
+    };
+    const uint32_t wbest = max64(kbest), wmax = max64(kmax);
+    if (lane == 0) skey[wid] = wbest, skey[SR_WAVES + wid] = wmax;
+    lkey[tid] = kmax;
+    if (tid == 0) listed = 0, chosen = V, sarg = V;
     __syncthreads();
+    static_assert(SR_WAVES <= 16, "");
+    const uint32_t rbest = (uint32_t)__builtin_amdgcn_readfirstlane((int)max16(skey[lane & (SR_WAVES - 1)]));
+    const uint32_t rmax = (uint32_t)__builtin_amdgcn_readfirstlane((int)max16(skey[SR_WAVES + (lane & (SR_WAVES - 1))]));
+    // (two zeros are equal, their keys are not: the first of either)
+    auto as_best = [&](uint32_t k) { return k == rbest || (k + 1 == rbest && rbest == 0x80000000u); };
+    if (rbest >= KNINF && kbest >= rbest - 1) {      // (a few threads)
+        auto find4 = [&](int i, const uint32_t* k) {
 #pragma unroll
-    for (int w = 0; w < SR_WAVES; ++w) {
-        const float v = bestv[w];
-        const int c = bestc[w];
-        if (v > best || (v == best && c < bi)) best = v, bi = c;
-        rmax = max(rmax, skey[w]);
+            for (int j = 0; j < 4; ++j)
+                if (as_best(k[j]) && i * STEP + tid * 4 + j < V) atomicMin(&sarg, i * STEP + tid * 4 + j);
+        };
+        if (NV > 0) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) find4(i, key[i]);
+        } else {
+            for (int i = 0; i < chunks; ++i) {
+                load4(i, key[0]);
+                find4(i, key[0]);
+            }
+        }
     }
-    const int arg = bi < V ? bi : 0;
+    __syncthreads();
+    const int arg = sarg < V ? sarg : 0;
+    const float best = rbest >= KNINF ? ordered_to_f32(rbest) : -INFINITY;      // (nothing but NaNs: token 0)
     const float T = temperature ? temperature[r] : 0.0f;
     if (!(T > 0.0f) || (u && u[r] < 0.0f)) {
         if (tid == 0) out[r] = arg;
@@ -619,10 +635,22 @@ __global__ __launch_bounds__(64 * SR_WAVES) void sample_rows_kernel(const float*
         return thr;
     };
     if (k > 0 && k < V && k <= SR_TOPK) {
-        const uint32_t bound = bisect([&](uint32_t cand) {
-            const int n = sum_i(wave_count(kmax >= cand));
-            return n == k ? 2 : (n > k ? 1 : 0);
-        });
+        // a key that at least k of the threads' maxima reach and no more than k or a wave's width: one wave looks for it, without a barrier a bit
+        if (wid == 0) {
+            uint32_t mine[SR_WAVES];
+#pragma unroll
+            for (int w = 0; w < SR_WAVES; ++w) mine[w] = lkey[w * 64 + lane];
+            const int most = max(k, 64);
+            const uint32_t found = bisect([&](uint32_t cand) {
+                int n = 0;
+#pragma unroll
+                for (int w = 0; w < SR_WAVES; ++w) n += wave_count(mine[w] >= cand);
+                return n < k ? 0 : (n <= most ? 2 : 1);
+            });
+            if (lane == 0) sbound = found;
+        }
+        __syncthreads();
+        const uint32_t bound = sbound;
         auto list4 = [&](int i, const uint32_t* q) {
 #pragma unroll
             for (int j = 0; j < 4; ++j)
@@ -642,6 +670,92 @@ __global__ __launch_bounds__(64 * SR_WAVES) void sample_rows_kernel(const float*
         }
         __syncthreads();
         const int n = listed;
+        // One wave holds up to 128 of them, one or two a lane, and needs no barrier.  Sorted by index (the order of the sums, which are added as those of two waves
+        // are below) and by value: the k-th largest is top-k's bound, and top-p's lies at one of the values, found in as many sums as their number has bits.
+        auto few = [&](auto per) {
+            constexpr int PER = decltype(per)::value;
+            int c[PER], at[PER] = {}, above[PER] = {};
+            uint32_t q[PER];
+            float w[PER], run[PER], total[PER], sum = 0.0f;
+#pragma unroll
+            for (int h = 0; h < PER; ++h) {
+                const bool mine = h * 64 + lane < n;
+                c[h] = mine ? lidx[h * 64 + lane] : V;
+                q[h] = mine ? lkey[h * 64 + lane] : 0u;
+            }
+#pragma unroll
+            for (int g = 0; g < PER; ++g)
+                for (int j = 0; j < min(n - g * 64, 64); ++j) {
+                    const int oc = __builtin_amdgcn_readlane(c[g], j);
+                    const uint32_t oq = (uint32_t)__builtin_amdgcn_readlane((int)q[g], j);
+#pragma unroll
+                    for (int h = 0; h < PER; ++h) {
+                        const bool front = oc < c[h];
+                        at[h] += front ? 1 : 0;
+                        above[h] += oq > q[h] || (oq == q[h] && front) ? 1 : 0;
+                    }
+                }
+#pragma unroll
+            for (int h = 0; h < PER; ++h)
+                if (h * 64 + lane < n) skey[at[h]] = q[h], sidx[at[h]] = c[h], svalue[above[h]] = q[h];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            __builtin_amdgcn_wave_barrier();
+            uint32_t thr = svalue[k - 1];
+#pragma unroll
+            for (int h = 0; h < PER; ++h) {
+                q[h] = h * 64 + lane < n ? skey[h * 64 + lane] : 0u;      // (0: past the end; no bound is that low)
+                w[h] = h * 64 + lane < n ? weight(q[h]) : 0.0f;
+            }
+            auto mass = [&](uint32_t cut) {
+                float s = 0.0f;
+#pragma unroll
+                for (int h = 0; h < PER; ++h) s += wave_sum(h * 64 + lane < n && q[h] >= cut ? w[h] : 0.0f);
+                return s;
+            };
+            if (pp < 1.0f) {
+                const float need = pp * mass(thr);
+                if (!(need > 0.0f)) {      // nothing is asked for (or the sum is no number): the most likely token
+                    if (lane == 0) out[r] = arg;
+                    return;
+                }
+                int lo = 0, hi = 0;      // the first place of the values in descending order whose values at or above it hold enough: in [lo, hi]
+#pragma unroll
+                for (int h = 0; h < PER; ++h) hi += wave_count(h * 64 + lane < n && q[h] >= thr);
+                --hi;
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (mass(svalue[mid]) >= need) hi = mid;
+                    else lo = mid + 1;
+                }
+                thr = svalue[lo];
+            }
+#pragma unroll
+            for (int h = 0; h < PER; ++h) {      // running sums in index order
+                run[h] = h * 64 + lane < n && q[h] >= thr ? w[h] : 0.0f;
+#pragma unroll
+                for (int d = 1; d < 64; d <<= 1) {
+                    const float up = __shfl_up(run[h], d);
+                    run[h] += lane >= d ? up : 0.0f;
+                }
+                total[h] = __shfl(run[h], 63);
+                sum += total[h];
+            }
+            int pick = -1;
+            float before = 0.0f;
+#pragma unroll
+            for (int h = 0; h < PER; ++h) {
+                const unsigned long long past = __ballot(h * 64 + lane < n && q[h] >= thr && before + run[h] > uu * sum);
+                if (pick < 0 && past) pick = sidx[h * 64 + __ffsll(past) - 1];
+                before += total[h];
+            }
+            if (lane == 0) out[r] = pick >= 0 ? pick : arg;  // rounding at the far end of the walk: the most likely token
+        };
+        if (n <= 128) {
+            if (wid > 0) return;
+            if (n <= 64) few(std::integral_constant<int, 1>{});
+            else few(std::integral_constant<int, 2>{});
+            return;
+        }
         if (n <= SR_LIST) {
             if (tid < n) {
                 const int c = lidx[tid];
@@ -711,9 +825,16 @@ __global__ __launch_bounds__(64 * SR_WAVES) void sample_rows_kernel(const float*
             n = sum_i(n);
             return n == k ? 2 : (n > k ? 1 : 0);
         });
-    if (thr == 0u && sum_i(wave_count(kmin == 0u)) > 0) {      // the NaN of all bits set is kept: the sum is no number
-        if (tid == 0) out[r] = arg;
-        return;
+    if (thr == 0u) {      // the NaN of all bits set is kept: the sum is no number
+        int lost = 0;
+        each([&](int i, const uint32_t* q) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) lost += wave_count(q[j] == 0u && i * STEP + tid * 4 + j < V);
+        });
+        if (sum_i(lost) > 0) {
+            if (tid == 0) out[r] = arg;
+            return;
+        }
     }
     thr = max(thr, 1u);      // (0: the places past the end)
     auto mass = [&](uint32_t cut) {
