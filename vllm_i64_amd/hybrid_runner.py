@@ -11,6 +11,7 @@ from typing import Callable, Dict, Optional
 import torch
 
 from . import ops_dense as D
+from .ops import upload
 
 UNIT_EPS = 1e-6     # inside the root of the delta rule's unit vectors: a constant of the mechanism, not of a checkpoint
 
@@ -37,20 +38,28 @@ class HybridRunner:
         self.side = torch.cuda.Stream(device=self.device) if self.SIDE_STREAM and self.device.type == "cuda" else None
 
     # ---- two sublayers side by side ----
+    # Eager steps of little work (rows times width) are bound by the host, and the events of a fork and its meeting take 40 to 65 us of it.
+    # Microseconds a step, forked | not: width 1024, 77 rows 1120 | 797, 400 rows 1105 | 745, 700 rows 1088 | 1025, 32-bit 376 rows 1114 to 1300 | 1191;
+    # width 2048, 216 rows 959 | 828, 256 rows 1091 | 978, 512 rows 988 | 1163; 1024 x 4096 rows 3623 | 3893.
+    FORK_WORK = int(os.environ.get("I64H_FORK_WORK", "850000"))
+
+    def _forks(self, n: int) -> bool:
+        return self.side is not None and (n * self.cfg.width >= self.FORK_WORK or torch.cuda.is_current_stream_capturing())
+
     @contextmanager
-    def _beside(self):
-        """The launches of the body run on the side stream (of default priority), behind what the current stream holds so far and beside what
-        it gets next, until _meet(); a captured graph keeps the two branches.  Without a side stream they simply run here.  One level only:
-        the body forks no further."""
-        if self.side is None:
+    def _beside(self, n: int):
+        """The launches of the body (a step of n rows) run on the side stream (of default priority), behind what the current stream holds so far and
+        beside what it gets next, until _meet(n); a captured graph keeps the two branches.  Without a side stream, and in eager steps of few rows, they
+        simply run here.  One level only: the body forks no further."""
+        if not self._forks(n):
             yield
             return
         self.side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(self.side):
             yield
 
-    def _meet(self) -> None:
-        if self.side is not None:
+    def _meet(self, n: int) -> None:
+        if self._forks(n):
             torch.cuda.current_stream().wait_stream(self.side)
 
     # ---- rows that only Linears read: their producer rounds them to bf16 once where enough rows share a tile ----
@@ -149,7 +158,7 @@ class HybridRunner:
                 starts.append(starts[-1] + int(t))
         if starts[-1] != n:
             raise ValueError(f"tokens_per_seq adds up to {starts[-1]} rows, the step has {n}")
-        return torch.tensor(starts, dtype=torch.int32).to(self.device), len(starts) - 1
+        return upload(starts, torch.int32, self.device), len(starts) - 1
 
     def _splits(self, B, rows: int, heads: int, kv_heads: int, vals: int, width: int, ctx_hint: int, floats):
         """How many waves share a decode row's keys (about ATTN_WAVES waves in the launch, a wave keeping at least two tiles of 32 keys),
@@ -375,7 +384,7 @@ class HybridRunner:
         gate = B.sgate if f.shared_ff and f.shared_gate else None
         shared = None
         if f.shared_ff:
-            with self._beside() if beside else nullcontext():
+            with self._beside(n) if beside else nullcontext():
                 sact, sact16 = self._act(B.sact, n, f.shared_ff, h16)
                 D.linear(h, d["s_gate_up"], sact, a16=h16, out16=sact16, exact=ex, **self._glu(f.shared_limit, f.glu_alpha))
                 shared = D.linear(sact, d["s_down"], shared_out, a16=sact16, exact=ex)
@@ -391,5 +400,5 @@ class HybridRunner:
         D.linear(h, d["gate_up"], act, a16=h16, out16=act16, m=n, a_rows=B.pair_token, batch=E, w_batch=2 * f.ff * W, exact=ex, group_off=B.group_off, row_scale=pair_wgt, **self._glu(f.limit, f.glu_alpha))
         D.linear(act, d["e_down"], B.ey, a16=act16, m=n, batch=E, w_batch=W * f.ff, exact=ex, group_off=B.group_off)
         if shared is not None and beside:
-            self._meet()
+            self._meet(n)
         D.moe_combine(B.ey, B.pair_row, None if f.weigh_input else B.wgt, h, shared, out, n=n, top=top, width=W, shared_gate=gate)

@@ -28,6 +28,14 @@ def _stream() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
+def upload(values, dtype, device) -> torch.Tensor:
+    """A short host list on the device, through page-locked memory: the host goes on, the copy takes its place in the current stream (a copy from
+    pageable memory waits for all that the stream holds).  While a stream is captured the copy is the waiting kind, which a capture refuses."""
+    if torch.device(device).type != "cuda" or torch.cuda.is_current_stream_capturing():
+        return torch.tensor(values, dtype=dtype).to(device)
+    return torch.tensor(values, dtype=dtype, pin_memory=True).to(device, non_blocking=True)
+
+
 def _chk(t: torch.Tensor, dtype=None, name="tensor"):
     if not t.is_cuda:
         raise _lib.I64HError(f"{name}: expected a GPU tensor (this package has no CPU path)")

@@ -183,7 +183,7 @@ class PukatarModel(HybridRunner):
                 D.streams_step(B.x[cur], **normed(d))
             # mixer and feed-forward read the same input and meet at the residual: they run side by side
             if d["mlp"] is not None:
-                with self._beside():
+                with self._beside(n):
                     self._feed_forward(B, d, n, record, r, B.h16)
             P = B.p[: n * d["ld"]].view(n, d["ld"])
             D.linear(B.h, d["w_in"], P, a16=B.h16, exact=ex)
@@ -194,7 +194,7 @@ class PukatarModel(HybridRunner):
             write = dict(y=B.y, out_w=self.ones1)
             if d["mlp"] is not None:
                 write["y2"] = B.y2
-                self._meet()
+                self._meet(n)
             if r + 1 < len(self.layer_runs) and self.layer_runs[r + 1][1] is None:
                 write.update(normed(self.layers[self.layer_runs[r + 1][0]]))
             D.streams_step(B.x[cur], **write)

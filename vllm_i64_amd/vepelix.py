@@ -135,10 +135,10 @@ class VepelixModel(HybridRunner):
         if d["type"] == "latent_attention":
             self._latent_attention(B, d, m, P, r, n, positions, slot_ids, kvc, runs, hint, B.y)
             return dict(y=B.y)
-        with self._beside():      # attention and recurrence share nothing but the projection rows
+        with self._beside(n):      # attention and recurrence share nothing but the projection rows
             self._rotary_attention(B, d, m.left, P, r, n, positions, slot_ids, kvc, runs, hint, B.y, m.left_scale)
         self._gated_linear(B, d, m.right, P, r, n, positions, slot_ids, kvc, seg, nseg, B.y2, m.right_scale)
-        self._meet()
+        self._meet(n)
         return dict(y=B.y, y2=B.y2)
 
     def _feed_forward(self, B, d, n, record, r, h16=None) -> None:
