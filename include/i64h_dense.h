@@ -252,7 +252,9 @@ int i64h_embed_bigram(const i64h_embed_bigram_args* d, void* stream);
  *                       or with h_center the centred norm (u - mean) / sqrt(mean((u - mean)^2) + eps) * norm_w;  norm_b (may be NULL, [W])
  *                       is added behind the weight
  * rows (may be NULL, read only launches): h[m] is computed from row rows[m] of the streams (the rows whose logits are wanted).
- * h16 (may be NULL): the rows of h rounded to bf16 [n, W] (or [m_rows, W]), beside h or (h = NULL) in its place. */
+ * h16 (may be NULL): the rows of h rounded to bf16 [n, W] (or [m_rows, W]), beside h or (h = NULL) in its place.
+ * moe_y (may be NULL; one stream, no result norms, W % 4 == 0 up to 8192, 16-byte rows): a mixture's result stands for y, or is added to it in y2's
+ * place: what i64h_moe_combine gives for Y = moe_y, pair_row = moe_row, wgt = moe_wgt, h = moe_h, shared = moe_shared, shared_gate = moe_gate, top = moe_top. */
 typedef struct {
     float* streams;
     int32_t S;
@@ -280,6 +282,13 @@ typedef struct {
     const float* norm_b;
     const float* y_scale;
     void* h16;
+    const float* moe_y;
+    const int32_t* moe_row;
+    const float* moe_wgt;
+    const float* moe_h;
+    const float* moe_shared;
+    const float* moe_gate;
+    int32_t moe_top;
 } i64h_streams_args;
 int i64h_streams_step(const i64h_streams_args* d, void* stream);
 int i64h_set_residual_form(int32_t on); /* tuning / test knob: 1 (default) = one stream and results without norms of their own take the kernel that keeps the row in registers (16-byte rows) */
@@ -615,7 +624,8 @@ int i64h_route_topk(const i64h_route_args* d, void* stream);
  * i64h_moe_plan: from idx int32 [n, top] (entries >= experts are not experts and get no row) the (token, choice) pairs grouped by expert:
  *   group_off int32 [experts + 1] (ascending offsets), pair_token int32 [n * top] (the token of every grouped row, the a_rows of a grouped
  *   Linear), pair_row int32 [n, top] (where the pair's row lies, -1 for a non-expert).  The order of rows inside a group is not fixed;
- *   no result depends on it.  pair_wgt (fp32 [n * top], may be NULL): the choice's weight wgt[t, k] for every grouped row (row_scale of a
+ *   no result depends on it.  shared != 0: a group in front of the experts' that holds every token once (a shared expert in the same grouped
+ *   Linears: the rows [0, n), weight one) - group_off has one entry more, the grouped arrays n.  pair_wgt (fp32 [n * top], may be NULL): the choice's weight wgt[t, k] for every grouped row (row_scale of a
  *   grouped Linear, where the weight belongs on the expert's input).  One launch of one workgroup; experts <= 4096.
  * i64h_moe_combine: out[t, :] = sum_k wgt[t, k] * (pair_row[t, k] >= 0 ? Y[pair_row[t, k], :] : h[t, :]) + (shared ? shared[t, :] : 0),
  *   summed in the order k = 0 .. top - 1, the shared row last (wgt NULL: weights of one).  Y fp32 [pairs, W].  shared_gate (fp32 [n], may be NULL) multiplies the shared row. */
@@ -628,6 +638,7 @@ typedef struct {
     int32_t* pair_row;
     const float* wgt;
     float* pair_wgt;
+    int32_t shared;
 } i64h_moe_plan_args;
 int i64h_moe_plan(const i64h_moe_plan_args* d, void* stream);
 typedef struct {

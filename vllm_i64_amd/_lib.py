@@ -286,7 +286,8 @@ class Streams(ctypes.Structure):
     """Mirror of i64h_streams_args (include/i64h_dense.h)."""
     _fields_ = [("streams", _P), ("S", _I), ("n", _L), ("W", _I), ("y", _P), ("ldy", _L), ("y2", _P), ("ldy2", _L), ("yn_w", _P), ("y2n_w", _P),
                 ("y_eps", _F), ("mix", _P), ("out_w", _P), ("in_w", _P), ("norm_w", _P), ("norm_w_len", _I), ("eps", _F), ("h", _P), ("rows", _P),
-                ("m_rows", _L), ("post_w", _P), ("post_center", _I), ("h_center", _I), ("norm_b", _P), ("y_scale", _P), ("h16", _P)]
+                ("m_rows", _L), ("post_w", _P), ("post_center", _I), ("h_center", _I), ("norm_b", _P), ("y_scale", _P), ("h16", _P), ("moe_y", _P), ("moe_row", _P), ("moe_wgt", _P), ("moe_h", _P), ("moe_shared", _P),
+                ("moe_gate", _P), ("moe_top", _I)]
 
 
 class CausalConv(ctypes.Structure):
@@ -372,7 +373,7 @@ class Route(ctypes.Structure):
 
 class MoePlan(ctypes.Structure):
     """Mirror of i64h_moe_plan_args (include/i64h_dense.h)."""
-    _fields_ = [("idx", _P), ("n", _L), ("top", _I), ("experts", _I), ("group_off", _P), ("pair_token", _P), ("pair_row", _P), ("wgt", _P), ("pair_wgt", _P)]
+    _fields_ = [("idx", _P), ("n", _L), ("top", _I), ("experts", _I), ("group_off", _P), ("pair_token", _P), ("pair_row", _P), ("wgt", _P), ("pair_wgt", _P), ("shared", _I)]
 
 
 class MoeCombine(ctypes.Structure):

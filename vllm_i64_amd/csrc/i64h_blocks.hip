@@ -540,33 +540,41 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const i64h_moe_plan_args
     extern __shared__ int pl_lds[];   // [experts + 1] counts, then offsets; [experts] cursors
     int* cnt = pl_lds;
     int* cur = pl_lds + p.experts + 1;
-    const int tid = threadIdx.x;
-    const int64_t pairs = p.n * p.top;
-    for (int e = tid; e <= p.experts; e += 1024) cnt[e] = 0;
+    const int tid = threadIdx.x, E = p.experts;
+    const int64_t pairs = p.n * p.top, base = p.shared ? p.n : 0;
+    if (p.shared) {
+        if (tid == 0) p.group_off[0] = 0;
+        for (int64_t t = tid; t < p.n; t += 1024) {
+            p.pair_token[t] = (int)t;
+            if (p.pair_wgt) p.pair_wgt[t] = 1.0f;
+        }
+    }
+    int32_t* group_off = p.group_off + (p.shared ? 1 : 0);
+    for (int e = tid; e <= E; e += 1024) cnt[e] = 0;
     __syncthreads();
     for (int64_t i = tid; i < pairs; i += 1024) {
         const int e = p.idx[i];
-        if (e >= 0 && e < p.experts) atomicAdd(&cnt[e], 1);
+        if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);
     }
     __syncthreads();
     if (tid == 0) {
-        int run = 0;
-        for (int e = 0; e < p.experts; ++e) {
+        int run = (int)base;
+        for (int e = 0; e < E; ++e) {
             const int c = cnt[e];
             cnt[e] = run;
             cur[e] = run;
             run += c;
         }
-        cnt[p.experts] = run;
+        cnt[E] = run;
     }
     __syncthreads();
-    for (int e = tid; e <= p.experts; e += 1024) p.group_off[e] = cnt[e];
+    for (int e = tid; e <= E; e += 1024) group_off[e] = cnt[e];
     for (int64_t i = tid; i < pairs; i += 1024) {
         const int e = p.idx[i];
         int r = -1;
-        if (e >= 0 && e < p.experts) {
+        if (e >= 0 && e < E) {
             r = atomicAdd(&cur[e], 1);
-            p.pair_token[r] = (int)(i / p.top);
+            p.pair_token[r] = (int)((uint32_t)i / (uint32_t)p.top);
             if (p.pair_wgt) p.pair_wgt[r] = p.wgt[i];
         }
         p.pair_row[i] = r;
@@ -760,7 +768,7 @@ int i64h_moe_plan(const i64h_moe_plan_args* dp, void* stream) {
     const i64h_moe_plan_args& d = *dp;
     I64H_CHECK_ARG(d.experts > 0 && d.experts <= 4096 && d.top > 0 && d.n >= 0, "moe_plan: %d experts (at most 4096), top %d", d.experts, d.top);
     I64H_CHECK_ARG(d.idx && d.group_off && d.pair_token && d.pair_row, "moe_plan: null operand");
-    I64H_CHECK_ARG(d.n * d.top < (1ll << 31), "moe_plan: too many pairs");
+    I64H_CHECK_ARG(d.n * ((int64_t)d.top + 1) < (1ll << 31), "moe_plan: too many pairs");
     I64H_CHECK_ARG(!d.pair_wgt || d.wgt, "moe_plan: weights per row come from the weights per choice");
     hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(1024), (size_t)(2 * d.experts + 1) * 4, (hipStream_t)stream, d);
     I64H_CHECK_LAUNCH();

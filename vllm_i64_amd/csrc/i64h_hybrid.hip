@@ -197,7 +197,8 @@ __global__ __launch_bounds__(256) void residual_kernel(const i64h_streams_args p
     const int tid = threadIdx.x, W = p.W;
     const int64_t m = blockIdx.x;
     float* xs = p.streams + (p.rows ? (int64_t)p.rows[m] : m) * W;
-    const float ow = p.y ? p.out_w[0] : 0.0f;
+    const bool add = p.y || p.moe_y;
+    const float ow = add ? p.out_w[0] : 0.0f;
     float v[NV][4];
     float ss = 0.0f, su = 0.0f;
 #pragma unroll
@@ -208,9 +209,32 @@ __global__ __launch_bounds__(256) void residual_kernel(const i64h_streams_args p
         if (c >= W) continue;
         const float4 x = *(const float4*)(xs + c);
         v[i][0] = x.x, v[i][1] = x.y, v[i][2] = x.z, v[i][3] = x.w;
-        if (p.y) {
-            const float4 y = *(const float4*)(p.y + m * p.ldy + c);
-            float u[4] = {y.x, y.y, y.z, y.w};
+        if (add) {
+            float u[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (p.y) {
+                const float4 y = *(const float4*)(p.y + m * p.ldy + c);
+                u[0] = y.x, u[1] = y.y, u[2] = y.z, u[3] = y.w;
+            }
+            if (p.moe_y) {      // the sum of moe_combine_kernel, in its order; loads of four choices on their way together
+                const dn_v4f sh = p.moe_shared ? *(const dn_v4f*)(p.moe_shared + m * W + c) : dn_v4f{0, 0, 0, 0};
+                dn_v4f a = {0, 0, 0, 0};
+                for (int k0 = 0; k0 < p.moe_top; k0 += 4) {
+                    dn_v4f z[4];
+                    float wk[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const int kk = min(k0 + k, p.moe_top - 1), r = p.moe_row[m * p.moe_top + kk];
+                        z[k] = *(const dn_v4f*)(r >= 0 ? p.moe_y + (int64_t)r * W + c : p.moe_h + m * W + c);
+                        wk[k] = p.moe_wgt ? p.moe_wgt[m * p.moe_top + kk] : 1.0f;
+                    }
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (k0 + k < p.moe_top) a += wk[k] * z[k];
+                }
+                if (p.moe_shared) a += p.moe_gate ? p.moe_gate[m] * sh : sh;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) u[k] = p.y ? u[k] + a[k] : a[k];
+            }
             if (p.y2) {
                 const float4 z = *(const float4*)(p.y2 + m * p.ldy2 + c);
                 u[0] += z.x, u[1] += z.y, u[2] += z.z, u[3] += z.w;
@@ -865,16 +889,18 @@ int i64h_streams_step(const i64h_streams_args* dp, void* stream) {
     I64H_CHECK_ARG(dp != nullptr, "streams: no descriptor");
     const i64h_streams_args& d = *dp;
     I64H_CHECK_ARG(d.S >= 1 && d.S <= HY_MAX_STREAMS && d.W > 0 && d.n >= 0, "streams: %d streams (at most %d), width %d", d.S, HY_MAX_STREAMS, d.W);
-    I64H_CHECK_ARG(d.streams && (d.y || d.h || d.h16), "streams: nothing to do");
-    I64H_CHECK_ARG(!d.y || d.out_w, "streams: the write needs out_w");
+    I64H_CHECK_ARG(d.streams && (d.y || d.moe_y || d.h || d.h16), "streams: nothing to do");
+    I64H_CHECK_ARG(!(d.y || d.moe_y) || d.out_w, "streams: the write needs out_w");
     I64H_CHECK_ARG(!d.y2 || (d.y && !d.yn_w == !d.y2n_w), "streams: two results take both norm weights or none");
     I64H_CHECK_ARG(!(d.h || d.h16) || (d.norm_w && (d.norm_w_len == 1 || d.norm_w_len == d.W)), "streams: the read needs a norm weight of 1 or W values");
-    I64H_CHECK_ARG(!d.rows || !d.y, "streams: gathered rows are read only");
+    I64H_CHECK_ARG(!d.moe_y || (d.moe_row && d.moe_h && d.moe_top > 0 && !d.y2), "streams: a mixture's result needs its rows and choices, and no second result beside it");
+    I64H_CHECK_ARG(!d.rows || !(d.y || d.moe_y), "streams: gathered rows are read only");
     const int64_t rows = d.rows ? d.m_rows : d.n;
     const size_t lds = ((size_t)d.W + 4) * 4;
     I64H_CHECK_ARG(lds <= 64 * 1024, "streams: a row of %d values does not fit the kernel's LDS buffer", d.W);
     if (rows == 0) return 0;
-    const uintptr_t at = (uintptr_t)d.streams | (uintptr_t)d.y | (uintptr_t)d.y2 | (uintptr_t)d.y_scale | (uintptr_t)d.norm_w | (uintptr_t)d.norm_b | (uintptr_t)d.h | (uintptr_t)d.h16;
+    const uintptr_t at = (uintptr_t)d.streams | (uintptr_t)d.y | (uintptr_t)d.y2 | (uintptr_t)d.y_scale | (uintptr_t)d.norm_w | (uintptr_t)d.norm_b | (uintptr_t)d.h | (uintptr_t)d.h16 | (uintptr_t)d.moe_y |
+                         (uintptr_t)d.moe_h | (uintptr_t)d.moe_shared;
     if (g_residual_form && d.S == 1 && !d.mix && !d.in_w && !d.yn_w && !d.post_w && d.W % 4 == 0 && d.W <= 8 * 1024 && at % 16 == 0 && (!d.y || d.ldy % 4 == 0) &&
         (!d.y2 || d.ldy2 % 4 == 0) && (!(d.h || d.h16) || d.norm_w_len == d.W)) {
         const dim3 grid((unsigned)rows);
@@ -885,6 +911,7 @@ int i64h_streams_step(const i64h_streams_args* dp, void* stream) {
         I64H_CHECK_LAUNCH();
         return 0;
     }
+    I64H_CHECK_ARG(!d.moe_y, "streams: a mixture's result with several streams, result norms or rows that are not read 16 bytes at a time");
     hipLaunchKernelGGL(streams_kernel, dim3((unsigned)rows), dim3(256), lds, (hipStream_t)stream, d);
     I64H_CHECK_LAUNCH();
     return 0;

@@ -324,34 +324,45 @@ class HybridRunner:
         d["router"] = bf(router)
         d["router_b"] = self._f(need(p + "router.b", (f.entries,))) if f.router_bias else None
         # per expert [gate rows; up rows], all experts stacked: one grouped launch for the pair, one for the way down
-        d["gate_up"] = bf(torch.stack([torch.cat([need(f"{p}e{e}.gate", (f.ff, W)), need(f"{p}e{e}.up", (f.ff, W))], 0) for e in range(f.experts)]))
-        d["e_down"] = bf(torch.stack([need(f"{p}e{e}.down", (W, f.ff)) for e in range(f.experts)]))
-        if f.shared_ff:
+        # (a shared expert of the experts' size and activation is the first of the stack, its rows a group of all tokens)
+        d["merged"] = self._shared_in_stack(f)
+        names = ([p + "shared"] if d["merged"] else []) + [f"{p}e{e}" for e in range(f.experts)]
+        d["gate_up"] = bf(torch.stack([torch.cat([need(x + ".gate", (f.ff, W)), need(x + ".up", (f.ff, W))], 0) for x in names]))
+        d["e_down"] = bf(torch.stack([need(x + ".down", (W, f.ff)) for x in names]))
+        if d["merged"]:
+            d["s_gate_up"], d["s_down"] = d["gate_up"][0], d["e_down"][0]
+        elif f.shared_ff:
             s = f.shared_ff
             d["s_gate_up"] = bf(torch.cat([need(p + "shared.gate", (s, W)), need(p + "shared.up", (s, W))], 0))
             d["s_down"] = bf(need(p + "shared.down", (W, s)))
 
     @staticmethod
+    def _shared_in_stack(f) -> bool:
+        return bool(f.shared_ff) and f.shared_ff == f.ff and f.shared_limit == f.limit
+
+    @staticmethod
     def moe_buffers(B, model, n: int) -> None:
         """The step buffers of _moe_ff on B (model.max_top == 0: no mixtures)."""
         i32, f32 = dict(dtype=torch.int32, device=model.device), dict(dtype=torch.float32, device=model.device)
-        t = model.max_top
-        B.ey = torch.empty(n * t, model.cfg.width, **f32) if t else None   # the chosen experts' outputs, grouped by expert
+        t, g = model.max_top, model.max_grouped
+        B.ey = torch.empty(n * g, model.cfg.width, **f32) if t else None   # the outputs, grouped by expert
         B.idx = torch.empty(n * max(t, 1), **i32)
         B.wgt = torch.empty(n * max(t, 1), **f32)
-        B.pair_token = torch.empty(n * max(t, 1), **i32)
+        B.pair_token = torch.empty(n * max(g, 1), **i32)
         B.pair_row = torch.empty(n * max(t, 1), **i32)
-        B.pair_wgt = torch.empty(n * max(t, 1), **f32)
-        B.group_off = torch.empty(model.max_experts + 1, **i32)
+        B.pair_wgt = torch.empty(n * max(g, 1), **f32)
+        B.group_off = torch.empty(model.max_groups + 1, **i32)
         B.sgate = torch.empty(n, **f32)
         B.sact = torch.empty(n * max(model.max_shared, 1), **f32)
 
     def _moe_sizes(self, mlps) -> None:
         moes = [m for m in mlps if m is not None and m.kind == "moe"]
         self.max_top = max([m.top for m in moes] or [0])
-        self.max_experts = max([m.experts for m in moes] or [0])
+        self.max_groups = max([m.experts + int(self._shared_in_stack(m)) for m in moes] or [0])
         self.max_shared = max([m.shared_ff for m in moes] or [0])
-        self.max_act = max([m.ff for m in mlps if m is not None and m.kind == "dense"] + [m.ff * m.top for m in moes] + [0])
+        grouped = [m.top + int(self._shared_in_stack(m)) for m in moes]      # rows a token has in the grouped Linears
+        self.max_grouped = max(grouped or [0])
+        self.max_act = max([m.ff for m in mlps if m is not None and m.kind == "dense"] + [m.ff * g for m, g in zip(moes, grouped)] + [0])
 
     @staticmethod
     def _glu(limit: float, alpha: float) -> dict:
@@ -376,29 +387,45 @@ class HybridRunner:
         D.linear(h, d["ff_gate_up"], act, a16=h16, out16=act16, exact=self.exact, **self._glu(f.limit, f.glu_alpha))
         D.linear(act, d["ff_down"], out, a16=act16, exact=self.exact)
 
-    def _moe_ff(self, B, d, n, h, out, shared_out, record: Optional[dict] = None, tag: str = "", beside: bool = False, h16=None) -> None:
-        """out <- the mixture of d["mlp"] on h fp32 [n, width] (h16: its rows in bf16, which the experts read); shared_out [n, width] receives the shared expert's rows on the way (beside: on
-        the side stream, while the routed experts run)."""
+    def _moe_merges(self) -> bool:
+        """Whether the residual's launch sums a mixture's rows itself (i64h_streams_args.moe_y)."""
+        return self.cfg.width % 4 == 0 and self.cfg.width <= 8192
+
+    def _moe_ff(self, B, d, n, h, out, shared_out, record: Optional[dict] = None, tag: str = "", beside: bool = False, h16=None, combine: bool = True):
+        """out <- the mixture of d["mlp"] on h fp32 [n, width] (h16: its rows in bf16, which the experts read); shared_out [n, width] receives the rows of a
+        shared expert that is not in the experts' stack on the way (beside: on the side stream, while the routed experts run).  combine False: the
+        weighted sum is left to the caller's residual launch, whose operands are returned."""
         f, ex, W = d["mlp"], self.exact, self.cfg.width
         E, top = f.experts, f.top
+        # a shared expert in the experts' stack joins their launches, but where it can run beside the choice and the plan of much work (8 prompts of
+        # 512, width 1024: 3572 us a step joined, 3432 beside; where the whole feed-forward runs beside a mixer joined is better, 5593 and 5804)
+        merged = d["merged"] and not (beside and n * W >= self.FORK_WORK)
         gate = B.sgate if f.shared_ff and f.shared_gate else None
         shared = None
-        if f.shared_ff:
+        if f.shared_ff and not merged:
             with self._beside(n) if beside else nullcontext():
                 sact, sact16 = self._act(B.sact, n, f.shared_ff, h16)
                 D.linear(h, d["s_gate_up"], sact, a16=h16, out16=sact16, exact=ex, **self._glu(f.shared_limit, f.glu_alpha))
                 shared = D.linear(sact, d["s_down"], shared_out, a16=sact16, exact=ex)
+        gate_up, e_down = (d["gate_up"], d["e_down"]) if merged or not d["merged"] else (d["gate_up"][1:], d["e_down"][1:])
         # the router's products in 32 bits in both modes (a choice between experts is not rounding's to make), inside the choice's launch
         D.route_topk(None, h=h, w=d["router"], entries=f.entries, correction=d.get("correction"), groups=f.groups, keep=f.keep, top=top, scale=f.scale,
                      idx=B.idx, wgt=B.wgt, n=n, bias=d["router_b"], chosen_softmax=f.chosen_softmax, gate_out=gate, sigmoid_scores=f.sigmoid_scores, raw_weights=f.raw_weights)
         if record is not None:
             record[f"{tag}.route"] = B.idx[: n * top].view(n, top).clone()
         pair_wgt = B.pair_wgt if f.weigh_input else None      # the weight multiplies what the expert reads, not what it returns
-        D.moe_plan(B.idx, n=n, top=top, experts=E, group_off=B.group_off, pair_token=B.pair_token, pair_row=B.pair_row, wgt=B.wgt, pair_wgt=pair_wgt)
+        D.moe_plan(B.idx, n=n, top=top, experts=E, group_off=B.group_off, pair_token=B.pair_token, pair_row=B.pair_row, wgt=B.wgt, pair_wgt=pair_wgt, shared=merged)
         # the (token, expert) pairs lie grouped by expert: one launch runs every expert over its own rows, the counts stay on the device
-        act, act16 = self._act(B.act, n * top, f.ff, h16)
-        D.linear(h, d["gate_up"], act, a16=h16, out16=act16, m=n, a_rows=B.pair_token, batch=E, w_batch=2 * f.ff * W, exact=ex, group_off=B.group_off, row_scale=pair_wgt, **self._glu(f.limit, f.glu_alpha))
-        D.linear(act, d["e_down"], B.ey, a16=act16, m=n, batch=E, w_batch=W * f.ff, exact=ex, group_off=B.group_off)
+        rows, groups = n * (top + int(merged)), E + int(merged)
+        act, act16 = self._act(B.act, rows, f.ff, h16)
+        D.linear(h, gate_up, act, a16=h16, out16=act16, m=n, a_rows=B.pair_token[:rows], batch=groups, w_batch=2 * f.ff * W, exact=ex, group_off=B.group_off, row_scale=pair_wgt,
+                 **self._glu(f.limit, f.glu_alpha))
+        D.linear(act, e_down, B.ey[:rows], a16=act16, m=n, batch=groups, w_batch=W * f.ff, exact=ex, group_off=B.group_off)
         if shared is not None and beside:
             self._meet(n)
-        D.moe_combine(B.ey, B.pair_row, None if f.weigh_input else B.wgt, h, shared, out, n=n, top=top, width=W, shared_gate=gate)
+        if merged:
+            shared = B.ey[:n]
+        sums = dict(y=B.ey, pair_row=B.pair_row, wgt=None if f.weigh_input else B.wgt, h=h, shared=shared, top=top, shared_gate=gate)
+        if not combine:
+            return sums
+        D.moe_combine(sums.pop("y"), sums.pop("pair_row"), sums.pop("wgt"), sums.pop("h"), sums.pop("shared"), out, n=n, width=W, **sums)

@@ -235,11 +235,12 @@ def streams_step(streams: torch.Tensor, *, y: Optional[torch.Tensor] = None, y2:
                  in_w: Optional[torch.Tensor] = None, norm_w: Optional[torch.Tensor] = None, eps: float = 0.0, h: Optional[torch.Tensor] = None,
                  rows: Optional[torch.Tensor] = None, post_w: Optional[torch.Tensor] = None, post_center: bool = False,
                  h_center: bool = False, norm_b: Optional[torch.Tensor] = None, y_scale: Optional[torch.Tensor] = None,
-                 h16: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+                 h16: Optional[torch.Tensor] = None, moe: Optional[dict] = None) -> Optional[torch.Tensor]:
     """See i64h_streams_step.  streams fp32 [S, n, W], updated in place when y is given; h fp32 [n, W] (or [rows, W]).  post_w fp32 [W]: a
     norm over the result as a whole (centred with post_center) before it is added; h_center: the read's norm is centred; norm_b: added behind
     the read's norm weight.  y2 without norm weights is simply added to y.  y_scale fp32 [W]: a factor per column on what is added.
-    h16 bf16 [n, W]: the rows of h rounded, beside h or (h None) in its place."""
+    h16 bf16 [n, W]: the rows of h rounded, beside h or (h None) in its place.  moe (one stream, no result norms): the arguments of moe_combine but `out`, whose
+    result stands for y or is added to it."""
     _chk(streams, torch.float32, "streams")
     S, n, W = streams.shape
     for t, name in ((y, "y"), (y2, "y2"), (yn_w, "yn_w"), (y2n_w, "y2n_w"), (mix, "mix"), (out_w, "out_w"), (in_w, "in_w"), (norm_w, "norm_w"), (h, "h"),
@@ -265,10 +266,15 @@ def streams_step(streams: torch.Tensor, *, y: Optional[torch.Tensor] = None, y2:
         _chk(h16, torch.bfloat16, "h16")
         if h16.numel() < m_rows * W:
             raise _lib.I64HError("streams_step: h16 smaller than the rows it receives")
+    mk = {}
+    if moe is not None:
+        _moe_ok(moe["y"], moe["pair_row"], moe["wgt"], moe["h"], moe["shared"], n, moe["top"], W, moe.get("shared_gate"), "streams_step")
+        mk = dict(moe_y=ptr(moe["y"]), moe_row=ptr(moe["pair_row"]), moe_wgt=ptr(moe["wgt"]), moe_h=ptr(moe["h"]), moe_shared=ptr(moe["shared"]),
+                  moe_gate=ptr(moe.get("shared_gate")), moe_top=moe["top"])
     d = _lib.Streams(streams=ptr(streams), S=S, n=n, W=W, y=ptr(y), ldy=W, y2=ptr(y2), ldy2=W, yn_w=ptr(yn_w), y2n_w=ptr(y2n_w), y_eps=float(y_eps),
                      mix=ptr(mix), out_w=ptr(out_w), in_w=ptr(in_w), norm_w=ptr(norm_w), norm_w_len=norm_w.numel() if norm_w is not None else 0,
                      eps=float(eps), h=ptr(h), rows=ptr(rows), m_rows=m_rows, post_w=ptr(post_w), post_center=int(bool(post_center)), h_center=int(bool(h_center)),
-                     norm_b=ptr(norm_b), y_scale=ptr(y_scale), h16=ptr(h16))
+                     norm_b=ptr(norm_b), y_scale=ptr(y_scale), h16=ptr(h16), **mk)
     call_dense("i64h_streams_step", _ref(d), _stream())
     return h
 
@@ -639,34 +645,42 @@ def route_topk(logits: Optional[torch.Tensor], *, entries: int, correction: Opti
 
 
 def moe_plan(idx: torch.Tensor, *, n: int, top: int, experts: int, group_off: torch.Tensor, pair_token: torch.Tensor, pair_row: torch.Tensor,
-             wgt: Optional[torch.Tensor] = None, pair_wgt: Optional[torch.Tensor] = None) -> None:
-    """See i64h_moe_plan.  pair_wgt fp32 [n * top] receives the choices' weights wgt fp32 [n, top] in the grouped order."""
+             wgt: Optional[torch.Tensor] = None, pair_wgt: Optional[torch.Tensor] = None, shared: bool = False) -> None:
+    """See i64h_moe_plan.  pair_wgt fp32 [n * top] receives the choices' weights wgt fp32 [n, top] in the grouped order.  shared: one more group, in
+    front, of every token once."""
+    rows = n * top + (n if shared else 0)
     if pair_wgt is not None:
         _chk(wgt, torch.float32, "wgt"), _chk(pair_wgt, torch.float32, "pair_wgt")
-        if min(wgt.numel(), pair_wgt.numel()) < n * top:
+        if wgt.numel() < n * top or pair_wgt.numel() < rows:
             raise _lib.I64HError("moe_plan: fewer weights than choices")
     for t, name in ((idx, "idx"), (group_off, "group_off"), (pair_token, "pair_token"), (pair_row, "pair_row")):
         _chk(t, torch.int32, name)
-    if idx.numel() < n * top or group_off.numel() < experts + 1 or pair_token.numel() < n * top or pair_row.numel() < n * top:
+    if idx.numel() < n * top or group_off.numel() < experts + 1 + int(bool(shared)) or pair_token.numel() < rows or pair_row.numel() < n * top:
         raise _lib.I64HError("moe_plan: shapes do not fit the sizes")
     d = _lib.MoePlan(idx=ptr(idx), n=n, top=top, experts=experts, group_off=ptr(group_off), pair_token=ptr(pair_token), pair_row=ptr(pair_row),
-                     wgt=ptr(wgt) if pair_wgt is not None else 0, pair_wgt=ptr(pair_wgt))
+                     wgt=ptr(wgt) if pair_wgt is not None else 0, pair_wgt=ptr(pair_wgt), shared=int(bool(shared)))
     call_dense("i64h_moe_plan", _ref(d), _stream())
+
+
+def _moe_ok(y, pair_row, wgt, h, shared, n: int, top: int, width: int, shared_gate, who: str) -> None:
+    if shared_gate is not None:
+        _chk(shared_gate, torch.float32, "shared_gate")
+        _rows_ok(who, n, shared_gate)
+    _chk(y, torch.float32, "y"), _chk(pair_row, torch.int32, "pair_row"), _chk(h, torch.float32, "h")
+    for t, name in ((wgt, "wgt"), (shared, "shared")):
+        if t is not None:
+            _chk(t, torch.float32, name)
+    if min(h.numel(), shared.numel() if shared is not None else h.numel()) < n * width or min(pair_row.numel(), wgt.numel() if wgt is not None else pair_row.numel()) < n * top or \
+            y.numel() < n * top * width:
+        raise _lib.I64HError(f"{who}: shapes do not fit the sizes")
 
 
 def moe_combine(y: torch.Tensor, pair_row: torch.Tensor, wgt: Optional[torch.Tensor], h: torch.Tensor, shared: Optional[torch.Tensor], out: torch.Tensor, *,
                 n: int, top: int, width: int, shared_gate: Optional[torch.Tensor] = None) -> torch.Tensor:
     """See i64h_moe_combine.  y fp32 [pairs, width]; h, shared, out fp32 [n, width]; shared_gate fp32 [n]; wgt None: weights of one."""
-    if shared_gate is not None:
-        _chk(shared_gate, torch.float32, "shared_gate")
-        _rows_ok("moe_combine", n, shared_gate)
-    _chk(y, torch.float32, "y"), _chk(pair_row, torch.int32, "pair_row"), _chk(h, torch.float32, "h"), _chk(out, torch.float32, "out")
-    if wgt is not None:
-        _chk(wgt, torch.float32, "wgt")
-    if shared is not None:
-        _chk(shared, torch.float32, "shared")
-    if min(h.numel(), out.numel(), shared.numel() if shared is not None else out.numel()) < n * width or min(pair_row.numel(), wgt.numel() if wgt is not None else pair_row.numel()) < n * top or \
-            y.numel() < n * top * width:
+    _moe_ok(y, pair_row, wgt, h, shared, n, top, width, shared_gate, "moe_combine")
+    _chk(out, torch.float32, "out")
+    if out.numel() < n * width:
         raise _lib.I64HError("moe_combine: shapes do not fit the sizes")
     d = _lib.MoeCombine(Y=ptr(y), pair_row=ptr(pair_row), wgt=ptr(wgt), h=ptr(h), shared=ptr(shared), out=ptr(out), n=n, top=top, W=width,
                         shared_gate=ptr(shared_gate))

@@ -133,11 +133,13 @@ class PukatarModel(HybridRunner):
             self._load_moe(p + "mlp.", ff, need, d)
         return d
 
-    def _feed_forward(self, B, d, n, record, r, h16=None) -> None:
+    def _feed_forward(self, B, d, n, record, r, h16=None, combine=True) -> dict:
+        """Returns what the residual's write adds to the mixer's result (combine: the result itself in B.y2)."""
         if d["mlp"].kind == "dense":
             self._dense_glu(B, d, n, B.h, B.y2, h16)
-        else:
-            self._moe_ff(B, d, n, B.h, B.y2, B.y3, record, f"r{r}", h16=h16)
+            return dict(y2=B.y2)
+        sums = self._moe_ff(B, d, n, B.h, B.y2, B.y3, record, f"r{r}", h16=h16, combine=combine)
+        return dict(y2=B.y2) if combine else dict(moe=sums)
 
     @torch.no_grad()
     def forward(self, token_ids: torch.Tensor, positions: torch.Tensor, slot_ids: torch.Tensor, ctx_len: Optional[torch.Tensor] = None,
@@ -184,7 +186,7 @@ class PukatarModel(HybridRunner):
             # mixer and feed-forward read the same input and meet at the residual: they run side by side
             if d["mlp"] is not None:
                 with self._beside(n):
-                    self._feed_forward(B, d, n, record, r, B.h16)
+                    ff = self._feed_forward(B, d, n, record, r, B.h16, not self._moe_merges())
             P = B.p[: n * d["ld"]].view(n, d["ld"])
             D.linear(B.h, d["w_in"], P, a16=B.h16, exact=ex)
             if d["type"] == "attention":
@@ -193,7 +195,7 @@ class PukatarModel(HybridRunner):
                 self._gated_delta(B, d, d["m"], P, r, n, positions, slot_ids, kvc, seg, nseg, single, B.y)
             write = dict(y=B.y, out_w=self.ones1)
             if d["mlp"] is not None:
-                write["y2"] = B.y2
+                write.update(ff)
                 self._meet(n)
             if r + 1 < len(self.layer_runs) and self.layer_runs[r + 1][1] is None:
                 write.update(normed(self.layers[self.layer_runs[r + 1][0]]))

@@ -141,11 +141,13 @@ class VepelixModel(HybridRunner):
         self._meet(n)
         return dict(y=B.y, y2=B.y2)
 
-    def _feed_forward(self, B, d, n, record, r, h16=None) -> None:
+    def _feed_forward(self, B, d, n, record, r, h16=None, combine=True) -> dict:
+        """Returns the operands of the residual's write (combine: the result itself in B.y)."""
         if d["mlp"].kind == "dense":
             self._dense_glu(B, d, n, B.h, B.y, h16)
-        else:
-            self._moe_ff(B, d, n, B.h, B.y, B.y2, record, f"r{r}", beside=True, h16=h16)
+            return dict(y=B.y)
+        sums = self._moe_ff(B, d, n, B.h, B.y, B.y2, record, f"r{r}", beside=True, h16=h16, combine=combine)
+        return dict(y=B.y) if combine else dict(moe=sums)
 
     @torch.no_grad()
     def forward(self, token_ids: torch.Tensor, positions: torch.Tensor, slot_ids: torch.Tensor, ctx_len: Optional[torch.Tensor] = None,
@@ -185,8 +187,8 @@ class VepelixModel(HybridRunner):
             write.update(out_w=self.ones1, y_scale=d["ls1"])
             if d["mlp"] is not None:
                 D.streams_step(x, **write, **(normed(d["norm2"]) if d["mlp"].kind == "dense" else read(d["norm2"], B.h, h16=B.h16)))
-                self._feed_forward(B, d, n, record, r, B.h16)
-                write = dict(y=B.y, out_w=self.ones1, y_scale=d["ls2"])
+                write = self._feed_forward(B, d, n, record, r, B.h16, not self._moe_merges())
+                write.update(out_w=self.ones1, y_scale=d["ls2"])
             if r + 1 < len(self.layer_runs) and not self.layer_runs[r + 1][1]:
                 write.update(normed(self.layers[self.layer_runs[r + 1][0]]["norm1"]))
             D.streams_step(x, **write)
