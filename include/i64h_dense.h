@@ -482,7 +482,8 @@ int i64h_kv_prep(const i64h_kv_prep_args* d, void* stream);
  * k_t = 1 - f_t (the forget gate also decides what is written).  state fp32 [slots, heads, vdim, dim] (S transposed; dim <= 256).
  * i64h_gla_gates prepares q and f in place:  q <- q_act ? silu(q) : q;   f <- lower + (1 - lower) * sigmoid(f)   (lower fp32 [heads * dim] or NULL = 0).
  * The scan multiplies its read-out by q_scale.  F: decays that are no columns of P (see I64H_EPI_DECAY).
- * All arithmetic fp32, the tokens of a sequence strictly in their order.  Runs of many rows with separate keys are staged through LDS. */
+ * All arithmetic fp32, the tokens of a sequence strictly in their order.  Runs of many rows with separate keys are staged through LDS,
+ * or (work) summed in tiles as i64h_gdn_scan's. */
 typedef struct {
     float* P;
     int64_t ldp;
@@ -501,6 +502,8 @@ typedef struct {
     const float* F;      /* the decays in a matrix of their own (fp32, row stride ldf, columns [f_off, + heads * dim)); NULL: columns of P */
     int64_t ldf;
     float q_scale;       /* multiplies the read-out S^T q (scan only) */
+    float* work;         /* as in i64h_gdn_args */
+    int64_t work_floats;
 } i64h_gla_args;
 int i64h_gla_gates(const i64h_gla_args* d, void* stream);
 int i64h_gla_scan(const i64h_gla_args* d, void* stream);
@@ -561,7 +564,8 @@ int i64h_rot_post(const i64h_rot_post_args* d, void* stream);
  * i64h_gdn_gates prepares them: q and k of every query / key head divided by sqrt(sum of squares + unit_eps) in place (unit_eps < 0: left as
  * they are), q times q_scale;  G[t, a] = sigmoid(R[t, b_off + a]),  G[t, heads + a] = exp(-exp(A_log[a]) * softplus(R[t, a_off + a] + dt_bias[a]))
  * (a_off < 0: no decay per head is computed - the caller's F holds one per channel, see I64H_EPI_DECAY).
- * state fp32 [slots, heads, vdim, dim] (S transposed; dim <= 256).  All arithmetic fp32, the tokens of a sequence strictly in their order. */
+ * state fp32 [slots, heads, vdim, dim] (S transposed; dim <= 256).  All arithmetic fp32, the tokens of a sequence strictly in their order;
+ * with a workspace (work) long runs in tiles of 16 tokens from the run's first row on: the same values in another order of the sums. */
 typedef struct {
     float* X;
     int64_t ldx;
@@ -584,11 +588,15 @@ typedef struct {
     int64_t n;
     const float* F;
     int64_t ldf;
+    float* work;         /* scan only, may be NULL: at least i64h_scan_work_floats floats, 16-byte aligned - long runs may then be summed in tiles */
+    int64_t work_floats;
 } i64h_gdn_args;
 int i64h_gdn_gates(const i64h_gdn_args* d, void* stream);
 int i64h_gdn_scan(const i64h_gdn_args* d, void* stream);
+int64_t i64h_scan_work_floats(int64_t n, int32_t nseg, int32_t heads, int32_t dim);
 int i64h_set_gdn_scan_form(int32_t form); /* tuning / test knob: 0 (default) = by the runs' length; 1 = loads straight into registers; 2, 3, 4 = staged
-                                             through LDS with 1, 2, 4 value columns per lane (where 16-byte rows allow); same results bit for bit */
+                                             through LDS with 1, 2, 4 value columns per lane (where 16-byte rows allow); same results bit for bit.
+                                             5 = tiles of 16 tokens whatever the runs' length (with work, 16-byte rows, keys of their own) */
 
 /* ---- router: softmax scores, corrected choice, groups of neighbours, top-k ---------------------------------------------------------------------
  * Per row t of logits (fp32, row stride ld, E entries):  s = softmax(logits[t]);  choice = s + correction (correction may be NULL);

@@ -19,7 +19,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libi64hip.so")
 DENSE_OUT = os.path.join(HERE, "libi64hip_dense.so")
-DENSE_SOURCES = ["i64h_api.hip", "i64h_dense.hip", "i64h_linear_block.hip", "i64h_linear_wide.hip", "i64h_latent.hip", "i64h_hybrid.hip", "i64h_blocks.hip"]
+DENSE_SOURCES = ["i64h_api.hip", "i64h_dense.hip", "i64h_linear_block.hip", "i64h_linear_wide.hip", "i64h_latent.hip", "i64h_hybrid.hip", "i64h_blocks.hip", "i64h_scan_tile.hip"]
 SOURCES = ["i64h_api.hip", "i64h_route.hip", "i64h_quant.hip", "i64h_norm.hip", "i64h_gemm.hip", "i64h_gemm_os.hip", "i64h_attn.hip", "i64h_moe.hip", "i64h_fp8.hip", "i64h_fp8_tile.hip", "i64h_kv.hip", "i64h_decode.hip", "i64h_variants.hip", "i64h_group_f32.hip", "i64h_lmhead.hip"]
 # -ffp-contract=off: a*b+c stays two roundings unless the source says fmaf, so fp32 element-wise math has the
 # same rounding steps as the reference's CPU ops.
@@ -31,7 +31,7 @@ FLAGS = ["-O3", "--offload-arch=gfx950", "-fPIC", "-std=c++17", "-ffp-contract=o
 
 # per-file extras.  MFMA accumulators that element-wise code reads right after the matrix instructions (softmax on the
 # scores, rescaling of the output tile) stay in ordinary VGPRs instead of being copied out of the accumulator registers.
-EXTRA = {"i64h_attn.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}  # measured: no gain for the int8 GEMMs
+EXTRA = {"i64h_attn.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "i64h_scan_tile.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}  # measured: no gain for the int8 GEMMs
 
 
 def _stale(obj: str, src: str) -> bool:

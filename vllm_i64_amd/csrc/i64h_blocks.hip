@@ -12,6 +12,8 @@
 #include "i64h_common.h"
 #include "i64h_dense.h"
 
+int i64h_scan_tiles(const i64h_gdn_args& d, bool delta, void* stream);      // i64h_scan_tile.hip
+
 __device__ __forceinline__ float bl_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
 
 // ---------------------------------------------------------------------------------------------------------------------------
@@ -649,7 +651,7 @@ int i64h_gdn_gates(const i64h_gdn_args* dp, void* stream) {
 
 static int g_gdn_form = 0;
 int i64h_set_gdn_scan_form(int32_t form) {
-    I64H_CHECK_ARG(form >= 0 && form <= 4, "gdn_scan: form %d", form);
+    I64H_CHECK_ARG(form >= 0 && form <= 5, "gdn_scan: form %d", form);
     g_gdn_form = form;
     return 0;
 }
@@ -664,6 +666,17 @@ static int gdn_launch(const i64h_gdn_args& d, void* stream) {
                (!d.F || (d.ldf % 4 == 0 && (uintptr_t)d.F % 16 == 0));
     };
     const int kround = kpt <= 4 ? 4 : (kpt <= 8 ? 8 : 16);
+    // Tiles of 16 tokens on the matrix cores: two launches, so that a few dozen rows stay with the chain from token to token.  Microseconds, token by
+    // token | in tiles, delta rule (linear attention), heads of 128: 16 heads, a run of 1531 rows 242 | 130 (214 | 81), 27 single rows beside 229 and 256
+    // 65 | 59 (56 | 41), 40 beside 300 75 | 64; 8 heads, 8 runs of 512 120 | 82 (100 | 57), runs of 300, 75 and 1 51 | 32; 77 rows 16 | 17, 24 rows 10 | 14.
+    // Many short runs are little more than reading and writing their states, and a tile of them is mostly empty: 64 of 17 rows, 32 heads of 64, 43 | 62.
+    const bool tiles = d.n >= 96 && d.n >= 8 * (int64_t)d.nseg && (d.n >= 32 * (int64_t)d.nseg || (int64_t)d.heads * ((d.vdim + 15) / 16) * d.nseg < 6144);
+    if (RULE != GD_FORGET && d.work && ((g_gdn_form == 0 && tiles) || g_gdn_form == 5) && vec_ok(4) && (uintptr_t)d.work % 16 == 0 && d.ldx < (1 << 25) &&
+        (d.n / 16 + d.nseg) * (int64_t)d.heads < (1ll << 31)) {
+        I64H_CHECK_ARG(d.work_floats >= i64h_scan_work_floats(d.n, d.nseg, d.heads, d.dim), "scan: a workspace of %lld floats, %lld needed", (long long)d.work_floats,
+                       (long long)i64h_scan_work_floats(d.n, d.nseg, d.heads, d.dim));
+        return i64h_scan_tiles(d, RULE == GD_DELTA, stream);
+    }
     if (g_gdn_form != 1 && vec_ok(kround) && (g_gdn_form > 1 || d.n >= 8 * (int64_t)d.nseg)) {
         // One value column per lane: a token then takes the longest run least time, and it is the longest run that the launch waits for (16
         // heads of 128, runs of 1531, 257, 64, 3 and 1101 rows: 264 us, two columns 448; 27 single rows beside 229 and 256: 68 and 100).  Two
@@ -740,6 +753,7 @@ int i64h_gla_scan(const i64h_gla_args* dp, void* stream) {
     a.X = d.P, a.ldx = d.ldp, a.q_off = d.q_off, a.k_off = d.k_off >= 0 ? d.k_off : 0, a.v_off = d.v_off, a.heads = a.kv_heads = d.heads, a.dim = d.dim, a.vdim = d.vdim;
     a.F = (d.F ? d.F : d.P) + d.f_off, a.ldf = d.F ? d.ldf : d.ldp, a.q_scale = d.q_scale, a.seg_start = d.seg_start, a.nseg = d.nseg;
     a.positions = d.positions, a.slot_ids = d.slot_ids, a.state = d.state, a.out = d.out, a.ldo = d.ldo, a.n = d.n;
+    a.work = d.work, a.work_floats = d.work_floats;
     return d.k_off >= 0 ? gdn_launch<GD_KEYS>(a, stream) : gdn_launch<GD_FORGET>(a, stream);
 }
 

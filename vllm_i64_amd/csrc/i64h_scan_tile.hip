@@ -1,0 +1,327 @@
+// The recurrences of i64h_gdn_scan (delta rule) and i64h_gla_scan (keys of their own), runs of rows in tiles of 16 tokens on the 32-bit matrix
+// instruction (include/i64h_dense.h).  With P_t the product of a tile's decays up to token t (per key channel), S the state in front of the tile:
+//   scan_pairs_kernel : per tile and head k P, q P and k P_16 / P as the operands' registers hold them, and what tokens of a tile are to each other: A_ts = sum_c k_t k_s P_t / P_s (s < t) and B_ts with q_t in
+//                       k_t's place (s <= t), the quotients as running products of the decays between (nothing is divided: decays may underflow);
+//                       delta rule: T = (1 + diag(beta) A)^-1 diag(beta) by forward substitution
+//   scan_tile_kernel  : U = T (V - (k P)^T S)  (linear attention: U = V);   O = (q P)^T S + B U;   S <- P_16 S + (k P_16 / P)^T U
+// Every product's result already lies in the registers as the next product's operand (which of a product's terms an instruction sums is free), so
+// a tile is a chain of matrix instructions; four waves share the key channels and meet once a tile, in LDS.
+// All arithmetic fp32.  A row that holds no finite number reaches no token before it, as in the scans token by token.
+#include <type_traits>
+
+#include "i64h_common.h"
+#include "i64h_dense.h"
+
+typedef float stf4 __attribute__((ext_vector_type(4)));
+enum { ST_TOK = 16, ST_PAIR = ST_TOK * ST_TOK };
+
+// tile `i` of run `seg` keeps its pairs at slot (r0 >> 4) + seg + i: slots of different runs never meet, and there are at most n / 16 + nseg
+__device__ __forceinline__ int64_t st_slot(int64_t r0, int seg) { return (r0 >> 4) + seg; }
+
+// what one tile of a head leaves for the scan, in floats: three operands, P_16, B and (delta rule) T
+__host__ __device__ constexpr int st_floats(int NP) { return 3 * ST_TOK * NP + NP + 2 * ST_PAIR; }
+
+// One workgroup per (slot, head), 154 MB through memory for 3008 rows and 16 heads of 128 (38 us): 16 lanes walk from a token s to the tile's end, k_s times the decays so far in their registers; then a thread per
+// channel takes the products from the tile's start and from its end.
+template <int NP, bool DELTA>
+__global__ __launch_bounds__(256) void scan_pairs_kernel(const i64h_gdn_args p) {
+    constexpr int KPT = NP / 16, LD = NP + 4;
+    __shared__ __attribute__((aligned(16))) float sF[ST_TOK][LD], sK[ST_TOK][LD], sQ[ST_TOK][LD];
+    __shared__ float sA[ST_TOK][ST_TOK + 1], sB[ST_TOK][ST_TOK + 1], sBeta[ST_TOK];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int a = blockIdx.x % p.heads, slot = blockIdx.x / p.heads, N = p.dim;
+    int seg = -1;
+    for (int b = 0; b < p.nseg; b += 64) {      // the last run that starts at or before this slot (run starts grow)
+        const int s = b + lane;
+        const int c = __popcll(__ballot(s < p.nseg && st_slot(p.seg_start[min(s, p.nseg - 1)], s) <= slot));
+        seg += c;
+        if (c < 64) break;
+    }
+    if (seg < 0) return;
+    const int64_t r0 = p.seg_start[seg], r1 = p.seg_start[seg + 1];
+    const int64_t t0 = r0 + ST_TOK * (slot - st_slot(r0, seg));
+    if (t0 >= r1) return;      // (the whole workgroup)
+    const int kh = a / (p.heads / p.kv_heads);
+#pragma unroll
+    for (int e = tid; e < ST_TOK * NP / 4; e += 256) {      // (tokens behind the run's end neither decay, write nor read; nor do channels behind the last)
+        const int i = e / (NP / 4), c = e % (NP / 4) * 4;
+        const int64_t t = t0 + i;
+        const bool ok = t < r1 && c < N;
+        const stf4 zero = (stf4)0.0f;
+        const float* row = p.X + t * p.ldx + kh * N + c;
+        *(stf4*)&sK[i][c] = ok ? *(const stf4*)(row + p.k_off) : zero;
+        *(stf4*)&sQ[i][c] = ok ? *(const stf4*)(row + p.q_off) : zero;
+        if (p.F) *(stf4*)&sF[i][c] = ok ? *(const stf4*)(p.F + t * p.ldf + a * N + c) : (stf4)1.0f;
+        else *(stf4*)&sF[i][c] = (stf4)(t < r1 ? p.G[t * 2 * p.heads + p.heads + a] : 1.0f);
+    }
+    if (DELTA && tid < ST_TOK) sBeta[tid] = t0 + tid < r1 ? p.G[(t0 + tid) * 2 * p.heads + a] : 0.0f;
+    __syncthreads();
+    {
+        const int s = tid >> 4, l = tid & 15;
+        stf4 wk[KPT / 4];
+#pragma unroll
+        for (int i = 0; i < KPT / 4; ++i) wk[i] = *(const stf4*)&sK[s][4 * l + 64 * i];
+        auto walk = [&](int t, bool on) {
+            float x0 = 0.0f, x1 = 0.0f, y0 = 0.0f, y1 = 0.0f;
+#pragma unroll
+            for (int i = 0; i < KPT / 4; ++i) {
+                const stf4 f = *(const stf4*)&sF[t][4 * l + 64 * i], q = *(const stf4*)&sQ[t][4 * l + 64 * i];
+                wk[i] = on ? wk[i] * f : wk[i];
+                y0 = fmaf(wk[i][0], q[0], y0), y1 = fmaf(wk[i][1], q[1], y1), y0 = fmaf(wk[i][2], q[2], y0), y1 = fmaf(wk[i][3], q[3], y1);
+                if (DELTA) {
+                    const stf4 k = *(const stf4*)&sK[t][4 * l + 64 * i];
+                    x0 = fmaf(wk[i][0], k[0], x0), x1 = fmaf(wk[i][1], k[1], x1), x0 = fmaf(wk[i][2], k[2], x0), x1 = fmaf(wk[i][3], k[3], x1);
+                }
+            }
+            const float y = group_sum(y0 + y1, 16), x = DELTA ? group_sum(x0 + x1, 16) : 0.0f;
+            if (l == 0) {
+                sB[t][s] = y;
+                if (DELTA) sA[t][s] = x;
+            }
+        };
+        for (int t = 4 * w; t < 4 * w + 4; ++t) walk(t, t > s);      // (a wave holds the tokens 4 w .. 4 w + 3)
+        for (int t = 4 * w + 4; t < ST_TOK; ++t) walk(t, true);
+    }
+    __syncthreads();
+    float* out = p.work + ((int64_t)slot * p.heads + a) * st_floats(NP);
+    // a channel's products: from the tile's start (first NP threads), to its end (next NP)
+    float x[(2 * NP + 255) / 256][2 * ST_TOK];
+#pragma unroll
+    for (int u = 0; u < (2 * NP + 255) / 256; ++u) {
+        const int e = tid + 256 * u, c = e % NP;
+        if (e < NP) {
+            float P = 1.0f;
+#pragma unroll
+            for (int t = 0; t < ST_TOK; ++t) {
+                P *= sF[t][c];
+                x[u][t] = sQ[t][c] * P;
+                if (DELTA) x[u][ST_TOK + t] = sK[t][c] * P;
+            }
+            out[3 * ST_TOK * NP + c] = P;
+        } else if (e < 2 * NP) {
+            float E = 1.0f;
+#pragma unroll
+            for (int t = ST_TOK - 1; t >= 0; --t) {
+                x[u][t] = sK[t][c] * E;
+                E *= sF[t][c];
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < (2 * NP + 255) / 256; ++u) {
+        const int e = tid + 256 * u, c = e % NP;
+#pragma unroll
+        for (int t = 0; t < ST_TOK; ++t) {
+            if (e < NP) {
+                sQ[t][c] = x[u][t];
+                if (DELTA) sK[t][c] = x[u][ST_TOK + t];
+            } else if (e < 2 * NP) sF[t][c] = x[u][t];
+        }
+    }
+    out += 3 * ST_TOK * NP + NP;
+    out[tid] = (tid & 15) <= (tid >> 4) ? sB[tid >> 4][tid & 15] : 0.0f;
+    if (DELTA && tid < ST_TOK) {
+        const int j = tid;      // a column of T
+        float col[ST_TOK];
+#pragma unroll
+        for (int t = 0; t < ST_TOK; ++t) {
+            float s0 = t == j ? 1.0f : 0.0f;
+#pragma unroll
+            for (int s = 0; s < t; ++s) s0 = s >= j ? fmaf(-sA[t][s], col[s], s0) : s0;
+            col[t] = t >= j ? sBeta[t] * s0 : 0.0f;
+            out[ST_PAIR + t * ST_TOK + j] = col[t];
+        }
+    }
+    __syncthreads();
+    out -= 3 * ST_TOK * NP + NP;
+#pragma unroll
+    for (int e = tid; e < ST_TOK * NP / 4; e += 256) {      // lane (g, c) of block b: token c, channels 4 g ..; tokens 4 g .., channel c
+        const int b = e >> 6, g = (e >> 4) & 3, c = e & 15;
+        *(stf4*)(out + 4 * e) = *(const stf4*)&sQ[c][16 * b + 4 * g];
+        *(stf4*)(out + ST_TOK * NP + 4 * e) = stf4{sF[4 * g][16 * b + c], sF[4 * g + 1][16 * b + c], sF[4 * g + 2][16 * b + c], sF[4 * g + 3][16 * b + c]};
+        if (DELTA) *(stf4*)(out + 2 * ST_TOK * NP + 4 * e) = *(const stf4*)&sK[c][16 * b + 4 * g];
+    }
+}
+
+// One workgroup per (16 value columns, head, run); wave w holds the key channels [16 BPW w, + 16 BPW) of the state, lane (g, c) of column c the
+// channels 4 g .. 4 g + 3 of every block of 16.  Operands come two tiles ahead, straight into registers.
+// What bounds a long run is a tile's chain - 8 matrix instructions, LDS and a barrier, 4, 8 more: 1.1 us of 16 tokens (token by token 2.5); reading q, k and
+// decays here and taking the products in every workgroup was 2.0 (29 narrow loads a wave are 1550 cycles of address and L1 work, their products 650).
+// The workgroups of a head are a multiple of eight apart where there are eight heads: one die's L2 then serves them all.
+template <int BPW, bool DELTA>
+__global__ __launch_bounds__(256, BPW > 2 ? 1 : 2) void scan_tile_kernel(const i64h_gdn_args p) {
+    constexpr int NP = 64 * BPW, FL = st_floats(NP);
+    __shared__ stf4 sX[2][DELTA ? 4 : 1][64], sY[2][4][64];
+    const int N = p.dim, P = p.vdim;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane & 15, g = lane >> 4;
+    const int a = blockIdx.x % p.heads, seg = blockIdx.y;
+    const int col = blockIdx.x / p.heads * 16 + c;
+    const bool cok = col < P;
+    const int64_t r0 = p.seg_start[seg], r1 = p.seg_start[seg + 1];
+    if (r1 <= r0) return;      // (the whole workgroup)
+    const int ch0 = 16 * BPW * w + 4 * g;
+    float* gS = p.state + (((int64_t)p.slot_ids[r0] * p.heads + a) * P + (cok ? col : 0)) * N;
+    const bool fresh = p.positions[r0] == 0;
+    stf4 S[BPW];
+#pragma unroll
+    for (int b = 0; b < BPW; ++b) {
+        S[b] = (stf4)0.0f;
+        if (!fresh && cok && ch0 + 16 * b < N) S[b] = *(const stf4*)(gS + ch0 + 16 * b);
+    }
+    const int nt = (int)((r1 - r0 + ST_TOK - 1) / ST_TOK);
+    const float* tiles = p.work + (st_slot(r0, seg) * p.heads + a) * FL;
+    const float* vbase = p.X + r0 * p.ldx + p.v_off + a * P;
+    const int64_t tstep = (int64_t)p.heads * FL;
+    const uint32_t ldx4 = 4 * (uint32_t)p.ldx, vc = cok ? 4 * col : 0;      // (16 rows span less than 4 GiB: the launch's check)
+    const int rows_last = (int)(r1 - r0) - ST_TOK * (nt - 1);      // of the last tile
+    struct Ops {      // k P and q P (lane: token c, channels 4 g ..), k P_16 / P (tokens 4 g .., channel c), P_16 (channels 4 g ..), values (tokens 4 g ..)
+        stf4 qp[BPW], kd[BPW], kp[DELTA ? BPW : 1], tot[BPW], T;
+        float v[4], B;
+    };
+    auto ld4 = [](const float* base, uint32_t off) { return *(const stf4*)((const char*)base + off); };
+    auto ld1 = [](const float* base, uint32_t off) { return *(const float*)((const char*)base + off); };
+    auto load = [&](int i, Ops& u) {
+        i = min(i, nt - 1);      // (past the end: the last tile once more, nobody reads it)
+        const float *m = tiles + i * tstep, *vt = vbase + (int64_t)i * ST_TOK * p.ldx;
+        const uint32_t vl = (i == nt - 1 ? rows_last - 1 : ST_TOK - 1) * ldx4;
+        const uint32_t at = 4 * (256 * BPW * w + 4 * lane);
+#pragma unroll
+        for (int b = 0; b < BPW; ++b) {
+            if (DELTA) u.kp[b] = ld4(m + 2 * ST_TOK * NP + 256 * b, at);
+            u.qp[b] = ld4(m + 256 * b, at);
+            u.kd[b] = ld4(m + ST_TOK * NP + 256 * b, at);
+            u.tot[b] = ld4(m + 3 * ST_TOK * NP + 16 * b, 4 * ch0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) u.v[r] = ld1(vt, min((4 * g + r) * ldx4, vl) + vc);
+        u.B = ld1(m + 3 * ST_TOK * NP + NP, 4 * (c * ST_TOK + 4 * g + w));
+        if (DELTA) u.T = ld4(m + 3 * ST_TOK * NP + NP + ST_PAIR, 4 * (c * ST_TOK + 4 * g));
+    };
+    // a tile's read-out, once every wave's share lies in LDS: wave w stores the tokens 4 g + w
+    float* obase = p.out + r0 * p.ldo + a * P + col;
+    auto store = [&](int i) {
+        const int t = ST_TOK * i + 4 * g + w;
+        const float* y = (const float*)&sY[i & 1][0][lane] + w;
+        const float o = (y[0] + y[256]) + (y[512] + y[768]);
+        if (cok && t < (int)(r1 - r0)) obase[t * p.ldo] = DELTA ? o : o * p.q_scale;
+    };
+    // M v over the tokens up to and with a row's own, term by term: the terms from `first` on, every `stride`th
+    auto below = [&](const float* M, const stf4& v, int first, int stride, stf4 o) {
+#pragma unroll 1
+        for (int s = first; s < ST_TOK; s += stride) {
+            const float lo = (s & 1) ? v[1] : v[0], hi = (s & 1) ? v[3] : v[2];
+            const float vs = __shfl((s & 2) ? hi : lo, 16 * (s >> 2) + c);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (s <= 4 * g + r) o[r] = fmaf(M[(4 * g + r) * ST_TOK + s], vs, o[r]);
+        }
+        return o;
+    };
+    auto tile = [&](int i, const Ops& o, Ops& ahead) {
+        const int pb = i & 1;
+        load(i + 2, ahead);
+        if constexpr (DELTA) {
+            stf4 x[2] = {(stf4)0.0f, (stf4)0.0f};
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int b = 0; b < BPW; ++b) x[b & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kp[b][r], S[b][r], x[b & 1], 0, 0, 0);
+            sX[pb][w][lane] = x[0] + x[1];
+        }
+        stf4 y[2] = {(stf4)0.0f, (stf4)0.0f};
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int b = 0; b < BPW; ++b) y[b & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.qp[b][r], S[b][r], y[b & 1], 0, 0, 0);
+        // one barrier a tile: LDS holds two tiles' shares, and the one that is written again was read in front of it
+        __syncthreads();
+        stf4 V, W, U;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) V[r] = o.v[r];
+        W = V;
+        if constexpr (DELTA) W = V - ((sX[pb][0][lane] + sX[pb][1][lane]) + (sX[pb][2][lane] + sX[pb][3][lane]));
+        if (i == nt - 1) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) W[r] = 4 * g + r < rows_last ? W[r] : 0.0f;
+        }
+        U = W;
+        if constexpr (DELTA) {
+            stf4 u0 = (stf4)0.0f, u1 = (stf4)0.0f;
+            u0 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.T[0], W[0], u0, 0, 0, 0);
+            u1 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.T[2], W[2], u1, 0, 0, 0);
+            u0 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.T[1], W[1], u0, 0, 0, 0);
+            u1 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.T[3], W[3], u1, 0, 0, 0);
+            U = u0 + u1;
+        }
+        // a sum over all 16 tokens would carry what is no finite number to tokens in front of it, through a zero: such a tile is summed term by term
+        float mag = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) mag += DELTA ? fabsf(W[r]) + fabsf(U[r]) : fabsf(U[r]);
+        const bool odd = __ballot(!(mag < INFINITY)) != 0;
+        const float* pr = tiles + i * tstep + 3 * ST_TOK * NP + NP;
+        if (DELTA && odd) U = below(pr + ST_PAIR, W, 0, 1, (stf4)0.0f);
+#pragma unroll
+        for (int b = 0; b < BPW; ++b) S[b] = S[b] * o.tot[b];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int b = 0; b < BPW; ++b) S[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kd[b][r], U[r], S[b], 0, 0, 0);
+        // a wave's share of the read-out: its channels of the state, and every fourth token's write
+        stf4 O = y[0] + y[1];
+        if (odd) O = below(pr, U, w, 4, O);
+        else O = __builtin_amdgcn_mfma_f32_16x16x4f32(o.B, w == 0 ? U[0] : (w == 1 ? U[1] : (w == 2 ? U[2] : U[3])), O, 0, 0, 0);
+        if (i > 0) store(i - 1);
+        sY[pb][w][lane] = O;
+    };
+    Ops A, B, C;
+    // (the sets' loads stay apart: waiting for one must not wait for the next)
+#define ST_APART                       \
+    asm volatile("" ::: "memory");     \
+    __builtin_amdgcn_sched_barrier(0);
+    ST_APART
+    load(0, A);
+    ST_APART
+    load(1, B);
+    ST_APART
+#undef ST_APART
+    int i = 0;
+    for (; i + 3 <= nt; i += 3) {      // (not left in the middle: round the loop every set is as many loads behind the next)
+        tile(i, A, C);
+        tile(i + 1, B, A);
+        tile(i + 2, C, B);
+    }
+    if (i < nt) tile(i, A, C);
+    if (i + 1 < nt) tile(i + 1, B, A);
+    __syncthreads();
+    store(nt - 1);
+#pragma unroll
+    for (int b = 0; b < BPW; ++b)
+        if (cok && ch0 + 16 * b < N) *(stf4*)(gS + ch0 + 16 * b) = S[b];
+}
+
+static int st_padded(int dim) { return dim <= 64 ? 64 : (dim <= 128 ? 128 : 256); }
+
+extern "C" int64_t i64h_scan_work_floats(int64_t n, int32_t nseg, int32_t heads, int32_t dim) {
+    return (n / ST_TOK + nseg) * heads * st_floats(st_padded(dim));
+}
+
+// both launches; the caller (the scans' own dispatch) has checked sizes, alignment and the workspace
+int i64h_scan_tiles(const i64h_gdn_args& d, bool delta, void* stream) {
+    const dim3 pairs((unsigned)((d.n / ST_TOK + d.nseg) * d.heads)), tiles((unsigned)(d.heads * ((d.vdim + 15) / 16)), (unsigned)d.nseg);
+    auto run = [&](auto a, auto b) {
+        hipLaunchKernelGGL(a, pairs, dim3(256), 0, (hipStream_t)stream, d);
+        hipLaunchKernelGGL(b, tiles, dim3(256), 0, (hipStream_t)stream, d);
+    };
+    auto pick = [&](auto bpw) {
+        constexpr int B = decltype(bpw)::value;
+        if (delta) run(scan_pairs_kernel<64 * B, true>, scan_tile_kernel<B, true>);
+        else run(scan_pairs_kernel<64 * B, false>, scan_tile_kernel<B, false>);
+    };
+    if (d.dim <= 64) pick(std::integral_constant<int, 1>());
+    else if (d.dim <= 128) pick(std::integral_constant<int, 2>());
+    else pick(std::integral_constant<int, 4>());
+    I64H_CHECK_LAUNCH();
+    return 0;
+}

@@ -174,6 +174,17 @@ class HybridRunner:
             ws = B.attn_ws[key] = torch.empty(max(1, floats(splits)), dtype=torch.float32, device=self.device)
         return splits, ws
 
+    def _scan_work(self, B, n: int, nseg: int, r) -> Optional[torch.Tensor]:
+        """The workspace of a recurrence's scan over runs of more than a row."""
+        if n == nseg:
+            return None
+        runs = (nseg + 15) // 16 * 16
+        key = ("scan", runs, r.heads, r.dim)
+        ws = B.attn_ws.get(key)
+        if ws is None:
+            ws = B.attn_ws[key] = torch.empty(D.scan_work_floats(n, runs, r.heads, r.dim), dtype=torch.float32, device=self.device)
+        return ws
+
     # ---- attention over grouped key / value heads, separate keys and values in one cached row ----
     def _kattn(self, B, a, Q, O, rows, kvc, slot_ids, positions, runs, ctx_hint: int, *, bias=None, softcap: float = 0.0, window: int = 0,
                keep_first: int = 0, sink_w=None) -> None:
@@ -282,7 +293,8 @@ class HybridRunner:
         wide = self._wide(n, rv)
         R, Rn, Rn16 = B.r[: n * rv].view(n, rv), None if wide else B.rn[: n * rv].view(n, rv), self._as16(B.rn, n, rv) if wide else None
         D.gla_scan(P, f=F, q_off=d["rq_off"], k_off=d["rk_off"], f_off=0, v_off=d["rv_off"], heads=r.heads, dim=r.dim, vdim=r.vdim, seg_start=seg, nseg=nseg,
-                   positions=positions, slot_ids=slot_ids, state=kvc.state[l]["gla"], out=R, n=n, q_scale=r.dim ** -0.5)
+                   positions=positions, slot_ids=slot_ids, state=kvc.state[l]["gla"], out=R, n=n, q_scale=r.dim ** -0.5,
+                   work=self._scan_work(B, n, nseg, r))
         D.gate_norm(R, d["r_norm"], Rn, groups=r.heads, eps=self.cfg.norm_eps, z=P, z_off=d["rg_off"], ldz=P.shape[-1], n=n, gate_after=True, width=rv, out16=Rn16)
         self._out(Rn, d["o_right"], out, scale, Rn16)
 
@@ -308,7 +320,8 @@ class HybridRunner:
             D.linear(P, d["a2"], F, m=n, a_off=d["a1_off"], exact=ex, bias=d["dt_bias"], epilogue=D.EPI_DECAY, e=d["a_rate"])
             D.linear(P, d["g2"], Z, m=n, a_off=d["g1_off"], exact=ex)
         R = B.b[: n * rv].view(n, rv)
-        D.gdn_scan(X, G, f=F, seg_start=seg, nseg=nseg, positions=positions, slot_ids=slot_ids, state=st["gdn"], out=R, **cols)
+        D.gdn_scan(X, G, f=F, seg_start=seg, nseg=nseg, positions=positions, slot_ids=slot_ids, state=st["gdn"], out=R, work=self._scan_work(B, n, nseg, r),
+                   **cols)
         wide = self._wide(n, rv)
         Rn, Rn16 = None if wide else B.c[: n * rv].view(n, rv), self._as16(B.c, n, rv) if wide else None
         D.gate_norm(R, d["r_norm"], Rn, groups=r.heads, eps=self.cfg.norm_eps, z=Z, z_off=z_off, ldz=ldz, n=n, gate_after=True, width=rv, sigmoid=r.gate == "sigmoid", out16=Rn16)
