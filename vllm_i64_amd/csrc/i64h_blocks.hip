@@ -31,15 +31,48 @@ __global__ __launch_bounds__(256) void gla_gates_kernel(const i64h_gla_args p) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
-// Gated delta rule.  gdn_gates_kernel: one workgroup per token - a wave per query / key head makes the head a unit vector in place (the
-// query also scaled), and the first threads turn the raw gate projections into the write strength and the decay of every head.
+// Gated delta rule.  gdn_gates_kernel: one workgroup per token - the heads of query and key become unit vectors in place (the query also
+// scaled), and threads turn the raw gate projections into the write strength and the decay of every head.
+// VEC (16-byte rows): 16 lanes take a head, the loads of GT_ROUNDS rounds of 16 heads on their way together; else a wave takes a head, one
+// after the other.  What bounds it is the way to memory and back of a row's heads: 3008 rows of 2 x 16 heads of 128, 28 | 16 us beside nothing else.
 __device__ __forceinline__ float bl_softplus(float x) { return x > 20.0f ? x : log1pf(expf(x)); }
 
+#define GT_ROUNDS 2
+template <int VEC>      // stripes of 64 channels a head has; 0: any row
 __global__ __launch_bounds__(256) void gdn_gates_kernel(const i64h_gdn_args p) {
     const int64_t t = blockIdx.x;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     float* row = p.X + t * p.ldx;
-    if (p.unit_eps >= 0.0f || p.q_scale != 1.0f) {
+    if (VEC && (p.unit_eps >= 0.0f || p.q_scale != 1.0f)) {
+        const int l = threadIdx.x & 15;
+        for (int u0 = threadIdx.x >> 4; u0 < 2 * p.kv_heads; u0 += 16 * GT_ROUNDS) {
+            float4 v[GT_ROUNDS][VEC ? VEC : 1];
+            auto head = [&](int u) { return row + (u < p.kv_heads ? p.q_off + u * p.dim : p.k_off + (u - p.kv_heads) * p.dim); };
+#pragma unroll
+            for (int r = 0; r < GT_ROUNDS; ++r)
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) {
+                    const int u = u0 + 16 * r, d = 64 * i + 4 * l;
+                    v[r][i] = make_float4(0, 0, 0, 0);
+                    if (u < 2 * p.kv_heads && d < p.dim) v[r][i] = *(const float4*)(head(u) + d);
+                }
+#pragma unroll
+            for (int r = 0; r < GT_ROUNDS; ++r) {
+                const int u = u0 + 16 * r;
+                float s = 0.0f;
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) s += (v[r][i].x * v[r][i].x + v[r][i].y * v[r][i].y) + (v[r][i].z * v[r][i].z + v[r][i].w * v[r][i].w);
+                s = group_sum(s, 16);
+                float f = p.unit_eps >= 0.0f ? 1.0f / sqrtf(s + p.unit_eps) : 1.0f;
+                if (u < p.kv_heads) f *= p.q_scale;
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) {
+                    const int d = 64 * i + 4 * l;
+                    if (u < 2 * p.kv_heads && d < p.dim) *(float4*)(head(u) + d) = make_float4(v[r][i].x * f, v[r][i].y * f, v[r][i].z * f, v[r][i].w * f);
+                }
+            }
+        }
+    } else if (p.unit_eps >= 0.0f || p.q_scale != 1.0f) {
         for (int u = wid; u < 2 * p.kv_heads; u += 4) {
             const bool isq = u < p.kv_heads;
             float* x = row + (isq ? p.q_off + u * p.dim : p.k_off + (u - p.kv_heads) * p.dim);
@@ -644,7 +677,12 @@ int i64h_gdn_gates(const i64h_gdn_args* dp, void* stream) {
     if (gdn_check(d, "gdn_gates")) return 1;
     I64H_CHECK_ARG(d.G && d.R && d.b_off >= 0 && (d.a_off < 0 || (d.A_log && d.dt_bias)), "gdn_gates: null operand or negative column");
     if (d.n == 0) return 0;
-    hipLaunchKernelGGL(gdn_gates_kernel, dim3((unsigned)d.n), dim3(256), 0, (hipStream_t)stream, d);
+    auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, dim3((unsigned)d.n), dim3(256), 0, (hipStream_t)stream, d); };
+    const bool vec = d.dim % 4 == 0 && d.dim <= 256 && d.ldx % 4 == 0 && d.q_off % 4 == 0 && d.k_off % 4 == 0 && (uintptr_t)d.X % 16 == 0;
+    if (!vec) launch(gdn_gates_kernel<0>);
+    else if (d.dim <= 64) launch(gdn_gates_kernel<1>);
+    else if (d.dim <= 128) launch(gdn_gates_kernel<2>);
+    else launch(gdn_gates_kernel<4>);
     I64H_CHECK_LAUNCH();
     return 0;
 }
