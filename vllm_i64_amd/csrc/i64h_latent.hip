@@ -159,6 +159,7 @@ __global__ __launch_bounds__(256) void latent_attn_row_kernel(const i64h_latent_
 #define LT_VLD 40  // halves per row of the transposed tile and of the weight planes (32 keys + 8: 16-byte aligned, conflict-poor)
 typedef __bf16 lt_v8bf __attribute__((ext_vector_type(8)));
 typedef float lt_v4f __attribute__((ext_vector_type(4)));
+typedef short lt_v4s __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ uint32_t lt_rne(float f) {  // nearest even: the hardware conversion of this chip
     return (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)f);
@@ -170,27 +171,30 @@ __device__ __forceinline__ void lt_split(float x, uint32_t& hi, uint32_t& lo) {
 
 // Matrix-core form (bf16 cache) of rows that are one per sequence.  One wave per task of 16 query vectors that walk the same cached rows: the (up to) 16
 // heads of a group of one token, a share of its keys.
-// Per tile of 32 keys: scores S[16, 32] = Q K^T on v_mfma_f32_16x16x32_bf16 with the cached rows read straight from memory as B
-// fragments (8 consecutive values of one key per lane) and the scaled query carried as TWO bf16 terms (hi + lo, 16 mantissa bits),
-// masking and the online softmax in fp32 on the accumulator layout, the weights again as two bf16 terms through LDS into the
-// A layout, the tile's latent columns transposed through LDS (8 two-byte writes per fragment) into the B
-// layout of the second product, out[16, kv_rank] += P V in fp32.  Every product of two bf16 values is exact in fp32.
-// Arranged around the memory latency that dominates such launches: a tile's 18 fragment loads are requested together, the NEXT tile's are
+// Per tile of 32 keys: scores S^T[32, 16] = K Q^T on v_mfma_f32_16x16x32_bf16 with the cached rows read straight from memory as A
+// fragments (8 consecutive values of one key per lane) and the scaled query carried as TWO bf16 terms (hi + lo, 16 mantissa bits);
+// masking and the online softmax in fp32 as the accumulators lie - a lane holds eight keys of one query, whose weights, again as two bf16 terms, are
+// the second product's operand without a move -; the tile's latent columns through LDS, written as they came and read transposed
+// (ds_read_b64_tr_b16), out^T[kv_rank, 16] += V^T P^T in fp32.  Every product of two bf16 values is exact in fp32.
+// What bounds it is the instructions of one wave a SIMD, and branches most of all: 64 tokens of 32 heads over one row of 288, 2048 keys, 63 | 40 us against
+// the form with a branch around every step, score and query fragment (a tile 14000 cycles; the weights through LDS and columns transposed by 144 two-byte
+// writes were the smaller part), one token, 500 keys 26 | 14, 32 heads of 64 over 8 key heads, 64 tokens, 1024 keys 38 | 30 (with the merge).
+// Arranged around the memory latency of such launches: a tile's 18 fragment loads are requested together, the NEXT tile's are
 // requested as soon as this tile's scores and transposed columns are done - under its softmax and second product - and the cache rows of the tile
 // after that are looked up a tile ahead.  The workgroup is one wave, so LDS traffic needs program order only (no barrier, whose
 // fence would wait for the loads in flight).  Registers: a whole SIMD's (one wave per SIMD is all such a launch has anyway).
-// KD, NB: 32-wide steps over a cached row and 16-column blocks of the output that an instance holds registers for (rows of at most
-// 32 KD values, kv_rank <= 16 NB).
-template <int KD, int NB>
+// KD, NB: 32-wide steps over a cached row and 16-column blocks of the output that an instance holds registers for.  ANY: rows of at most 32 KD values,
+// kv_rank <= 16 NB, key scales, soft cap, bias; else rows of exactly 32 KD values, kv_rank 16 NB, keys from step KO on and none of the others: without
+// a branch around any, the query's fragments asked for together.
+template <int KD, int NB, int KO, bool ANY>
 __global__ __launch_bounds__(64) void latent_attn_mfma_decode_kernel(const i64h_latent_attn_args p, const int splits) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int lane = threadIdx.x, n = lane & 15, kg = lane >> 4;
     const int r = p.kv_rank, D = r + p.rot_dim, H = p.heads, bs = p.block_size, win = p.window;
     const int keep = p.chunk <= 0 && win > 0 ? p.keep_first : 0;
-    uint16_t* Vt = (uint16_t*)smem;
-    uint16_t* Ph = Vt + r * LT_VLD;
-    uint16_t* Pl = Ph + 16 * LT_VLD;
-    int* rowoff = (int*)(Pl + 16 * LT_VLD);   // [2][32] cache rows of two tiles' keys
+    const int vld = ANY ? r + 16 : 16 * NB + 16;      // halves per key in LDS (rows 8 banks apart where r is a multiple of 128)
+    uint16_t* V = (uint16_t*)smem;            // [32][vld]
+    int* rowoff = (int*)(V + 32 * vld);       // [2][32] cache rows of two tiles' keys
     const int64_t task = blockIdx.x;
     const int split = blockIdx.y;
     const int G = p.kv_groups > 1 ? p.kv_groups : 1, rep = H / G, tpg = (rep + 15) / 16;
@@ -222,10 +226,17 @@ __global__ __launch_bounds__(64) void latent_attn_mfma_decode_kernel(const i64h_
 #pragma unroll
             for (int ks = 0; ks < KD; ++ks) {
                 const int d0 = ks * 32 + kg * 8;
-                kf[b][ks] = (ks * 32 < D && d0 < D) ? *(const uint4*)(rowp + d0) : make_uint4(0, 0, 0, 0);
+                if (ANY) kf[b][ks] = (ks * 32 < D && d0 < D) ? *(const uint4*)(rowp + d0) : make_uint4(0, 0, 0, 0);
+                else kf[b][ks] = *(const uint4*)(rowp + d0);
             }
         }
     };
+    const int hq = min(head0 + n, H - 1);       // this lane's query (one without a head of its own: nobody reads its result)
+    const float* q = p.Q + (tok * H + hq) * D;
+    float4 qv[ANY ? 1 : 2 * KD];
+    if (!ANY)
+#pragma unroll
+        for (int i = 0; i < 2 * KD; ++i) qv[i] = *(const float4*)(q + (i >> 1) * 32 + kg * 8 + 4 * (i & 1));
     if (split < tiles) {
         lookup(first_key(split), 0);
         if (split + splits < tiles) lookup(first_key(split + splits), 1);
@@ -236,14 +247,13 @@ __global__ __launch_bounds__(64) void latent_attn_mfma_decode_kernel(const i64h_
     uint4 Qh[KD], Ql[KD];
     {
         const bool valid_n = hin + n < rep;
-        const float* q = p.Q + (tok * H + head0 + n) * D;
         const float qs = p.scale * 1.4426950408889634f;
 #pragma unroll
         for (int ks = 0; ks < KD; ++ks) {
             const int d0 = ks * 32 + kg * 8;
             uint32_t h[8], l[8];
-            if (valid_n && d0 < D) {
-                const float4 a = *(const float4*)(q + d0), b = *(const float4*)(q + d0 + 4);
+            if (!ANY || (valid_n && d0 < D)) {
+                const float4 a = ANY ? *(const float4*)(q + d0) : qv[ANY ? 0 : 2 * ks], b = ANY ? *(const float4*)(q + d0 + 4) : qv[ANY ? 0 : 2 * ks + 1];
                 const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
                 for (int i = 0; i < 8; ++i) lt_split(v[i] * qs, h[i], l[i]);
@@ -258,115 +268,116 @@ __global__ __launch_bounds__(64) void latent_attn_mfma_decode_kernel(const i64h_
     lt_v4f acc[NB];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[nb] = lt_v4f{0, 0, 0, 0};
-    float mrow[4], lrow[4];
-    int hrow[4];
     const bool sink = p.sink && split == 0;     // the extra score of zero counts once: in the first share of the keys
     const float capl = p.softcap * 1.4426950408889634f;     // the cap in the units of the scores (powers of two)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        hrow[g] = min(head0 + kg * 4 + g, H - 1);
-        mrow[g] = sink ? (p.sink_w ? p.sink_w[hrow[g]] * 1.4426950408889634f : 0.0f) : -INFINITY;
-        lrow[g] = sink ? 1.0f : 0.0f;
-    }
+    float m = sink ? (p.sink_w ? p.sink_w[hq] * 1.4426950408889634f : 0.0f) : -INFINITY, l = sink && kg == 0 ? 1.0f : 0.0f;      // (the sum in four shares)
     int it = 0;
     for (int tile = split; tile < tiles; tile += splits, ++it) {
         const int cur = it & 1, kb = first_key(tile);
-        lt_v4f S[2];
-        float ksc[2] = {1.0f, 1.0f};
-        if (p.kscale) {
-            ksc[0] = p.kscale[rowoff[cur * 32 + n]];
-            ksc[1] = p.kscale[rowoff[cur * 32 + 16 + n]];
+        lt_v4f S[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+        float ksc[2][4];
+        if (ANY && p.kscale) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) ksc[b][g] = p.kscale[rowoff[cur * 32 + 16 * b + 4 * kg + g]];
         }
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            S[b] = lt_v4f{0, 0, 0, 0};
+        for (int ks = 0; ks < KD; ++ks) {
+            if (!ANY || ks * 32 < D) {
+                const int d0 = ks * 32 + kg * 8;
 #pragma unroll
-            for (int ks = 0; ks < KD; ++ks) {
-                if (ks * 32 < D) {
-                    const int d0 = ks * 32 + kg * 8;
+                for (int b = 0; b < 2; ++b) {
                     const uint4 f = kf[b][ks];
-                    if ((ks + 1) * 32 > p.key_off) {     // (a step of value-only columns: the query is zero there)
-                        S[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lt_v8bf, Qh[ks]), __builtin_bit_cast(lt_v8bf, f), S[b], 0, 0, 0);
-                        S[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lt_v8bf, Ql[ks]), __builtin_bit_cast(lt_v8bf, f), S[b], 0, 0, 0);
+                    if (ANY ? (ks + 1) * 32 > p.key_off : ks >= KO) {     // (a step of value-only columns: the query is zero there)
+                        S[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lt_v8bf, f), __builtin_bit_cast(lt_v8bf, Qh[ks]), S[b], 0, 0, 0);
+                        S[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lt_v8bf, f), __builtin_bit_cast(lt_v8bf, Ql[ks]), S[b], 0, 0, 0);
                     }
-                    if (d0 < r) {
-                        const uint32_t kw[4] = {f.x, f.y, f.z, f.w};
-#pragma unroll
-                        for (int c = 0; c < 8; ++c) Vt[(d0 + c) * LT_VLD + 16 * b + n] = (uint16_t)(kw[c >> 1] >> (16 * (c & 1)));
-                    }
+                    if (ANY ? d0 < r : ks < NB / 2) *(uint4*)&V[(16 * b + n) * vld + d0] = f;
                 }
             }
         }
         __builtin_amdgcn_wave_barrier();
         if (tile + splits < tiles) request(cur ^ 1);          // the next tile travels under this tile's softmax and second product
-        float al[4];
+        // scores of keys kb + 16 b + 4 kg + g
+        float mx = -INFINITY;
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int rr = kg * 4 + g;
-            float sv[2];
+        for (int b = 0; b < 2; ++b)
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                const int j = kb + 16 * b + n;
-                float sc = S[b][g] * ksc[b];
-                if (capl > 0.0f) sc = capl * tanhf(sc / capl);
-                if (p.bias) sc += 1.4426950408889634f * p.bias[(int64_t)min(max(pos - j, 0), p.bias_rows - 1) * H + hrow[g]];
-                sv[b] = (j <= pos && (j >= lo || j < keep)) ? sc : -INFINITY;
+            for (int g = 0; g < 4; ++g) {
+                const int j = kb + 16 * b + 4 * kg + g;
+                float sc = ANY && p.kscale ? S[b][g] * ksc[b][g] : S[b][g];
+                if (ANY && capl > 0.0f) sc = capl * tanhf(sc / capl);
+                if (ANY && p.bias) sc += 1.4426950408889634f * p.bias[(int64_t)min(max(pos - j, 0), p.bias_rows - 1) * H + hq];
+                S[b][g] = (j <= pos && (j >= lo || j < keep)) ? sc : -INFINITY;
+                mx = fmaxf(mx, S[b][g]);
             }
-            const float mx = row16_max(fmaxf(sv[0], sv[1]));
-            const float mn = fmaxf(mrow[g], mx);
-            const float ms = mn == -INFINITY ? 0.0f : mn;
-            al[g] = __builtin_amdgcn_exp2f(mrow[g] - ms);
-            const float p0 = __builtin_amdgcn_exp2f(sv[0] - ms), p1 = __builtin_amdgcn_exp2f(sv[1] - ms);
-            lrow[g] = lrow[g] * al[g] + group_sum(p0 + p1, 16);
-            mrow[g] = mn;
-            uint32_t h0, l0, h1, l1;
-            lt_split(p0, h0, l0);
-            lt_split(p1, h1, l1);
-            Ph[rr * LT_VLD + n] = (uint16_t)h0;
-            Pl[rr * LT_VLD + n] = (uint16_t)l0;
-            Ph[rr * LT_VLD + 16 + n] = (uint16_t)h1;
-            Pl[rr * LT_VLD + 16 + n] = (uint16_t)l1;
+        const PairF m1 = swap_rows(mx);
+        mx = fmaxf(m1.lo, m1.hi);
+        const PairF m2 = swap_halves(mx);
+        const float mn = fmaxf(m, fmaxf(m2.lo, m2.hi)), ms = mn == -INFINITY ? 0.0f : mn;
+        const float al = __builtin_amdgcn_exp2f(m - ms);
+        m = mn;
+        float sum = 0.0f;
+        uint32_t ph[4], pl[4];
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int g = 0; g < 4; g += 2) {
+                const float p0 = __builtin_amdgcn_exp2f(S[b][g] - ms), p1 = __builtin_amdgcn_exp2f(S[b][g + 1] - ms);
+                sum += p0 + p1;
+                uint32_t h0, l0, h1, l1;
+                lt_split(p0, h0, l0);
+                lt_split(p1, h1, l1);
+                ph[b * 2 + g / 2] = h0 | (h1 << 16);
+                pl[b * 2 + g / 2] = l0 | (l1 << 16);
+            }
+        l = l * al + sum;
+        if (__ballot(al != 1.0f)) {
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) acc[nb][g] *= al;
         }
-        __builtin_amdgcn_wave_barrier();
-        const uint4 pah = *(const uint4*)&Ph[n * LT_VLD + kg * 8], pal = *(const uint4*)&Pl[n * LT_VLD + kg * 8];
+        const lt_v8bf Ph = __builtin_bit_cast(lt_v8bf, make_uint4(ph[0], ph[1], ph[2], ph[3])), Pl = __builtin_bit_cast(lt_v8bf, make_uint4(pl[0], pl[1], pl[2], pl[3]));
+        // V^T fragments: lane 4 q + c of 16 addresses key 4 kg + q (and 16 keys further), columns 16 nb + 4 c .. + 3, and receives its own column of four keys
+        const uint16_t* vp = &V[(4 * kg + (n >> 2)) * vld + 4 * (n & 3)];
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
-            if (nb * 16 < r) {
-                const uint4 vf = *(const uint4*)&Vt[(nb * 16 + n) * LT_VLD + kg * 8];
-#pragma unroll
-                for (int g = 0; g < 4; ++g) acc[nb][g] *= al[g];
-                acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lt_v8bf, pah), __builtin_bit_cast(lt_v8bf, vf), acc[nb], 0, 0, 0);
-                acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lt_v8bf, pal), __builtin_bit_cast(lt_v8bf, vf), acc[nb], 0, 0, 0);
+            if (!ANY || nb * 16 < r) {
+                const lt_v4s a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) lt_v4s*)(vp + nb * 16));
+                const lt_v4s b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) lt_v4s*)(vp + 16 * vld + nb * 16));
+                const lt_v8bf vf = __builtin_bit_cast(lt_v8bf, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+                acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, Ph, acc[nb], 0, 0, 0);
+                acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, Pl, acc[nb], 0, 0, 0);
             }
         }
         __builtin_amdgcn_wave_barrier();
         if (tile + 2 * splits < tiles) lookup(first_key(tile + 2 * splits), cur);   // rows of the tile after next, into the buffer this tile is done with
     }
+    const PairF l1 = swap_rows(l);
+    const PairF l2 = swap_halves(l1.lo + l1.hi);
+    l = l2.lo + l2.hi;
+    // query n's columns 16 nb + 4 kg .. + 3
     if (splits > 1) {
-        float* w = p.workspace + ((int64_t)task * splits + split) * 16 * (r + 2);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            float* o = w + (kg * 4 + g) * (r + 2);
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-                if (nb * 16 < r) o[nb * 16 + n] = acc[nb][g];
-            if (n == 0) {
-                o[r] = mrow[g];
-                o[r + 1] = lrow[g];
-            }
-        }
-        return;
-    }
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        const int head = head0 + kg * 4 + g;
-        if (hin + kg * 4 + g >= rep) continue;
-        float* o = p.out + (tok * H + head) * r;
-        const float inv = 1.0f / lrow[g];
+        float* o = p.workspace + ((int64_t)task * splits + split) * 16 * (r + 2) + n * (r + 2);
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
-            if (nb * 16 < r) o[nb * 16 + n] = acc[nb][g] * inv;
+            if (!ANY || nb * 16 < r) {
+                *(float2*)(o + nb * 16 + 4 * kg) = make_float2(acc[nb][0], acc[nb][1]);
+                *(float2*)(o + nb * 16 + 4 * kg + 2) = make_float2(acc[nb][2], acc[nb][3]);
+            }
+        if (kg == 0) *(float2*)(o + r) = make_float2(m, l);
+        return;
     }
+    if (hin + n >= rep) return;
+    float* o = p.out + (tok * H + head0 + n) * r;
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+        if (!ANY || nb * 16 < r)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) o[nb * 16 + 4 * kg + g] = acc[nb][g] * inv;
 }
 
 // One row and head by one wave, over the keys that it sees only: a key per lane for the scores, the columns (at most 256) spread over the lanes for the
@@ -1046,7 +1057,7 @@ int i64h_latent_attn(const i64h_latent_attn_args* dp, void* stream) {
         const int64_t tasks = row_tiles ? (d.n + 15) / 16 * d.heads : d.n * G * ((d.heads / G + 15) / 16);
         I64H_CHECK_ARG(tasks < (1ll << 31), "latent_attn: too many tiles");
         const int splits = (!row_tiles && d.workspace && d.splits > 1) ? (d.splits > 64 ? 64 : d.splits) : 1;
-        const size_t bytes = (size_t)d.kv_rank * LT_VLD * 2 + 2 * 16 * LT_VLD * 2 + 64 * 4;
+        const size_t bytes = (size_t)32 * (d.kv_rank + 16) * 2 + 64 * 4;
         const dim3 grid((unsigned)tasks, (unsigned)splits);
         hipStream_t st = (hipStream_t)stream;
         const int size = (D <= 64 && d.kv_rank <= 64) ? 0 : ((D <= 128 && d.kv_rank <= 128) ? 1 : 2);     // the narrowest instance that holds the rows
@@ -1066,9 +1077,15 @@ int i64h_latent_attn(const i64h_latent_attn_args* dp, void* stream) {
             else LT_ROWS(LT_KD, LT_NB);
 #undef LT_ROWS
         } else {
-            if (size == 0) hipLaunchKernelGGL((latent_attn_mfma_decode_kernel<2, 4>), grid, dim3(64), bytes, st, d, splits);
-            else if (size == 1) hipLaunchKernelGGL((latent_attn_mfma_decode_kernel<4, 8>), grid, dim3(64), bytes, st, d, splits);
-            else hipLaunchKernelGGL((latent_attn_mfma_decode_kernel<LT_KD, LT_NB>), grid, dim3(64), bytes, st, d, splits);
+            const bool plain = !d.kscale && !d.bias && d.softcap <= 0.0f;
+            auto exact = [&](int kd, int nb, int ko) { return plain && D == 32 * kd && d.kv_rank == 16 * nb && d.key_off / 32 == ko; };
+            auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(64), bytes, st, d, splits); };
+            if (exact(9, 16, 0)) launch(latent_attn_mfma_decode_kernel<9, 16, 0, false>);             // a latent row of 256 + 32
+            else if (exact(4, 4, 2)) launch(latent_attn_mfma_decode_kernel<4, 4, 2, false>);          // values and keys of 64
+            else if (exact(8, 8, 4)) launch(latent_attn_mfma_decode_kernel<8, 8, 4, false>);          // ... of 128
+            else if (size == 0) launch(latent_attn_mfma_decode_kernel<2, 4, 0, true>);
+            else if (size == 1) launch(latent_attn_mfma_decode_kernel<4, 8, 0, true>);
+            else launch(latent_attn_mfma_decode_kernel<LT_KD, LT_NB, 0, true>);
         }
         I64H_CHECK_LAUNCH();
         if (splits > 1) {
