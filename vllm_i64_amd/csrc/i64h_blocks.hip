@@ -425,7 +425,9 @@ __device__ __forceinline__ int bl_wave_argmax(float v, int idx, float& best) {
 #define RT_WIDE_ROWS 256       // launches of at most so many rows have the four groups; all of more than RT_MANY entries do
 #define RT_MANY 32
 #define RT_SPLIT_ROWS 512      // launches of at most so many rows are split; twice as many over more than RT_MANY entries
-template <bool SPLIT>
+// NINE: the last entry behind a multiple of eight goes with the eight before it (eight experts and a gate's row, 3008 rows of 2048: 20 | 15 us, 64 and a gate
+// 53 | 34); a kernel of its own, for its registers cost the launches beside it where there is no such entry (a step of 4096 rows 0.6 %).
+template <bool SPLIT, bool NINE>
 __global__ __launch_bounds__(SPLIT ? 1024 : 256) void route_topk_kernel(const i64h_route_args p) {
     extern __shared__ float rt_lds[];   // per wave: [E] scores, [E] choice values, [groups] group flags; SPLIT: once, and [4][E + 1] partial products
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -443,9 +445,28 @@ __global__ __launch_bounds__(SPLIT ? 1024 : 256) void route_topk_kernel(const i6
         const int K = p.K;
         const bool vec = (K & 3) == 0 && (p.ldh & 3) == 0 && ((uintptr_t)p.h & 15) == 0 && ((uintptr_t)p.W & 7) == 0;
         const int rows = p.gate_out ? E + 1 : E;
-        for (int e0 = SPLIT ? wid / 4 * 8 : 0; e0 < rows; e0 += SPLIT ? blockDim.x / 32 : 8) {
-            float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-            if (vec) {
+        bool nine = false;
+        for (int e0 = SPLIT ? wid / 4 * 8 : 0; e0 < rows; e0 += SPLIT ? blockDim.x / 32 : (NINE && nine ? 9 : 8)) {
+            float acc[9] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+            nine = NINE && rows - e0 == 9;
+            if (NINE && vec && rows - e0 >= 8) {
+                const uint16_t* we = W + (int64_t)e0 * K;
+#pragma unroll 2
+                for (int k = lane * 4; k < K; k += 256) {
+                    const float4 x = *(const float4*)(h + k);
+                    uint2 w[9];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) w[j] = *(const uint2*)(we + (int64_t)j * K + k);
+                    w[8] = nine ? *(const uint2*)(we + (int64_t)8 * K + k) : make_uint2(0, 0);
+#pragma unroll
+                    for (int j = 0; j < 9; ++j) {
+                        acc[j] = fmaf(x.x, __uint_as_float(w[j].x << 16), acc[j]);
+                        acc[j] = fmaf(x.y, __uint_as_float(w[j].x & 0xffff0000u), acc[j]);
+                        acc[j] = fmaf(x.z, __uint_as_float(w[j].y << 16), acc[j]);
+                        acc[j] = fmaf(x.w, __uint_as_float(w[j].y & 0xffff0000u), acc[j]);
+                    }
+                }
+            } else if (vec) {
                 for (int k = (SPLIT ? threadIdx.x & 255 : lane) * 4; k < K; k += SPLIT ? 1024 : 256) {
                     const float4 x = *(const float4*)(h + k);
 #pragma unroll
@@ -463,12 +484,13 @@ __global__ __launch_bounds__(SPLIT ? 1024 : 256) void route_topk_kernel(const i6
                 for (int k = SPLIT ? threadIdx.x & 255 : lane; k < K; k += SPLIT ? 256 : 64) {
                     const float x = h[k];
 #pragma unroll
-                    for (int j = 0; j < 8; ++j)
-                        if (e0 + j < rows) acc[j] = fmaf(x, __uint_as_float((uint32_t)W[(int64_t)(e0 + j) * K + k] << 16), acc[j]);
+                    for (int j = 0; j < (NINE ? 9 : 8); ++j)
+                        if (j < 8 ? e0 + j < rows : nine) acc[j] = fmaf(x, __uint_as_float((uint32_t)W[(int64_t)(e0 + j) * K + k] << 16), acc[j]);
                 }
             }
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
+            for (int j = 0; j < (NINE ? 9 : 8); ++j) {
+                if (NINE && j == 8 && !nine) break;
                 const float v = wave_sum(acc[j]);
                 if (SPLIT) {
                     if (lane == 0 && e0 + j < rows) part[(wid & 3) * rows + e0 + j] = v;
@@ -808,9 +830,13 @@ int i64h_route_topk(const i64h_route_args* dp, void* stream) {
     const size_t own = (size_t)(2 * d.E + (d.groups > 1 ? d.groups : 1));
     const int many = d.E > RT_MANY;
     if (d.W && d.n <= (RT_SPLIT_ROWS << many))
-        hipLaunchKernelGGL(route_topk_kernel<true>, dim3((unsigned)d.n), dim3(many || d.n <= RT_WIDE_ROWS ? 1024 : 256), (own + 4 * (size_t)(d.E + 1)) * 4, (hipStream_t)stream, d);
-    else
-        hipLaunchKernelGGL(route_topk_kernel<false>, dim3((unsigned)((d.n + 3) / 4)), dim3(256), 4 * own * 4, (hipStream_t)stream, d);
+        hipLaunchKernelGGL((route_topk_kernel<true, false>), dim3((unsigned)d.n), dim3(many || d.n <= RT_WIDE_ROWS ? 1024 : 256), (own + 4 * (size_t)(d.E + 1)) * 4, (hipStream_t)stream, d);
+    else {
+        const int rows = d.E + (d.gate_out ? 1 : 0);
+        auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, dim3((unsigned)((d.n + 3) / 4)), dim3(256), 4 * own * 4, (hipStream_t)stream, d); };
+        if (d.W && rows > 8 && rows % 8 == 1) launch(route_topk_kernel<false, true>);
+        else launch(route_topk_kernel<false, false>);
+    }
     I64H_CHECK_LAUNCH();
     return 0;
 }
