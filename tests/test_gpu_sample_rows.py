@@ -114,3 +114,14 @@ def test_first_of_the_largest():
         x[3, 3:] = -1.0
         want = [1, 0, 2, 3, 0]
         assert draw(x, 0.0, 0, 1.0, torch.zeros(5)).tolist() == want
+
+
+def test_first_of_two_zeros():
+    """Zeros of either sign are one largest value, wherever they lie: in a thread's four values, in those it reads 4096 places on, with another thread."""
+    for V in (3000, 40000, 70000):
+        at = [(5, 6), (8, 8 + V // 4096 * 1024), (8, V - 1), (9, 1030), (V // 2, V // 2 + 4096 if V > 8192 else V // 2 + 3)]
+        x = torch.full((2 * len(at), V), -1.0)
+        for i, (a, b) in enumerate(at):
+            for j, (p, q) in enumerate(((-0.0, 0.0), (0.0, -0.0))):
+                x[2 * i + j, a], x[2 * i + j, b] = p, q
+        assert draw(x, 0.0, 0, 1.0, torch.zeros(len(x))).tolist() == [a for a, _ in at for _ in range(2)]

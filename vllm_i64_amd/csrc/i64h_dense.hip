@@ -501,8 +501,10 @@ __global__ __launch_bounds__(256) void gated_postnorm_kernel(const i64h_postnorm
 // What bounds it is the chain of dependent sums, one per bit, so each is made short.  With top-k of at most half as many as there are threads the row
 // is read once: a bound that at least k of the threads' maxima reach and few others do is found by one wave that holds them all, the values above it
 // (at most one a thread, sorted by index) lie one to a thread from there on - and up to 128 of them in one wave, whose sums need no barrier.  Without
-// top-k the row's keys stay in registers (NV float4 per thread; NV = 0: read again, vocabularies beyond 32768).  64 rows of 32000, top-k 50 and
-// top-p 0.95: 1280 us with four waves that read the row again for every bit, 33 us with sixteen and a barrier a bit, 15.7 with one wave's sums.  Up to 4096
+// top-k the row's keys and weights stay in registers (NV float4 per thread; NV = 0: read again, vocabularies beyond 32768).  64 rows of 32000, top-k 50 and
+// top-p 0.95: 1280 us with four waves that read the row again for every bit, 33 us with sixteen and a barrier a bit, 15.3 with one wave's sums.  Without
+// top-k, top-p 0.9, 45.8 us with a maximum and its index looked for together, 54 where the weights were taken again for every bit, 42.8; rows of
+// 50257 drawn without either 56, 71 (read once more for a NaN and again for the maximum's place), 53.  Up to 4096
 // values four waves have the shorter sums: 64 rows of 1000 drawn without top-k 11 us, sixteen waves 16, rows of 4000 13 and 17.
 template <int NV, int SR_WAVES>
 __global__ __launch_bounds__(64 * SR_WAVES) void sample_rows_kernel(const float* __restrict__ logits, int64_t* __restrict__ out, int V, const int vec,
@@ -554,13 +556,22 @@ __global__ __launch_bounds__(64 * SR_WAVES) void sample_rows_kernel(const float*
     uint32_t key[NV > 0 ? NV : 1][4];
     // the largest number (kbest: its key, of what is no NaN; 0: none) and the largest key; where the first value that large lies is looked up behind them
     constexpr uint32_t KINF = 0xff800000u, KNINF = 0x007fffffu;      // the keys of the infinities: beyond them lie the NaNs
-    uint32_t kmax = 0, kbest = 0;
+    uint32_t kmax = 0, kbest = 0, kmin = ~0u;      // (NV = 0: the smallest key too, and the chunk of the first value that large)
+    int where = 0;
+    auto lowest = [&](int i, const uint32_t* q) {
+        if (i < V / STEP) kmin = min(min(min(q[0], q[1]), min(q[2], q[3])), kmin);
+        else
+#pragma unroll
+            for (int j = 0; j < 4; ++j) kmin = i * STEP + tid * 4 + j < V ? min(kmin, q[j]) : kmin;
+    };
     auto look = [&](int i, const uint32_t* k) {
+        const uint32_t front = kbest;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             kmax = max(kmax, k[j]);
             kbest = max(kbest, k[j] <= KINF ? k[j] : 0u);
         }
+        if (NV == 0 && kbest != front && !(kbest == 0x80000000u && front == 0x7fffffffu)) where = i;
     };
     if (NV > 0) {
 #pragma unroll
@@ -571,6 +582,7 @@ __global__ __launch_bounds__(64 * SR_WAVES) void sample_rows_kernel(const float*
         for (int i = 0; i < chunks; ++i) {
             load4(i, key[0]);
             look(i, key[0]);
+            lowest(i, key[0]);
         }
     }
     auto max16 = [](uint32_t v) {      // over sixteen neighbouring lanes
@@ -594,22 +606,21 @@ __global__ __launch_bounds__(64 * SR_WAVES) void sample_rows_kernel(const float*
     const uint32_t rbest = (uint32_t)__builtin_amdgcn_readfirstlane((int)max16(skey[lane & (SR_WAVES - 1)]));
     const uint32_t rmax = (uint32_t)__builtin_amdgcn_readfirstlane((int)max16(skey[SR_WAVES + (lane & (SR_WAVES - 1))]));
     // (two zeros are equal, their keys are not: the first of either)
-    auto as_best = [&](uint32_t k) { return k == rbest || (k + 1 == rbest && rbest == 0x80000000u); };
+    const uint32_t twin = rbest == 0x80000000u ? rbest - 1 : rbest;
     if (rbest >= KNINF && kbest >= rbest - 1) {      // (a few threads)
+        int first = V;
         auto find4 = [&](int i, const uint32_t* k) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (as_best(k[j]) && i * STEP + tid * 4 + j < V) atomicMin(&sarg, i * STEP + tid * 4 + j);
+            for (int j = 3; j >= 0; --j) first = k[j] == rbest || k[j] == twin ? i * STEP + tid * 4 + j : first;
         };
         if (NV > 0) {
 #pragma unroll
-            for (int i = 0; i < NV; ++i) find4(i, key[i]);
+            for (int i = NV - 1; i >= 0; --i) find4(i, key[i]);
         } else {
-            for (int i = 0; i < chunks; ++i) {
-                load4(i, key[0]);
-                find4(i, key[0]);
-            }
+            load4(where, key[0]);
+            find4(where, key[0]);
         }
+        if (first < V) atomicMin(&sarg, first);
     }
     __syncthreads();
     const int arg = sarg < V ? sarg : 0;
@@ -826,22 +837,28 @@ __global__ __launch_bounds__(64 * SR_WAVES) void sample_rows_kernel(const float*
             return n == k ? 2 : (n > k ? 1 : 0);
         });
     if (thr == 0u) {      // the NaN of all bits set is kept: the sum is no number
-        int lost = 0;
-        each([&](int i, const uint32_t* q) {
+        if (NV > 0)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) lost += wave_count(q[j] == 0u && i * STEP + tid * 4 + j < V);
-        });
-        if (sum_i(lost) > 0) {
+            for (int i = 0; i < NV; ++i) lowest(i, key[i]);
+        if (sum_i(wave_count(kmin == 0u)) > 0) {
             if (tid == 0) out[r] = arg;
             return;
         }
     }
     thr = max(thr, 1u);      // (0: the places past the end)
+    // (NV > 0: the weights beside their keys: left to the compiler they were taken again for every bit, a branch around each)
+    float held[NV > 0 ? NV : 1][4];
+    if (NV > 0)
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) held[i][j] = weight(key[i][j]);
+    auto weight_of = [&](int i, int j, uint32_t q) { return NV > 0 ? held[i][j] : weight(q); };
     auto mass = [&](uint32_t cut) {
         float s = 0.0f;
-        each([&](int, const uint32_t* q) {
+        each([&](int i, const uint32_t* q) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) s += q[j] >= cut ? weight(q[j]) : 0.0f;
+            for (int j = 0; j < 4; ++j) s += q[j] >= cut ? weight_of(i, j, q[j]) : 0.0f;
         });
         return sum_f(s);
     };
@@ -862,7 +879,7 @@ __global__ __launch_bounds__(64 * SR_WAVES) void sample_rows_kernel(const float*
         if (!open || i >= chunks) return;
         float w[4], s = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) w[j] = q[j] >= thr ? weight(q[j]) : 0.0f, s += w[j];
+        for (int j = 0; j < 4; ++j) w[j] = q[j] >= thr ? weight_of(i, j, q[j]) : 0.0f, s += w[j];
         float run = s;
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
