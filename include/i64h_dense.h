@@ -594,6 +594,9 @@ typedef struct {
 int i64h_gdn_gates(const i64h_gdn_args* d, void* stream);
 int i64h_gdn_scan(const i64h_gdn_args* d, void* stream);
 int64_t i64h_scan_work_floats(int64_t n, int32_t nseg, int32_t heads, int32_t dim);
+/* Whether either scan (delta != 0: i64h_gdn_scan, else i64h_gla_scan with keys of its own) of nseg runs of n rows, the longest of `longest` rows, is the
+ * faster in tiles, and a caller that knows its runs should give it a workspace.  The launch itself knows n and nseg only. */
+int32_t i64h_scan_in_tiles(int64_t n, int32_t nseg, int32_t longest, int32_t heads, int32_t dim, int32_t vdim, int32_t delta);
 int i64h_set_gdn_scan_form(int32_t form); /* tuning / test knob: 0 (default) = by the runs' length; 1 = loads straight into registers; 2, 3, 4 = staged
                                              through LDS with 1, 2, 4 value columns per lane (where 16-byte rows allow); same results bit for bit.
                                              5 = tiles of 16 tokens whatever the runs' length (with work, 16-byte rows, keys of their own) */

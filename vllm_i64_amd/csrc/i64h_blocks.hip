@@ -716,6 +716,18 @@ int i64h_set_gdn_scan_form(int32_t form) {
     return 0;
 }
 
+// Tiles of 16 tokens on the matrix cores are two launches and a tile costs the same however few rows it holds; token by token a launch takes as long as
+// its longest run.  So it is the longest run that decides.  Microseconds in replayed graphs, token by token | in tiles, delta rule (linear attention), heads
+// of 128: 16 heads, a run of 1531 rows 242 | 130 (218 | 83), of 160 29 | 23 (27 | 17), of 96 18.5 | 18.9 (17 | 14), 30 single rows beside 300 78 | 61 (67 | 44);
+// 8 heads, 8 runs of 512 120 | 82 (100 | 57), 20 single rows beside 128 33 | 35 (27 | 25); 8 heads of 64, 8 runs of 17 5.6 | 11.6 (5.0 | 9.0), 16 of 64
+// 14.7 | 17.8 (12.2 | 13.3), 4 of 96 14.0 | 15.4 (11.4 | 11.8).  Narrow heads in thousands of workgroups are little more than their reads either way (32 heads of 64, 32 runs of
+// 192 rows 172 | 187, 121 | 139), as are many short runs (64 of 17 rows 43 | 62).
+int32_t i64h_scan_in_tiles(int64_t n, int32_t nseg, int32_t longest, int32_t heads, int32_t dim, int32_t vdim, int32_t delta) {
+    const int64_t groups = (int64_t)heads * ((vdim + 15) / 16) * nseg;      // workgroups of the second launch
+    return dim % 4 == 0 && dim <= 256 && n >= 96 && n >= 8 * (int64_t)nseg && longest >= (delta ? 144 : 112) && (n >= 32 * (int64_t)nseg || groups < 6144) &&
+           (dim > 64 || groups <= 2048);
+}
+
 // the recurrence's launch, with the delta rule's correction or (a decay per key channel, every head its own keys) without it
 extern "C++" {
 template <int RULE>
@@ -726,11 +738,7 @@ static int gdn_launch(const i64h_gdn_args& d, void* stream) {
                (!d.F || (d.ldf % 4 == 0 && (uintptr_t)d.F % 16 == 0));
     };
     const int kround = kpt <= 4 ? 4 : (kpt <= 8 ? 8 : 16);
-    // Tiles of 16 tokens on the matrix cores: two launches, so that a few dozen rows stay with the chain from token to token.  Microseconds, token by
-    // token | in tiles, delta rule (linear attention), heads of 128: 16 heads, a run of 1531 rows 242 | 130 (214 | 81), 27 single rows beside 229 and 256
-    // 65 | 59 (56 | 41), 40 beside 300 75 | 64; 8 heads, 8 runs of 512 120 | 82 (100 | 57), runs of 300, 75 and 1 51 | 32; 77 rows 16 | 17, 24 rows 10 | 14.
-    // Many short runs are little more than reading and writing their states, and a tile of them is mostly empty: 64 of 17 rows, 32 heads of 64, 43 | 62.
-    const bool tiles = d.n >= 96 && d.n >= 8 * (int64_t)d.nseg && (d.n >= 32 * (int64_t)d.nseg || (int64_t)d.heads * ((d.vdim + 15) / 16) * d.nseg < 6144);
+    const bool tiles = i64h_scan_in_tiles(d.n, d.nseg, INT32_MAX, d.heads, d.dim, d.vdim, RULE == GD_DELTA);
     if (RULE != GD_FORGET && d.work && ((g_gdn_form == 0 && tiles) || g_gdn_form == 5) && vec_ok(4) && (uintptr_t)d.work % 16 == 0 && d.ldx < (1 << 25) &&
         (d.n / 16 + d.nseg) * (int64_t)d.heads < (1ll << 31)) {
         I64H_CHECK_ARG(d.work_floats >= i64h_scan_work_floats(d.n, d.nseg, d.heads, d.dim), "scan: a workspace of %lld floats, %lld needed", (long long)d.work_floats,

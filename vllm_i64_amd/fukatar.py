@@ -27,7 +27,7 @@ import torch
 
 from . import ops_dense as D
 from .config import FukatarConfig
-from .hybrid_runner import HybridRunner
+from .hybrid_runner import NO_WORK, HybridRunner
 from .model import attention_segments
 from .paged_cache import HybridCache
 
@@ -81,6 +81,7 @@ class FukatarModel(HybridRunner):
         self.max_a = max(d["n_a"] for d in self.layers)
         self.max_b = max(d["n_b"] for d in self.layers)
         self.max_gdn_heads = max([l.mixer.right.heads for l in cfg.layers if l.type == "parallel"] or [0])
+        self.scans = {(r.heads, r.dim, r.vdim) for r in (l.mixer.right for l in cfg.layers if l.type == "parallel")}
         self.max_ff = max([l.mlp.ff for l in cfg.layers if l.mlp is not None] or [0])
         if cache_dtype is None:
             cache_dtype = torch.float32 if self.exact else torch.bfloat16
@@ -146,12 +147,12 @@ class FukatarModel(HybridRunner):
         D.linear(B.h, d["w_in"], P, exact=self.exact)
         self._latent_attention(B, d, d["m"], P, l, n, positions, slot_ids, kvc, runs, ctx_hint, B.y)
 
-    def _parallel(self, B, d, l, n, positions, slot_ids, kvc, seg, nseg, runs, ctx_hint, single) -> None:
+    def _parallel(self, B, d, l, n, positions, slot_ids, kvc, seg, nseg, runs, ctx_hint, single, work=NO_WORK) -> None:
         a, r = d["m"].left, d["m"].right
         P = B.p[: n * d["n_in"]].view(n, d["n_in"])
         D.linear(B.h, d["w_in"], P, exact=self.exact)
         self._rotary_attention(B, d, a, P, l, n, positions, slot_ids, kvc, runs, ctx_hint, B.y)
-        self._gated_delta(B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, single, B.y2)
+        self._gated_delta(B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, single, B.y2, work)
 
     @torch.no_grad()
     def forward(self, token_ids: torch.Tensor, positions: torch.Tensor, slot_ids: torch.Tensor, ctx_len: Optional[torch.Tensor] = None,
@@ -171,7 +172,8 @@ class FukatarModel(HybridRunner):
         if n == 0:
             return B.logits
         eps, ex = cfg.norm_eps, self.exact
-        seg, nseg = self._runs(n, slot_ids, tokens_per_seq, rows_are_slots)
+        seg, nseg, longest = self._runs(n, slot_ids, tokens_per_seq, rows_are_slots)
+        work = self._scan_work(n, nseg, longest, self.scans, delta=True)
         if tokens_per_seq is not None:
             runs = attention_segments(tokens_per_seq, n, self.ATTN_MAX_SEGMENTS)
         else:
@@ -194,7 +196,7 @@ class FukatarModel(HybridRunner):
             elif d["type"] == "attention":
                 self._attention(B, d, l, n, positions, slot_ids, kvc, runs, hint)
             else:
-                self._parallel(B, d, l, n, positions, slot_ids, kvc, seg, nseg, runs, hint, single)
+                self._parallel(B, d, l, n, positions, slot_ids, kvc, seg, nseg, runs, hint, single, work)
                 write.update(y2=B.y2, yn_w=d["out_left"], y2n_w=d["out_right"])
             D.streams_step(B.streams, **write)
             if d["mlp"] is not None:

@@ -13,6 +13,7 @@ import torch
 from . import ops_dense as D
 from .ops import upload
 
+NO_WORK: Dict[tuple, torch.Tensor] = {}     # a step whose scans take no workspace (_scan_work)
 UNIT_EPS = 1e-6     # inside the root of the delta rule's unit vectors: a constant of the mechanism, not of a checkpoint
 
 
@@ -139,12 +140,12 @@ class HybridRunner:
         self.kv.restore(held)
 
     def _runs(self, n: int, slot_ids: torch.Tensor, tokens_per_seq, rows_are_slots: bool):
-        """First rows of the runs of consecutive rows of one sequence, int32 [runs + 1] on the device, and their number."""
+        """First rows of the runs of consecutive rows of one sequence, int32 [runs + 1] on the device, their number and the longest one's rows."""
         if rows_are_slots:
             t = self._arange.get(n)
             if t is None:
                 t = self._arange[n] = torch.arange(n + 1, dtype=torch.int32, device=self.device)
-            return t, n
+            return t, n, 1
         if tokens_per_seq is None:      # (a caller that does not say how its rows are grouped: read it off the slot ids)
             s = slot_ids.tolist()
             tokens_per_seq, k = [], 0
@@ -158,7 +159,7 @@ class HybridRunner:
                 starts.append(starts[-1] + int(t))
         if starts[-1] != n:
             raise ValueError(f"tokens_per_seq adds up to {starts[-1]} rows, the step has {n}")
-        return upload(starts, torch.int32, self.device), len(starts) - 1
+        return upload(starts, torch.int32, self.device), len(starts) - 1, max(b - a for a, b in zip(starts, starts[1:]))
 
     def _splits(self, B, rows: int, heads: int, kv_heads: int, vals: int, width: int, ctx_hint: int, floats):
         """How many waves share a decode row's keys (about ATTN_WAVES waves in the launch, a wave keeping at least two tiles of 32 keys),
@@ -174,16 +175,18 @@ class HybridRunner:
             ws = B.attn_ws[key] = torch.empty(max(1, floats(splits)), dtype=torch.float32, device=self.device)
         return splits, ws
 
-    def _scan_work(self, B, n: int, nseg: int, r) -> Optional[torch.Tensor]:
-        """The workspace of a recurrence's scan over runs of more than a row."""
-        if n == nseg:
-            return None
-        runs = (nseg + 15) // 16 * 16
-        key = ("scan", runs, r.heads, r.dim)
-        ws = B.attn_ws.get(key)
-        if ws is None:
-            ws = B.attn_ws[key] = torch.empty(D.scan_work_floats(n, runs, r.heads, r.dim), dtype=torch.float32, device=self.device)
-        return ws
+    def _scan_work(self, n: int, nseg: int, longest: int, scans, delta: bool) -> Dict[tuple, torch.Tensor]:
+        """The workspace of a step's scans by (heads, dim, vdim), for those of `scans` whose runs are worth the form that takes one.  The caller holds it for
+        the step and no longer: 27 KB a tile of 16 rows and head of 128 would otherwise lie beside every kept buffer set.  Where the card has no room for
+        it the scans go token by token: the same values in another order of the sums."""
+        sizes = {s: D.scan_work_floats(n, nseg, s[0], s[1]) for s in scans if D.scan_in_tiles(n, nseg, longest, *s, delta=delta)}
+        if not sizes:
+            return {}
+        try:
+            ws = torch.empty(max(sizes.values()), dtype=torch.float32, device=self.device)
+        except torch.OutOfMemoryError:
+            return {}
+        return {s: ws for s in sizes}      # (one after the other on one stream)
 
     # ---- attention over grouped key / value heads, separate keys and values in one cached row ----
     def _kattn(self, B, a, Q, O, rows, kvc, slot_ids, positions, runs, ctx_hint: int, *, bias=None, softcap: float = 0.0, window: int = 0,
@@ -283,7 +286,7 @@ class HybridRunner:
         D.linear(og, d["o"], out, m=n, k=H * m.vdim, lda=H * m.vdim, exact=ex)
 
     # ---- gated linear attention ----
-    def _gated_linear(self, B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, out, scale: float = 1.0) -> None:
+    def _gated_linear(self, B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, out, scale: float = 1.0, work=NO_WORK) -> None:
         """Gated linear attention on the projection rows P (columns d["rq_off"], d["rk_off"], d["rv_off"], d["rg_off"]: queries, keys, values, output
         gates; d["a1_off"]: the low-rank decay map's first factor).  sigmoid(z)^(1 / tau) = exp(-softplus(-z) / tau): the second factor and
         its bias are held negated, the exponent's rate is d["a_rate"]."""
@@ -294,12 +297,12 @@ class HybridRunner:
         R, Rn, Rn16 = B.r[: n * rv].view(n, rv), None if wide else B.rn[: n * rv].view(n, rv), self._as16(B.rn, n, rv) if wide else None
         D.gla_scan(P, f=F, q_off=d["rq_off"], k_off=d["rk_off"], f_off=0, v_off=d["rv_off"], heads=r.heads, dim=r.dim, vdim=r.vdim, seg_start=seg, nseg=nseg,
                    positions=positions, slot_ids=slot_ids, state=kvc.state[l]["gla"], out=R, n=n, q_scale=r.dim ** -0.5,
-                   work=self._scan_work(B, n, nseg, r))
+                   work=work.get((r.heads, r.dim, r.vdim)))
         D.gate_norm(R, d["r_norm"], Rn, groups=r.heads, eps=self.cfg.norm_eps, z=P, z_off=d["rg_off"], ldz=P.shape[-1], n=n, gate_after=True, width=rv, out16=Rn16)
         self._out(Rn, d["o_right"], out, scale, Rn16)
 
     # ---- gated delta rule ----
-    def _gated_delta(self, B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, single: bool, out) -> None:
+    def _gated_delta(self, B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, single: bool, out, work=NO_WORK) -> None:
         """Gated delta rule on the projection rows P: the convolved parts q | k | v from column d["r_off"] on, the write strength's at
         d["rb_off"].  A decay per head comes from the columns d["ra_off"]; a decay per key channel (r.decay 'channel') and its output gate are
         low-rank maps whose first factors' results lie at d["a1_off"] and d["g1_off"]."""
@@ -320,8 +323,8 @@ class HybridRunner:
             D.linear(P, d["a2"], F, m=n, a_off=d["a1_off"], exact=ex, bias=d["dt_bias"], epilogue=D.EPI_DECAY, e=d["a_rate"])
             D.linear(P, d["g2"], Z, m=n, a_off=d["g1_off"], exact=ex)
         R = B.b[: n * rv].view(n, rv)
-        D.gdn_scan(X, G, f=F, seg_start=seg, nseg=nseg, positions=positions, slot_ids=slot_ids, state=st["gdn"], out=R, work=self._scan_work(B, n, nseg, r),
-                   **cols)
+        D.gdn_scan(X, G, f=F, seg_start=seg, nseg=nseg, positions=positions, slot_ids=slot_ids, state=st["gdn"], out=R,
+                   work=work.get((r.heads, r.dim, r.vdim)), **cols)
         wide = self._wide(n, rv)
         Rn, Rn16 = None if wide else B.c[: n * rv].view(n, rv), self._as16(B.c, n, rv) if wide else None
         D.gate_norm(R, d["r_norm"], Rn, groups=r.heads, eps=self.cfg.norm_eps, z=Z, z_off=z_off, ldz=ldz, n=n, gate_after=True, width=rv, sigmoid=r.gate == "sigmoid", out16=Rn16)

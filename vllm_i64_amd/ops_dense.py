@@ -544,6 +544,11 @@ def scan_work_floats(n: int, nseg: int, heads: int, dim: int) -> int:
     return int(_lib.load_dense().i64h_scan_work_floats(int(n), int(nseg), int(heads), int(dim)))
 
 
+def scan_in_tiles(n: int, nseg: int, longest: int, heads: int, dim: int, vdim: int, *, delta: bool) -> bool:
+    """Whether a scan over nseg runs of n rows, the longest of `longest` rows, is worth a workspace (see i64h_scan_in_tiles)."""
+    return bool(_lib.load_dense().i64h_scan_in_tiles(int(n), int(nseg), int(longest), int(heads), int(dim), int(vdim), int(bool(delta))))
+
+
 def _scan_work(work: Optional[torch.Tensor]) -> dict:
     if work is None:
         return {}

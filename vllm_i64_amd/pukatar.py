@@ -95,6 +95,7 @@ class PukatarModel(HybridRunner):
         self.max_rk = max([m.heads * m.dim for m in deltas] or [0])
         self.max_rv = max([m.heads * m.vdim for m in deltas] or [0])
         self.max_delta_heads = max([m.heads for m in deltas] or [0])
+        self.scans = {(m.heads, m.dim, m.vdim) for m in deltas}
         self._moe_sizes([l.mlp for l in cfg.layers])
         if cache_dtype is None:
             cache_dtype = torch.float32 if self.exact else torch.bfloat16
@@ -159,7 +160,8 @@ class PukatarModel(HybridRunner):
         if n == 0:
             return B.logits
         eps, ex, hint = cfg.norm_eps, self.exact, int(max_ctx_hint)
-        seg, nseg = self._runs(n, slot_ids, tokens_per_seq, rows_are_slots)
+        seg, nseg, longest = self._runs(n, slot_ids, tokens_per_seq, rows_are_slots)
+        work = self._scan_work(n, nseg, longest, self.scans, delta=True)
         if tokens_per_seq is not None:
             runs = attention_segments(tokens_per_seq, n, self.ATTN_MAX_SEGMENTS)
         else:
@@ -192,7 +194,7 @@ class PukatarModel(HybridRunner):
             if d["type"] == "attention":
                 self._rotary_attention(B, d, d["m"], P, r, n, positions, slot_ids, kvc, runs, hint, B.y)
             else:
-                self._gated_delta(B, d, d["m"], P, r, n, positions, slot_ids, kvc, seg, nseg, single, B.y)
+                self._gated_delta(B, d, d["m"], P, r, n, positions, slot_ids, kvc, seg, nseg, single, B.y, work)
             write = dict(y=B.y, out_w=self.ones1)
             if d["mlp"] is not None:
                 write.update(ff)

@@ -27,7 +27,7 @@ import torch
 
 from . import ops_dense as D
 from .config import VepelixConfig
-from .hybrid_runner import HybridRunner
+from .hybrid_runner import NO_WORK, HybridRunner
 from .model import attention_segments
 from .paged_cache import HybridCache
 
@@ -88,6 +88,7 @@ class VepelixModel(HybridRunner):
         self.max_q = max([m.q_width for m in latents] or [0])
         self.max_rk = max([r.heads * r.dim for r in rights] or [0])
         self.max_rv = max([r.heads * r.vdim for r in rights] or [0])
+        self.scans = {(r.heads, r.dim, r.vdim) for r in rights}
         self._moe_sizes([l.mlp for l in cfg.layers])
         if cache_dtype is None:
             cache_dtype = torch.float32 if self.exact else torch.bfloat16
@@ -127,7 +128,7 @@ class VepelixModel(HybridRunner):
         return d
 
     # ---- sublayers: the input is B.h, the result lands in B.y (and B.y2, to be added) ----
-    def _mixer(self, B, d, r, n, positions, slot_ids, kvc, seg, nseg, runs, hint, h16=None) -> dict:
+    def _mixer(self, B, d, r, n, positions, slot_ids, kvc, seg, nseg, runs, hint, h16=None, work=NO_WORK) -> dict:
         """Returns the operands of the residual's write.  h16: the input rows in bf16, read in B.h's place."""
         m = d["m"]
         P = B.p[: n * d["ld"]].view(n, d["ld"])
@@ -137,7 +138,7 @@ class VepelixModel(HybridRunner):
             return dict(y=B.y)
         with self._beside(n):      # attention and recurrence share nothing but the projection rows
             self._rotary_attention(B, d, m.left, P, r, n, positions, slot_ids, kvc, runs, hint, B.y, m.left_scale)
-        self._gated_linear(B, d, m.right, P, r, n, positions, slot_ids, kvc, seg, nseg, B.y2, m.right_scale)
+        self._gated_linear(B, d, m.right, P, r, n, positions, slot_ids, kvc, seg, nseg, B.y2, m.right_scale, work)
         self._meet(n)
         return dict(y=B.y, y2=B.y2)
 
@@ -166,7 +167,8 @@ class VepelixModel(HybridRunner):
         B = self.buffers(n, M)
         if n == 0:
             return B.logits
-        seg, nseg = self._runs(n, slot_ids, tokens_per_seq, rows_are_slots)
+        seg, nseg, longest = self._runs(n, slot_ids, tokens_per_seq, rows_are_slots)
+        work = self._scan_work(n, nseg, longest, self.scans, delta=False)
         if tokens_per_seq is not None:
             runs = attention_segments(tokens_per_seq, n, self.ATTN_MAX_SEGMENTS)
         else:
@@ -183,7 +185,7 @@ class VepelixModel(HybridRunner):
             elif t:
                 D.streams_step(x, y=B.xe[1], out_w=self.ones1, **normed(d["norm1"]))
             # (elsewhere the launch that wrote the residual has normed it)
-            write = self._mixer(B, d, r, n, positions, slot_ids, kvc, seg, nseg, runs, int(max_ctx_hint), B.h16)
+            write = self._mixer(B, d, r, n, positions, slot_ids, kvc, seg, nseg, runs, int(max_ctx_hint), B.h16, work)
             write.update(out_w=self.ones1, y_scale=d["ls1"])
             if d["mlp"] is not None:
                 D.streams_step(x, **write, **(normed(d["norm2"]) if d["mlp"].kind == "dense" else read(d["norm2"], B.h, h16=B.h16)))

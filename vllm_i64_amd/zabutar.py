@@ -184,7 +184,7 @@ class ZabutarModel(HybridRunner):
         if n == 0:
             return B.logits
         eps = cfg.norm_eps
-        seg, nseg = self._runs(n, slot_ids, tokens_per_seq, rows_are_slots)
+        seg, nseg, _ = self._runs(n, slot_ids, tokens_per_seq, rows_are_slots)
         if tokens_per_seq is not None:
             runs = attention_segments(tokens_per_seq, n, self.ATTN_MAX_SEGMENTS)
         else:
