@@ -358,9 +358,11 @@ class HybridRunner:
 
     @staticmethod
     def moe_buffers(B, model, n: int) -> None:
-        """The step buffers of _moe_ff on B (model.max_top == 0: no mixtures)."""
+        """The step buffers of the feed-forwards on B (model.max_top == 0: no mixtures)."""
         i32, f32 = dict(dtype=torch.int32, device=model.device), dict(dtype=torch.float32, device=model.device)
-        t, g = model.max_top, model.max_grouped
+        B.joined = model._joins(n)
+        t, (g, act, shared) = model.max_top, model.ff_sizes[B.joined]
+        B.act = torch.empty(n * max(act, 1), **f32)
         B.ey = torch.empty(n * g, model.cfg.width, **f32) if t else None   # the outputs, grouped by expert
         B.idx = torch.empty(n * max(t, 1), **i32)
         B.wgt = torch.empty(n * max(t, 1), **f32)
@@ -369,16 +371,19 @@ class HybridRunner:
         B.pair_wgt = torch.empty(n * max(g, 1), **f32)
         B.group_off = torch.empty(model.max_groups + 1, **i32)
         B.sgate = torch.empty(n, **f32)
-        B.sact = torch.empty(n * max(model.max_shared, 1), **f32)
+        B.sact = torch.empty(n * max(shared, 1), **f32)                    # the inner rows of a shared expert beside the grouped launches
+        B.shared_rows = n if shared else 0
 
     def _moe_sizes(self, mlps) -> None:
         moes = [m for m in mlps if m is not None and m.kind == "moe"]
         self.max_top = max([m.top for m in moes] or [0])
         self.max_groups = max([m.experts + int(self._shared_in_stack(m)) for m in moes] or [0])
-        self.max_shared = max([m.shared_ff for m in moes] or [0])
-        grouped = [m.top + int(self._shared_in_stack(m)) for m in moes]      # rows a token has in the grouped Linears
-        self.max_grouped = max(grouped or [0])
-        self.max_act = max([m.ff for m in mlps if m is not None and m.kind == "dense"] + [m.ff * g for m, g in zip(moes, grouped)] + [0])
+        dense = [m.ff for m in mlps if m is not None and m.kind == "dense"]
+        self.ff_sizes = {}      # by B.joined: rows a token has in the grouped Linears, its widest inner rows, the widest shared expert beside the grouped launches
+        for joined in (False, True):
+            inside = [joined and self._shared_in_stack(m) for m in moes]
+            rows = [m.top + int(i) for m, i in zip(moes, inside)]
+            self.ff_sizes[joined] = (max(rows or [0]), max(dense + [m.ff * r for m, r in zip(moes, rows)] + [0]), max([m.shared_ff for m, i in zip(moes, inside) if not i] or [0]))
 
     @staticmethod
     def _glu(limit: float, alpha: float) -> dict:
@@ -403,6 +408,13 @@ class HybridRunner:
         D.linear(h, d["ff_gate_up"], act, a16=h16, out16=act16, exact=self.exact, **self._glu(f.limit, f.glu_alpha))
         D.linear(act, d["ff_down"], out, a16=act16, exact=self.exact)
 
+    MOE_BESIDE = False      # the shared expert of a mixture may run on the side stream, beside the choice and the plan
+
+    def _joins(self, n: int) -> bool:
+        """Whether a shared expert in its experts' stack joins their launches in a step of n rows, but where it can run beside the choice and the plan of much work (8
+        prompts of 512, width 1024: 3572 us a step joined, 3432 beside; where the whole feed-forward runs beside a mixer joined is better, 5593 and 5804)."""
+        return not (self.MOE_BESIDE and self.side is not None and n * self.cfg.width >= self.FORK_WORK)
+
     def _moe_merges(self) -> bool:
         """Whether the residual's launch sums a mixture's rows itself (i64h_streams_args.moe_y)."""
         return self.cfg.width % 4 == 0 and self.cfg.width <= 8192
@@ -413,9 +425,7 @@ class HybridRunner:
         weighted sum is left to the caller's residual launch, whose operands are returned."""
         f, ex, W = d["mlp"], self.exact, self.cfg.width
         E, top = f.experts, f.top
-        # a shared expert in the experts' stack joins their launches, but where it can run beside the choice and the plan of much work (8 prompts of
-        # 512, width 1024: 3572 us a step joined, 3432 beside; where the whole feed-forward runs beside a mixer joined is better, 5593 and 5804)
-        merged = d["merged"] and not (beside and n * W >= self.FORK_WORK)
+        merged = d["merged"] and B.joined
         gate = B.sgate if f.shared_ff and f.shared_gate else None
         shared = None
         if f.shared_ff and not merged:

@@ -43,7 +43,6 @@ class _StepBuffers:
         self.h16 = torch.empty(n, W, dtype=torch.bfloat16, device=model.device) if model._wide(n, W) else None      # ... in bf16
         self.y = torch.empty(n, W, **f32)                       # the mixer's result
         self.y2 = torch.empty(n, W, **f32)                      # the feed-forward's
-        self.y3 = torch.empty(n if model.max_shared else 0, W, **f32)
         self.p = torch.empty(n * model.max_proj, **f32)         # everything projected from the layer's input
         self.a = torch.empty(n * model.max_a, **f32)            # query rows / convolution output
         self.b = torch.empty(n * model.max_b, **f32)            # attention output / recurrence output
@@ -51,8 +50,8 @@ class _StepBuffers:
         self.f = torch.empty(n * model.max_rk, **f32)           # decays per key channel
         self.z = torch.empty(n * model.max_rv, **f32)           # raw output gates
         self.g = torch.empty(n * 2 * model.max_delta_heads, **f32)      # write strengths
-        self.act = torch.empty(n * max(model.max_act, 1), **f32)
         HybridRunner.moe_buffers(self, model, n)
+        self.y3 = torch.empty(self.shared_rows, W, **f32)       # a shared expert's, where it is not in the experts' stack
         self.xf = torch.empty(m, W, **f32)
         self.logits = torch.empty(m, model.cfg.vocab, **f32)
         self.attn_ws: Dict[tuple, torch.Tensor] = {}

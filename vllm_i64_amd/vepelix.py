@@ -49,7 +49,6 @@ class _StepBuffers:
         self.f = torch.empty(n * model.max_rk, **f32)           # decays per key channel
         self.r = torch.empty(n * model.max_rv, **f32)           # recurrence output
         self.rn = torch.empty(n * model.max_rv, **f32)          # ... normed and gated
-        self.act = torch.empty(n * max(model.max_act, 1), **f32)
         HybridRunner.moe_buffers(self, model, n)
         self.xf = torch.empty(m, W, **f32)
         self.logits = torch.empty(m, model.cfg.vocab, **f32)
@@ -59,6 +58,7 @@ class _StepBuffers:
 class VepelixModel(HybridRunner):
     BUFFERS = _StepBuffers
     SIDE_STREAM = True
+    MOE_BESIDE = True
 
     def __init__(self, cfg: VepelixConfig, weights: Dict[str, torch.Tensor], device="cuda:0", dtype: str = "bfloat16", max_seqs: int = 4,
                  num_kv_blocks: int = 256, kv_block: int = 16, cache_dtype: Optional[torch.dtype] = None):

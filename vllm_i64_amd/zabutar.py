@@ -49,7 +49,6 @@ class _StepBuffers:
         self.p = torch.empty(n * model.max_proj, **f32)         # everything projected from the sublayer input
         self.a = torch.empty(n * model.max_a, **f32)            # queries / recurrence output
         self.b = torch.empty(n * model.max_a, **f32)            # attention output / normed recurrence output
-        self.act = torch.empty(n * max(model.max_act, 1), **f32)
         HybridRunner.moe_buffers(self, model, n)
         self.xf = torch.empty(m, W, **f32)
         self.logits = torch.empty(m, model.cfg.vocab, **f32)
