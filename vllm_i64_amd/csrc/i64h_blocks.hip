@@ -854,7 +854,7 @@ int i64h_moe_plan(const i64h_moe_plan_args* dp, void* stream) {
     const i64h_moe_plan_args& d = *dp;
     I64H_CHECK_ARG(d.experts > 0 && d.experts <= 4096 && d.top > 0 && d.n >= 0, "moe_plan: %d experts (at most 4096), top %d", d.experts, d.top);
     I64H_CHECK_ARG(d.idx && d.group_off && d.pair_token && d.pair_row, "moe_plan: null operand");
-    I64H_CHECK_ARG(d.n * ((int64_t)d.top + 1) < (1ll << 31), "moe_plan: too many pairs");
+    I64H_CHECK_ARG(d.n * ((int64_t)d.top + (d.shared ? 1 : 0)) < (1ll << 31), "moe_plan: too many pairs");
     I64H_CHECK_ARG(!d.pair_wgt || d.wgt, "moe_plan: weights per row come from the weights per choice");
     hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(1024), (size_t)(2 * d.experts + 1) * 4, (hipStream_t)stream, d);
     I64H_CHECK_LAUNCH();

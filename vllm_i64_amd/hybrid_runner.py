@@ -36,6 +36,7 @@ class HybridRunner:
         self._bufs: Dict[tuple, object] = {}
         self._pinned: set = set()
         self._arange: Dict[int, torch.Tensor] = {}
+        self.max_ff = 0      # the widest feed-forward's inner rows
         self.side = torch.cuda.Stream(device=self.device) if self.SIDE_STREAM and self.device.type == "cuda" else None
 
     # ---- two sublayers side by side ----
@@ -64,11 +65,12 @@ class HybridRunner:
             torch.cuda.current_stream().wait_stream(self.side)
 
     # ---- rows that only Linears read: their producer rounds them to bf16 once where enough rows share a tile ----
-    WIDE_ROWS = 64      # more rows than this
+    WIDE_ROWS = 64                  # more rows than this
+    WIDE_BYTES = 0xfffffff0 - 64    # what the 32-bit offsets of the tiles on such rows reach: gathered rows, and the gate and up rows of a pair's weight
 
     def _wide(self, n: int, *widths: int) -> bool:
         """Whether Linears over rows of these widths read them in bf16 (the values their tiles would round to: results are the same)."""
-        return not self.exact and n > self.WIDE_ROWS and all(w % 64 == 0 for w in widths)
+        return not self.exact and n > self.WIDE_ROWS and all(w % 64 == 0 and 2 * w * max(n, self.max_ff + 256) < self.WIDE_BYTES for w in widths)
 
     @staticmethod
     def _as16(t: torch.Tensor, n: int, width: int) -> torch.Tensor:
@@ -379,6 +381,7 @@ class HybridRunner:
         self.max_top = max([m.top for m in moes] or [0])
         self.max_groups = max([m.experts + int(self._shared_in_stack(m)) for m in moes] or [0])
         dense = [m.ff for m in mlps if m is not None and m.kind == "dense"]
+        self.max_ff = max(dense + [w for m in moes for w in (m.ff, m.shared_ff)] + [0])
         self.ff_sizes = {}      # by B.joined: rows a token has in the grouped Linears, its widest inner rows, the widest shared expert beside the grouped launches
         for joined in (False, True):
             inside = [joined and self._shared_in_stack(m) for m in moes]
