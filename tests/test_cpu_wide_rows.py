@@ -27,3 +27,8 @@ def test_pairs_of_a_plan_without_a_shared_group():
         d = _lib.MoePlan(idx=buf, n=n, top=top, experts=4, group_off=buf, pair_token=buf, pair_row=buf, wgt=0, pair_wgt=buf, shared=shared)
         with pytest.raises(_lib.I64HError, match=what):
             _lib.call_dense("i64h_moe_plan", ctypes.addressof(d), 0)
+
+
+def test_experts_of_a_few_rows_each():
+    fills = HybridRunner._fills
+    assert fills(2, 8) and fills(8 * 40, 8) and not fills(319, 16) and fills(320, 16) and not fills(2 * 500, 64) and fills(8 * 200, 64)

@@ -418,6 +418,14 @@ class HybridRunner:
         prompts of 512, width 1024: 3572 us a step joined, 3432 beside; where the whole feed-forward runs beside a mixer joined is better, 5593 and 5804)."""
         return not (self.MOE_BESIDE and self.side is not None and n * self.cfg.width >= self.FORK_WORK)
 
+    @staticmethod
+    def _fills(pairs: int, experts: int) -> bool:
+        """Whether the experts' rows are enough for the wide tiles, whose smallest is 64 rows high: many experts of a few rows each read rows that are not there as
+        often as weights.  Microseconds of a pair's two launches, rows in fp32 | in bf16, width 2048, 768 inner: 16 experts of two, 100 tokens 37 | 39, 200
+        44 | 41; 32 of two, 100 tokens 65 | 69, 320 69 | 69, 400 77 | 70; 64 of two, 200 tokens 113 | 121, 700 134 | 127; 64 of eight, 100 tokens 120 | 126, 200 136 | 126; 128 of
+        eight, 100 tokens 217 | 226, 320 242 | 234; 8 of two (1792 inner), 65 tokens 48 | 45."""
+        return experts < 16 or pairs >= 20 * experts
+
     def _moe_merges(self) -> bool:
         """Whether the residual's launch sums a mixture's rows itself (i64h_streams_args.moe_y)."""
         return self.cfg.width % 4 == 0 and self.cfg.width <= 8192
@@ -445,9 +453,10 @@ class HybridRunner:
         pair_wgt = B.pair_wgt if f.weigh_input else None      # the weight multiplies what the expert reads, not what it returns
         D.moe_plan(B.idx, n=n, top=top, experts=E, group_off=B.group_off, pair_token=B.pair_token, pair_row=B.pair_row, wgt=B.wgt, pair_wgt=pair_wgt, shared=merged)
         # the (token, expert) pairs lie grouped by expert: one launch runs every expert over its own rows, the counts stay on the device
+        x16 = h16 if self._fills(n * top, E) else None
         rows, groups = n * (top + int(merged)), E + int(merged)
-        act, act16 = self._act(B.act, rows, f.ff, h16)
-        D.linear(h, gate_up, act, a16=h16, out16=act16, m=n, a_rows=B.pair_token[:rows], batch=groups, w_batch=2 * f.ff * W, exact=ex, group_off=B.group_off, row_scale=pair_wgt,
+        act, act16 = self._act(B.act, rows, f.ff, x16)
+        D.linear(h, gate_up, act, a16=x16, out16=act16, m=n, a_rows=B.pair_token[:rows], batch=groups, w_batch=2 * f.ff * W, exact=ex, group_off=B.group_off, row_scale=pair_wgt,
                  **self._glu(f.limit, f.glu_alpha))
         D.linear(act, e_down, B.ey[:rows], a16=act16, m=n, batch=groups, w_batch=W * f.ff, exact=ex, group_off=B.group_off)
         if shared is not None and beside:
