@@ -67,3 +67,37 @@ def test_decode_rows(form, r, rot, heads, window, keep, splits, bad):
         for h in range(H):
             want = oracle(Q[s, h:h + 1], rows[:, h // heads], r, koff, scale, seen, sink[h:h + 1])
             assert float((got[s, h] - want[0]).abs().max() / want.abs().max()) < TOL, (T, h)
+
+
+@pytest.mark.parametrize("cap", [0.0, 2.5])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("scaled", [False, True])
+@pytest.mark.parametrize("r,rot", [(64, 64), (32, 24), (128, 128), (48, 80)])
+def test_options_of_the_scores(r, rot, cap, bias, scaled):
+    """Key scales, soft cap and distance bias, in that order, alone and together; contexts that end at the edges of the tiles of 32 keys."""
+    from vllm_i64_amd import ops_dense as D
+    dev, block, G, H, lens = torch.device("cuda:0"), 16, 2, 10, [1, 31, 32, 33, 64, 97, 200]
+    g = torch.Generator().manual_seed(r + rot)
+    n, width, per = len(lens), r + rot, (max(lens) + block - 1) // block
+    bt = torch.randperm(n * per, generator=g).int().view(n, per)
+    cache = torch.randn(n * per, block, G * width, generator=g).to(torch.bfloat16)
+    ks = torch.rand(n * per, block, generator=g) + 0.5
+    table = torch.randn(70, H, generator=g)      # (distances beyond take its last row)
+    Q = torch.randn(n, H, width, generator=g) * 0.1
+    Q[:, :, :r] = 0.0
+    pos, slots, out = torch.tensor([T - 1 for T in lens], dtype=torch.int32, device=dev), torch.arange(n, dtype=torch.int32, device=dev), torch.full((n, H * r), 7.0, device=dev)
+    ws = torch.empty(D.kattn_workspace_floats(n, H, G, r, 3), device=dev)
+    D.kattn(Q.view(n, -1).to(dev), cache.to(dev), ks.to(dev) if scaled else None, bt.to(dev), slots, pos, chunk=0, bias=table.to(dev) if bias else None, sink=False, heads=H, kv_heads=G,
+            dim=rot, vdim=r, out=out, n=n, mode=2, splits=3, workspace=ws, softcap=cap)
+    got = out.cpu().double().view(n, H, r)
+    for s, T in enumerate(lens):
+        j = torch.arange(T)
+        at = bt[s].long()[j // block] * block + j % block
+        rows = cache.view(-1, G, width)[at].double()
+        for h in range(H):
+            z = rows[:, h // (H // G), r:] @ Q[s, h, r:].double()
+            z = z * ks.view(-1)[at].double() if scaled else z
+            z = cap * torch.tanh(z / cap) if cap else z
+            z = z + table.double()[(T - 1 - j).clamp(max=69), h] if bias else z
+            want = torch.softmax(z, 0) @ rows[:, h // (H // G), :r]
+            assert float((got[s, h] - want).abs().max() / want.abs().max()) < TOL, (T, h)

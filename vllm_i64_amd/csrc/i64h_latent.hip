@@ -178,7 +178,9 @@ __device__ __forceinline__ void lt_split(float x, uint32_t& hi, uint32_t& lo) {
 // (ds_read_b64_tr_b16), out^T[kv_rank, 16] += V^T P^T in fp32.  Every product of two bf16 values is exact in fp32.
 // What bounds it is the instructions of one wave a SIMD, and branches most of all: 64 tokens of 32 heads over one row of 288, 2048 keys, 63 | 40 us against
 // the form with a branch around every step, score and query fragment (a tile 14000 cycles; the weights through LDS and columns transposed by 144 two-byte
-// writes were the smaller part), one token, 500 keys 26 | 14, 32 heads of 64 over 8 key heads, 64 tokens, 1024 keys 38 | 30 (with the merge).
+// writes were the smaller part), one token, 500 keys 26 | 14, 32 heads of 64 over 8 key heads, 64 tokens, 1024 keys 38 | 30 (with the merge), 16 heads of 128 over 4,
+// 2048 keys 88 | 51.  The general instance, 64 tokens, 2048 keys: one row of 256 with 32 heads 60 | 54, values of 128 and keys of 64 77 | 67, heads of 64
+// with a soft cap 67 | 66.5 (72.5 with a branch around every score), with a bias 89 | 72 (88).
 // Arranged around the memory latency of such launches: a tile's 18 fragment loads are requested together, the NEXT tile's are
 // requested as soon as this tile's scores and transposed columns are done - under its softmax and second product - and the cache rows of the tile
 // after that are looked up a tile ahead.  The workgroup is one wave, so LDS traffic needs program order only (no barrier, whose
@@ -299,19 +301,25 @@ __global__ __launch_bounds__(64) void latent_attn_mfma_decode_kernel(const i64h_
         }
         __builtin_amdgcn_wave_barrier();
         if (tile + splits < tiles) request(cur ^ 1);          // the next tile travels under this tile's softmax and second product
-        // scores of keys kb + 16 b + 4 kg + g
+        // scores of keys kb + 16 b + 4 kg + g; one branch around the eight of an option, whose chains then run side by side
+        auto scores = [&](auto f) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) f(b, g, kb + 16 * b + 4 * kg + g);
+        };
+        if (ANY && p.kscale) scores([&](int b, int g, int) { S[b][g] *= ksc[b][g]; });
+        if (ANY && capl > 0.0f) scores([&](int b, int g, int) { S[b][g] = capl * tanhf(S[b][g] / capl); });
+        if (ANY && p.bias) {
+            float add[2][4];
+            scores([&](int b, int g, int j) { add[b][g] = p.bias[(int64_t)min(max(pos - j, 0), p.bias_rows - 1) * H + hq]; });
+            scores([&](int b, int g, int) { S[b][g] += 1.4426950408889634f * add[b][g]; });
+        }
         float mx = -INFINITY;
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int j = kb + 16 * b + 4 * kg + g;
-                float sc = ANY && p.kscale ? S[b][g] * ksc[b][g] : S[b][g];
-                if (ANY && capl > 0.0f) sc = capl * tanhf(sc / capl);
-                if (ANY && p.bias) sc += 1.4426950408889634f * p.bias[(int64_t)min(max(pos - j, 0), p.bias_rows - 1) * H + hq];
-                S[b][g] = (j <= pos && (j >= lo || j < keep)) ? sc : -INFINITY;
-                mx = fmaxf(mx, S[b][g]);
-            }
+        scores([&](int b, int g, int j) {
+            S[b][g] = (j <= pos && (j >= lo || j < keep)) ? S[b][g] : -INFINITY;
+            mx = fmaxf(mx, S[b][g]);
+        });
         const PairF m1 = swap_rows(mx);
         mx = fmaxf(m1.lo, m1.hi);
         const PairF m2 = swap_halves(mx);
