@@ -114,7 +114,7 @@ def test_qkv_with_its_tail(dev, n, kv_dtype, norm):
 
 @pytest.mark.parametrize("moe", [True, False])
 def test_step_of_a_model(dev, moe):
-    """A mixed step of 512-odd rows on either path: the same logits and cache."""
+    """A prompt of 300 rows on codes and with the rows quantized in front of every launch's tiles: the same logits and cache."""
     import dataclasses
     from oracle import model_ref as M
     from vllm_i64_amd.config import ModelConfig
@@ -133,3 +133,52 @@ def test_step_of_a_model(dev, moe):
         lg = model.forward(ids, pos, slots, (pos + 1).contiguous(), max_ctx_hint=n, tokens_per_seq=[n])
         runs.append([lg.clone()] + [t.clone() for t in (*model.kv.k, *model.kv.v)])
     assert all(torch.equal(a, b) for a, b in zip(*runs)) and bool(runs[0][0].isfinite().all())
+
+
+@pytest.mark.parametrize("moe", [True, False])
+@pytest.mark.parametrize("decode,prompt", [(31, 269), (40, 660), (7, 2093)])
+def test_mixed_steps_of_a_model(dev, moe, decode, prompt):
+    """Decoding sequences beside a new prompt on each of the three ways: rows quantized in front of every launch's tiles, once for the older tiled products, once for
+    the 64 x 64 tiles.  The first and the last give the same logits and cache bit for bit."""
+    import dataclasses
+    from oracle import model_ref as M
+    from vllm_i64_amd.config import ModelConfig
+    from vllm_i64_amd.model import I64MoEModel
+    ocfg = dataclasses.replace(M.named_config("trhash500m-synth"), num_layers=2, vocab_size=500, name="cut", **({} if moe else dict(num_experts=1, shared_intermediate_size=0, top_k=1, intermediate_size=1024)))
+    model = I64MoEModel(ModelConfig.from_any(ocfg), M.make_weights(ocfg, seed=1), device=dev, max_seqs=decode + 1, num_kv_blocks=3 * decode + prompt // 16 + 2, quant="fp8")
+    g = torch.Generator().manual_seed(decode)
+    past = [5 + 2 * s % 30 for s in range(decode)]
+    for s, p in enumerate(past + [0]):
+        model.kv.reserve(s, p + (1 if s < decode else prompt))
+    for t in (*model.kv.k, *model.kv.v):
+        t.copy_(torch.randn(t.shape, generator=g))
+    held = [t.clone() for t in (*model.kv.k, *model.kv.v)]
+    ids = torch.randint(0, 500, (decode + prompt,), generator=g).to(dev)
+    pos = torch.cat([torch.tensor(past), torch.arange(prompt)]).to(torch.int32).to(dev)
+    slots = torch.cat([torch.arange(decode), torch.full((prompt,), decode)]).to(torch.int32).to(dev)
+    tps = [1] * decode + [prompt]
+    runs = []
+    for tiles, fused in ((False, 1 << 30), (False, 0), (True, 1024)):
+        model.FP8_TILE_ROWS = model.FP8_TILE_ROWS_MOE = 1 if tiles else 1 << 30
+        model.FP8_FUSE_MAX_ROWS = fused
+        for t, h in zip((*model.kv.k, *model.kv.v), held):
+            t.copy_(h)
+        lg = model.forward(ids, pos, slots, (pos + 1).contiguous(), max_ctx_hint=max(past + [prompt]) + 1, tokens_per_seq=tps)
+        runs.append([lg.clone()] + [t.clone() for t in (*model.kv.k, *model.kv.v)])
+    assert all(torch.equal(a, b) for a, b in zip(runs[2], runs[0]))
+    # the older tiles add in another order: 2^-24 of a sum, and where that moves a code of the next product by a step (a sixteenth of one of 1024 or more terms) 2e-3 of a
+    # row - a few rows of these steps at the outside
+    assert all(float((a.double() - b.double()).norm() / b.double().norm()) < 1e-3 for a, b in zip(runs[2], runs[1]))
+    assert bool(runs[2][0].isfinite().all())
+
+
+def test_which_steps_take_the_tiles():
+    """Neither an eager step that more launches bind to the host nor a recording one."""
+    from oracle import model_ref as M
+    from vllm_i64_amd.config import ModelConfig
+    from vllm_i64_amd.model import I64MoEModel
+    for moe, first in ((True, 256), (False, 176)):
+        m = I64MoEModel.__new__(I64MoEModel)
+        m.cfg = ModelConfig.from_any(M.named_config("trhash500m-synth" if moe else "dense306-synth"))
+        m.layers = [dict(q_norm=None, k_norm=None)]
+        assert [m._fp8_tiles(n) for n in (1, first - 1, first, 12288, 12289)] == [False, False, True, True, False]

@@ -349,11 +349,13 @@ class I64MoEModel:
     # e4m3 runner: routed rows of a decode-sized step (ms/step at 256 | 512 | 1024: 200 sequences 4.97 | 3.48 | 3.48, 256 sequences
     # 5.75 | 4.41 | 4.40, 512 sequences 6.15 | 6.14 | 5.48)
     FP8_FUSE_MAX_ROWS = int(os.environ.get("I64H_FP8_FUSE_MAX_ROWS", "1024"))
-    # ... and from this many rows on the rows are quantized once and the products run in 64 x 64 tiles (us a step of two layers, without | with: mixture of
-    # experts 128 rows 193 | 241 - the host's launches -, 231 238 | 236, 512 341 | 255, 900 353 | 280, 4000 808 | 711, 12000 1627 | 1567, 16384 2002 | 2130; dense
-    # 128 199 | 204, 231 245 | 205, 512 341 | 237, 900 509 | 260, 4000 766 | 676, 12000 1680 | 1602, 16384 2158 | 2200)
-    FP8_TILE_ROWS = int(os.environ.get("I64H_FP8_TILE_ROWS", "160"))
-    FP8_TILE_ROWS_MOE = int(os.environ.get("I64H_FP8_TILE_ROWS_MOE", "240"))
+    # ... and from this many rows on the rows are quantized once and the products run in 64 x 64 tiles, in eager steps and in captured ones: below, more
+    # launches bind an eager step to the host (us a step of two layers, without | with: mixture of experts, a quarter of the rows decoding beside a prompt, 128 rows
+    # 194 | 241, 240 229 | 245, 256 258 | 249, 512 390 | 312, 1500 627 | 569; prompts alone 4000 808 | 711, 12000 1627 | 1567, 16384 2002 | 2130; captured decode of
+    # 160 sequences 263 | 275, 200 330 | 310, 256 354 | 323, 512 579 | 489, 1500 1193 | 1129; dense, mixed 160 rows 199 | 207, 176 217 | 207, 512 376 | 294, 1500
+    # 598 | 544; prompts 4000 766 | 676, 12000 1680 | 1602, 16384 2158 | 2200; captured 160 277 | 272, 512 570 | 476)
+    FP8_TILE_ROWS = int(os.environ.get("I64H_FP8_TILE_ROWS", "176"))
+    FP8_TILE_ROWS_MOE = int(os.environ.get("I64H_FP8_TILE_ROWS_MOE", "256"))
     FP8_TILE_MAX_ROWS = int(os.environ.get("I64H_FP8_TILE_MAX_ROWS", "12288"))
     EP_FUSE_MAX_ROWS = 1024  # the same for the pooled expert rows of the expert-parallel runner (8 ranks x 64 sequences x top-2)
     # expert-parallel runner, steps with more pooled expert rows than that (prefill chunks): dispatch every (route, token) row to the
@@ -800,8 +802,8 @@ class I64MoEModel:
             ops.fused_residual_norm(hbuf, self.final_norm, eps, normed=B.normed, h_out=B.h, lm_workspace=lm_ws)
 
     def _fp8_tiles(self, n: int) -> bool:
-        """Whether the e4m3 Linears of a step of n rows run on rows quantized once, in 64 x 64 tiles (see FP8_TILE_ROWS); same bits as the step that
-        quantizes in front of every launch's tiles."""
+        """Whether the e4m3 Linears of a step of n rows run on rows quantized once, in 64 x 64 tiles (see FP8_TILE_ROWS): the bits of the step that
+        quantizes in front of every launch's tiles (up to FP8_FUSE_MAX_ROWS routed rows); the older tiles of larger steps add in another order."""
         cfg = self.cfg
         if not ((self.FP8_TILE_ROWS_MOE if cfg.is_moe else self.FP8_TILE_ROWS) <= n <= self.FP8_TILE_MAX_ROWS and self.FP8_FUSE_NORM and cfg.head_dim == 64 and cfg.hidden_size <= 1024 and cfg.hidden_size % 64 == 0):
             return False
