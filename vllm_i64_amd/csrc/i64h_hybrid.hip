@@ -190,14 +190,15 @@ __global__ __launch_bounds__(256) void streams_kernel(const i64h_streams_args p)
 }
 
 // The ordinary residual sum (one stream, results without norms of their own) with rows of whole 16-byte slices: the row stays in registers
-// between the write and the norm, NV slices of four columns per thread.
-template <int NV>
+// between the write and the norm, NV slices of four columns per thread.  MIX: with a mixture's weighted sum; instances of their own, for its
+// registers and branches cost the launches without one (4096 rows of 2048: 26.2 us, 27.6 with them).
+template <int NV, bool MIX>
 __global__ __launch_bounds__(256) void residual_kernel(const i64h_streams_args p) {
     __shared__ float red[4];
     const int tid = threadIdx.x, W = p.W;
     const int64_t m = blockIdx.x;
     float* xs = p.streams + (p.rows ? (int64_t)p.rows[m] : m) * W;
-    const bool add = p.y || p.moe_y;
+    const bool add = MIX || p.y;
     const float ow = add ? p.out_w[0] : 0.0f;
     float v[NV][4];
     float ss = 0.0f, su = 0.0f;
@@ -215,7 +216,7 @@ __global__ __launch_bounds__(256) void residual_kernel(const i64h_streams_args p
                 const float4 y = *(const float4*)(p.y + m * p.ldy + c);
                 u[0] = y.x, u[1] = y.y, u[2] = y.z, u[3] = y.w;
             }
-            if (p.moe_y) {      // the sum of moe_combine_kernel, in its order; loads of four choices on their way together
+            if (MIX) {      // the sum of moe_combine_kernel, in its order; loads of four choices on their way together
                 const dn_v4f sh = p.moe_shared ? *(const dn_v4f*)(p.moe_shared + m * W + c) : dn_v4f{0, 0, 0, 0};
                 dn_v4f a = {0, 0, 0, 0};
                 for (int k0 = 0; k0 < p.moe_top; k0 += 4) {
@@ -904,10 +905,11 @@ int i64h_streams_step(const i64h_streams_args* dp, void* stream) {
     if (g_residual_form && d.S == 1 && !d.mix && !d.in_w && !d.yn_w && !d.post_w && d.W % 4 == 0 && d.W <= 8 * 1024 && at % 16 == 0 && (!d.y || d.ldy % 4 == 0) &&
         (!d.y2 || d.ldy2 % 4 == 0) && (!(d.h || d.h16) || d.norm_w_len == d.W)) {
         const dim3 grid((unsigned)rows);
-        if (d.W <= 1024) hipLaunchKernelGGL(residual_kernel<1>, grid, dim3(256), 0, (hipStream_t)stream, d);
-        else if (d.W <= 2048) hipLaunchKernelGGL(residual_kernel<2>, grid, dim3(256), 0, (hipStream_t)stream, d);
-        else if (d.W <= 4096) hipLaunchKernelGGL(residual_kernel<4>, grid, dim3(256), 0, (hipStream_t)stream, d);
-        else hipLaunchKernelGGL(residual_kernel<8>, grid, dim3(256), 0, (hipStream_t)stream, d);
+        auto launch = [&](auto sum, auto mix) { hipLaunchKernelGGL(d.moe_y ? mix : sum, grid, dim3(256), 0, (hipStream_t)stream, d); };
+        if (d.W <= 1024) launch(residual_kernel<1, false>, residual_kernel<1, true>);
+        else if (d.W <= 2048) launch(residual_kernel<2, false>, residual_kernel<2, true>);
+        else if (d.W <= 4096) launch(residual_kernel<4, false>, residual_kernel<4, true>);
+        else launch(residual_kernel<8, false>, residual_kernel<8, true>);
         I64H_CHECK_LAUNCH();
         return 0;
     }
