@@ -355,10 +355,11 @@ __device__ __forceinline__ void frr_flush(const uint32_t* tab_lo, const uint32_t
         }
 }
 
-__global__ __launch_bounds__(256) void fused_residual_norm_rows_kernel(FrrArgs p, const float* __restrict__ w, float* __restrict__ normed,
+template <int RPW, int WAVES>      // rows a wave takes, waves a workgroup has
+__global__ __launch_bounds__(64 * WAVES) void fused_residual_norm_rows_kernel(FrrArgs p, const float* __restrict__ w, float* __restrict__ normed,
                                                                        const int32_t* __restrict__ slots, int spr, int slot_base,
                                                                        uint32_t* __restrict__ stats, uint8_t* __restrict__ f8q = nullptr,
-                                                                       float* __restrict__ f8s = nullptr, int rpw = FRR_RPW) {
+                                                                       float* __restrict__ f8s = nullptr) {
     __shared__ uint32_t tab_lo[I64H_STAT_TAB], tab_hi[I64H_STAT_TAB];
     if (stats) {
         for (int i = threadIdx.x; i < I64H_STAT_TAB; i += 256) { tab_lo[i] = I64H_ORDERED_ZERO; tab_hi[i] = I64H_ORDERED_ZERO; }
@@ -366,14 +367,14 @@ __global__ __launch_bounds__(256) void fused_residual_norm_rows_kernel(FrrArgs p
     }
     const int lane = threadIdx.x & 63;
     const int nv = p.H / 4;  // <= 256 (launcher)
-    const int64_t t0 = ((int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * rpw;
+    const int64_t t0 = ((int64_t)blockIdx.x * WAVES + (threadIdx.x >> 6)) * RPW;
     float4 gw[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
         const int i = lane + 64 * v;
         gw[v] = ((normed || f8q) && i < nv) ? ((const float4*)w)[i] : make_float4(0, 0, 0, 0);
     }
-    for (int64_t t = t0; t < t0 + rpw && t < p.n; ++t) {
+    for (int64_t t = t0; t < t0 + RPW && t < p.n; ++t) {
         float4 y[4];
         float lo, hi;
         frr_row(p, t, lane, nv, [&](int v) { return gw[v]; },
@@ -890,7 +891,7 @@ static int frn_launch(const float* h, const float* add, const float* moe_rows, c
         const int64_t waves = (n + FRR_RPW - 1) / FRR_RPW;
         FrrArgs fa;
         fa.h = h; fa.add = add; fa.mc = mc; fa.n = n; fa.h_out = h_out; fa.eps = eps; fa.H = (int)H;
-        hipLaunchKernelGGL(fused_residual_norm_rows_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, (hipStream_t)stream, fa, norm_weight,
+        hipLaunchKernelGGL((fused_residual_norm_rows_kernel<FRR_RPW, 4>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, (hipStream_t)stream, fa, norm_weight,
                            normed, slots, (int)slots_per_row, (int)slot_base, stats, (uint8_t*)nullptr, (float*)nullptr);
         I64H_CHECK_LAUNCH();
         return 0;
@@ -941,10 +942,14 @@ int i64h_fused_residual_norm_fp8(const float* h, const float* add, const float* 
     fa.mc.rows = moe_rows; fa.mc.inv = moe_inv; fa.mc.shared = moe_shared; fa.mc.top_k = top_k;
     for (int k = 0; k < 8; ++k) fa.mc.wk[k] = (moe_rows && k < top_k) ? route_weights[k] : 0.0f;
     fa.mc.routed_scale = routed_scale; fa.mc.shared_scale = shared_scale;
-    // up to 2048 rows a wave of its own for each (512 rows: 32 workgroups of sixteen rows 15.8 us, a wave each 6.7)
-    const int rpw = n <= 2048 ? 1 : FRR_RPW, nt = n <= 2048 ? 64 : 256, per = rpw * (nt / 64);
-    hipLaunchKernelGGL(fused_residual_norm_rows_kernel, dim3((unsigned)((n + per - 1) / per)), dim3(nt), 0, (hipStream_t)stream, fa, norm_weight, normed,
-                       (const int32_t*)nullptr, 1, 0, (uint32_t*)nullptr, q_rows, q_scale, rpw);
+    // up to 2048 rows a wave of its own for each (512 rows: 32 workgroups of sixteen rows 15.8 us, a wave each 6.7; rows of a replayed graph 13.5 and 5.2, 2048
+    // rows 14.2 and 7.0)
+    auto launch = [&](auto kern, int waves, int rows) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)((n + rows - 1) / rows)), dim3(64 * waves), 0, (hipStream_t)stream, fa, norm_weight, normed, (const int32_t*)nullptr, 1, 0, (uint32_t*)nullptr,
+                           q_rows, q_scale);
+    };
+    if (n <= 2048) launch(fused_residual_norm_rows_kernel<1, 1>, 1, 1);
+    else launch(fused_residual_norm_rows_kernel<FRR_RPW, 4>, 4, 4 * FRR_RPW);
     I64H_CHECK_LAUNCH();
     return 0;
 }
