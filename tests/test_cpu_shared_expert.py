@@ -20,8 +20,18 @@ def test_apart_only_where_it_runs_beside_something(monkeypatch, design):
     m = make(monkeypatch, design)
     assert m.side is None and all(m._joins(n) for n in (1, 100, 1 << 20))      # no second stream: nothing to run beside
     m.side = object()
-    m.FORK_WORK = 128 * 200
+    m.FORK_WORK = 128 * 128 * 200
     assert m._joins(199) and m._joins(200) == (design == "pukatar")
+
+
+@pytest.mark.parametrize("width,rows,exact", [(1024, 1574, False), (2048, 394, False), (1024, 787, True)])
+def test_a_step_forks_where_its_launches_outlast_the_host(width, rows, exact):
+    """Rows times the square of the width: a fork's events cost the host the same whatever the width."""
+    from types import SimpleNamespace
+    from vllm_i64_amd.hybrid_runner import HybridRunner
+    r = HybridRunner.__new__(HybridRunner)
+    r.cfg, r.exact, r.side = SimpleNamespace(width=width), exact, object()
+    assert not r._heavy(rows - 1) and r._heavy(rows) and r._forks(rows)
 
 
 @pytest.mark.parametrize("design", ["vepelix", "pukatar"])

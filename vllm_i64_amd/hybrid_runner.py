@@ -40,13 +40,18 @@ class HybridRunner:
         self.side = torch.cuda.Stream(device=self.device) if self.SIDE_STREAM and self.device.type == "cuda" else None
 
     # ---- two sublayers side by side ----
-    # Eager steps of little work (rows times width) are bound by the host, and the events of a fork and its meeting take 40 to 65 us of it.
-    # Microseconds a step, forked | not: width 1024, 77 rows 1120 | 797, 400 rows 1105 | 745, 700 rows 1088 | 1025, 32-bit 376 rows 1114 to 1300 | 1191;
-    # width 2048, 216 rows 959 | 828, 256 rows 1091 | 978, 512 rows 988 | 1163; 1024 x 4096 rows 3623 | 3893.
-    FORK_WORK = int(os.environ.get("I64H_FORK_WORK", "850000"))
+    # Eager steps of little work (rows times the square of the width, twice as much with 32-bit products) are bound by the host, and the events of a fork and its
+    # meeting take 40 to 65 us of it.  Microseconds a step of two blocks, forked | not, on a host that needs 1200 to 1300 for its launches: width 1024, Vepelix
+    # 600 rows 2200 | 1560, 1024 2300 | 1724, 1536 2354 | 2117, 2048 in four prompts 2450 | 2182, in one 2893 | 3074, 3072 2909 | 3005; Pukatar 1024 1696 | 1385, 1536 1784 |
+    # 1698, 2048 1700 | 1808, 2285 | 2440; width 2048, 200 rows 2160 | 1610 and 1673 | 1382, 400 2160 | 2178 and 1708 | 1840, 600 2436 | 2727 and 1770 | 2142; 32-bit
+    # (a block), width 1024, 600 rows 1478 | 1543 and 1197 | 1134, 1024 1716 | 1796 and 1271 | 1414.
+    FORK_WORK = int(os.environ.get("I64H_FORK_WORK", "1650000000"))
+
+    def _heavy(self, n: int) -> bool:
+        return n * self.cfg.width ** 2 * (2 if self.exact else 1) >= self.FORK_WORK
 
     def _forks(self, n: int) -> bool:
-        return self.side is not None and (n * self.cfg.width >= self.FORK_WORK or torch.cuda.is_current_stream_capturing())
+        return self.side is not None and (self._heavy(n) or torch.cuda.is_current_stream_capturing())
 
     @contextmanager
     def _beside(self, n: int):
@@ -416,7 +421,7 @@ class HybridRunner:
     def _joins(self, n: int) -> bool:
         """Whether a shared expert in its experts' stack joins their launches in a step of n rows, but where it can run beside the choice and the plan of much work (8
         prompts of 512, width 1024: 3572 us a step joined, 3432 beside; where the whole feed-forward runs beside a mixer joined is better, 5593 and 5804)."""
-        return not (self.MOE_BESIDE and self.side is not None and n * self.cfg.width >= self.FORK_WORK)
+        return not (self.MOE_BESIDE and self.side is not None and self._heavy(n))
 
     @staticmethod
     def _fills(pairs: int, experts: int) -> bool:
