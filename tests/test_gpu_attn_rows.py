@@ -250,3 +250,45 @@ def test_scores_of_minus_infinity_beside_a_value_that_is_no_number(dev, dtype):
     assert bool(got[-1, :, 7].isnan().all())
     tol = 1e-3 if dtype == torch.bfloat16 else 2e-5
     assert torch.allclose(got[:-1], ref, atol=2 * tol, rtol=tol), float((got[:-1] - ref).abs().max())
+
+
+# (one to seven tiles of 32 keys, a last one of one key and of all, several runs a tile of rows; the sizes whose tiles go from memory to LDS by themselves)
+TILES = [([1, 16, 31], [0, 15, 1]), ([2, 17, 5, 3], [30, 48, 91, 93]), ([40, 3], [88, 157]), ([7, 64], [0, 150])]
+
+
+@pytest.mark.parametrize("lens,past", TILES)
+@pytest.mark.parametrize("H,G,w,r,off", [(4, 1, 288, 256, 0), (3, 1, 288, 256, 0), (8, 2, 128, 64, 64), (2, 2, 128, 64, 64), (6, 3, 256, 128, 128), (4, 1, 256, 128, 128)])
+@pytest.mark.parametrize("block,window,keep", [(16, 0, 0), (5, 0, 0), (16, 45, 3), (12, 33, 40)])
+def test_rows_of_exact_sizes(dev, lens, past, H, G, w, r, off, block, window, keep):
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator().manual_seed(H + w + window)
+    bt, pos, slots, blocks = pages(lens, past, block, g)
+    n = int(pos.numel())
+    cache = torch.randn(blocks, block, G * w, generator=g).to(torch.bfloat16)
+    q = torch.randn(n, H, w, generator=g)
+    q[:, :, :off] = 0
+    sink = torch.randn(H, generator=g)
+    out = torch.full((n * H * r,), 7.0, device=dev)
+    args = (q.to(dev).flatten(), cache.to(dev), bt.to(dev), slots.to(dev), pos.to(dev))
+    if off:
+        D.kattn(args[0].view(n, -1), args[1], None, *args[2:], chunk=0, bias=None, sink=True, heads=H, kv_heads=G, dim=w - r, vdim=r, out=out.view(n, -1), n=n, mode=3, window=window,
+                keep_first=keep, sink_w=sink.to(dev))
+        scale = 1.0
+    else:
+        keep, scale = 0, 0.1
+        D.latent_attn(*args, window=window, scale=scale, heads=H, kv_rank=r, rot_dim=w - r, out=out, n=n, mode=3, sink=sink.to(dev))
+    at = 0
+    for i, (m, p) in enumerate(zip(lens, past)):
+        j = torch.arange(m + p)
+        rows = cache[bt[i].long()[j // block], j % block].view(m + p, G, w).repeat_interleave(H // G, 1).transpose(0, 1)
+        ref = reference(q[at:at + m, :, off:], rows[..., off:], rows[..., :r], pos[at:at + m], scale, window, keep, 0.0, sink)
+        got = out.view(n, H, r)[at:at + m].double().cpu()
+        tol = 1e-3      # two bf16 terms of query and weight: 2^-16 relative each, scores of up to sqrt(dim) * 4
+        assert torch.allclose(got, ref, atol=2 * tol, rtol=tol), float((got - ref).abs().max())
+        at += m
+
+
+@pytest.mark.parametrize("H,G,dim,vdim,window,keep", [(4, 1, 64, 64, 0, 0), (2, 1, 128, 128, 9, 2), (8, 2, 64, 64, 9, 2)])
+def test_unseen_values_in_rows_of_exact_sizes(dev, H, G, dim, vdim, window, keep):
+    for bad in (math.inf, -math.inf, math.nan):
+        unseen_values(dev, H, G, dim, vdim, window, keep, bad, torch.bfloat16, 1e-3)

@@ -12,6 +12,7 @@
 //                            cached row), online softmax over the wave, weighted row sum with the columns spread over the lanes
 #include "i64h_common.h"
 #include "i64h_dense.h"
+#include <type_traits>
 
 __device__ __forceinline__ float lt_load(const void* cache, int dtype, int64_t idx) {
     return dtype == 0 ? ((const float*)cache)[idx] : __uint_as_float((uint32_t)((const uint16_t*)cache)[idx] << 16);
@@ -167,6 +168,14 @@ __device__ __forceinline__ uint32_t lt_rne(float f) {  // nearest even: the hard
 __device__ __forceinline__ void lt_split(float x, uint32_t& hi, uint32_t& lo) {
     hi = lt_rne(x);
     lo = lt_rne(x - __uint_as_float(hi << 16));
+}
+
+// two of them, the first in the low halves: both conversions in one instruction
+__device__ __forceinline__ void lt_split_pair(float x, float y, uint32_t& hi, uint32_t& lo) {
+    typedef float v2f __attribute__((ext_vector_type(2)));
+    typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+    hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{x, y}), v2bf));
+    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{x - __uint_as_float(hi << 16), y - __uint_as_float(hi & 0xffff0000u)}), v2bf));
 }
 
 // Matrix-core form (bf16 cache) of rows that are one per sequence.  One wave per task of 16 query vectors that walk the same cached rows: the (up to) 16
@@ -476,6 +485,7 @@ __device__ __forceinline__ lt_run lt_run_at(int s0, const int* info, int wr) {
 //
 // Bound by LDS and its latency: per 32 keys of 256 + 32 values a workgroup reads 136 KiB of fragments for 68 matrix instructions a wave, and
 // the registers of two waves per SIMD leave few reads on their way (one wave per SIMD with all it wants: 194 us where two take 130).
+// (For rows of 288, 128 and 256 values and for launches without an option the kernel behind this one; figures of both:)
 // 8 prompts of 512 tokens, 16 heads over one cached row of 288: 304 -> 130 us against the form before (a wave per workgroup that read every
 // fragment from memory itself and transposed it two bytes at a time), 16 heads of 64 over 4 key heads 120 -> 43 us, 32 heads of 64 over 8 key heads
 // on prompts of 1531, 257, 64, 3 and 1101 tokens 285 -> 74 us, one prompt of 77 tokens 29 -> 19 and 17 -> 10 us.
@@ -712,6 +722,255 @@ __global__ __launch_bounds__(256, 2) void latent_attn_rows_kernel(const i64h_lat
             if (((uintptr_t)p.out & 15) == 0) *(float4*)dst = v;
             else dst[0] = v.x, dst[1] = v.y, dst[2] = v.z, dst[3] = v.w;
         }
+}
+
+// The same for rows of exactly D values, the first R of them value columns, keys from column KO on, without key scales, soft cap or bias.  A tile's rows go
+// from memory to LDS by themselves, 16 bytes a lane, two tiles ahead, and lie there once: score fragments are read as rows, value fragments transposed
+// (ds_read_b64_tr_b16).  The chunk of 16 bytes at place c of row i is chunk c ^ lt_swizzle(i): rows whose pitch is a multiple of the banks would meet in
+// the same ones.  The kernel above moves a tile through registers, 40 of which it holds for it, and writes the value columns a second time, transposed.
+// Bound by vector instructions and the chain barrier - scores - softmax - second product (heads of 64), by these, the fragments' way out of LDS and the
+// query and result rows (latent rows: 142 MB at 8 x 512, 30 us at a copy's rate).  Two heads a wave, which reads every fragment once for both: 31 us as
+// well for heads of 64, 113 for latent rows, whose 320 registers do not stay where the products take them.  Microseconds, the kernel above | this:
+//   16 heads over one row of 288: 8 prompts of 512 125 | 74, one of 77 19 | 12.5, 64 portions of 3 behind 500 69 | 41; 32 heads, 229 behind 512 83 | 43
+//   16 heads of 64 over 4: 8 x 512 44 | 31, one of 77 9.8 | 9.5; 32 over 8, prompts of 1531, 257, 64, 3, 1101 73 | 51; 24 heads of 128 over 8, 8 x 512 89 | 62
+template <int D>
+__device__ __forceinline__ int lt_swizzle(int row) {
+    if constexpr (D % 128 == 0) return (row & 7) << 1 | (row >> 3 & 1);      // every row starts in bank 0: sixteen places, neighbours in pairs
+    else return (row >> 1 & 2) | (row >> 3 & 1);                             // (rows a quarter of the banks apart: four places)
+}
+struct lt_place {      // a cached row: its page, its place in the page
+    int page, in;
+};
+template <int D, int R, int KO>
+__global__ __launch_bounds__(256, 2) void latent_attn_rows_direct_kernel(const i64h_latent_attn_args p, const int hw) {
+    static_assert(D % 32 == 0 && (D % 128 == 0 || D % 128 == 32) && R % 16 == 0 && KO % 32 == 0, "");
+    constexpr int KD = (D - KO) / 32, NB = R / 16, CH = D / 8, NL = CH / 2, LW = (NL + 3) / 4;      // chunks of a row, a tile's loads of 64 chunks, a wave's
+    __shared__ __attribute__((aligned(1024))) uint16_t s0[32 * D], s1[32 * D], s2[32 * D];
+    __shared__ int info[128];
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, kg = lane >> 4;
+    const int H = p.heads, bs = p.block_size, win = p.window;
+    const int keep = p.chunk <= 0 && win > 0 ? p.keep_first : 0;
+    const int G = p.kv_groups > 1 ? p.kv_groups : 1, rep = H / G;
+    const int rstride = p.row_stride > 0 ? p.row_stride : D;
+    const int hgroups = H / hw, rows = 16 * (4 / hw), row_tiles = (int)((p.n + rows - 1) / rows);
+    const int task = blockIdx.x, hg = task % hgroups, rt = row_tiles - 1 - task / hgroups;      // (the longest contexts first)
+    const int head = hg * hw + wid % hw, coff = hg * hw / rep * D, wr = wid / hw * 16;
+    const int64_t row0 = (int64_t)rt * rows;
+    const bool row_l = lane < rows && row0 + lane < p.n;
+    const int pos_l = row_l ? p.positions[row0 + lane] : -1, slot_l = row_l ? p.slot_ids[row0 + lane] : -1;
+    const uint64_t starts = lt_run_starts(slot_l);
+    if (blockIdx.y > 0 && (int)blockIdx.y >= __popcll(starts)) return;
+    info[lane] = pos_l, info[64 + lane] = slot_l;
+    __syncthreads();
+    bool mine = info[64 + wr + n] < 0 && blockIdx.y == 0;      // this workgroup's rows: those of its runs
+    const int64_t tok = row0 + wr + n;
+    const bool valid = tok < p.n;
+    // the query of row n times scale * log2(e) (the softmax runs on powers of two), columns KO + ks * 32 + kg * 8 .. + 7, as two bf16 terms
+    uint4 Qh[KD], Ql[KD];
+    {
+        const float* q = p.Q + ((valid ? tok : row0) * H + head) * D + KO + kg * 8;
+        const float qs = valid ? p.scale * 1.4426950408889634f : 0.0f;
+        float4 v[2 * KD];
+#pragma unroll
+        for (int i = 0; i < 2 * KD; ++i) v[i] = *(const float4*)(q + (i >> 1) * 32 + 4 * (i & 1));
+#pragma unroll
+        for (int ks = 0; ks < KD; ++ks) {
+            const float4 a = v[2 * ks], b = v[2 * ks + 1];
+            const float x[8] = {a.x * qs, a.y * qs, a.z * qs, a.w * qs, b.x * qs, b.y * qs, b.z * qs, b.w * qs};
+            uint32_t h[4], l[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) lt_split_pair(x[2 * i], x[2 * i + 1], h[i], l[i]);
+            Qh[ks] = make_uint4(h[0], h[1], h[2], h[3]);
+            Ql[ks] = make_uint4(l[0], l[1], l[2], l[3]);
+        }
+    }
+    lt_v4f acc[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[nb] = lt_v4f{0, 0, 0, 0};
+    // (the weight sum of a row is kept in four shares, one per group of keys: the sink belongs to one of them)
+    float m = p.sink ? (p.sink_w ? p.sink_w[head] * 1.4426950408889634f : 0.0f) : -INFINITY, l = p.sink && kg == 0 ? 1.0f : 0.0f;
+    const uint16_t* const cache = (const uint16_t*)p.cache + coff;
+    auto first_seen = [&](int pos) { return p.chunk > 0 ? pos / p.chunk * p.chunk : (win > 0 ? max(0, pos - win + 1) : 0); };
+    // this lane's chunk of a load of its wave: the key it belongs to and its first column (a wave without a last load of its own repeats the tile's)
+    int key_l[LW], col_l[LW];
+#pragma unroll
+    for (int i = 0; i < LW; ++i) {
+        const int at = min(i * 4 + wid, NL - 1) * 64 + lane;
+        key_l[i] = at / CH, col_l[i] = (at % CH ^ lt_swizzle<D>(at / CH)) * 8;
+    }
+    constexpr std::integral_constant<int, 0> S0{};
+    constexpr std::integral_constant<int, 1> S1{};
+    constexpr std::integral_constant<int, 2> S2{};
+    auto stage = [&](auto set) -> uint16_t* {      // (variables of their own: the compiler then knows which loads a read of one has to wait for)
+        constexpr int S = decltype(set)::value;
+        return S == 0 ? s0 : S == 1 ? s1 : s2;
+    };
+    const int krow = n * D, ksw = lt_swizzle<D>(n);
+    const int vrow = (4 * kg + (n >> 2)) * D + (n & 1) * 4, vsw = ((n & 3) >> 1) ^ lt_swizzle<D>(4 * kg + (n >> 2));
+    int turn = 0;
+    for (uint64_t left = starts; left; left &= left - 1) {
+        if ((turn++ & (gridDim.y - 1)) != blockIdx.y) continue;
+        const lt_run u = lt_run_at(__ffsll((unsigned long long)left) - 1, info, wr);
+        const bool in_run = wr + n >= u.s0 && wr + n < u.s1, whole = wr >= u.s0 && wr + 16 <= u.s1;      // (all of this wave's rows)
+        mine |= in_run;
+        const int pos = in_run ? info[wr + n] : -1, from = first_seen(max(pos, 0));
+        // the keys of the run; of this wave's rows of it: the first and the last one that any sees, from where to where all see every key
+        const int lo = first_seen(max(u.low, 0)), hi = u.high, wlo = first_seen(max(u.wlow, 0)), whi = u.whigh, wfrom = first_seen(max(whi, 0)), wall = whole ? u.wlow : -1;
+        const int32_t* bt = p.block_table + (int64_t)u.slot * p.max_blocks_per_seq;
+        // tiles of 32 keys: those of the kept first positions that lie in front of the window's first tile, then the window's
+        const int t0 = lo >> 5, kt = min((keep + 31) >> 5, t0), tiles = hi < 0 ? 0 : kt + (hi >> 5) - t0 + 1;
+        if (tiles == 0) continue;
+        auto key_base = [&](int tile) { return (tile < kt ? tile : t0 + tile - kt) * 32; };
+        // lane l < 32: the tile's key l
+        auto look_up = [&](int tile) {
+            const int j = min(key_base(min(tile, tiles - 1)) + (lane & 31), hi), pg = j / bs;
+            return lt_place{bt[pg], j - pg * bs};
+        };
+        auto load = [&](lt_place at, auto set) {
+            uint16_t* sm = stage(set);
+            const int row = at.page * bs + at.in;
+            int src[LW];
+#pragma unroll
+            for (int i = 0; i < LW; ++i) src[i] = __shfl(row, key_l[i]);
+#pragma unroll
+            for (int i = 0; i < LW; ++i)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(cache + (int64_t)src[i] * rstride + col_l[i]),
+                                                 (__attribute__((address_space(3))) void*)(sm + min(i * 4 + wid, NL - 1) * 512), 16, 0, 0);
+        };
+        // this wave's loads of the tile are in LDS, its reads of the one before done; then everybody's.  On their way: the loads of the next tile
+        lt_place next;      // of the tile after the next
+        auto meet = [&]() {
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0x0070 | (LW & 15));      // vmcnt LW, lgkmcnt 0
+            asm volatile("s_barrier" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto step = [&](int tile, auto cur, auto free) {
+            meet();
+            // (past the end the last tile again, which nobody reads: without a branch the loads on their way are the same everywhere)
+            const lt_place then = look_up(tile + 3);
+            load(next, free);
+            next = then;
+            const int kb = key_base(tile);
+            if (kb > whi || (kb + 31 < wlo && kb >= keep)) return;      // (nothing that a row of this wave sees)
+            const uint16_t* T = stage(cur);
+            lt_v4f S[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+            __builtin_amdgcn_sched_barrier(0);
+            lt_v8bf kf[KD][2];
+#pragma unroll
+            for (int ks = 0; ks < KD; ++ks)
+#pragma unroll
+                for (int b = 0; b < 2; ++b) kf[ks][b] = __builtin_bit_cast(lt_v8bf, *(const uint4*)&T[krow + 16 * b * D + ((KO / 8 + ks * 4 + kg) ^ ksw) * 8]);
+#pragma unroll
+            for (int ks = 0; ks < KD; ++ks) {
+#pragma unroll
+                for (int b = 0; b < 2; ++b) S[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks][b], __builtin_bit_cast(lt_v8bf, Qh[ks]), S[b], 0, 0, 0);
+#pragma unroll
+                for (int b = 0; b < 2; ++b) S[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks][b], __builtin_bit_cast(lt_v8bf, Ql[ks]), S[b], 0, 0, 0);
+            }
+            // four steps' fragments on their way
+            __builtin_amdgcn_sched_group_barrier(0x100, 2 * (KD < 4 ? KD : 4), 0);
+#pragma unroll
+            for (int ks = 0; ks < KD; ++ks) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+                if (ks + 4 < KD) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (kb + 31 > wall || kb < wfrom) {
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        const int j = kb + 16 * b + kg * 4 + g;
+                        S[b][g] = j <= pos && (j >= from || j < keep) ? S[b][g] : -INFINITY;
+                    }
+            }
+            float mx = fmaxf(fmaxf(fmaxf(S[0][0], S[0][1]), fmaxf(S[0][2], S[0][3])), fmaxf(fmaxf(S[1][0], S[1][1]), fmaxf(S[1][2], S[1][3])));
+            const PairF m1 = swap_rows(mx);
+            mx = fmaxf(m1.lo, m1.hi);
+            const PairF m2 = swap_halves(mx);
+            const float mn = fmaxf(m, fmaxf(m2.lo, m2.hi)), ms = mn == -INFINITY ? 0.0f : mn;
+            const float al = __builtin_amdgcn_exp2f(m - ms);
+            m = mn;
+            float w[2][4], sum = 0.0f;
+            uint32_t ph[4], pl[4];
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    w[b][g] = __builtin_amdgcn_exp2f(S[b][g] - ms);
+                    sum += w[b][g];
+                }
+#pragma unroll
+                for (int g = 0; g < 4; g += 2) lt_split_pair(w[b][g], w[b][g + 1], ph[b * 2 + g / 2], pl[b * 2 + g / 2]);
+            }
+            l = l * al + sum;
+            if (__ballot(al != 1.0f)) {
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) acc[nb][g] *= al;
+            }
+            const lt_v8bf Ph = __builtin_bit_cast(lt_v8bf, make_uint4(ph[0], ph[1], ph[2], ph[3])), Pl = __builtin_bit_cast(lt_v8bf, make_uint4(pl[0], pl[1], pl[2], pl[3]));
+            // V^T fragments: lane 4 q + c of 16 addresses key 4 kg + q (and 16 keys further), columns 16 nb + 4 c .. + 3, and receives its own column of four keys
+            __builtin_amdgcn_sched_barrier(0);
+            lt_v4s va[NB][2];
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                const uint16_t* vp = &T[vrow + ((2 * nb) ^ vsw) * 8];
+#pragma unroll
+                for (int b = 0; b < 2; ++b) va[nb][b] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) lt_v4s*)(vp + 16 * b * D));
+            }
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                const lt_v8bf vf = __builtin_bit_cast(lt_v8bf, __builtin_shufflevector(va[nb][0], va[nb][1], 0, 1, 2, 3, 4, 5, 6, 7));
+                acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, Ph, acc[nb], 0, 0, 0);
+                acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, Pl, acc[nb], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x100, 2 * (NB < 6 ? NB : 6), 0);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                if (nb + 6 < NB) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        __syncthreads();      // (the run before has been read)
+        const lt_place at0 = look_up(0), at1 = look_up(1);
+        next = look_up(2);
+        load(at0, S0);
+        load(at1, S1);
+        int tile = 0;
+        for (; tile + 3 <= tiles; tile += 3) {
+            step(tile, S0, S2);
+            step(tile + 1, S1, S0);
+            step(tile + 2, S2, S1);
+        }
+        if (tile < tiles) step(tile, S0, S2);
+        if (tile + 1 < tiles) step(tile + 1, S1, S0);
+        __builtin_amdgcn_s_waitcnt(0x0f70);      // (nothing is on its way into LDS when a run ends)
+    }
+    const PairF l1 = swap_rows(l), l2 = swap_halves(l1.lo + l1.hi);
+    bool nan = false;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) nan |= acc[nb][g] != acc[nb][g];
+    const uint64_t lanes = __ballot(valid && mine && nan);
+    const uint32_t by_key = (uint32_t)(lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) & 0xffffu;      // rows of this wave
+    for (uint32_t left = by_key; left; left &= left - 1) latent_row<uint16_t>(p, row0 + wr + __ffs((int)left) - 1, head);
+    if (!valid || !mine || (by_key >> n & 1)) return;
+    float* o = p.out + (tok * H + head) * R + kg * 4;
+    const float inv = 1.0f / (l2.lo + l2.hi);
+    if (((uintptr_t)p.out & 15) == 0) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) *(float4*)(o + nb * 16) = make_float4(acc[nb][0] * inv, acc[nb][1] * inv, acc[nb][2] * inv, acc[nb][3] * inv);
+    } else {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) o[nb * 16 + g] = acc[nb][g] * inv;
+    }
 }
 
 // The same for caches of 32-bit rows, with 32-bit products: keys and transposed values once in LDS (twice would be a workgroup per CU), the next tile
@@ -1092,7 +1351,12 @@ int i64h_latent_attn(const i64h_latent_attn_args* dp, void* stream) {
                 else hipLaunchKernelGGL((latent_attn_rows_kernel<KD, NB, false>), grid_rows, dim3(256), lds, st, d, hw); \
             } while (0)
             const int steps = (D - (d.key_off & ~31) + 31) / 32;
-            if (steps <= 2 && d.kv_rank <= 64) LT_ROWS(2, 4);
+            auto exact = [&](int width, int rank, int off) { return !extra && D == width && d.kv_rank == rank && d.key_off == off; };
+            auto direct = [&](auto kern) { hipLaunchKernelGGL(kern, grid_rows, dim3(256), 0, st, d, hw); };
+            if (exact(288, 256, 0)) direct(latent_attn_rows_direct_kernel<288, 256, 0>);                // a latent row of 256 + 32
+            else if (exact(128, 64, 64)) direct(latent_attn_rows_direct_kernel<128, 64, 64>);           // values and keys of 64
+            else if (exact(256, 128, 128)) direct(latent_attn_rows_direct_kernel<256, 128, 128>);       // ... of 128
+            else if (steps <= 2 && d.kv_rank <= 64) LT_ROWS(2, 4);
             else if (steps <= 4 && d.kv_rank <= 128) LT_ROWS(4, 8);
             else if (steps <= 9) LT_ROWS(9, LT_NB);
             else LT_ROWS(LT_KD, LT_NB);
