@@ -88,3 +88,43 @@ def test_rot_prep_forms(dev, H, G, dim, vdim, rot, turned, heads):
     one, two = run([(0, n)]), run([(0, 256), (256, n)])
     for a, b in zip(one, two):
         close(a, b.double().cpu(), 2e-6)
+
+
+@pytest.mark.parametrize("H,G,dim,vdim,rot,inter", [(3, 1, 64, 16, 64, True), (16, 4, 64, 64, 32, False), (33, 3, 128, 32, 8, False), (2, 2, 16, 256, 12, True), (1, 1, 256, 64, 0, False), (70, 10, 64, 64, 64, False)])
+@pytest.mark.parametrize("norm", ["", "heads", "behind"])
+@pytest.mark.parametrize("n,dtype", [(1, torch.bfloat16), (37, torch.float32)])
+def test_rot_prep_of_whole_heads(dev, H, G, dim, vdim, rot, inter, norm, n, dtype):
+    """Heads whose sizes are powers of two: against the same in 64 bits, and against rows at an offset that only four-byte loads can read."""
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator().manual_seed(H * dim + rot)
+    W = (H + G) * dim + G * vdim
+    P, pos = torch.randn(n, W, generator=g), torch.randint(0, 32, (n,), generator=g, dtype=torch.int32)
+    sl, bt = torch.arange(n, dtype=torch.int32), torch.randperm(2 * n, generator=g).to(torch.int32).view(n, 2)
+    w1, w2, fr, mult = torch.rand(dim, generator=g), torch.rand(dim, generator=g), torch.rand(max(rot // 2, 1), generator=g), 1.1
+    def run(shift):
+        buf = torch.zeros(n, W + 4, device=dev)
+        buf[:, shift:shift + W] = P.to(dev)
+        cache, q = torch.zeros(2 * n, 16, G * (vdim + dim), device=dev, dtype=dtype), torch.empty(n, H * (vdim + dim), device=dev)
+        D.rot_prep(buf, q_off=shift, k_off=shift + H * dim, v_off=shift + (H + G) * dim, heads=H, kv_heads=G, dim=dim, vdim=vdim, q_norm_w=w1.to(dev) if norm == "heads" else None,
+                   k_norm_w=w2.to(dev) if norm == "heads" else None, eps=1e-6, rot_dims=rot, interleaved=inter, inv_freq=fr.to(dev), rot_mult=mult, head_norm=norm == "behind", v_freq=None,
+                   scale=0.25, positions=pos.to(dev), slot_ids=sl.to(dev), block_table=bt.to(dev), cache=cache, q=q, n=n, norm_heads=norm == "heads")
+        return q.view(n, H, vdim + dim), cache[bt.to(dev).long()[torch.arange(n), pos.long() // 16], pos.long() % 16].view(n, G, vdim + dim)
+    def turned(x, w):
+        if norm == "heads":
+            x = x / torch.sqrt(x.pow(2).mean(-1, keepdim=True) + 1e-6) * w.double()
+        if rot:
+            a = (pos.float()[:, None] * fr).double()[:, None, :]      # (the kernel's angle is a 32-bit product)
+            c, s, r = a.cos() * mult, a.sin() * mult, x[..., :rot]
+            u, v = (r[..., 0::2], r[..., 1::2]) if inter else r.chunk(2, -1)
+            p1, p2 = u * c - v * s, v * c + u * s
+            x = torch.cat([torch.stack([p1, p2], -1).flatten(-2) if inter else torch.cat([p1, p2], -1), x[..., rot:]], -1)
+        if norm == "behind":
+            x = x / torch.sqrt(x.pow(2).mean(-1, keepdim=True) + 1e-6)
+        return x
+    x = P.double()
+    q, k, v = x[:, :H * dim].view(n, H, dim), x[:, H * dim:(H + G) * dim].view(n, G, dim), x[:, (H + G) * dim:].view(n, G, vdim)
+    want = [torch.cat([torch.zeros(n, H, vdim).double(), 0.25 * turned(q, w1)], -1), torch.cat([v, turned(k, w2)], -1)]
+    tol = 1e-5      # values of order one through about ten 32-bit operations, sines and cosines of angles to 32
+    for a, b, c, t in zip(run(0), run(1), want, (tol, tol if dtype == torch.float32 else 2.0 ** -8)):
+        assert torch.allclose(a.double().cpu(), c, atol=t * (4 if t > tol else 1), rtol=t), float((a.double().cpu() - c).abs().max())
+        assert torch.allclose(a.float(), b.float(), atol=t * (4 if t > tol else 1), rtol=t)

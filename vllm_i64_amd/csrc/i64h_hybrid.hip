@@ -827,6 +827,104 @@ __global__ __launch_bounds__(NT) void rot_prep_kernel(const i64h_rot_prep_args p
     }
 }
 
+// The same where every head's dim and vdim are powers of two from 16 to 256, rows are read and written 16 bytes at a time, no norm is over a whole row and
+// values are not rotated: a lane holds four neighbouring values of a head in registers from the projection row to where they go, a head's lanes
+// (dim / 4, neighbours in one wave) sum its squares and hand each other the other half of a pair.  Only the angles are in LDS.  The kernel above sends
+// every value through LDS three times, four bytes at a time; this one is bound by the rows (32 + 8 heads of 64 + 64: 30 KB a token, 4.6 TB/s at 4096).
+// Microseconds in replayed graphs, the kernel above (sixteen waves up to 256 rows) | this: 16 + 4 heads of 64 + 64, interleaved, normed per head: 1 row 5.0 | 3.8,
+// 64 5.3 | 4.1, 256 5.7 | 4.3, 300 8.8 | 4.6, 1024 11.7 | 6.0, 4096 31 | 14; 32 + 8 heads, halves: 7 rows 5.2 | 3.8, 2956 31 | 15; 24 + 8 heads of 128 + 128: 4096 51 | 28.
+// lsh, vsh: log2 of dim / 4 and of vdim / 4.
+template <int NT>
+__global__ __launch_bounds__(NT) void rot_prep_heads_kernel(const i64h_rot_prep_args p, const int lsh, const int vsh) {
+    extern __shared__ float ang[];      // [half] cosines, [half] sines: every head turns by the same angles
+    const int tid = threadIdx.x, lane = tid & 63, L = 1 << lsh;
+    const int64_t t = blockIdx.x;
+    const int dim = 4 << lsh, vd = 4 << vsh, gs = vd + dim, half = p.rot_dims >> 1;
+    const int nq = p.heads << lsh, items = (p.heads + p.kv_heads) << lsh, nv = p.kv_heads << vsh, nz = p.heads << vsh;
+    const float* row = p.P + t * p.ldp;
+    constexpr int U = 4;
+    float4 x[U];
+    auto load = [&](int base) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = base + u * NT + tid;
+            x[u] = i < items ? *(const float4*)(row + (i < nq ? p.q_off + 4 * i : p.k_off + 4 * (i - nq))) : make_float4(0, 0, 0, 0);
+        }
+    };
+    load(0);
+    float4 v = tid < nv ? *(const float4*)(row + p.v_off + 4 * tid) : make_float4(0, 0, 0, 0);
+    const int pos = p.positions[t];
+    const int64_t cr = cache_row(p.block_table, p.max_blocks_per_seq, p.block_size, p.slot_ids[t], pos) * p.kv_heads * gs;
+    for (int i = NT - 1 - tid; i < half; i += NT) {      // (the last waves have least of the row)
+        float sn, cs;
+        sincosf((float)pos * p.inv_freq[i], &sn, &cs);
+        ang[i] = cs * p.rot_mult, ang[half + i] = sn * p.rot_mult;
+    }
+    float* Q = p.Q + t * p.heads * gs;
+    auto cached = [&](int at, const float4& o) {
+        if (p.cache_dtype == 0) *(float4*)((float*)p.cache + cr + at) = o;
+        else *(uint2*)((__bf16*)p.cache + cr + at) = make_uint2(dn_bf16_pair(o.x, o.y), dn_bf16_pair(o.z, o.w));
+    };
+    for (int j = tid; j < nz; j += NT) *(float4*)(Q + (j >> vsh) * gs + (j & ((1 << vsh) - 1)) * 4) = make_float4(0, 0, 0, 0);
+    for (int j = tid; j < nv; j += NT) {
+        if (j >= NT) v = *(const float4*)(row + p.v_off + 4 * j);
+        cached((j >> vsh) * gs + (j & ((1 << vsh) - 1)) * 4, v);
+    }
+    __syncthreads();
+    for (int base = 0; base < items; base += U * NT) {
+        if (base > 0) load(base);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = base + u * NT + tid;
+            if (i >= items) continue;      // (whole heads: a head's lanes go together)
+            const int h = i >> lsh, l = i & (L - 1), e = 4 * l;
+            const bool isq = i < nq, turns = e < p.rot_dims;
+            float a[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
+            float inv = 1.0f;
+            if (p.head_norm || p.norm_heads) {
+                const float m2 = !p.norm_heads && turns ? p.rot_mult * p.rot_mult : 1.0f;
+                float s = (a[0] * a[0] + a[1] * a[1] + a[2] * a[2] + a[3] * a[3]) * m2;
+                for (int o = 1; o < L; o <<= 1) s += __shfl_xor(s, o);
+                inv = 1.0f / sqrtf(s / (float)dim + p.eps);
+            }
+            if (p.norm_heads) {
+                const float4 w = *(const float4*)((isq ? p.q_norm_w : p.k_norm_w) + e);
+                a[0] = a[0] * inv * w.x, a[1] = a[1] * inv * w.y, a[2] = a[2] * inv * w.z, a[3] = a[3] * inv * w.w;
+            }
+            if (p.interleaved) {
+                if (turns) {
+                    const float2 cs = *(const float2*)(ang + (e >> 1)), sn = make_float2(ang[half + (e >> 1)], ang[half + (e >> 1) + 1]);
+                    const float b[4] = {a[0] * cs.x - a[1] * sn.x, a[1] * cs.x + a[0] * sn.x, a[2] * cs.y - a[3] * sn.y, a[3] * cs.y + a[2] * sn.y};
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) a[c] = b[c];
+                }
+            } else if (half > 0) {
+                const int h4 = half >> 2;
+                const bool second = l >= h4;
+                const int from = turns ? (second ? lane - h4 : lane + h4) : lane, at = second ? e - half : e;
+                float b[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) b[c] = __shfl(a[c], from);
+                if (turns)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        const float cs = ang[at + c], sn = ang[half + at + c];
+                        a[c] = second ? a[c] * cs + b[c] * sn : a[c] * cs - b[c] * sn;
+                    }
+            }
+            if (p.head_norm || isq) {
+                const float hn = (p.head_norm ? inv : 1.0f) * (isq ? p.scale : 1.0f);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) a[c] *= hn;
+            }
+            const float4 o = make_float4(a[0], a[1], a[2], a[3]);
+            if (isq) *(float4*)(Q + h * gs + vd + e) = o;
+            else cached((h - p.heads) * gs + vd + e, o);
+        }
+    }
+}
+static int hy_log2_quads(int v) { return v >= 16 && v <= 256 && (v & (v - 1)) == 0 ? __builtin_ctz((unsigned)v) - 2 : -1; }
+
 // the attention output of every head turned back by the row's own position and multiplied by the head's sigmoid gate, in place:
 // a thread takes whole pairs
 __global__ __launch_bounds__(256) void rot_post_kernel(const i64h_rot_post_args p) {
@@ -1094,7 +1192,12 @@ int i64h_rot_prep(const i64h_rot_prep_args* dp, void* stream) {
     const size_t lds = ((size_t)(d.heads + d.kv_heads) * (d.dim + 1) + 8 + d.rot_dims + (d.v_freq ? d.vdim : 0)) * 4;
     I64H_CHECK_ARG(lds <= 64 * 1024, "rot_prep: %d + %d heads of %d values do not fit the kernel's LDS buffer", d.heads, d.kv_heads, d.dim);
     if (d.n == 0) return 0;
-    if (d.n <= HY_WIDE_ROWS && lds + 24 * 4 <= 64 * 1024)
+    const int lsh = hy_log2_quads(d.dim), vsh = hy_log2_quads(d.vdim);
+    const bool quads = ((uintptr_t)d.P | (uintptr_t)d.Q | (uintptr_t)d.cache | (d.norm_heads ? (uintptr_t)d.q_norm_w | (uintptr_t)d.k_norm_w : 0)) % 16 == 0 && d.ldp % 4 == 0 &&
+                       d.q_off % 4 == 0 && d.k_off % 4 == 0 && d.v_off % 4 == 0 && d.rot_dims % (d.interleaved ? 4 : 8) == 0;
+    if (quads && lsh >= 0 && vsh >= 0 && !d.v_freq && (!d.q_norm_w || d.norm_heads))
+        hipLaunchKernelGGL(rot_prep_heads_kernel<256>, dim3((unsigned)d.n), dim3(256), (size_t)d.rot_dims * 4, (hipStream_t)stream, d, lsh, vsh);
+    else if (d.n <= HY_WIDE_ROWS && lds + 24 * 4 <= 64 * 1024)
         hipLaunchKernelGGL(rot_prep_kernel<1024>, dim3((unsigned)d.n), dim3(1024), lds + 24 * 4, (hipStream_t)stream, d);
     else
         hipLaunchKernelGGL(rot_prep_kernel<256>, dim3((unsigned)d.n), dim3(256), lds, (hipStream_t)stream, d);
