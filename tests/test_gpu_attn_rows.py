@@ -259,12 +259,13 @@ TILES = [([1, 16, 31], [0, 15, 1]), ([2, 17, 5, 3], [30, 48, 91, 93]), ([40, 3],
 @pytest.mark.parametrize("lens,past", TILES)
 @pytest.mark.parametrize("H,G,w,r,off", [(4, 1, 288, 256, 0), (3, 1, 288, 256, 0), (8, 2, 128, 64, 64), (2, 2, 128, 64, 64), (6, 3, 256, 128, 128), (4, 1, 256, 128, 128)])
 @pytest.mark.parametrize("block,window,keep", [(16, 0, 0), (5, 0, 0), (16, 45, 3), (12, 33, 40)])
-def test_rows_of_exact_sizes(dev, lens, past, H, G, w, r, off, block, window, keep):
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rows_of_exact_sizes(dev, lens, past, H, G, w, r, off, block, window, keep, dtype):
     from vllm_i64_amd import ops_dense as D
     g = torch.Generator().manual_seed(H + w + window)
     bt, pos, slots, blocks = pages(lens, past, block, g)
     n = int(pos.numel())
-    cache = torch.randn(blocks, block, G * w, generator=g).to(torch.bfloat16)
+    cache = torch.randn(blocks, block, G * w, generator=g).to(dtype)
     q = torch.randn(n, H, w, generator=g)
     q[:, :, :off] = 0
     sink = torch.randn(H, generator=g)
@@ -283,12 +284,32 @@ def test_rows_of_exact_sizes(dev, lens, past, H, G, w, r, off, block, window, ke
         rows = cache[bt[i].long()[j // block], j % block].view(m + p, G, w).repeat_interleave(H // G, 1).transpose(0, 1)
         ref = reference(q[at:at + m, :, off:], rows[..., off:], rows[..., :r], pos[at:at + m], scale, window, keep, 0.0, sink)
         got = out.view(n, H, r)[at:at + m].double().cpu()
-        tol = 1e-3      # two bf16 terms of query and weight: 2^-16 relative each, scores of up to sqrt(dim) * 4
+        # two bf16 terms of query and weight: 2^-16 relative each, scores of up to sqrt(dim) * 4; 32-bit products: 2^-24 times the score
+        tol = 1e-3 if dtype == torch.bfloat16 else 2e-5
         assert torch.allclose(got, ref, atol=2 * tol, rtol=tol), float((got - ref).abs().max())
         at += m
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("H,G,dim,vdim,window,keep", [(4, 1, 64, 64, 0, 0), (2, 1, 128, 128, 9, 2), (8, 2, 64, 64, 9, 2)])
-def test_unseen_values_in_rows_of_exact_sizes(dev, H, G, dim, vdim, window, keep):
+def test_unseen_values_in_rows_of_exact_sizes(dev, H, G, dim, vdim, window, keep, dtype):
     for bad in (math.inf, -math.inf, math.nan):
-        unseen_values(dev, H, G, dim, vdim, window, keep, bad, torch.bfloat16, 1e-3)
+        unseen_values(dev, H, G, dim, vdim, window, keep, bad, dtype, 1e-3 if dtype == torch.bfloat16 else 2e-5)
+
+
+def test_many_32_bit_rows_of_exact_sizes(dev):
+    """Enough workgroups for the form that gives each wave its own rows: 1700 rows of 16 heads over 4, the same rows in one launch and in portions."""
+    from vllm_i64_amd import ops_dense as D
+    H, G, w, n = 16, 4, 128, 1700
+    g = torch.Generator().manual_seed(3)
+    bt, pos, slots, blocks = pages([n], [0], 16, g)
+    args = [torch.randn(n, H * w, generator=g).to(dev), torch.randn(blocks, 16, G * w, generator=g).to(dev)]
+    args[0].view(n, H, w)[:, :, :64] = 0
+    def run(cuts):
+        out = torch.empty(n, H * 64, device=dev)
+        for a, b in cuts:
+            D.kattn(args[0][a:b], args[1], None, bt.to(dev), slots[a:b].to(dev), pos[a:b].to(dev), chunk=0, bias=None, sink=False, heads=H, kv_heads=G, dim=64, vdim=64, out=out[a:b],
+                    n=b - a, mode=3, window=100, keep_first=2)
+        return out
+    one, cut = run([(0, n)]), run([(0, 700), (700, 1501), (1501, n)])
+    assert torch.allclose(one, cut, atol=4e-5, rtol=2e-5), float((one - cut).abs().max())

@@ -1193,6 +1193,210 @@ __global__ __launch_bounds__(256, NB > 8 ? 1 : 2) void latent_attn_rows_f32_kern
         }
 }
 
+// The same for rows of exactly D values without an option (as latent_attn_rows_direct_kernel), in launches whose workgroups of four heads would leave CUs
+// without work: a workgroup takes 16 rows of ONE head, its four waves share every tile's products.  A wave multiplies its quarter of the key columns,
+// the waves hand each other the sums through LDS, and each takes its quarter of the value columns: a tile's chain of matrix instructions is a quarter as
+// long.  The tile lies in LDS once, as its rows come from memory (the 32-bit products take single values, so no order of them has to be turned), the next
+// one on its way into the other buffer; exactly half of a CU's LDS for latent rows.  Bound by that chain in short launches (a tile 1.6 us where it was 4), by the
+// matrix instructions at their 32-bit rate in long ones.  Microseconds, the kernel above | this:
+//   16 heads over one row of 288: 16 rows 18 | 10, 77 33 | 14, 300 85 | 35, 600 153 | 67, 2000 509 | 456, 8 x 512 391 | 286
+//   heads of 64, 16 over 4: 16 rows 8.8 | 9.1, 77 12.5 | 9.4, 300 30 | 17, 1000 86 | 52, 2000 106 | 110, 4000 198 | 242; 32 over 8: 1000 98 | 77, 2000 160 | 213;
+//   16 over 16, windows of 128: 300 23 | 13.5, 1000 22.9 | 21.7, 2000 30 | 37; heads of 128, 24 over 8: 300 49 | 24, 1000 157 | 109, 2000 285 | 305
+template <int D, int R, int KO>
+__global__ __launch_bounds__(256, 2) void latent_attn_rows_f32_quarters_kernel(const i64h_latent_attn_args p) {
+    constexpr int KC = (D - KO) / 16, CW = (KC + 3) / 4, NBW = R / 64, CH = D / 4, LW = CH / 8;      // 16-column steps, a wave's of them and its column blocks; chunks of a row, a wave's loads
+    static_assert(D % 32 == 0 && R % 64 == 0 && KO % 16 == 0 && (D % 64 == 0 || D % 64 == 32), "");
+    __shared__ __attribute__((aligned(1024))) float s0[32 * D], s1[32 * D];
+    __shared__ __attribute__((aligned(16))) float ex[4 * 2 * 64 * 4];
+    int* const info = (int*)ex;
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, kg = lane >> 4;
+    const int H = p.heads, bs = p.block_size, win = p.window;
+    const int keep = p.chunk <= 0 && win > 0 ? p.keep_first : 0;
+    const int G = p.kv_groups > 1 ? p.kv_groups : 1, rep = H / G;
+    const int rstride = p.row_stride > 0 ? p.row_stride : D;
+    const int row_tiles = (int)((p.n + 15) / 16), task = blockIdx.x, head = task % H, rt = row_tiles - 1 - task / H;      // (the longest contexts first)
+    const int64_t row0 = (int64_t)rt * 16;
+    const bool row_l = lane < 16 && row0 + lane < p.n;
+    const int pos_l = row_l ? p.positions[row0 + lane] : -1, slot_l = row_l ? p.slot_ids[row0 + lane] : -1;
+    const uint64_t starts = lt_run_starts(slot_l);
+    if (blockIdx.y > 0 && (int)blockIdx.y >= __popcll(starts)) return;
+    bool mine = __shfl(slot_l, n) < 0 && blockIdx.y == 0;      // this workgroup's rows: those of its runs
+    const int64_t tok = row0 + n;
+    const bool valid = tok < p.n;
+    // (key place c of a row lies at c ^ swizzle: rows a multiple of the banks apart would meet in the same ones)
+    auto swizzle = [](int row) { return D % 64 == 0 ? row & 15 : row >> 1 & 7; };
+    // the query of row n times scale * log2(e), this wave's steps: columns KO + (4 i + wid) * 16 + kg * 4 .. + 3
+    lt_v4f Q[CW];
+    {
+        const float* q = p.Q + ((valid ? tok : row0) * H + head) * D + KO + kg * 4;
+        const float qs = valid ? p.scale * 1.4426950408889634f : 0.0f;
+#pragma unroll
+        for (int i = 0; i < CW; ++i) Q[i] = *(const lt_v4f*)(q + min(4 * i + wid, KC - 1) * 16) * (4 * i + wid < KC ? qs : 0.0f);
+    }
+    lt_v4f acc[NBW];
+#pragma unroll
+    for (int i = 0; i < NBW; ++i) acc[i] = lt_v4f{0, 0, 0, 0};
+    // (the weight sum of a row is kept in four shares, one per group of keys: the sink belongs to one of them)
+    float m = p.sink ? (p.sink_w ? p.sink_w[head] * 1.4426950408889634f : 0.0f) : -INFINITY, l = p.sink && kg == 0 ? 1.0f : 0.0f;
+    const float* const cache = (const float*)p.cache + head / rep * D;
+    auto first_seen = [&](int pos) { return p.chunk > 0 ? pos / p.chunk * p.chunk : (win > 0 ? max(0, pos - win + 1) : 0); };
+    int key_l[LW], col_l[LW];      // this lane's chunk of a load of its wave
+#pragma unroll
+    for (int i = 0; i < LW; ++i) {
+        const int at = (i * 4 + wid) * 64 + lane;
+        key_l[i] = at / CH, col_l[i] = (at % CH ^ swizzle(at / CH)) * 4;
+    }
+    constexpr std::integral_constant<int, 0> S0{};
+    constexpr std::integral_constant<int, 1> S1{};
+    auto stage = [&](auto set) -> float* { return decltype(set)::value == 0 ? s0 : s1; };      // (variables of their own: see above)
+    const int krow = n * D, ksw = swizzle(n);
+    int turn = 0;
+    for (uint64_t left = starts; left; left &= left - 1) {
+        if ((turn++ & (gridDim.y - 1)) != blockIdx.y) continue;
+        __syncthreads();      // (the run before has been read)
+        info[lane] = pos_l, info[64 + lane] = slot_l;
+        __syncthreads();
+        const lt_run u = lt_run_at(__ffsll((unsigned long long)left) - 1, info, 0);
+        __syncthreads();
+        const bool in_run = n >= u.s0 && n < u.s1;
+        mine |= in_run;
+        const int pos = in_run ? __shfl(pos_l, n) : -1, from = first_seen(max(pos, 0));
+        // the keys of the run; from where to where all rows see every key
+        const int lo = first_seen(max(u.low, 0)), hi = u.high, wfrom = first_seen(max(hi, 0)), wall = u.s0 == 0 && u.s1 >= 16 ? u.low : -1;
+        const int32_t* bt = p.block_table + (int64_t)u.slot * p.max_blocks_per_seq;
+        // tiles of 32 keys: those of the kept first positions that lie in front of the window's first tile, then the window's
+        const int t0 = lo >> 5, kt = min((keep + 31) >> 5, t0), tiles = hi < 0 ? 0 : kt + (hi >> 5) - t0 + 1;
+        if (tiles == 0) continue;
+        auto key_base = [&](int tile) { return (tile < kt ? tile : t0 + tile - kt) * 32; };
+        // lane l < 32: the tile's key l
+        auto look_up = [&](int tile) {
+            const int j = min(key_base(min(tile, tiles - 1)) + (lane & 31), hi), pg = j / bs;
+            return lt_place{bt[pg], j - pg * bs};
+        };
+        auto load = [&](lt_place at, auto set) {
+            float* sm = stage(set);
+            const int row = at.page * bs + at.in;
+            int src[LW];
+#pragma unroll
+            for (int i = 0; i < LW; ++i) src[i] = __shfl(row, key_l[i]);
+#pragma unroll
+            for (int i = 0; i < LW; ++i)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(cache + (int64_t)src[i] * rstride + col_l[i]),
+                                                 (__attribute__((address_space(3))) void*)(sm + (i * 4 + wid) * 256), 16, 0, 0);
+        };
+        lt_place next;
+        auto step = [&](int tile, auto cur, auto other) {
+            // this wave's loads of the tile are in LDS, its reads of the one before done; then everybody's
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0x0070);
+            asm volatile("s_barrier" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            const lt_place then = look_up(tile + 2);
+            load(next, other);      // (past the end the last tile again, which nobody reads)
+            next = then;
+            const int kb = key_base(tile);
+            const float* T = stage(cur);
+            lt_v4f S[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+            for (int i = 0; i < CW; ++i) {
+                lt_v4f kf[2];
+#pragma unroll
+                for (int b = 0; b < 2; ++b) kf[b] = *(const lt_v4f*)&T[krow + 16 * b * D + ((KO / 4 + min(4 * i + wid, KC - 1) * 4 + kg) ^ ksw) * 4];
+                if (KC % 4 == 0 || 4 * i + wid < KC)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)      // (a lane's four neighbouring columns go to four products)
+#pragma unroll
+                        for (int b = 0; b < 2; ++b) S[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[b][g], Q[i][g], S[b], 0, 0, 0);
+            }
+#pragma unroll
+            for (int b = 0; b < 2; ++b) *(lt_v4f*)&ex[((wid * 2 + b) * 64 + lane) * 4] = S[b];
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt 0; the next tile's loads stay on their way
+            asm volatile("s_barrier" ::: "memory");
+            {
+                lt_v4f part[4][2];
+#pragma unroll
+                for (int w = 0; w < 4; ++w)
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) part[w][b] = *(const lt_v4f*)&ex[((w * 2 + b) * 64 + lane) * 4];
+#pragma unroll
+                for (int b = 0; b < 2; ++b) S[b] = (part[0][b] + part[1][b]) + (part[2][b] + part[3][b]);
+            }
+            if (kb + 31 > wall || kb < wfrom) {
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        const int j = kb + 16 * b + kg * 4 + g;
+                        S[b][g] = j <= pos && (j >= from || j < keep) ? S[b][g] : -INFINITY;
+                    }
+            }
+            float mx = fmaxf(fmaxf(fmaxf(S[0][0], S[0][1]), fmaxf(S[0][2], S[0][3])), fmaxf(fmaxf(S[1][0], S[1][1]), fmaxf(S[1][2], S[1][3])));
+            const PairF m1 = swap_rows(mx);
+            mx = fmaxf(m1.lo, m1.hi);
+            const PairF m2 = swap_halves(mx);
+            const float mn = fmaxf(m, fmaxf(m2.lo, m2.hi)), ms = mn == -INFINITY ? 0.0f : mn;
+            const float al = exp2f(m - ms);
+            m = mn;
+            float w[2][4], sum = 0.0f;
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    w[b][g] = exp2f(S[b][g] - ms);
+                    sum += w[b][g];
+                }
+            l = l * al + sum;
+#pragma unroll
+            for (int i = 0; i < NBW; ++i) acc[i] *= al;
+            // a value fragment's lane holds column n of key 4 kg + g, the order that the weights lie in
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+#pragma unroll
+                    for (int i = 0; i < NBW; ++i) {
+                        const int key = 4 * kg + g;
+                        const float vf = T[(16 * b + key) * D + (((wid * NBW + i) * 4 + (n >> 2)) ^ swizzle(key)) * 4 + (n & 3)];
+                        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf, w[b][g], acc[i], 0, 0, 0);
+                    }
+        };
+        const lt_place at0 = look_up(0);
+        next = look_up(1);
+        load(at0, S0);
+        int tile = 0;
+        for (; tile + 2 <= tiles; tile += 2) {
+            step(tile, S0, S1);
+            step(tile + 1, S1, S0);
+        }
+        if (tile < tiles) step(tile, S0, S1);
+        __builtin_amdgcn_s_waitcnt(0x0f70);      // (nothing is on its way into LDS when a run ends)
+    }
+    const PairF l1 = swap_rows(l), l2 = swap_halves(l1.lo + l1.hi);
+    bool nan = false;
+#pragma unroll
+    for (int i = 0; i < NBW; ++i)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) nan |= acc[i][g] != acc[i][g];
+    // a value that is no finite number under a weight of zero: such rows key by key, each the keys that it sees (any wave's columns speak for the row)
+    const uint64_t lanes = __ballot(valid && mine && nan);
+    __syncthreads();
+    if (lane == 0) info[wid] = (int)((uint32_t)(lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) & 0xffffu);
+    __syncthreads();
+    const uint32_t by_key = (uint32_t)(info[0] | info[1] | info[2] | info[3]);
+    for (uint32_t left = by_key, k = 0; left; left &= left - 1, ++k)
+        if ((int)(k & 3) == wid) latent_row<float>(p, row0 + __ffs((int)left) - 1, head);
+    if (!valid || !mine || (by_key >> n & 1)) return;
+    float* o = p.out + (tok * H + head) * R + wid * NBW * 16 + kg * 4;
+    const float inv = 1.0f / (l2.lo + l2.hi);
+#pragma unroll
+    for (int i = 0; i < NBW; ++i) {
+        const float4 v = make_float4(acc[i][0] * inv, acc[i][1] * inv, acc[i][2] * inv, acc[i][3] * inv);
+        if (((uintptr_t)p.out & 15) == 0) *(float4*)(o + i * 16) = v;
+        else o[i * 16] = v.x, o[i * 16 + 1] = v.y, o[i * 16 + 2] = v.z, o[i * 16 + 3] = v.w;
+    }
+}
+
 // the shares of a token's keys, merged: one wave per (token, head); lane s holds share s's maximum and weight sum (at most 64
 // shares), then every lane sums its columns over the shares, eight loads in flight at a time
 template <int NC>      // columns a lane takes at a time: kv_rank <= 64, 128 or more
@@ -1273,11 +1477,22 @@ int latent_rows_f32_run(const i64h_latent_attn_args& d, void* stream) {
     const int kcols = D - (d.key_off & ~15), chunks = (kcols + 15) / 16;
     const size_t bytes = ((size_t)32 * (kcols + 4) + (size_t)d.kv_rank * LT_FLD) * 4 + 129 * 4;
     const bool extra = d.kscale || d.bias || d.softcap > 0.0f;
+    auto exact = [&](int width, int rank, int off) { return !extra && D == width && d.kv_rank == rank && d.key_off == off; };
+    // quarters: for latent rows always (they were faster in every launch timed), for heads of 64 and 128 while the workgroups of four waves on their own
+    // rows would be fewer than about 400 (256 CUs, two or more a CU): the figures beside the kernel
+    const int64_t wgs = (d.n + 15) / 16 * d.heads;
+    int shares = 4;
+    while (shares < 16 && wgs * shares < 2048) shares *= 2;
+    while (shares > d.n) shares /= 2;
+    auto quarters = [&](auto kern) { hipLaunchKernelGGL(kern, dim3((unsigned)wgs, (unsigned)shares), dim3(256), 0, (hipStream_t)stream, d); };
 #define LT_ROWS(KC, NB) do { \
         if (extra) hipLaunchKernelGGL((latent_attn_rows_f32_kernel<KC, NB, true>), grid, dim3(256), bytes, (hipStream_t)stream, d, hw); \
         else hipLaunchKernelGGL((latent_attn_rows_f32_kernel<KC, NB, false>), grid, dim3(256), bytes, (hipStream_t)stream, d, hw); \
     } while (0)
-    if (chunks <= 4 && d.kv_rank <= 64) LT_ROWS(4, 4);
+    if (exact(288, 256, 0)) quarters(latent_attn_rows_f32_quarters_kernel<288, 256, 0>);
+    else if (grid.x <= 400 && exact(128, 64, 64)) quarters(latent_attn_rows_f32_quarters_kernel<128, 64, 64>);
+    else if (grid.x <= 400 && exact(256, 128, 128)) quarters(latent_attn_rows_f32_quarters_kernel<256, 128, 128>);
+    else if (chunks <= 4 && d.kv_rank <= 64) LT_ROWS(4, 4);
     else if (chunks <= 8 && d.kv_rank <= 128) LT_ROWS(8, 8);
     else if (chunks <= 18) LT_ROWS(18, 16);
     else LT_ROWS(20, 16);
