@@ -726,7 +726,7 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
         rows = min(BMR, p.M_total - row0);
         if (rows <= 0) return;
     } else {
-        if (wid == 0) locate_mtile<BMR>(p, mt, lane, s_info);  // one round trip: lane i looks at group i
+        if (wid == 0) locate_mtile<BMR>(p, mt, lane, s_info, s_info + 3);  // one round trip: lane i looks at group i
         __syncthreads();
         g = s_info[0]; row0 = s_info[1]; rows = s_info[2];
         if (g < 0) return;
@@ -849,14 +849,14 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
     // the operand rows are requested before the weights (loads return in order: the rows, which come from the cache levels,
     // can then be quantized while the weight fragments are still on their way from HBM), then the quantization parameters of
     // the rows are derived while all of it is in flight
+    // (rows past the tile's last are neither read nor parked: what lies in their place meets only accumulator rows that nobody stores.  One row of K = 4096:
+    // 16 times as many chunks quantized as it has, 5500 cycles of a workgroup's 18400)
     const int mfr = (rows + 15) / 16;          // live row fragments
     const int cpr = K / 16;                    // 16-element chunks per row
-    const int total_chunks = mfr * 16 * cpr;   // rows padded to whole fragments (padding rows are zero)
+    const int total_chunks = rows * cpr;
     float4 f[CPT][4];
     int rr[CPT], kc[CPT];
-    bool aok[CPT];
-    // every load is issued (clamped to a valid address) so that the compiler can count the loads in flight; rows outside the
-    // tile are zeroed when they are used
+    // every load is issued (clamped to a valid address) so that the compiler can count the loads in flight
     auto a_issue = [&](int c0) {
         int src[CPT];
 #pragma unroll
@@ -865,8 +865,7 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
             const int cc = min(c, total_chunks - 1);
             rr[u] = cc / cpr;
             kc[u] = cc - rr[u] * cpr;
-            aok[u] = c < total_chunks && rr[u] < rows;
-            src[u] = row0 + (rr[u] < rows ? rr[u] : 0);
+            src[u] = row0 + rr[u];
         }
         if (p.a_src_row) {  // all indices are requested before the first one is waited for
 #pragma unroll
@@ -878,9 +877,7 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
         }
 #pragma unroll
         for (int u = 0; u < CPT; ++u) {
-            // a chunk of a padding row is never used: its lanes all ask for the tile's first 64 bytes, one request per instruction
-            // instead of 64 (the load itself stays, so that the loads in flight can be counted)
-            const float* ap = (const float*)p.A + (int64_t)src[u] * K + (aok[u] ? kc[u] : 0) * 16;
+            const float* ap = (const float*)p.A + (int64_t)src[u] * K + kc[u] * 16;
 #pragma unroll
             for (int e = 0; e < 4; ++e) f[u][e] = *(const float4*)(ap + e * 4);
         }
@@ -911,7 +908,7 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
                 q.inv_scale = q_inv[rr[u]]; q.zp = q_zp[rr[u]]; q.scale = 0.0f;
                 uint32_t w[4];
     #pragma unroll
-                for (int e = 0; e < 4; ++e) w[e] = aok[u] ? quantize4_u7_signed(f[u][e], q) : 0u;
+                for (int e = 0; e < 4; ++e) w[e] = quantize4_u7_signed(f[u][e], q);
                 *(uint4*)(smem + rr[u] * LDA + kc[u] * 16) = make_uint4(w[0], w[1], w[2], w[3]);
             }
             if (c0 + NT * CPT < total_chunks) a_issue(c0 + NT * CPT);
@@ -926,6 +923,11 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
         const bool lane_in = lane < cpr;
         const int kq = lane_in ? lane : 0;
         const bool pub = pub_problem && nt == 0;  // uniform over the workgroup
+        // a tile that holds every row that its slots count (one call of at most 16 rows; a group of them whose slots are its own) has their ranges itself:
+        // nothing to wait for.  One token, three such launches a step: a record's way there and back was 5000 of their 17600 cycles
+        const bool alone = p.group_off ? (p.a_group_slots == 1 || p.a_group_slots == 2) && p.a_row_slot && s_info[3] <= BMR : !p.a_row_slot && p.M_total <= BMR;
+        uint32_t* own_lo = (uint32_t*)(q_zp + BMR);      // [2] ranges of the group's slots
+        uint32_t* own_hi = own_lo + 2;
         int src[2];
         bool rok[2];
 #pragma unroll
@@ -946,6 +948,11 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
         // (lane j: the row's j-th slot) - both requested now, ahead of the rows
         int my_slot = p.a_slot_base;
         if (wid == 0 && p.a_row_slot && (lane & 15) < rows) my_slot += p.a_row_slot[row0 + (lane & 15)];
+        int own[2] = {0, 0};      // alone: which of the group's slots this wave's rows belong to
+        if (alone && p.group_off) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) own[u] = p.a_row_slot[row0 + (rok[u] ? wid + 8 * u : 0)] - g * p.a_group_slots;
+        }
         const int ns = np.tok_slots ? np.spr : 1;
         int ts[2] = {0, 0};
         if (pub && np.tok_slots && lane < ns) {
@@ -963,25 +970,32 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
         SK_STAMP(1);
         uint32_t* tab_lo = (uint32_t*)smem;  // publishers: (min, max) per relative slot over the tile's rows, in the operand area
         uint32_t* tab_hi = tab_lo + I64H_STAT_TAB;
-        if (pub) {
-            for (int i = tid; i < np.n_rel; i += NT) { tab_lo[i] = I64H_ORDERED_ZERO; tab_hi[i] = I64H_ORDERED_ZERO; }
+        if (pub || alone) {
+            if (pub)
+                for (int i = tid; i < np.n_rel; i += NT) { tab_lo[i] = I64H_ORDERED_ZERO; tab_hi[i] = I64H_ORDERED_ZERO; }
+            if (tid < 4) own_lo[tid] = I64H_ORDERED_ZERO;
             __syncthreads();
         }
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
+            if (!rok[u]) break;      // (uniform over the wave)
             float lo, hi;
             pro_norm_row(x[u], gw, lane_in, K, np.eps, lo, hi);
-            if (pub) {
+            if (pub || alone) {
                 lo = wave_min(lo);
                 hi = wave_max(hi);
-                if (rok[u] && lane < ns) {
+                if (pub && lane < ns) {
                     atomicMin(&tab_lo[ts[u]], f32_to_ordered(lo));
                     atomicMax(&tab_hi[ts[u]], f32_to_ordered(hi));
                 }
+                if (alone && lane == 0) {
+                    atomicMin(&own_lo[own[u] & 1], f32_to_ordered(lo));
+                    atomicMax(&own_hi[own[u] & 1], f32_to_ordered(hi));
+                }
             }
         }
+        if (pub || alone) __syncthreads();
         if (pub) {
-            __syncthreads();
             if (tid < np.n_rel) {
                 v4u rec;
                 rec.x = tab_lo[tid]; rec.y = tab_hi[tid]; rec.z = 1u; rec.w = 0u;
@@ -991,7 +1005,12 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
         // every workgroup: wave 0 collects the records of its rows' slots (lane = row + 16 q looks at publishers q, q + 4, ...)
         if (wid == 0) {
             uint32_t mn = 0xffffffffu, mx = 0u;
-            if ((lane & 15) < rows) {
+            if (alone) {
+                if ((lane & 15) < rows) {
+                    const int s = p.group_off ? (my_slot - p.a_slot_base - g * p.a_group_slots) & 1 : 0;
+                    mn = own_lo[s], mx = own_hi[s];
+                }
+            } else if ((lane & 15) < rows) {
                 const uint32_t* rec = np.stats + (int64_t)my_slot * I64H_SLOT_WORDS;
                 const unsigned long long t0 = __builtin_amdgcn_s_memtime();
                 for (int j = lane >> 4; j < np.n_pub; j += 4) {
@@ -1027,10 +1046,10 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
             const int r = wid + 8 * u;
             QParams q;
             q.inv_scale = q_inv[r]; q.zp = q_zp[r]; q.scale = 0.0f;
-            if (lane_in) {
+            if (lane_in && rok[u]) {
                 uint32_t w[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) w[e] = rok[u] ? quantize4_u7_signed(x[u][e], q) : 0u;
+                for (int e = 0; e < 4; ++e) w[e] = quantize4_u7_signed(x[u][e], q);
                 *(uint4*)(smem + r * LDA + lane * 16) = make_uint4(w[0], w[1], w[2], w[3]);
             }
         }
@@ -1623,7 +1642,7 @@ static int launch_skinny_norm(const i64h_gemm_desc* a, const i64h_gemm_desc* b, 
     }
     size_t area = (size_t)SK_BM * (a->K + 32);
     if (area < SK_AREA_MIN) area = SK_AREA_MIN;
-    const size_t lds = area + 16 + 3 * SK_BM * 4;
+    const size_t lds = area + 16 + 3 * SK_BM * 4 + 16;
     hipLaunchKernelGGL((gemm_i8_skinny_norm_kernel<EPI, 1>), dim3((unsigned)total), dim3(512), lds, st, pp, ta, pr);
     I64H_CHECK_LAUNCH();
     return 0;

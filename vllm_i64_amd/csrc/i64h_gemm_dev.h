@@ -88,9 +88,10 @@ __device__ __forceinline__ v4u ld16_sys(const uint32_t* p) {
 
 // Wave-wide search for m-tile mt of a grouped problem: lane i looks at group c0 + i, 64 groups per pass; writes
 // (group or -1, first row, rows in the tile) to s_info.  The grid is an upper bound on the number of m-tiles.
+// group_rows (optional): the rows of that group.
 template <int BM>
-__device__ __forceinline__ void locate_mtile(const GemmI8Args& p, const int mt, const int lane, int* s_info) {
-    int g = -1, row0 = 0, rows = 0, base = 0;
+__device__ __forceinline__ void locate_mtile(const GemmI8Args& p, const int mt, const int lane, int* s_info, int* group_rows = nullptr) {
+    int g = -1, row0 = 0, rows = 0, base = 0, all = 0;
     const int G = p.group_off ? p.G : 1;
     for (int c0 = 0; c0 < G && g < 0; c0 += 64) {
         const int i = c0 + lane;
@@ -113,10 +114,14 @@ __device__ __forceinline__ void locate_mtile(const GemmI8Args& p, const int mt, 
             g = c0 + src;
             row0 = __shfl(b, src) + (mt - __shfl(excl, src)) * BM;
             rows = min(BM, __shfl(e, src) - row0);
+            all = __shfl(e - b, src);
         }
         base += __shfl(incl, 63);
     }
-    if (lane == 0) { s_info[0] = g; s_info[1] = row0; s_info[2] = rows; }
+    if (lane == 0) {
+        s_info[0] = g; s_info[1] = row0; s_info[2] = rows;
+        if (group_rows) *group_rows = all;
+    }
 }
 
 __device__ __forceinline__ void kv_store(void* cache, int64_t idx, float v, int kv_dtype) {
