@@ -180,3 +180,31 @@ def test_tiled_gemm_on_64_and_128_row_tiles_gives_the_same_bits(dev, rows, K, N,
         ops.call("i64h_set_gemm_big_tile_min", 384)
     assert torch.equal(outs[0][0], outs[1][0]) and outs[0][0].abs().sum() > 0
     assert all(torch.equal(x, y) for x, y in zip(outs[0][1], outs[1][1]))
+
+
+@pytest.mark.parametrize("rows,K,N", [(1, 4096, 1024), (16, 2048, 1000), (17, 2048, 520), (3, 640, 64), (16, 704, 100), (1, 1088, 16), (33, 1024, 1024), (112, 4096, 1024), (2, 2112, 40), (16, 8192, 48)])
+@pytest.mark.parametrize("packed", [True, False])
+def test_narrow_workgroups_of_few_rows_give_the_same_bits(dev, rows, K, N, packed):
+    """Launches of few workgroups: 32 or 16 columns each, K steps in four or eight shares (also shares of unequal size, and the last ones empty)."""
+    from vllm_i64_amd import ops
+    if packed and N % 16:
+        pytest.skip("fragment packs hold whole blocks of 16 columns")
+    g = torch.Generator().manual_seed(rows + K + N)
+    x, h = torch.randn(rows, K, generator=g).to(dev), torch.randn(rows, N, generator=g).to(dev)
+    w = torch.randint(-128, 128, (1, N, K), dtype=torch.int8, generator=g).to(dev)
+    ws = torch.full((1,), 3e-3, device=dev)
+    stats = ops.stats_alloc(1, dev)
+    ops.stats_reset(stats)
+    ops.rows_minmax(x, stats, slot_base=0)
+
+    def run():
+        out = h.clone()
+        ops.gemm_i8_pair(ops.gemm_desc(x, w, ws, out, a_slot_base=0, stats=stats, w_frags=ops.pack_weight_frags(w) if packed else None, c_residual=out))
+        return out
+    a, b = _both(ops, run)
+    assert torch.equal(a, b)
+    lo, hi = min(float(x.min()), 0.0), max(float(x.max()), 0.0)
+    # codes of 7 bits: a value is off by at most half a step, times sums of K weights of up to 128
+    step = (hi - lo) / 127.0
+    want = h.double() + x.double() @ (w[0].double() * 3e-3).t()
+    assert float((a.double() - want).abs().max()) <= 0.51 * step * 3e-3 * float(w[0].double().abs().sum(1).max())

@@ -675,7 +675,7 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
     constexpr int MF = BMR / 16;                     // MFMA row fragments of the tile
     // K steps (64 deep) whose B fragments are in flight together: all of K = 1024 in one batch (half with two fragments per step)
     // (with helper waves a wave streams half of K: 8 steps cover K = 1024 in one batch for either epilogue)
-    constexpr int SK_STEPS = HW > 1 ? 8 : 16 / NF;
+    constexpr int SK_STEPS = HW == 4 ? 4 : HW > 1 ? 8 : 16 / NF;
     const int K = p.K, LDA = K + 32;
     // LDS: operand rows [16][LDA] int8, reused by the epilogues (statistics table, head tile of EPI_QKR: SK_AREA_MIN bytes at
     // least, which matters for K < 224) | info (16 B) | q_inv[16] q_scale[16] q_zp[16]
@@ -687,8 +687,8 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
 
     const int nout = (EPI == EPI_SWIGLU) ? p.N / 2 : p.N;
     constexpr int BNB = NW * 16, NT = NW * HW * 64;  // output columns / threads per workgroup
-    constexpr int CPT = 4 / HW;                     // 16-element operand chunks per thread and pass
-    static_assert(HW == 1 || HW == 2, "helper factor (16 waves leave 128 registers per lane: measured 3.28 against 1.94 ms per step)");
+    constexpr int CPT = HW > 1 ? 2 : 4;             // 16-element operand chunks per thread and pass
+    static_assert(HW == 1 || NW * HW == 8 || NW * HW == 4, "helper factor (16 waves leave 128 registers per lane: measured 3.28 against 1.94 ms per step)");
     // workgroups are dealt to the 8 XCDs round-robin and every XCD has an L2 of its own: with the column-tile count padded to a
     // multiple of 8, the row tiles that stream the same weight slice run on ONE XCD and the slice crosses the fabric once
     const int n_tiles = (nout + BNB - 1) / BNB, n_pad = sk_pad_tiles(n_tiles);
@@ -716,7 +716,8 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
     }
     if (nt >= n_tiles) return;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const bool helper = HW > 1 && wid >= NW;  // wave-uniform
+    const int share = HW > 1 ? wid / NW : 0;  // which of the K steps' shares this wave takes (wave-uniform)
+    const bool helper = share > 0;
 #define SK_STAMP(i) do { if (p.stamps && tid == 0) p.stamps[(int64_t)blockIdx.x * 8 + (i)] = __builtin_amdgcn_s_memtime(); } while (0)
     SK_STAMP(0);
     int g, row0, rows;
@@ -755,17 +756,17 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
     const int8_t* Bg = p.B + (int64_t)g * p.N * K;
     const int I = p.N / 2;
     // this lane's weight rows (output columns)
-    // With helper waves and room in LDS for the partial sums, a helper wave also takes the second half of the K steps of the
-    // column fragment of main wave wid - NW (integer partial sums add exactly, in any order)
-    const int wcol = helper ? wid - NW : wid;
+    // With helper waves and room in LDS for the partial sums, a helper wave also takes its share of the K steps of the
+    // column fragment of main wave wid % NW (integer partial sums add exactly, in any order)
+    const int wcol = wid % NW;
     const int col = nt * BNB + wcol * 16 + fr;
     const bool col_in = col < nout;
     const bool col_ok = col_in && !helper;
-    constexpr int PART_OFF = SK_AREA_MIN, PART_BYTES = NW * MF * NF * 64 * 16;
-    const bool ksplit = HW > 1 && BMR * LDA >= PART_OFF + PART_BYTES && nsteps >= 2;  // uniform over the workgroup
-    const int s_half = (nsteps + 1) / 2;
-    const int s_begin = (ksplit && helper) ? s_half : 0;
-    const int s_end = ksplit ? (helper ? nsteps : s_half) : (helper ? 0 : nsteps);
+    constexpr int PART_OFF = SK_AREA_MIN, PART_BYTES = (HW - 1) * NW * MF * NF * 64 * 16;
+    const bool ksplit = HW > 1 && BMR * LDA >= PART_OFF + PART_BYTES && nsteps >= HW;  // uniform over the workgroup
+    const int s_share = (nsteps + HW - 1) / HW;
+    const int s_begin = ksplit ? min(share * s_share, nsteps) : 0;
+    const int s_end = ksplit ? min(s_begin + s_share, nsteps) : (helper ? 0 : nsteps);
     const int8_t* bp[NF];
     int bstep = 64;  // bytes from one K step of a lane's weight stream to the next
     if (p.b_frags) {
@@ -917,7 +918,7 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
         SK_STAMP(3);
     } else {
 #if BMR == 16   // (a build with taller tiles, for measurements, must not be given these launches)
-        static_assert(!PRO || (NW == 4 && HW == 2 && BMR == 16), "the norm prologue is laid out for eight waves and one row fragment");
+        static_assert(!PRO || (NW * HW == 8 && BMR == 16), "the norm prologue is laid out for eight waves and one row fragment");
 #endif
         // wave wid holds rows wid and wid + 8 of the tile, lane l elements [16 l, 16 l + 16) of each (K <= 1024: launcher)
         const bool lane_in = lane < cpr;
@@ -1084,8 +1085,10 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
 
     if (HW > 1 && ksplit) {
         __syncthreads();  // every wave is done with the operand rows: their LDS takes the helper waves' partial sums
-        v4i* part = (v4i*)(smem + PART_OFF) + (wcol * (MF * NF)) * 64 + lane;
+        v4i* part = (v4i*)(smem + PART_OFF) + (wcol * (MF * NF)) * 64 + lane;      // (share i: NW * MF * NF * 64 further)
+        constexpr int SHARE = NW * MF * NF * 64;
         if (helper) {
+            part += (share - 1) * SHARE;
 #pragma unroll
             for (int i = 0; i < MF; ++i)
 #pragma unroll
@@ -1096,7 +1099,9 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
 #pragma unroll
             for (int i = 0; i < MF; ++i)
 #pragma unroll
-                for (int f = 0; f < NF; ++f) acc[i][f] += part[(i * NF + f) * 64];
+                for (int f = 0; f < NF; ++f)
+#pragma unroll
+                    for (int h = 0; h < HW - 1; ++h) acc[i][f] += part[h * SHARE + (i * NF + f) * 64];
         }
     }
     SK_STAMP(4);
@@ -1217,12 +1222,12 @@ __global__ __launch_bounds__(NW * HW * 64) void gemm_i8_skinny_kernel(GemmI8Pair
 }
 
 // The same with the RMSNorm prologue (NormPro): the first problem's column-tile-0 workgroups publish the call statistics.
-template <int EPI, int PRO>
+template <int EPI, int PRO, int NW = 4>
 __global__ __launch_bounds__(512) void gemm_i8_skinny_norm_kernel(GemmI8Pair pp, RowTailArgs ta, NormPro np) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int bid = blockIdx.x;
-    if (bid < pp.nblk0) gemm_i8_skinny_body<EPI, 4, 2, PRO>(pp.p[0], bid, smem, ta, np, true);
-    else gemm_i8_skinny_body<EPI, 4, 2, PRO>(pp.p[1], bid - pp.nblk0, smem, ta, np, false);
+    if (bid < pp.nblk0) gemm_i8_skinny_body<EPI, NW, 8 / NW, PRO>(pp.p[0], bid, smem, ta, np, true);
+    else gemm_i8_skinny_body<EPI, NW, 8 / NW, PRO>(pp.p[1], bid - pp.nblk0, smem, ta, np, false);
 }
 
 // ---- fp32 GEMM on the f32 matrix cores: C[M,N] = A[M,K] @ B[N,K]^T ------------------------------------------------
@@ -1582,6 +1587,16 @@ static int launch_skinny_nw(const i64h_gemm_desc* a, const i64h_gemm_desc* b, hi
         if (bm == 64) return launch_skinny<EPI, 4, 2, 64>(a, b, st);
         if (bm == 32) return launch_skinny<EPI, 4, 2, 32>(a, b, st);
     }
+    if constexpr (EPI == EPI_STORE) {
+        // A single call of a few workgroups leaves most CUs idle while each streams 64 columns: 32 columns a workgroup and K in four shares below 129 workgroups of
+        // 64, 16 columns and K in eight where they would be at most 16 and K is long.  2-layer dense model (o: K = 1024, down: 4096), us a step with 64 columns |
+        // 32 | 16: 1 token 128.2 | 125.8 | 122.7, 7 140.8 | 137.3 | 137.3, 24 151.1 | 147.6 | 148.3, 64 159.8 | 156.0 | 158.7, 100 200.7 | 198.3 | 220,
+        // 150 252 | 275 | 294.  K from where the partial sums fit beside the statistics in the rows' LDS.  (A down projection of one token by itself 6.7 | 5.3 | 4.7.)  Launches with experts have workgroups enough: 24 tokens 152.2 | 154.3 | 162.
+        const int nb = skinny_blocks(a, 64);
+        const bool one = !b && !a->group_offsets && nw == 4 && g_skinny_helpers;
+        if (one && nb <= 16 && a->K >= 2048) return launch_skinny<EPI, 1, 8>(a, b, st);
+        if (one && nb <= 128 && a->K >= 640) return launch_skinny<EPI, 2, 4>(a, b, st);
+    }
     if (nw == 4) return launch_skinny<EPI, 4>(a, b, st);
     if (nw == 16) return launch_skinny<EPI, 16>(a, b, st);
     return launch_skinny<EPI, 8>(a, b, st);
@@ -1632,10 +1647,15 @@ static int launch_skinny_norm(const i64h_gemm_desc* a, const i64h_gemm_desc* b, 
     GemmI8Pair pp;
     pp.p[0] = to_args(a);
     pp.p[1] = b ? to_args(b) : pp.p[0];
+    // few workgroups: 32 columns each, K in four shares.  Us a step, 64 columns | 32: dense, 1 token 128.2 | 126.4, 16 150.5 | 149.2, 24 (128 workgroups of 64) 151.1 | 152.6,
+    // 33 149.8 | 152.3; mixture, 3 tokens 137.3 | 132.9, 12 147 | 144.5, 24 (152) 152.2 | 153.1, 64 224.5 | 229.3
+    constexpr int few = EPI == EPI_QKR ? 4 : 2;      // (a tile of 64 columns is a head there)
+    const bool narrow = EPI != EPI_QKR && skinny_blocks(a, 64) + (b ? skinny_blocks(b, 64) : 0) < 128 && a->K >= 992;
+    const int bnb = narrow ? 32 : 64;
     const int nout_a = a->epilogue == EPI_SWIGLU ? a->N / 2 : a->N;
     // the publishing workgroups lead the launch: inside the grid where its column slots allow the trade, else as extra workgroups
-    pp.nblk0 = skinny_blocks(a, 64) + (pr.n_pub <= sk_pad_tiles((nout_a + 63) / 64) ? 0 : ((pr.n_pub + 7) & ~7));
-    const int total = pp.nblk0 + (b ? skinny_blocks(b, 64) : 0);
+    pp.nblk0 = skinny_blocks(a, bnb) + (pr.n_pub <= sk_pad_tiles((nout_a + bnb - 1) / bnb) ? 0 : ((pr.n_pub + 7) & ~7));
+    const int total = pp.nblk0 + (b ? skinny_blocks(b, bnb) : 0);
     if (g_stamps && g_stamp_cur + total <= g_stamp_cap) {
         pp.p[0].stamps = pp.p[1].stamps = g_stamps + g_stamp_cur * 8;
         g_stamp_cur += total;
@@ -1643,7 +1663,8 @@ static int launch_skinny_norm(const i64h_gemm_desc* a, const i64h_gemm_desc* b, 
     size_t area = (size_t)SK_BM * (a->K + 32);
     if (area < SK_AREA_MIN) area = SK_AREA_MIN;
     const size_t lds = area + 16 + 3 * SK_BM * 4 + 16;
-    hipLaunchKernelGGL((gemm_i8_skinny_norm_kernel<EPI, 1>), dim3((unsigned)total), dim3(512), lds, st, pp, ta, pr);
+    if (narrow) hipLaunchKernelGGL((gemm_i8_skinny_norm_kernel<EPI, 1, few>), dim3((unsigned)total), dim3(512), lds, st, pp, ta, pr);
+    else hipLaunchKernelGGL((gemm_i8_skinny_norm_kernel<EPI, 1>), dim3((unsigned)total), dim3(512), lds, st, pp, ta, pr);
     I64H_CHECK_LAUNCH();
     return 0;
 }
