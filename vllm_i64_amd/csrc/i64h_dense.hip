@@ -998,7 +998,7 @@ int i64h_linear_run(const i64h_linear* dp, void* stream) {
     I64H_CHECK_ARG(d.batch <= 65535 && (d.M + 63) / 64 <= 65535, "linear: grid too large");
     I64H_CHECK_ARG(d.A16 || !d.C16, "linear: results in bf16 belong to input rows in bf16");
     if (d.A16) {
-        I64H_CHECK_ARG(!d.exact && (dn_dual(d.epilogue) || d.epilogue == I64H_EPI_STORE || d.epilogue == I64H_EPI_SCALE || d.epilogue == I64H_EPI_ADD),
+        I64H_CHECK_ARG(!d.exact && (dn_dual(d.epilogue) || d.epilogue == I64H_EPI_STORE || d.epilogue == I64H_EPI_SCALE || d.epilogue == I64H_EPI_ADD || d.epilogue == I64H_EPI_ROW_SIGMOID),
                        "linear: input rows in bf16 with epilogue %d or 32-bit products", d.epilogue);
         I64H_CHECK_ARG(d.K % 64 == 0 && d.lda % 8 == 0 && d.a_batch % 8 == 0 && d.w_batch % 8 == 0 && ((uintptr_t)d.A16 | (uintptr_t)d.W) % 16 == 0,
                        "linear: input rows in bf16 need K a multiple of 64 (%d) and rows at 16 bytes", d.K);

@@ -1136,7 +1136,7 @@ int i64h_kattn(const i64h_kattn_args* dp, void* stream) {
     I64H_CHECK_ARG(d.heads > 0 && d.kv_heads > 0 && d.heads % d.kv_heads == 0 && d.dim > 0 && d.dim <= KA_MAX_DIM, "kattn: heads %d, kv heads %d, dim %d (at most %d)",
                    d.heads, d.kv_heads, d.dim, KA_MAX_DIM);
     I64H_CHECK_ARG(d.vdim >= 0 && d.vdim <= KA_MAX_DIM, "kattn: vdim %d (at most %d)", d.vdim, KA_MAX_DIM);
-    I64H_CHECK_ARG(d.Q && d.cache && (d.kscale || d.vdim > 0) && d.block_table && d.slot_ids && d.positions && d.out, "kattn: null operand");
+    I64H_CHECK_ARG(d.Q && d.cache && (d.kscale || d.vdim > 0) && d.block_table && d.slot_ids && d.positions && (d.out || d.out16), "kattn: null operand");
     I64H_CHECK_ARG(d.cache_dtype == 0 || d.cache_dtype == 2, "kattn: cache type %d", d.cache_dtype);
     I64H_CHECK_ARG(!d.bias || d.bias_rows > 0, "kattn: an empty bias table");
     I64H_CHECK_ARG(d.keep_first >= 0 && (!d.sink_w || d.sink), "kattn: %d kept positions, or sink scores without the sink", d.keep_first);
@@ -1154,9 +1154,12 @@ int i64h_kattn(const i64h_kattn_args* dp, void* stream) {
         a.row_stride = d.kv_heads * gs, a.kv_groups = d.kv_heads, a.chunk = d.chunk, a.kscale = d.kscale, a.bias = d.bias, a.bias_rows = d.bias_rows;
         a.sink = d.sink, a.sink_w = d.sink_w, a.softcap = d.softcap;
         a.key_off = d.vdim > 0 ? d.vdim : 0;
+        a.out16 = d.out16;
+        I64H_CHECK_ARG(bf16_form || !d.out16, "kattn: a result in bf16 belongs to the matrix-core form over a bf16 cache");
         if (latent_rows_f32_ok(a)) return latent_rows_f32_run(a, stream);
         return i64h_latent_attn(&a, stream);
     }
+    I64H_CHECK_ARG(!d.out16, "kattn: a result in bf16 belongs to the matrix-core form over a bf16 cache");
     const int64_t items = d.n * d.heads;
     const dim3 grid((unsigned)((items + 3) / 4));
     if (d.cache_dtype == 0) hipLaunchKernelGGL((kattn_row_kernel<float>), grid, dim3(256), 0, (hipStream_t)stream, d);

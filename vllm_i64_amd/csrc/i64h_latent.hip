@@ -178,6 +178,19 @@ __device__ __forceinline__ void lt_split_pair(float x, float y, uint32_t& hi, ui
     lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{x - __uint_as_float(hi << 16), y - __uint_as_float(hi & 0xffff0000u)}), v2bf));
 }
 
+// a value, or four neighbours, of the result: rounded where the caller wants it so
+__device__ __forceinline__ void lt_put(const i64h_latent_attn_args& p, int64_t at, float v) {
+    if (p.out16) ((uint16_t*)p.out16)[at] = (uint16_t)lt_rne(v);
+    else p.out[at] = v;
+}
+__device__ __forceinline__ void lt_put4(const i64h_latent_attn_args& p, int64_t at, const float4& v) {
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
+    if (p.out16) *(uint2*)((uint16_t*)p.out16 + at) = __builtin_bit_cast(uint2, __builtin_convertvector((v4f{v.x, v.y, v.z, v.w}), v4bf));
+    else if (((uintptr_t)p.out & 15) == 0) *(float4*)(p.out + at) = v;
+    else p.out[at] = v.x, p.out[at + 1] = v.y, p.out[at + 2] = v.z, p.out[at + 3] = v.w;
+}
+
 // Matrix-core form (bf16 cache) of rows that are one per sequence.  One wave per task of 16 query vectors that walk the same cached rows: the (up to) 16
 // heads of a group of one token, a share of its keys.
 // Per tile of 32 keys: scores S^T[32, 16] = K Q^T on v_mfma_f32_16x16x32_bf16 with the cached rows read straight from memory as A
@@ -388,13 +401,11 @@ __global__ __launch_bounds__(64) void latent_attn_mfma_decode_kernel(const i64h_
         return;
     }
     if (hin + n >= rep) return;
-    float* o = p.out + (tok * H + head0 + n) * r;
+    const int64_t o = (tok * H + head0 + n) * r;
     const float inv = 1.0f / l;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
-        if (!ANY || nb * 16 < r)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) o[nb * 16 + 4 * kg + g] = acc[nb][g] * inv;
+        if (!ANY || nb * 16 < r) lt_put4(p, o + nb * 16 + 4 * kg, make_float4(acc[nb][0] * inv, acc[nb][1] * inv, acc[nb][2] * inv, acc[nb][3] * inv));
 }
 
 // One row and head by one wave, over the keys that it sees only: a key per lane for the scores, the columns (at most 256) spread over the lanes for the
@@ -441,10 +452,10 @@ __device__ __forceinline__ void latent_row(const i64h_latent_attn_args& p, const
                 if (lane + 64 * c < r) acc[c] = fmaf(wk, value(v[lane + 64 * c]), acc[c]);
         }
     }
-    float* const o = p.out + (t * p.heads + h) * r;
+    const int64_t o = (t * p.heads + h) * r;
 #pragma unroll
     for (int c = 0; c < 4; ++c)
-        if (lane + 64 * c < r) o[lane + 64 * c] = acc[c] / l;
+        if (lane + 64 * c < r) lt_put(p, o + lane + 64 * c, acc[c] / l);
 }
 
 // A tile's rows, [64] positions and [64] slots (-1: no such row) in LDS; lane l reads row l's.  (Every wave writes all of them, and reads what it wrote.)
@@ -712,16 +723,11 @@ __global__ __launch_bounds__(256, 2) void latent_attn_rows_kernel(const i64h_lat
     const uint32_t by_key = (uint32_t)(lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) & 0xffffu;      // rows of this wave
     for (uint32_t left = by_key; left; left &= left - 1) latent_row<uint16_t>(p, row0 + wr + __ffs((int)left) - 1, head);
     if (!valid || !mine || (by_key >> n & 1)) return;
-    float* o = p.out + (tok * H + head) * r;
+    const int64_t o = (tok * H + head) * r;
     const float inv = 1.0f / l;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
-        if (nb * 16 < r) {
-            const float4 v = make_float4(acc[nb][0] * inv, acc[nb][1] * inv, acc[nb][2] * inv, acc[nb][3] * inv);
-            float* dst = o + nb * 16 + kg * 4;
-            if (((uintptr_t)p.out & 15) == 0) *(float4*)dst = v;
-            else dst[0] = v.x, dst[1] = v.y, dst[2] = v.z, dst[3] = v.w;
-        }
+        if (nb * 16 < r) lt_put4(p, o + nb * 16 + kg * 4, make_float4(acc[nb][0] * inv, acc[nb][1] * inv, acc[nb][2] * inv, acc[nb][3] * inv));
 }
 
 // The same for rows of exactly D values, the first R of them value columns, keys from column KO on, without key scales, soft cap or bias.  A tile's rows go
@@ -960,17 +966,10 @@ __global__ __launch_bounds__(256, 2) void latent_attn_rows_direct_kernel(const i
     const uint32_t by_key = (uint32_t)(lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) & 0xffffu;      // rows of this wave
     for (uint32_t left = by_key; left; left &= left - 1) latent_row<uint16_t>(p, row0 + wr + __ffs((int)left) - 1, head);
     if (!valid || !mine || (by_key >> n & 1)) return;
-    float* o = p.out + (tok * H + head) * R + kg * 4;
+    const int64_t o = (tok * H + head) * R + kg * 4;
     const float inv = 1.0f / (l2.lo + l2.hi);
-    if (((uintptr_t)p.out & 15) == 0) {
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) *(float4*)(o + nb * 16) = make_float4(acc[nb][0] * inv, acc[nb][1] * inv, acc[nb][2] * inv, acc[nb][3] * inv);
-    } else {
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) o[nb * 16 + g] = acc[nb][g] * inv;
-    }
+    for (int nb = 0; nb < NB; ++nb) lt_put4(p, o + nb * 16, make_float4(acc[nb][0] * inv, acc[nb][1] * inv, acc[nb][2] * inv, acc[nb][3] * inv));
 }
 
 // The same for caches of 32-bit rows, with 32-bit products: keys and transposed values once in LDS (twice would be a workgroup per CU), the next tile
@@ -1181,16 +1180,11 @@ __global__ __launch_bounds__(256, NB > 8 ? 1 : 2) void latent_attn_rows_f32_kern
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
     if (!valid || !mine) return;
-    float* o = p.out + (tok * H + head) * r;
+    const int64_t o = (tok * H + head) * r;
     const float inv = 1.0f / l;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
-        if (nb * 16 < r) {
-            const float4 v = make_float4(acc[nb][0] * inv, acc[nb][1] * inv, acc[nb][2] * inv, acc[nb][3] * inv);
-            float* dst = o + nb * 16 + kg * 4;
-            if (((uintptr_t)p.out & 15) == 0) *(float4*)dst = v;
-            else dst[0] = v.x, dst[1] = v.y, dst[2] = v.z, dst[3] = v.w;
-        }
+        if (nb * 16 < r) lt_put4(p, o + nb * 16 + kg * 4, make_float4(acc[nb][0] * inv, acc[nb][1] * inv, acc[nb][2] * inv, acc[nb][3] * inv));
 }
 
 // The same for rows of exactly D values without an option (as latent_attn_rows_direct_kernel), in launches whose workgroups of four heads would leave CUs
@@ -1387,14 +1381,10 @@ __global__ __launch_bounds__(256, 2) void latent_attn_rows_f32_quarters_kernel(c
     for (uint32_t left = by_key, k = 0; left; left &= left - 1, ++k)
         if ((int)(k & 3) == wid) latent_row<float>(p, row0 + __ffs((int)left) - 1, head);
     if (!valid || !mine || (by_key >> n & 1)) return;
-    float* o = p.out + (tok * H + head) * R + wid * NBW * 16 + kg * 4;
+    const int64_t o = (tok * H + head) * R + wid * NBW * 16 + kg * 4;
     const float inv = 1.0f / (l2.lo + l2.hi);
 #pragma unroll
-    for (int i = 0; i < NBW; ++i) {
-        const float4 v = make_float4(acc[i][0] * inv, acc[i][1] * inv, acc[i][2] * inv, acc[i][3] * inv);
-        if (((uintptr_t)p.out & 15) == 0) *(float4*)(o + i * 16) = v;
-        else o[i * 16] = v.x, o[i * 16 + 1] = v.y, o[i * 16 + 2] = v.z, o[i * 16 + 3] = v.w;
-    }
+    for (int i = 0; i < NBW; ++i) lt_put4(p, o + i * 16, make_float4(acc[i][0] * inv, acc[i][1] * inv, acc[i][2] * inv, acc[i][3] * inv));
 }
 
 // the shares of a token's keys, merged: one wave per (token, head); lane s holds share s's maximum and weight sum (at most 64
@@ -1441,7 +1431,7 @@ __global__ __launch_bounds__(64) void latent_attn_merge_kernel(const i64h_latent
         }
 #pragma unroll
         for (int i = 0; i < NC; ++i)
-            if (c0 + 64 * i < r) p.out[(tok * H + head) * r + c0 + 64 * i] = num[i] / den;
+            if (c0 + 64 * i < r) lt_put(p, (tok * H + head) * r + c0 + 64 * i, num[i] / den);
     }
 }
 
@@ -1535,7 +1525,7 @@ int i64h_latent_attn(const i64h_latent_attn_args* dp, void* stream) {
     I64H_CHECK_ARG(d.n >= 0 && d.heads > 0 && d.kv_rank > 0 && d.rot_dim >= 0 && d.block_size > 0, "latent_attn: bad sizes");
     I64H_CHECK_ARG(d.kv_rank <= 64 * LT_MAXC, "latent_attn: kv_rank %d above %d", d.kv_rank, 64 * LT_MAXC);
     I64H_CHECK_ARG(d.cache_dtype == 0 || d.cache_dtype == 2, "latent_attn: cache dtype %d", d.cache_dtype);
-    I64H_CHECK_ARG(d.Q && d.cache && d.block_table && d.slot_ids && d.positions && d.out, "latent_attn: null operand");
+    I64H_CHECK_ARG(d.Q && d.cache && d.block_table && d.slot_ids && d.positions && (d.out || d.out16), "latent_attn: null operand");
     I64H_CHECK_ARG(d.key_off >= 0 && d.key_off <= d.kv_rank, "latent_attn: %d value-only columns of %d value columns", d.key_off, d.kv_rank);
     if (d.n == 0) return 0;
     const int D = d.kv_rank + d.rot_dim;
@@ -1544,6 +1534,7 @@ int i64h_latent_attn(const i64h_latent_attn_args* dp, void* stream) {
     I64H_CHECK_ARG(mfma_ok || (d.kv_groups <= 1 && d.row_stride <= 0 && d.chunk <= 0 && !d.kscale && !d.bias),
                    "latent_attn: key heads, chunks, key scales and bias are built for the matrix-core form only");
     I64H_CHECK_ARG(!d.sink_w || d.sink, "latent_attn: sink scores without the sink");
+    I64H_CHECK_ARG(!d.out16 || (mfma_ok && d.mode != 1 && (uintptr_t)d.out16 % 16 == 0), "latent_attn: a result in bf16 belongs to the matrix-core form, at 16 bytes");
     I64H_CHECK_ARG(d.keep_first >= 0, "latent_attn: %d kept positions", d.keep_first);
     if (d.mode != 1 && mfma_ok) {
         const int row_tiles = d.mode == 3;

@@ -205,7 +205,7 @@ __global__ __launch_bounds__(64 * NWM * NWN, PER_CU * NWM * NWN / 4) void linear
     if constexpr (DUAL) {
         switch (p.epilogue) { DN_FINISH(I64H_EPI_CLAMP_GLU) DN_FINISH(I64H_EPI_GELU_MUL) DN_FINISH(I64H_EPI_SILU_MUL) }
     } else {
-        switch (p.epilogue) { DN_FINISH(I64H_EPI_SCALE) DN_FINISH(I64H_EPI_ADD) DN_FINISH(I64H_EPI_STORE) }
+        switch (p.epilogue) { DN_FINISH(I64H_EPI_SCALE) DN_FINISH(I64H_EPI_ADD) DN_FINISH(I64H_EPI_ROW_SIGMOID) DN_FINISH(I64H_EPI_STORE) }
     }
 #undef DN_FINISH
 }

@@ -77,6 +77,11 @@ class HybridRunner:
         """Whether Linears over rows of these widths read them in bf16 (the values their tiles would round to: results are the same)."""
         return not self.exact and n > self.WIDE_ROWS and all(w % 64 == 0 and 2 * w * max(n, self.max_ff + 256) < self.WIDE_BYTES for w in widths)
 
+    def _wide_attention(self, n: int, width: int, vals: int, part: int, cache: torch.Tensor) -> bool:
+        """Whether an attention over rows of `part` values a key head, the first `vals` of them summed, leaves its result (rows of `width`) in bf16: the matrix-core form
+        and Linears that read it so."""
+        return self._wide(n, width) and cache.dtype == torch.bfloat16 and vals % 16 == 0 and vals <= 256 and part % 8 == 0 and part <= 320
+
     @staticmethod
     def _as16(t: torch.Tensor, n: int, width: int) -> torch.Tensor:
         """The memory of a buffer of fp32 rows as rows in bf16."""
@@ -230,12 +235,14 @@ class HybridRunner:
                    k_norm_w=d.get("k_norm"), eps=self.cfg.norm_eps, rot_dims=a.rot.dims if a.rot is not None else 0, interleaved=a.interleaved,
                    inv_freq=d["inv_freq"], rot_mult=d["rot_mult"], head_norm=a.qk_norm == "head", v_freq=d["v_freq"], scale=a.scale, positions=positions,
                    slot_ids=slot_ids, block_table=kvc.block_table, cache=rows, q=Q, n=n, norm_heads=a.qk_norm == "head_weight")
-        O = B.b[: n * a.heads * a.vdim].view(n, a.heads * a.vdim)
+        behind = d["v_freq"] is not None or a.head_gate
+        wide = not behind and self._wide_attention(n, a.heads * a.vdim, a.vdim, gs, rows)
+        O = self._as16(B.b, n, a.heads * a.vdim) if wide else B.b[: n * a.heads * a.vdim].view(n, a.heads * a.vdim)
         self._kattn(B, a, Q, O, rows, kvc, slot_ids, positions, runs, ctx_hint, softcap=a.softcap, window=a.window, keep_first=a.keep_first, sink_w=d.get("sink"))
-        if d["v_freq"] is not None or a.head_gate:
+        if behind:
             D.rot_post(O, heads=a.heads, vdim=a.vdim, interleaved=a.interleaved, v_freq=d["v_freq"], positions=positions,
                        gate=P if a.head_gate else None, gate_off=d.get("g_off", 0), ldg=P.shape[-1], n=n)
-        self._out(O, d["o"], out, scale)
+        self._out(None if wide else O, d["o"], out, scale, O if wide else None)
 
     def _out(self, a, w, out, scale: float = 1.0, a16=None) -> None:
         D.linear(a, w, out, a16=a16, exact=self.exact, epilogue=D.EPI_STORE if scale == 1.0 else D.EPI_SCALE, scale=scale)
@@ -278,7 +285,8 @@ class HybridRunner:
                       q_src=src if m.q_rank else None, rot_mult=d["rot_mult"])
         # queries into latent space, per head: Q[:, h, :r] = q_unrotated[:, h, :] @ U_h
         D.linear(src, d["uk_t"], Q, m=n, n=r, k=m.dim, a_off=q_off, lda=src.shape[-1], ldc=H * width, batch=H, a_batch=qh, w_batch=r * m.dim, c_batch=width, exact=ex)
-        olat = B.b[: n * H * r]
+        wide = self._wide_attention(n, H * r, r, width, cache) and r % 64 == 0 and self._wide(n, H * m.vdim)
+        olat = (B.b.view(torch.bfloat16) if wide else B.b)[: n * H * r]
         keys = min(ctx_hint, m.window + 64) if m.window > 0 else ctx_hint
         for r0, r1, one_per_seq in runs:
             splits, ws = 1, None
@@ -287,10 +295,15 @@ class HybridRunner:
             D.latent_attn(Q[r0 * H * width: r1 * H * width], cache, kvc.block_table, slot_ids[r0:r1], positions[r0:r1], window=m.window, scale=m.scale, heads=H, kv_rank=r,
                           rot_dim=rd, out=olat[r0 * H * r: r1 * H * r], n=r1 - r0, mode=2 if one_per_seq else 3, splits=splits, workspace=ws, sink=d["sink"])
         # summed latents into value space, per head
-        og = B.c[: n * H * m.vdim]
+        og = (B.c.view(torch.bfloat16) if wide else B.c)[: n * H * m.vdim]
         gate = dict(epilogue=D.EPI_ROW_SIGMOID, e=P, e_off=d["g_off"], lde=N1, e_batch=1) if m.head_gate else {}
-        D.linear(olat, d["uv"], og, m=n, n=m.vdim, k=r, lda=H * r, ldc=H * m.vdim, batch=H, a_batch=r, w_batch=m.vdim * r, c_batch=m.vdim, exact=ex, **gate)
-        D.linear(og, d["o"], out, m=n, k=H * m.vdim, lda=H * m.vdim, exact=ex)
+        maps = dict(m=n, n=m.vdim, k=r, lda=H * r, ldc=H * m.vdim, batch=H, a_batch=r, w_batch=m.vdim * r, c_batch=m.vdim, exact=ex, **gate)
+        if wide:
+            D.linear(None, d["uv"], None, a16=olat, out16=og, **maps)
+            D.linear(None, d["o"], out, a16=og, m=n, k=H * m.vdim, lda=H * m.vdim)
+        else:
+            D.linear(olat, d["uv"], og, **maps)
+            D.linear(og, d["o"], out, m=n, k=H * m.vdim, lda=H * m.vdim, exact=ex)
 
     # ---- gated linear attention ----
     def _gated_linear(self, B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, out, scale: float = 1.0, work=NO_WORK) -> None:

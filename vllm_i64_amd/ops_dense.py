@@ -36,7 +36,7 @@ def linear(a: Optional[torch.Tensor], w: torch.Tensor, out: Optional[torch.Tenso
     batch may have, and a_rows / a / out must hold group_off[batch] rows (the caller's business: the counts stay on the device).
     row_scale fp32, one factor per row of out (the gate / up epilogues): the input row times that factor.
     in_norm_w fp32 [k] with in_eps: the input rows are RMS-normed first (plain result: the epilogue is then EPI_IN_NORM).
-    a16 bf16 (k a multiple of 64; the plain, scaled, adding and gate / up epilogues): the rows of a, rounded by whoever wrote them, in a's place.
+    a16 bf16 (k a multiple of 64; the plain, scaled, adding, row-gated and gate / up epilogues): the rows of a, rounded by whoever wrote them, in a's place.
     out16 bf16 (with a16): receives the result rounded, beside out or (out None) in its place."""
     if a16 is None:
         if a is None or out is None or out16 is not None:
@@ -159,12 +159,18 @@ def latent_prep(p: torch.Tensor, *, q_off: int, dkv_off: int, heads: int, dim: i
     call_dense("i64h_latent_prep", _ref(d), _stream())
 
 
+def _as(t: torch.Tensor, dtype: torch.dtype) -> int:
+    """The address of a tensor of this type, null of another."""
+    return ptr(t) if t.dtype == dtype else 0
+
+
 def latent_attn(q: torch.Tensor, cache: torch.Tensor, block_table: torch.Tensor, slot_ids: torch.Tensor, positions: torch.Tensor, *,
                 window: int, scale: float, heads: int, kv_rank: int, rot_dim: int, out: torch.Tensor, n: Optional[int] = None,
                 mode: int = 0, splits: int = 1, workspace: Optional[torch.Tensor] = None, sink: Optional[torch.Tensor] = None,
                 softcap: float = 0.0) -> torch.Tensor:
-    """See i64h_latent_attn.  sink fp32 [heads]: a learned extra score per head in the softmax's denominator."""
-    _chk(q, torch.float32, "q"), _chk(out, torch.float32, "out"), _chk(cache, None, "cache")
+    """See i64h_latent_attn.  sink fp32 [heads]: a learned extra score per head in the softmax's denominator.  out: fp32 or, in the matrix-core form over a
+    bf16 cache, bf16 (the result rounded)."""
+    _chk(q, torch.float32, "q"), _chk(out, torch.bfloat16 if out.dtype == torch.bfloat16 else torch.float32, "out"), _chk(cache, None, "cache")
     _chk(positions, torch.int32, "positions"), _chk(slot_ids, torch.int32, "slot_ids"), _chk(block_table, torch.int32, "block_table")
     rows = int(n if n is not None else positions.numel())
     D = kv_rank + rot_dim
@@ -183,7 +189,7 @@ def latent_attn(q: torch.Tensor, cache: torch.Tensor, block_table: torch.Tensor,
             raise _lib.I64HError(f"latent_attn: workspace of {workspace.numel()} floats, {need} needed")
     d = _lib.LatentAttn(Q=ptr(q), cache=ptr(cache), cache_dtype=CACHE_DTYPE_CODE[cache.dtype], block_table=ptr(block_table),
                         max_blocks_per_seq=block_table.shape[1], block_size=cache.shape[-2], slot_ids=ptr(slot_ids), positions=ptr(positions),
-                        window=int(window), scale=float(scale), out=ptr(out), n=rows, heads=heads, kv_rank=kv_rank, rot_dim=rot_dim, mode=mode,
+                        window=int(window), scale=float(scale), out=_as(out, torch.float32), out16=_as(out, torch.bfloat16), n=rows, heads=heads, kv_rank=kv_rank, rot_dim=rot_dim, mode=mode,
                         splits=int(splits) if splits > 1 else 1, workspace=ptr(workspace) if splits > 1 else 0, sink=int(sink is not None), sink_w=ptr(sink),
                         softcap=float(softcap))
     call_dense("i64h_latent_attn", _ref(d), _stream())
@@ -403,8 +409,9 @@ def kattn(q: torch.Tensor, cache: torch.Tensor, kscale: torch.Tensor, block_tabl
           window: int = 0, keep_first: int = 0, sink_w: Optional[torch.Tensor] = None) -> torch.Tensor:
     """See i64h_kattn.  q, out fp32 [n, heads * dim]; bias fp32 [distances, heads].  vdim > 0: separate values - the cache rows are
     [kv_heads, vdim + dim], q fp32 [n, heads, vdim + dim], out fp32 [n, heads * vdim], kscale may be None.  window > 0: the last `window`
-    positions and the first keep_first ones are seen.  sink_w fp32 [heads]: the sink's score per head."""
-    _chk(q, torch.float32, "q"), _chk(out, torch.float32, "out"), _chk(cache, None, "cache")
+    positions and the first keep_first ones are seen.  sink_w fp32 [heads]: the sink's score per head.  out: fp32 or, in the matrix-core form over a bf16
+    cache, bf16 (the result rounded)."""
+    _chk(q, torch.float32, "q"), _chk(out, torch.bfloat16 if out.dtype == torch.bfloat16 else torch.float32, "out"), _chk(cache, None, "cache")
     if kscale is not None or vdim <= 0:
         _chk(kscale, torch.float32, "kscale")
     _chk(positions, torch.int32, "positions"), _chk(slot_ids, torch.int32, "slot_ids"), _chk(block_table, torch.int32, "block_table")
@@ -431,7 +438,7 @@ def kattn(q: torch.Tensor, cache: torch.Tensor, kscale: torch.Tensor, block_tabl
             raise _lib.I64HError(f"kattn: workspace of {workspace.numel()} floats, {need} needed")
     d = _lib.KAttn(Q=ptr(q), cache=ptr(cache), cache_dtype=CACHE_DTYPE_CODE[cache.dtype], kscale=ptr(kscale), block_table=ptr(block_table),
                    max_blocks_per_seq=block_table.shape[1], block_size=cache.shape[-2], slot_ids=ptr(slot_ids), positions=ptr(positions), chunk=int(chunk),
-                   bias=ptr(bias), bias_rows=bias.shape[0] if bias is not None else 0, sink=int(bool(sink)), out=ptr(out), n=rows, heads=heads,
+                   bias=ptr(bias), bias_rows=bias.shape[0] if bias is not None else 0, sink=int(bool(sink)), out=_as(out, torch.float32), out16=_as(out, torch.bfloat16), n=rows, heads=heads,
                    kv_heads=kv_heads, dim=dim, mode=int(mode), splits=int(splits) if splits > 1 else 1, workspace=ptr(workspace) if splits > 1 else 0,
                    vdim=int(vdim), softcap=float(softcap), window=int(window), keep_first=int(keep_first), sink_w=ptr(sink_w))
     call_dense("i64h_kattn", _ref(d), _stream())
