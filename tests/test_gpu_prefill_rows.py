@@ -215,3 +215,59 @@ def test_fused_residual_norm_quant_equals_norm_then_quantize(dev, mode, n, H):
         if mode == "add_gather":
             assert torch.equal(gs, gs2) and torch.equal(ga, g2)
         assert int(sync.abs().sum()) == 0   # the launch leaves its sync words zero (and its wait budget was not exceeded)
+
+
+@pytest.mark.parametrize("nh,kvh,block", [(16, 4, 16), (3, 3, 6), (8, 4, 64), (16, 2, 3)])
+def test_prefill_attention_over_bf16_pages(dev, nh, kvh, block):
+    """Prompt portions over a bf16 cache at the edges of its 64-token tiles: contexts of 1, 63 .. 65, 127 .. 129 and 191 .. 193, several
+    sequences in one 16-row tile, a row that sees nothing, tokens without a page (some, a whole tile, the first ones, all of a sequence's)
+    behind which lies NaN, NaN in every page that no sequence uses, the range of the result.  Against 64-bit arithmetic: fp32 products and
+    sums of at most 260 terms with weights that sum to 1 and values below 6 leave a few 1e-7 of the sum of the terms' magnitudes."""
+    ops = _ops()
+    hd = 64
+    g = torch.Generator().manual_seed(nh + block)
+    seqs = [(0, 1), (62, 3), (126, 3), (190, 3), (0, 65), (250, 10), (0, 140), (120, 20), (60, 40), (0, 3), (70, 5)]      # (cached, new)
+    per = [(p + t + block - 1) // block for p, t in seqs]
+    pages = sum(per) + 3
+    k = torch.randn(pages, block, kvh, hd, generator=g).bfloat16()
+    v = torch.randn(pages, block, kvh, hd, generator=g).bfloat16()
+    perm = (torch.randperm(pages - 1, generator=g) + 1).to(torch.int32)
+    bt = torch.full((len(seqs), max(per) + 1), -1, dtype=torch.int32)
+    at = 0
+    for s, n_ in enumerate(per):
+        bt[s, :n_] = perm[at:at + n_]
+        at += n_
+    gone = {4: [0], 5: range(64 // block, (128 + block - 1) // block), 7: [per[7] // 2], 8: [0, 1][:per[8] - 1], 9: range(per[9])}
+    for s, which in gone.items():
+        for i in which:
+            bt[s, i] = -1
+    used = set(int(i) for i in bt.flatten() if i >= 0)
+    for i in range(pages):
+        if i not in used:
+            k[i] = v[i] = float("nan")
+    slot = [s for s, (_, t) in enumerate(seqs) for _ in range(t)]
+    ctx = [p + i + 1 for p, t in seqs for i in range(t)]
+    ctx[100] = 0
+    rows = len(slot)
+    assert rows >= 256
+    q = torch.randn(rows, nh, hd, generator=g)
+    stats = ops.stats_alloc(2, dev)
+    ops.stats_reset(stats)
+    out = ops.paged_attn(q.to(dev), k.to(dev), v.to(dev), bt.to(dev), torch.tensor(ctx, dtype=torch.int32, device=dev),
+                         slot_ids=torch.tensor(slot, dtype=torch.int32, device=dev), splits=1, stats=stats, stat_slot=1).cpu()
+    assert torch.isfinite(out).all()
+    kd, vd, qd = k.double(), v.double(), q.double().view(rows, kvh, nh // kvh, hd)
+    for r in range(rows):
+        t = torch.arange(ctx[r])
+        page = bt[slot[r], t // block].long()
+        t, page = t[page >= 0], page[page >= 0]
+        if not len(t):
+            assert not out[r].any()
+            continue
+        w = torch.softmax(torch.einsum("hgd,thd->hgt", qd[r], kd[page, t % block]) / hd ** 0.5, -1)
+        ref = torch.einsum("hgt,thd->hgd", w, vd[page, t % block]).reshape(nh, hd)
+        assert (out[r].double() - ref).abs().max() <= 3e-6, r
+    same = ops.stats_alloc(2, dev)
+    ops.stats_reset(same)
+    ops.rows_minmax(out.view(rows, nh * hd).to(dev), same, slots=torch.ones(rows, dtype=torch.int32, device=dev))
+    assert torch.equal(ops.qparams(stats, 2)[2][1], ops.qparams(same, 2)[2][1])

@@ -11,6 +11,7 @@
 // for the operator form); 0 gives an all-zero output row, as the reference does for an empty sequence.
 #include "i64h_common.h"
 #include "../../include/i64h.h"
+#include <type_traits>
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
 #include <math.h>
@@ -449,13 +450,7 @@ __device__ __forceinline__ void split3_pair(float x, float y, uint32_t& hi, uint
 __device__ __forceinline__ int pb_k(int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 1) & 7)) << 3); }
 __device__ __forceinline__ int pb_v(int row, int chunk) { return row * 64 + ((chunk ^ (((row >> 1) & 3) << 1)) << 3); }
 
-// eight cache elements of a token row as eight bf16 (16 bytes): a bf16 cache as it is; the 8-bit float formats convert exactly
-template <typename KV> struct Stage8;
-template <> struct Stage8<__hip_bfloat16> {
-    v4i32 r;
-    __device__ __forceinline__ void load(const __hip_bfloat16* p) { r = *(const v4i32*)p; }
-    __device__ __forceinline__ v4i32 bf16x8() const { return r; }
-};
+// eight cache elements of a token row as eight bf16 (16 bytes): the 8-bit float formats convert exactly
 template <typename KV> struct Stage8 {
     Raw8<KV> r;
     __device__ __forceinline__ void load(const KV* p) { r.load(p); }
@@ -659,6 +654,232 @@ __global__ __launch_bounds__(GS * 64, I64H_PF_OCC) void paged_attn_prefill_bf16_
                 for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[j], __builtin_bit_cast(v8bf, ph), acc[j], 0, 0, 0);
                 acc[4] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, __builtin_bit_cast(v8bf, ph), acc[4], 0, 0, 0);
             }
+        }
+        const float lsum = acc[4][0];  // every row of the ones fragment carries the normaliser of query row c
+        if (active) {
+            float* op = out + ((int64_t)r * nh + head) * HD + g * 4;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                float4 o = make_float4(0, 0, 0, 0);
+                if (lsum > 0.0f) o = make_float4(acc[j][0] / lsum, acc[j][1] / lsum, acc[j][2] / lsum, acc[j][3] / lsum);
+                *(float4*)(op + 16 * j) = o;
+                olo = fminf(olo, fminf(fminf(o.x, o.y), fminf(o.z, o.w)));
+                ohi = fmaxf(ohi, fmaxf(fmaxf(o.x, o.y), fmaxf(o.z, o.w)));
+            }
+            done = true;
+        }
+    }
+    pf_fold_range(stats, stat_slot, olo, ohi);
+}
+
+// ---- the same for bf16 caches: tiles go from memory to LDS by themselves ------------------------------------------------------------------
+// The form above spends its time between the products: a tile passes through registers (64 of them), its rows' flags through LDS, two barriers a tile, and the
+// registers leave two waves a SIMD.  Here a tile is loaded straight into LDS, 16 bytes a lane, the column that a lane brings chosen so that the piece lands where
+// pb_k / pb_v say, while the tile before it is worked on: one barrier a tile, three waves a SIMD.  A lane looks up the page of one token a tile (every wave all
+// 64) a tile ahead of the loads; a ballot of them says, without LDS, which tokens have a page, and whether a tile needs a mask at all.
+// The operations and their order are the form above's, the results the same bits.  16 heads over 4 KV heads, before and after, us: 8 sequences of 2048 rows
+// 291 -> 248, one of 481 17.6 -> 14.1, 1500 + 77 52 -> 42.5; 12 heads over 12, 2 of 2048 204 -> 118; 16 over 8 150 -> 108; 32 over 4 182 -> 160; forty of 16 rows
+// 8.5 -> 8.5.  With three tiles in LDS (and two on their way) 250, 14.1, 43.0, 137, 115, 165: fewer workgroups fit.  Four waves a SIMD spill (309).
+// 8-bit caches stay with the form above, which converts on the way into LDS.
+template <int GS>
+__global__ __launch_bounds__(GS * 64, 3) void paged_attn_prefill_direct_kernel(const float* __restrict__ q, const __hip_bfloat16* __restrict__ k_cache,
+                                                                         const __hip_bfloat16* __restrict__ v_cache, const int32_t* __restrict__ block_table,
+                                                                         int max_blocks_per_seq, const int32_t* __restrict__ slot_ids, const int32_t* __restrict__ ctx_len,
+                                                                         float scale, float* __restrict__ out, int n, int kvh, int block, uint32_t* __restrict__ stats, int stat_slot) {
+    constexpr int HD = 64, LW = 16 / GS;      // a wave's loads a tile: as many of K's 8-row pieces as of V's
+    static_assert(LW >= 2, "");
+    constexpr float LOG2E = 1.4426950408889634f;
+    __shared__ __attribute__((aligned(1024))) unsigned short s0[PF_TOK * 128], s1[PF_TOK * 128];      // K rows, V rows
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, c = lane & 15;
+    const int kh = blockIdx.y, head = kh * GS + wid, nh = kvh * GS;
+    const int r = (gridDim.x - 1 - blockIdx.x) * 16 + c;  // this lane's query row (tiles are taken from the back)
+    const bool valid = r < n;
+    const int my_slot = valid ? (slot_ids ? slot_ids[r] : r) : -1;
+    const int my_ctx = valid ? ctx_len[r] : 0;
+    bool done = !valid;
+    float olo = 0.0f, ohi = 0.0f;  // range of the rows this lane stores (with zero, as the quantizer's range has it)
+    const int bshift = (block & (block - 1)) == 0 ? __builtin_ctz(block) : -1;
+
+    uint4 qh[2], qm[2], ql[2];      // as above
+    {
+        const float* qp = q + ((int64_t)(valid ? r : 0) * nh + head) * HD;
+#pragma unroll
+        for (int h2 = 0; h2 < 2; ++h2) {
+            float v[8];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const float4 a = valid ? *(const float4*)(qp + 32 * h2 + 8 * g + 4 * i) : make_float4(0, 0, 0, 0);
+                v[4 * i] = a.x * scale * LOG2E; v[4 * i + 1] = a.y * scale * LOG2E;
+                v[4 * i + 2] = a.z * scale * LOG2E; v[4 * i + 3] = a.w * scale * LOG2E;
+            }
+            split3_pair(v[0], v[1], qh[h2].x, qm[h2].x, ql[h2].x);
+            split3_pair(v[2], v[3], qh[h2].y, qm[h2].y, ql[h2].y);
+            split3_pair(v[4], v[5], qh[h2].z, qm[h2].z, ql[h2].z);
+            split3_pair(v[6], v[7], qh[h2].w, qm[h2].w, ql[h2].w);
+        }
+    }
+    constexpr std::integral_constant<int, 0> S0{};
+    constexpr std::integral_constant<int, 1> S1{};
+    auto stage = [&](auto set) -> unsigned short* {      // (variables of their own: the compiler then knows which loads a read of one has to wait for)
+        constexpr int S = decltype(set)::value;
+        return S == 0 ? s0 : s1;
+    };
+    // pieces of eight token rows, i * GS + wid of K and of V for this wave; this lane's row of a piece, and the column that it brings
+    const int lr = lane >> 3, row_stride = kvh * HD;
+    const __hip_bfloat16 *kc[2], *const vc = v_cache + kh * HD + ((lane & 7) ^ (((lr >> 1) & 3) << 1)) * 8;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) kc[i] = k_cache + kh * HD + ((lane & 7) ^ ((4 * (i * GS + wid) + (lr >> 1)) & 7)) * 8;
+    const int vrow = (4 * g + (c >> 2)) * 64 + 4 * (c & 1), vsw = ((c >> 1) & 1) ^ (((4 * g + (c >> 2)) >> 1 & 3) << 1);
+
+    while (true) {
+        // rows of one sequence per pass: the first unfinished row picks the sequence
+        const unsigned long long pending = __ballot(!done) & 0xffffull;
+        if (!pending) break;
+        const int lead = __ffsll(pending) - 1;
+        const int cur_slot = __builtin_amdgcn_readlane(my_slot, lead);
+        const bool active = !done && my_slot == cur_slot;
+        const int lim = active ? my_ctx : 0;      // causal limit of this lane's query row
+        int kv_end = lim, lim_min = active ? lim : 0x7fffffff;  // a tile below every active row's limit needs no causal mask
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) kv_end = max(kv_end, __shfl_xor(kv_end, o)), lim_min = min(lim_min, __shfl_xor(lim_min, o));
+        kv_end = __builtin_amdgcn_readfirstlane(kv_end), lim_min = __builtin_amdgcn_readfirstlane(lim_min);
+        const int32_t* bt = block_table + (int64_t)cur_slot * max_blocks_per_seq;
+
+        float m = -INFINITY;
+        v4f acc[5];  // acc[j][e] = O^T[dim 16 j + 4 g + e][query row c]; acc[4][*] = the row's normaliser
+#pragma unroll
+        for (int j = 0; j < 5; ++j) acc[j] = (v4f){0, 0, 0, 0};
+        const int tiles = (kv_end + PF_TOK - 1) / PF_TOK;
+        struct Row {      // of token t0 + lane: its page, its place there
+            int pb, in;
+        };
+        auto look_up = [&](int tile) {
+            const int t = max(0, min(min(tile, tiles - 1) * PF_TOK + lane, kv_end - 1));
+            const int bi = bshift >= 0 ? t >> bshift : t / block;
+            return Row{bt[bi], bshift >= 0 ? t & (block - 1) : t - bi * block};
+        };
+        auto load = [&](const Row& row, unsigned long long has, auto set) {
+            unsigned short* sm = stage(set);
+            // (a token that is not there reads another's row: its weight will be nothing, which nothing but a number may meet)
+            const int mine = row.pb * block + row.in, other = has ? __builtin_amdgcn_readlane(mine, __ffsll(has) - 1) : 0;
+            const int at = has >> lane & 1 ? mine : other;
+            int src[LW / 2];
+#pragma unroll
+            for (int i = 0; i < LW / 2; ++i) src[i] = __shfl(at, 8 * (i * GS + wid) + lr);
+#pragma unroll
+            for (int i = 0; i < LW / 2; ++i) {
+                const int64_t off = (int64_t)src[i] * row_stride;
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(kc[GS == 1 ? i & 1 : 0] + off), (__attribute__((address_space(3))) void*)(sm + 8 * (i * GS + wid) * 64), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(vc + off), (__attribute__((address_space(3))) void*)(sm + PF_TOK * 64 + 8 * (i * GS + wid) * 64), 16, 0, 0);
+            }
+        };
+        Row next;      // of the next tile
+        unsigned long long ok[2];      // the tokens of the tiles on their way that have a page
+        auto ok_of = [&](int tile, const Row& row) { return __ballot(row.pb >= 0 && tile * PF_TOK + lane < kv_end); };
+        auto step = [&](int tile, auto cur, auto free) {
+            // this wave's loads of the tile are in LDS, its reads of the one before done; then everybody's.  On their way: the loads of later tiles
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0x0070);      // vmcnt, lgkmcnt 0
+            asm volatile("s_barrier" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            constexpr int C = decltype(cur)::value, F = decltype(free)::value;
+            const Row then = look_up(tile + 2);
+            ok[F] = ok_of(tile + 1, next);
+            load(next, ok[F], free);      // (past the end the last tile again, which nobody reads: without a branch the loads on their way are the same everywhere)
+            next = then;
+            if (!ok[C]) return;
+            const unsigned short* Kb = stage(cur);
+            const int t0 = tile * PF_TOK;
+            // scores of 64 tokens: S^T tile t holds tokens t0 + 16 t + 4 g + reg of query row c; small terms first
+            v4f sc[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) sc[t] = (v4f){0, 0, 0, 0};
+#pragma unroll
+            for (int h2 = 0; h2 < 2; ++h2) {
+                v8bf kf[4];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) kf[t] = __builtin_bit_cast(v8bf, *(const uint4*)&Kb[pb_k(16 * t + c, 4 * h2 + g)]);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t], __builtin_bit_cast(v8bf, ql[h2]), sc[t], 0, 0, 0);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t], __builtin_bit_cast(v8bf, qm[h2]), sc[t], 0, 0, 0);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t], __builtin_bit_cast(v8bf, qh[h2]), sc[t], 0, 0, 0);
+            }
+            if (t0 + PF_TOK > lim_min || ok[C] != ~0ull) {      // the tokens that this lane's row sees, the lane's own from bit 0 of each half
+                const int left = max(0, min(lim - t0, PF_TOK));
+                const unsigned long long see = ok[C] & (left < PF_TOK ? (1ull << left) - 1 : ~0ull);
+                const uint32_t half[2] = {(uint32_t)see >> (4 * g), (uint32_t)(see >> 32) >> (4 * g)};
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sc[t][e] = half[t >> 1] & 1u << (16 * (t & 1) + e) ? sc[t][e] : -INFINITY;
+            }
+            float mx = -INFINITY;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) mx = fmaxf(mx, fmaxf(fmaxf(sc[t][0], sc[t][1]), fmaxf(sc[t][2], sc[t][3])));
+            {  // over the four lanes of a query row (lane ^ 16, lane ^ 32) through register swaps, no LDS round trip
+                const PairF sr = swap_rows(mx);
+                mx = fmaxf(sr.lo, sr.hi);
+                const PairF sh = swap_halves(mx);
+                mx = fmaxf(sh.lo, sh.hi);
+            }
+            const float mn = fmaxf(m, mx);
+            if (__ballot(mn != m)) {  // some row's running maximum moved: rescale (rare after the first tiles)
+                const float alpha = (mn == -INFINITY) ? 1.0f : exp2f(m - mn);
+#pragma unroll
+                for (int j = 0; j < 5; ++j) acc[j] *= alpha;
+            }
+            m = mn;
+            const float mref = (mn == -INFINITY) ? 0.0f : mn;  // exp2(-inf - 0) = 0 for masked scores, no per-element test
+#pragma unroll
+            for (int kp = 0; kp < 2; ++kp) {  // 32 tokens per step: the lane's slots are its registers of score tiles 2 kp and 2 kp + 1
+                float pv[8];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    pv[e] = __builtin_amdgcn_exp2f(sc[2 * kp][e] - mref);
+                    pv[4 + e] = __builtin_amdgcn_exp2f(sc[2 * kp + 1][e] - mref);
+                }
+                uint4 ph, pm, pl;
+                split3_pair(pv[0], pv[1], ph.x, pm.x, pl.x);
+                split3_pair(pv[2], pv[3], ph.y, pm.y, pl.y);
+                split3_pair(pv[4], pv[5], ph.z, pm.z, pl.z);
+                split3_pair(pv[6], pv[7], ph.w, pm.w, pl.w);
+                v8bf vf[4];      // V^T fragments, as above
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const unsigned short* vp = &Kb[PF_TOK * 64 + 32 * 64 * kp + vrow + ((2 * j) ^ vsw) * 8];
+                    v4s half[2];
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) half[b] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(vp + 16 * 64 * b));
+                    vf[j] = __builtin_bit_cast(v8bf, __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7));
+                }
+                const v8bf ones = __builtin_bit_cast(v8bf, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[j], __builtin_bit_cast(v8bf, pl), acc[j], 0, 0, 0);
+                acc[4] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, __builtin_bit_cast(v8bf, pl), acc[4], 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[j], __builtin_bit_cast(v8bf, pm), acc[j], 0, 0, 0);
+                acc[4] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, __builtin_bit_cast(v8bf, pm), acc[4], 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[j], __builtin_bit_cast(v8bf, ph), acc[j], 0, 0, 0);
+                acc[4] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, __builtin_bit_cast(v8bf, ph), acc[4], 0, 0, 0);
+            }
+        };
+        if (tiles > 0) {
+            __syncthreads();      // (the rows before have been read)
+            const Row at0 = look_up(0);
+            next = look_up(1);
+            ok[0] = ok_of(0, at0);
+            load(at0, ok[0], S0);
+            int tile = 0;
+            for (; tile + 2 <= tiles; tile += 2) {
+                step(tile, S0, S1);
+                step(tile + 1, S1, S0);
+            }
+            if (tile < tiles) step(tile, S0, S1);
+            __builtin_amdgcn_s_waitcnt(0x0f70);      // (nothing is on its way into LDS when a pass ends)
         }
         const float lsum = acc[4][0];  // every row of the ones fragment carries the normaliser of query row c
         if (active) {
@@ -1382,11 +1603,14 @@ int i64h_paged_attn(const float* q, const void* k_cache, const void* v_cache, in
 #define PFB(G, T)                                                                                                                          \
     hipLaunchKernelGGL((paged_attn_prefill_bf16_kernel<G, T>), grid, dim3(G * 64), 0, st, q, (const T*)k_cache, (const T*)v_cache, block_table, \
                        (int)max_blocks_per_seq, slot_ids, ctx_len, softmax_scale, out, (int)rows, (int)num_kv_heads, (int)block_size, stats, (int)stat_slot)
+#define PFD(G)                                                                                                                               \
+    hipLaunchKernelGGL((paged_attn_prefill_direct_kernel<G>), grid, dim3(G * 64), 0, st, q, (const __hip_bfloat16*)k_cache, (const __hip_bfloat16*)v_cache, block_table, \
+                       (int)max_blocks_per_seq, slot_ids, ctx_len, softmax_scale, out, (int)rows, (int)num_kv_heads, (int)block_size, stats, (int)stat_slot)
 #define PFG(G)                                                  \
     do {                                                        \
         if (kv_dtype == 0) PF(G, float);                        \
         else if (kv_dtype == 1) PF(G, __half);                  \
-        else if (kv_dtype == 2 && g_prefill_mfma == 1) PFB(G, __hip_bfloat16); \
+        else if (kv_dtype == 2 && g_prefill_mfma == 1) PFD(G);  \
         else if (kv_dtype == 3 && g_prefill_mfma == 1) PFB(G, F8E4);           \
         else if (kv_dtype == 4 && g_prefill_mfma == 1) PFB(G, F8E5);           \
         else if (kv_dtype == 2) PF(G, __hip_bfloat16);          \
