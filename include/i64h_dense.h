@@ -51,7 +51,7 @@ int i64h_device_check(void);
  * the 64 x 64 tile form beyond.
  * A16 (may be NULL; exact = 0): A's rows rounded to bf16 by whoever wrote them, strides as A's; they are read in A's place and A may be NULL.  Such a
  * launch needs K a multiple of 64, 16-byte aligned rows (lda, a_batch, w_batch multiples of eight) and
- * I64H_EPI_STORE, I64H_EPI_SCALE, I64H_EPI_ADD or one of the gate / up epilogues; its products are those of A.
+ * I64H_EPI_STORE, I64H_EPI_SCALE, I64H_EPI_ADD, I64H_EPI_ROW_SIGMOID or one of the gate / up epilogues; its products are those of A.
  * C16 (may be NULL; with A16): the results rounded to bf16, strides as C's, beside C or (C = NULL) in its place.
  * Any M, N, K >= 1; 16-byte loads are used where strides and addresses allow, element loads otherwise.
  * Launches with M <= I64H_SKINNY_ROWS take a weight-streaming form (one wave per output column group); the form of the others follows from
@@ -204,7 +204,7 @@ typedef struct {
     const float* sink_w; /* with sink: fp32 [heads], the extra score of head h is sink_w[h] instead of zero (NULL: zero) */
     float softcap;       /* > 0: a score s (after scale and key scale, before any bias) becomes softcap * tanh(s / softcap) */
     int32_t keep_first;  /* with a window: the first positions of a sequence that stay visible to everyone */
-    void* out16;         /* bf16, laid out as out, 16-byte aligned: receives the result rounded in out's place (matrix-core form over a bf16 cache only) */
+    void* out16;         /* bf16, laid out as out, 16-byte aligned: receives the result rounded in out's place (matrix-core form over a bf16 cache only: modes 0 and 2 then take it whatever the knob says) */
 } i64h_latent_attn_args;
 int i64h_set_latent_attn_decode_form(int32_t on); /* tuning / test knob: 1 (default) = mode 0 / 2 launches over bf16 caches of fitting sizes take the matrix-core form; 0 = all of them take the row form */
 int64_t i64h_latent_attn_workspace_floats(int64_t n, int32_t heads, int32_t kv_rank, int32_t splits);
@@ -451,7 +451,7 @@ typedef struct {
     float softcap;       /* > 0: the score Q . k * kscale becomes softcap * tanh(. / softcap) before the bias is added */
     int32_t window, keep_first;
     const float* sink_w;
-    void* out16;         /* bf16, laid out as out, 16-byte aligned: receives the result rounded in out's place (matrix-core form over a bf16 cache only) */
+    void* out16;         /* bf16, laid out as out, 16-byte aligned: receives the result rounded in out's place (matrix-core form over a bf16 cache only: modes 0 and 2 then take it whatever the knob says) */
 } i64h_kattn_args;
 int64_t i64h_kattn_workspace_floats(int64_t n, int32_t heads, int32_t kv_heads, int32_t dim, int32_t splits);
 int i64h_kattn(const i64h_kattn_args* d, void* stream);

@@ -313,3 +313,55 @@ def test_many_32_bit_rows_of_exact_sizes(dev):
         return out
     one, cut = run([(0, n)]), run([(0, 700), (700, 1501), (1501, n)])
     assert torch.allclose(one, cut, atol=4e-5, rtol=2e-5), float((one - cut).abs().max())
+
+
+@pytest.mark.parametrize("mode,splits", [(3, 1), (2, 1), (2, 3)])
+@pytest.mark.parametrize("H,G,dim,vdim", [(4, 2, 64, 64), (6, 3, 128, 128), (3, 1, 32, 48)])
+def test_kattn_result_in_bf16(dev, mode, splits, H, G, dim, vdim):
+    """A result asked for in bf16 is the 32-bit one, rounded once: rows of whole tiles and rest, whole prompts and one row a sequence, its keys in one part or
+    several; nothing beyond the rows is written, and the forms that have no such result say so."""
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator().manual_seed(H)
+    lens, past = ([1, 15, 17, 40, 70], [0, 3, 31, 0, 9]) if mode == 3 else ([1] * 5, [0, 3, 31, 130, 200])
+    bt, pos, slots, blocks = pages(lens, past, 16, g)
+    n, w = int(pos.numel()), vdim + dim
+    cache = torch.randn(blocks, 16, G * w, generator=g).bfloat16().to(dev)
+    q = torch.randn(n, H, w, generator=g)
+    q[:, :, :vdim] = 0
+    kw = dict(chunk=0, bias=None, sink=False, heads=H, kv_heads=G, dim=dim, vdim=vdim, n=n, mode=mode, splits=splits)
+    args = (q.to(dev), cache, None, bt.to(dev), slots.to(dev), pos.to(dev))
+    out = D.kattn(*args, out=torch.empty(n, H * vdim, device=dev), **kw)
+    out16 = D.kattn(*args, out=torch.full((n + 1, H * vdim), 7.0, device=dev, dtype=torch.bfloat16), **kw)
+    assert torch.equal(out16[:n], out.bfloat16()) and bool((out16[n] == 7).all())
+    if mode == 2:      # (the knob that keeps such rows off the matrix cores leaves a launch with this result where it is)
+        D.call_dense("i64h_set_latent_attn_decode_form", 0)
+        try:
+            again = D.kattn(*args, out=torch.empty_like(out16), **kw)
+        finally:
+            D.call_dense("i64h_set_latent_attn_decode_form", 1)
+        assert torch.equal(again[:n], out16[:n])
+    with pytest.raises(Exception, match="bf16"):
+        D.kattn(*args, out=out16, **{**kw, "mode": 1, "splits": 1})
+    with pytest.raises(Exception, match="bf16"):
+        D.kattn(args[0], cache.float(), *args[2:], out=out16, **kw)
+
+
+@pytest.mark.parametrize("mode,splits", [(3, 1), (2, 1), (2, 3)])
+@pytest.mark.parametrize("H,r,e", [(16, 256, 32), (4, 128, 16), (5, 64, 32)])
+def test_latent_result_in_bf16(dev, mode, splits, H, r, e):
+    """The same of latent rows."""
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator().manual_seed(H + r)
+    lens, past = ([1, 15, 17, 40, 70], [0, 3, 31, 0, 9]) if mode == 3 else ([1] * 5, [0, 3, 31, 130, 200])
+    bt, pos, slots, blocks = pages(lens, past, 16, g)
+    n = int(pos.numel())
+    cache = torch.randn(blocks, 16, r + e, generator=g).bfloat16().to(dev)
+    args = (torch.randn(n * H * (r + e), generator=g).to(dev), cache, bt.to(dev), slots.to(dev), pos.to(dev))
+    kw = dict(window=0, scale=0.1, heads=H, kv_rank=r, rot_dim=e, n=n, mode=mode, splits=splits)
+    out = D.latent_attn(*args, out=torch.empty(n * H * r, device=dev), **kw)
+    out16 = D.latent_attn(*args, out=torch.full(((n + 1) * H * r,), 7.0, device=dev, dtype=torch.bfloat16), **kw)
+    assert torch.equal(out16[: n * H * r], out.bfloat16()) and bool((out16[n * H * r:] == 7).all())
+    with pytest.raises(Exception, match="bf16"):
+        D.latent_attn(args[0], cache.float(), *args[2:], out=out16, **kw)
+    with pytest.raises(Exception, match="bf16"):
+        D.latent_attn(*args, out=out16, **{**kw, "mode": 1, "splits": 1})

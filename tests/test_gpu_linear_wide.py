@@ -130,3 +130,20 @@ def test_producers_round_once(dev):
         D.gate_norm(y, w[0].contiguous(), o, out16=o16, **kw)
         D.gate_norm(y, w[0].contiguous(), None, out16=alone, **kw)
         assert torch.equal(o16, o.bfloat16()) and torch.equal(alone, o16)
+
+
+@pytest.mark.parametrize("M,K", [(66, 64), (130, 256), (700, 128)])
+def test_row_gates_over_rounded_rows(dev, M, K):
+    """A head's value map over rows in bf16 with the head's gate per row: the fp32 result is that of the same numbers given in 32 bits, the bf16 one that, rounded."""
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator().manual_seed(M)
+    H, N = 5, 48
+    a = torch.randn(M, H, K, generator=g).bfloat16().to(dev)
+    w = torch.randn(H, N, K, generator=g).bfloat16().to(dev)
+    e = torch.randn(M, H + 2, generator=g).to(dev)
+    kw = dict(m=M, n=N, k=K, lda=H * K, ldc=H * N, batch=H, a_batch=K, w_batch=N * K, c_batch=N, epilogue=D.EPI_ROW_SIGMOID, e=e, e_off=1, lde=H + 2, e_batch=1)
+    wide, wide16 = torch.empty(M, H * N, device=dev), torch.empty(M, H * N, device=dev, dtype=torch.bfloat16)
+    D.linear(None, w, wide, a16=a.view(M, H * K), out16=wide16, **kw)
+    ref = torch.matmul(a.double().transpose(0, 1), w.double().transpose(1, 2)).transpose(0, 1) * torch.sigmoid(e[:, 1:1 + H].double())[..., None]
+    # K exact products summed in 32 bits: at most K 2^-24 of the sum of their magnitudes, below 6 sqrt(K)
+    assert float((wide.view(M, H, N) - ref).abs().max()) <= K * 2.0 ** -24 * 6 * K ** 0.5 + 1e-5 and torch.equal(wide16, wide.bfloat16())

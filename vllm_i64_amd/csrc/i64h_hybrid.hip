@@ -1145,7 +1145,7 @@ int i64h_kattn(const i64h_kattn_args* dp, void* stream) {
     // the matrix-core kernel of the latent attention scores against a whole cached row part and sums its first columns: the keys as values
     // (all columns) or [values | keys] with zeros in the query's value columns
     const int vals = d.vdim > 0 ? d.vdim : d.dim, gs = d.vdim > 0 ? d.vdim + d.dim : d.dim;
-    const bool bf16_form = d.mode != 1 && d.cache_dtype == 2 && gs % 8 == 0 && (d.mode == 3 || latent_decode_form()), f32_form = d.mode == 3 && d.cache_dtype == 0 && gs % 4 == 0;      // (the latter: portions of prompts)
+    const bool bf16_form = d.mode != 1 && d.cache_dtype == 2 && gs % 8 == 0 && (d.mode == 3 || latent_decode_form() || d.out16), f32_form = d.mode == 3 && d.cache_dtype == 0 && gs % 4 == 0;      // (the latter: portions of prompts)
     if ((bf16_form || f32_form) && vals % 16 == 0 && vals <= 256 && gs <= 320 && (uintptr_t)d.Q % 16 == 0 && (uintptr_t)d.cache % 16 == 0) {
         i64h_latent_attn_args a = {};
         a.Q = d.Q, a.cache = d.cache, a.cache_dtype = d.cache_dtype, a.block_table = d.block_table, a.max_blocks_per_seq = d.max_blocks_per_seq;

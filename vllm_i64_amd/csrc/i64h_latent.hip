@@ -1530,7 +1530,7 @@ int i64h_latent_attn(const i64h_latent_attn_args* dp, void* stream) {
     if (d.n == 0) return 0;
     const int D = d.kv_rank + d.rot_dim;
     const bool mfma_ok = d.cache_dtype == 2 && D % 8 == 0 && d.kv_rank % 16 == 0 && d.kv_rank <= 16 * LT_NB && D <= 32 * LT_KD &&
-                         (uintptr_t)d.Q % 16 == 0 && (uintptr_t)d.cache % 16 == 0 && d.row_stride % 8 == 0 && (d.mode == 3 || g_decode_form);
+                         (uintptr_t)d.Q % 16 == 0 && (uintptr_t)d.cache % 16 == 0 && d.row_stride % 8 == 0 && (d.mode == 3 || g_decode_form || d.out16);
     I64H_CHECK_ARG(mfma_ok || (d.kv_groups <= 1 && d.row_stride <= 0 && d.chunk <= 0 && !d.kscale && !d.bias),
                    "latent_attn: key heads, chunks, key scales and bias are built for the matrix-core form only");
     I64H_CHECK_ARG(!d.sink_w || d.sink, "latent_attn: sink scores without the sink");
