@@ -147,3 +147,30 @@ def test_row_gates_over_rounded_rows(dev, M, K):
     ref = torch.matmul(a.double().transpose(0, 1), w.double().transpose(1, 2)).transpose(0, 1) * torch.sigmoid(e[:, 1:1 + H].double())[..., None]
     # K exact products summed in 32 bits: at most K 2^-24 of the sum of their magnitudes, below 6 sqrt(K)
     assert float((wide.view(M, H, N) - ref).abs().max()) <= K * 2.0 ** -24 * 6 * K ** 0.5 + 1e-5 and torch.equal(wide16, wide.bfloat16())
+
+
+@pytest.mark.parametrize("M,N,pad", [(66, 8, 8), (65, 72, 4), (193, 132, 12), (257, 264, 8), (300, 384, 0)])
+def test_lines_of_results(dev, form, M, N, pad):
+    """Results that go out as whole lines: ends in rows and columns, both widths of a store, in fp32, in bf16 and in both; row gates, a bias, a pair; two batches beside
+    each other.  What lies between the batches' columns and behind the rows stays."""
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator().manual_seed(M + N)
+    B, K, W = 2, 128, N + pad
+    a = torch.randn(M, B * K, generator=g).bfloat16().to(dev)
+    w = (torch.randn(B, 2 * N, K, generator=g) / 8).bfloat16().to(dev)
+    e, bias = torch.randn(M, B, generator=g).to(dev), torch.randn(B, N, generator=g).to(dev)
+    x = a.view(M, B, K).double().transpose(0, 1)
+    first, second = torch.matmul(x, w[:, :N].double().transpose(1, 2)), torch.matmul(x, w[:, N:].double().transpose(1, 2))
+    for opts, ref in ((dict(epilogue=D.EPI_ROW_SIGMOID, e=e, lde=B, e_batch=1, bias=bias, bias_batch=N), (first + bias[:, None].double()) * torch.sigmoid(e.double()).T[..., None]),
+                      (dict(epilogue=D.EPI_SILU_MUL), first * torch.sigmoid(first) * second)):
+        kw = dict(m=M, n=N, k=K, lda=B * K, ldc=B * W, batch=B, a_batch=K, w_batch=2 * N * K, c_batch=W, a16=a, **opts)
+        out, out16 = torch.full((M + 1, B * W), 7.0, device=dev), torch.full((M + 1, B * W), 7.0, device=dev, dtype=torch.bfloat16)
+        D.linear(None, w, out, out16=out16, **kw)
+        alone, alone16 = torch.full_like(out, 7.0), torch.full_like(out16, 7.0)
+        D.linear(None, w, alone, **kw)
+        D.linear(None, w, None, out16=alone16, **kw)
+        got = out[:M].view(M, B, W)
+        # (the products below 64: their rounding through two factors)
+        assert float((got[:, :, :N].transpose(0, 1) - ref).abs().max()) <= 64 * K * 2.0 ** -24
+        assert bool((got[:, :, N:] == 7).all()) and bool((out[M] == 7).all())
+        assert torch.equal(out16, out.bfloat16()) and torch.equal(alone, out) and torch.equal(alone16, out16)

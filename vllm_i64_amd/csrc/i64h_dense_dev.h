@@ -18,6 +18,16 @@ __device__ __forceinline__ uint32_t dn_bf16_pair(float a, float b) {
 }
 __device__ __forceinline__ float dn_bf16_to_f32(uint32_t h) { return __uint_as_float(h << 16); }
 __device__ __forceinline__ float dn_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
+// x sigmoid(z) = x / (1 + e^-z), z a multiple of x (so a NaN is in x already): e^-z = 2^n 2^f with f at most half, log2(e) in two parts, from the native base-2
+// exponential; the quotient from a native reciprocal and its own remainder, one rounding less than by way of 1 / (1 + e^-z).  Against 64 bits, times another factor:
+// 2.05e-7 of the result at most and 4.6e-8 on average over z of +- 20, 2.15e-7 and 5.0e-8 with expf and a division, in 15 instructions for 27.  (The ends of the range
+// are where 1 + e^-z is 1 or its reciprocal below the smallest normal number; no remainder of an infinite x is let in.)
+__device__ __forceinline__ float dn_gated(float x, float z) {
+    const float c = __builtin_amdgcn_fmed3f(z, -88.0f, 88.0f), n = __builtin_rintf(c * -1.44269504f);
+    const float f = __builtin_fmaf(c, -1.92596299e-8f, __builtin_fmaf(c, -1.44269504f, -n));
+    const float d = 1.0f + __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)n), y = __builtin_amdgcn_rcpf(d), q = x * y;
+    return __builtin_fmaf(fmaxf(__builtin_fmaf(-d, q, x), -3.4e38f), y, q);
+}
 __device__ __forceinline__ float dn_gelu_tanh(float z) {
     const float inner = 0.7978845608028654f * (z + 0.044715f * z * z * z);
     return 0.5f * z * (1.0f + tanhf(inner));
@@ -45,10 +55,10 @@ __device__ __forceinline__ float dn_epilogue(const i64h_linear& p, float acc, fl
         acc *= s, acc2 *= s;
     }
     if (EPI == I64H_EPI_GELU_MUL) return dn_gelu_tanh(acc) * acc2;
-    if (EPI == I64H_EPI_SILU_MUL) return acc * dn_sigmoid(acc) * acc2;
+    if (EPI == I64H_EPI_SILU_MUL) return dn_gated(acc, acc) * acc2;
     if (EPI == I64H_EPI_CLAMP_GLU) {
         const float u = fminf(acc, p.act_b), w = fminf(fmaxf(acc2, -p.act_b), p.act_b);
-        return u * dn_sigmoid(p.act_a * u) * (w + 1.0f);
+        return dn_gated(u, p.act_a * u) * (w + 1.0f);
     }
     if (p.bias) acc += p.bias[b * p.bias_batch + c];
     if (EPI == I64H_EPI_XIELU) return dn_xielu(acc, p.act_a, p.act_b);

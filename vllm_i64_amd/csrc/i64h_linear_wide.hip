@@ -7,17 +7,17 @@
 // stage is small enough (512 x 2048 x 5504 in 64 x 64 tiles: 41.8 us with two stages, 24.7 with three, 21.6 with four).  Microseconds in replayed
 // graphs, the weights of eight launches in turn:
 //   rows x columns x k            rounded while staged   256x256  256x128  192x128  128x128  64x128  64x64
-//   4096 x 5760 x 1024                  92                  62       56       54       55      69      82
-//   4096 x 1024 x 1024                  20                  28       18       18       16      15      17
-//   4096 x 2752 x 1024, pair            77                  60       52       50       53      59      70
-//   2956 x 8352 x 2048                 168                 109      111      112      115     135     156
-//   2956 x 5504 x 2048, pair           197                 154      140      133      147     166     196
-//   2956 x 2048 x 5504                 123                 114       66       75       72      84     102
-//   8 batches, 5912 x 2048 x 1792       95                  55       63       75       71      78      90
-//    512 x 5504 x 2048, pair            50                  54       32       40       39      42      48
-//    512 x 2048 x 2048                  13.5                41       23       25       22      13       9.4
-//    200 x 5760 x 1024                  13.3                26       15       16       14       9.4     9.9
-//     77 x 1024 x 1024                   5.9                21       13       12       10       7.3     5.6
+//   4096 x 5760 x 1024                  92                  60       59       52       55      67      80
+//   4096 x 1024 x 1024                  20                  27       18       18       16      15      17
+//   4096 x 2752 x 1024, pair            77                  55       52       48       50      58      77
+//   2956 x 8352 x 2048                 168                  98      113      106      114     128     149
+//   2956 x 5504 x 2048, pair           197                 142      140      124      137     150     184
+//   2956 x 2048 x 5504                 123                 100       62       73       70      79     101
+//   8 batches, 5912 x 2048 x 1792       95                  55       61       64       70      73      86
+//    512 x 5504 x 2048, pair            50                  42       26       36       28      30      36
+//    512 x 2048 x 2048                  13.5                39       22       25       22      13       9.5
+//    200 x 5760 x 1024                  13.3                24       15       16       14       9.1     9.8
+//     77 x 1024 x 1024                   5.9                23       14       12       10       7.1     5.5
 // Wider shares of a tile for a wave cost LDS reads the least (a 64 x 64 share reads as many bytes of LDS a cycle as the products take), so the large
 // tiles win as soon as their rounds fill the chip.
 #include "i64h_dense_dev.h"
@@ -28,6 +28,8 @@
 __device__ __forceinline__ void dn_load_lds(__amdgpu_buffer_rsrc_t r, uint16_t* lds, uint32_t lane_bytes, uint32_t step_bytes) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, lane_bytes, step_bytes, 0, 0);
 }
+
+constexpr uint32_t DN_STORE_END = 0x7fffff00u;      // offsets from here on are not stored
 
 template <bool DUAL, int BM, int BN, int NWM, int NWN, int NS, int PER_CU>
 __global__ __launch_bounds__(64 * NWM * NWN, PER_CU * NWM * NWN / 4) void linear_wide_kernel(const i64h_linear p, const int n_tiles, const int m_tiles, const int vecC) {
@@ -172,32 +174,117 @@ __global__ __launch_bounds__(64 * NWM * NWN, PER_CU * NWM * NWN / 4) void linear
     if constexpr (NS > 3)
         if (kt + 2 < KT) step(kt + 2, S2, S3);
     __builtin_amdgcn_s_waitcnt(0x0f70);      // (nothing is on its way into LDS when the workgroup ends)
-    // the weights are the left operand: a lane holds four neighbouring columns of a row
+    // The weights are the left operand: a lane holds four neighbouring columns of a row, a block of 16 rows 64 bytes (bf16: 32) of each.  Stored so, half or a
+    // quarter of a line at a time, a round of 256 x 256 tiles took 10.5 us to end, in fp32 and in bf16 alike: the lines, not the bytes.  So 16 rows at a time pass
+    // through LDS of the wave's own and leave as whole lines.  What a launch may have or not (a bias, factors of the rows) is asked once, not at every value, and rows and
+    // columns past the end are stored where the buffer ends.  8192 x 2048 x 64 in 256 x 256 / 128 x 128 tiles, us: fp32 16.8 / 20.4 -> 15.6 / 17.8 (67 MB), bf16
+    // 16.1 / 16.4 -> 11.9 / 12.9; a pair to bf16, 8192 x 896 x 64, 16.2 / 17.1 -> 12.4 / 13.5 (9.9 of it without the activation); 4096 x 5760 x 1024 in 192 x 128 tiles
+    // 53.5 -> 50, as a pair of 2752 51.5 -> 46.
+    constexpr int FO = DUAL ? FN / 2 : FN;      // blocks of output columns
     auto finish = [&](auto epi, auto vec) {      // (vec: a lane's four columns at a time)
         constexpr int EPI = decltype(epi)::value;
+        int at_lane = lane, at_row = wm * WM, at_col = wn * (COLS / NWN);
+        asm volatile("" : "+v"(at_lane), "+s"(at_row), "+s"(at_col));      // (nothing of what follows is worked out, and kept, ahead of the loop, nor shared with its addresses)
+        const int c0 = at_col + (at_lane >> 4) * 4, r0 = at_row + (at_lane & 15);      // this lane's first column and row in the tile
+        if constexpr (decltype(vec)::value) {
+            i64h_linear q = p;      // (what the values below have already)
+            q.bias = nullptr, q.row_scale = nullptr;
+            float add[DUAL ? 1 : FO][4];
+            if constexpr (!DUAL) {
 #pragma unroll
-        for (int i = 0; i < FM; ++i) {
-            const int rl = wm * WM + i * 16 + fr;
-            if (rl >= M) continue;
-            const int64_t r = m0 + rl, row = b * p.c_batch + r * p.ldc;
+                for (int j = 0; j < FO; ++j)
 #pragma unroll
-            for (int j = 0; j < (DUAL ? FN / 2 : FN); ++j) {
-                const int c = n0 + wn * (COLS / NWN) + j * 16 + fk * 4;
-                auto out = [&](int g) { return dn_epilogue<EPI>(p, acc[i][j][g], DUAL ? acc[i][DUAL ? j + FN / 2 : j][g] : 0.0f, b, r, c + g); };
-                if constexpr (decltype(vec)::value) {
-                    if (c >= N) continue;
-                    const float4 v = make_float4(out(0), out(1), out(2), out(3));
-                    if (p.C16) *(uint2*)((uint16_t*)p.C16 + row + c) = make_uint2(dn_bf16_pair(v.x, v.y), dn_bf16_pair(v.z, v.w));
-                    if (p.C) *(float4*)(p.C + row + c) = v;
-                } else {
+                    for (int g = 0; g < 4; ++g) add[j][g] = -0.0f;      // (changes no value, not even a zero's sign)
+                if (p.bias) {
+#pragma unroll
+                    for (int j = 0; j < FO; ++j)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) add[j][g] = p.bias[b * p.bias_batch + min(n0 + c0 + j * 16 + g, N - 1)];
+                }
+            }
+            // 16 rows at a time through LDS of the wave's own, so that a store takes whole lines
+            constexpr int OC = FO * 16, PITCH = OC + 4;
+            static_assert(NW * 16 * PITCH * 4 <= STAGE * 2, "");
+            float* const own = (float*)s0 + wid * 16 * PITCH;
+            const int64_t at = b * p.c_batch + m0 * p.ldc + n0;
+            const __amdgpu_buffer_rsrc_t buf = __builtin_amdgcn_make_buffer_rsrc(p.C + at, 0, (int)DN_STORE_END, 0x00020000);
+            const __amdgpu_buffer_rsrc_t buf16 = __builtin_amdgcn_make_buffer_rsrc((uint16_t*)p.C16 + at, 0, (int)DN_STORE_END, 0x00020000);
+            const bool eight = ((N | (int)p.ldc | (int)p.c_batch) & 7) == 0;
+            const int cw = at_col, ldc = (int)p.ldc;
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < FM; ++i) {
+                const int64_t r = m0 + min(r0 + i * 16, M - 1);
+                if (DUAL && p.row_scale) {
+                    const float factor = p.row_scale[r];
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) acc[i][j] *= factor;
+                }
+                float gate = 1.0f;
+                if constexpr (EPI == I64H_EPI_ROW_SIGMOID) gate = dn_sigmoid(p.E[b * p.e_batch + r * p.lde]);
+#pragma unroll
+                for (int j = 0; j < FO; ++j) {
+                    const int c = min(n0 + c0 + j * 16, N - 4);
+                    dn_v4f o;
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
-                        if (c + g >= N) continue;
-                        const float v = out(g);
-                        if (p.C16) ((uint16_t*)p.C16)[row + c + g] = (uint16_t)dn_bf16_rne(v);
-                        if (p.C) p.C[row + c + g] = v;
+                        if constexpr (DUAL) o[g] = dn_epilogue<EPI>(q, acc[i][j][g], acc[i][j + FN / 2][g], b, r, c + g);
+                        else if constexpr (EPI == I64H_EPI_ROW_SIGMOID) o[g] = (acc[i][j][g] + add[j][g]) * gate;
+                        else o[g] = dn_epilogue<EPI>(q, acc[i][j][g] + add[j][g], 0.0f, b, r, c + g);
+                    }
+                    *(dn_v4f*)&own[(at_lane & 15) * PITCH + j * 16 + (at_lane >> 4) * 4] = o;
+                }
+                const int r1 = at_row + i * 16;
+                if (p.C16) {
+                    if (eight) {
+#pragma unroll
+                        for (int t = 0; t < (FO + 1) / 2; ++t) {
+                            const int e = t * 64 + at_lane, row = e / (OC / 8), c = e % (OC / 8) * 8;
+                            const dn_v4f x = *(const dn_v4f*)&own[min(row, 15) * PITCH + c], y = *(const dn_v4f*)&own[min(row, 15) * PITCH + c + 4];
+                            const uint32_t off = r1 + row < M && row < 16 && n0 + cw + c < N ? (uint32_t)((r1 + row) * ldc + cw + c) * 2 : DN_STORE_END;
+                            __builtin_amdgcn_raw_buffer_store_b128(dn_v4u{dn_bf16_pair(x[0], x[1]), dn_bf16_pair(x[2], x[3]), dn_bf16_pair(y[0], y[1]), dn_bf16_pair(y[2], y[3])}, buf16, off, 0, 0);
+                        }
+                    } else {
+#pragma unroll
+                        for (int t = 0; t < FO; ++t) {
+                            const int e = t * 64 + at_lane, row = e / (OC / 4), c = e % (OC / 4) * 4;
+                            const dn_v4f x = *(const dn_v4f*)&own[row * PITCH + c];
+                            const uint32_t off = r1 + row < M && n0 + cw + c < N ? (uint32_t)((r1 + row) * ldc + cw + c) * 2 : DN_STORE_END;
+                            __builtin_amdgcn_raw_buffer_store_b64(dn_v2u{dn_bf16_pair(x[0], x[1]), dn_bf16_pair(x[2], x[3])}, buf16, off, 0, 0);
+                        }
                     }
                 }
+                if (p.C) {
+#pragma unroll
+                    for (int t = 0; t < FO; ++t) {
+                        const int e = t * 64 + at_lane, row = e / (OC / 4), c = e % (OC / 4) * 4;
+                        const dn_v4f x = *(const dn_v4f*)&own[row * PITCH + c];
+                        const uint32_t off = r1 + row < M && n0 + cw + c < N ? (uint32_t)((r1 + row) * ldc + cw + c) * 4 : DN_STORE_END;
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(dn_v4u, x), buf, off, 0, 0);
+                    }
+                }
+                if (i + 1 < FM) {      // (a row's work at a time: the registers are full)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) asm volatile("" : "+v"(acc[i + 1 < FM ? i + 1 : i][j]));
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < FM; ++i) {
+                const int rl = r0 + i * 16;
+                if (rl >= M) continue;
+                const int64_t r = m0 + rl, row = b * p.c_batch + r * p.ldc;
+#pragma unroll
+                for (int j = 0; j < FO; ++j)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        const int c = n0 + c0 + j * 16 + g;
+                        if (c >= N) continue;
+                        const float v = dn_epilogue<EPI>(p, acc[i][j][g], DUAL ? acc[i][DUAL ? j + FN / 2 : j][g] : 0.0f, b, r, c);
+                        if (p.C16) ((uint16_t*)p.C16)[row + c] = (uint16_t)dn_bf16_rne(v);
+                        if (p.C) p.C[row + c] = v;
+                    }
             }
         }
     };
@@ -220,7 +307,7 @@ static void launch(const i64h_linear& d, hipStream_t s) {
         const int64_t most = mt * d.batch;
         mt = d.rows_total > 0 ? (most < d.rows_total / BM + d.batch ? most : d.rows_total / BM + d.batch) : most;
     }
-    const int vecC = ((uintptr_t)d.C | (uintptr_t)d.C16) % 16 == 0 && d.ldc % 4 == 0 && d.c_batch % 4 == 0 && d.N % 4 == 0;
+    const int vecC = ((uintptr_t)d.C | (uintptr_t)d.C16) % 16 == 0 && d.ldc % 4 == 0 && d.c_batch % 4 == 0 && d.N % 4 == 0 && d.ldc < (DN_STORE_END / 4 - 256) / 256;
     const dim3 grid((unsigned)(mt * nt), 1, d.group_off ? 1u : (unsigned)d.batch);
     if (dual) hipLaunchKernelGGL((linear_wide_kernel<true, BM, BN, NWM, NWN, NS, PER_CU>), grid, dim3(64 * NWM * NWN), 0, s, d, nt, (int)mt, vecC);
     else hipLaunchKernelGGL((linear_wide_kernel<false, BM, BN, NWM, NWN, NS, PER_CU>), grid, dim3(64 * NWM * NWN), 0, s, d, nt, (int)mt, vecC);
