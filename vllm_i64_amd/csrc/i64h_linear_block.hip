@@ -206,11 +206,32 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
     }
     // the weights are the left operand: a lane holds four neighbouring columns of a row
     float* C = p.C + b * p.c_batch;
+    // (a bias and factors of rows are asked for once, not at every value)
+    i64h_linear q = p;
+    q.bias = nullptr, q.row_scale = nullptr;
+    float add[DUAL ? 1 : FN][4];
+    if constexpr (!DUAL) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) add[j][g] = -0.0f;      // (changes no value, not even a zero's sign)
+        if (p.bias) {
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) add[j][g] = p.bias[b * p.bias_batch + min(n0 + wn * (COLS / NWN) + j * 16 + fk * 4 + g, N - 1)];
+        }
+    }
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
         const int rl = wm * WM + i * 16 + fr;
         if (rl >= M) continue;
         const int64_t r = m0 + rl;
+        if (DUAL && p.row_scale) {
+            const float factor = p.row_scale[r];
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] *= factor;
+        }
         float f = 1.0f;
         if (INN) {
             float q = 0.0f;
@@ -221,7 +242,7 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
 #pragma unroll
         for (int j = 0; j < (DUAL ? FN / 2 : FN); ++j) {
             const int c = n0 + wn * (COLS / NWN) + j * 16 + fk * 4;
-            auto out = [&](int g) { return dn_epilogue<EPI>(p, INN ? acc[i][j][g] * f : acc[i][j][g], DUAL ? acc[i][DUAL ? j + FN / 2 : j][g] : 0.0f, b, r, c + g); };
+            auto out = [&](int g) { return DUAL ? dn_epilogue<EPI>(q, acc[i][j][g], acc[i][DUAL ? j + FN / 2 : j][g], b, r, c + g) : dn_epilogue<EPI>(q, (INN ? acc[i][j][g] * f : acc[i][j][g]) + add[DUAL ? 0 : j][g], 0.0f, b, r, c + g); };
             float* dst = C + r * p.ldc + c;
             if (vecC && c + 4 <= N) {
                 *(float4*)dst = make_float4(out(0), out(1), out(2), out(3));
