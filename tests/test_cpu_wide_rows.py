@@ -32,3 +32,13 @@ def test_pairs_of_a_plan_without_a_shared_group():
 def test_experts_of_a_few_rows_each():
     fills = HybridRunner._fills
     assert fills(2, 8) and fills(8 * 40, 8) and not fills(319, 16) and fills(320, 16) and not fills(2 * 500, 64) and fills(8 * 200, 64)
+
+
+def test_steps_of_few_rows_round_as_well():
+    """From three rows on, where the sizes allow what the wide tiles need; a runner of 32-bit products never."""
+    r = runner(5504)
+    assert not r._rounded(2, 2048) and r._rounded(3, 2048) and r._rounded(64, 2048) and r._rounded(65, 2048)
+    assert not r._rounded(7, 2048, 2050) and not runner(5504, True)._rounded(7, 2048)
+    for n in (65, 100, (1 << 20) - 1, 1 << 20):
+        assert r._rounded(n, 2048) == r._wide(n, 2048) and runner(1 << 20)._rounded(n, 2048) == runner(1 << 20)._wide(n, 2048)
+    assert not runner(1 << 20)._rounded(7, 2048)

@@ -174,3 +174,50 @@ def test_lines_of_results(dev, form, M, N, pad):
         assert float((got[:, :, :N].transpose(0, 1) - ref).abs().max()) <= 64 * K * 2.0 ** -24
         assert bool((got[:, :, N:] == 7).all()) and bool((out[M] == 7).all())
         assert torch.equal(out16, out.bfloat16()) and torch.equal(alone, out) and torch.equal(alone16, out16)
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64, 65, 128, 150])
+@pytest.mark.parametrize("N,K,B", [(16, 64, 1), (60, 256, 3), (130, 320, 1), (256, 1088, 2), (36, 2752, 1)])
+def test_steps_of_k_dealt_to_waves(dev, M, N, K, B):
+    """16 columns a workgroup, fewer and more steps of k than waves and stages, ends in rows and columns, one to three tiles of rows, batches; every epilogue, both results;
+    and by size the same bits where the rule says so."""
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator().manual_seed(M + N + K)
+    W = N + 4
+    a = torch.randn(M, B * K + 8, generator=g).bfloat16().to(dev)
+    w = (torch.randn(B, N, K, generator=g) / math.sqrt(K)).bfloat16().to(dev)
+    e, gate, bias = torch.randn(M, B * N, generator=g).to(dev), torch.randn(M, B, generator=g).to(dev), torch.randn(B, N, generator=g).to(dev)
+    ref = torch.matmul(a[:, 8:].double().view(M, B, K).transpose(0, 1), w.double().transpose(1, 2)) + bias[:, None].double()
+    kw = dict(m=M, n=N, k=K, a_off=8, lda=B * K + 8, ldc=B * W, batch=B, a_batch=K, w_batch=N * K, c_batch=W, bias=bias, bias_batch=N, a16=a)
+    for opts, want in ((dict(), ref), (dict(epilogue=D.EPI_SCALE, scale=0.5), 0.5 * ref), (dict(epilogue=D.EPI_ADD, e=e, lde=B * N, e_batch=N), ref + e.double().view(M, B, N).transpose(0, 1)),
+                       (dict(epilogue=D.EPI_ROW_SIGMOID, e=gate, lde=B, e_batch=1), ref * torch.sigmoid(gate.double()).T[..., None])):
+        out, out16 = torch.full((M + 1, B * W), 7.0, device=dev), torch.full((M + 1, B * W), 7.0, device=dev, dtype=torch.bfloat16)
+        D.call_dense("i64h_set_linear_skinny", 112)
+        try:
+            D.linear(None, w, out, out16=out16, **kw, **opts)
+        finally:
+            D.call_dense("i64h_set_linear_skinny", 3)
+        got = out[:M].view(M, B, W)
+        # (K products of about 1 / sqrt(K), their sum and what is added below 16: a rounding of 2^-24 each)
+        assert float((got[:, :, :N].transpose(0, 1) - want).abs().max()) <= 2e-6 * K ** 0.5 + 1e-5
+        assert bool((got[:, :, N:] == 7).all()) and bool((out[M] == 7).all()) and torch.equal(out16, out.bfloat16())
+        if M <= 128 and K >= 256:
+            sized = torch.full_like(out, 7.0)
+            D.linear(None, w, sized, **kw, **opts)
+            assert torch.equal(sized, out)
+
+
+def test_rows_past_a_tiles_end(dev):
+    """Infinities and NaN in rows behind a batch's last are none of its business."""
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator().manual_seed(0)
+    a = torch.randn(40, 256, generator=g).bfloat16()
+    a[7:9] = float("nan")
+    a[39] = float("inf")
+    w = torch.randn(3, 128, 256, generator=g).bfloat16().to(dev)
+    off = torch.tensor([0, 7, 9, 39], dtype=torch.int32, device=dev)
+    out = torch.zeros(40, 128, device=dev)
+    D.linear(None, w, out, a16=a.to(dev), m=40, batch=3, w_batch=128 * 256, group_off=off)
+    assert torch.isfinite(out[:7]).all() and torch.isfinite(out[9:39]).all() and not torch.isfinite(out[7:9]).any() and not out[39].any()
+    few = D.linear(None, w[0], torch.empty(7, 128, device=dev), a16=a[:7].to(dev))
+    assert torch.isfinite(few).all()

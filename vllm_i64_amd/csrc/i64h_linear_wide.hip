@@ -54,9 +54,9 @@ __global__ __launch_bounds__(64 * NWM * NWN, PER_CU * NWM * NWN / 4) void linear
     const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 16;
     uint32_t oa[LA], ow[LB];
 #pragma unroll
-    for (int i = 0; i < LA; ++i) {      // (rows past the end repeat the last one and are not stored)
-        const int r = min((i * NW + wid) * 8 + lr, M - 1);
-        oa[i] = (uint32_t)((p.a_rows ? p.a_rows[m0 + r] : r) * p.lda) * 2u + lc;
+    for (int i = 0; i < LA; ++i) {      // (rows past the end are zeros that nobody asks memory for, and are not stored)
+        const int r = (i * NW + wid) * 8 + lr, at = min(r, M - 1);
+        oa[i] = r < M ? (uint32_t)((p.a_rows ? p.a_rows[m0 + at] : at) * p.lda) * 2u + lc : DN_BUF_END;
     }
 #pragma unroll
     for (int i = 0; i < LB; ++i) {
@@ -313,6 +313,151 @@ static void launch(const i64h_linear& d, hipStream_t s) {
     else hipLaunchKernelGGL((linear_wide_kernel<false, BM, BN, NWM, NWN, NS, PER_CU>), grid, dim3(64 * NWM * NWN), 0, s, d, nt, (int)mt, vecC);
 }
 
+// ---- up to 64 rows under few columns: 16 columns a workgroup, the steps of k dealt to its waves ------------------------------------------------
+// What bounds it: the latency of a step, a few of them on their way.  A 64 x 64 tile walks all of k alone, and 1024 or 2048 columns are 16 or 32 of them on 256 CUs.
+// Here every wave takes every NW-th step of 64 k for 16 columns and all rows, with loads, LDS and waits of its own: nobody meets before the end, where the waves' sums
+// are added in their order.  The rows are read once for 16 columns, from L2: at 64 rows of 5504 that is 90 MB, and the launch's time.  Microseconds in replayed graphs, the
+// weights of twelve launches in turn, the fp32 rows' kernels | 64 x 64 tiles | here:
+//   rows:                   3                     16                   64                   77                  128
+//   1024 x 1024     3.5 | 4.9 | 3.5     4.6 | 5.0 | 3.4      5.8 | 5.1 | 4.3      5.7 | 5.1 | 4.5      5.8 | 5.1 | 4.5
+//   1024 x 2752     6.6 | 9.3 | 4.7     9.6 | 9.3 | 5.1      9.4 | 10.5 | 7.6     9.3 | 9.4 | 6.9      9.5 | 10.1 | 7.6
+//   2048 x 2048     5.7 | 7.8 | 4.7     7.9 | 7.8 | 4.8      8.3 | 8.2 | 6.6      8.3 | 7.9 | 6.4      8.5 | 8.2 | 6.9
+//   2048 x 5504     11.8 | 21.6 | 8.2   23.8 | 22.1 | 9.5    22.5 | 27.1 | 16.6   22.0 | 22.2 | 13.2   22.1 | 25.9 | 16.5
+//   4352 x 2048                         8.4 | 8.1 | 8.4      9.8 | 8.5 | 12.5
+// (more than 256 tiles, the last row: a second round)
+template <int MB, int NW, int NS, int EPI>
+__global__ __launch_bounds__(64 * NW, NW / 4) void linear_thin_kernel(const i64h_linear p, const int vecC) {
+    constexpr int LA = 2 * MB, LB = 2, ROWS = 16 * MB + 16, STAGE = NW * ROWS * 64;      // loads a step: eight rows of 64 values each
+    static_assert(NS == 3 || NS == 4, "");
+    __shared__ __attribute__((aligned(1024))) uint16_t s0[STAGE], s1[STAGE], s2[STAGE], s3[NS > 3 ? STAGE : 8];
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int N = p.N, K = p.K, KT = K / 64;
+    const int n0 = blockIdx.x * 16;
+    const int64_t b = blockIdx.z, m0 = (int64_t)blockIdx.y * (16 * MB);
+    const int M = (int)min((int64_t)16 * MB, p.M - m0);
+    const uint16_t *baseA = (const uint16_t*)p.A16 + b * p.a_batch + m0 * p.lda, *baseW = (const uint16_t*)p.W + b * p.w_batch + (int64_t)n0 * K;
+    const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 16;      // (chunks permuted per row, as above)
+    uint32_t oa[LA], ow[LB];
+#pragma unroll
+    for (int i = 0; i < LA; ++i) oa[i] = i * 8 + lr < M ? (uint32_t)((i * 8 + lr) * p.lda) * 2u + lc : DN_BUF_END;
+#pragma unroll
+    for (int i = 0; i < LB; ++i) ow[i] = (uint32_t)(min(i * 8 + lr, N - 1 - n0) * K) * 2u + lc;
+    constexpr std::integral_constant<int, 0> S0{};
+    constexpr std::integral_constant<int, 1> S1{};
+    constexpr std::integral_constant<int, 2> S2{};
+    constexpr std::integral_constant<int, 3> S3{};
+    auto stage = [&](auto set) -> uint16_t* {
+        constexpr int S = decltype(set)::value;
+        return (S == 0 ? s0 : S == 1 ? s1 : S == 2 ? s2 : s3) + wid * ROWS * 64;
+    };
+    auto load = [&](int t, auto set) {      // (a step past the end asks for nothing: a buffer of no bytes)
+        const int kt = t * NW + wid;
+        uint16_t* sm = stage(set);
+        const uint32_t bytes = kt < KT ? DN_BUF_END : 0u;
+        const __amdgpu_buffer_rsrc_t bufA = __builtin_amdgcn_make_buffer_rsrc((void*)baseA, 0, (int)bytes, 0x00020000), bufW = __builtin_amdgcn_make_buffer_rsrc((void*)baseW, 0, (int)bytes, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < LB; ++i) dn_load_lds(bufW, sm + (16 * MB + i * 8) * 64, ow[i], kt * 128);
+#pragma unroll
+        for (int i = 0; i < LA; ++i) dn_load_lds(bufA, sm + i * 512, oa[i], kt * 128);
+    };
+    dn_v4f acc[MB];
+#pragma unroll
+    for (int i = 0; i < MB; ++i) acc[i] = dn_v4f{0, 0, 0, 0};
+    const int fr = lane & 15, fk = lane >> 4;
+    auto step = [&](int t, auto cur) {
+        constexpr int LEFT = (NS - 1) * (LA + LB);
+        static_assert(LEFT < 64, "");
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0f70 | (LEFT & 15) | (LEFT >> 4) << 14);      // this step's loads are in LDS (the wave's own)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        const uint16_t* sm = stage(cur);
+        dn_v4u a[2][MB], w[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int ch = ((h * 4 + fk) ^ (fr & 7)) << 3;
+            w[h] = *(const dn_v4u*)&sm[(16 * MB + fr) * 64 + ch];
+#pragma unroll
+            for (int i = 0; i < MB; ++i) a[h][i] = *(const dn_v4u*)&sm[(i * 16 + fr) * 64 + ch];
+        }
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt 0: they are in registers, the place is free
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        load(t + NS, cur);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int i = 0; i < MB; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_v8bf, w[h]), __builtin_bit_cast(dn_v8bf, a[h][i]), acc[i], 0, 0, 0);
+    };
+    load(0, S0);
+    load(1, S1);
+    load(2, S2);
+    if constexpr (NS > 3) load(3, S3);
+    const int T = (KT + NW - 1) / NW;
+    int t = 0;
+    for (; t + NS <= T; t += NS) {
+        step(t, S0);
+        step(t + 1, S1);
+        step(t + 2, S2);
+        if constexpr (NS > 3) step(t + 3, S3);
+    }
+    if (t < T) step(t, S0);
+    if (t + 1 < T) step(t + 1, S1);
+    if constexpr (NS > 3)
+        if (t + 2 < T) step(t + 2, S2);
+    __builtin_amdgcn_s_waitcnt(0x0f70);      // (nothing is on its way into LDS)
+    __syncthreads();
+    // the waves' sums meet in LDS; wave i adds those of rows 16 i .. in the waves' order
+    dn_v4f* sum = (dn_v4f*)s0;
+    static_assert(NW * MB * 64 * 16 <= STAGE * 2 && MB <= NW, "");
+#pragma unroll
+    for (int i = 0; i < MB; ++i) sum[(wid * MB + i) * 64 + lane] = acc[i];
+    __syncthreads();
+    if (wid >= MB) return;
+    dn_v4f o = sum[wid * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) o += sum[(w * MB + wid) * 64 + lane];
+    const int c = n0 + fk * 4;
+    if (wid * 16 + fr >= M) return;
+    const int64_t r = m0 + wid * 16 + fr;
+    const int64_t at = b * p.c_batch + r * p.ldc + c;
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+        if (c + g < N) o[g] = dn_epilogue<EPI>(p, o[g], 0.0f, b, r, c + g);
+    if (vecC && c < N) {
+        if (p.C16) *(uint2*)((uint16_t*)p.C16 + at) = make_uint2(dn_bf16_pair(o[0], o[1]), dn_bf16_pair(o[2], o[3]));
+        if (p.C) *(dn_v4f*)(p.C + at) = o;
+        return;
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        if (c + g >= N) continue;
+        if (p.C16) ((uint16_t*)p.C16)[at + g] = (uint16_t)dn_bf16_rne(o[g]);
+        if (p.C) p.C[at + g] = o[g];
+    }
+}
+
+static bool thin_fits(const i64h_linear& d) {
+    return !dn_dual(d.epilogue) && !d.a_rows && !d.group_off && d.batch <= 65535 && d.M <= 64 * 65535;
+}
+template <int EPI>
+static void launch_thin(const i64h_linear& d, hipStream_t s) {
+    const int vecC = ((uintptr_t)d.C | (uintptr_t)d.C16) % 16 == 0 && d.ldc % 4 == 0 && d.c_batch % 4 == 0 && d.N % 4 == 0;
+    const dim3 grid((unsigned)((d.N + 15) / 16), (unsigned)((d.M + 63) / 64), (unsigned)d.batch);
+    if (d.M <= 16) hipLaunchKernelGGL((linear_thin_kernel<1, 8, 4, EPI>), grid, dim3(512), 0, s, d, vecC);
+    else if (d.M <= 32) hipLaunchKernelGGL((linear_thin_kernel<2, 8, 3, EPI>), grid, dim3(512), 0, s, d, vecC);
+    else hipLaunchKernelGGL((linear_thin_kernel<4, 4, 3, EPI>), grid, dim3(256), 0, s, d, vecC);
+}
+static void launch_thin(const i64h_linear& d, hipStream_t s) {
+    switch (d.epilogue) {
+        case I64H_EPI_SCALE: launch_thin<I64H_EPI_SCALE>(d, s); break;
+        case I64H_EPI_ADD: launch_thin<I64H_EPI_ADD>(d, s); break;
+        case I64H_EPI_ROW_SIGMOID: launch_thin<I64H_EPI_ROW_SIGMOID>(d, s); break;
+        default: launch_thin<I64H_EPI_STORE>(d, s); break;
+    }
+}
+
 // The form of a launch by what it costs: its workgroups' rounds on the 256 CUs times a round's microseconds, fitted to the measurements above (weights
 // that come from memory: a step is not shorter than the microsecond that its loads take, divided by the steps on their way).
 struct dn_wide_form {
@@ -331,7 +476,11 @@ bool dn_linear_wide(const i64h_linear& d, int form, hipStream_t s) {
     static const dn_wide_form forms[] = {{256, 256, true, 1.3f, 1.3f, 12.0f}, {256, 128, true, 0.72f, 0.72f, 7.0f}, {192, 128, false, 1.0f, 1.7f, 0.0f},
                                          {128, 128, false, 1.0f, 1.2f, 0.0f}, {64, 128, false, 0.5f, 0.75f, 0.0f}, {64, 64, false, 0.33f, 0.4f, 0.0f}};
     constexpr int FORMS = sizeof(forms) / sizeof(forms[0]);
+    // few tiles of 16 columns: one for every CU at most (its LDS holds three or four steps of all its waves)
+    if (form < 0 && thin_fits(d) && d.M <= 128 && d.K >= 256 && (d.M + 63) / 64 * ((d.N + 15) / 16) * d.batch <= 256) form = FORMS;
     if (form < 0) {
+        // (what every form waits for: the weights; of forms that wait no longer than that the largest, which reads the rows least often)
+        const float weights = (float)d.batch * (float)cols * (float)d.K * 2.0f / 4.7e6f;
         float best = 0.0f;
         for (int i = 0; i < FORMS; ++i) {
             const dn_wide_form& f = forms[i];
@@ -340,9 +489,13 @@ bool dn_linear_wide(const i64h_linear& d, int form, hipStream_t s) {
             if (d.group_off && d.rows_total > 0 && d.rows_total / f.BM + (d.batch + 1) / 2 < mt) mt = d.rows_total / f.BM + (d.batch + 1) / 2;
             const float q = (float)(mt * ((cols + f.BN - 1) / f.BN)) / 256.0f;
             const float step = f.alone ? ceilf(q) * f.step : fmaxf(f.first, fmaxf(0.5f * q, q > 1.0f ? 0.75f : 0.0f) * f.step);
-            const float cost = (float)(d.K / 64) * step + (f.alone ? ceilf(q) * f.end : 0.0f);
+            const float cost = fmaxf((float)(d.K / 64) * step + (f.alone ? ceilf(q) * f.end : 0.0f), weights);
             if (i == 0 || cost < best) best = cost, form = i;
         }
+    }
+    if (form == FORMS && thin_fits(d)) {
+        launch_thin(d, s);
+        return true;
     }
     switch (form) {
         case 0: launch<256, 256, 2, 4, 2, 1>(d, s); break;

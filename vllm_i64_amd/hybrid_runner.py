@@ -77,15 +77,29 @@ class HybridRunner:
         """Whether Linears over rows of these widths read them in bf16 (the values their tiles would round to: results are the same)."""
         return not self.exact and n > self.WIDE_ROWS and all(w % 64 == 0 and 2 * w * max(n, self.max_ff + 256) < self.WIDE_BYTES for w in widths)
 
+    FEW_ROWS = 2                    # up to this many rows: the forms that stream the weights past rows in 32 bits
+
+    def _rounded(self, n: int, *widths: int) -> bool:
+        """Whether a step of n rows rounds them where they are written: the wide tiles' rule, and below their rows as well, where the kernels of rows in bf16 are the faster ones
+        from three rows on (64 rows, width 2048, us: 11392 columns 19.4 | 14.8, a pair of 5504 19.0 | 14.5, 2048 columns of 5504 22.5 | 16.6; steps of 64 rows 1608 | 1534, of 7
+        rows and width 1024 526 | 497).  One row under 1024 x 1024 takes 3.0 | 3.4."""
+        if self.exact or n <= self.FEW_ROWS:
+            return False
+        top = 2 * max(n, self.max_ff + 256)
+        for w in widths:      # (asked a few times a layer by steps that wait for the host)
+            if w % 64 or w * top >= self.WIDE_BYTES:
+                return False
+        return True
+
     def _wide_attention(self, n: int, width: int, vals: int, part: int, cache: torch.Tensor) -> bool:
         """Whether an attention over rows of `part` values a key head, the first `vals` of them summed, leaves its result (rows of `width`) in bf16: the matrix-core form
         and Linears that read it so."""
-        return self._wide(n, width) and cache.dtype == torch.bfloat16 and vals % 16 == 0 and vals <= 256 and part % 8 == 0 and part <= 320
+        return self._rounded(n, width) and cache.dtype == torch.bfloat16 and vals % 16 == 0 and vals <= 256 and part % 8 == 0 and part <= 320
 
     @staticmethod
-    def _as16(t: torch.Tensor, n: int, width: int) -> torch.Tensor:
+    def _as16(t16: torch.Tensor, n: int, width: int) -> torch.Tensor:
         """The memory of a buffer of fp32 rows as rows in bf16."""
-        return t.view(torch.bfloat16)[: n * width].view(n, width)
+        return t16[: n * width].view(n, width)
 
     # ---- tensors by name and shape, in the two forms the kernels read ----
     def _bf(self, t: torch.Tensor) -> torch.Tensor:
@@ -131,6 +145,9 @@ class HybridRunner:
         B = self._bufs.pop(key, None)
         if B is None:
             B = type(self).BUFFERS(self, n, m)
+            for name in ("b", "c", "rn", "act", "sact"):      # rows that may be written rounded, in the same memory
+                if hasattr(B, name):
+                    setattr(B, name + "16", getattr(B, name).view(torch.bfloat16))
         self._bufs[key] = B
         loose = [k for k in self._bufs if k not in self._pinned and k != key]
         for k in loose[:max(0, len(loose) + 1 - self.MAX_BUFFER_SETS)]:
@@ -237,7 +254,7 @@ class HybridRunner:
                    slot_ids=slot_ids, block_table=kvc.block_table, cache=rows, q=Q, n=n, norm_heads=a.qk_norm == "head_weight")
         behind = d["v_freq"] is not None or a.head_gate
         wide = not behind and self._wide_attention(n, a.heads * a.vdim, a.vdim, gs, rows)
-        O = self._as16(B.b, n, a.heads * a.vdim) if wide else B.b[: n * a.heads * a.vdim].view(n, a.heads * a.vdim)
+        O = self._as16(B.b16, n, a.heads * a.vdim) if wide else B.b[: n * a.heads * a.vdim].view(n, a.heads * a.vdim)
         self._kattn(B, a, Q, O, rows, kvc, slot_ids, positions, runs, ctx_hint, softcap=a.softcap, window=a.window, keep_first=a.keep_first, sink_w=d.get("sink"))
         if behind:
             D.rot_post(O, heads=a.heads, vdim=a.vdim, interleaved=a.interleaved, v_freq=d["v_freq"], positions=positions,
@@ -285,8 +302,8 @@ class HybridRunner:
                       q_src=src if m.q_rank else None, rot_mult=d["rot_mult"])
         # queries into latent space, per head: Q[:, h, :r] = q_unrotated[:, h, :] @ U_h
         D.linear(src, d["uk_t"], Q, m=n, n=r, k=m.dim, a_off=q_off, lda=src.shape[-1], ldc=H * width, batch=H, a_batch=qh, w_batch=r * m.dim, c_batch=width, exact=ex)
-        wide = self._wide_attention(n, H * r, r, width, cache) and r % 64 == 0 and self._wide(n, H * m.vdim)
-        olat = (B.b.view(torch.bfloat16) if wide else B.b)[: n * H * r]
+        wide = self._wide_attention(n, H * r, r, width, cache) and r % 64 == 0 and self._rounded(n, H * m.vdim)
+        olat = (B.b16 if wide else B.b)[: n * H * r]
         keys = min(ctx_hint, m.window + 64) if m.window > 0 else ctx_hint
         for r0, r1, one_per_seq in runs:
             splits, ws = 1, None
@@ -295,7 +312,7 @@ class HybridRunner:
             D.latent_attn(Q[r0 * H * width: r1 * H * width], cache, kvc.block_table, slot_ids[r0:r1], positions[r0:r1], window=m.window, scale=m.scale, heads=H, kv_rank=r,
                           rot_dim=rd, out=olat[r0 * H * r: r1 * H * r], n=r1 - r0, mode=2 if one_per_seq else 3, splits=splits, workspace=ws, sink=d["sink"])
         # summed latents into value space, per head
-        og = (B.c.view(torch.bfloat16) if wide else B.c)[: n * H * m.vdim]
+        og = (B.c16 if wide else B.c)[: n * H * m.vdim]
         gate = dict(epilogue=D.EPI_ROW_SIGMOID, e=P, e_off=d["g_off"], lde=N1, e_batch=1) if m.head_gate else {}
         maps = dict(m=n, n=m.vdim, k=r, lda=H * r, ldc=H * m.vdim, batch=H, a_batch=r, w_batch=m.vdim * r, c_batch=m.vdim, exact=ex, **gate)
         if wide:
@@ -313,8 +330,8 @@ class HybridRunner:
         rv = r.heads * r.vdim
         F = B.f[: n * r.heads * r.dim].view(n, r.heads * r.dim)
         D.linear(P, d["a2"], F, m=n, a_off=d["a1_off"], exact=self.exact, bias=d["a2_b"], epilogue=D.EPI_DECAY, e=d["a_rate"])
-        wide = self._wide(n, rv)
-        R, Rn, Rn16 = B.r[: n * rv].view(n, rv), None if wide else B.rn[: n * rv].view(n, rv), self._as16(B.rn, n, rv) if wide else None
+        wide = self._rounded(n, rv)
+        R, Rn, Rn16 = B.r[: n * rv].view(n, rv), None if wide else B.rn[: n * rv].view(n, rv), self._as16(B.rn16, n, rv) if wide else None
         D.gla_scan(P, f=F, q_off=d["rq_off"], k_off=d["rk_off"], f_off=0, v_off=d["rv_off"], heads=r.heads, dim=r.dim, vdim=r.vdim, seg_start=seg, nseg=nseg,
                    positions=positions, slot_ids=slot_ids, state=kvc.state[l]["gla"], out=R, n=n, q_scale=r.dim ** -0.5,
                    work=work.get((r.heads, r.dim, r.vdim)))
@@ -345,8 +362,8 @@ class HybridRunner:
         R = B.b[: n * rv].view(n, rv)
         D.gdn_scan(X, G, f=F, seg_start=seg, nseg=nseg, positions=positions, slot_ids=slot_ids, state=st["gdn"], out=R,
                    work=work.get((r.heads, r.dim, r.vdim)), **cols)
-        wide = self._wide(n, rv)
-        Rn, Rn16 = None if wide else B.c[: n * rv].view(n, rv), self._as16(B.c, n, rv) if wide else None
+        wide = self._rounded(n, rv)
+        Rn, Rn16 = None if wide else B.c[: n * rv].view(n, rv), self._as16(B.c16, n, rv) if wide else None
         D.gate_norm(R, d["r_norm"], Rn, groups=r.heads, eps=self.cfg.norm_eps, z=Z, z_off=z_off, ldz=ldz, n=n, gate_after=True, width=rv, sigmoid=r.gate == "sigmoid", out16=Rn16)
         D.linear(Rn, d["o_right"], out, a16=Rn16, exact=ex)
 
@@ -416,16 +433,16 @@ class HybridRunner:
         d["ff_gate_up"] = self._bf(torch.cat([need(p + "gate", (f.ff, W)), need(p + "up", (f.ff, W))], 0))
         d["ff_down"] = self._bf(need(p + "down", (W, f.ff)))
 
-    def _act(self, buf, n: int, width: int, h16):
+    def _act(self, buf, buf16, n: int, width: int, h16):
         """A feed-forward's inner rows: (fp32, bf16), one of them None."""
         if h16 is not None and width % 64 == 0:
-            return None, self._as16(buf, n, width)
+            return None, self._as16(buf16, n, width)
         return buf[: n * width].view(n, width), None
 
     def _dense_glu(self, B, d, n, h, out, h16=None) -> None:
         """h16: the input rows in bf16, read in h's place."""
         f = d["mlp"]
-        act, act16 = self._act(B.act, n, f.ff, h16)
+        act, act16 = self._act(B.act, B.act16, n, f.ff, h16)
         D.linear(h, d["ff_gate_up"], act, a16=h16, out16=act16, exact=self.exact, **self._glu(f.limit, f.glu_alpha))
         D.linear(act, d["ff_down"], out, a16=act16, exact=self.exact)
 
@@ -459,7 +476,7 @@ class HybridRunner:
         shared = None
         if f.shared_ff and not merged:
             with self._beside(n) if beside else nullcontext():
-                sact, sact16 = self._act(B.sact, n, f.shared_ff, h16)
+                sact, sact16 = self._act(B.sact, B.sact16, n, f.shared_ff, h16)
                 D.linear(h, d["s_gate_up"], sact, a16=h16, out16=sact16, exact=ex, **self._glu(f.shared_limit, f.glu_alpha))
                 shared = D.linear(sact, d["s_down"], shared_out, a16=sact16, exact=ex)
         gate_up, e_down = (d["gate_up"], d["e_down"]) if merged or not d["merged"] else (d["gate_up"][1:], d["e_down"][1:])
@@ -473,7 +490,7 @@ class HybridRunner:
         # the (token, expert) pairs lie grouped by expert: one launch runs every expert over its own rows, the counts stay on the device
         x16 = h16 if self._fills(n * top, E) else None
         rows, groups = n * (top + int(merged)), E + int(merged)
-        act, act16 = self._act(B.act, rows, f.ff, x16)
+        act, act16 = self._act(B.act, B.act16, rows, f.ff, x16)
         D.linear(h, gate_up, act, a16=x16, out16=act16, m=n, a_rows=B.pair_token[:rows], batch=groups, w_batch=2 * f.ff * W, exact=ex, group_off=B.group_off, row_scale=pair_wgt,
                  **self._glu(f.limit, f.glu_alpha))
         D.linear(act, e_down, B.ey[:rows], a16=act16, m=n, batch=groups, w_batch=W * f.ff, exact=ex, group_off=B.group_off)

@@ -40,7 +40,7 @@ class _StepBuffers:
         self.e = torch.empty(1, n, W, **f32)                    # embedding rows
         self.x0 = torch.empty(n, W, **f32) if model.cfg.loop is not None else None    # the embedding output's part of what a pass starts from
         self.h = torch.empty(n, W, **f32)                       # the normed input of the current layer
-        self.h16 = torch.empty(n, W, dtype=torch.bfloat16, device=model.device) if model._wide(n, W) else None      # ... in bf16
+        self.h16 = torch.empty(n, W, dtype=torch.bfloat16, device=model.device) if model._rounded(n, W) else None      # ... in bf16
         self.y = torch.empty(n, W, **f32)                       # the mixer's result
         self.y2 = torch.empty(n, W, **f32)                      # the feed-forward's
         self.p = torch.empty(n * model.max_proj, **f32)         # everything projected from the layer's input

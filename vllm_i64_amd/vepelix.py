@@ -38,7 +38,7 @@ class _StepBuffers:
         W = model.cfg.width
         self.xe = torch.empty(2 if model.repeats else 1, n, W, **f32)      # the residual; the embedding output, where a further pass adds it
         self.h = torch.empty(n, W, **f32)                       # the normed input of the current sublayer
-        self.h16 = torch.empty(n, W, dtype=torch.bfloat16, device=model.device) if model._wide(n, W) else None      # ... in bf16
+        self.h16 = torch.empty(n, W, dtype=torch.bfloat16, device=model.device) if model._rounded(n, W) else None      # ... in bf16
         self.y = torch.empty(n, W, **f32)                       # a sublayer's result
         self.y2 = torch.empty(n, W, **f32)                      # that of the right one of two side-by-side mixers / the shared expert's
         self.p = torch.empty(n * model.max_proj, **f32)         # everything projected from the mixer's input
