@@ -458,7 +458,8 @@ class HybridRunner:
         """Whether the experts' rows are enough for the wide tiles, whose smallest is 64 rows high: many experts of a few rows each read rows that are not there as
         often as weights.  Microseconds of a pair's two launches, rows in fp32 | in bf16, width 2048, 768 inner: 16 experts of two, 100 tokens 37 | 39, 200
         44 | 41; 32 of two, 100 tokens 65 | 69, 320 69 | 69, 400 77 | 70; 64 of two, 200 tokens 113 | 121, 700 134 | 127; 64 of eight, 100 tokens 120 | 126, 200 136 | 126; 128 of
-        eight, 100 tokens 217 | 226, 320 242 | 234; 8 of two (1792 inner), 65 tokens 48 | 45."""
+        eight, 100 tokens 217 | 226, 320 242 | 234; 8 of two (1792 inner), 65 tokens 48 | 45; with a shared one, 7 tokens 43 | 37, 33 58 | 54, 64 61 | 57, and of width 1024,
+        896 inner, 5 tokens 13.6 | 18.2, 27 17.7 | 16.3, 64 19.1 | 16.8 (hence the rule beside this one's call)."""
         return experts < 16 or pairs >= 20 * experts
 
     def _moe_merges(self) -> bool:
@@ -488,7 +489,7 @@ class HybridRunner:
         pair_wgt = B.pair_wgt if f.weigh_input else None      # the weight multiplies what the expert reads, not what it returns
         D.moe_plan(B.idx, n=n, top=top, experts=E, group_off=B.group_off, pair_token=B.pair_token, pair_row=B.pair_row, wgt=B.wgt, pair_wgt=pair_wgt, shared=merged)
         # the (token, expert) pairs lie grouped by expert: one launch runs every expert over its own rows, the counts stay on the device
-        x16 = h16 if self._fills(n * top, E) else None
+        x16 = h16 if self._fills(n * top, E) and (n > 8 or W * f.ff >= 1 << 21) else None      # (up to eight rows of small experts: 16 columns a workgroup)
         rows, groups = n * (top + int(merged)), E + int(merged)
         act, act16 = self._act(B.act, B.act16, rows, f.ff, x16)
         D.linear(h, gate_up, act, a16=x16, out16=act16, m=n, a_rows=B.pair_token[:rows], batch=groups, w_batch=2 * f.ff * W, exact=ex, group_off=B.group_off, row_scale=pair_wgt,
