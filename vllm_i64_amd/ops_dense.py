@@ -86,14 +86,34 @@ def linear(a: Optional[torch.Tensor], w: torch.Tensor, out: Optional[torch.Tenso
         _chk(group_off, torch.int32, "group_off")
         if group_off.numel() < batch + 1:
             raise _lib.I64HError("linear: group_off needs batch + 1 entries")
-    d = _lib.Linear(A=ptr(a) + 4 * a_off if a16 is None else 0, lda=lda, a_rows=ptr(a_rows), W=ptr(w), C=ptr(out) + 4 * c_off if out is not None else 0, ldc=ldc, M=M, N=N, K=K, batch=batch,
-                    a_batch=a_batch, w_batch=w_batch, c_batch=c_batch, exact=int(exact), epilogue=epilogue,
-                    E=(ptr(e) + 4 * e_off) if e is not None else 0, lde=lde, e_batch=e_batch, softcap=float(softcap),
-                    bias=ptr(bias), bias_batch=int(bias_batch), scale=float(scale), act_a=float(act_a), act_b=float(act_b), group_off=ptr(group_off),
-                    row_scale=ptr(row_scale), in_norm_w=ptr(in_norm_w), in_eps=float(in_eps),
-                    rows_total=min((a_rows.numel() if a_rows is not None else a.numel() // lda), o.numel() // ldc) if group_off is not None else 0,
-                    a_height=-(-a.numel() // lda) if a_rows is not None else 0, A16=ptr(a16) + 2 * a_off if a16 is not None else 0,
-                    C16=ptr(out16) + 2 * c_off if out16 is not None else 0)
+    # (a step makes a few dozen of these: only what is not zero is put in)
+    d = _lib.Linear(lda=lda, W=ptr(w), ldc=ldc, M=M, N=N, K=K, batch=batch, exact=exact, epilogue=epilogue, scale=scale)
+    if a16 is None:
+        d.A = ptr(a) + 4 * a_off
+    else:
+        d.A16 = ptr(a16) + 2 * a_off
+    if out is not None:
+        d.C = ptr(out) + 4 * c_off
+    if out16 is not None:
+        d.C16 = ptr(out16) + 2 * c_off
+    if a_batch or w_batch or c_batch:
+        d.a_batch, d.w_batch, d.c_batch = a_batch, w_batch, c_batch
+    if e is not None:
+        d.E, d.lde, d.e_batch = ptr(e) + 4 * e_off, lde, e_batch
+    if bias is not None:
+        d.bias, d.bias_batch = ptr(bias), bias_batch
+    if a_rows is not None:
+        d.a_rows, d.a_height = ptr(a_rows), -(-a.numel() // lda)
+    if group_off is not None:
+        d.group_off, d.rows_total = ptr(group_off), min((a_rows.numel() if a_rows is not None else a.numel() // lda), o.numel() // ldc)
+    if row_scale is not None:
+        d.row_scale = ptr(row_scale)
+    if in_norm_w is not None:
+        d.in_norm_w, d.in_eps = ptr(in_norm_w), in_eps
+    if epilogue == EPI_SOFTCAP:
+        d.softcap = softcap
+    elif epilogue == EPI_CLAMP_GLU or epilogue == EPI_XIELU:
+        d.act_a, d.act_b = act_a, act_b
     call_dense("i64h_linear_run", _ref(d), _stream())
     return o
 
@@ -159,18 +179,14 @@ def latent_prep(p: torch.Tensor, *, q_off: int, dkv_off: int, heads: int, dim: i
     call_dense("i64h_latent_prep", _ref(d), _stream())
 
 
-def _as(t: torch.Tensor, dtype: torch.dtype) -> int:
-    """The address of a tensor of this type, null of another."""
-    return ptr(t) if t.dtype == dtype else 0
-
-
 def latent_attn(q: torch.Tensor, cache: torch.Tensor, block_table: torch.Tensor, slot_ids: torch.Tensor, positions: torch.Tensor, *,
                 window: int, scale: float, heads: int, kv_rank: int, rot_dim: int, out: torch.Tensor, n: Optional[int] = None,
                 mode: int = 0, splits: int = 1, workspace: Optional[torch.Tensor] = None, sink: Optional[torch.Tensor] = None,
                 softcap: float = 0.0) -> torch.Tensor:
     """See i64h_latent_attn.  sink fp32 [heads]: a learned extra score per head in the softmax's denominator.  out: fp32 or, in the matrix-core form over a
     bf16 cache, bf16 (the result rounded)."""
-    _chk(q, torch.float32, "q"), _chk(out, torch.bfloat16 if out.dtype == torch.bfloat16 else torch.float32, "out"), _chk(cache, None, "cache")
+    half = out.dtype == torch.bfloat16
+    _chk(q, torch.float32, "q"), _chk(out, None if half else torch.float32, "out"), _chk(cache, None, "cache")
     _chk(positions, torch.int32, "positions"), _chk(slot_ids, torch.int32, "slot_ids"), _chk(block_table, torch.int32, "block_table")
     rows = int(n if n is not None else positions.numel())
     D = kv_rank + rot_dim
@@ -189,7 +205,7 @@ def latent_attn(q: torch.Tensor, cache: torch.Tensor, block_table: torch.Tensor,
             raise _lib.I64HError(f"latent_attn: workspace of {workspace.numel()} floats, {need} needed")
     d = _lib.LatentAttn(Q=ptr(q), cache=ptr(cache), cache_dtype=CACHE_DTYPE_CODE[cache.dtype], block_table=ptr(block_table),
                         max_blocks_per_seq=block_table.shape[1], block_size=cache.shape[-2], slot_ids=ptr(slot_ids), positions=ptr(positions),
-                        window=int(window), scale=float(scale), out=_as(out, torch.float32), out16=_as(out, torch.bfloat16), n=rows, heads=heads, kv_rank=kv_rank, rot_dim=rot_dim, mode=mode,
+                        window=int(window), scale=float(scale), out=0 if half else ptr(out), out16=ptr(out) if half else 0, n=rows, heads=heads, kv_rank=kv_rank, rot_dim=rot_dim, mode=mode,
                         splits=int(splits) if splits > 1 else 1, workspace=ptr(workspace) if splits > 1 else 0, sink=int(sink is not None), sink_w=ptr(sink),
                         softcap=float(softcap))
     call_dense("i64h_latent_attn", _ref(d), _stream())
@@ -411,7 +427,8 @@ def kattn(q: torch.Tensor, cache: torch.Tensor, kscale: torch.Tensor, block_tabl
     [kv_heads, vdim + dim], q fp32 [n, heads, vdim + dim], out fp32 [n, heads * vdim], kscale may be None.  window > 0: the last `window`
     positions and the first keep_first ones are seen.  sink_w fp32 [heads]: the sink's score per head.  out: fp32 or, in the matrix-core form over a bf16
     cache, bf16 (the result rounded)."""
-    _chk(q, torch.float32, "q"), _chk(out, torch.bfloat16 if out.dtype == torch.bfloat16 else torch.float32, "out"), _chk(cache, None, "cache")
+    half = out.dtype == torch.bfloat16
+    _chk(q, torch.float32, "q"), _chk(out, None if half else torch.float32, "out"), _chk(cache, None, "cache")
     if kscale is not None or vdim <= 0:
         _chk(kscale, torch.float32, "kscale")
     _chk(positions, torch.int32, "positions"), _chk(slot_ids, torch.int32, "slot_ids"), _chk(block_table, torch.int32, "block_table")
@@ -438,7 +455,7 @@ def kattn(q: torch.Tensor, cache: torch.Tensor, kscale: torch.Tensor, block_tabl
             raise _lib.I64HError(f"kattn: workspace of {workspace.numel()} floats, {need} needed")
     d = _lib.KAttn(Q=ptr(q), cache=ptr(cache), cache_dtype=CACHE_DTYPE_CODE[cache.dtype], kscale=ptr(kscale), block_table=ptr(block_table),
                    max_blocks_per_seq=block_table.shape[1], block_size=cache.shape[-2], slot_ids=ptr(slot_ids), positions=ptr(positions), chunk=int(chunk),
-                   bias=ptr(bias), bias_rows=bias.shape[0] if bias is not None else 0, sink=int(bool(sink)), out=_as(out, torch.float32), out16=_as(out, torch.bfloat16), n=rows, heads=heads,
+                   bias=ptr(bias), bias_rows=bias.shape[0] if bias is not None else 0, sink=int(bool(sink)), out=0 if half else ptr(out), out16=ptr(out) if half else 0, n=rows, heads=heads,
                    kv_heads=kv_heads, dim=dim, mode=int(mode), splits=int(splits) if splits > 1 else 1, workspace=ptr(workspace) if splits > 1 else 0,
                    vdim=int(vdim), softcap=float(softcap), window=int(window), keep_first=int(keep_first), sink_w=ptr(sink_w))
     call_dense("i64h_kattn", _ref(d), _stream())
