@@ -479,8 +479,11 @@ bool dn_linear_wide(const i64h_linear& d, int form, hipStream_t s) {
     // few tiles of 16 columns: one for every CU at most (its LDS holds three or four steps of all its waves)
     if (form < 0 && thin_fits(d) && d.M <= 128 && d.K >= 256 && (d.M + 63) / 64 * ((d.N + 15) / 16) * d.batch <= 256) form = FORMS;
     if (form < 0) {
-        // (what every form waits for: the weights; of forms that wait no longer than that the largest, which reads the rows least often)
-        const float weights = (float)d.batch * (float)cols * (float)d.K * 2.0f / 4.7e6f;
+        // What every form waits for: the weights of the batches that have rows (dealt to batches by chance, one of them perhaps with all), and longer where its workgroups do
+        // not fill the rounds that they take; of forms that wait equally long the largest, which reads the rows least often.  9 batches of 2048 x 1792, 64 x 128 | 64 x 64 tiles,
+        // us: 7 tokens of two and a shared batch 15.8 | 11.7, 27 tokens 18.8 | 20.4, 64 tokens 19.8 | 23.7; a pair of 1792 x 2048, 64 tokens 32.6 | 36.5.
+        const float others = (float)(d.batch - 1), live = d.group_off && d.rows_total > 0 && others > 0.0f ? 1.0f + others * (1.0f - expf(-fmaxf(0.0f, (float)(d.rows_total - d.M)) / others)) : (float)d.batch;
+        const float weights = live * (float)cols * (float)d.K * 2.0f / 4.7e6f;
         float best = 0.0f;
         for (int i = 0; i < FORMS; ++i) {
             const dn_wide_form& f = forms[i];
@@ -489,7 +492,8 @@ bool dn_linear_wide(const i64h_linear& d, int form, hipStream_t s) {
             if (d.group_off && d.rows_total > 0 && d.rows_total / f.BM + (d.batch + 1) / 2 < mt) mt = d.rows_total / f.BM + (d.batch + 1) / 2;
             const float q = (float)(mt * ((cols + f.BN - 1) / f.BN)) / 256.0f;
             const float step = f.alone ? ceilf(q) * f.step : fmaxf(f.first, fmaxf(0.5f * q, q > 1.0f ? 0.75f : 0.0f) * f.step);
-            const float cost = fmaxf((float)(d.K / 64) * step + (f.alone ? ceilf(q) * f.end : 0.0f), weights);
+            const float full = fmaxf(1.0f, fminf(q, live * (float)((d.M + f.BM - 1) / f.BM) * (float)((cols + f.BN - 1) / f.BN) / 256.0f));      // rounds, were they all full
+            const float cost = fmaxf((float)(d.K / 64) * step + (f.alone ? ceilf(q) * f.end : 0.0f), weights * ceilf(full) / full);
             if (i == 0 || cost < best) best = cost, form = i;
         }
     }
