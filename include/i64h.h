@@ -130,9 +130,10 @@ typedef struct i64h_gemm_desc {
     int32_t want_stats;
     const float* col_scale;       /* epilogue 0, int8 operand, optional: per-output-channel scale [G][N] replacing w_scale[g] */
     const int32_t* c_row_map;     /* epilogue 0, optional: operand row r is stored as output row c_row_map[r] (e.g. expert outputs straight back in (route, token) order) */
-    int32_t a_group_slots;        /* fp32 operand, optional promise (0 = none): a_row_slot[r] of every row of group g lies in [g * S, g * S + S), S = this value; lets the decode-sized kernel request the statistics without waiting for the row's slot index.  With a norm prologue also: these slots count the rows of group g and no others (a group of at most 16 rows then takes their ranges from its own tile) */
+    int32_t a_group_slots;        /* fp32 operand, optional promise (0 = none): a_row_slot[r] of every row of group g lies in [g * S, g * S + S), S = this value; lets the decode-sized kernel request the statistics without waiting for the row's slot index */
     int32_t b_frags;              /* decode-sized (fp32-operand) problems only: 1 = B points to the fragment pack of the weights (i64h_pack_weight_frags; N % 16 == 0, SwiGLU: N % 32 == 0, K % 64 == 0): every weight load of a wave is then 1 KB of consecutive bytes */
     const float* c_residual;      /* epilogue 0, decode-sized (fp32-operand) problems only, optional: C = c_residual + product (same layout as C, may be C itself): the residual add of the decoder layer (vllm_i64/models/complexity_deep/model.py:355-357) in the projection's epilogue */
+    int32_t a_own_ranges;         /* problems of a launch with a norm prologue, optional promise (0 = none): the slots that the rows of a group (without groups: of the problem) name count these rows and no others, each row in the slot that it names; with groups: a_group_slots of 1 or 2.  A group of at most 16 rows then takes its ranges from its own tile instead of waiting for the publishers' records (the first problem does so without the promise where tok_slots is NULL: every row then reports to its slot) */
 } i64h_gemm_desc;
 int i64h_gemm_i8_pair(const i64h_gemm_desc* a, const i64h_gemm_desc* b, void* stream);
 /* RMSNorm in front of the quantizer of a decode-sized launch.  The operand rows of the problem(s) are the residual stream

@@ -152,3 +152,50 @@ def test_norm_fused_small_shapes_more_row_tiles_than_column_tiles(dev, kind, bat
         assert torch.equal(x, y), (kind, batch, i, (x - y).abs().max().item())
     for l in range(ocfg.num_layers):
         assert torch.equal(ka[l], kb[l]) and torch.equal(va[l], vb[l])
+
+
+@pytest.mark.parametrize("form", ["gathered", "grouped", "first"])
+@pytest.mark.parametrize("K,N", [(1024, 256), (512, 1024)])
+def test_norm_prologue_quantizes_with_the_range_of_the_slot(dev, form, K, N):
+    """A slot counts the rows that report to it, whichever of them a problem reads: a second problem over some of the rows with the slot of all, groups that
+    leave out a row of their slot, a first problem with a row that reports to another slot only.  The row left out has the largest values.  Against the norm and the
+    statistics as launches of their own; the same bits."""
+    from vllm_i64_amd import ops
+    g = torch.Generator().manual_seed(K + N)
+    n, out_row = 11, 4
+    h = torch.randn(n, K, generator=g)
+    h[out_row, 7] = 40.0
+    h, nw = h.to(dev), (torch.rand(K, generator=g) + 0.5).to(dev)
+    w = torch.randint(-128, 128, (2, N, K), dtype=torch.int8, generator=g).to(dev)
+    ws = torch.full((2,), 3e-3, device=dev)
+    bucket = torch.arange(n) % 4      # two groups of two slots
+    first = torch.zeros(n, dtype=torch.long)
+    if form == "first":
+        first[out_row] = 5
+    tok = torch.stack([first, 1 + bucket], 1).to(torch.int32).to(dev)
+    rows = torch.tensor([r for r in torch.argsort(bucket, stable=True).tolist() if r != out_row])
+    off = torch.tensor([0, int((bucket[rows] < 2).sum()), n - 1], dtype=torch.int32, device=dev)
+    idx, slot = rows.to(torch.int32).to(dev), bucket[rows].to(torch.int32).to(dev)
+    stats = ops.stats_alloc(6, dev)
+
+    def descs(x):
+        a, b = torch.zeros(n, N, device=dev), torch.zeros(n - 1, N, device=dev)
+        da = ops.gemm_desc(x, w[:1], ws[:1], a, a_slot_base=0, stats=stats)
+        if form == "grouped":
+            db = ops.gemm_desc(x, w, ws, b, a_src_row=idx, a_src_mod=n, a_row_slot=slot, a_slot_base=1, group_offsets=off, stats=stats, m_total=n - 1, a_group_slots=2)
+        else:
+            db = ops.gemm_desc(x, w[1:], ws[1:], b, a_src_row=idx, a_src_mod=n, a_slot_base=0, stats=stats, m_total=n - 1)
+        return da, db, a, b
+    ops.stats_reset(stats)
+    normed = torch.empty_like(h)
+    ops.fused_residual_norm(h, nw, 1e-6, normed=normed)
+    ops.rows_minmax(normed, stats, slots=tok, slot_base=0)
+    da, db, a, b = descs(normed)
+    ops.gemm_i8_pair(da, db)
+    ops.stats_reset(stats)
+    sync = ops.decode_sync_alloc(dev)
+    da, db, a2, b2 = descs(h)
+    ops.gemm_i8_pair_norm(da, db, ops.norm_prologue(nw, 1e-6, sync, slot_base=0, tok_slots=tok, num_slots=6))
+    torch.cuda.synchronize()
+    assert int(sync[1]) == 0 and a.abs().sum() > 0 and b.abs().sum() > 0
+    assert torch.equal(a, a2) and torch.equal(b, b2)

@@ -924,9 +924,9 @@ __device__ __forceinline__ void gemm_i8_skinny_body(const GemmI8Args& p, const i
         const bool lane_in = lane < cpr;
         const int kq = lane_in ? lane : 0;
         const bool pub = pub_problem && nt == 0;  // uniform over the workgroup
-        // a tile that holds every row that its slots count (one call of at most 16 rows; a group of them whose slots are its own) has their ranges itself:
+        // a tile that holds every row that its slots count (the caller's promise, or a first problem to whose slot every row reports) has their ranges itself:
         // nothing to wait for.  One token, three such launches a step: a record's way there and back was 5000 of their 17600 cycles
-        const bool alone = p.group_off ? (p.a_group_slots == 1 || p.a_group_slots == 2) && p.a_row_slot && s_info[3] <= BMR : !p.a_row_slot && p.M_total <= BMR;
+        const bool alone = p.a_own_ranges && (p.group_off ? (p.a_group_slots == 1 || p.a_group_slots == 2) && p.a_row_slot && s_info[3] <= BMR : !p.a_row_slot && p.M_total <= BMR);
         uint32_t* own_lo = (uint32_t*)(q_zp + BMR);      // [2] ranges of the group's slots
         uint32_t* own_hi = own_lo + 2;
         int src[2];
@@ -1406,6 +1406,7 @@ struct i64h_gemm_desc {
     int32_t a_group_slots;
     int32_t b_frags;
     const float* c_residual;
+    int32_t a_own_ranges;
 };
 
 // mirrors i64h_norm_prologue in include/i64h.h
@@ -1452,6 +1453,7 @@ static GemmI8Args to_args(const i64h_gemm_desc* d) {
     p.a_group_slots = d->a_group_slots;
     p.b_frags = d->b_frags;
     p.c_add = d->c_residual;
+    p.a_own_ranges = d->a_own_ranges;
     return p;
 }
 
@@ -1647,6 +1649,7 @@ static int launch_skinny_norm(const i64h_gemm_desc* a, const i64h_gemm_desc* b, 
     GemmI8Pair pp;
     pp.p[0] = to_args(a);
     pp.p[1] = b ? to_args(b) : pp.p[0];
+    pp.p[0].a_own_ranges |= np->tok_slots == nullptr;
     // few workgroups: 32 columns each, K in four shares.  Us a step, 64 columns | 32: dense, 1 token 128.2 | 126.4, 16 150.5 | 149.2, 24 (128 workgroups of 64) 151.1 | 152.6,
     // 33 149.8 | 152.3; mixture, 3 tokens 137.3 | 132.9, 12 147 | 144.5, 24 (152) 152.2 | 153.1, 64 224.5 | 229.3
     constexpr int few = EPI == EPI_QKR ? 4 : 2;      // (a tile of 64 columns is a head there)

@@ -29,6 +29,7 @@ struct GemmI8Args {
     const float* c_add;        // EPI_STORE, decode-sized kernel, optional: C = c_add + product (same layout as C; may be C itself)
     int b_frags;               // decode-sized kernel: B is the fragment pack of the weights
     int a_group_slots;         // a_fp32, optional promise: a_row_slot[r] of a row of group g lies in [g * S, g * S + S) (S = this value)
+    int a_own_ranges;          // norm prologue, optional promise: the slots of a group's rows (no groups: of the problem's) count these rows and no others
     const int32_t* group_off;  // [G+1] device, or nullptr => one group [0, M_total)
     int G, M_total, N, K;
     float* C;                  // EPI_STORE: [M_total, N]; EPI_SWIGLU: [M_total, N/2]

@@ -771,11 +771,11 @@ class I64MoEModel:
                 plan = B.plan
                 R = plan.rows
                 s_gu = ops.gemm_desc(hbuf, W["sh_gu"].w_q, W["sh_gu"].w_s, B.sh_inter, a_slot_base=base + 2, epilogue=ops.EPI_SWIGLU,
-                                     out_slot_base=base + 3 + nbk, stats=st, want_stats=True, w_frags=self._wf(W["sh_gu"], ops.EPI_SWIGLU, W["exp_gu"]))
+                                     out_slot_base=base + 3 + nbk, stats=st, want_stats=True, own_ranges=True, w_frags=self._wf(W["sh_gu"], ops.EPI_SWIGLU, W["exp_gu"]))
                 e_gu = ops.gemm_desc(hbuf, W["exp_gu"].w_q, W["exp_gu"].w_s, B.e_inter, a_src_row=plan.perm[l], a_src_mod=n,
                                      a_row_slot=plan.sorted_bucket[l], a_slot_base=base + 3, group_offsets=plan.expert_offsets[l],
                                      epilogue=ops.EPI_SWIGLU, out_row_slot=plan.sorted_bucket[l], out_slot_base=base + 4 + nbk, stats=st,
-                                     want_stats=True, m_total=R, a_group_slots=cfg.top_k, w_frags=self._wf(W["exp_gu"], ops.EPI_SWIGLU, W["sh_gu"]))
+                                     want_stats=True, m_total=R, a_group_slots=cfg.top_k, own_ranges=True, w_frags=self._wf(W["exp_gu"], ops.EPI_SWIGLU, W["sh_gu"]))
                 ops.gemm_i8_pair_norm(s_gu, e_gu, ops.norm_prologue(W["ln2"], eps, self.dec_sync, slot_base=base + 2, tok_slots=plan.tok_slots[l],
                                                                     num_slots=1 + nbk))
                 e_dn = ops.gemm_desc(B.e_inter, W["exp_dn"].w_q, W["exp_dn"].w_s, B.e_out, a_row_slot=plan.sorted_bucket[l],

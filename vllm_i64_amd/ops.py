@@ -277,9 +277,10 @@ def gemm_i8_frags(a: torch.Tensor, row_scale: torch.Tensor, w_frags: torch.Tenso
 def gemm_desc(a: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor, out: torch.Tensor, *, row_scale=None, a_src_row=None,
               a_src_mod: int = 0, a_row_slot=None, a_slot_base: int = 0, group_offsets=None, epilogue: int = EPI_STORE,
               out_row_slot=None, out_slot_base: int = 0, stats=None, want_stats: bool = False, m_total: Optional[int] = None,
-              c_row_map=None, a_group_slots: int = 0, w_frags: Optional[torch.Tensor] = None, c_residual=None):
+              c_row_map=None, a_group_slots: int = 0, w_frags: Optional[torch.Tensor] = None, c_residual=None, own_ranges: bool = False):
     """Build an i64h_gemm_desc.  a is int8 [M, K] (with row_scale) or fp32 [*, K] (quantized on the fly from the stat slots).
-    w_frags: the fragment pack of w (pack_weight_frags), read instead of w by the decode-sized kernel."""
+    w_frags: the fragment pack of w (pack_weight_frags), read instead of w by the decode-sized kernel.
+    own_ranges (launches with a norm prologue): the slots that a group's rows name count these rows and no others."""
     if w.dim() == 2:
         w = w.unsqueeze(0)
     G, N, K = w.shape
@@ -293,6 +294,7 @@ def gemm_desc(a: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor, out: torc
     d.N, d.K, d.C, d.epilogue = N, K, ptr(out), epilogue
     d.out_row_slot, d.out_slot_base, d.stats, d.want_stats = ptr(out_row_slot), out_slot_base, ptr(stats), int(want_stats)
     d.c_row_map, d.a_group_slots = ptr(c_row_map), a_group_slots
+    d.a_own_ranges = int(own_ranges)
     d.c_residual = ptr(c_residual)   # decode-sized problems, plain epilogue: out = c_residual + product
     return d
 
