@@ -221,3 +221,17 @@ def test_rows_past_a_tiles_end(dev):
     assert torch.isfinite(out[:7]).all() and torch.isfinite(out[9:39]).all() and not torch.isfinite(out[7:9]).any() and not out[39].any()
     few = D.linear(None, w[0], torch.empty(7, 128, device=dev), a16=a[:7].to(dev))
     assert torch.isfinite(few).all()
+
+
+def test_blocks_of_a_tile_follow_each_other(dev, form):
+    """A wave hands itself one block of 16 rows after the other through the same LDS: whole numbers, exact in every sum and result, in all blocks of two tall tiles; several times."""
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator().manual_seed(5)
+    M, N, K = 512, 520, 64
+    a, w = torch.randint(-2, 3, (M, K), generator=g), torch.randint(-1, 2, (N, K), generator=g)
+    want = (a @ w.T).to(dev)      # at most 128: exact in bf16
+    a16, w16 = a.bfloat16().to(dev), w.bfloat16().to(dev)
+    for _ in range(5):
+        out, out16 = torch.empty(M, N, device=dev), torch.empty(M, N, device=dev, dtype=torch.bfloat16)
+        D.linear(None, w16, out, a16=a16, out16=out16)
+        assert torch.equal(out.long(), want) and torch.equal(out16.long(), want)

@@ -211,6 +211,11 @@ __global__ __launch_bounds__(64 * NWM * NWN, PER_CU * NWM * NWN / 4) void linear
             const __amdgpu_buffer_rsrc_t buf16 = __builtin_amdgcn_make_buffer_rsrc((uint16_t*)p.C16 + at, 0, (int)DN_STORE_END, 0x00020000);
             const bool eight = ((N | (int)p.ldc | (int)p.c_batch) & 7) == 0;
             const int cw = at_col, ldc = (int)p.ldc;
+            // (a lane reads what others of its wave wrote: LDS operations of a wave happen in their order, and the fence keeps the compiler to it)
+            auto handed = [&]() {
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            };
             __syncthreads();
 #pragma unroll
             for (int i = 0; i < FM; ++i) {
@@ -234,6 +239,7 @@ __global__ __launch_bounds__(64 * NWM * NWN, PER_CU * NWM * NWN / 4) void linear
                     }
                     *(dn_v4f*)&own[(at_lane & 15) * PITCH + j * 16 + (at_lane >> 4) * 4] = o;
                 }
+                handed();
                 const int r1 = at_row + i * 16;
                 if (p.C16) {
                     if (eight) {
@@ -264,6 +270,7 @@ __global__ __launch_bounds__(64 * NWM * NWN, PER_CU * NWM * NWN / 4) void linear
                     }
                 }
                 if (i + 1 < FM) {      // (a row's work at a time: the registers are full)
+                    handed();
 #pragma unroll
                     for (int j = 0; j < FN; ++j) asm volatile("" : "+v"(acc[i + 1 < FM ? i + 1 : i][j]));
                 }
