@@ -458,6 +458,12 @@ __device__ __forceinline__ void latent_row(const i64h_latent_attn_args& p, const
         if (lane + 64 * c < r) lt_put(p, o + lane + 64 * c, acc[c] / l);
 }
 
+// between words of LDS that a wave's lanes write and those that other lanes of the wave then read (such operations happen in their order: the compiler has to keep it)
+__device__ __forceinline__ void lt_handed() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // A tile's rows, [64] positions and [64] slots (-1: no such row) in LDS; lane l reads row l's.  (Every wave writes all of them, and reads what it wrote.)
 // A run is a stretch of neighbouring rows of one sequence: rows s0 .. s1 - 1, the least and the largest position of them and of those
 // among the wave's rows wr .. wr + 15.
@@ -524,6 +530,7 @@ __global__ __launch_bounds__(256, 2) void latent_attn_rows_kernel(const i64h_lat
     const uint64_t starts = lt_run_starts(slot_l);
     if (blockIdx.y > 0 && (int)blockIdx.y >= __popcll(starts)) return;
     info[lane] = pos_l, info[64 + lane] = slot_l;
+    lt_handed();
     bool mine = info[64 + wr + n] < 0 && blockIdx.y == 0;      // this workgroup's rows: those of its runs
     const int64_t tok = row0 + wr + n;
     const bool valid = tok < p.n;
@@ -999,6 +1006,7 @@ __global__ __launch_bounds__(256, NB > 8 ? 1 : 2) void latent_attn_rows_f32_kern
     const uint64_t starts = lt_run_starts(slot_l);
     if (blockIdx.y > 0 && (int)blockIdx.y >= __popcll(starts)) return;
     info[lane] = pos_l, info[64 + lane] = slot_l;
+    lt_handed();
     bool mine = info[64 + wr + n] < 0 && blockIdx.y == 0;      // this workgroup's rows: those of its runs
     const int64_t tok = row0 + wr + n;
     const bool valid = tok < p.n;
