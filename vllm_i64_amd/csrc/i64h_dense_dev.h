@@ -19,13 +19,15 @@ __device__ __forceinline__ uint32_t dn_bf16_pair(float a, float b) {
 __device__ __forceinline__ float dn_bf16_to_f32(uint32_t h) { return __uint_as_float(h << 16); }
 __device__ __forceinline__ float dn_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
 // x sigmoid(z) = x / (1 + e^-z), z a multiple of x (so a NaN is in x already): e^-z = 2^n 2^f with f at most half, log2(e) in two parts, from the native base-2
-// exponential; the quotient from a native reciprocal and its own remainder, one rounding less than by way of 1 / (1 + e^-z).  Against 64 bits, times another factor:
-// 2.05e-7 of the result at most and 4.6e-8 on average over z of +- 20, 2.15e-7 and 5.0e-8 with expf and a division, in 15 instructions for 27.  (The ends of the range
-// are where 1 + e^-z is 1 or its reciprocal below the smallest normal number; no remainder of an infinite x is let in.)
+// exponential; the quotient from a native reciprocal and its own remainder, one rounding less than by way of 1 / (1 + e^-z).  The reciprocal is that of a sixteenth: by itself
+// it is zero where it would lie below the smallest normal number, which 1 / (1 + e^-z) does for z from -87.4 on, down to -88.7, where e^-z ends (as with expf, the result is
+// zero from there on).  No remainder of an infinite x, or of no quotient, is let in.
+// Against 64 bits, times another factor, of the result at most and on average: 2.16e-7 and 4.6e-8 over z of +- 20, 1.7e-7 and 4.5e-8 from -88.7 to -20; with expf and a division
+// 2.20e-7 and 5.0e-8, 1.95e-7 and 5.1e-8 down to -87.2, 3.3e-7 and 8.8e-8 below.  17 instructions for 27.
 __device__ __forceinline__ float dn_gated(float x, float z) {
-    const float c = __builtin_amdgcn_fmed3f(z, -88.0f, 88.0f), n = __builtin_rintf(c * -1.44269504f);
+    const float c = __builtin_amdgcn_fmed3f(z, -100.0f, 88.0f), n = __builtin_rintf(c * -1.44269504f);
     const float f = __builtin_fmaf(c, -1.92596299e-8f, __builtin_fmaf(c, -1.44269504f, -n));
-    const float d = 1.0f + __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)n), y = __builtin_amdgcn_rcpf(d), q = x * y;
+    const float d = 1.0f + __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)n), y = __builtin_amdgcn_rcpf(d * 0.0625f) * 0.0625f, q = x * y;
     return __builtin_fmaf(fmaxf(__builtin_fmaf(-d, q, x), -3.4e38f), y, q);
 }
 __device__ __forceinline__ float dn_gelu_tanh(float z) {
