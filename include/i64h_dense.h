@@ -100,6 +100,9 @@ typedef struct {
     void* C16;
 } i64h_linear;
 int i64h_linear_run(const i64h_linear* d, void* stream);
+/* The kernel that a launch over rows in bf16 (A16) takes by its sizes: 0 .. 5 = tiles of 256 x 256, 256 x 128, 192 x 128, 128 x 128, 64 x 128, 64 x 64; 6 = 16 columns a
+ * workgroup; -1 = operands beyond their 32-bit offsets.  Launches nothing, reads the sizes only. */
+int i64h_linear_form(const i64h_linear* d);
 
 /* out[t, :] = float(table[ids[t], :]) * scale; table bf16 [V, W]; ids outside [0, V) are clamped. */
 int i64h_embed_scaled(const int64_t* ids, const void* table_bf16, float scale, float* out, int64_t n, int32_t W, int64_t V, void* stream);

@@ -385,7 +385,7 @@ _dense: Optional[ctypes.CDLL] = None
 
 
 def dense_exported_symbols():
-    return ["i64h_last_error", "i64h_version", "i64h_device_check", "i64h_latent_attn_workspace_floats", "i64h_kattn_workspace_floats", "i64h_scan_work_floats", "i64h_scan_in_tiles", *DENSE_SIGNATURES.keys()]
+    return ["i64h_last_error", "i64h_version", "i64h_device_check", "i64h_latent_attn_workspace_floats", "i64h_kattn_workspace_floats", "i64h_scan_work_floats", "i64h_scan_in_tiles", "i64h_linear_form", *DENSE_SIGNATURES.keys()]
 
 
 def load_dense() -> ctypes.CDLL:
@@ -404,6 +404,8 @@ def load_dense() -> ctypes.CDLL:
     lib.i64h_scan_work_floats.argtypes = [_L, _I, _I, _I]
     lib.i64h_scan_in_tiles.restype = _I
     lib.i64h_scan_in_tiles.argtypes = [_L, _I, _I, _I, _I, _I, _I]
+    lib.i64h_linear_form.restype = _I
+    lib.i64h_linear_form.argtypes = [_P]
     lib.i64h_latent_attn_workspace_floats.restype = _L
     lib.i64h_latent_attn_workspace_floats.argtypes = [_L, _I, _I, _I]
     lib.i64h_kattn_workspace_floats.restype = _L

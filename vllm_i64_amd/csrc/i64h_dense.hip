@@ -982,6 +982,10 @@ int i64h_set_linear_skinny(int32_t on) {
     return 0;
 }
 
+int i64h_linear_form(const i64h_linear* d) {
+    return d && d->M > 0 && d->N > 0 && d->K > 0 && d->batch > 0 ? dn_linear_wide_form(*d) : -1;
+}
+
 int i64h_linear_run(const i64h_linear* dp, void* stream) {
     I64H_CHECK_ARG(dp != nullptr, "linear: no descriptor");
     const i64h_linear& d = *dp;

@@ -146,5 +146,6 @@ bool dn_linear_block(const i64h_linear& d, int form, hipStream_t s);
 
 // launches whose input rows come in bf16 (i64h_linear_wide.hip).  form as above.  False: the launch does not fit.
 bool dn_linear_wide(const i64h_linear& d, int form, hipStream_t s);
+int dn_linear_wide_form(const i64h_linear& d);
 
 #endif

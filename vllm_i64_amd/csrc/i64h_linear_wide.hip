@@ -474,37 +474,51 @@ struct dn_wide_form {
     float end;            // a round's stores
 };
 
-bool dn_linear_wide(const i64h_linear& d, int form, hipStream_t s) {
+enum { DN_WIDE_FORMS = 6 };      // tile forms; the number itself stands for linear_thin_kernel
+
+// -1: operands beyond what the tiles' 32-bit offsets reach
+int dn_linear_wide_form(const i64h_linear& d) {
     const bool dual = dn_dual(d.epilogue);
     const int64_t span = (d.a_rows ? d.a_height : 256) * d.lda * 2;
-    if ((d.a_rows && d.a_height <= 0) || span >= (int64_t)DN_BUF_END - 64 || ((dual ? (int64_t)d.N : 0) + 256) * 2 * d.K >= (int64_t)DN_BUF_END - 64) return false;
+    if ((d.a_rows && d.a_height <= 0) || span >= (int64_t)DN_BUF_END - 64 || ((dual ? (int64_t)d.N : 0) + 256) * 2 * d.K >= (int64_t)DN_BUF_END - 64) return -1;
     const int64_t cols = dual ? 2 * (int64_t)d.N : d.N;
-    if ((d.M + 63) / 64 * d.batch * ((cols + 63) / 64) > 0x7fffffff) return false;
-    static const dn_wide_form forms[] = {{256, 256, true, 1.3f, 1.3f, 12.0f}, {256, 128, true, 0.72f, 0.72f, 7.0f}, {192, 128, false, 1.0f, 1.7f, 0.0f},
-                                         {128, 128, false, 1.0f, 1.2f, 0.0f}, {64, 128, false, 0.5f, 0.75f, 0.0f}, {64, 64, false, 0.33f, 0.4f, 0.0f}};
-    constexpr int FORMS = sizeof(forms) / sizeof(forms[0]);
+    if ((d.M + 63) / 64 * d.batch * ((cols + 63) / 64) > 0x7fffffff) return -1;
     // few tiles of 16 columns: one for every CU at most (its LDS holds three or four steps of all its waves)
-    if (form < 0 && thin_fits(d) && d.M <= 128 && d.K >= 256 && (d.M + 63) / 64 * ((d.N + 15) / 16) * d.batch <= 256) form = FORMS;
-    if (form < 0) {
-        // What every form waits for: the weights of the batches that have rows (dealt to batches by chance, one of them perhaps with all), and longer where its workgroups do
-        // not fill the rounds that they take; of forms that wait equally long the largest, which reads the rows least often.  9 batches of 2048 x 1792, 64 x 128 | 64 x 64 tiles,
-        // us: 7 tokens of two and a shared batch 15.8 | 11.7, 27 tokens 18.8 | 20.4, 64 tokens 19.8 | 23.7; a pair of 1792 x 2048, 64 tokens 32.6 | 36.5.
-        const float others = (float)(d.batch - 1), live = d.group_off && d.rows_total > 0 && others > 0.0f ? 1.0f + others * (1.0f - expf(-fmaxf(0.0f, (float)(d.rows_total - d.M)) / others)) : (float)d.batch;
-        const float weights = live * (float)cols * (float)d.K * 2.0f / 4.7e6f;
-        float best = 0.0f;
-        for (int i = 0; i < FORMS; ++i) {
-            const dn_wide_form& f = forms[i];
-            int64_t mt = (d.M + f.BM - 1) / f.BM * d.batch;
-            // rows dealt to batches: half a tile more than the rows fill, on average
-            if (d.group_off && d.rows_total > 0 && d.rows_total / f.BM + (d.batch + 1) / 2 < mt) mt = d.rows_total / f.BM + (d.batch + 1) / 2;
-            const float q = (float)(mt * ((cols + f.BN - 1) / f.BN)) / 256.0f;
-            const float step = f.alone ? ceilf(q) * f.step : fmaxf(f.first, fmaxf(0.5f * q, q > 1.0f ? 0.75f : 0.0f) * f.step);
-            const float full = fmaxf(1.0f, fminf(q, live * (float)((d.M + f.BM - 1) / f.BM) * (float)((cols + f.BN - 1) / f.BN) / 256.0f));      // rounds, were they all full
-            const float cost = fmaxf((float)(d.K / 64) * step + (f.alone ? ceilf(q) * f.end : 0.0f), weights * ceilf(full) / full);
-            if (i == 0 || cost < best) best = cost, form = i;
-        }
+    if (thin_fits(d) && d.M <= 128 && d.K >= 256 && (d.M + 63) / 64 * ((d.N + 15) / 16) * d.batch <= 256) return DN_WIDE_FORMS;
+    static const dn_wide_form forms[DN_WIDE_FORMS] = {{256, 256, true, 1.3f, 1.3f, 12.0f}, {256, 128, true, 0.72f, 0.72f, 7.0f}, {192, 128, false, 1.0f, 1.7f, 0.0f},
+                                                      {128, 128, false, 1.0f, 1.2f, 0.0f}, {64, 128, false, 0.5f, 0.75f, 0.0f}, {64, 64, false, 0.33f, 0.4f, 0.0f}};
+    int form = 0;
+    float best = 0.0f;
+    for (int i = 0; i < DN_WIDE_FORMS; ++i) {
+        const dn_wide_form& f = forms[i];
+        int64_t mt = (d.M + f.BM - 1) / f.BM * d.batch;
+        // rows dealt to batches: half a tile more than the rows fill, on average
+        if (d.group_off && d.rows_total > 0 && d.rows_total / f.BM + (d.batch + 1) / 2 < mt) mt = d.rows_total / f.BM + (d.batch + 1) / 2;
+        const float q = (float)(mt * ((cols + f.BN - 1) / f.BN)) / 256.0f;
+        const float step = f.alone ? ceilf(q) * f.step : fmaxf(f.first, fmaxf(0.5f * q, q > 1.0f ? 0.75f : 0.0f) * f.step);
+        const float cost = (float)(d.K / 64) * step + (f.alone ? ceilf(q) * f.end : 0.0f);
+        if (i == 0 || cost < best) best = cost, form = i;
     }
-    if (form == FORMS && thin_fits(d)) {
+    // At most 64 rows, dealt to batches by chance: a launch waits for the weights of the batches that have any (one of them perhaps with all).  Where 64 x 128 tiles of these
+    // fill a round of the 256 CUs by half and no more than once, they read the rows half as often for the same wait.  Microseconds, 64 x 128 | 64 x 64: 9 batches, pairs of 1792
+    // x 2048 (252 tiles), 12 tokens 34.4 | 35.6, 64 tokens 35.1 | 37.8; 2048 x 1792 (144), 40 tokens 18.3 | 20.8; 13 batches, pairs of 896 x 1024 (182), 64 tokens 14.2 | 16.3.  Less
+    // than half: 8 batches, pairs of 896 x 1024 (112), 64 tokens 10.6 | 9.3.  More than once, or longer k, where the four steps that a 64 x 64 tile has on their way count: 12
+    // batches, pairs of 1792 x 2048 (336), 12 tokens 44.0 | 41.8; 8 of 5504 x 2048 (688), 64 tokens 87.7 | 81.6; 15 of 1024 x 4096 (240), 27 tokens 63.4 | 58.7; but 64 of 2048 x 768
+    // (1024), 40 tokens 42.4 | 47.3.  (Taller tiles are never the fastest there: 59 to 107 us for these.)
+    if (form >= 4 && d.group_off && d.rows_total > 0 && d.M <= 64) {
+        const float others = (float)(d.batch - 1), live = others > 0.0f ? 1.0f + others * (1.0f - expf(-fmaxf(0.0f, (float)(d.rows_total - d.M)) / others)) : 1.0f;
+        const float tiles = live * (float)((cols + 127) / 128);
+        if (form == 5 && d.K <= 2048 && tiles >= 128.0f && tiles < 256.0f) form = 4;
+        else if (form == 4 && d.K >= 2048 && tiles >= 256.0f) form = 5;
+    }
+    return form;
+}
+
+bool dn_linear_wide(const i64h_linear& d, int form, hipStream_t s) {
+    const int by_size = dn_linear_wide_form(d);
+    if (by_size < 0) return false;
+    if (form < 0) form = by_size;
+    if (form == DN_WIDE_FORMS && thin_fits(d)) {
         launch_thin(d, s);
         return true;
     }
