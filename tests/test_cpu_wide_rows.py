@@ -117,3 +117,13 @@ def test_tiles_by_size_are_among_the_fastest(G, rows, M, N, K, pair, times):
 def test_form_of_sizes_beyond_the_tiles_offsets():
     form = lambda **k: _lib.load_dense().i64h_linear_form(ctypes.addressof(_lib.Linear(**{**dict(A16=16, W=16, C=16, lda=64, ldc=64, M=64, N=64, K=64, batch=1), **k})))
     assert form(K=256, lda=256) == 6 and form() == 5 and form(lda=1 << 24) == -1 and form(M=0) == -1 and form(a_rows=16) == -1 and form(a_rows=16, a_height=64) == 5
+
+
+@pytest.mark.parametrize("width,experts,merged,n,ratio", [
+    # rows in bf16 over rows in 32 bits, both launches
+    (1024, 8, True, 3, 1.08), (1024, 8, True, 8, 1.06), (1024, 8, True, 16, 0.98), (1024, 8, True, 64, 0.89), (1024, 8, False, 3, 1.11), (1024, 8, False, 16, 1.10), (1024, 8, False, 27, 0.95),
+    (512, 8, True, 7, 1.38), (1024, 4, False, 3, 1.25), (1024, 4, False, 16, 1.21), (1024, 4, False, 27, 0.96), (2048, 2, False, 3, 1.40), (2048, 2, False, 16, 1.32), (2048, 2, False, 27, 0.85),
+    (2048, 4, False, 8, 1.28), (1536, 4, True, 5, 1.10), (1536, 4, True, 16, 0.90), (2048, 4, True, 5, 0.96), (2048, 8, True, 3, 0.81), (1280, 8, True, 5, 0.95), (4096, 8, True, 7, 0.91),
+    (1024, 4, True, 3, 1.02), (1024, 4, True, 16, 0.86), (1024, 15, True, 7, 0.91)])
+def test_mixtures_of_few_rows_on_the_faster_rows(width, experts, merged, n, ratio):
+    assert HybridRunner._streams(n, width, experts, merged) == (ratio > 1)

@@ -459,8 +459,18 @@ class HybridRunner:
         often as weights.  Microseconds of a pair's two launches, rows in fp32 | in bf16, width 2048, 768 inner: 16 experts of two, 100 tokens 37 | 39, 200
         44 | 41; 32 of two, 100 tokens 65 | 69, 320 69 | 69, 400 77 | 70; 64 of two, 200 tokens 113 | 121, 700 134 | 127; 64 of eight, 100 tokens 120 | 126, 200 136 | 126; 128 of
         eight, 100 tokens 217 | 226, 320 242 | 234; 8 of two (1792 inner), 65 tokens 48 | 45; with a shared one, 7 tokens 43 | 37, 33 58 | 54, 64 61 | 57, and of width 1024,
-        896 inner, 5 tokens 13.6 | 18.2, 27 17.7 | 16.3, 64 19.1 | 16.8 (hence the rule beside this one's call)."""
+        896 inner, 5 tokens 13.6 | 18.2, 27 17.7 | 16.3, 64 19.1 | 16.8 (hence the rule behind this one)."""
         return experts < 16 or pairs >= 20 * experts
+
+    @staticmethod
+    def _streams(n: int, width: int, experts: int, merged: bool) -> bool:
+        """Whether a mixture of few rows stays with rows in 32 bits, whose launches of at most 16 rows take 16 columns a workgroup: the second one, of `width` columns a group, has then
+        about two such workgroups a CU (256) at most, where the 64 x 64 tiles of rows in bf16 leave most CUs without one.  A shared expert's group has all rows, and with more than eight
+        its tile reads them less often than that.  Microseconds of both launches over five draws of experts, rows in fp32 | in bf16: 8 experts of 896 and a shared one, width 1024 (576
+        workgroups), 3 tokens 14.0 | 15.1, 8 17.0 | 18.1, 16 18.6 | 18.2, without it (512) 3 13.1 | 14.6, 16 15.9 | 17.5; 4 of 2048, width 1024 (256), 3 15.6 | 19.6, 16 18.2 | 22.1; 2 of
+        2048, width 2048 (256), 8 17.7 | 23.8; 8 of 2752, width 1024 (512), 8 33.0 | 35.8; 4 of 1344 and a shared one, width 1536 (480), 5 20.9 | 22.9, 16 25.4 | 22.9.  More workgroups: 4
+        of 896 and a shared one, width 2048 (640), 5 23.1 | 22.2; 8 of 1024 and a shared one, width 1280 (720), 5 21.1 | 20.0."""
+        return n <= (8 if merged else 16) and width * (experts + int(merged)) <= 576 * 16
 
     def _moe_merges(self) -> bool:
         """Whether the residual's launch sums a mixture's rows itself (i64h_streams_args.moe_y)."""
@@ -489,7 +499,7 @@ class HybridRunner:
         pair_wgt = B.pair_wgt if f.weigh_input else None      # the weight multiplies what the expert reads, not what it returns
         D.moe_plan(B.idx, n=n, top=top, experts=E, group_off=B.group_off, pair_token=B.pair_token, pair_row=B.pair_row, wgt=B.wgt, pair_wgt=pair_wgt, shared=merged)
         # the (token, expert) pairs lie grouped by expert: one launch runs every expert over its own rows, the counts stay on the device
-        x16 = h16 if self._fills(n * top, E) and (n > 8 or W * f.ff >= 1 << 21) else None      # (up to eight rows of small experts: 16 columns a workgroup)
+        x16 = h16 if self._fills(n * top, E) and not self._streams(n, W, E, merged) else None
         rows, groups = n * (top + int(merged)), E + int(merged)
         act, act16 = self._act(B.act, B.act16, rows, f.ff, x16)
         D.linear(h, gate_up, act, a16=x16, out16=act16, m=n, a_rows=B.pair_token[:rows], batch=groups, w_batch=2 * f.ff * W, exact=ex, group_off=B.group_off, row_scale=pair_wgt,
