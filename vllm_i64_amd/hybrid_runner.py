@@ -82,12 +82,14 @@ class HybridRunner:
     def _rounded(self, n: int, *widths: int) -> bool:
         """Whether a step of n rows rounds them where they are written: the wide tiles' rule, and below their rows as well, where the kernels of rows in bf16 are the faster ones
         from three rows on (64 rows, width 2048, us: 11392 columns 19.4 | 14.8, a pair of 5504 19.0 | 14.5, 2048 columns of 5504 22.5 | 16.6; steps of 64 rows 1608 | 1534, of 7
-        rows and width 1024 526 | 497).  One row under 1024 x 1024 takes 3.0 | 3.4."""
+        rows and width 1024 526 | 497).  One row under 1024 x 1024 takes 3.0 | 3.4.  Short k is soon read: up to eight rows of fewer than 1024 values, and up to 16 of fewer than 512, stay
+        in 32 bits.  1024 columns of 512, 3 rows 3.2 | 3.6, 8 3.4 | 3.6, 12 3.6 | 3.7, 32 5.0 | 3.9, a pair of 1344 4.1 | 4.9, 4.4 | 4.9, 4.6 | 5.0; columns of 256, 3 rows 2.8 | 3.6, 16
+        3.1 | 3.6, 48 4.1 | 3.8."""
         if self.exact or n <= self.FEW_ROWS:
             return False
-        top = 2 * max(n, self.max_ff + 256)
+        top, narrow = 2 * max(n, self.max_ff + 256), 1024 if n <= 8 else 512 if n <= 16 else 0
         for w in widths:      # (asked a few times a layer by steps that wait for the host)
-            if w % 64 or w * top >= self.WIDE_BYTES:
+            if w % 64 or w < narrow or w * top >= self.WIDE_BYTES:
                 return False
         return True
 
@@ -302,7 +304,9 @@ class HybridRunner:
                       q_src=src if m.q_rank else None, rot_mult=d["rot_mult"])
         # queries into latent space, per head: Q[:, h, :r] = q_unrotated[:, h, :] @ U_h
         D.linear(src, d["uk_t"], Q, m=n, n=r, k=m.dim, a_off=q_off, lda=src.shape[-1], ldc=H * width, batch=H, a_batch=qh, w_batch=r * m.dim, c_batch=width, exact=ex)
-        wide = self._wide_attention(n, H * r, r, width, cache) and r % 64 == 0 and self._rounded(n, H * m.vdim)
+        # (few rows: the value map's short k is faster over rows in 32 bits, by as much as an out-projection of 1024 loses; both, us, 8 heads of 256 to 64: 16 rows 7.0 | 7.7, 16 heads 3
+        # rows 6.9 | 7.9, 12 7.9 | 8.0, 16 8.3 | 8.0, 32 heads 3 rows 9.1 | 9.1, 8 10.0 | 9.2)
+        wide = self._wide_attention(n, H * r, r, width, cache) and r % 64 == 0 and self._rounded(n, H * m.vdim) and (n > 16 or H * m.vdim >= 2048)
         olat = (B.b16 if wide else B.b)[: n * H * r]
         keys = min(ctx_hint, m.window + 64) if m.window > 0 else ctx_hint
         for r0, r1, one_per_seq in runs:
@@ -466,11 +470,11 @@ class HybridRunner:
     def _streams(n: int, width: int, experts: int, merged: bool) -> bool:
         """Whether a mixture of few rows stays with rows in 32 bits, whose launches of at most 16 rows take 16 columns a workgroup: the second one, of `width` columns a group, has then
         about two such workgroups a CU (256) at most, where the 64 x 64 tiles of rows in bf16 leave most CUs without one.  A shared expert's group has all rows, and with more than eight
-        its tile reads them less often than that.  Microseconds of both launches over five draws of experts, rows in fp32 | in bf16: 8 experts of 896 and a shared one, width 1024 (576
+        its tile reads them less often than that (below a width of 1024, 16).  Microseconds of both launches over five draws of experts, rows in fp32 | in bf16: 8 experts of 896 and a shared one, width 1024 (576
         workgroups), 3 tokens 14.0 | 15.1, 8 17.0 | 18.1, 16 18.6 | 18.2, without it (512) 3 13.1 | 14.6, 16 15.9 | 17.5; 4 of 2048, width 1024 (256), 3 15.6 | 19.6, 16 18.2 | 22.1; 2 of
-        2048, width 2048 (256), 8 17.7 | 23.8; 8 of 2752, width 1024 (512), 8 33.0 | 35.8; 4 of 1344 and a shared one, width 1536 (480), 5 20.9 | 22.9, 16 25.4 | 22.9.  More workgroups: 4
+        2048, width 2048 (256), 8 17.7 | 23.8; 8 of 2752, width 1024 (512), 8 33.0 | 35.8; 4 of 1344 and a shared one, width 1536 (480), 5 20.9 | 22.9, 16 25.4 | 22.9; 8 of 512 and a shared one, width 512 (288), 12 12.2 | 13.6.  More workgroups: 4
         of 896 and a shared one, width 2048 (640), 5 23.1 | 22.2; 8 of 1024 and a shared one, width 1280 (720), 5 21.1 | 20.0."""
-        return n <= (8 if merged else 16) and width * (experts + int(merged)) <= 576 * 16
+        return n <= (8 if merged and width >= 1024 else 16) and width * (experts + int(merged)) <= 576 * 16
 
     def _moe_merges(self) -> bool:
         """Whether the residual's launch sums a mixture's rows itself (i64h_streams_args.moe_y)."""
