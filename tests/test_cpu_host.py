@@ -146,3 +146,17 @@ def test_attention_segments_of_a_step():
     assert attention_segments([], 0, 4) == [] and attention_segments([0, 0], 0, 4) == []
     with pytest.raises(ValueError):
         attention_segments([3, 1], 5, 4)
+
+
+def test_linear_takes_numbers_of_any_kind(monkeypatch):
+    """Switches and distances may come as numpy or float numbers, factors as tensors: a descriptor holds their values."""
+    import numpy as np
+    import torch
+    from vllm_i64_amd import ops_dense as D
+    seen = []
+    for name, stand_in in (("_chk", lambda *a: None), ("_stream", lambda: 0), ("ptr", lambda t: 0), ("_ref", lambda d: d), ("call_dense", lambda name, d, stream: seen.append(d))):
+        monkeypatch.setattr(D, name, stand_in)
+    a, w, out = torch.zeros(3, 32), torch.zeros(2, 8, 32, dtype=torch.bfloat16), torch.zeros(3, 16)
+    for exact, apart, scale in ((True, 8, 2.5), (np.bool_(True), np.int64(8), np.float32(2.5)), (1.0, 8.0, torch.tensor(2.5))):
+        D.linear(a, w, out, n=8, batch=2, w_batch=256, c_batch=8, bias=torch.zeros(2, 8), bias_batch=apart, exact=exact, epilogue=D.EPI_SCALE, scale=scale)
+        assert (seen[-1].exact, seen[-1].bias_batch, seen[-1].scale) == (1, 8, 2.5)

@@ -87,7 +87,7 @@ def linear(a: Optional[torch.Tensor], w: torch.Tensor, out: Optional[torch.Tenso
         if group_off.numel() < batch + 1:
             raise _lib.I64HError("linear: group_off needs batch + 1 entries")
     # (a step makes a few dozen of these: only what is not zero is put in)
-    d = _lib.Linear(lda=lda, W=ptr(w), ldc=ldc, M=M, N=N, K=K, batch=batch, exact=exact, epilogue=epilogue, scale=scale)
+    d = _lib.Linear(lda=lda, W=ptr(w), ldc=ldc, M=M, N=N, K=K, batch=batch, exact=int(exact), epilogue=epilogue, scale=scale)
     if a16 is None:
         d.A = ptr(a) + 4 * a_off
     else:
@@ -101,7 +101,7 @@ def linear(a: Optional[torch.Tensor], w: torch.Tensor, out: Optional[torch.Tenso
     if e is not None:
         d.E, d.lde, d.e_batch = ptr(e) + 4 * e_off, lde, e_batch
     if bias is not None:
-        d.bias, d.bias_batch = ptr(bias), bias_batch
+        d.bias, d.bias_batch = ptr(bias), int(bias_batch)
     if a_rows is not None:
         d.a_rows, d.a_height = ptr(a_rows), -(-a.numel() // lda)
     if group_off is not None:
