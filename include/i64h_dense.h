@@ -208,6 +208,7 @@ typedef struct {
     float softcap;       /* > 0: a score s (after scale and key scale, before any bias) becomes softcap * tanh(s / softcap) */
     int32_t keep_first;  /* with a window: the first positions of a sequence that stay visible to everyone */
     void* out16;         /* bf16, laid out as out, 16-byte aligned: receives the result rounded in out's place (matrix-core form over a bf16 cache only: modes 0 and 2 then take it whatever the knob says) */
+    int32_t seqs;        /* mode 3: how many sequences the rows belong to (0: not known).  A hint: which form is the faster one */
 } i64h_latent_attn_args;
 int i64h_set_latent_attn_decode_form(int32_t on); /* tuning / test knob: 1 (default) = mode 0 / 2 launches over bf16 caches of fitting sizes take the matrix-core form; 0 = all of them take the row form */
 int64_t i64h_latent_attn_workspace_floats(int64_t n, int32_t heads, int32_t kv_rank, int32_t splits);
@@ -455,6 +456,7 @@ typedef struct {
     int32_t window, keep_first;
     const float* sink_w;
     void* out16;         /* bf16, laid out as out, 16-byte aligned: receives the result rounded in out's place (matrix-core form over a bf16 cache only: modes 0 and 2 then take it whatever the knob says) */
+    int32_t seqs;        /* as in i64h_latent_attn_args */
 } i64h_kattn_args;
 int64_t i64h_kattn_workspace_floats(int64_t n, int32_t heads, int32_t kv_heads, int32_t dim, int32_t splits);
 int i64h_kattn(const i64h_kattn_args* d, void* stream);

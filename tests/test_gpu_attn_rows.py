@@ -365,3 +365,28 @@ def test_latent_result_in_bf16(dev, mode, splits, H, r, e):
         D.latent_attn(args[0], cache.float(), *args[2:], out=out16, **kw)
     with pytest.raises(Exception, match="bf16"):
         D.latent_attn(*args, out=out16, **{**kw, "mode": 1, "splits": 1})
+
+
+@pytest.mark.parametrize("H,G,dim", [(32, 8, 64), (8, 2, 64), (16, 4, 128)])
+@pytest.mark.parametrize("lens,past", [([3] * 64, 40), ([2] * 150, 9), ([16] * 24, 0)])
+def test_32_bit_rows_of_many_sequences_by_their_number(dev, H, G, dim, lens, past):
+    """The number of sequences chooses between forms whose sums run in another order, and nothing else: with and without it, against 64 bits."""
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator().manual_seed(len(lens))
+    bt, pos, slots, blocks = pages(lens, [past] * len(lens), 16, g)
+    n, w = int(pos.numel()), 2 * dim
+    cache = torch.randn(blocks, 16, G * w, generator=g)
+    q = torch.randn(n, H, w, generator=g) * dim ** -0.5
+    q[:, :, :dim] = 0
+    sink = torch.randn(H, generator=g)
+    args = (q.to(dev).view(n, -1), cache.to(dev), None, bt.to(dev), slots.to(dev), pos.to(dev))
+    got = [D.kattn(*args, chunk=0, bias=None, sink=True, sink_w=sink.to(dev), heads=H, kv_heads=G, dim=dim, vdim=dim, out=torch.full((n, H * dim), 7.0, device=dev), n=n, mode=3, seqs=k).double().cpu().view(n, H, dim)
+           for k in (0, len(lens))]
+    at = 0
+    for i, m in enumerate(lens):
+        j = torch.arange(m + past)
+        rows = cache[bt[i].long()[j // 16], j % 16].view(m + past, G, w).repeat_interleave(H // G, 1).transpose(0, 1)
+        ref = reference(q[at:at + m, :, dim:], rows[..., dim:], rows[..., :dim], pos[at:at + m], 1.0, 0, 0, 0.0, sink)
+        for x in got:
+            assert torch.allclose(x[at:at + m], ref, atol=4e-5, rtol=2e-5), (i, float((x[at:at + m] - ref).abs().max()))
+        at += m

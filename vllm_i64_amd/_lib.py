@@ -273,7 +273,7 @@ class LatentAttn(ctypes.Structure):
     _fields_ = [("Q", _P), ("cache", _P), ("cache_dtype", _I), ("block_table", _P), ("max_blocks_per_seq", _I), ("block_size", _I),
                 ("slot_ids", _P), ("positions", _P), ("window", _I), ("scale", _F), ("out", _P), ("n", _L), ("heads", _I), ("kv_rank", _I),
                 ("rot_dim", _I), ("mode", _I), ("splits", _I), ("workspace", _P), ("row_stride", _I), ("kv_groups", _I), ("chunk", _I), ("kscale", _P),
-                ("bias", _P), ("bias_rows", _I), ("sink", _I), ("key_off", _I), ("sink_w", _P), ("softcap", _F), ("keep_first", _I), ("out16", _P)]
+                ("bias", _P), ("bias_rows", _I), ("sink", _I), ("key_off", _I), ("sink_w", _P), ("softcap", _F), ("keep_first", _I), ("out16", _P), ("seqs", _I)]
 
 
 class EmbedBigram(ctypes.Structure):
@@ -327,7 +327,7 @@ class KAttn(ctypes.Structure):
     _fields_ = [("Q", _P), ("cache", _P), ("cache_dtype", _I), ("kscale", _P), ("block_table", _P), ("max_blocks_per_seq", _I), ("block_size", _I),
                 ("slot_ids", _P), ("positions", _P), ("chunk", _I), ("bias", _P), ("bias_rows", _I), ("sink", _I), ("out", _P), ("n", _L), ("heads", _I),
                 ("kv_heads", _I), ("dim", _I), ("mode", _I), ("splits", _I), ("workspace", _P), ("vdim", _I), ("softcap", _F),
-                ("window", _I), ("keep_first", _I), ("sink_w", _P), ("out16", _P)]
+                ("window", _I), ("keep_first", _I), ("sink_w", _P), ("out16", _P), ("seqs", _I)]
 
 
 class KvPrep(ctypes.Structure):

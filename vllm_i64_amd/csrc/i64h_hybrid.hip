@@ -1154,7 +1154,7 @@ int i64h_kattn(const i64h_kattn_args* dp, void* stream) {
         a.row_stride = d.kv_heads * gs, a.kv_groups = d.kv_heads, a.chunk = d.chunk, a.kscale = d.kscale, a.bias = d.bias, a.bias_rows = d.bias_rows;
         a.sink = d.sink, a.sink_w = d.sink_w, a.softcap = d.softcap;
         a.key_off = d.vdim > 0 ? d.vdim : 0;
-        a.out16 = d.out16;
+        a.out16 = d.out16, a.seqs = d.seqs;
         I64H_CHECK_ARG(bf16_form || !d.out16, "kattn: a result in bf16 belongs to the matrix-core form over a bf16 cache");
         if (latent_rows_f32_ok(a)) return latent_rows_f32_run(a, stream);
         return i64h_latent_attn(&a, stream);

@@ -746,6 +746,8 @@ __global__ __launch_bounds__(256, 2) void latent_attn_rows_kernel(const i64h_lat
 // well for heads of 64, 113 for latent rows, whose 320 registers do not stay where the products take them.  Microseconds, the kernel above | this:
 //   16 heads over one row of 288: 8 prompts of 512 125 | 74, one of 77 19 | 12.5, 64 portions of 3 behind 500 69 | 41; 32 heads, 229 behind 512 83 | 43
 //   16 heads of 64 over 4: 8 x 512 44 | 31, one of 77 9.8 | 9.5; 32 over 8, prompts of 1531, 257, 64, 3, 1101 73 | 51; 24 heads of 128 over 8, 8 x 512 89 | 62
+// Heads of 128 whose every context is one tile are slower, by the tiles past the end that are loaded all the same: 24 over 8, 40 prompts of 16 17.7 | 19.4, 300 portions of 2
+// behind 30 67 | 75.  (A way of their own for such runs took 70, and 3 to 40 % more in the other launches of this kernel: registers.)
 template <int D>
 __device__ __forceinline__ int lt_swizzle(int row) {
     if constexpr (D % 128 == 0) return (row & 7) << 1 | (row >> 3 & 1);      // every row starts in bank 0: sixteen places, neighbours in pairs
@@ -1476,20 +1478,24 @@ int latent_rows_f32_run(const i64h_latent_attn_args& d, void* stream) {
     const size_t bytes = ((size_t)32 * (kcols + 4) + (size_t)d.kv_rank * LT_FLD) * 4 + 129 * 4;
     const bool extra = d.kscale || d.bias || d.softcap > 0.0f;
     auto exact = [&](int width, int rank, int off) { return !extra && D == width && d.kv_rank == rank && d.key_off == off; };
-    // quarters: for latent rows always (they were faster in every launch timed), for heads of 64 and 128 while the workgroups of four waves on their own
-    // rows would be fewer than about 400 (256 CUs, two or more a CU): the figures beside the kernel
+    // quarters: for latent rows always (they were faster in every launch timed), for heads of 64 and 128 while the workgroups of four waves on their own rows would be at most
+    // 400 (256 CUs, two or more a CU; the figures beside the kernel), 256 where a row sees few keys.  Several sequences in 16 rows are as many workgroups, of which a quarter's
+    // reads for itself what four heads of the other form share.  Microseconds, four heads over their rows | quarters: 64 portions of 3 behind 500, 32 heads over 8 (96 of six sequences)
+    // 84 | 100, 16 over 4 (48 of six) 62.5 | 62.5, 8 over 2 62 | 57; 300 of 2 behind 30, 8 over 2 (76 of eight) 12.7 | 19.4; 40 of 16, 32 over 8 (320) 11.9 | 12.6
     const int64_t wgs = (d.n + 15) / 16 * d.heads;
     int shares = 4;
     while (shares < 16 && wgs * shares < 2048) shares *= 2;
     while (shares > d.n) shares /= 2;
+    const int64_t many = hw > 1 && d.seqs > 0 && d.seqs <= d.n ? ((int64_t)d.seqs * 16 + d.n - 1) / d.n : 1;      // sequences in 16 rows
+    const bool brief = (d.window > 0 && d.window <= 256) || (hw > 1 && d.seqs > 0 && d.n <= 16 * (int64_t)d.seqs), few = grid.x * many <= (brief ? 256 : 400);
     auto quarters = [&](auto kern) { hipLaunchKernelGGL(kern, dim3((unsigned)wgs, (unsigned)shares), dim3(256), 0, (hipStream_t)stream, d); };
 #define LT_ROWS(KC, NB) do { \
         if (extra) hipLaunchKernelGGL((latent_attn_rows_f32_kernel<KC, NB, true>), grid, dim3(256), bytes, (hipStream_t)stream, d, hw); \
         else hipLaunchKernelGGL((latent_attn_rows_f32_kernel<KC, NB, false>), grid, dim3(256), bytes, (hipStream_t)stream, d, hw); \
     } while (0)
     if (exact(288, 256, 0)) quarters(latent_attn_rows_f32_quarters_kernel<288, 256, 0>);
-    else if (grid.x <= 400 && exact(128, 64, 64)) quarters(latent_attn_rows_f32_quarters_kernel<128, 64, 64>);
-    else if (grid.x <= 400 && exact(256, 128, 128)) quarters(latent_attn_rows_f32_quarters_kernel<256, 128, 128>);
+    else if (few && exact(128, 64, 64)) quarters(latent_attn_rows_f32_quarters_kernel<128, 64, 64>);
+    else if (few && exact(256, 128, 128)) quarters(latent_attn_rows_f32_quarters_kernel<256, 128, 128>);
     else if (chunks <= 4 && d.kv_rank <= 64) LT_ROWS(4, 4);
     else if (chunks <= 8 && d.kv_rank <= 128) LT_ROWS(8, 8);
     else if (chunks <= 18) LT_ROWS(18, 16);

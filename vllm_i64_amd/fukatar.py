@@ -137,10 +137,10 @@ class FukatarModel(HybridRunner):
         return d
 
     # ---- mixers: the input is B.h; the result lands in B.y (and B.y2 for the second of two side-by-side mixers) ----
-    def _attention(self, B, d, l, n, positions, slot_ids, kvc, runs, ctx_hint) -> None:
+    def _attention(self, B, d, l, n, positions, slot_ids, kvc, runs, ctx_hint, nseg) -> None:
         P = B.p[: n * d["n_in"]].view(n, d["n_in"])
         D.linear(B.h, d["w_in"], P, exact=self.exact)
-        self._rotary_attention(B, d, d["m"], P, l, n, positions, slot_ids, kvc, runs, ctx_hint, B.y)
+        self._rotary_attention(B, d, d["m"], P, l, n, positions, slot_ids, kvc, runs, ctx_hint, B.y, nseg=nseg)
 
     def _latent(self, B, d, l, n, positions, slot_ids, kvc, runs, ctx_hint) -> None:
         P = B.p[: n * d["n_in"]].view(n, d["n_in"])
@@ -151,7 +151,7 @@ class FukatarModel(HybridRunner):
         a, r = d["m"].left, d["m"].right
         P = B.p[: n * d["n_in"]].view(n, d["n_in"])
         D.linear(B.h, d["w_in"], P, exact=self.exact)
-        self._rotary_attention(B, d, a, P, l, n, positions, slot_ids, kvc, runs, ctx_hint, B.y)
+        self._rotary_attention(B, d, a, P, l, n, positions, slot_ids, kvc, runs, ctx_hint, B.y, nseg=nseg)
         self._gated_delta(B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, single, B.y2, work)
 
     @torch.no_grad()
@@ -194,7 +194,7 @@ class FukatarModel(HybridRunner):
             if d["type"] == "latent_attention":
                 self._latent(B, d, l, n, positions, slot_ids, kvc, runs, hint)
             elif d["type"] == "attention":
-                self._attention(B, d, l, n, positions, slot_ids, kvc, runs, hint)
+                self._attention(B, d, l, n, positions, slot_ids, kvc, runs, hint, nseg)
             else:
                 self._parallel(B, d, l, n, positions, slot_ids, kvc, seg, nseg, runs, hint, single, work)
                 write.update(y2=B.y2, yn_w=d["out_left"], y2n_w=d["out_right"])

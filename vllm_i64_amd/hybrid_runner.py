@@ -221,10 +221,11 @@ class HybridRunner:
 
     # ---- attention over grouped key / value heads, separate keys and values in one cached row ----
     def _kattn(self, B, a, Q, O, rows, kvc, slot_ids, positions, runs, ctx_hint: int, *, bias=None, softcap: float = 0.0, window: int = 0,
-               keep_first: int = 0, sink_w=None) -> None:
+               keep_first: int = 0, sink_w=None, nseg: int = 0) -> None:
         """Runs of rows that are one per sequence (a wave takes a token's query heads of one key head, the keys dealt to several waves) and
-        runs of prompt portions (a wave takes 16 consecutive rows of one head), each one launch."""
+        runs of prompt portions (a wave takes 16 consecutive rows of one head), each one launch.  nseg: the step's sequences (0: not known)."""
         gs = a.vdim + a.dim
+        portions = max(0, nseg - sum(r1 - r0 for r0, r1, one in runs if one)) if self.exact else 0      # (what the choice between the 32-bit forms asks)
         keys = min(ctx_hint, window + keep_first + 64) if window > 0 else ctx_hint
         for r0, r1, one_per_seq in runs:
             splits, ws = 1, None
@@ -233,7 +234,7 @@ class HybridRunner:
                                           lambda s: D.kattn_workspace_floats(r1 - r0, a.heads, a.kv_heads, a.vdim, s))
             D.kattn(Q[r0:r1], rows, None, kvc.block_table, slot_ids[r0:r1], positions[r0:r1], chunk=0, bias=bias, sink=sink_w is not None,
                     heads=a.heads, kv_heads=a.kv_heads, dim=a.dim, vdim=a.vdim, out=O[r0:r1], n=r1 - r0, mode=2 if one_per_seq else 3, splits=splits,
-                    workspace=ws, softcap=softcap, window=window, keep_first=keep_first, sink_w=sink_w)
+                    workspace=ws, softcap=softcap, window=window, keep_first=keep_first, sink_w=sink_w, seqs=portions)
 
     def _rotary_tables(self, a, d: dict) -> None:
         """Frequency tables of a rotated attention: evaluated in 64 bits on the host, rounded once to fp32."""
@@ -244,7 +245,7 @@ class HybridRunner:
         if a.rot is not None and a.rotate_values:
             d["v_freq"] = self._f(torch.tensor([a.rot.base ** (-2.0 * i / a.vdim) for i in range(a.vdim // 2)], dtype=torch.float64))
 
-    def _rotary_attention(self, B, d, a, P, l, n, positions, slot_ids, kvc, runs, ctx_hint, out, scale: float = 1.0) -> None:
+    def _rotary_attention(self, B, d, a, P, l, n, positions, slot_ids, kvc, runs, ctx_hint, out, scale: float = 1.0, nseg: int = 0) -> None:
         """Rotated attention on the projection rows P (already computed; columns d["q_off"], d["k_off"], d["v_off"]): prep -> paged
         [values | keys] rows and query rows, attention, the turn back and the head gate, out-projection (times `scale`) into `out`."""
         gs = a.vdim + a.dim
@@ -257,7 +258,7 @@ class HybridRunner:
         behind = d["v_freq"] is not None or a.head_gate
         wide = not behind and self._wide_attention(n, a.heads * a.vdim, a.vdim, gs, rows)
         O = self._as16(B.b16, n, a.heads * a.vdim) if wide else B.b[: n * a.heads * a.vdim].view(n, a.heads * a.vdim)
-        self._kattn(B, a, Q, O, rows, kvc, slot_ids, positions, runs, ctx_hint, softcap=a.softcap, window=a.window, keep_first=a.keep_first, sink_w=d.get("sink"))
+        self._kattn(B, a, Q, O, rows, kvc, slot_ids, positions, runs, ctx_hint, softcap=a.softcap, window=a.window, keep_first=a.keep_first, sink_w=d.get("sink"), nseg=nseg)
         if behind:
             D.rot_post(O, heads=a.heads, vdim=a.vdim, interleaved=a.interleaved, v_freq=d["v_freq"], positions=positions,
                        gate=P if a.head_gate else None, gate_off=d.get("g_off", 0), ldg=P.shape[-1], n=n)

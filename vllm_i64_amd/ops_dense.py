@@ -422,11 +422,11 @@ def kattn_prep(p: torch.Tensor, *, q_off: int, k_off: int, heads: int, kv_heads:
 def kattn(q: torch.Tensor, cache: torch.Tensor, kscale: torch.Tensor, block_table: torch.Tensor, slot_ids: torch.Tensor, positions: torch.Tensor, *,
           chunk: int, bias: Optional[torch.Tensor], sink: bool, heads: int, kv_heads: int, dim: int, out: torch.Tensor, n: Optional[int] = None,
           mode: int = 0, splits: int = 1, workspace: Optional[torch.Tensor] = None, vdim: int = 0, softcap: float = 0.0,
-          window: int = 0, keep_first: int = 0, sink_w: Optional[torch.Tensor] = None) -> torch.Tensor:
+          window: int = 0, keep_first: int = 0, sink_w: Optional[torch.Tensor] = None, seqs: int = 0) -> torch.Tensor:
     """See i64h_kattn.  q, out fp32 [n, heads * dim]; bias fp32 [distances, heads].  vdim > 0: separate values - the cache rows are
     [kv_heads, vdim + dim], q fp32 [n, heads, vdim + dim], out fp32 [n, heads * vdim], kscale may be None.  window > 0: the last `window`
     positions and the first keep_first ones are seen.  sink_w fp32 [heads]: the sink's score per head.  out: fp32 or, in the matrix-core form over a bf16
-    cache, bf16 (the result rounded)."""
+    cache, bf16 (the result rounded).  seqs: how many sequences the rows of a mode 3 launch belong to (0: not known)."""
     half = out.dtype == torch.bfloat16
     _chk(q, torch.float32, "q"), _chk(out, None if half else torch.float32, "out"), _chk(cache, None, "cache")
     if kscale is not None or vdim <= 0:
@@ -457,7 +457,7 @@ def kattn(q: torch.Tensor, cache: torch.Tensor, kscale: torch.Tensor, block_tabl
                    max_blocks_per_seq=block_table.shape[1], block_size=cache.shape[-2], slot_ids=ptr(slot_ids), positions=ptr(positions), chunk=int(chunk),
                    bias=ptr(bias), bias_rows=bias.shape[0] if bias is not None else 0, sink=int(bool(sink)), out=0 if half else ptr(out), out16=ptr(out) if half else 0, n=rows, heads=heads,
                    kv_heads=kv_heads, dim=dim, mode=int(mode), splits=int(splits) if splits > 1 else 1, workspace=ptr(workspace) if splits > 1 else 0,
-                   vdim=int(vdim), softcap=float(softcap), window=int(window), keep_first=int(keep_first), sink_w=ptr(sink_w))
+                   vdim=int(vdim), softcap=float(softcap), window=int(window), keep_first=int(keep_first), sink_w=ptr(sink_w), seqs=int(seqs))
     call_dense("i64h_kattn", _ref(d), _stream())
     return out
 

@@ -191,7 +191,7 @@ class PukatarModel(HybridRunner):
             P = B.p[: n * d["ld"]].view(n, d["ld"])
             D.linear(B.h, d["w_in"], P, a16=B.h16, exact=ex)
             if d["type"] == "attention":
-                self._rotary_attention(B, d, d["m"], P, r, n, positions, slot_ids, kvc, runs, hint, B.y)
+                self._rotary_attention(B, d, d["m"], P, r, n, positions, slot_ids, kvc, runs, hint, B.y, nseg=nseg)
             else:
                 self._gated_delta(B, d, d["m"], P, r, n, positions, slot_ids, kvc, seg, nseg, single, B.y, work)
             write = dict(y=B.y, out_w=self.ones1)

@@ -137,7 +137,7 @@ class VepelixModel(HybridRunner):
             self._latent_attention(B, d, m, P, r, n, positions, slot_ids, kvc, runs, hint, B.y)
             return dict(y=B.y)
         with self._beside(n):      # attention and recurrence share nothing but the projection rows
-            self._rotary_attention(B, d, m.left, P, r, n, positions, slot_ids, kvc, runs, hint, B.y, m.left_scale)
+            self._rotary_attention(B, d, m.left, P, r, n, positions, slot_ids, kvc, runs, hint, B.y, m.left_scale, nseg)
         self._gated_linear(B, d, m.right, P, r, n, positions, slot_ids, kvc, seg, nseg, B.y2, m.right_scale, work)
         self._meet(n)
         return dict(y=B.y, y2=B.y2)
