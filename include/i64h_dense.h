@@ -210,7 +210,7 @@ typedef struct {
     void* out16;         /* bf16, laid out as out, 16-byte aligned: receives the result rounded in out's place (matrix-core form over a bf16 cache only: modes 0 and 2 then take it whatever the knob says) */
     int32_t seqs;        /* mode 3: how many sequences the rows belong to (0: not known).  A hint: which form is the faster one */
 } i64h_latent_attn_args;
-int i64h_set_latent_attn_decode_form(int32_t on); /* tuning / test knob: 1 (default) = mode 0 / 2 launches over bf16 caches of fitting sizes take the matrix-core form; 0 = all of them take the row form */
+int i64h_set_latent_attn_decode_form(int32_t on); /* tuning / test knob: 1 (default) = mode 0 / 2 launches over bf16 caches of fitting sizes take the matrix-core form; 0 = they take the row form, but for those whose result is wanted in bf16 (out16), which only the matrix-core form gives */
 int64_t i64h_latent_attn_workspace_floats(int64_t n, int32_t heads, int32_t kv_rank, int32_t splits);
 int i64h_latent_attn(const i64h_latent_attn_args* d, void* stream);
 

@@ -786,7 +786,7 @@ __global__ __launch_bounds__(GS * 64, 3) void paged_attn_prefill_direct_kernel(c
             constexpr int C = decltype(cur)::value, F = decltype(free)::value;
             const Row then = look_up(tile + 2);
             ok[F] = ok_of(tile + 1, next);
-            load(next, ok[F], free);      // (past the end the last tile again, which nobody reads: without a branch the loads on their way are the same everywhere)
+            load(next, ok[F], free);      // (past the end every lane asks for row 0 of page 0, which every cache has and nobody reads: without a branch the loads on their way are the same everywhere)
             next = then;
             if (!ok[C]) return;
             const unsigned short* Kb = stage(cur);
@@ -1622,6 +1622,7 @@ int i64h_paged_attn(const float* q, const void* k_cache, const void* v_cache, in
         else if (gs == 4) PFG(4);
         else PFG(8);
 #undef PFG
+#undef PFD
 #undef PFB
 #undef PF
         I64H_CHECK_LAUNCH();

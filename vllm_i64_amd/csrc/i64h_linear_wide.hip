@@ -320,11 +320,11 @@ static void launch(const i64h_linear& d, hipStream_t s) {
     else hipLaunchKernelGGL((linear_wide_kernel<false, BM, BN, NWM, NWN, NS, PER_CU>), grid, dim3(64 * NWM * NWN), 0, s, d, nt, (int)mt, vecC);
 }
 
-// ---- up to 64 rows under few columns: 16 columns a workgroup, the steps of k dealt to its waves ------------------------------------------------
+// ---- up to 128 rows under few columns: 16 columns and 64 rows a workgroup, the steps of k dealt to its waves ------------------------------------
 // What bounds it: the latency of a step, a few of them on their way.  A 64 x 64 tile walks all of k alone, and 1024 or 2048 columns are 16 or 32 of them on 256 CUs.
 // Here every wave takes every NW-th step of 64 k for 16 columns and all rows, with loads, LDS and waits of its own: nobody meets before the end, where the waves' sums
 // are added in their order.  The rows are read once for 16 columns, from L2: at 64 rows of 5504 that is 90 MB, and the launch's time.  Microseconds in replayed graphs, the
-// weights of twelve launches in turn, the fp32 rows' kernels | 64 x 64 tiles | here:
+// weights of twelve launches in turn, the fp32 rows' kernels | 64 x 64 tiles | here (more than 64 rows: two tiles of them):
 //   rows:                   3                     16                   64                   77                  128
 //   1024 x 1024     3.5 | 4.9 | 3.5     4.6 | 5.0 | 3.4      5.8 | 5.1 | 4.3      5.7 | 5.1 | 4.5      5.8 | 5.1 | 4.5
 //   1024 x 2752     6.6 | 9.3 | 4.7     9.6 | 9.3 | 5.1      9.4 | 10.5 | 7.6     9.3 | 9.4 | 6.9      9.5 | 10.1 | 7.6

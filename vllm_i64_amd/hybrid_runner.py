@@ -69,19 +69,13 @@ class HybridRunner:
         if self._forks(n):
             torch.cuda.current_stream().wait_stream(self.side)
 
-    # ---- rows that only Linears read: their producer rounds them to bf16 once where enough rows share a tile ----
-    WIDE_ROWS = 64                  # more rows than this
+    # ---- rows that only Linears read: their producer rounds them to bf16 once ----
     WIDE_BYTES = 0xfffffff0 - 64    # what the 32-bit offsets of the tiles on such rows reach: gathered rows, and the gate and up rows of a pair's weight
-
-    def _wide(self, n: int, *widths: int) -> bool:
-        """Whether Linears over rows of these widths read them in bf16 (the values their tiles would round to: results are the same)."""
-        return not self.exact and n > self.WIDE_ROWS and all(w % 64 == 0 and 2 * w * max(n, self.max_ff + 256) < self.WIDE_BYTES for w in widths)
-
     FEW_ROWS = 2                    # up to this many rows: the forms that stream the weights past rows in 32 bits
 
     def _rounded(self, n: int, *widths: int) -> bool:
-        """Whether a step of n rows rounds them where they are written: the wide tiles' rule, and below their rows as well, where the kernels of rows in bf16 are the faster ones
-        from three rows on (64 rows, width 2048, us: 11392 columns 19.4 | 14.8, a pair of 5504 19.0 | 14.5, 2048 columns of 5504 22.5 | 16.6; steps of 64 rows 1608 | 1534, of 7
+        """Whether a step of n rows rounds them where they are written (the values the Linears' tiles would round to: results are the same), for rows of these widths: whatever their
+        number within the tiles' offsets, and below 65 as well, where the kernels of rows in bf16 are the faster ones from three rows on (64 rows, width 2048, us: 11392 columns 19.4 | 14.8, a pair of 5504 19.0 | 14.5, 2048 columns of 5504 22.5 | 16.6; steps of 64 rows 1608 | 1534, of 7
         rows and width 1024 526 | 497).  One row under 1024 x 1024 takes 3.0 | 3.4.  Short k is soon read: up to eight rows of fewer than 1024 values, and up to 16 of fewer than 512, stay
         in 32 bits.  1024 columns of 512, 3 rows 3.2 | 3.6, 8 3.4 | 3.6, 12 3.6 | 3.7, 32 5.0 | 3.9, a pair of 1344 4.1 | 4.9, 4.4 | 4.9, 4.6 | 5.0; columns of 256, 3 rows 2.8 | 3.6, 16
         3.1 | 3.6, 48 4.1 | 3.8."""
@@ -100,7 +94,7 @@ class HybridRunner:
 
     @staticmethod
     def _as16(t16: torch.Tensor, n: int, width: int) -> torch.Tensor:
-        """The memory of a buffer of fp32 rows as rows in bf16."""
+        """The first rows of a buffer's bf16 view (which shares the memory of its fp32 rows) as a matrix."""
         return t16[: n * width].view(n, width)
 
     # ---- tensors by name and shape, in the two forms the kernels read ----
