@@ -235,3 +235,22 @@ def test_blocks_of_a_tile_follow_each_other(dev, form):
         out, out16 = torch.empty(M, N, device=dev), torch.empty(M, N, device=dev, dtype=torch.bfloat16)
         D.linear(None, w16, out, a16=a16, out16=out16)
         assert torch.equal(out.long(), want) and torch.equal(out16.long(), want)
+
+
+@pytest.mark.parametrize("M,N,K", [(7, 64, 256), (16, 100, 576), (33, 48, 320), (70, 96, 1088), (128, 256, 256)])
+def test_rows_that_are_no_numbers_beside_finite_ones(dev, M, N, K):
+    """16 columns a workgroup: a row with an infinity or NaN is its own row's business, in the waves' sums as well, and a weight that is one its column's."""
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator().manual_seed(M)
+    a, w = torch.randn(M, K, generator=g).bfloat16(), (torch.randn(N, K, generator=g) / math.sqrt(K)).bfloat16()
+    clean = D.linear(None, w.to(dev), torch.empty(M, N, device=dev), a16=a.to(dev))
+    assert torch.isfinite(clean).all()
+    bad = torch.tensor([0, M // 2, M - 1])
+    a[0, K - 1], a[M // 2, 0], a[M - 1, K // 2] = float("inf"), float("nan"), float("-inf")
+    w[N - 1, 5] = float("nan")
+    out, out16 = torch.full((M, N), 7.0, device=dev), torch.full((M, N), 7.0, device=dev, dtype=torch.bfloat16)
+    D.linear(None, w.to(dev), out, a16=a.to(dev), out16=out16)
+    good = torch.ones(M, dtype=torch.bool)
+    good[bad] = False
+    assert torch.equal(out.cpu()[good, :N - 1], clean.cpu()[good, :N - 1]) and not torch.isfinite(out.cpu()[bad]).any() and out[:, N - 1].isnan().all()
+    assert torch.equal(out16.isnan(), out.isnan()) and torch.equal(out16.nan_to_num(0.0), out.bfloat16().nan_to_num(0.0))

@@ -1479,7 +1479,8 @@ int latent_rows_f32_run(const i64h_latent_attn_args& d, void* stream) {
     const bool extra = d.kscale || d.bias || d.softcap > 0.0f;
     auto exact = [&](int width, int rank, int off) { return !extra && D == width && d.kv_rank == rank && d.key_off == off; };
     // quarters: for latent rows always (they were faster in every launch timed), for heads of 64 and 128 while the workgroups of four waves on their own rows would be at most
-    // 400 (256 CUs, two or more a CU; the figures beside the kernel), 256 where a row sees few keys.  Several sequences in 16 rows are as many workgroups, of which a quarter's
+    // 400 (256 CUs, two or more a CU; the figures beside the kernel: 1000 rows of 32 heads over 8 would be 504 and still gain, 2000 of them and 2000 of 24 heads of 128 over 8 lose), 256
+    // where a row sees few keys.  Several sequences in 16 rows are as many workgroups, of which a quarter's
     // reads for itself what four heads of the other form share.  Microseconds, four heads over their rows | quarters: 64 portions of 3 behind 500, 32 heads over 8 (96 of six sequences)
     // 84 | 100, 16 over 4 (48 of six) 62.5 | 62.5, 8 over 2 62 | 57; 300 of 2 behind 30, 8 over 2 (76 of eight) 12.7 | 19.4; 40 of 16, 32 over 8 (320) 11.9 | 12.6
     const int64_t wgs = (d.n + 15) / 16 * d.heads;
