@@ -124,7 +124,9 @@ def test_tiles_by_size_are_among_the_fastest(G, rows, M, N, K, pair, times):
 
 def test_form_of_sizes_beyond_the_tiles_offsets():
     form = lambda **k: _lib.load_dense().i64h_linear_form(ctypes.addressof(_lib.Linear(**{**dict(A16=16, W=16, C=16, lda=64, ldc=64, M=64, N=64, K=64, batch=1), **k})))
-    assert form(K=256, lda=256) == 6 and form() == 5 and form(lda=1 << 24) == -1 and form(M=0) == -1 and form(a_rows=16) == -1 and form(a_rows=16, a_height=64) == 5
+    assert form(K=256, lda=256) == 6 and form() == 5 and form(M=32, N=5120, K=4096, lda=4096) == 6 and form(M=32, N=8193, K=4096, lda=4096) != 6
+    assert form(M=48, N=5120, K=4096, lda=4096) != 6 and form(M=16, N=5120, K=2048, lda=2048) != 6 and form(M=128, N=2048, K=2048, lda=2048) == 6 and form(M=129, N=64, K=256, lda=256) != 6
+    assert form(lda=64) == 5 and form(lda=1 << 24) == -1 and form(M=0) == -1 and form(a_rows=16) == -1 and form(a_rows=16, a_height=64) == 5
 
 
 @pytest.mark.parametrize("width,experts,merged,n,ratio", [

@@ -254,3 +254,20 @@ def test_rows_that_are_no_numbers_beside_finite_ones(dev, M, N, K):
     good[bad] = False
     assert torch.equal(out.cpu()[good, :N - 1], clean.cpu()[good, :N - 1]) and not torch.isfinite(out.cpu()[bad]).any() and out[:, N - 1].isnan().all()
     assert torch.equal(out16.isnan(), out.isnan()) and torch.equal(out16.nan_to_num(0.0), out.bfloat16().nan_to_num(0.0))
+
+
+@pytest.mark.parametrize("M,N,K,thin", [(3, 4112, 3072, True), (32, 8192, 3072, True), (33, 4112, 3072, False), (32, 8193, 3072, False), (32, 4112, 3008, False)])
+def test_two_rounds_of_narrow_tiles_under_a_long_k(dev, M, N, K, thin):
+    """Either side of the line up to which 16 columns a workgroup are taken for two rounds: the bits of that form, or of the 64 x 64 tiles; close to 64 bits."""
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator(device=dev).manual_seed(M)
+    a, w = torch.randn(M, K, generator=g, device=dev).bfloat16(), (torch.randn(N, K, generator=g, device=dev) / math.sqrt(K)).bfloat16()
+    out, forced = torch.empty(M, N, device=dev), torch.empty(M, N, device=dev)
+    D.linear(None, w, out, a16=a)
+    D.call_dense("i64h_set_linear_skinny", 112 if thin else 96)
+    try:
+        D.linear(None, w, forced, a16=a)
+    finally:
+        D.call_dense("i64h_set_linear_skinny", 3)
+    assert torch.equal(out, forced)
+    assert float((out.double() - a.double() @ w.double().t()).abs().max()) <= 2e-6 * K ** 0.5 + 1e-5

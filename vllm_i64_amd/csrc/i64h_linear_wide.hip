@@ -331,7 +331,7 @@ static void launch(const i64h_linear& d, hipStream_t s) {
 //   2048 x 2048     5.7 | 7.8 | 4.7     7.9 | 7.8 | 4.8      8.3 | 8.2 | 6.6      8.3 | 7.9 | 6.4      8.5 | 8.2 | 6.9
 //   2048 x 5504     11.8 | 21.6 | 8.2   23.8 | 22.1 | 9.5    22.5 | 27.1 | 16.6   22.0 | 22.2 | 13.2   22.1 | 25.9 | 16.5
 //   4352 x 2048                         8.4 | 8.1 | 8.4      9.8 | 8.5 | 12.5
-// (more than 256 tiles, the last row: a second round)
+// (more than 256 tiles, the last row: a second round, worth it only under a long k)
 template <int MB, int NW, int NS, int EPI>
 __global__ __launch_bounds__(64 * NW, NW / 4) void linear_thin_kernel(const i64h_linear p, const int vecC) {
     constexpr int LA = 2 * MB, LB = 2, ROWS = 16 * MB + 16, STAGE = NW * ROWS * 64;      // loads a step: eight rows of 64 values each
@@ -483,8 +483,11 @@ int dn_linear_wide_form(const i64h_linear& d) {
     if ((d.a_rows && d.a_height <= 0) || span >= (int64_t)DN_BUF_END - 64 || ((dual ? (int64_t)d.N : 0) + 256) * 2 * d.K >= (int64_t)DN_BUF_END - 64) return -1;
     const int64_t cols = dual ? 2 * (int64_t)d.N : d.N;
     if ((d.M + 63) / 64 * d.batch * ((cols + 63) / 64) > 0x7fffffff) return -1;
-    // few tiles of 16 columns: one for every CU at most (its LDS holds three or four steps of all its waves)
-    if (thin_fits(d) && d.M <= 128 && d.K >= 256 && (d.M + 63) / 64 * ((d.N + 15) / 16) * d.batch <= 256) return DN_WIDE_FORMS;
+    // few tiles of 16 columns: one for every CU at most (its LDS holds three or four steps of all its waves), two where up to 32 rows walk a long k.  Microseconds, here | 64 x 64
+    // tiles | rows in 32 bits: 5120 x 4096, 3 rows 14.3 | 19.4 | 18.5, 32 rows 19.4 | 20.3 | 19.5, 48 rows 23.6 | 21.1 | 18.9; 8192 x 3072, 16 rows 15.0 | 16.8 | 20.1; 4352 x 2048, 16 rows 9.0 |
+    // 8.6 | 8.7
+    const int64_t thin_tiles = (d.M + 63) / 64 * ((d.N + 15) / 16) * d.batch;
+    if (thin_fits(d) && d.M <= 128 && d.K >= 256 && (thin_tiles <= 256 || (thin_tiles <= 512 && d.M <= 32 && d.K >= 3072))) return DN_WIDE_FORMS;
     static const dn_wide_form forms[DN_WIDE_FORMS] = {{256, 256, true, 1.3f, 1.3f, 12.0f}, {256, 128, true, 0.72f, 0.72f, 7.0f}, {192, 128, false, 1.0f, 1.7f, 0.0f},
                                                       {128, 128, false, 1.0f, 1.2f, 0.0f}, {64, 128, false, 0.5f, 0.75f, 0.0f}, {64, 64, false, 0.33f, 0.4f, 0.0f}};
     int form = 0;
