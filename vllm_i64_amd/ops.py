@@ -294,7 +294,8 @@ def gemm_desc(a: torch.Tensor, w: torch.Tensor, w_scale: torch.Tensor, out: torc
     d.N, d.K, d.C, d.epilogue = N, K, ptr(out), epilogue
     d.out_row_slot, d.out_slot_base, d.stats, d.want_stats = ptr(out_row_slot), out_slot_base, ptr(stats), int(want_stats)
     d.c_row_map, d.a_group_slots = ptr(c_row_map), a_group_slots
-    d.a_own_ranges = int(own_ranges)
+    if own_ranges:
+        d.a_own_ranges = 1
     d.c_residual = ptr(c_residual)   # decode-sized problems, plain epilogue: out = c_residual + product
     return d
 
