@@ -507,7 +507,9 @@ int dn_linear_wide_form(const i64h_linear& d) {
     // x 2048 (252 tiles), 12 tokens 34.4 | 35.6, 64 tokens 35.1 | 37.8; 2048 x 1792 (144), 40 tokens 18.3 | 20.8; 13 batches, pairs of 896 x 1024 (182), 64 tokens 14.2 | 16.3.  Less
     // than half: 8 batches, pairs of 896 x 1024 (112), 64 tokens 10.6 | 9.3.  More than once, or longer k, where the four steps that a 64 x 64 tile has on their way count: 12
     // batches, pairs of 1792 x 2048 (336), 12 tokens 44.0 | 41.8; 8 of 5504 x 2048 (688), 64 tokens 87.7 | 81.6; 15 of 1024 x 4096 (240), 27 tokens 63.4 | 58.7; but 64 of 2048 x 768
-    // (1024), 40 tokens 42.4 | 47.3.  (Taller tiles are never the fastest there: 59 to 107 us for these.)
+    // (1024), 40 tokens 42.4 | 47.3.  (Taller tiles are never the fastest there: 59 to 107 us for these.)  Where 64 x 64 tiles under a longer
+    // k are one to one and a half of a round, 64 x 128 ones are faster alone, 9 of 2048 x 5504 (144), 64 tokens 61.9 | 73.2, but not beside a second stream's scan (92 | 85): of steps with
+    // such experts one with the recurrent branch beside them took 747 | 718, one without 1024 | 1058.
     if (form >= 4 && d.group_off && d.rows_total > 0 && d.M <= 64) {
         const float others = (float)(d.batch - 1), live = others > 0.0f ? 1.0f + others * (1.0f - expf(-fmaxf(0.0f, (float)(d.rows_total - d.M)) / others)) : 1.0f;
         const float tiles = live * (float)((cols + 127) / 128);
