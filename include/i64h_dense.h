@@ -600,6 +600,41 @@ typedef struct {
 } i64h_gdn_args;
 int i64h_gdn_gates(const i64h_gdn_args* d, void* stream);
 int i64h_gdn_scan(const i64h_gdn_args* d, void* stream);
+
+/* ---- one step of a recurrence, from the projections to the normed and gated result ----------------------------------------------------------
+ * Every row t of P the only row of its sequence.  conv_w (delta rule; kv_heads = heads): the columns [q_off, + heads * (2 dim + vdim)) - q | k | v - pass the
+ * convolution of i64h_causal_conv (w conv_w fp32 [channels, taps], 2 .. 8 taps, silu; carried inputs conv fp32 [slots, taps - 1, channels]), q and k become unit vectors (unit_eps),
+ * q times q_scale, beta = sigmoid(P[t, b_off + a]), and i64h_gdn_scan's step follows.  conv_w = NULL: i64h_gla_scan's step on the columns q_off, k_off, v_off, its
+ * read-out times q_scale.  Decay per head and key channel: exp(-a_rate * softplus(A P[t, a_off : + a_rank] + a_bias)), A bf16 [heads * dim, a_rank], a_rate and a_bias fp32
+ * [heads * dim].  out[t, a * vdim : + vdim] = o / sqrt(mean(o^2) + eps) * norm_w * act(z), act = sigmoid (gate_act) or silu; z = Z P[t, z_off : + z_rank] (delta rule, Z bf16
+ * [heads * vdim, z_rank]) or the columns z_off of P.  The maps' input rows are rounded to bf16 unless exact.
+ * state as in i64h_gdn_scan; dim <= 128 (a multiple of four), vdim <= 128; out and out16 (bf16): either or both, row stride ldo.  All other arithmetic fp32. */
+typedef struct {
+    const float* P;
+    int64_t ldp;
+    int32_t q_off, k_off, v_off;
+    int32_t heads, dim, vdim;
+    const float* conv_w;
+    float* conv;
+    int32_t taps, b_off;
+    float unit_eps, q_scale;
+    const void* A;
+    const float* a_bias;
+    const float* a_rate;
+    int32_t a_off, a_rank;
+    const void* Z;
+    int32_t z_off, z_rank, gate_act, exact;
+    const float* norm_w;
+    float eps;
+    const int32_t* positions;
+    const int32_t* slot_ids;
+    float* state;
+    float* out;
+    void* out16;
+    int64_t ldo;
+    int64_t n;
+} i64h_rec_step_args;
+int i64h_rec_step(const i64h_rec_step_args* d, void* stream);
 int64_t i64h_scan_work_floats(int64_t n, int32_t nseg, int32_t heads, int32_t dim);
 /* Whether either scan (delta != 0: i64h_gdn_scan, else i64h_gla_scan with keys of its own) of nseg runs of n rows, the longest of `longest` rows, is the
  * faster in tiles, and a caller that knows its runs should give it a workspace.  The launch itself knows n and nseg only. */

@@ -1,0 +1,79 @@
+"""i64h_rec_step: a decode step's recurrence in one launch against the launches it stands for (convolution, gates, decays' Linear, scan, norm and gate)."""
+import pytest
+import torch
+
+from vllm_i64_amd import ops_dense as D
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+# heads, dim, vdim, ranks, taps, rows
+SIZES = [(8, 128, 128, (128, 128), 4, 7), (1, 4, 1, (8, 8), 2, 1), (3, 64, 64, (16, 136), 4, 33), (2, 68, 65, (264, 8), 8, 5), (5, 60, 128, (128, 40), 3, 2), (16, 128, 64, (128, 128), 4, 64)]
+
+
+def _close(got, want, what):
+    """Both sides round the same inputs; they differ in the order of 32-bit sums of at most a few hundred terms, through a decay, a step and a norm: 1e-5 of the largest value is
+    some eighty roundings of it."""
+    g, w = got.double(), want.double()
+    assert torch.isfinite(g).all(), what
+    assert (g - w).abs().max() <= 1e-5 * w.abs().max().clamp(min=1e-20), (what, ((g - w).abs().max() / w.abs().max()).item())
+
+
+@pytest.mark.parametrize("exact", [False, True])
+@pytest.mark.parametrize("delta", [True, False])
+@pytest.mark.parametrize("H,d,dv,ranks,taps,n", SIZES)
+def test_one_launch_is_the_six(H, d, dv, ranks, taps, n, delta, exact):
+    g = torch.Generator(device=DEV).manual_seed(H * d + dv + n)
+    r = lambda *s, std=1.0: torch.randn(*s, generator=g, device=DEV) * std
+    pad4 = lambda x: (x + 3) // 4 * 4
+    nd, rv, slots = H * d, H * dv, n + 3
+    C = 2 * nd + rv
+    a_off = pad4(C)
+    z_off = a_off + pad4(ranks[0])
+    b_off = z_off + max(pad4(ranks[1]), pad4(rv))
+    P = r(n, pad4(b_off + H))
+    ld = P.shape[-1]
+    a, bias, rate = r(nd, ranks[0], std=ranks[0] ** -0.5).bfloat16(), r(nd), torch.rand(nd, generator=g, device=DEV) + 0.1
+    z, norm_w, eps = r(rv, ranks[1], std=ranks[1] ** -0.5).bfloat16(), r(dv), 1e-6
+    conv_w, conv = r(C, taps, std=0.5), r(slots, taps - 1, C)
+    pos = torch.randint(1, 2000, (n,), generator=g, device=DEV, dtype=torch.int32)
+    pos[::3] = torch.arange(len(pos[::3]), device=DEV, dtype=torch.int32) % taps      # rows at a sequence's start: no state, fewer carried inputs
+    slot = torch.randperm(slots, generator=g, device=DEV)[:n].to(torch.int32)
+    state = r(slots, H, dv, d, std=0.3)
+    seg = torch.arange(n + 1, dtype=torch.int32, device=DEV)
+    s1, s2, c1, c2 = state.clone(), state.clone(), conv.clone(), conv.clone()
+
+    F, R, want, got, got16 = (torch.empty(n, w, device=DEV) for w in (nd, rv, rv, rv, rv))
+    got16 = got16.bfloat16()
+    D.linear(P, a, F, m=n, a_off=a_off, exact=exact, bias=bias, epilogue=D.EPI_DECAY, e=rate)
+    if delta:
+        X, G, Z = torch.empty(n, C, device=DEV), torch.empty(n, 2 * H, device=DEV), torch.empty(n, rv, device=DEV)
+        D.causal_conv(P, off=0, channels=C, w=conv_w, bias=None, positions=pos, slot_ids=slot, state=c1, out=X, n=n, single_rows=True)
+        cols = dict(q_off=0, k_off=nd, v_off=2 * nd, heads=H, kv_heads=H, dim=d, vdim=dv, n=n)
+        D.gdn_gates(X, G, P, b_off=b_off, a_off=-1, a_log=None, dt_bias=None, unit_eps=1e-6, q_scale=d ** -0.5, **cols)
+        D.linear(P, z, Z, m=n, a_off=z_off, exact=exact)
+        D.gdn_scan(X, G, f=F, seg_start=seg, nseg=n, positions=pos, slot_ids=slot, state=s1, out=R, **cols)
+        D.gate_norm(R, norm_w, want, groups=H, eps=eps, z=Z, ldz=rv, n=n, gate_after=True, width=rv, sigmoid=True)
+        kw = dict(q_off=0, conv_w=conv_w, conv=c2, b_off=b_off, unit_eps=1e-6, z=z, z_off=z_off, sigmoid=True)
+    else:
+        D.gla_scan(P, f=F, q_off=0, k_off=nd, f_off=0, v_off=2 * nd, heads=H, dim=d, vdim=dv, seg_start=seg, nseg=n, positions=pos, slot_ids=slot, state=s1, out=R, n=n, q_scale=d ** -0.5)
+        D.gate_norm(R, norm_w, want, groups=H, eps=eps, z=P, z_off=z_off, ldz=ld, n=n, gate_after=True, width=rv)
+        kw = dict(q_off=0, k_off=nd, v_off=2 * nd, z_off=z_off)
+    D.rec_step(P, heads=H, dim=d, vdim=dv, a=a, a_off=a_off, a_bias=bias, a_rate=rate, norm_w=norm_w, eps=eps, positions=pos, slot_ids=slot, state=s2, n=n, out=got, out16=got16,
+               q_scale=d ** -0.5, exact=exact, **kw)
+    _close(s2, s1, "state")
+    _close(got, want, "result")
+    assert torch.equal(got16, got.bfloat16())
+    assert torch.equal(c1, c2)
+    idle = torch.ones(slots, dtype=torch.bool, device=DEV)
+    idle[slot.long()] = False
+    assert torch.equal(s2[idle], state[idle])      # other sequences' states are left alone
+
+
+def test_what_does_not_fit_is_refused():
+    t = torch.zeros(4, 64, device=DEV)
+    i = torch.zeros(4, dtype=torch.int32, device=DEV)
+    kw = dict(a=torch.zeros(8, 8, device=DEV).bfloat16(), a_off=16, a_bias=t[0], a_rate=t[0], z_off=24, norm_w=t[0], eps=0.0, positions=i, slot_ids=i, n=1, out=t, heads=1)
+    with pytest.raises(Exception, match="rec_step"):      # the gate's columns lie outside the row
+        D.rec_step(t, q_off=0, k_off=8, v_off=8, dim=8, vdim=48, state=torch.zeros(1, 1, 48, 8, device=DEV), **kw)
+    with pytest.raises(Exception, match="rec_step"):      # key channels that are no four
+        D.rec_step(t, q_off=0, k_off=8, v_off=8, dim=6, vdim=4, state=torch.zeros(1, 1, 4, 6, device=DEV), **{**kw, "a": kw["a"][:6]})

@@ -237,6 +237,7 @@ DENSE_SIGNATURES: Dict[str, str] = {
     "i64h_rot_post": "pp",
     "i64h_gdn_gates": "pp",
     "i64h_gdn_scan": "pp",
+    "i64h_rec_step": "pp",
     "i64h_set_gdn_scan_form": "i",
     "i64h_set_residual_form": "i",
     "i64h_gla_gates": "pp",
@@ -363,6 +364,14 @@ class Gla(ctypes.Structure):
     _fields_ = [("P", _P), ("ldp", _L), ("q_off", _I), ("f_off", _I), ("k_off", _I), ("v_off", _I), ("heads", _I), ("dim", _I), ("vdim", _I),
                 ("lower", _P), ("q_act", _I), ("seg_start", _P), ("nseg", _I), ("positions", _P), ("slot_ids", _P), ("state", _P), ("out", _P),
                 ("ldo", _L), ("n", _L), ("F", _P), ("ldf", _L), ("q_scale", _F), ("work", _P), ("work_floats", _L)]
+
+
+class RecStep(ctypes.Structure):
+    """Mirror of i64h_rec_step_args (include/i64h_dense.h)."""
+    _fields_ = [("P", _P), ("ldp", _L), ("q_off", _I), ("k_off", _I), ("v_off", _I), ("heads", _I), ("dim", _I), ("vdim", _I), ("conv_w", _P), ("conv", _P),
+                ("taps", _I), ("b_off", _I), ("unit_eps", _F), ("q_scale", _F), ("A", _P), ("a_bias", _P), ("a_rate", _P), ("a_off", _I), ("a_rank", _I), ("Z", _P),
+                ("z_off", _I), ("z_rank", _I), ("gate_act", _I), ("exact", _I), ("norm_w", _P), ("eps", _F), ("positions", _P), ("slot_ids", _P), ("state", _P), ("out", _P),
+                ("out16", _P), ("ldo", _L), ("n", _L)]
 
 
 class Route(ctypes.Structure):

@@ -11,6 +11,7 @@
 // A row continues the row before it iff slot and position say so; state is taken as empty at position 0.  All arithmetic fp32.
 #include "i64h_common.h"
 #include "i64h_dense.h"
+#include "i64h_scan_dev.h"
 
 int i64h_scan_tiles(const i64h_gdn_args& d, bool delta, void* stream);      // i64h_scan_tile.hip
 
@@ -98,47 +99,7 @@ __global__ __launch_bounds__(256) void gdn_gates_kernel(const i64h_gdn_args p) {
 // a prompt is cut); loads run TG tokens ahead in two alternating register sets.  State layout [slot, head, value column, key channel].
 // CHD: a decay per head and key channel (F) in the place of one per head.  RULE: the delta rule's correction and write strength, or gated
 // linear attention: the token writes k v^T as it is, the read-out is multiplied by q_scale; the keys are the row's own or one minus the decay.
-enum { GD_DELTA = 0, GD_KEYS = 1, GD_FORGET = 2 };
 // TG is chosen so that two waves fit a SIMD's registers (the loads in flight are most of them); one where every run is a single row.
-// A lane's KPT channels: four neighbours in every stripe of 64 (so that 16 lanes read 256 consecutive bytes at a time).
-template <int KPT>
-__device__ __forceinline__ int gd_channel(int nlane, int k) {
-    return KPT >= 4 ? 4 * (nlane + 16 * (k >> 2)) + (k & 3) : nlane * KPT + k;
-}
-// A token's part in a column's state and what it reads, shared by both kernels: a lane's sums run in two chains (even and odd channels), whose
-// instructions follow each other without waiting.
-template <int KPT, bool CHD>
-__device__ __forceinline__ float gd_delta(float (&S)[KPT], const float* f, const float* k, const float* q, float v, float beta) {
-    float s0 = 0.0f, s1 = 0.0f;
-#pragma unroll
-    for (int i = 0; i < KPT; ++i) {
-        S[i] *= f[CHD ? i : 0];
-        if (i & 1) s1 = fmaf(S[i], k[i], s1);
-        else s0 = fmaf(S[i], k[i], s0);
-    }
-    const float d = beta * (v - group_sum(s0 + s1, 16));
-    float o0 = 0.0f, o1 = 0.0f;
-#pragma unroll
-    for (int i = 0; i < KPT; ++i) {
-        S[i] = fmaf(k[i], d, S[i]);
-        if (i & 1) o1 = fmaf(S[i], q[i], o1);
-        else o0 = fmaf(S[i], q[i], o0);
-    }
-    return group_sum(o0 + o1, 16);
-}
-template <int KPT, bool CHD, bool FORGET>
-__device__ __forceinline__ float gd_linear(float (&S)[KPT], const float* f, const float* k, const float* q, float v) {
-    float o0 = 0.0f, o1 = 0.0f;
-#pragma unroll
-    for (int i = 0; i < KPT; ++i) {
-        const float fi = f[CHD ? i : 0];
-        S[i] = fmaf(fi, S[i], (FORGET ? 1.0f - fi : k[FORGET ? 0 : i]) * v);
-        if (i & 1) o1 = fmaf(S[i], q[i], o1);
-        else o0 = fmaf(S[i], q[i], o0);
-    }
-    return group_sum(o0 + o1, 16);
-}
-
 template <int KPT, int CPT, bool CHD, int TG, int RULE>
 __global__ __launch_bounds__(256) void gdn_scan_kernel(const i64h_gdn_args p, const int ctiles, const int vec) {
     const int N = p.dim, P = p.vdim;

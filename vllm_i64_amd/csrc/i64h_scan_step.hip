@@ -1,0 +1,200 @@
+// A decode step of the recurrences (include/i64h_dense.h, i64h_rec_step): everything between a layer's projections and its out-projection that belongs to one head
+// of one row - convolution and unit vectors (delta rule), the low-rank decays and output gates, the recurrence's one step, the head's norm and gate -
+// in one workgroup, so that a layer waits for one launch in the place of six (linear attention: three).
+// What bounds it: few rows the chain inside a workgroup (loads of the sequence's slot, of the state behind it, sums, norm), many rows the state's way from memory and
+// back; the low-rank maps' 64 KB a head come from L2.  7 rows of 8 heads of 128 in a graph: six launches of the delta rule 23 us, this one 9, a step of eight such layers 510 -> 404; 64 rows
+// of 16 heads, linear attention beside an attention over 134 MB: 16 + 45 + 6 -> 42 (134 MB of state at the copy rate: 28), a step 1524 -> 1508.
+#include "i64h_dense_dev.h"
+#include "i64h_scan_dev.h"
+
+// 512 threads: the 16 lanes of a DPP row share CPT value columns and hold KPT key channels of each in registers; a workgroup has 32 such rows.
+// DELTA: the delta rule behind a convolution; else linear attention with keys of its own, its gates columns of P.
+template <int KPT, int CPT, bool DELTA>
+__global__ __launch_bounds__(512) void rec_step_kernel(const i64h_rec_step_args p) {
+    constexpr int NP = 16 * KPT, RPT = NP / 32;      // RPT: rows of the decays' map a DPP row takes
+    __shared__ __attribute__((aligned(16))) float sX[DELTA ? 2 * NP + 32 * CPT : 4], sF[NP], sS[32];
+    const int tid = threadIdx.x, l = tid & 15, g = tid >> 4;
+    const int N = p.dim, V = p.vdim, a = blockIdx.x % p.heads;
+    const int64_t t = blockIdx.x / p.heads;
+    const float* row = p.P + t * p.ldp;
+    const int64_t slot = p.slot_ids[t];
+    const int pos = p.positions[t];
+    // the maps' input rows, rounded as the Linears round them, and the products: 16 lanes a row of the map, eight values a lane and stripe of 128
+    auto map = [&](const void* M, int off, int rank, int first, int count, int top, auto& sum) {
+        constexpr int R = sizeof(sum) / sizeof(float);
+#pragma unroll
+        for (int r = 0; r < R; ++r) sum[r] = 0.0f;
+        for (int k = 8 * l; k < rank; k += 128) {
+            dn_v4u w[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) w[r] = first + r < top ? *(const dn_v4u*)((const uint16_t*)M + ((int64_t)a * top + first + r) * rank + k) : (dn_v4u)0u;
+            float x[8];
+            *(dn_v4f*)x = *(const dn_v4f*)(row + off + k), *(dn_v4f*)(x + 4) = *(const dn_v4f*)(row + off + k + 4);
+            if (!p.exact) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) x[i] = dn_bf16_to_f32(dn_bf16_rne(x[i]));
+            }
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    s0 = fmaf(x[2 * i], __uint_as_float(w[r][i] << 16), s0);
+                    s1 = fmaf(x[2 * i + 1], __uint_as_float(w[r][i] & 0xffff0000u), s1);
+                }
+                sum[r] += s0 + s1;
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) sum[r] = group_sum(sum[r], 16);
+    };
+    // ---- what does not wait for the sequence's slot: decays and gates ----
+    float zs[CPT], fs[RPT];
+    map(p.A, p.a_off, p.a_rank, RPT * g, RPT, N, fs);
+    if (DELTA) map(p.Z, p.z_off, p.z_rank, CPT * g, CPT, V, zs);
+    // ---- the state, on its way from here on ----
+    float S[CPT][KPT];
+    float* gS = p.state + ((slot * p.heads + a) * V + CPT * g) * N;
+#pragma unroll
+    for (int j = 0; j < CPT; ++j)
+#pragma unroll
+        for (int k = 0; k < KPT; k += 4) {
+            const int c = gd_channel<KPT>(l, k);
+            dn_v4f v = {0, 0, 0, 0};
+            if (pos != 0 && CPT * g + j < V && c < N) v = *(const dn_v4f*)(gS + j * N + c);
+            *(dn_v4f*)&S[j][k] = v;
+        }
+    if (l < RPT) {
+        const int c = RPT * g + l;
+        float f = fs[0];
+#pragma unroll
+        for (int r = 1; r < RPT; ++r) f = l == r ? fs[r] : f;
+        sF[c] = c < N ? expf(-p.a_rate[a * N + c] * dn_softplus(f + p.a_bias[a * N + c])) : 1.0f;
+    }
+    float q[KPT], k[KPT], f[KPT], v[CPT], beta = 0.0f;
+    if constexpr (DELTA) {      // a thread per channel of q | k | v: its convolution, and the carried inputs one position on
+        const int part = tid < NP ? 0 : (tid < 2 * NP ? 1 : 2), c = tid - part * NP;
+        if (tid < 2 * NP + 32 * CPT) {
+            float o = 0.0f;
+            if (c < (part < 2 ? N : V)) {
+                const int H = p.heads, ch = part < 2 ? (part * H + a) * N + c : 2 * H * N + a * V + c, C = H * (2 * N + V), T = p.taps;
+                const float* w = p.conv_w + (int64_t)ch * T;
+                float* st = p.conv + slot * (T - 1) * C + ch;
+                const float x = row[p.q_off + ch];
+                float in[7];
+#pragma unroll
+                for (int d = 1; d < 8; ++d) in[d - 1] = d < T && pos >= d ? st[(int64_t)(T - 1 - d) * C] : 0.0f;
+                for (int d = T - 1; d > 0; --d) {
+                    float y = in[0];
+#pragma unroll
+                    for (int i = 1; i < 7; ++i) y = d == i + 1 ? in[i] : y;
+                    o += w[T - 1 - d] * y;
+                }
+                o += w[T - 1] * x;
+                o = o / (1.0f + expf(-o));
+#pragma unroll
+                for (int d = 1; d < 7; ++d)
+                    if (d < T - 1) st[(int64_t)(T - 2 - d) * C] = in[d - 1];
+                st[(int64_t)(T - 2) * C] = x;
+            }
+            sX[tid] = o;
+        }
+        beta = dn_sigmoid(row[p.b_off + a]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < KPT; i += 4) {
+            const int c = gd_channel<KPT>(l, i);
+            dn_v4f x = {0, 0, 0, 0}, y = x;
+            if (c < N) x = *(const dn_v4f*)(row + p.q_off + a * N + c), y = *(const dn_v4f*)(row + p.k_off + a * N + c);
+            *(dn_v4f*)&q[i] = x, *(dn_v4f*)&k[i] = y;
+        }
+#pragma unroll
+        for (int j = 0; j < CPT; ++j) {
+            const int c = CPT * g + j;
+            v[j] = c < V ? row[p.v_off + a * V + c] : 0.0f, zs[j] = c < V ? row[p.z_off + a * V + c] : 0.0f;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < KPT; i += 4) {
+        const int c = gd_channel<KPT>(l, i);
+        *(dn_v4f*)&f[i] = *(const dn_v4f*)&sF[c];
+        if constexpr (DELTA) *(dn_v4f*)&q[i] = *(const dn_v4f*)&sX[c], *(dn_v4f*)&k[i] = *(const dn_v4f*)&sX[NP + c];
+    }
+    if constexpr (DELTA) {
+#pragma unroll
+        for (int j = 0; j < CPT; ++j) v[j] = sX[2 * NP + CPT * g + j];
+        auto unit = [&](float (&x)[KPT], float scale) {
+            float s = 0.0f;
+#pragma unroll
+            for (int i = 0; i < KPT; i += 4) s += (x[i] * x[i] + x[i + 1] * x[i + 1]) + (x[i + 2] * x[i + 2] + x[i + 3] * x[i + 3]);
+            const float u = 1.0f / sqrtf(group_sum(s, 16) + p.unit_eps) * scale;
+#pragma unroll
+            for (int i = 0; i < KPT; ++i) x[i] *= u;
+        };
+        unit(q, p.q_scale);
+        unit(k, 1.0f);
+    }
+    float o[CPT], ss = 0.0f;
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) {
+        if constexpr (DELTA) o[j] = gd_delta<KPT, true>(S[j], f, k, q, v[j], beta);
+        else o[j] = gd_linear<KPT, true, false>(S[j], f, k, q, v[j]) * p.q_scale;
+        ss += CPT * g + j < V ? o[j] * o[j] : 0.0f;
+    }
+    if (l == 0) sS[g] = ss;
+#pragma unroll
+    for (int j = 0; j < CPT; ++j)
+#pragma unroll
+        for (int i = 0; i < KPT; i += 4) {
+            const int c = gd_channel<KPT>(l, i);
+            if (CPT * g + j < V && c < N) *(dn_v4f*)(gS + j * N + c) = *(const dn_v4f*)&S[j][i];
+        }
+    __syncthreads();
+    float all = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 32; i += 4) {
+        const dn_v4f s = *(const dn_v4f*)&sS[i];
+        all += (s[0] + s[1]) + (s[2] + s[3]);
+    }
+    const int c = CPT * g + l;
+    if (l >= CPT || c >= V) return;
+    float y = o[0], z = zs[0];
+#pragma unroll
+    for (int j = 1; j < CPT; ++j) y = l == j ? o[j] : y, z = l == j ? zs[j] : z;
+    y = y / sqrtf(all / (float)V + p.eps) * p.norm_w[c] * (p.gate_act ? dn_sigmoid(z) : z / (1.0f + expf(-z)));
+    if (p.out) p.out[t * p.ldo + a * V + c] = y;
+    if (p.out16) ((uint16_t*)p.out16)[t * p.ldo + a * V + c] = (uint16_t)dn_bf16_rne(y);
+}
+
+extern "C" {
+
+int i64h_rec_step(const i64h_rec_step_args* dp, void* stream) {
+    I64H_CHECK_ARG(dp != nullptr, "rec_step: no descriptor");
+    const i64h_rec_step_args& d = *dp;
+    const bool delta = d.conv_w != nullptr;
+    I64H_CHECK_ARG(d.heads > 0 && d.dim > 0 && d.dim <= 128 && d.dim % 4 == 0 && d.vdim > 0 && d.vdim <= 128 && d.n >= 0,
+                   "rec_step: heads %d, dim %d, vdim %d (dims to 128, key channels in fours)", d.heads, d.dim, d.vdim);
+    I64H_CHECK_ARG(d.P && d.positions && d.slot_ids && d.state && d.A && d.a_bias && d.a_rate && d.norm_w && (d.out || d.out16), "rec_step: null operand");
+    I64H_CHECK_ARG(d.q_off >= 0 && d.a_off >= 0 && d.z_off >= 0 && (delta ? d.b_off >= 0 : d.k_off >= 0 && d.v_off >= 0), "rec_step: negative column");
+    I64H_CHECK_ARG(!delta || (d.conv && d.Z && d.taps >= 2 && d.taps <= 8 && d.z_rank > 0), "rec_step: the delta rule takes a convolution of 2 to 8 taps (%d) and a low-rank gate", d.taps);
+    I64H_CHECK_ARG(d.a_rank > 0 && d.a_rank % 8 == 0 && (!delta || d.z_rank % 8 == 0), "rec_step: ranks %d and %d, multiples of eight", d.a_rank, d.z_rank);
+    I64H_CHECK_ARG((((uintptr_t)d.P | (uintptr_t)d.A | (uintptr_t)d.Z | (uintptr_t)d.state) & 15) == 0 && d.ldp % 4 == 0 && d.a_off % 4 == 0 &&
+                   (delta ? d.z_off % 4 == 0 : d.q_off % 4 == 0 && d.k_off % 4 == 0), "rec_step: rows and states are read 16 bytes at a time");
+    I64H_CHECK_ARG(d.n * d.heads < (1ll << 31), "rec_step: %lld rows of %d heads", (long long)d.n, d.heads);
+    if (d.n == 0) return 0;
+    auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, dim3((unsigned)(d.n * d.heads)), dim3(512), 0, (hipStream_t)stream, d); };
+#define REC_PICK(K, C)                                  \
+    if (delta) launch(rec_step_kernel<K, C, true>);     \
+    else launch(rec_step_kernel<K, C, false>);
+    if (d.dim <= 64) {
+        if (d.vdim <= 64) { REC_PICK(4, 2) } else { REC_PICK(4, 4) }
+    } else {
+        if (d.vdim <= 64) { REC_PICK(8, 2) } else { REC_PICK(8, 4) }
+    }
+#undef REC_PICK
+    I64H_CHECK_LAUNCH();
+    return 0;
+}
+
+}  // extern "C"

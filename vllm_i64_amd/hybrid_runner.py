@@ -321,16 +321,30 @@ class HybridRunner:
             D.linear(olat, d["uv"], og, **maps)
             D.linear(og, d["o"], out, m=n, k=H * m.vdim, lda=H * m.vdim, exact=ex)
 
+    # ---- a recurrence's step where every row is a sequence of its own: one launch from the projections to the normed and gated rows ----
+    # (The separate launches | one, us in graphs, delta rule and linear attention: 8 heads of 128, 1 row 18.5 | 7.0 and 10.2 | 5.1, 64 rows 34.6 | 14.7 and 23.1 | 11.3, 256 74 | 52 and 57 | 44,
+    # 1024 271 | 250 and 220 | 201; 32 heads of 64, 64 rows 40 | 22 and 24 | 15, 1024 327 | 319 and 224 | 214; 2 heads of 32, 1 row 17 | 5.3 and 10 | 3.9, 1024 26 | 17 and 15 | 11: always the one.)
+    @staticmethod
+    def _steps_at_once(r) -> bool:
+        return r.dim <= D.REC_STEP_DIM and r.vdim <= D.REC_STEP_DIM and r.dim % 4 == 0
+
     # ---- gated linear attention ----
     def _gated_linear(self, B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, out, scale: float = 1.0, work=NO_WORK) -> None:
         """Gated linear attention on the projection rows P (columns d["rq_off"], d["rk_off"], d["rv_off"], d["rg_off"]: queries, keys, values, output
         gates; d["a1_off"]: the low-rank decay map's first factor).  sigmoid(z)^(1 / tau) = exp(-softplus(-z) / tau): the second factor and
         its bias are held negated, the exponent's rate is d["a_rate"]."""
         rv = r.heads * r.vdim
+        wide = self._rounded(n, rv)
+        Rn, Rn16 = None if wide else B.rn[: n * rv].view(n, rv), self._as16(B.rn16, n, rv) if wide else None
+        if nseg == n and self._steps_at_once(r):
+            D.rec_step(P, q_off=d["rq_off"], k_off=d["rk_off"], v_off=d["rv_off"], heads=r.heads, dim=r.dim, vdim=r.vdim, a=d["a2"], a_off=d["a1_off"], a_bias=d["a2_b"],
+                       a_rate=d["a_rate"], z_off=d["rg_off"], norm_w=d["r_norm"], eps=self.cfg.norm_eps, positions=positions, slot_ids=slot_ids, state=kvc.state[l]["gla"], n=n,
+                       out=Rn, out16=Rn16, q_scale=r.dim ** -0.5, exact=self.exact)
+            self._out(Rn, d["o_right"], out, scale, Rn16)
+            return
         F = B.f[: n * r.heads * r.dim].view(n, r.heads * r.dim)
         D.linear(P, d["a2"], F, m=n, a_off=d["a1_off"], exact=self.exact, bias=d["a2_b"], epilogue=D.EPI_DECAY, e=d["a_rate"])
-        wide = self._rounded(n, rv)
-        R, Rn, Rn16 = B.r[: n * rv].view(n, rv), None if wide else B.rn[: n * rv].view(n, rv), self._as16(B.rn16, n, rv) if wide else None
+        R = B.r[: n * rv].view(n, rv)
         D.gla_scan(P, f=F, q_off=d["rq_off"], k_off=d["rk_off"], f_off=0, v_off=d["rv_off"], heads=r.heads, dim=r.dim, vdim=r.vdim, seg_start=seg, nseg=nseg,
                    positions=positions, slot_ids=slot_ids, state=kvc.state[l]["gla"], out=R, n=n, q_scale=r.dim ** -0.5,
                    work=work.get((r.heads, r.dim, r.vdim)))
@@ -345,12 +359,20 @@ class HybridRunner:
         ex = self.exact
         st = kvc.state[l]
         C, rk, rv = r.conv_channels, r.kv_heads * r.dim, r.heads * r.vdim
+        channel = r.decay == "channel"
+        wide = self._rounded(n, rv)
+        Rn, Rn16 = None if wide else B.c[: n * rv].view(n, rv), self._as16(B.c16, n, rv) if wide else None
+        if nseg == n and channel and r.kv_heads == r.heads and "conv" in st and st["conv"].shape[-2] < D.REC_STEP_TAPS and self._steps_at_once(r):
+            D.rec_step(P, q_off=d["r_off"], heads=r.heads, dim=r.dim, vdim=r.vdim, a=d["a2"], a_off=d["a1_off"], a_bias=d["dt_bias"], a_rate=d["a_rate"], z=d["g2"], z_off=d["g1_off"],
+                       norm_w=d["r_norm"], eps=self.cfg.norm_eps, positions=positions, slot_ids=slot_ids, state=st["gdn"], n=n, out=Rn, out16=Rn16, conv_w=d["conv_w"],
+                       conv=st["conv"], b_off=d["rb_off"], unit_eps=UNIT_EPS, q_scale=r.dim ** -0.5, sigmoid=r.gate == "sigmoid", exact=ex)
+            D.linear(Rn, d["o_right"], out, a16=Rn16, exact=ex)
+            return
         X = B.a[: n * C].view(n, C)
         D.causal_conv(P, off=d["r_off"], channels=C, w=d["conv_w"], bias=None, positions=positions, slot_ids=slot_ids, state=st.get("conv"), out=X, n=n,
                       single_rows=single, seg_start=seg, nseg=nseg)
         G = B.g[: n * 2 * r.heads].view(n, 2 * r.heads)
         cols = dict(q_off=0, k_off=rk, v_off=2 * rk, heads=r.heads, kv_heads=r.kv_heads, dim=r.dim, vdim=r.vdim, n=n)
-        channel = r.decay == "channel"
         D.gdn_gates(X, G, P, b_off=d["rb_off"], a_off=-1 if channel else d["ra_off"], a_log=None if channel else d["A_log"],
                     dt_bias=None if channel else d["dt_bias"], unit_eps=UNIT_EPS, q_scale=r.dim ** -0.5, **cols)
         F, Z, z_off, ldz = None, P, d.get("rg_off", 0), P.shape[-1]
@@ -361,8 +383,6 @@ class HybridRunner:
         R = B.b[: n * rv].view(n, rv)
         D.gdn_scan(X, G, f=F, seg_start=seg, nseg=nseg, positions=positions, slot_ids=slot_ids, state=st["gdn"], out=R,
                    work=work.get((r.heads, r.dim, r.vdim)), **cols)
-        wide = self._rounded(n, rv)
-        Rn, Rn16 = None if wide else B.c[: n * rv].view(n, rv), self._as16(B.c16, n, rv) if wide else None
         D.gate_norm(R, d["r_norm"], Rn, groups=r.heads, eps=self.cfg.norm_eps, z=Z, z_off=z_off, ldz=ldz, n=n, gate_after=True, width=rv, sigmoid=r.gate == "sigmoid", out16=Rn16)
         D.linear(Rn, d["o_right"], out, a16=Rn16, exact=ex)
 
