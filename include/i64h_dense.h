@@ -694,6 +694,10 @@ typedef struct {
     int32_t shared;
 } i64h_moe_plan_args;
 int i64h_moe_plan(const i64h_moe_plan_args* d, void* stream);
+/* i64h_streams_step with i64h_route_topk on the rows of h behind it (r: W, K = the rows' width, at most 17 rows of W, no groups; r->h is not read, and d may leave h and h16 away), and
+ * for n <= 128 i64h_moe_plan on that choice (m may be NULL), all in one launch.  sync int32 [32 * 17] (with m): zeros before the first launch, zeros again behind every one; launches that share it
+ * follow each other. */
+int i64h_streams_route(const i64h_streams_args* d, const i64h_route_args* r, const i64h_moe_plan_args* m, int32_t* sync, void* stream);
 typedef struct {
     const float* Y;
     const int32_t* pair_row;

@@ -226,6 +226,7 @@ DENSE_SIGNATURES: Dict[str, str] = {
     "i64h_sample_rows": "pplippppp",
     "i64h_embed_bigram": "pp",
     "i64h_streams_step": "pp",
+    "i64h_streams_route": "ppppp",
     "i64h_causal_conv": "pp",
     "i64h_ssm_scan": "pp",
     "i64h_gate_norm": "pp",

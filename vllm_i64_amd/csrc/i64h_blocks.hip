@@ -11,6 +11,7 @@
 // A row continues the row before it iff slot and position say so; state is taken as empty at position 0.  All arithmetic fp32.
 #include "i64h_common.h"
 #include "i64h_dense.h"
+#include "i64h_route_dev.h"
 #include "i64h_scan_dev.h"
 
 int i64h_scan_tiles(const i64h_gdn_args& d, bool delta, void* stream);      // i64h_scan_tile.hip
@@ -378,7 +379,6 @@ __device__ __forceinline__ int bl_wave_argmax(float v, int idx, float& best) {
     return -wave_max_i(-cand);
 }
 
-#define RT_MAX_TOP 32
 // SPLIT: a workgroup per row - four waves share the columns of the router's products, four such groups (or one) the entries, eight at a time, the first
 // wave goes on with their sums (few rows: one wave's chain of loads is what a launch would wait for).
 // One group | four, rows of 2048: 16 entries 64 rows 10.4 | 8.0 us, 256 rows 10.5 | 8.3, 512 rows 10.9 | 12.0; 64 entries 28.4 | 13.8, 28.6 | 14.5,
@@ -449,16 +449,16 @@ __global__ __launch_bounds__(SPLIT ? 1024 : 256) void route_topk_kernel(const i6
                         if (j < 8 ? e0 + j < rows : nine) acc[j] = fmaf(x, __uint_as_float((uint32_t)W[(int64_t)(e0 + j) * K + k] << 16), acc[j]);
                 }
             }
-#pragma unroll
-            for (int j = 0; j < (NINE ? 9 : 8); ++j) {
-                if (NINE && j == 8 && !nine) break;
-                const float v = wave_sum(acc[j]);
-                if (SPLIT) {
-                    if (lane == 0 && e0 + j < rows) part[(wid & 3) * rows + e0 + j] = v;
-                    continue;
-                }
-                if (lane == 0 && e0 + j < E) ch[e0 + j] = p.bias ? v + p.bias[e0 + j] : v;
-                if (lane == 0 && e0 + j == E && p.gate_out) p.gate_out[t] = bl_sigmoid(v);
+            auto keep = [&](int e, float v) {
+                if (SPLIT) part[(wid & 3) * rows + e] = v;
+                else if (e < E) ch[e] = p.bias ? v + p.bias[e] : v;
+                else if (p.gate_out) p.gate_out[t] = bl_sigmoid(v);
+            };
+            const float v8 = rt_sum8(acc);
+            if ((lane & 7) == 0 && e0 + (lane >> 3) < rows) keep(e0 + (lane >> 3), v8);
+            if (NINE && nine) {
+                const float v9 = wave_sum(acc[8]);
+                if (lane == 0) keep(e0 + 8, v9);
             }
         }
         if (SPLIT) {
@@ -473,6 +473,10 @@ __global__ __launch_bounds__(SPLIT ? 1024 : 256) void route_topk_kernel(const i6
     } else {
         const float* z = p.logits + t * p.ld;
         for (int e = lane; e < E; e += 64) ch[e] = p.bias ? z[e] + p.bias[e] : z[e];
+    }
+    if (E <= 64 && G == 1) {
+        rt_choose_few<false>(p, t, lane, lane < E ? ch[lane] : 0.0f);
+        return;
     }
     if (p.sigmoid_scores) {     // scores of their own, in the logits' order: the choice falls on the logits unless it is corrected
         for (int e = lane; e < E; e += 64) {
@@ -542,61 +546,13 @@ __global__ __launch_bounds__(SPLIT ? 1024 : 256) void route_topk_kernel(const i6
         if (lane == k) mine_w = s, mine_i = pick;
         if (lane == 0) ch[pick] = __builtin_nanf("");     // taken: out of every later comparison
     }
-    if (p.chosen_softmax) {     // ... and the weights are the softmax over the chosen ones
-        const float top1 = wave_max(lane < p.top ? mine_w : -INFINITY);
-        mine_w = lane < p.top ? expf(mine_w - top1) : 0.0f;
-        wsum = wave_sum(mine_w);
-    }
-    if (lane < p.top) {
-        p.idx[t * p.top + lane] = mine_i;
-        p.wgt[t * p.top + lane] = (p.raw_weights ? mine_w : mine_w / (wsum + 1e-20f)) * p.scale;
-    }
+    rt_store<false>(p, t, lane, mine_w, mine_i, wsum);
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(1024) void moe_plan_kernel(const i64h_moe_plan_args p) {
-    extern __shared__ int pl_lds[];   // [experts + 1] counts, then offsets; [experts] cursors
-    int* cnt = pl_lds;
-    int* cur = pl_lds + p.experts + 1;
-    const int tid = threadIdx.x, E = p.experts;
-    const int64_t pairs = p.n * p.top, base = p.shared ? p.n : 0;
-    if (p.shared) {
-        if (tid == 0) p.group_off[0] = 0;
-        for (int64_t t = tid; t < p.n; t += 1024) {
-            p.pair_token[t] = (int)t;
-            if (p.pair_wgt) p.pair_wgt[t] = 1.0f;
-        }
-    }
-    int32_t* group_off = p.group_off + (p.shared ? 1 : 0);
-    for (int e = tid; e <= E; e += 1024) cnt[e] = 0;
-    __syncthreads();
-    for (int64_t i = tid; i < pairs; i += 1024) {
-        const int e = p.idx[i];
-        if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);
-    }
-    __syncthreads();
-    if (tid == 0) {
-        int run = (int)base;
-        for (int e = 0; e < E; ++e) {
-            const int c = cnt[e];
-            cnt[e] = run;
-            cur[e] = run;
-            run += c;
-        }
-        cnt[E] = run;
-    }
-    __syncthreads();
-    for (int e = tid; e <= E; e += 1024) group_off[e] = cnt[e];
-    for (int64_t i = tid; i < pairs; i += 1024) {
-        const int e = p.idx[i];
-        int r = -1;
-        if (e >= 0 && e < E) {
-            r = atomicAdd(&cur[e], 1);
-            p.pair_token[r] = (int)((uint32_t)i / (uint32_t)p.top);
-            if (p.pair_wgt) p.pair_wgt[r] = p.wgt[i];
-        }
-        p.pair_row[i] = r;
-    }
+    extern __shared__ int pl_lds[];
+    rt_plan<1024>(p, pl_lds, [&](int64_t i) { return p.idx[i]; }, [&](int64_t i) { return p.wgt[i]; });
 }
 
 // A thread's loads of four choices are on their way together (as one after the other, each behind its row's number: 7.9 us for 64 rows of

@@ -18,6 +18,7 @@
 //                           and values turned by their own position; rot_post_kernel turns a head's sum back and applies a gate per head
 // A row continues the row before it iff slot and position say so; state is taken as empty at position 0.  All arithmetic fp32.
 #include "i64h_dense_dev.h"
+#include "i64h_route_dev.h"
 
 // i64h_latent.hip
 bool latent_decode_form();
@@ -192,9 +193,9 @@ __global__ __launch_bounds__(256) void streams_kernel(const i64h_streams_args p)
 // The ordinary residual sum (one stream, results without norms of their own) with rows of whole 16-byte slices: the row stays in registers
 // between the write and the norm, NV slices of four columns per thread.  MIX: with a mixture's weighted sum; instances of their own, for its
 // registers and branches cost the launches without one (4096 rows of 2048: 26.2 us, 27.6 with them).
-template <int NV, bool MIX>
-__global__ __launch_bounds__(256) void residual_kernel(const i64h_streams_args p) {
-    __shared__ float red[4];
+// The norm's weights are asked for in front of the sums.  read(v): what a caller does with the normed row.
+template <int NV, bool MIX, typename Read>
+__device__ __forceinline__ void residual_row(const i64h_streams_args& p, float* red, Read read) {
     const int tid = threadIdx.x, W = p.W;
     const int64_t m = blockIdx.x;
     float* xs = p.streams + (p.rows ? (int64_t)p.rows[m] : m) * W;
@@ -251,7 +252,15 @@ __global__ __launch_bounds__(256) void residual_kernel(const i64h_streams_args p
 #pragma unroll
         for (int k = 0; k < 4; ++k) ss += v[i][k] * v[i][k], su += v[i][k];
     }
-    if (!p.h && !p.h16) return;
+    if (!p.norm_w) return;
+    float4 nw[NV], nb[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int c = (i * 256 + tid) * 4;
+        nw[i] = nb[i] = make_float4(0, 0, 0, 0);
+        if (c < W) nw[i] = *(const float4*)(p.norm_w + c);
+        if (c < W && p.norm_b) nb[i] = *(const float4*)(p.norm_b + c);
+    }
     float mean = 0.0f;
     if (p.h_center) {
         mean = hy_block_sum(su, red) / (float)W;
@@ -269,15 +278,124 @@ __global__ __launch_bounds__(256) void residual_kernel(const i64h_streams_args p
     for (int i = 0; i < NV; ++i) {
         const int c = (i * 256 + tid) * 4;
         if (c >= W) continue;
-        const float4 w = *(const float4*)(p.norm_w + c);
-        float4 o = make_float4((v[i][0] - mean) / den * w.x, (v[i][1] - mean) / den * w.y, (v[i][2] - mean) / den * w.z, (v[i][3] - mean) / den * w.w);
-        if (p.norm_b) {
-            const float4 b = *(const float4*)(p.norm_b + c);
-            o.x += b.x, o.y += b.y, o.z += b.z, o.w += b.w;
-        }
+        float4 o = make_float4((v[i][0] - mean) / den * nw[i].x, (v[i][1] - mean) / den * nw[i].y, (v[i][2] - mean) / den * nw[i].z, (v[i][3] - mean) / den * nw[i].w);
+        if (p.norm_b) o.x += nb[i].x, o.y += nb[i].y, o.z += nb[i].z, o.w += nb[i].w;
         if (p.h) *(float4*)(p.h + m * W + c) = o;
         if (p.h16) *(uint2*)((uint16_t*)p.h16 + m * W + c) = make_uint2(dn_bf16_pair(o.x, o.y), dn_bf16_pair(o.z, o.w));
+        v[i][0] = o.x, v[i][1] = o.y, v[i][2] = o.z, v[i][3] = o.w;
     }
+    read(v);
+}
+
+template <int NV, bool MIX>
+__global__ __launch_bounds__(256) void residual_kernel(const i64h_streams_args p) {
+    __shared__ float red[4];
+    residual_row<NV, MIX>(p, red, [](const float (&)[NV][4]) {});
+}
+
+// The same with the choice of the row's experts behind the norm, the row still in registers, and of few rows the whole step's plan by the workgroup that ends last: the sums
+// in the order of route_topk_kernel's rows of their own, so the same bits.  The router's rows are asked for in front of the norm's sums (RT_AHEAD_NV; wider rows ask for them eight at a time).
+// What it saves is a launch's wait and the rows' way through memory; norm, choice and plan as launches of their own | together, us in graphs, two of 8 experts and a gate, width 1024:
+// 7 rows 10.2 | 6.4, 64 rows 10.4 | 7.1, 512 12.7 | 8.5, 4096 32 | 25, 16384 98 | 75; 8 experts, width 2048: 7 rows 11.8 | 7.4, 64 12.2 | 8.1, 4096 54 | 34; 16 experts, width 8192: 7 rows
+// 22.5 | 16.7, 4096 273 | 185; 4 experts, width 512, 4096 rows 21 | 20.
+#define RT_AHEAD_NV 2
+#define RT_NORM_ENTRIES 17      // the router's rows at most: more would be read by every row's workgroup one behind the other
+#define RT_PLAN_ROWS 128        // the last workgroup's plan: arrivals are counted in eights, then at the root (about 0.1 us each behind the other); against a launch behind: 7 rows 7.1 | 6.4, 128 7.4 | 7.1
+template <int NV, bool MIX>
+__global__ __launch_bounds__(256) void residual_route_kernel(const i64h_streams_args p, const i64h_route_args q, const i64h_moe_plan_args pl, int32_t* sync) {
+    __shared__ float red[4], part[4][RT_NORM_ENTRIES + 7];
+    __shared__ int plan_lds[2 * RT_NORM_ENTRIES + 1], last, sIdx[RT_PLAN_ROWS * RT_NORM_ENTRIES];
+    __shared__ float sWgt[RT_PLAN_ROWS * RT_NORM_ENTRIES];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, W = p.W, rows = q.gate_out ? q.E + 1 : q.E;
+    const int64_t t = blockIdx.x;
+    const uint16_t* Wr = (const uint16_t*)q.W;
+    auto weights = [&](int e, int i) {
+        const int c = (i * 256 + tid) * 4;
+        return e < rows && c < W ? *(const uint2*)(Wr + (int64_t)e * W + c) : make_uint2(0, 0);
+    };
+    constexpr bool AHEAD = NV <= RT_AHEAD_NV;
+    uint2 ahead[AHEAD ? NV : 1][9];
+    if constexpr (AHEAD) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int j = 0; j < 9; ++j) ahead[i][j] = weights(j, i);
+    }
+    residual_row<NV, MIX>(p, red, [&](const float (&v)[NV][4]) {
+        auto dot = [&](float a, int i, uint2 w) {
+            a = fmaf(v[i][0], __uint_as_float(w.x << 16), a);
+            a = fmaf(v[i][1], __uint_as_float(w.x & 0xffff0000u), a);
+            a = fmaf(v[i][2], __uint_as_float(w.y << 16), a);
+            return fmaf(v[i][3], __uint_as_float(w.y & 0xffff0000u), a);
+        };
+        auto keep = [&](const float* acc, int e0) {
+            const float s = rt_sum8(acc);
+            if ((lane & 7) == 0) part[wid][e0 + (lane >> 3)] = s;
+        };
+        int e0 = 0;
+        if constexpr (AHEAD) {
+            float acc[9] = {};
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+#pragma unroll
+                for (int j = 0; j < 9; ++j) acc[j] = dot(acc[j], i, ahead[i][j]);
+            keep(acc, 0);
+            e0 = 8;
+            if (rows == 9) {
+                const float s = wave_sum(acc[8]);
+                if (lane == 0) part[wid][8] = s;
+                e0 = 9;
+            }
+        }
+        for (; e0 < rows; e0 += 8) {
+            float acc[8] = {};
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+                uint2 w[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) w[j] = weights(e0 + j, i);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) acc[j] = dot(acc[j], i, w[j]);
+            }
+            keep(acc, e0);
+        }
+    });
+    __syncthreads();
+    if (wid == 0) {
+        float z = 0.0f;
+        if (lane < rows) {
+            z = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+            if (lane == q.E) q.gate_out[t] = rt_sigmoid(z);
+            else if (q.bias) z += q.bias[lane];
+        }
+        if (!sync) rt_choose_few<false>(q, t, lane, z);
+        else {
+            rt_choose_few<true>(q, t, lane, z);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (the choice has left the CU before the arrival is counted)
+            if (lane == 0) {
+                // counters at zero between launches: whoever comes last in a group of eight, and of the groups, puts its counter back
+                const int g = (int)(t >> 3), of = min(8, (int)gridDim.x - 8 * g), groups = (gridDim.x + 7) >> 3;
+                int end = 0;
+                if (__hip_atomic_fetch_add(sync + 32 + 32 * g, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == of - 1) {
+                    __hip_atomic_store(sync + 32 + 32 * g, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (groups == 1) end = 1;
+                    else if (__hip_atomic_fetch_add(sync, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == groups - 1) {
+                        __hip_atomic_store(sync, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        end = 1;
+                    }
+                }
+                last = end;
+            }
+        }
+    }
+    if (!sync) return;
+    __syncthreads();
+    if (!last) return;
+    for (int i = tid; i < (int)pl.n * pl.top; i += 256) {
+        sIdx[i] = __hip_atomic_load(pl.idx + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (pl.pair_wgt) sWgt[i] = ld_agent(pl.wgt + i);
+    }
+    rt_plan<256>(pl, plan_lds, [&](int64_t i) { return sIdx[i]; }, [&](int64_t i) { return sWgt[i]; });      // (a thread reads what it wrote)
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------
@@ -984,14 +1102,13 @@ int i64h_set_residual_form(int32_t on) {
     return 0;
 }
 
-int i64h_streams_step(const i64h_streams_args* dp, void* stream) {
-    I64H_CHECK_ARG(dp != nullptr, "streams: no descriptor");
-    const i64h_streams_args& d = *dp;
+static int streams_run(const i64h_streams_args& d, const i64h_route_args* route, const i64h_moe_plan_args* plan, int32_t* sync, void* stream) {
     I64H_CHECK_ARG(d.S >= 1 && d.S <= HY_MAX_STREAMS && d.W > 0 && d.n >= 0, "streams: %d streams (at most %d), width %d", d.S, HY_MAX_STREAMS, d.W);
-    I64H_CHECK_ARG(d.streams && (d.y || d.moe_y || d.h || d.h16), "streams: nothing to do");
+    I64H_CHECK_ARG(d.streams && (d.y || d.moe_y || d.h || d.h16 || route), "streams: nothing to do");
     I64H_CHECK_ARG(!(d.y || d.moe_y) || d.out_w, "streams: the write needs out_w");
     I64H_CHECK_ARG(!d.y2 || (d.y && !d.yn_w == !d.y2n_w), "streams: two results take both norm weights or none");
-    I64H_CHECK_ARG(!(d.h || d.h16) || (d.norm_w && (d.norm_w_len == 1 || d.norm_w_len == d.W)), "streams: the read needs a norm weight of 1 or W values");
+    const bool reads = d.h || d.h16 || route;
+    I64H_CHECK_ARG(!reads || (d.norm_w && (d.norm_w_len == 1 || d.norm_w_len == d.W)), "streams: the read needs a norm weight of 1 or W values");
     I64H_CHECK_ARG(!d.moe_y || (d.moe_row && d.moe_h && d.moe_top > 0 && !d.y2), "streams: a mixture's result needs its rows and choices, and no second result beside it");
     I64H_CHECK_ARG(!d.rows || !(d.y || d.moe_y), "streams: gathered rows are read only");
     const int64_t rows = d.rows ? d.m_rows : d.n;
@@ -1001,9 +1118,21 @@ int i64h_streams_step(const i64h_streams_args* dp, void* stream) {
     const uintptr_t at = (uintptr_t)d.streams | (uintptr_t)d.y | (uintptr_t)d.y2 | (uintptr_t)d.y_scale | (uintptr_t)d.norm_w | (uintptr_t)d.norm_b | (uintptr_t)d.h | (uintptr_t)d.h16 | (uintptr_t)d.moe_y |
                          (uintptr_t)d.moe_h | (uintptr_t)d.moe_shared;
     if (g_residual_form && d.S == 1 && !d.mix && !d.in_w && !d.yn_w && !d.post_w && d.W % 4 == 0 && d.W <= 8 * 1024 && at % 16 == 0 && (!d.y || d.ldy % 4 == 0) &&
-        (!d.y2 || d.ldy2 % 4 == 0) && (!(d.h || d.h16) || d.norm_w_len == d.W)) {
+        (!d.y2 || d.ldy2 % 4 == 0) && (!reads || d.norm_w_len == d.W)) {
         const dim3 grid((unsigned)rows);
-        auto launch = [&](auto sum, auto mix) { hipLaunchKernelGGL(d.moe_y ? mix : sum, grid, dim3(256), 0, (hipStream_t)stream, d); };
+        i64h_streams_args a = d;
+        if (!reads) a.norm_w = nullptr;      // (nobody reads the row)
+        if (route) {
+            const i64h_moe_plan_args none = {};
+            auto launch = [&](auto sum, auto mix) { hipLaunchKernelGGL(d.moe_y ? mix : sum, grid, dim3(256), 0, (hipStream_t)stream, a, *route, plan ? *plan : none, plan ? sync : nullptr); };
+            if (d.W <= 1024) launch(residual_route_kernel<1, false>, residual_route_kernel<1, true>);
+            else if (d.W <= 2048) launch(residual_route_kernel<2, false>, residual_route_kernel<2, true>);
+            else if (d.W <= 4096) launch(residual_route_kernel<4, false>, residual_route_kernel<4, true>);
+            else launch(residual_route_kernel<8, false>, residual_route_kernel<8, true>);
+            I64H_CHECK_LAUNCH();
+            return 0;
+        }
+        auto launch = [&](auto sum, auto mix) { hipLaunchKernelGGL(d.moe_y ? mix : sum, grid, dim3(256), 0, (hipStream_t)stream, a); };
         if (d.W <= 1024) launch(residual_kernel<1, false>, residual_kernel<1, true>);
         else if (d.W <= 2048) launch(residual_kernel<2, false>, residual_kernel<2, true>);
         else if (d.W <= 4096) launch(residual_kernel<4, false>, residual_kernel<4, true>);
@@ -1011,10 +1140,32 @@ int i64h_streams_step(const i64h_streams_args* dp, void* stream) {
         I64H_CHECK_LAUNCH();
         return 0;
     }
+    I64H_CHECK_ARG(!route, "streams: a router behind several streams, result norms or rows that are not read 16 bytes at a time");
     I64H_CHECK_ARG(!d.moe_y, "streams: a mixture's result with several streams, result norms or rows that are not read 16 bytes at a time");
     hipLaunchKernelGGL(streams_kernel, dim3((unsigned)rows), dim3(256), lds, (hipStream_t)stream, d);
     I64H_CHECK_LAUNCH();
     return 0;
+}
+
+int i64h_streams_step(const i64h_streams_args* dp, void* stream) {
+    I64H_CHECK_ARG(dp != nullptr, "streams: no descriptor");
+    return streams_run(*dp, nullptr, nullptr, nullptr, stream);
+}
+
+int i64h_streams_route(const i64h_streams_args* dp, const i64h_route_args* rp, const i64h_moe_plan_args* pp, int32_t* sync, void* stream) {
+    I64H_CHECK_ARG(dp != nullptr && rp != nullptr, "streams_route: no descriptor");
+    const i64h_streams_args& d = *dp;
+    const i64h_route_args& r = *rp;
+    I64H_CHECK_ARG(r.E > 0 && r.E + (r.gate_out ? 1 : 0) <= RT_NORM_ENTRIES && r.top > 0 && r.top <= r.E && r.groups <= 1, "streams_route: %d entries in %d groups, top %d (one group of at most %d with a gate's row)",
+                   r.E, r.groups, r.top, RT_NORM_ENTRIES);
+    I64H_CHECK_ARG(r.W && (uintptr_t)r.W % 8 == 0 && r.K == d.W && !d.rows && r.n == d.n && r.idx && r.wgt && !(r.sigmoid_scores && r.chosen_softmax), "streams_route: the router does not fit the rows");
+    if (pp) {
+        const i64h_moe_plan_args& m = *pp;
+        I64H_CHECK_ARG(sync && d.n <= RT_PLAN_ROWS, "streams_route: a plan of %lld rows (at most %d), with counters", (long long)d.n, RT_PLAN_ROWS);
+        I64H_CHECK_ARG(m.idx == r.idx && m.n == d.n && m.top == r.top && m.experts > 0 && m.experts <= r.E && m.group_off && m.pair_token && m.pair_row && (!m.pair_wgt || m.wgt == r.wgt),
+                       "streams_route: the plan is not that of the choice");
+    }
+    return streams_run(d, rp, pp, sync, stream);
 }
 
 int i64h_causal_conv(const i64h_causal_conv_args* dp, void* stream) {

@@ -427,6 +427,7 @@ class HybridRunner:
         B.pair_wgt = torch.empty(n * max(g, 1), **f32)
         B.group_off = torch.empty(model.max_groups + 1, **i32)
         B.sgate = torch.empty(n, **f32)
+        B.sync = torch.zeros(32 * (D.PLAN_ROWS // 8 + 1), **i32) if t else None      # counters of the launches that plan a step behind its norm
         B.sact = torch.empty(n * max(shared, 1), **f32)                    # the inner rows of a shared expert beside the grouped launches
         B.shared_rows = n if shared else 0
 
@@ -495,10 +496,37 @@ class HybridRunner:
         """Whether the residual's launch sums a mixture's rows itself (i64h_streams_args.moe_y)."""
         return self.cfg.width % 4 == 0 and self.cfg.width <= 8192
 
-    def _moe_ff(self, B, d, n, h, out, shared_out, record: Optional[dict] = None, tag: str = "", beside: bool = False, h16=None, combine: bool = True):
+    # the router's products in 32 bits in both modes (a choice between experts is not rounding's to make), inside the choice's launch
+    def _route(self, B, d) -> dict:
+        f = d["mlp"]
+        return dict(w=d["router"], entries=f.entries, correction=d.get("correction"), groups=f.groups, keep=f.keep, top=f.top, scale=f.scale, idx=B.idx, wgt=B.wgt, bias=d["router_b"],
+                    chosen_softmax=f.chosen_softmax, gate_out=B.sgate if f.shared_ff and f.shared_gate else None, sigmoid_scores=f.sigmoid_scores, raw_weights=f.raw_weights)
+
+    def _plan(self, B, d) -> dict:
+        f = d["mlp"]
+        return dict(experts=f.experts, group_off=B.group_off, pair_token=B.pair_token, pair_row=B.pair_row, pair_wgt=B.pair_wgt if f.weigh_input else None,      # the weight multiplies what the expert reads, not what it returns
+                    shared=d["merged"] and B.joined)
+
+    def _routes_in_norm(self, f) -> bool:
+        """Whether the launch that norms a mixture's input also chooses its experts (i64h_streams_route), and plans the step where it is small."""
+        return f.entries + int(bool(f.shared_ff and f.shared_gate)) <= D.ROUTE_ENTRIES and f.groups <= 1 and self._moe_merges()
+
+    def _moe_read(self, B, d, n, h, h16) -> dict:
+        """What the launch that norms a mixture's input is to write and choose: h stays away where everybody behind it reads rows in bf16."""
+        f = d["mlp"]
+        if not self._routes_in_norm(f):
+            return dict(h=h, h16=h16)
+        bare = h16 is not None and f.entries == f.experts and self._experts_read16(d, n, d["merged"] and B.joined)
+        return dict(h=None if bare else h, h16=h16, route=self._route(B, d), **(dict(plan=self._plan(B, d), sync=B.sync) if n <= D.PLAN_ROWS else {}))
+
+    def _experts_read16(self, d, n: int, merged: bool) -> bool:
+        f = d["mlp"]
+        return self._fills(n * f.top, f.experts) and not self._streams(n, self.cfg.width, f.experts, merged)
+
+    def _moe_ff(self, B, d, n, h, out, shared_out, record: Optional[dict] = None, tag: str = "", beside: bool = False, h16=None, combine: bool = True, routed: bool = False):
         """out <- the mixture of d["mlp"] on h fp32 [n, width] (h16: its rows in bf16, which the experts read); shared_out [n, width] receives the rows of a
         shared expert that is not in the experts' stack on the way (beside: on the side stream, while the routed experts run).  combine False: the
-        weighted sum is left to the caller's residual launch, whose operands are returned."""
+        weighted sum is left to the caller's residual launch, whose operands are returned.  routed: the launch that normed h was given _moe_read's operands."""
         f, ex, W = d["mlp"], self.exact, self.cfg.width
         E, top = f.experts, f.top
         merged = d["merged"] and B.joined
@@ -510,18 +538,19 @@ class HybridRunner:
                 D.linear(h, d["s_gate_up"], sact, a16=h16, out16=sact16, exact=ex, **self._glu(f.shared_limit, f.glu_alpha))
                 shared = D.linear(sact, d["s_down"], shared_out, a16=sact16, exact=ex)
         gate_up, e_down = (d["gate_up"], d["e_down"]) if merged or not d["merged"] else (d["gate_up"][1:], d["e_down"][1:])
-        # the router's products in 32 bits in both modes (a choice between experts is not rounding's to make), inside the choice's launch
-        D.route_topk(None, h=h, w=d["router"], entries=f.entries, correction=d.get("correction"), groups=f.groups, keep=f.keep, top=top, scale=f.scale,
-                     idx=B.idx, wgt=B.wgt, n=n, bias=d["router_b"], chosen_softmax=f.chosen_softmax, gate_out=gate, sigmoid_scores=f.sigmoid_scores, raw_weights=f.raw_weights)
+        routed = routed and self._routes_in_norm(f)
+        if not routed:
+            D.route_topk(None, h=h, n=n, **self._route(B, d))
         if record is not None:
             record[f"{tag}.route"] = B.idx[: n * top].view(n, top).clone()
-        pair_wgt = B.pair_wgt if f.weigh_input else None      # the weight multiplies what the expert reads, not what it returns
-        D.moe_plan(B.idx, n=n, top=top, experts=E, group_off=B.group_off, pair_token=B.pair_token, pair_row=B.pair_row, wgt=B.wgt, pair_wgt=pair_wgt, shared=merged)
+        plan = self._plan(B, d)
+        if not (routed and n <= D.PLAN_ROWS):
+            D.moe_plan(B.idx, n=n, top=top, wgt=B.wgt, **plan)
         # the (token, expert) pairs lie grouped by expert: one launch runs every expert over its own rows, the counts stay on the device
-        x16 = h16 if self._fills(n * top, E) and not self._streams(n, W, E, merged) else None
+        x16 = h16 if self._experts_read16(d, n, merged) else None
         rows, groups = n * (top + int(merged)), E + int(merged)
         act, act16 = self._act(B.act, B.act16, rows, f.ff, x16)
-        D.linear(h, gate_up, act, a16=x16, out16=act16, m=n, a_rows=B.pair_token[:rows], batch=groups, w_batch=2 * f.ff * W, exact=ex, group_off=B.group_off, row_scale=pair_wgt,
+        D.linear(h, gate_up, act, a16=x16, out16=act16, m=n, a_rows=B.pair_token[:rows], batch=groups, w_batch=2 * f.ff * W, exact=ex, group_off=B.group_off, row_scale=plan["pair_wgt"],
                  **self._glu(f.limit, f.glu_alpha))
         D.linear(act, e_down, B.ey[:rows], a16=act16, m=n, batch=groups, w_batch=W * f.ff, exact=ex, group_off=B.group_off)
         if shared is not None and beside:

@@ -257,12 +257,14 @@ def streams_step(streams: torch.Tensor, *, y: Optional[torch.Tensor] = None, y2:
                  in_w: Optional[torch.Tensor] = None, norm_w: Optional[torch.Tensor] = None, eps: float = 0.0, h: Optional[torch.Tensor] = None,
                  rows: Optional[torch.Tensor] = None, post_w: Optional[torch.Tensor] = None, post_center: bool = False,
                  h_center: bool = False, norm_b: Optional[torch.Tensor] = None, y_scale: Optional[torch.Tensor] = None,
-                 h16: Optional[torch.Tensor] = None, moe: Optional[dict] = None) -> Optional[torch.Tensor]:
+                 h16: Optional[torch.Tensor] = None, moe: Optional[dict] = None, route: Optional[dict] = None, plan: Optional[dict] = None,
+                 sync: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """See i64h_streams_step.  streams fp32 [S, n, W], updated in place when y is given; h fp32 [n, W] (or [rows, W]).  post_w fp32 [W]: a
     norm over the result as a whole (centred with post_center) before it is added; h_center: the read's norm is centred; norm_b: added behind
     the read's norm weight.  y2 without norm weights is simply added to y.  y_scale fp32 [W]: a factor per column on what is added.
     h16 bf16 [n, W]: the rows of h rounded, beside h or (h None) in its place.  moe (one stream, no result norms): the arguments of moe_combine but `out`, whose
-    result stands for y or is added to it."""
+    result stands for y or is added to it.  route: the arguments of route_topk but logits and h, the choice on the rows of h in the same launch (see i64h_streams_route); plan: those of
+    moe_plan but idx, n and top, for at most PLAN_ROWS rows, with sync int32 [32 * 17], zeros between launches."""
     _chk(streams, torch.float32, "streams")
     S, n, W = streams.shape
     for t, name in ((y, "y"), (y2, "y2"), (yn_w, "yn_w"), (y2n_w, "y2n_w"), (mix, "mix"), (out_w, "out_w"), (in_w, "in_w"), (norm_w, "norm_w"), (h, "h"),
@@ -297,8 +299,22 @@ def streams_step(streams: torch.Tensor, *, y: Optional[torch.Tensor] = None, y2:
                      mix=ptr(mix), out_w=ptr(out_w), in_w=ptr(in_w), norm_w=ptr(norm_w), norm_w_len=norm_w.numel() if norm_w is not None else 0,
                      eps=float(eps), h=ptr(h), rows=ptr(rows), m_rows=m_rows, post_w=ptr(post_w), post_center=int(bool(post_center)), h_center=int(bool(h_center)),
                      norm_b=ptr(norm_b), y_scale=ptr(y_scale), h16=ptr(h16), **mk)
-    call_dense("i64h_streams_step", _ref(d), _stream())
+    if route is None:
+        call_dense("i64h_streams_step", _ref(d), _stream())
+        return h
+    if rows is not None or route["w"].shape[-1] != W:
+        raise _lib.I64HError("streams_step: a router on rows that are not its own")
+    r, m = _route_args(n=n, **route), None
+    if plan is not None:
+        m = _plan_args(route["idx"], n=n, top=route["top"], wgt=route["wgt"], **plan)
+        _chk(sync, torch.int32, "sync")
+        if sync.numel() < 32 * 17:
+            raise _lib.I64HError("streams_step: fewer counters than the plan needs")
+    call_dense("i64h_streams_route", _ref(d), _ref(r), _ref(m) if m is not None else 0, ptr(sync) if m is not None else 0, _stream())
     return h
+
+
+ROUTE_ENTRIES, PLAN_ROWS = 17, 128      # the router's rows, and the rows of a plan, that a norm's launch takes
 
 
 def causal_conv(p: torch.Tensor, *, off: int, channels: int, w: torch.Tensor, bias: Optional[torch.Tensor], positions: torch.Tensor,
@@ -683,26 +699,14 @@ def rec_step(p: torch.Tensor, *, q_off: int, k_off: int = 0, v_off: int = 0, hea
     call_dense("i64h_rec_step", _ref(d), _stream())
 
 
-def route_topk(logits: Optional[torch.Tensor], *, entries: int, correction: Optional[torch.Tensor], groups: int, keep: int, top: int, scale: float, idx: torch.Tensor,
-               wgt: torch.Tensor, n: Optional[int] = None, h: Optional[torch.Tensor] = None, w: Optional[torch.Tensor] = None,
-               bias: Optional[torch.Tensor] = None, chosen_softmax: bool = False, gate_out: Optional[torch.Tensor] = None,
-               sigmoid_scores: bool = False, raw_weights: bool = False) -> None:
-    """See i64h_route_topk.  logits fp32 [n, ld >= entries], or None with h fp32 [n, K] and w bf16 [entries, K]: the launch computes the
-    logits itself in 32 bits; idx int32 [n, top]; wgt fp32 [n, top].  bias fp32 [entries]; gate_out fp32 [n]: w has one more row, whose
-    product's sigmoid it receives.  sigmoid_scores: sigmoid in the softmax's place; raw_weights: scores as weights, not renormalised."""
+def _route_args(*, entries: int, top: int, scale: float, idx: torch.Tensor, wgt: torch.Tensor, n: int, correction: Optional[torch.Tensor] = None, groups: int = 1, keep: int = 1,
+                w: Optional[torch.Tensor] = None, bias: Optional[torch.Tensor] = None, chosen_softmax: bool = False, gate_out: Optional[torch.Tensor] = None,
+                sigmoid_scores: bool = False, raw_weights: bool = False, **rows) -> "_lib.Route":
     _chk(idx, torch.int32, "idx"), _chk(wgt, torch.float32, "wgt")
-    if logits is None:
-        if h is None or w is None:
-            raise _lib.I64HError("route_topk: logits, or the router's input and weight")
-        _chk(h, torch.float32, "h"), _chk(w, torch.bfloat16, "w")
-        rows = int(n if n is not None else h.shape[0])
-        if w.dim() != 2 or w.shape[0] != entries + (1 if gate_out is not None else 0) or h.shape[-1] != w.shape[1] or h.numel() < rows * h.shape[-1]:
+    if w is not None:
+        _chk(w, torch.bfloat16, "w")
+        if w.dim() != 2 or w.shape[0] != entries + (1 if gate_out is not None else 0):
             raise _lib.I64HError("route_topk: the router's input and weight do not fit the sizes")
-    else:
-        _chk(logits, torch.float32, "logits")
-        rows = int(n if n is not None else logits.shape[0])
-        if logits.shape[-1] < entries or logits.numel() < rows * logits.shape[-1]:
-            raise _lib.I64HError("route_topk: shapes do not fit the sizes")
     if correction is not None:
         _chk(correction, torch.float32, "correction")
         if correction.numel() != entries:
@@ -713,22 +717,43 @@ def route_topk(logits: Optional[torch.Tensor], *, entries: int, correction: Opti
             raise _lib.I64HError("route_topk: the bias is not [entries]")
     if gate_out is not None:
         _chk(gate_out, torch.float32, "gate_out")
-        if logits is not None or gate_out.numel() < rows:
+        if w is None or gate_out.numel() < n:
             raise _lib.I64HError("route_topk: the gate needs the router's weight and a value per row")
-    if idx.numel() < rows * top or wgt.numel() < rows * top:
+    if idx.numel() < n * top or wgt.numel() < n * top:
         raise _lib.I64HError("route_topk: shapes do not fit the sizes")
-    d = _lib.Route(logits=ptr(logits), ld=logits.shape[-1] if logits is not None else 0, E=entries, correction=ptr(correction), groups=int(groups), keep=int(keep),
-                   top=int(top), scale=float(scale), idx=ptr(idx), wgt=ptr(wgt), n=rows, h=ptr(h) if logits is None else 0,
-                   ldh=h.shape[-1] if logits is None else 0, W=ptr(w) if logits is None else 0, K=w.shape[1] if logits is None else 0,
-                   bias=ptr(bias), chosen_softmax=int(bool(chosen_softmax)), gate_out=ptr(gate_out), sigmoid_scores=int(bool(sigmoid_scores)),
-                   raw_weights=int(bool(raw_weights)))
+    return _lib.Route(E=entries, correction=ptr(correction), groups=int(groups), keep=int(keep), top=int(top), scale=float(scale), idx=ptr(idx), wgt=ptr(wgt), n=n,
+                      W=ptr(w), K=w.shape[1] if w is not None else 0, bias=ptr(bias), chosen_softmax=int(bool(chosen_softmax)), gate_out=ptr(gate_out),
+                      sigmoid_scores=int(bool(sigmoid_scores)), raw_weights=int(bool(raw_weights)), **rows)
+
+
+def route_topk(logits: Optional[torch.Tensor], *, entries: int, correction: Optional[torch.Tensor], groups: int, keep: int, top: int, scale: float, idx: torch.Tensor,
+               wgt: torch.Tensor, n: Optional[int] = None, h: Optional[torch.Tensor] = None, w: Optional[torch.Tensor] = None,
+               bias: Optional[torch.Tensor] = None, chosen_softmax: bool = False, gate_out: Optional[torch.Tensor] = None,
+               sigmoid_scores: bool = False, raw_weights: bool = False) -> None:
+    """See i64h_route_topk.  logits fp32 [n, ld >= entries], or None with h fp32 [n, K] and w bf16 [entries, K]: the launch computes the
+    logits itself in 32 bits; idx int32 [n, top]; wgt fp32 [n, top].  bias fp32 [entries]; gate_out fp32 [n]: w has one more row, whose
+    product's sigmoid it receives.  sigmoid_scores: sigmoid in the softmax's place; raw_weights: scores as weights, not renormalised."""
+    if logits is None:
+        if h is None or w is None:
+            raise _lib.I64HError("route_topk: logits, or the router's input and weight")
+        _chk(h, torch.float32, "h")
+        rows = int(n if n is not None else h.shape[0])
+        if h.shape[-1] != w.shape[-1] or h.numel() < rows * h.shape[-1]:
+            raise _lib.I64HError("route_topk: the router's input and weight do not fit the sizes")
+        src = dict(w=w, h=ptr(h), ldh=h.shape[-1])
+    else:
+        _chk(logits, torch.float32, "logits")
+        rows = int(n if n is not None else logits.shape[0])
+        if logits.shape[-1] < entries or logits.numel() < rows * logits.shape[-1]:
+            raise _lib.I64HError("route_topk: shapes do not fit the sizes")
+        src = dict(logits=ptr(logits), ld=logits.shape[-1])
+    d = _route_args(entries=entries, correction=correction, groups=groups, keep=keep, top=top, scale=scale, idx=idx, wgt=wgt, n=rows, bias=bias, chosen_softmax=chosen_softmax,
+                    gate_out=gate_out, sigmoid_scores=sigmoid_scores, raw_weights=raw_weights, **src)
     call_dense("i64h_route_topk", _ref(d), _stream())
 
 
-def moe_plan(idx: torch.Tensor, *, n: int, top: int, experts: int, group_off: torch.Tensor, pair_token: torch.Tensor, pair_row: torch.Tensor,
-             wgt: Optional[torch.Tensor] = None, pair_wgt: Optional[torch.Tensor] = None, shared: bool = False) -> None:
-    """See i64h_moe_plan.  pair_wgt fp32 [n * top] receives the choices' weights wgt fp32 [n, top] in the grouped order.  shared: one more group, in
-    front, of every token once."""
+def _plan_args(idx: torch.Tensor, *, n: int, top: int, experts: int, group_off: torch.Tensor, pair_token: torch.Tensor, pair_row: torch.Tensor,
+             wgt: Optional[torch.Tensor] = None, pair_wgt: Optional[torch.Tensor] = None, shared: bool = False) -> "_lib.MoePlan":
     rows = n * top + (n if shared else 0)
     if pair_wgt is not None:
         _chk(wgt, torch.float32, "wgt"), _chk(pair_wgt, torch.float32, "pair_wgt")
@@ -738,8 +763,15 @@ def moe_plan(idx: torch.Tensor, *, n: int, top: int, experts: int, group_off: to
         _chk(t, torch.int32, name)
     if idx.numel() < n * top or group_off.numel() < experts + 1 + int(bool(shared)) or pair_token.numel() < rows or pair_row.numel() < n * top:
         raise _lib.I64HError("moe_plan: shapes do not fit the sizes")
-    d = _lib.MoePlan(idx=ptr(idx), n=n, top=top, experts=experts, group_off=ptr(group_off), pair_token=ptr(pair_token), pair_row=ptr(pair_row),
-                     wgt=ptr(wgt) if pair_wgt is not None else 0, pair_wgt=ptr(pair_wgt), shared=int(bool(shared)))
+    return _lib.MoePlan(idx=ptr(idx), n=n, top=top, experts=experts, group_off=ptr(group_off), pair_token=ptr(pair_token), pair_row=ptr(pair_row),
+                        wgt=ptr(wgt) if pair_wgt is not None else 0, pair_wgt=ptr(pair_wgt), shared=int(bool(shared)))
+
+
+def moe_plan(idx: torch.Tensor, *, n: int, top: int, experts: int, group_off: torch.Tensor, pair_token: torch.Tensor, pair_row: torch.Tensor,
+             wgt: Optional[torch.Tensor] = None, pair_wgt: Optional[torch.Tensor] = None, shared: bool = False) -> None:
+    """See i64h_moe_plan.  pair_wgt fp32 [n * top] receives the choices' weights wgt fp32 [n, top] in the grouped order.  shared: one more group, in
+    front, of every token once."""
+    d = _plan_args(idx, n=n, top=top, experts=experts, group_off=group_off, pair_token=pair_token, pair_row=pair_row, wgt=wgt, pair_wgt=pair_wgt, shared=shared)
     call_dense("i64h_moe_plan", _ref(d), _stream())
 
 

@@ -138,7 +138,7 @@ class PukatarModel(HybridRunner):
         if d["mlp"].kind == "dense":
             self._dense_glu(B, d, n, B.h, B.y2, h16)
             return dict(y2=B.y2)
-        sums = self._moe_ff(B, d, n, B.h, B.y2, B.y3, record, f"r{r}", h16=h16, combine=combine)
+        sums = self._moe_ff(B, d, n, B.h, B.y2, B.y3, record, f"r{r}", h16=h16, combine=combine, routed=True)
         return dict(y2=B.y2) if combine else dict(moe=sums)
 
     @torch.no_grad()
@@ -171,7 +171,7 @@ class PukatarModel(HybridRunner):
 
         def normed(d):      # a layer's input: in bf16 alone where no router reads it
             moe = d["mlp"] is not None and d["mlp"].kind == "moe"
-            return read(d["norm1"], B.h if moe or B.h16 is None else None, h16=B.h16)
+            return read(d["norm1"], **(self._moe_read(B, d, n, B.h, B.h16) if moe else dict(h=B.h if B.h16 is None else None, h16=B.h16)))
         D.embed_scaled(token_ids, self.embed, 1.0, B.e)
         cur = 0
         D.streams_step(B.e, **read(self.embed_norm, B.x[0]))

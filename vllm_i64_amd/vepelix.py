@@ -147,7 +147,7 @@ class VepelixModel(HybridRunner):
         if d["mlp"].kind == "dense":
             self._dense_glu(B, d, n, B.h, B.y, h16)
             return dict(y=B.y)
-        sums = self._moe_ff(B, d, n, B.h, B.y, B.y2, record, f"r{r}", beside=True, h16=h16, combine=combine)
+        sums = self._moe_ff(B, d, n, B.h, B.y, B.y2, record, f"r{r}", beside=True, h16=h16, combine=combine, routed=True)
         return dict(y=B.y) if combine else dict(moe=sums)
 
     @torch.no_grad()
@@ -188,7 +188,7 @@ class VepelixModel(HybridRunner):
             write = self._mixer(B, d, r, n, positions, slot_ids, kvc, seg, nseg, runs, int(max_ctx_hint), B.h16, work)
             write.update(out_w=self.ones1, y_scale=d["ls1"])
             if d["mlp"] is not None:
-                D.streams_step(x, **write, **(normed(d["norm2"]) if d["mlp"].kind == "dense" else read(d["norm2"], B.h, h16=B.h16)))
+                D.streams_step(x, **write, **(normed(d["norm2"]) if d["mlp"].kind == "dense" else read(d["norm2"], **self._moe_read(B, d, n, B.h, B.h16))))
                 write = self._feed_forward(B, d, n, record, r, B.h16, not self._moe_merges())
                 write.update(out_w=self.ones1, y_scale=d["ls2"])
             if r + 1 < len(self.layer_runs) and not self.layer_runs[r + 1][1]:
