@@ -205,3 +205,36 @@ def test_gathered_rows_of_a_matrix_of_unknown_height(dev, use_form, M):
     d = _lib.Linear(A=D.ptr(ad), lda=K, a_rows=D.ptr(rd), W=D.ptr(wd), C=D.ptr(out), ldc=N, M=M, N=N, K=K, batch=1)
     D.call_dense("i64h_linear_run", D._ref(d), D._stream())
     assert close(out, bf16(a[rows.long()]).double() @ w.double().T, K)
+
+
+@pytest.mark.parametrize("form", ["64x64", "64x128 (32x64 in 32 bits)", "32x64/4", "16x64/4", "16x128/2 pair", "32x128/2", "by size"])
+def test_parts_of_32_bit_rows(dev, use_form, form):
+    """Rows of 32-bit values as three bf16 parts: values of all magnitudes keep their 24 bits, infinities and NaN stay what a product term by term makes of them, in rows and in weights."""
+    from vllm_i64_amd import ops_dense as D
+    use_form(form)
+    M, N, K = 37, 72, 200
+    g = torch.Generator().manual_seed(5)
+    a = torch.randn(M, K, generator=g) * 10.0 ** torch.randint(-18, 18, (M, 1), generator=g)
+    w = bf16(torch.randn(2 * N, K, generator=g))
+    a[3] = torch.randint(-(1 << 24) + 1, 1 << 24, (K,), generator=g).float()      # all 24 bits used
+    w[5] = 0
+    w[5, 7] = 1
+    out = torch.empty(M, N, device=dev)
+    D.linear(a.to(dev), w[:N].contiguous().to(dev), out, exact=True)
+    ref = a.double() @ w[:N].double().T
+    assert torch.equal(out.cpu()[:, 5], a[:, 7])                                 # a value comes through as it is
+    scale = a.double().abs() @ w[:N].double().abs().T
+    assert ((out.double().cpu() - ref).abs() <= scale * 2.0 ** -23).all()        # (a sum of K terms rounded a few dozen times, each time by 2^-24 of a partial sum)
+    a[1, 3], a[2, 4], a[4, 5], a[4, 6], a[6, 8] = float("inf"), float("-inf"), float("inf"), float("-inf"), float("nan")
+    a[8, 0] = 3.3e38
+    w[9, 11], w[10, 0], w[N + 9, 11] = float("inf"), float("-inf"), float("inf")
+    D.linear(a.to(dev), w[:N].contiguous().to(dev), out, exact=True)
+    ref = (a[:, None, :].double() * w[None, :N].double()).sum(-1).float()
+    got = out.cpu()
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got[ref.isinf()], ref[ref.isinf()])
+    D.linear(a.to(dev), w.to(dev), out, exact=True, epilogue=D.EPI_SILU_MUL)
+    up = (a[:, None, :].double() * w[None, N:].double()).sum(-1).float()
+    z = ref.double()
+    want = (z * torch.sigmoid(z) * up.double()).float()
+    ok = torch.isfinite(ref) & torch.isfinite(up)
+    assert torch.equal(out.cpu()[ok].isnan(), want[ok].isnan()) and out.cpu()[(ref.isnan() | up.isnan())].isnan().all()

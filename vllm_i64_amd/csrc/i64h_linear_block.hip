@@ -1,4 +1,4 @@
-// C = epilogue(A W^T), A fp32, W bf16 [N, K], on v_mfma_f32_16x16x32_bf16 (A rounded to bf16 while it is staged) or with true 32-bit products: BM x BN tiles staged
+// C = epilogue(A W^T), A fp32, W bf16 [N, K], on v_mfma_f32_16x16x32_bf16 (A rounded to bf16 while it is staged, or in three parts for 32-bit products): BM x BN tiles staged
 // through LDS, four waves a tile and KG groups of four waves that share a tile's k steps.
 //
 // What bounds it.  Large launches: the step from memory to LDS - A is read as 32-bit values and rounded on the way, so a 128 x 128 tile moves
@@ -11,18 +11,19 @@
 #include "i64h_dense_dev.h"
 #include <type_traits>
 
-// EX: 32-bit products on v_mfma_f32_16x16x4_f32, W widened while it is staged.  A staged row is 128 bytes either way: steps of 64 or of 32 values.
+// EX: products of 32-bit rows.  W is bf16, so a row's value x = hi + mid + lo, three bf16 of eight bits each cut off in turn, makes x w the sum of three products that the bf16
+// instruction takes exactly, summed in 32 bits: three instructions in the place of eight v_mfma_f32_16x16x4_f32 of twice their length.  (lo and mid first.)
 template <int EPI, int BM, int BN, int KG, bool EX>
 __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kernel(const i64h_linear p, const int n_tiles, const int m_tiles, const int vecC) {
     constexpr bool DUAL = dn_dual(EPI), INN = EPI == I64H_EPI_IN_NORM;
-    constexpr int BK = EX ? 32 : 64, CH = BK / 8;      // values of a step, of a 16-byte chunk
+    constexpr int BK = 64, CH = 8, PARTS = EX ? 3 : 1;      // values of a step, of a thread's chunk; bf16 rows a staged row of A becomes
     constexpr int NWM = BM >= 64 ? 2 : 1, NWN = 4 / NWM;      // waves of a group over rows and columns
     constexpr int WM = BM / NWM, WN = BN / NWN, FM = WM / 16, FN = WN / 16;
     static_assert(FM > 0 && FN > (DUAL ? 1 : 0), "");
     constexpr int PA = (BM + 31) / 32, PB = BN / 32;       // staging passes: 32 rows of 64 values, 8 values a thread
     constexpr int COLS = DUAL ? BN / 2 : BN;               // output columns of a tile
-    constexpr int PLANE = (BM + BN) * 64;                  // (in 16-bit units)
-    // [buffer][group][A rows, W rows]; (variables of their own, so that the writes of one step may be scheduled between the reads of the other)
+    constexpr int PLANE = (PARTS * BM + BN) * 64;          // (in 16-bit units)
+    // [buffer][group][A rows (EX: hi, mid, lo), W rows]; (variables of their own, so that the writes of one step may be scheduled between the reads of the other)
     __shared__ __attribute__((aligned(16))) uint16_t s0[KG * PLANE], s1[KG * PLANE];
     __shared__ float sRow[INN ? KG : 1][INN ? BM : 1];
     const int grp = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
@@ -64,17 +65,14 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
 #pragma unroll
         for (int i = 0; i < PA; ++i) {
             ra[S][i][0] = dn_load16(bufA, oa[i] | past, k0 * 4);
-            if (!EX) ra[S][i][1] = dn_load16(bufA, (oa[i] + 16) | past, k0 * 4);
+            ra[S][i][1] = dn_load16(bufA, (oa[i] + 16) | past, k0 * 4);
         }
 #pragma unroll
-        for (int i = 0; i < PB; ++i) {
-            if (EX) rb[S][i].xy = __builtin_bit_cast(dn_v2u, __builtin_amdgcn_raw_buffer_load_b64(bufW, ow[i] | past, k0 * 2, 0));
-            else rb[S][i] = dn_load16(bufW, ow[i] | past, k0 * 2);
-        }
+        for (int i = 0; i < PB; ++i) rb[S][i] = dn_load16(bufW, ow[i] | past, k0 * 2);
         if (INN) {
             const float* nw = p.in_norm_w + (past ? 0 : k0 + lc * CH);
             rn[S][0] = *(const dn_v4u*)nw;
-            if (!EX) rn[S][1] = *(const dn_v4u*)(nw + 4);
+            rn[S][1] = *(const dn_v4u*)(nw + 4);
         }
     };
     // 128-byte rows; a row's chunks are stored exclusive-or its number, so that the 16 rows of a fragment read lie in different banks
@@ -83,26 +81,44 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
         uint16_t* sm = (S ? s1 : s0) + grp * PLANE;
 #pragma unroll
         for (int i = 0; i < PA; ++i) {
-            dn_v4f u = __builtin_bit_cast(dn_v4f, ra[S][i][0]), v = __builtin_bit_cast(dn_v4f, ra[S][i][EX ? 0 : 1]);
+            dn_v4f u = __builtin_bit_cast(dn_v4f, ra[S][i][0]), v = __builtin_bit_cast(dn_v4f, ra[S][i][1]);
             if (INN) {      // the row's squares as they come, the norm's weights on what is staged
-                const dn_v4f nu = __builtin_bit_cast(dn_v4f, rn[S][0]), nv = __builtin_bit_cast(dn_v4f, rn[S][EX ? 0 : 1]);
+                const dn_v4f nu = __builtin_bit_cast(dn_v4f, rn[S][0]), nv = __builtin_bit_cast(dn_v4f, rn[S][1]);
 #pragma unroll
                 for (int g = 0; g < 4; ++g) ssq[i] = fmaf(u[g], u[g], ssq[i]);
-                if (!EX)
 #pragma unroll
-                    for (int g = 0; g < 4; ++g) ssq[i] = fmaf(v[g], v[g], ssq[i]);
+                for (int g = 0; g < 4; ++g) ssq[i] = fmaf(v[g], v[g], ssq[i]);
 #pragma unroll
                 for (int g = 0; g < 4; ++g) u[g] *= nu[g], v[g] *= nv[g];
             }
-            const int r = i * 32 + lr;
-            const dn_v4u w = EX ? __builtin_bit_cast(dn_v4u, u) : dn_v4u{dn_bf16_pair(u[0], u[1]), dn_bf16_pair(u[2], u[3]), dn_bf16_pair(v[0], v[1]), dn_bf16_pair(v[2], v[3])};
-            if (BM >= 32 || lr < BM) *(dn_v4u*)&sm[r * 64 + ((lc ^ (r & 7)) << 3)] = w;
+            const int r = i * 32 + lr, at = r * 64 + ((lc ^ (r & 7)) << 3);
+            if constexpr (EX) {
+                dn_v4u w[PARTS];
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    uint32_t part[2][PARTS];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        const float x = g < 2 ? u[2 * g + e] : v[2 * g - 4 + e];
+                        const float hi = __uint_as_float(__float_as_uint(x) & 0xffff0000u), rest = x == hi ? 0.0f : x - hi;      // (an infinity leaves none)
+                        const float mid = __uint_as_float(__float_as_uint(rest) & 0xffff0000u);
+                        part[e][0] = __float_as_uint(hi), part[e][1] = __float_as_uint(mid), part[e][2] = __float_as_uint(rest - mid);
+                    }
+#pragma unroll
+                    for (int q = 0; q < PARTS; ++q) w[q][g] = __builtin_amdgcn_perm(part[1][q], part[0][q], 0x07060302u);      // the upper halves
+                }
+#pragma unroll
+                for (int q = 0; q < PARTS; ++q)
+                    if (BM >= 32 || lr < BM) *(dn_v4u*)&sm[q * BM * 64 + at] = w[q];
+            } else {
+                const dn_v4u w{dn_bf16_pair(u[0], u[1]), dn_bf16_pair(u[2], u[3]), dn_bf16_pair(v[0], v[1]), dn_bf16_pair(v[2], v[3])};
+                if (BM >= 32 || lr < BM) *(dn_v4u*)&sm[at] = w;
+            }
         }
 #pragma unroll
         for (int i = 0; i < PB; ++i) {
             const int r = i * 32 + lr;
-            const dn_v4u x = rb[S][i];
-            *(dn_v4u*)&sm[(BM + r) * 64 + ((lc ^ (r & 7)) << 3)] = EX ? dn_v4u{x[0] << 16, x[0] & 0xffff0000u, x[1] << 16, x[1] & 0xffff0000u} : x;
+            *(dn_v4u*)&sm[(PARTS * BM + r) * 64 + ((lc ^ (r & 7)) << 3)] = rb[S][i];
         }
     };
     dn_v4f acc[FM][FN];
@@ -117,23 +133,20 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
             const int ch = ((kk * 4 + fk) ^ (fr & 7)) << 3;
-            dn_v4u a[FM], w[FN];
+            dn_v4u a[PARTS][FM], w[FN];
 #pragma unroll
-            for (int i = 0; i < FM; ++i) a[i] = *(const dn_v4u*)&sm[(wm * WM + i * 16 + fr) * 64 + ch];
+            for (int q = 0; q < PARTS; ++q)
 #pragma unroll
-            for (int j = 0; j < FN; ++j) w[j] = *(const dn_v4u*)&sm[(BM + wn * WN + j * 16 + fr) * 64 + ch];
+                for (int i = 0; i < FM; ++i) a[q][i] = *(const dn_v4u*)&sm[(q * BM + wm * WM + i * 16 + fr) * 64 + ch];
 #pragma unroll
-            for (int i = 0; i < FM; ++i)
+            for (int j = 0; j < FN; ++j) w[j] = *(const dn_v4u*)&sm[(PARTS * BM + wn * WN + j * 16 + fr) * 64 + ch];
 #pragma unroll
-                for (int j = 0; j < FN; ++j) {
-                    if constexpr (EX) {      // (a lane's four neighbouring k go to four products: the same permutation on both sides)
-                        const dn_v4f wf = __builtin_bit_cast(dn_v4f, w[j]), af = __builtin_bit_cast(dn_v4f, a[i]);
+            for (int q = PARTS - 1; q >= 0; --q)
 #pragma unroll
-                        for (int g = 0; g < 4; ++g) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[g], af[g], acc[i][j], 0, 0, 0);
-                    } else {
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_v8bf, w[j]), __builtin_bit_cast(dn_v8bf, a[i]), acc[i][j], 0, 0, 0);
-                    }
-                }
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_v8bf, w[j]), __builtin_bit_cast(dn_v8bf, a[q][i]), acc[i][j], 0, 0, 0);
         }
     };
     // the next tile's writes and the loads behind it between the matrix instructions; small tiles are faster as the compiler orders them
@@ -205,6 +218,28 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
         }
     }
     // the weights are the left operand: a lane holds four neighbouring columns of a row
+    if constexpr (EX) {      // an infinite weight makes no number of a part that is zero: such sums are taken again term by term
+        auto again = [&](float v, int64_t rl, int c) {
+            if (v == v) return v;
+            const float* x = p.A + b * p.a_batch + (p.a_rows ? (int64_t)p.a_rows[m0 + rl] : m0 + rl) * p.lda;
+            const uint16_t* w = (const uint16_t*)p.W + b * p.w_batch + (int64_t)c * K;
+            v = 0.0f;
+            for (int k = 0; k < K; ++k) v = fmaf(INN ? x[k] * p.in_norm_w[k] : x[k], dn_bf16_to_f32(w[k]), v);
+            return v;
+        };
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            const int rl = wm * WM + i * 16 + fr;
+            if (rl >= M) continue;
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                const int c = n0 + wn * (COLS / NWN) + (DUAL ? j % (FN / 2) : j) * 16 + fk * 4;
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    if (c + g < N) acc[i][j][g] = again(acc[i][j][g], rl, c + g + (DUAL && j >= FN / 2 ? N : 0));
+            }
+        }
+    }
     float* C = p.C + b * p.c_batch;
     // (a bias and factors of rows are asked for once, not at every value)
     i64h_linear q = p;
@@ -295,35 +330,41 @@ bool dn_linear_block(const i64h_linear& d, int form, hipStream_t s) {
     const int64_t tall = d.group_off && d.rows_total > 0 ? (d.rows_total + d.batch - 1) / d.batch : d.M;
     // Short k and many tiles: two steps of registers and LDS on their way are little use, and the plainer kernel's smaller workgroups overlap their loads and
     // stores better.  Microseconds, here | there: 12000 x 4096 x 64 62 | 35, x 128 80 | 48, 4096 x 1024 x 128 11.1 | 9.7, 1000 x 4096 x 64 10.0 | 7.8, 320 x 4096 x 128 6.6 | 6.4, 1000 x
-    // 1024 x 128 5.2 | 5.7 (a gate / up pair: 2048 x 4096 x 128 25.3 | 23.3, 1000 x 4096 15.2 | 13.5, 1000 x 1024 6.2 | 8.4); 32-bit products 4096 x 1024 x 64 12.9 | 11.4,
-    // x 32 10.2 | 8.6, 512 x 1024 x 32 5.7 | 4.9.
-    auto short_k = [&](int64_t many, int k) { return (d.K <= 32 && !dual) || (d.K <= k && tiles(d, 64, 64) >= many); };
+    // 1024 x 128 5.2 | 5.7 (a gate / up pair: 2048 x 4096 x 128 25.3 | 23.3, 1000 x 4096 15.2 | 13.5, 1000 x 1024 6.2 | 8.4).
+    auto short_k = [&](int64_t many) { return (d.K <= 32 && !dual) || (d.K <= 128 && tiles(d, 64, 64) >= many); };
     if (d.exact) {
-        // Bound by the matrix instructions, a sixteenth of the bf16 rate: what counts is that every CU works, then that few values are staged per
-        // product.  Microseconds in replayed graphs, in front the 64 x 64 tile kernel with 32-wide steps:
-        //   rows x columns x k                 before   64x64  64x64/2  32x64  32x64/4  16x64/4  16x128/2 (a gate / up pair)
-        //   4096 x 1024 x 1024                    83      69       71     74       98       96
-        //    376 x 5760 x 1024                    66      54       54     49       62       56
-        //    376 x 1024 x 2752                    99      58       49     40       30       33
-        //     40 x 1024 x 1024                    35      23       20     16       14       10
-        //      3 x 32000 x 1024                   54      39       36     25       26       16
-        //    376 x 2752 x 1024, pair              91      54       55                                  59
-        //  8 x 10 x 896 x 1024, pair              66      26       22                                  17
+        // A third of the bf16 rate, and the parts are made while rows are staged (eight instructions a value), so a row is better staged for many columns; small launches are bound as those
+        // of bf16 are.  Microseconds in replayed graphs, in front v_mfma_f32_16x16x4_f32 in the form that was best for it:
+        //   rows x columns x k                 before   64x128  32x128/2  32x64  32x64/2  16x64/4  16x128/2 (a gate / up pair)
+        //   4096 x 5760 x 1024                   368      172      250      211      234      531
+        //    900 x 5760 x 1024                             49       66       55       58      123
+        //    376 x 5760 x 1024                    53       33       36       29       29       55
+        //   12000 x 4096 x 64                     92       84      197       64
+        //    150 x 5760 x 1024                             23       13       15       14       26
+        //    600 x 1024 x 2752                    50       48       26       31       28       34
+        //    376 x 1024 x 1024                    14       22       12       11        9       13
+        //     40 x 1024 x 1024                     9       21       12       11        9        7
+        //      3 x 32000 x 1024                   16       20       14       14       14       17
+        //   2000 x 2752 x 1024, pair             178       85      114                                 173
+        //    376 x 2752 x 1024, pair              55       30       33                                  42
+        //    100 x 2752 x 1024, pair              22       21       12                                  18
+        //  8 x 25 x 896 x 1024, pair              26       22       13                                  11
+        // Errors against 64 bits are 0.55 to 0.8 of what they were (376 x 5760 x 1024: 3.4e-7 of the result, 5.7e-7 before): fewer roundings of a sum.
         if (form < 0) {
-            if (!dual && short_k(1000, 64)) return false;
-            if (dual) form = tiles(d, 16, 128) <= 256 ? 6 : (d.K >= 512 && tiles(d, 64, 64) <= 256 ? 3 : 2);
-            else if (tall <= 16 || tiles(d, 16, 64) <= 256) form = 5;
-            else if (tiles(d, 32, 64) <= 256) form = 4;
-            else if (d.K >= 512 && tiles(d, 64, 64) <= 256) form = 3;
-            else form = tiles(d, 32, 64) < 1500 ? 1 : 2;
+            if (d.K < 64 && !dual) return false;      // (less than a step: 4096 x 1024 x 32 9.3, there 8.2; 512 rows 3.7 and 4.2)
+            if (dual) form = tiles(d, 16, 128) <= (tall <= 32 ? 512 : 256) ? 6 : (tiles(d, 32, 128) <= 256 ? 7 : 2);
+            else if (tiles(d, 16, 64) <= 256) form = 5;
+            else if (tall <= 16 || tiles(d, 32, 64) <= 256) form = 4;
+            else if (d.K >= 512 && tiles(d, 32, 128) <= 256) form = 7;
+            else form = d.K < 512 || tiles(d, 64, 128) < 384 ? 1 : 2;
         }
         switch (form) {
             case 1: if (!dual) { launch<32, 64, 1, PLAIN, true>(d, s); break; } [[fallthrough]];
-            case 3: launch<64, 64, 2, PLAIN | PAIR, true>(d, s); break;
-            case 4: if (!dual) { launch<32, 64, 4, PLAIN, true>(d, s); break; } [[fallthrough]];
+            case 4: if (!dual) { launch<32, 64, 2, PLAIN, true>(d, s); break; } [[fallthrough]];
             case 5: if (!dual) { launch<16, 64, 4, PLAIN, true>(d, s); break; } [[fallthrough]];
             case 6: if (dual) { launch<16, 128, 2, PAIR, true>(d, s); break; } [[fallthrough]];
-            default: launch<64, 64, 1, PLAIN | PAIR, true>(d, s); break;
+            case 7: launch<32, 128, 2, PLAIN | PAIR, true>(d, s); break;
+            default: launch<64, 128, 1, PLAIN | PAIR, true>(d, s); break;
         }
         return true;
     }
@@ -342,7 +383,7 @@ bool dn_linear_block(const i64h_linear& d, int form, hipStream_t s) {
         // Few rows under weights that take longer than everything else: 32 x 128 tiles, two groups (8 experts of 16 rows x 3584 x 2048: 24.4 us, in 128
         // x 128 tiles 33, in 64 x 64 30; 7 x 32000 x 1024 12.7, 64x64 13.4).
         const bool longer = d.K > 128, wide = (dual ? 2 * (int64_t)d.N : d.N) > 64;      // (half of a 128-column tile would be idle)
-        if (short_k(dual ? 2000 : 700, 128)) return false;
+        if (short_k(dual ? 2000 : 700)) return false;
         if (longer && wide && tall > 64 && tiles(d, 128, 128) >= 200) form = 0;
         else if (longer && wide && tall > 32 && tiles(d, 64, 128) >= 250) form = 1;
         else if (dual ? tiles(d, 16, 128) <= 256 : tiles(d, 16, 64) <= 256) form = dual ? 6 : 5;
