@@ -635,6 +635,9 @@ typedef struct {
     int64_t n;
 } i64h_rec_step_args;
 int i64h_rec_step(const i64h_rec_step_args* d, void* stream);
+/* The same for runs of rows of one sequence (s: seg_start and nseg, the read-out out [n, heads * vdim] of row stride ldo, the workspace of i64h_gdn_scan, and for the delta rule X with ldx and
+ * v_off: room for the convolved values), in tiles of 16 tokens: convolution, gates and the decays' map in the launch that prepares the tiles, the output gates' map in the one that norms.  Not exact; vdim a multiple of four, at most 4 taps. */
+int i64h_rec_tiles(const i64h_rec_step_args* d, const i64h_gdn_args* s, void* stream);
 int64_t i64h_scan_work_floats(int64_t n, int32_t nseg, int32_t heads, int32_t dim);
 /* Whether either scan (delta != 0: i64h_gdn_scan, else i64h_gla_scan with keys of its own) of nseg runs of n rows, the longest of `longest` rows, is the
  * faster in tiles, and a caller that knows its runs should give it a workspace.  The launch itself knows n and nseg only. */

@@ -77,3 +77,67 @@ def test_what_does_not_fit_is_refused():
         D.rec_step(t, q_off=0, k_off=8, v_off=8, dim=8, vdim=48, state=torch.zeros(1, 1, 48, 8, device=DEV), **kw)
     with pytest.raises(Exception, match="rec_step"):      # key channels that are no four
         D.rec_step(t, q_off=0, k_off=8, v_off=8, dim=6, vdim=4, state=torch.zeros(1, 1, 4, 6, device=DEV), **{**kw, "a": kw["a"][:6]})
+
+
+# heads, dim, vdim, ranks, taps, rows of the runs
+RUNS = [(8, 128, 128, (128, 128), 4, (150, 1, 16, 2, 33)), (3, 64, 64, (8, 136), 3, (17, 3, 160)), (2, 68, 60, (264, 8), 2, (31, 1, 1, 48)), (1, 4, 4, (8, 40), 4, (1, 2, 3, 4, 5)),
+        (5, 36, 128, (40, 128), 4, (145, 15))]
+
+
+@pytest.mark.parametrize("delta", [True, False])
+@pytest.mark.parametrize("H,d,dv,ranks,taps,runs", RUNS)
+def test_tiles_from_the_projections(H, d, dv, ranks, taps, runs, delta):
+    """The same in tiles of 16 tokens, runs that start afresh, inside the first taps, or far behind: against the separate launches, their scan in tiles too."""
+    from vllm_i64_amd import _lib
+    g = torch.Generator(device=DEV).manual_seed(H * d + dv + len(runs))
+    r = lambda *s, std=1.0: torch.randn(*s, generator=g, device=DEV) * std
+    pad4 = lambda x: (x + 3) // 4 * 4
+    n, nseg, nd, rv = sum(runs), len(runs), H * d, H * dv
+    slots, C = nseg + 2, 2 * nd + rv
+    a_off = pad4(C)
+    z_off = a_off + pad4(ranks[0])
+    b_off = z_off + max(pad4(ranks[1]), pad4(rv))
+    P = r(n, pad4(b_off + H))
+    a, bias, rate = r(nd, ranks[0], std=ranks[0] ** -0.5).bfloat16(), r(nd), torch.rand(nd, generator=g, device=DEV) + 0.1
+    z, norm_w, eps = r(rv, ranks[1], std=ranks[1] ** -0.5).bfloat16(), r(dv), 1e-6
+    conv_w, conv, state = r(C, taps, std=0.5), r(slots, taps - 1, C), r(slots, H, dv, d, std=0.3)
+    own = torch.randperm(slots, generator=g, device=DEV)[:nseg]
+    pos = torch.cat([torch.arange(m, device=DEV) + (0, 1, 2, 3, 700)[i % 5] for i, m in enumerate(runs)]).to(torch.int32)
+    slot = torch.cat([own[i].repeat(m) for i, m in enumerate(runs)]).to(torch.int32)
+    seg = torch.tensor([0, *torch.tensor(runs).cumsum(0).tolist()], dtype=torch.int32, device=DEV)
+    s1, s2, c1, c2 = state.clone(), state.clone(), conv.clone(), conv.clone()
+    work = torch.full((D.scan_work_floats(n, nseg, H, d),), float("nan"), device=DEV)
+    F, R, want, got, got16, X2, R2 = (torch.full((n, w), float("nan"), device=DEV) for w in (nd, rv, rv, rv, rv, rv, rv))
+    got16 = got16.bfloat16()
+    D.linear(P, a, F, m=n, a_off=a_off, bias=bias, epilogue=D.EPI_DECAY, e=rate)
+    scan = dict(seg_start=seg, nseg=nseg, positions=pos, slot_ids=slot)
+    try:
+        _lib.call_dense("i64h_set_gdn_scan_form", 5)
+        if delta:
+            X, G, Z = torch.empty(n, C, device=DEV), torch.empty(n, 2 * H, device=DEV), torch.empty(n, rv, device=DEV)
+            D.causal_conv(P, off=0, channels=C, w=conv_w, bias=None, positions=pos, slot_ids=slot, state=c1, out=X, n=n, seg_start=seg, nseg=nseg)
+            cols = dict(q_off=0, k_off=nd, v_off=2 * nd, heads=H, kv_heads=H, dim=d, vdim=dv, n=n)
+            D.gdn_gates(X, G, P, b_off=b_off, a_off=-1, a_log=None, dt_bias=None, unit_eps=1e-6, q_scale=d ** -0.5, **cols)
+            D.linear(P, z, Z, m=n, a_off=z_off)
+            D.gdn_scan(X, G, f=F, state=s1, out=R, work=work, **scan, **cols)
+            D.gate_norm(R, norm_w, want, groups=H, eps=eps, z=Z, ldz=rv, n=n, gate_after=True, width=rv, sigmoid=True)
+            kw = dict(q_off=0, conv_w=conv_w, conv=c2, b_off=b_off, unit_eps=1e-6, z=z, z_off=z_off, sigmoid=True, x=X2)
+        else:
+            D.gla_scan(P, f=F, q_off=0, k_off=nd, f_off=0, v_off=2 * nd, heads=H, dim=d, vdim=dv, state=s1, out=R, n=n, q_scale=d ** -0.5, work=work, **scan)
+            D.gate_norm(R, norm_w, want, groups=H, eps=eps, z=P, z_off=z_off, ldz=P.shape[-1], n=n, gate_after=True, width=rv)
+            kw = dict(q_off=0, k_off=nd, v_off=2 * nd, z_off=z_off)
+    finally:
+        _lib.call_dense("i64h_set_gdn_scan_form", 0)
+    work.fill_(float("nan"))
+    D.rec_tiles(P, heads=H, dim=d, vdim=dv, a=a, a_off=a_off, a_bias=bias, a_rate=rate, norm_w=norm_w, eps=eps, state=s2, n=n, out=got, out16=got16, q_scale=d ** -0.5, work=work, r=R2,
+                **scan, **kw)
+    _close(s2, s1, "state")
+    _close(R2, R, "read-out")
+    # (a head's row is divided by its root mean square: small read-outs carry the largest one's roundings, hence row by row)
+    e = (got.double() - want.double()).view(n, H, dv).abs().amax(-1) / want.double().view(n, H, dv).abs().amax(-1).clamp(min=1e-20)
+    big = R.view(n, H, dv).abs().amax(-1)
+    assert (e * (big / big.max()).double() <= 2e-5).all()
+    assert torch.equal(got16, got.bfloat16()) and torch.equal(c1, c2)
+    idle = torch.ones(slots, dtype=torch.bool, device=DEV)
+    idle[own] = False
+    assert torch.equal(s2[idle], state[idle])

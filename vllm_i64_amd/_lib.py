@@ -239,6 +239,7 @@ DENSE_SIGNATURES: Dict[str, str] = {
     "i64h_gdn_gates": "pp",
     "i64h_gdn_scan": "pp",
     "i64h_rec_step": "pp",
+    "i64h_rec_tiles": "ppp",
     "i64h_set_gdn_scan_form": "i",
     "i64h_set_residual_form": "i",
     "i64h_gla_gates": "pp",

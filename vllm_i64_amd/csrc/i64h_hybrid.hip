@@ -1077,6 +1077,14 @@ __global__ __launch_bounds__(256) void rot_post_kernel(const i64h_rot_post_args 
 // 512 rows 18.7 | 16.7 and 10.2 | 11.4.
 #define HY_WIDE_ROWS 256
 
+// the launch that stores the carried inputs, behind whoever read them (also i64h_scan_step.hip's)
+int i64h_conv_carry(const i64h_causal_conv_args& d, void* stream) {
+    const dim3 carry((unsigned)((d.channels + 255) / 256), d.seg_start ? (unsigned)d.nseg : (unsigned)d.n);
+    hipLaunchKernelGGL(conv_carry_kernel, carry, dim3(256), 0, (hipStream_t)stream, d);
+    I64H_CHECK_LAUNCH();
+    return 0;
+}
+
 extern "C" {
 
 int i64h_embed_bigram(const i64h_embed_bigram_args* dp, void* stream) {
@@ -1191,12 +1199,7 @@ int i64h_causal_conv(const i64h_causal_conv_args* dp, void* stream) {
         default: hipLaunchKernelGGL(causal_conv_kernel, grid, dim3(256), 0, s, d); break;
     }
     I64H_CHECK_LAUNCH();
-    if (d.taps > 1 && !d.single_rows) {
-        const dim3 carry(grid.x, d.seg_start ? (unsigned)d.nseg : grid.y);
-        hipLaunchKernelGGL(conv_carry_kernel, carry, dim3(256), 0, (hipStream_t)stream, d);
-        I64H_CHECK_LAUNCH();
-    }
-    return 0;
+    return d.taps > 1 && !d.single_rows ? i64h_conv_carry(d, stream) : 0;
 }
 
 int i64h_ssm_scan(const i64h_ssm_scan_args* dp, void* stream) {

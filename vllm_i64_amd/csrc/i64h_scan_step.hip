@@ -7,6 +7,9 @@
 #include "i64h_dense_dev.h"
 #include "i64h_scan_dev.h"
 
+int i64h_conv_carry(const i64h_causal_conv_args& d, void* stream);      // i64h_hybrid.hip
+int i64h_scan_tiles_raw(const i64h_gdn_args& d, const i64h_rec_step_args& raw, bool delta, void* stream);      // i64h_scan_tile.hip
+
 // 512 threads: the 16 lanes of a DPP row share CPT value columns and hold KPT key channels of each in registers; a workgroup has 32 such rows.
 // DELTA: the delta rule behind a convolution; else linear attention with keys of its own, its gates columns of P.
 template <int KPT, int CPT, bool DELTA>
@@ -167,21 +170,81 @@ __global__ __launch_bounds__(512) void rec_step_kernel(const i64h_rec_step_args 
     if (p.out16) ((uint16_t*)p.out16)[t * p.ldo + a * V + c] = (uint16_t)dn_bf16_rne(y);
 }
 
+// Norm and gate of many rows whose gate is a low-rank map: a workgroup per 16 rows of one head takes the map's products on the bf16 matrix instruction - lane (c, g): row c, columns 4 g ..
+// of a block of 16, as the norm's operands lie - so that the gates never pass memory (2956 rows of 16 heads of 128: a Linear of 12 us and gate_norm_kernel's 17, 26 together).
+template <int NV>      // blocks of 16 columns a wave has at most
+__global__ __launch_bounds__(256) void gate_map_kernel(const i64h_rec_step_args p, const float* y, const int64_t ldy) {
+    __shared__ float sS[4][16];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, g = lane >> 4;
+    const int V = p.vdim, a = blockIdx.x % p.heads;
+    const int64_t t = (int64_t)(blockIdx.x / p.heads) * 16 + c;
+    const bool ok = t < p.n;
+    const float* row = p.P + (ok ? t : p.n - 1) * p.ldp + p.z_off;
+    dn_v4f v[NV], acc[NV];
+    float ss = 0.0f;
+#pragma unroll
+    for (int b = 0; b < NV; ++b) {
+        const int col = 16 * (w + 4 * b) + 4 * g;
+        v[b] = acc[b] = dn_v4f{0, 0, 0, 0};
+        if (ok && col < V) v[b] = *(const dn_v4f*)(y + t * ldy + a * V + col);
+    }
+#pragma unroll 4
+    for (int k0 = 0; k0 < p.z_rank; k0 += 32) {
+        const int k = k0 + 8 * g;
+        dn_v4u x{0, 0, 0, 0};
+        if (k < p.z_rank) {
+            const dn_v4f u = *(const dn_v4f*)(row + k), q = *(const dn_v4f*)(row + k + 4);
+            x = dn_v4u{dn_bf16_pair(u[0], u[1]), dn_bf16_pair(u[2], u[3]), dn_bf16_pair(q[0], q[1]), dn_bf16_pair(q[2], q[3])};
+        }
+#pragma unroll
+        for (int b = 0; b < NV; ++b) {
+            const int col = 16 * (w + 4 * b) + c;
+            dn_v4u m{0, 0, 0, 0};
+            if (k < p.z_rank && col < V) m = *(const dn_v4u*)((const uint16_t*)p.Z + ((int64_t)a * V + col) * p.z_rank + k);
+            acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_v8bf, m), __builtin_bit_cast(dn_v8bf, x), acc[b], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < NV; ++b) ss += (v[b][0] * v[b][0] + v[b][1] * v[b][1]) + (v[b][2] * v[b][2] + v[b][3] * v[b][3]);
+    ss += __shfl_xor(ss, 16);
+    ss += __shfl_xor(ss, 32);
+    if (g == 0) sS[w][c] = ss;
+    __syncthreads();
+    const float den = sqrtf(((sS[0][c] + sS[1][c]) + (sS[2][c] + sS[3][c])) / (float)V + p.eps);
+#pragma unroll
+    for (int b = 0; b < NV; ++b) {
+        const int col = 16 * (w + 4 * b) + 4 * g;
+        if (!ok || col >= V) continue;
+        const dn_v4f nw = *(const dn_v4f*)(p.norm_w + col);
+        dn_v4f o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = v[b][i] / den * nw[i] * (p.gate_act ? dn_sigmoid(acc[b][i]) : acc[b][i] / (1.0f + expf(-acc[b][i])));
+        if (p.out) *(dn_v4f*)(p.out + t * p.ldo + a * V + col) = o;
+        if (p.out16) *(dn_v2u*)((uint16_t*)p.out16 + t * p.ldo + a * V + col) = dn_v2u{dn_bf16_pair(o[0], o[1]), dn_bf16_pair(o[2], o[3])};
+    }
+}
+
 extern "C" {
+
+static int rec_check(const i64h_rec_step_args& d, const char* what) {
+    const bool delta = d.conv_w != nullptr;
+    I64H_CHECK_ARG(d.heads > 0 && d.dim > 0 && d.dim <= 128 && d.dim % 4 == 0 && d.vdim > 0 && d.vdim <= 128 && d.n >= 0,
+                   "%s: heads %d, dim %d, vdim %d (dims to 128, key channels in fours)", what, d.heads, d.dim, d.vdim);
+    I64H_CHECK_ARG(d.P && d.positions && d.slot_ids && d.state && d.A && d.a_bias && d.a_rate && d.norm_w && (d.out || d.out16), "%s: null operand", what);
+    I64H_CHECK_ARG(d.q_off >= 0 && d.a_off >= 0 && d.z_off >= 0 && (delta ? d.b_off >= 0 : d.k_off >= 0 && d.v_off >= 0), "%s: negative column", what);
+    I64H_CHECK_ARG(!delta || (d.conv && d.Z && d.taps >= 2 && d.taps <= 8 && d.z_rank > 0), "%s: the delta rule takes a convolution of 2 to 8 taps (%d) and a low-rank gate", what, d.taps);
+    I64H_CHECK_ARG(d.a_rank > 0 && d.a_rank % 8 == 0 && (!delta || d.z_rank % 8 == 0), "%s: ranks %d and %d, multiples of eight", what, d.a_rank, d.z_rank);
+    I64H_CHECK_ARG((((uintptr_t)d.P | (uintptr_t)d.A | (uintptr_t)d.Z | (uintptr_t)d.state) & 15) == 0 && d.ldp % 4 == 0 && d.a_off % 4 == 0 &&
+                   (delta ? d.z_off % 4 == 0 : d.q_off % 4 == 0 && d.k_off % 4 == 0), "%s: rows and states are read 16 bytes at a time", what);
+    I64H_CHECK_ARG(d.n * d.heads < (1ll << 31), "%s: %lld rows of %d heads", what, (long long)d.n, d.heads);
+    return 0;
+}
 
 int i64h_rec_step(const i64h_rec_step_args* dp, void* stream) {
     I64H_CHECK_ARG(dp != nullptr, "rec_step: no descriptor");
     const i64h_rec_step_args& d = *dp;
     const bool delta = d.conv_w != nullptr;
-    I64H_CHECK_ARG(d.heads > 0 && d.dim > 0 && d.dim <= 128 && d.dim % 4 == 0 && d.vdim > 0 && d.vdim <= 128 && d.n >= 0,
-                   "rec_step: heads %d, dim %d, vdim %d (dims to 128, key channels in fours)", d.heads, d.dim, d.vdim);
-    I64H_CHECK_ARG(d.P && d.positions && d.slot_ids && d.state && d.A && d.a_bias && d.a_rate && d.norm_w && (d.out || d.out16), "rec_step: null operand");
-    I64H_CHECK_ARG(d.q_off >= 0 && d.a_off >= 0 && d.z_off >= 0 && (delta ? d.b_off >= 0 : d.k_off >= 0 && d.v_off >= 0), "rec_step: negative column");
-    I64H_CHECK_ARG(!delta || (d.conv && d.Z && d.taps >= 2 && d.taps <= 8 && d.z_rank > 0), "rec_step: the delta rule takes a convolution of 2 to 8 taps (%d) and a low-rank gate", d.taps);
-    I64H_CHECK_ARG(d.a_rank > 0 && d.a_rank % 8 == 0 && (!delta || d.z_rank % 8 == 0), "rec_step: ranks %d and %d, multiples of eight", d.a_rank, d.z_rank);
-    I64H_CHECK_ARG((((uintptr_t)d.P | (uintptr_t)d.A | (uintptr_t)d.Z | (uintptr_t)d.state) & 15) == 0 && d.ldp % 4 == 0 && d.a_off % 4 == 0 &&
-                   (delta ? d.z_off % 4 == 0 : d.q_off % 4 == 0 && d.k_off % 4 == 0), "rec_step: rows and states are read 16 bytes at a time");
-    I64H_CHECK_ARG(d.n * d.heads < (1ll << 31), "rec_step: %lld rows of %d heads", (long long)d.n, d.heads);
+    if (rec_check(d, "rec_step")) return 1;
     if (d.n == 0) return 0;
     auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, dim3((unsigned)(d.n * d.heads)), dim3(512), 0, (hipStream_t)stream, d); };
 #define REC_PICK(K, C)                                  \
@@ -193,6 +256,38 @@ int i64h_rec_step(const i64h_rec_step_args* dp, void* stream) {
         if (d.vdim <= 64) { REC_PICK(8, 2) } else { REC_PICK(8, 4) }
     }
 #undef REC_PICK
+    I64H_CHECK_LAUNCH();
+    return 0;
+}
+
+int i64h_rec_tiles(const i64h_rec_step_args* dp, const i64h_gdn_args* sp, void* stream) {
+    I64H_CHECK_ARG(dp != nullptr && sp != nullptr, "rec_tiles: no descriptor");
+    const i64h_rec_step_args& d = *dp;
+    const bool delta = d.conv_w != nullptr;
+    if (rec_check(d, "rec_tiles")) return 1;
+    I64H_CHECK_ARG(!d.exact && d.dim % 4 == 0 && d.vdim % 4 == 0 && (!delta || d.taps <= 4), "rec_tiles: products of bf16 values, columns in fours, at most 4 taps");
+    i64h_gdn_args a = *sp;
+    I64H_CHECK_ARG(a.seg_start && a.nseg > 0 && a.nseg <= 65535 && a.out && a.ldo >= (int64_t)d.heads * d.vdim && (!delta || a.X) && a.work && a.work_floats >= i64h_scan_work_floats(d.n, a.nseg, d.heads, d.dim),
+                   "rec_tiles: runs, a workspace and rows for the read-out");
+    I64H_CHECK_ARG((((uintptr_t)a.work | (uintptr_t)a.out | (uintptr_t)d.norm_w | (uintptr_t)d.a_rate | (uintptr_t)d.a_bias | (uintptr_t)d.out | (uintptr_t)d.out16) & 15) == 0 && a.ldo % 4 == 0 && d.ldo % 4 == 0 &&
+                   d.ldp < (1 << 25) && a.ldx < (1 << 25) && (d.n / 16 + a.nseg) * (int64_t)d.heads < (1ll << 31), "rec_tiles: rows are read 16 bytes at a time");
+    if (d.n == 0) return 0;
+    a.heads = a.kv_heads = d.heads, a.dim = d.dim, a.vdim = d.vdim, a.positions = d.positions, a.slot_ids = d.slot_ids, a.state = d.state, a.n = d.n, a.q_scale = d.q_scale;
+    if (!delta) a.X = const_cast<float*>(d.P), a.ldx = d.ldp, a.v_off = d.v_off;
+    if (i64h_scan_tiles_raw(a, d, delta, stream)) return 1;
+    if (!delta) {      // (the gates are columns)
+        i64h_gate_norm_args g = {};
+        g.y = a.out, g.ldy = a.ldo, g.z = d.P + d.z_off, g.ldz = d.ldp, g.w = d.norm_w, g.width = d.heads * d.vdim, g.groups = d.heads, g.eps = d.eps, g.out = d.out, g.out16 = d.out16, g.ldo = d.ldo;
+        g.n = d.n, g.gate_after = 1, g.w_len = d.vdim, g.gate_act = d.gate_act;
+        return i64h_gate_norm(&g, stream);
+    }
+    i64h_causal_conv_args c = {};
+    c.P = d.P, c.ldp = d.ldp, c.off = d.q_off, c.channels = d.heads * (2 * d.dim + d.vdim), c.taps = d.taps, c.positions = d.positions, c.slot_ids = d.slot_ids, c.state = d.conv, c.n = d.n;
+    c.seg_start = a.seg_start, c.nseg = a.nseg;
+    if (i64h_conv_carry(c, stream)) return 1;
+    const dim3 grid((unsigned)((d.n + 15) / 16 * d.heads));
+    if (d.vdim <= 64) hipLaunchKernelGGL(gate_map_kernel<1>, grid, dim3(256), 0, (hipStream_t)stream, d, (const float*)a.out, a.ldo);
+    else hipLaunchKernelGGL(gate_map_kernel<2>, grid, dim3(256), 0, (hipStream_t)stream, d, (const float*)a.out, a.ldo);
     I64H_CHECK_LAUNCH();
     return 0;
 }

@@ -3,14 +3,14 @@
 //   scan_pairs_kernel : per tile and head k P, q P and k P_16 / P as the operands' registers hold them, and what tokens of a tile are to each other: A_ts = sum_c k_t k_s P_t / P_s (s < t) and B_ts with q_t in
 //                       k_t's place (s <= t), the quotients as running products of the decays between (nothing is divided: decays may underflow);
 //                       delta rule: T = (1 + diag(beta) A)^-1 diag(beta) by forward substitution
+//                       (RAW: from the projections, with what else stands between them and the recurrence)
 //   scan_tile_kernel  : U = T (V - (k P)^T S)  (linear attention: U = V);   O = (q P)^T S + B U;   S <- P_16 S + (k P_16 / P)^T U
 // Every product's result already lies in the registers as the next product's operand (which of a product's terms an instruction sums is free), so
 // a tile is a chain of matrix instructions; four waves share the key channels and meet once a tile, in LDS.
 // All arithmetic fp32.  A row that holds no finite number reaches no token before it, as in the scans token by token.
 #include <type_traits>
 
-#include "i64h_common.h"
-#include "i64h_dense.h"
+#include "i64h_dense_dev.h"
 
 typedef float stf4 __attribute__((ext_vector_type(4)));
 enum { ST_TOK = 16, ST_PAIR = ST_TOK * ST_TOK };
@@ -21,10 +21,125 @@ __device__ __forceinline__ int64_t st_slot(int64_t r0, int seg) { return (r0 >> 
 // what one tile of a head leaves for the scan, in floats: three operands, P_16, B and (delta rule) T
 __host__ __device__ constexpr int st_floats(int NP) { return 3 * ST_TOK * NP + NP + 2 * ST_PAIR; }
 
-// One workgroup per (slot, head), 154 MB through memory for 3008 rows and 16 heads of 128 (38 us): 16 lanes walk from a token s to the tile's end, k_s times the decays so far in their registers; then a thread per
-// channel takes the products from the tile's start and from its end.
+// What stands in front of the pairs, for a tile of one head that is read from the projections as they are (i64h_rec_step's operands; RAW): the convolutions of q, k and v, unit
+// vectors, write strengths, and the decays' low-rank map on the bf16 matrix instruction, into sQ, sK, sF, sBeta; v goes to the values' columns of X.  (Every 16 rows of a convolution read three
+// more; carried inputs are read only here, and stored by a launch behind.)
 template <int NP, bool DELTA>
-__global__ __launch_bounds__(256) void scan_pairs_kernel(const i64h_gdn_args p) {
+__device__ __forceinline__ void st_raw(const i64h_gdn_args& p, const i64h_rec_step_args& r, int a, int64_t r0, int64_t r1, int64_t t0, float (*sQ)[NP + 4], float (*sK)[NP + 4], float (*sF)[NP + 4],
+                                       float* sBeta) {
+    static_assert(NP <= 128, "a thread per channel of q and k, two per channel of v");
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, N = p.dim, V = p.vdim, H = p.heads;
+    const int cnt = (int)min((int64_t)ST_TOK, r1 - t0);
+    const float* rows = r.P + t0 * r.ldp;
+    // the convolutions' inputs are asked for first: COUNT tokens of a channel from token `from` of the tile on, behind the three before them (before the run: carried)
+    constexpr int HALF = ST_TOK / 2;
+    float in[DELTA ? ST_TOK + 3 : 1], inv[DELTA ? HALF + 3 : 1], wt[4], wv[4];
+    const int part = tid / NP, qc = tid % NP, ch = (part * H + a) * N + qc, vc = tid % V, vfrom = tid / V * HALF, vch = 2 * H * N + a * V + vc, T = DELTA ? r.taps : 0;
+    const bool qk = part < 2 && qc < N, val = tid < 2 * V;
+    if constexpr (DELTA) {
+        const int C = H * (2 * N + V), pos = p.positions[t0];
+        const float* st = r.conv + (int64_t)p.slot_ids[r0] * (T - 1) * C;
+        auto load = [&](int c, int from, int count, float* x, float* wx) {
+#pragma unroll
+            for (int j = 0; j < count + 3; ++j) {
+                const int i = from + j - 3;
+                x[j] = 0.0f;
+                if (t0 + i >= r0) {
+                    if (i < cnt) x[j] = rows[(int64_t)i * r.ldp + r.q_off + c];
+                } else if (-i < T && pos + i >= 0) x[j] = st[(int64_t)(T - 1 + i) * C + c];
+            }
+#pragma unroll
+            for (int d = 0; d < 4; ++d) wx[d] = d < T ? r.conv_w[(int64_t)c * T + T - 1 - d] : 0.0f;
+        };
+        if (qk) load(ch, 0, ST_TOK, in, wt);
+        if (val) load(vch, vfrom, HALF, inv, wv);
+    }
+    // decays: a wave takes every fourth block of 16 channels; lane (c, g): token c, channels 4 g .. of a block
+    {
+        const int c = lane & 15, g = lane >> 4, tok = min(c, cnt - 1);
+        dn_v4f acc[NP / 64];
+#pragma unroll
+        for (int b = 0; b < NP / 64; ++b) acc[b] = dn_v4f{0, 0, 0, 0};
+#pragma unroll 4
+        for (int k0 = 0; k0 < r.a_rank; k0 += 32) {
+            const int k = k0 + 8 * g;
+            dn_v4u x{0, 0, 0, 0};
+            if (k < r.a_rank) {
+                const dn_v4f u = *(const dn_v4f*)(rows + tok * r.ldp + r.a_off + k), v = *(const dn_v4f*)(rows + tok * r.ldp + r.a_off + k + 4);
+                x = dn_v4u{dn_bf16_pair(u[0], u[1]), dn_bf16_pair(u[2], u[3]), dn_bf16_pair(v[0], v[1]), dn_bf16_pair(v[2], v[3])};
+            }
+#pragma unroll
+            for (int b = 0; b < NP / 64; ++b) {
+                const int m0 = 16 * (w + 4 * b) + c;
+                dn_v4u m{0, 0, 0, 0};
+                if (k < r.a_rank && m0 < N) m = *(const dn_v4u*)((const uint16_t*)r.A + ((int64_t)a * N + m0) * r.a_rank + k);
+                acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_v8bf, m), __builtin_bit_cast(dn_v8bf, x), acc[b], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < NP / 64; ++b) {
+            const int c0 = 16 * (w + 4 * b) + 4 * g;
+            stf4 f = (stf4)1.0f;
+            if (c0 < N && c < cnt) {
+                const stf4 rate = *(const stf4*)(r.a_rate + a * N + c0), bias = *(const stf4*)(r.a_bias + a * N + c0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) f[i] = expf(-rate[i] * dn_softplus(acc[b][i] + bias[i]));
+            }
+            *(stf4*)&sF[c][c0] = f;
+        }
+    }
+    if constexpr (!DELTA) {
+        for (int e = tid; e < ST_TOK * NP / 4; e += 256) {
+            const int i = e / (NP / 4), c = e % (NP / 4) * 4;
+            const bool ok = i < cnt && c < N;
+            const float* row = rows + i * r.ldp + a * N + c;
+            *(stf4*)&sK[i][c] = ok ? *(const stf4*)(row + r.k_off) : (stf4)0.0f;
+            *(stf4*)&sQ[i][c] = ok ? *(const stf4*)(row + r.q_off) : (stf4)0.0f;
+        }
+    } else {
+        auto silu = [&](const float* x, const float* wx, int j) {      // token j of what was loaded
+            float o = 0.0f;
+#pragma unroll
+            for (int d = 3; d > 0; --d)
+                if (d < T) o += wx[d] * x[j + 3 - d];
+            o += wx[0] * x[j + 3];
+            return o / (1.0f + expf(-o));
+        };
+        if (part < 2) {
+            float (*dst)[NP + 4] = part ? sK : sQ;
+#pragma unroll
+            for (int i = 0; i < ST_TOK; ++i) dst[i][qc] = qk && i < cnt ? silu(in, wt, i) : 0.0f;
+        }
+        if (val) {
+#pragma unroll
+            for (int i = 0; i < HALF; ++i)
+                if (vfrom + i < cnt) p.X[(t0 + vfrom + i) * p.ldx + p.v_off + a * V + vc] = silu(inv, wv, i);
+        }
+        if (tid < ST_TOK) sBeta[tid] = tid < cnt ? dn_sigmoid(rows[tid * r.ldp + r.b_off + a]) : 0.0f;
+        __syncthreads();
+        const int s = tid >> 4, l = tid & 15;      // 16 lanes a token
+        auto unit = [&](float (*x)[NP + 4], float scale) {
+            stf4 v[NP / 64];
+            float ss = 0.0f;
+#pragma unroll
+            for (int i = 0; i < NP / 64; ++i) {
+                v[i] = *(const stf4*)&x[s][64 * i + 4 * l];
+                ss += (v[i][0] * v[i][0] + v[i][1] * v[i][1]) + (v[i][2] * v[i][2] + v[i][3] * v[i][3]);
+            }
+            const float f = 1.0f / sqrtf(group_sum(ss, 16) + r.unit_eps) * scale;
+#pragma unroll
+            for (int i = 0; i < NP / 64; ++i) *(stf4*)&x[s][64 * i + 4 * l] = v[i] * f;
+        };
+        unit(sQ, r.q_scale);
+        unit(sK, 1.0f);
+    }
+}
+
+// One workgroup per (slot, head), 154 MB through memory for 3008 rows and 16 heads of 128 (38 us): 16 lanes walk from a token s to the tile's end, k_s times the decays so far in their registers; then a thread per
+// channel takes the products from the tile's start and from its end.  RAW: from the projections (st_raw), 73 us where convolution, gates,
+// the decays' Linear and this took 41 + 16 + 21 + 40 (linear attention 37 for 20 + 27): nothing but the values and the operands is written and read again.
+template <int NP, bool DELTA, bool RAW>
+__global__ __launch_bounds__(256) void scan_pairs_kernel(const i64h_gdn_args p, const i64h_rec_step_args raw) {
     constexpr int KPT = NP / 16, LD = NP + 4;
     __shared__ __attribute__((aligned(16))) float sF[ST_TOK][LD], sK[ST_TOK][LD], sQ[ST_TOK][LD];
     __shared__ float sA[ST_TOK][ST_TOK + 1], sB[ST_TOK][ST_TOK + 1], sBeta[ST_TOK];
@@ -41,20 +156,23 @@ __global__ __launch_bounds__(256) void scan_pairs_kernel(const i64h_gdn_args p) 
     const int64_t r0 = p.seg_start[seg], r1 = p.seg_start[seg + 1];
     const int64_t t0 = r0 + ST_TOK * (slot - st_slot(r0, seg));
     if (t0 >= r1) return;      // (the whole workgroup)
-    const int kh = a / (p.heads / p.kv_heads);
+    if constexpr (RAW) st_raw<NP, DELTA>(p, raw, a, r0, r1, t0, sQ, sK, sF, sBeta);
+    else {
+        const int kh = a / (p.heads / p.kv_heads);
 #pragma unroll
-    for (int e = tid; e < ST_TOK * NP / 4; e += 256) {      // (tokens behind the run's end neither decay, write nor read; nor do channels behind the last)
-        const int i = e / (NP / 4), c = e % (NP / 4) * 4;
-        const int64_t t = t0 + i;
-        const bool ok = t < r1 && c < N;
-        const stf4 zero = (stf4)0.0f;
-        const float* row = p.X + t * p.ldx + kh * N + c;
-        *(stf4*)&sK[i][c] = ok ? *(const stf4*)(row + p.k_off) : zero;
-        *(stf4*)&sQ[i][c] = ok ? *(const stf4*)(row + p.q_off) : zero;
-        if (p.F) *(stf4*)&sF[i][c] = ok ? *(const stf4*)(p.F + t * p.ldf + a * N + c) : (stf4)1.0f;
-        else *(stf4*)&sF[i][c] = (stf4)(t < r1 ? p.G[t * 2 * p.heads + p.heads + a] : 1.0f);
+        for (int e = tid; e < ST_TOK * NP / 4; e += 256) {      // (tokens behind the run's end neither decay, write nor read; nor do channels behind the last)
+            const int i = e / (NP / 4), c = e % (NP / 4) * 4;
+            const int64_t t = t0 + i;
+            const bool ok = t < r1 && c < N;
+            const stf4 zero = (stf4)0.0f;
+            const float* row = p.X + t * p.ldx + kh * N + c;
+            *(stf4*)&sK[i][c] = ok ? *(const stf4*)(row + p.k_off) : zero;
+            *(stf4*)&sQ[i][c] = ok ? *(const stf4*)(row + p.q_off) : zero;
+            if (p.F) *(stf4*)&sF[i][c] = ok ? *(const stf4*)(p.F + t * p.ldf + a * N + c) : (stf4)1.0f;
+            else *(stf4*)&sF[i][c] = (stf4)(t < r1 ? p.G[t * 2 * p.heads + p.heads + a] : 1.0f);
+        }
+        if (DELTA && tid < ST_TOK) sBeta[tid] = t0 + tid < r1 ? p.G[(t0 + tid) * 2 * p.heads + a] : 0.0f;
     }
-    if (DELTA && tid < ST_TOK) sBeta[tid] = t0 + tid < r1 ? p.G[(t0 + tid) * 2 * p.heads + a] : 0.0f;
     __syncthreads();
     {
         const int s = tid >> 4, l = tid & 15;
@@ -307,21 +425,26 @@ extern "C" int64_t i64h_scan_work_floats(int64_t n, int32_t nseg, int32_t heads,
     return (n / ST_TOK + nseg) * heads * st_floats(st_padded(dim));
 }
 
-// both launches; the caller (the scans' own dispatch) has checked sizes, alignment and the workspace
-int i64h_scan_tiles(const i64h_gdn_args& d, bool delta, void* stream) {
+template <bool RAW>
+static int st_run(const i64h_gdn_args& d, const i64h_rec_step_args& raw, bool delta, void* stream) {
     const dim3 pairs((unsigned)((d.n / ST_TOK + d.nseg) * d.heads)), tiles((unsigned)(d.heads * ((d.vdim + 15) / 16)), (unsigned)d.nseg);
     auto run = [&](auto a, auto b) {
-        hipLaunchKernelGGL(a, pairs, dim3(256), 0, (hipStream_t)stream, d);
+        hipLaunchKernelGGL(a, pairs, dim3(256), 0, (hipStream_t)stream, d, raw);
         hipLaunchKernelGGL(b, tiles, dim3(256), 0, (hipStream_t)stream, d);
     };
     auto pick = [&](auto bpw) {
         constexpr int B = decltype(bpw)::value;
-        if (delta) run(scan_pairs_kernel<64 * B, true>, scan_tile_kernel<B, true>);
-        else run(scan_pairs_kernel<64 * B, false>, scan_tile_kernel<B, false>);
+        if (delta) run(scan_pairs_kernel<64 * B, true, RAW>, scan_tile_kernel<B, true>);
+        else run(scan_pairs_kernel<64 * B, false, RAW>, scan_tile_kernel<B, false>);
     };
     if (d.dim <= 64) pick(std::integral_constant<int, 1>());
     else if (d.dim <= 128) pick(std::integral_constant<int, 2>());
-    else pick(std::integral_constant<int, 4>());
+    else if constexpr (!RAW) pick(std::integral_constant<int, 4>());
     I64H_CHECK_LAUNCH();
     return 0;
 }
+
+// both launches; the caller (the scans' own dispatch) has checked sizes, alignment and the workspace
+int i64h_scan_tiles(const i64h_gdn_args& d, bool delta, void* stream) { return st_run<false>(d, {}, delta, stream); }
+// the same from the projections (the caller, i64h_rec_tiles, has checked)
+int i64h_scan_tiles_raw(const i64h_gdn_args& d, const i64h_rec_step_args& raw, bool delta, void* stream) { return st_run<true>(d, raw, delta, stream); }

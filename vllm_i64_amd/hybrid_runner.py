@@ -324,9 +324,21 @@ class HybridRunner:
     # ---- a recurrence's step where every row is a sequence of its own: one launch from the projections to the normed and gated rows ----
     # (The separate launches | one, us in graphs, delta rule and linear attention: 8 heads of 128, 1 row 18.5 | 7.0 and 10.2 | 5.1, 64 rows 34.6 | 14.7 and 23.1 | 11.3, 256 74 | 52 and 57 | 44,
     # 1024 271 | 250 and 220 | 201; 32 heads of 64, 64 rows 40 | 22 and 24 | 15, 1024 327 | 319 and 224 | 214; 2 heads of 32, 1 row 17 | 5.3 and 10 | 3.9, 1024 26 | 17 and 15 | 11: always the one.)
-    @staticmethod
-    def _steps_at_once(r) -> bool:
-        return r.dim <= D.REC_STEP_DIM and r.vdim <= D.REC_STEP_DIM and r.dim % 4 == 0
+    def _recurs(self, r, P, n: int, seg, nseg: int, work, R, X, taps: int, **own) -> bool:
+        """A recurrence from its projections (own: D.rec_step's operands), where every row is a sequence of its own or the scan goes in tiles of bf16 products; False: nothing was
+        launched."""
+        ws = work.get((r.heads, r.dim, r.vdim))
+        if r.dim > D.REC_DIM or r.vdim > D.REC_DIM or r.dim % 4:
+            return False
+        if nseg == n and taps <= D.REC_STEP_TAPS:
+            D.rec_step(P, heads=r.heads, dim=r.dim, vdim=r.vdim, n=n, exact=self.exact, **own)
+            return True
+        # (linear attention in narrow heads has nothing to save but the decays' way through memory: 32 heads of 64, runs of 700 and 300, 55.6 us in launches of its own, 57.3 here; of 128, 16
+        # heads, 2956 rows 145 and 135; the delta rule 104 and 95, 270 and 210)
+        if ws is None or self.exact or r.vdim % 4 or taps > D.REC_TILE_TAPS or (taps == 0 and r.dim <= 64):
+            return False
+        D.rec_tiles(P, seg_start=seg, nseg=nseg, work=ws, r=R, x=X, heads=r.heads, dim=r.dim, vdim=r.vdim, n=n, **own)
+        return True
 
     # ---- gated linear attention ----
     def _gated_linear(self, B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, out, scale: float = 1.0, work=NO_WORK) -> None:
@@ -336,15 +348,14 @@ class HybridRunner:
         rv = r.heads * r.vdim
         wide = self._rounded(n, rv)
         Rn, Rn16 = None if wide else B.rn[: n * rv].view(n, rv), self._as16(B.rn16, n, rv) if wide else None
-        if nseg == n and self._steps_at_once(r):
-            D.rec_step(P, q_off=d["rq_off"], k_off=d["rk_off"], v_off=d["rv_off"], heads=r.heads, dim=r.dim, vdim=r.vdim, a=d["a2"], a_off=d["a1_off"], a_bias=d["a2_b"],
-                       a_rate=d["a_rate"], z_off=d["rg_off"], norm_w=d["r_norm"], eps=self.cfg.norm_eps, positions=positions, slot_ids=slot_ids, state=kvc.state[l]["gla"], n=n,
-                       out=Rn, out16=Rn16, q_scale=r.dim ** -0.5, exact=self.exact)
+        R = B.r[: n * rv].view(n, rv)
+        if self._recurs(r, P, n, seg, nseg, work, R, None, 0, q_off=d["rq_off"], k_off=d["rk_off"], v_off=d["rv_off"], a=d["a2"], a_off=d["a1_off"], a_bias=d["a2_b"], a_rate=d["a_rate"],
+                        z_off=d["rg_off"], norm_w=d["r_norm"], eps=self.cfg.norm_eps, positions=positions, slot_ids=slot_ids, state=kvc.state[l]["gla"], out=Rn, out16=Rn16,
+                        q_scale=r.dim ** -0.5):
             self._out(Rn, d["o_right"], out, scale, Rn16)
             return
         F = B.f[: n * r.heads * r.dim].view(n, r.heads * r.dim)
         D.linear(P, d["a2"], F, m=n, a_off=d["a1_off"], exact=self.exact, bias=d["a2_b"], epilogue=D.EPI_DECAY, e=d["a_rate"])
-        R = B.r[: n * rv].view(n, rv)
         D.gla_scan(P, f=F, q_off=d["rq_off"], k_off=d["rk_off"], f_off=0, v_off=d["rv_off"], heads=r.heads, dim=r.dim, vdim=r.vdim, seg_start=seg, nseg=nseg,
                    positions=positions, slot_ids=slot_ids, state=kvc.state[l]["gla"], out=R, n=n, q_scale=r.dim ** -0.5,
                    work=work.get((r.heads, r.dim, r.vdim)))
@@ -362,10 +373,11 @@ class HybridRunner:
         channel = r.decay == "channel"
         wide = self._rounded(n, rv)
         Rn, Rn16 = None if wide else B.c[: n * rv].view(n, rv), self._as16(B.c16, n, rv) if wide else None
-        if nseg == n and channel and r.kv_heads == r.heads and "conv" in st and st["conv"].shape[-2] < D.REC_STEP_TAPS and self._steps_at_once(r):
-            D.rec_step(P, q_off=d["r_off"], heads=r.heads, dim=r.dim, vdim=r.vdim, a=d["a2"], a_off=d["a1_off"], a_bias=d["dt_bias"], a_rate=d["a_rate"], z=d["g2"], z_off=d["g1_off"],
-                       norm_w=d["r_norm"], eps=self.cfg.norm_eps, positions=positions, slot_ids=slot_ids, state=st["gdn"], n=n, out=Rn, out16=Rn16, conv_w=d["conv_w"],
-                       conv=st["conv"], b_off=d["rb_off"], unit_eps=UNIT_EPS, q_scale=r.dim ** -0.5, sigmoid=r.gate == "sigmoid", exact=ex)
+        R = B.b[: n * rv].view(n, rv)
+        if channel and r.kv_heads == r.heads and "conv" in st and \
+                self._recurs(r, P, n, seg, nseg, work, R, B.a[: n * rv], r.conv, q_off=d["r_off"], a=d["a2"], a_off=d["a1_off"], a_bias=d["dt_bias"], a_rate=d["a_rate"], z=d["g2"],
+                             z_off=d["g1_off"], norm_w=d["r_norm"], eps=self.cfg.norm_eps, positions=positions, slot_ids=slot_ids, state=st["gdn"], out=Rn, out16=Rn16, conv_w=d["conv_w"],
+                             conv=st["conv"], b_off=d["rb_off"], unit_eps=UNIT_EPS, q_scale=r.dim ** -0.5, sigmoid=r.gate == "sigmoid"):
             D.linear(Rn, d["o_right"], out, a16=Rn16, exact=ex)
             return
         X = B.a[: n * C].view(n, C)
@@ -380,7 +392,6 @@ class HybridRunner:
             F, Z, z_off, ldz = B.f[: n * r.heads * r.dim].view(n, r.heads * r.dim), B.z[: n * rv].view(n, rv), 0, rv
             D.linear(P, d["a2"], F, m=n, a_off=d["a1_off"], exact=ex, bias=d["dt_bias"], epilogue=D.EPI_DECAY, e=d["a_rate"])
             D.linear(P, d["g2"], Z, m=n, a_off=d["g1_off"], exact=ex)
-        R = B.b[: n * rv].view(n, rv)
         D.gdn_scan(X, G, f=F, seg_start=seg, nseg=nseg, positions=positions, slot_ids=slot_ids, state=st["gdn"], out=R,
                    work=work.get((r.heads, r.dim, r.vdim)), **cols)
         D.gate_norm(R, d["r_norm"], Rn, groups=r.heads, eps=self.cfg.norm_eps, z=Z, z_off=z_off, ldz=ldz, n=n, gate_after=True, width=rv, sigmoid=r.gate == "sigmoid", out16=Rn16)

@@ -660,16 +660,13 @@ def gla_scan(p: torch.Tensor, *, q_off: int, f_off: int, v_off: int, heads: int,
     return out
 
 
-REC_STEP_DIM, REC_STEP_TAPS = 128, 8      # what a recurrence's step in one launch takes at most
+REC_DIM, REC_STEP_TAPS, REC_TILE_TAPS = 128, 8, 4      # what a recurrence from its projections takes at most, a row a sequence and in tiles
 
 
-def rec_step(p: torch.Tensor, *, q_off: int, k_off: int = 0, v_off: int = 0, heads: int, dim: int, vdim: int, a: torch.Tensor, a_off: int, a_bias: torch.Tensor, a_rate: torch.Tensor,
-             z_off: int, norm_w: torch.Tensor, eps: float, positions: torch.Tensor, slot_ids: torch.Tensor, state: torch.Tensor, n: int, out: Optional[torch.Tensor] = None,
-             out16: Optional[torch.Tensor] = None, conv_w: Optional[torch.Tensor] = None, conv: Optional[torch.Tensor] = None, b_off: int = 0, unit_eps: float = 0.0,
-             q_scale: float = 1.0, z: Optional[torch.Tensor] = None, sigmoid: bool = False, exact: bool = False) -> None:
-    """See i64h_rec_step.  p fp32 [n, ldp], every row the only row of its sequence; state fp32 [slots, heads, vdim, dim]; a bf16 [heads * dim, rank], a_bias and a_rate fp32
-    [heads * dim]; norm_w fp32 [vdim]; out fp32 / out16 bf16 [n, heads * vdim].  With conv_w fp32 [channels, taps] and conv fp32 [slots, taps - 1, channels] the delta rule, its output
-    gate the map z bf16 [heads * vdim, rank]; without, linear attention and the gate's columns z_off."""
+def _rec_args(p: torch.Tensor, *, q_off: int, k_off: int = 0, v_off: int = 0, heads: int, dim: int, vdim: int, a: torch.Tensor, a_off: int, a_bias: torch.Tensor, a_rate: torch.Tensor,
+              z_off: int, norm_w: torch.Tensor, eps: float, positions: torch.Tensor, slot_ids: torch.Tensor, state: torch.Tensor, n: int, out: Optional[torch.Tensor] = None,
+              out16: Optional[torch.Tensor] = None, conv_w: Optional[torch.Tensor] = None, conv: Optional[torch.Tensor] = None, b_off: int = 0, unit_eps: float = 0.0,
+              q_scale: float = 1.0, z: Optional[torch.Tensor] = None, sigmoid: bool = False, exact: bool = False) -> "_lib.RecStep":
     _chk(p, torch.float32, "p"), _chk(state, torch.float32, "state"), _chk(positions, torch.int32, "positions"), _chk(slot_ids, torch.int32, "slot_ids")
     _chk(a, torch.bfloat16, "a"), _chk(a_bias, torch.float32, "a_bias"), _chk(a_rate, torch.float32, "a_rate"), _chk(norm_w, torch.float32, "norm_w")
     _rows_ok("rec_step", n, positions, slot_ids)
@@ -692,11 +689,32 @@ def rec_step(p: torch.Tensor, *, q_off: int, k_off: int = 0, v_off: int = 0, hea
     if tuple(state.shape[1:]) != (heads, vdim, dim) or a.shape[0] != nd or min(a_bias.numel(), a_rate.numel()) < nd or norm_w.numel() < vdim or p.numel() < n * ld or \
             any(o < 0 or o + w > ld for o, w in cols):
         raise _lib.I64HError("rec_step: shapes do not fit the sizes")
-    d = _lib.RecStep(P=ptr(p), ldp=ld, q_off=q_off, k_off=k_off, v_off=v_off, heads=heads, dim=dim, vdim=vdim, conv_w=ptr(conv_w), conv=ptr(conv), taps=taps, b_off=b_off,
-                     unit_eps=float(unit_eps), q_scale=float(q_scale), A=ptr(a), a_bias=ptr(a_bias), a_rate=ptr(a_rate), a_off=a_off, a_rank=a.shape[-1], Z=ptr(z), z_off=z_off,
-                     z_rank=z.shape[-1] if z is not None else 0, gate_act=int(bool(sigmoid)), exact=int(bool(exact)), norm_w=ptr(norm_w), eps=float(eps), positions=ptr(positions),
-                     slot_ids=ptr(slot_ids), state=ptr(state), out=ptr(out), out16=ptr(out16), ldo=rv, n=n)
+    return _lib.RecStep(P=ptr(p), ldp=ld, q_off=q_off, k_off=k_off, v_off=v_off, heads=heads, dim=dim, vdim=vdim, conv_w=ptr(conv_w), conv=ptr(conv), taps=taps, b_off=b_off,
+                        unit_eps=float(unit_eps), q_scale=float(q_scale), A=ptr(a), a_bias=ptr(a_bias), a_rate=ptr(a_rate), a_off=a_off, a_rank=a.shape[-1], Z=ptr(z), z_off=z_off,
+                        z_rank=z.shape[-1] if z is not None else 0, gate_act=int(bool(sigmoid)), exact=int(bool(exact)), norm_w=ptr(norm_w), eps=float(eps), positions=ptr(positions),
+                        slot_ids=ptr(slot_ids), state=ptr(state), out=ptr(out), out16=ptr(out16), ldo=rv, n=n)
+
+
+def rec_step(p: torch.Tensor, **kw) -> None:
+    """See i64h_rec_step.  p fp32 [n, ldp], every row the only row of its sequence; state fp32 [slots, heads, vdim, dim]; a bf16 [heads * dim, rank], a_bias and a_rate fp32
+    [heads * dim]; norm_w fp32 [vdim]; out fp32 / out16 bf16 [n, heads * vdim].  With conv_w fp32 [channels, taps] and conv fp32 [slots, taps - 1, channels] the delta rule, its output
+    gate the map z bf16 [heads * vdim, rank]; without, linear attention and the gate's columns z_off."""
+    d = _rec_args(p, **kw)      # (held by name until the call returns: the reference is an address)
     call_dense("i64h_rec_step", _ref(d), _stream())
+
+
+def rec_tiles(p: torch.Tensor, *, seg_start: torch.Tensor, nseg: int, work: torch.Tensor, r: torch.Tensor, x: Optional[torch.Tensor] = None, **kw) -> None:
+    """See i64h_rec_tiles: rec_step's arguments for rows that are runs of sequences.  work fp32 [scan_work_floats]; r fp32 [n, heads * vdim]: room for the read-out; x, with conv_w, as
+    much for the convolved values."""
+    d = _rec_args(p, **kw)
+    rows = d.n * d.heads * d.vdim
+    _chk(seg_start, torch.int32, "seg_start"), _chk(r, torch.float32, "r")
+    if x is not None:
+        _chk(x, torch.float32, "x")
+    if seg_start.numel() < nseg + 1 or r.numel() < rows or (d.conv_w and (x is None or x.numel() < rows)):
+        raise _lib.I64HError("rec_tiles: runs, read-out or values do not fit the rows")
+    s = _lib.Gdn(X=ptr(x), ldx=d.heads * d.vdim, v_off=0, seg_start=ptr(seg_start), nseg=nseg, out=ptr(r), ldo=d.heads * d.vdim, **_scan_work(work))
+    call_dense("i64h_rec_tiles", _ref(d), _ref(s), _stream())
 
 
 def _route_args(*, entries: int, top: int, scale: float, idx: torch.Tensor, wgt: torch.Tensor, n: int, correction: Optional[torch.Tensor] = None, groups: int = 1, keep: int = 1,
