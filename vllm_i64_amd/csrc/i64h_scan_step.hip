@@ -171,7 +171,7 @@ __global__ __launch_bounds__(512) void rec_step_kernel(const i64h_rec_step_args 
 }
 
 // Norm and gate of many rows whose gate is a low-rank map: a workgroup per 16 rows of one head takes the map's products on the bf16 matrix instruction - lane (c, g): row c, columns 4 g ..
-// of a block of 16, as the norm's operands lie - so that the gates never pass memory (2956 rows of 16 heads of 128: a Linear of 12 us and gate_norm_kernel's 17, 26 together).
+// of a block of 16, as the norm's operands lie - so that the gates never pass memory (2956 rows of 16 heads of 128: a Linear of 12 us and gate_norm_kernel's 17, 23 together).
 template <int NV>      // blocks of 16 columns a wave has at most
 __global__ __launch_bounds__(256) void gate_map_kernel(const i64h_rec_step_args p, const float* y, const int64_t ldy) {
     __shared__ float sS[4][16];
@@ -180,28 +180,32 @@ __global__ __launch_bounds__(256) void gate_map_kernel(const i64h_rec_step_args 
     const int64_t t = (int64_t)(blockIdx.x / p.heads) * 16 + c;
     const bool ok = t < p.n;
     const float* row = p.P + (ok ? t : p.n - 1) * p.ldp + p.z_off;
+    const uint16_t* map = (const uint16_t*)p.Z + (int64_t)a * V * p.z_rank;
     dn_v4f v[NV], acc[NV];
     float ss = 0.0f;
 #pragma unroll
     for (int b = 0; b < NV; ++b) {
-        const int col = 16 * (w + 4 * b) + 4 * g;
+        const int col = 16 * (NV * w + b) + 4 * g;
         v[b] = acc[b] = dn_v4f{0, 0, 0, 0};
         if (ok && col < V) v[b] = *(const dn_v4f*)(y + t * ldy + a * V + col);
     }
-#pragma unroll 4
-    for (int k0 = 0; k0 < p.z_rank; k0 += 32) {
-        const int k = k0 + 8 * g;
-        dn_v4u x{0, 0, 0, 0};
-        if (k < p.z_rank) {
-            const dn_v4f u = *(const dn_v4f*)(row + k), q = *(const dn_v4f*)(row + k + 4);
-            x = dn_v4u{dn_bf16_pair(u[0], u[1]), dn_bf16_pair(u[2], u[3]), dn_bf16_pair(q[0], q[1]), dn_bf16_pair(q[2], q[3])};
-        }
+    for (int k0 = 0; k0 < p.z_rank; k0 += 128) {      // (four steps' loads together, none behind a branch: past the rank the rows' values are zeros, past the last column nobody uses the sum)
+        dn_v4f u[4][2];
+        dn_v4u m[4][NV];
 #pragma unroll
-        for (int b = 0; b < NV; ++b) {
-            const int col = 16 * (w + 4 * b) + c;
-            dn_v4u m{0, 0, 0, 0};
-            if (k < p.z_rank && col < V) m = *(const dn_v4u*)((const uint16_t*)p.Z + ((int64_t)a * V + col) * p.z_rank + k);
-            acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_v8bf, m), __builtin_bit_cast(dn_v8bf, x), acc[b], 0, 0, 0);
+        for (int s = 0; s < 4; ++s) {
+            const int k = min(k0 + 32 * s + 8 * g, p.z_rank - 8);
+            u[s][0] = *(const dn_v4f*)(row + k), u[s][1] = *(const dn_v4f*)(row + k + 4);
+#pragma unroll
+            for (int b = 0; b < NV; ++b) m[s][b] = *(const dn_v4u*)(map + (int64_t)min(16 * (NV * w + b) + c, V - 1) * p.z_rank + k);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            dn_v4u x{dn_bf16_pair(u[s][0][0], u[s][0][1]), dn_bf16_pair(u[s][0][2], u[s][0][3]), dn_bf16_pair(u[s][1][0], u[s][1][1]), dn_bf16_pair(u[s][1][2], u[s][1][3])};
+            if (k0 + 32 * s + 8 * g >= p.z_rank) x = dn_v4u{0, 0, 0, 0};
+#pragma unroll
+            for (int b = 0; b < NV; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_v8bf, m[s][b]), __builtin_bit_cast(dn_v8bf, x), acc[b], 0, 0, 0);
         }
     }
 #pragma unroll
@@ -213,12 +217,12 @@ __global__ __launch_bounds__(256) void gate_map_kernel(const i64h_rec_step_args 
     const float den = sqrtf(((sS[0][c] + sS[1][c]) + (sS[2][c] + sS[3][c])) / (float)V + p.eps);
 #pragma unroll
     for (int b = 0; b < NV; ++b) {
-        const int col = 16 * (w + 4 * b) + 4 * g;
+        const int col = 16 * (NV * w + b) + 4 * g;
         if (!ok || col >= V) continue;
         const dn_v4f nw = *(const dn_v4f*)(p.norm_w + col);
         dn_v4f o;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = v[b][i] / den * nw[i] * (p.gate_act ? dn_sigmoid(acc[b][i]) : acc[b][i] / (1.0f + expf(-acc[b][i])));
+        for (int i = 0; i < 4; ++i) o[i] = v[b][i] / den * nw[i] * dn_gated(p.gate_act && acc[b][i] == acc[b][i] ? 1.0f : acc[b][i], acc[b][i]);
         if (p.out) *(dn_v4f*)(p.out + t * p.ldo + a * V + col) = o;
         if (p.out16) *(dn_v2u*)((uint16_t*)p.out16 + t * p.ldo + a * V + col) = dn_v2u{dn_bf16_pair(o[0], o[1]), dn_bf16_pair(o[2], o[3])};
     }

@@ -37,42 +37,42 @@ __device__ __forceinline__ void st_raw(const i64h_gdn_args& p, const i64h_rec_st
     const int part = tid / NP, qc = tid % NP, ch = (part * H + a) * N + qc, vc = tid % V, vfrom = tid / V * HALF, vch = 2 * H * N + a * V + vc, T = DELTA ? r.taps : 0;
     const bool qk = part < 2 && qc < N, val = tid < 2 * V;
     if constexpr (DELTA) {
-        const int C = H * (2 * N + V), pos = p.positions[t0];
+        // (no branch at a load: a run's first tile repeats its first row, then takes what is carried; rows past the end repeat the last one and nobody uses them)
+        const int C = H * (2 * N + V), pos = p.positions[t0], before = t0 == r0 ? 0 : 3;
         const float* st = r.conv + (int64_t)p.slot_ids[r0] * (T - 1) * C;
-        auto load = [&](int c, int from, int count, float* x, float* wx) {
+        auto load = [&](int c, int from, auto count, float* x, float* wx) {
+            const float* in0 = rows + r.q_off + c;
 #pragma unroll
-            for (int j = 0; j < count + 3; ++j) {
-                const int i = from + j - 3;
-                x[j] = 0.0f;
-                if (t0 + i >= r0) {
-                    if (i < cnt) x[j] = rows[(int64_t)i * r.ldp + r.q_off + c];
-                } else if (-i < T && pos + i >= 0) x[j] = st[(int64_t)(T - 1 + i) * C + c];
-            }
+            for (int j = 0; j < decltype(count)::value + 3; ++j) x[j] = in0[(int64_t)min(max(from + j - 3, -before), cnt - 1) * r.ldp];
 #pragma unroll
             for (int d = 0; d < 4; ++d) wx[d] = d < T ? r.conv_w[(int64_t)c * T + T - 1 - d] : 0.0f;
+            if (before == 0 && from == 0) {
+#pragma unroll
+                for (int j = 0; j < 3; ++j) x[j] = 3 - j < T && pos + j >= 3 ? st[(int64_t)(T + j - 4) * C + c] : 0.0f;
+            }
         };
-        if (qk) load(ch, 0, ST_TOK, in, wt);
-        if (val) load(vch, vfrom, HALF, inv, wv);
+        if (qk) load(ch, 0, std::integral_constant<int, ST_TOK>(), in, wt);
+        if (val) load(vch, vfrom, std::integral_constant<int, HALF>(), inv, wv);
     }
     // decays: a wave takes every fourth block of 16 channels; lane (c, g): token c, channels 4 g .. of a block
     {
-        const int c = lane & 15, g = lane >> 4, tok = min(c, cnt - 1);
+        const int c = lane & 15, g = lane >> 4;
+        const float* arow = rows + min(c, cnt - 1) * r.ldp + r.a_off;
+        const uint16_t* map = (const uint16_t*)r.A + (int64_t)a * N * r.a_rank;
         dn_v4f acc[NP / 64];
 #pragma unroll
         for (int b = 0; b < NP / 64; ++b) acc[b] = dn_v4f{0, 0, 0, 0};
 #pragma unroll 4
         for (int k0 = 0; k0 < r.a_rank; k0 += 32) {
-            const int k = k0 + 8 * g;
-            dn_v4u x{0, 0, 0, 0};
-            if (k < r.a_rank) {
-                const dn_v4f u = *(const dn_v4f*)(rows + tok * r.ldp + r.a_off + k), v = *(const dn_v4f*)(rows + tok * r.ldp + r.a_off + k + 4);
-                x = dn_v4u{dn_bf16_pair(u[0], u[1]), dn_bf16_pair(u[2], u[3]), dn_bf16_pair(v[0], v[1]), dn_bf16_pair(v[2], v[3])};
-            }
+            // (no branch at a load: past the rank the rows' values are zeros, past the last channel nobody uses the sum; four steps' loads asked for together take 139 registers for 79 and
+            // longer, 70 us for 58)
+            const int k = min(k0 + 8 * g, r.a_rank - 8);
+            const dn_v4f u = *(const dn_v4f*)(arow + k), v = *(const dn_v4f*)(arow + k + 4);
+            dn_v4u x{dn_bf16_pair(u[0], u[1]), dn_bf16_pair(u[2], u[3]), dn_bf16_pair(v[0], v[1]), dn_bf16_pair(v[2], v[3])};
+            if (k != k0 + 8 * g) x = dn_v4u{0, 0, 0, 0};
 #pragma unroll
             for (int b = 0; b < NP / 64; ++b) {
-                const int m0 = 16 * (w + 4 * b) + c;
-                dn_v4u m{0, 0, 0, 0};
-                if (k < r.a_rank && m0 < N) m = *(const dn_v4u*)((const uint16_t*)r.A + ((int64_t)a * N + m0) * r.a_rank + k);
+                const dn_v4u m = *(const dn_v4u*)(map + (int64_t)min(16 * (w + 4 * b) + c, N - 1) * r.a_rank + k);
                 acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_v8bf, m), __builtin_bit_cast(dn_v8bf, x), acc[b], 0, 0, 0);
             }
         }
@@ -100,20 +100,25 @@ __device__ __forceinline__ void st_raw(const i64h_gdn_args& p, const i64h_rec_st
         auto silu = [&](const float* x, const float* wx, int j) {      // token j of what was loaded
             float o = 0.0f;
 #pragma unroll
-            for (int d = 3; d > 0; --d)
-                if (d < T) o += wx[d] * x[j + 3 - d];
+            for (int d = 3; d > 0; --d) o = d < T ? o + wx[d] * x[j + 3 - d] : o;
             o += wx[0] * x[j + 3];
-            return o / (1.0f + expf(-o));
+            return dn_gated(o, o);
         };
         if (part < 2) {
             float (*dst)[NP + 4] = part ? sK : sQ;
 #pragma unroll
-            for (int i = 0; i < ST_TOK; ++i) dst[i][qc] = qk && i < cnt ? silu(in, wt, i) : 0.0f;
+            for (int i = 0; i < ST_TOK; ++i) {
+                const float o = silu(in, wt, i);
+                dst[i][qc] = qk && i < cnt ? o : 0.0f;
+            }
         }
         if (val) {
+            float* out = p.X + (t0 + vfrom) * p.ldx + p.v_off + a * V + vc;
 #pragma unroll
-            for (int i = 0; i < HALF; ++i)
-                if (vfrom + i < cnt) p.X[(t0 + vfrom + i) * p.ldx + p.v_off + a * V + vc] = silu(inv, wv, i);
+            for (int i = 0; i < HALF; ++i) {
+                const float o = silu(inv, wv, i);
+                if (vfrom + i < cnt) out[i * p.ldx] = o;
+            }
         }
         if (tid < ST_TOK) sBeta[tid] = tid < cnt ? dn_sigmoid(rows[tid * r.ldp + r.b_off + a]) : 0.0f;
         __syncthreads();
@@ -136,8 +141,8 @@ __device__ __forceinline__ void st_raw(const i64h_gdn_args& p, const i64h_rec_st
 }
 
 // One workgroup per (slot, head), 154 MB through memory for 3008 rows and 16 heads of 128 (38 us): 16 lanes walk from a token s to the tile's end, k_s times the decays so far in their registers; then a thread per
-// channel takes the products from the tile's start and from its end.  RAW: from the projections (st_raw), 73 us where convolution, gates,
-// the decays' Linear and this took 41 + 16 + 21 + 40 (linear attention 37 for 20 + 27): nothing but the values and the operands is written and read again.
+// channel takes the products from the tile's start and from its end.  RAW: from the projections (st_raw), 58 us where convolution, gates,
+// the decays' Linear and this took 41 + 16 + 21 + 40 (linear attention 34 for 20 + 27): nothing but the values and the operands is written and read again.
 template <int NP, bool DELTA, bool RAW>
 __global__ __launch_bounds__(256) void scan_pairs_kernel(const i64h_gdn_args p, const i64h_rec_step_args raw) {
     constexpr int KPT = NP / 16, LD = NP + 4;

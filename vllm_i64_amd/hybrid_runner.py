@@ -333,8 +333,8 @@ class HybridRunner:
         if nseg == n and taps <= D.REC_STEP_TAPS:
             D.rec_step(P, heads=r.heads, dim=r.dim, vdim=r.vdim, n=n, exact=self.exact, **own)
             return True
-        # (linear attention in narrow heads has nothing to save but the decays' way through memory: 32 heads of 64, runs of 700 and 300, 55.6 us in launches of its own, 57.3 here; of 128, 16
-        # heads, 2956 rows 145 and 135; the delta rule 104 and 95, 270 and 210)
+        # (linear attention in narrow heads has nothing to save but the decays' way through memory: 32 heads of 64, runs of 700 and 300, 55.6 us in launches of its own, 56.2 here; of 128, 16
+        # heads, 2956 rows 145 and 131; the delta rule 104 and 90, 270 and 191)
         if ws is None or self.exact or r.vdim % 4 or taps > D.REC_TILE_TAPS or (taps == 0 and r.dim <= 64):
             return False
         D.rec_tiles(P, seg_start=seg, nseg=nseg, work=ws, r=R, x=X, heads=r.heads, dim=r.dim, vdim=r.vdim, n=n, **own)
