@@ -14,9 +14,12 @@
 // 47-50 us whatever the prefetch depth).  So a wave loads weight rows in memory order and turns them into operand order through
 // a private LDS strip.  A branch around a load makes the compiler wait for ALL loads in flight (it can no longer count them):
 // every load here is unconditional, on clamped addresses.
+#include <type_traits>
+
 #include "i64h_common.h"
 
 typedef float lm_v4f __attribute__((ext_vector_type(4)));
+typedef uint32_t lm_v4u __attribute__((ext_vector_type(4)));
 typedef __bf16 lm_v8b __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ uint32_t lm_top(float x, float y) { return __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302u); }
@@ -59,117 +62,133 @@ __global__ __launch_bounds__(256) void lm_split_rows_frag_kernel(const float* __
     }
 }
 
+// MF: fragments of 16 rows that there are (few rows need neither the products nor the activation fragments of a 64-row tile, and the registers these leave hold more
+// weights on their way); AHEAD: steps of weights in registers, beside the one in the strip.
+// us, 32000 columns of 1024, weights from memory (131 MB: 28 at the copy rate), all rows as 64 | so: 1 to 16 rows 36.5 | 30.5, 17 to 32 rows 37 | 32.5.  (64 rows 40: their activation
+// fragments are 196 MB from L2; cut weights held for two halves of the rows, with a step more on its way, spill: 51.)
+template <int MF, int AHEAD>
 __global__ __launch_bounds__(256, 2) void lm_head_bf16x3_ks_kernel(const uint32_t* __restrict__ planes, const float* __restrict__ B, float* __restrict__ C,
                                                                    int M, int N, int K, int Kpad) {
-    __shared__ __attribute__((aligned(16))) float smem[4 * 64 * 64];  // strips (4 x 64 x LMK_LD floats) during the loop, the partial tiles after it
+    constexpr int TILE = 16 * MF * 64, STRIPS = 4 * 64 * LMK_LD;      // floats: a wave's partial tile, the strips of all
+    __shared__ __attribute__((aligned(16))) float smem[4 * TILE > STRIPS ? 4 * TILE : STRIPS];  // strips during the loop, the partial tiles after it
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int fr = lane & 15, fq = lane >> 4;
     const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-    const int KT = K / 32, KTP = Kpad / 32, S = KTP / 4;  // S steps per wave (Kpad is a multiple of 256)
+    const int KT = K / 32, KTP = Kpad / 32, S = KTP / 4;  // S steps per wave (Kpad is a multiple of 256: an even number)
     const int k_first = wid * S;
     float* strip = smem + wid * (64 * LMK_LD);
     // weight loads: instruction j takes rows 8 j .. 8 j + 7 of the tile, 128 contiguous bytes each (one K step)
     const int wr = lane >> 3, wc = (lane & 7) * 4;
-#define LMK_ROW(j) const int64_t wrow##j = (int64_t)min(n0 + 8 * j + wr, N - 1) * K + wc
-    LMK_ROW(0); LMK_ROW(1); LMK_ROW(2); LMK_ROW(3); LMK_ROW(4); LMK_ROW(5); LMK_ROW(6); LMK_ROW(7);
-#undef LMK_ROW
-    const uint4* ap = (const uint4*)planes + ((int64_t)blockIdx.y * KTP * 12) * 64 + lane;  // fragment f of step kt: ap[(kt * 12 + f) * 64]
-    lm_v4f acc[4][4];
+    const float* Bt = B + (int64_t)n0 * K;
+    uint32_t wrow[8];      // (bytes from the tile's first row)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < 8; ++j) wrow[j] = ((uint32_t)min(8 * j + wr, N - 1 - n0) * (uint32_t)K + wc) * 4u;
+    const lm_v4u* ap = (const lm_v4u*)planes + ((int64_t)blockIdx.y * KTP * 12) * 64 + lane;  // fragment f = 4 p + i of step kt: ap[(kt * 12 + f) * 64]
+    lm_v4f acc[MF][4];
+#pragma unroll
+    for (int i = 0; i < MF; ++i)
 #pragma unroll
         for (int c = 0; c < 4; ++c) acc[i][c] = (lm_v4f){0.f, 0.f, 0.f, 0.f};
-    float4 g0, g1, g2, g3, g4, g5, g6, g7;
+    lm_v4f g[AHEAD][8];
+    lm_v4u af[2][3 * MF];
     // no branch around a load (the waits are counted): steps past the wave's share re-read its last step, steps past K read the
     // row's last step against zero planes
-#define LMK_W1(j, kt_) g##j = *(const float4*)(B + wrow##j + (kt_) * 32)
-#define LMK_WLOAD(s_)                                                                                               \
-    do {                                                                                                           \
-        const int kt_ = min(k_first + min((s_), S - 1), KT - 1);                                                   \
-        LMK_W1(0, kt_); LMK_W1(1, kt_); LMK_W1(2, kt_); LMK_W1(3, kt_); LMK_W1(4, kt_); LMK_W1(5, kt_); LMK_W1(6, kt_); LMK_W1(7, kt_); \
-    } while (0)
-#define LMK_ALOAD(s_, A_)                                                                                          \
-    do {                                                                                                           \
-        const int64_t kt_ = k_first + min((s_), S - 1);                                                            \
-        _Pragma("unroll") for (int f = 0; f < 12; ++f) A_[f] = ap[(kt_ * 12 + f) * 64];                            \
-    } while (0)
-#define LMK_S1(j) *(float4*)&strip[(8 * j + wr) * LMK_LD + wc] = g##j
-#define LMK_WSTORE()                                                                                               \
-    do {                                                                                                           \
-        __builtin_amdgcn_wave_barrier();                                                                           \
-        LMK_S1(0); LMK_S1(1); LMK_S1(2); LMK_S1(3); LMK_S1(4); LMK_S1(5); LMK_S1(6); LMK_S1(7);                    \
-        __builtin_amdgcn_wave_barrier();                                                                           \
-    } while (0)
-#define LMK_STEP(A_)                                                                                               \
-    do {                                                                                                           \
-        _Pragma("unroll") for (int c = 0; c < 4; ++c) {                                                            \
-            const float4 w0 = *(const float4*)&strip[(16 * c + fr) * LMK_LD + fq * 4];                             \
-            const float4 w1 = *(const float4*)&strip[(16 * c + fr) * LMK_LD + 16 + fq * 4];                        \
-            uint4 bh, bm, bl;                                                                                      \
-            lm_split_pair(w0.x, w0.y, bh.x, bm.x, bl.x);                                                           \
-            lm_split_pair(w0.z, w0.w, bh.y, bm.y, bl.y);                                                           \
-            lm_split_pair(w1.x, w1.y, bh.z, bm.z, bl.z);                                                           \
-            lm_split_pair(w1.z, w1.w, bh.w, bm.w, bl.w);                                                           \
-            const lm_v8b b1 = __builtin_bit_cast(lm_v8b, bh), b2 = __builtin_bit_cast(lm_v8b, bm), b3 = __builtin_bit_cast(lm_v8b, bl); \
-            _Pragma("unroll") for (int i = 0; i < 4; ++i) {                                                        \
-                const lm_v8b a1 = __builtin_bit_cast(lm_v8b, A_[i]), a2 = __builtin_bit_cast(lm_v8b, A_[4 + i]),   \
-                             a3 = __builtin_bit_cast(lm_v8b, A_[8 + i]);                                           \
-                lm_v4f t = acc[i][c];                                                                              \
-                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a3, b1, t, 0, 0, 0); /* small terms first */           \
-                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b3, t, 0, 0, 0);                                   \
-                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, b2, t, 0, 0, 0);                                   \
-                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, b1, t, 0, 0, 0);                                   \
-                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b2, t, 0, 0, 0);                                   \
-                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1, t, 0, 0, 0);                                   \
-                acc[i][c] = t;                                                                                     \
-            }                                                                                                      \
-        }                                                                                                          \
-    } while (0)
-    uint4 afa[12], afb[12];
-    LMK_WLOAD(0);
-    LMK_ALOAD(0, afa);
-    LMK_WSTORE();
-    LMK_WLOAD(1);
-    for (int s = 0; s < S; s += 2) {
-        // the scheduling barriers keep the next step's requests IN FRONT of this step's matrix-core instructions (left alone, the
-        // scheduler sinks them behind the 96 MFMAs, i.e. right in front of their use)
-        LMK_ALOAD(s + 1, afb);
+    auto wload = [&](int s, lm_v4f (&x)[8]) {
+        const int kt = min(k_first + min(s, S - 1), KT - 1);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = *(const lm_v4f*)((const char*)(Bt + kt * 32) + wrow[j]);
+    };
+    auto aload = [&](int s, lm_v4u (&x)[3 * MF]) {
+        const int64_t kt = k_first + min(s, S - 1);
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+#pragma unroll
+            for (int i = 0; i < MF; ++i) x[p * MF + i] = ap[(kt * 12 + 4 * p + i) * 64];
+    };
+    auto wstore = [&](const lm_v4f (&x)[8]) {
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < 8; ++j) *(lm_v4f*)&strip[(8 * j + wr) * LMK_LD + wc] = x[j];
+        __builtin_amdgcn_wave_barrier();
+    };
+    auto multiply = [&](const lm_v4u (&x)[3 * MF]) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const lm_v4f w0 = *(const lm_v4f*)&strip[(16 * c + fr) * LMK_LD + fq * 4];
+            const lm_v4f w1 = *(const lm_v4f*)&strip[(16 * c + fr) * LMK_LD + 16 + fq * 4];
+            lm_v4u bh, bm, bl;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                uint32_t hi, mid, lo;
+                lm_split_pair(e < 2 ? w0[2 * e] : w1[2 * e - 4], e < 2 ? w0[2 * e + 1] : w1[2 * e - 3], hi, mid, lo);
+                bh[e] = hi, bm[e] = mid, bl[e] = lo;
+            }
+            const lm_v8b b1 = __builtin_bit_cast(lm_v8b, bh), b2 = __builtin_bit_cast(lm_v8b, bm), b3 = __builtin_bit_cast(lm_v8b, bl);
+#pragma unroll
+            for (int i = 0; i < MF; ++i) {
+                const lm_v8b a1 = __builtin_bit_cast(lm_v8b, x[i]), a2 = __builtin_bit_cast(lm_v8b, x[MF + i]), a3 = __builtin_bit_cast(lm_v8b, x[2 * MF + i]);
+                lm_v4f t = acc[i][c];
+                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a3, b1, t, 0, 0, 0);  // small terms first
+                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b3, t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, b2, t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, b1, t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b2, t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1, t, 0, 0, 0);
+                acc[i][c] = t;
+            }
+        }
+    };
+    // a step: its weights are in the strip, those of the next AHEAD in registers
+    auto step = [&](int s, auto at) {
+        constexpr int U = decltype(at)::value;
+        // the scheduling barrier keeps the next steps' requests IN FRONT of this step's matrix-core instructions (left alone, the
+        // scheduler sinks them behind the MFMAs, i.e. right in front of their use)
+        aload(s + 1, af[(U + 1) & 1]);
         __builtin_amdgcn_sched_barrier(0);
-        LMK_STEP(afa);
-        LMK_WSTORE();      // step s + 1's weight rows (in registers since the previous step) replace step s's in the strip
-        LMK_WLOAD(s + 2);
-        LMK_ALOAD(s + 2, afa);
-        __builtin_amdgcn_sched_barrier(0);
-        LMK_STEP(afb);
-        LMK_WSTORE();
-        LMK_WLOAD(s + 3);
-    }
-#undef LMK_STEP
-#undef LMK_WSTORE
-#undef LMK_ALOAD
-#undef LMK_WLOAD
-#undef LMK_W1
-#undef LMK_S1
+        multiply(af[U & 1]);
+        wstore(g[U % AHEAD]);      // step s + 1's weight rows replace step s's in the strip
+        wload(s + 1 + AHEAD, g[U % AHEAD]);
+    };
+    wload(0, g[0]);
+    aload(0, af[0]);
+    wstore(g[0]);
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) wload(1 + u, g[u]);
+    constexpr std::integral_constant<int, 0> U0{};
+    constexpr std::integral_constant<int, 1> U1{};
+    constexpr std::integral_constant<int, 2> U2{};
+    constexpr std::integral_constant<int, 3> U3{};
+    int s = 0;
+    for (; s + 4 <= S; s += 4) step(s, U0), step(s + 1, U1), step(s + 2, U2), step(s + 3, U3);
+    if (s < S) step(s, U0), step(s + 1, U1);
     // the four partial tiles through LDS (the strips are dead: every wave is past its last read once the barrier is passed)
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MF; ++i)
 #pragma unroll
         for (int c = 0; c < 4; ++c)
 #pragma unroll
-            for (int reg = 0; reg < 4; ++reg) smem[(wid * 64 + i * 16 + fq * 4 + reg) * 64 + c * 16 + fr] = acc[i][c][reg];
+            for (int reg = 0; reg < 4; ++reg) smem[wid * TILE + (i * 16 + fq * 4 + reg) * 64 + c * 16 + fr] = acc[i][c][reg];
     __syncthreads();
-    for (int e = tid; e < 64 * 16; e += 256) {  // four consecutive columns per thread
+    for (int e = tid; e < 16 * MF * 16; e += 256) {  // four consecutive columns per thread
         const int r = e >> 4, c4 = (e & 15) * 4;
         if (m0 + r >= M) continue;
         float v[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = ((smem[(0 * 64 + r) * 64 + c4 + j] + smem[(1 * 64 + r) * 64 + c4 + j]) + smem[(2 * 64 + r) * 64 + c4 + j]) + smem[(3 * 64 + r) * 64 + c4 + j];
+        for (int j = 0; j < 4; ++j) v[j] = ((smem[r * 64 + c4 + j] + smem[TILE + r * 64 + c4 + j]) + smem[2 * TILE + r * 64 + c4 + j]) + smem[3 * TILE + r * 64 + c4 + j];
         float* cp = C + (int64_t)(m0 + r) * N + n0 + c4;
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             if (n0 + c4 + j < N) cp[j] = v[j];
     }
+}
+
+static void lm_head_launch(const void* planes, const float* B, float* C, int64_t M, int32_t N, int32_t K, hipStream_t st) {
+    const dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64));
+    auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, (const uint32_t*)planes, B, C, (int)M, (int)N, (int)K, (K + 255) / 256 * 256); };
+    if (M <= 16) launch(lm_head_bf16x3_ks_kernel<1, 4>);
+    else if (M <= 32) launch(lm_head_bf16x3_ks_kernel<2, 2>);
+    else launch(lm_head_bf16x3_ks_kernel<4, 1>);
 }
 
 extern "C" {
@@ -187,8 +206,7 @@ int i64h_lm_head(const float* A, const int32_t* a_rows, const float* B, float* C
     hipStream_t st = (hipStream_t)stream;
     hipLaunchKernelGGL(lm_split_rows_frag_kernel, dim3((unsigned)Mpad), dim3(256), 0, st, A, a_rows, (uint32_t*)workspace, (int)M, (int)K, Kpad);
     I64H_CHECK_LAUNCH();
-    hipLaunchKernelGGL(lm_head_bf16x3_ks_kernel, dim3((unsigned)((N + 63) / 64), (unsigned)(Mpad / 64)), dim3(256), 0, st, (const uint32_t*)workspace, B, C,
-                       (int)M, (int)N, (int)K, Kpad);
+    lm_head_launch(workspace, B, C, M, N, K, st);
     I64H_CHECK_LAUNCH();
     return 0;
 }
@@ -199,9 +217,7 @@ int i64h_lm_head_planes(const void* workspace, const float* B, float* C, int64_t
     I64H_CHECK_ARG(M >= 0 && M < (1ll << 24) && N > 0 && K > 0 && K % 32 == 0, "lm_head_planes: K=%d must be a multiple of 32", K);
     I64H_CHECK_ARG(workspace && ((uintptr_t)workspace | (uintptr_t)B) % 16 == 0, "lm_head_planes: workspace missing or operands not 16-byte aligned");
     if (M == 0) return 0;
-    const int Mpad = (int)((M + 63) / 64 * 64), Kpad = (K + 255) / 256 * 256;
-    hipLaunchKernelGGL(lm_head_bf16x3_ks_kernel, dim3((unsigned)((N + 63) / 64), (unsigned)(Mpad / 64)), dim3(256), 0, (hipStream_t)stream,
-                       (const uint32_t*)workspace, B, C, (int)M, (int)N, (int)K, Kpad);
+    lm_head_launch(workspace, B, C, M, N, K, (hipStream_t)stream);
     I64H_CHECK_LAUNCH();
     return 0;
 }
