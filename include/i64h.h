@@ -475,6 +475,11 @@ int i64h_fused_residual_norm_lm(const float* h, const float* add, const float* m
                                 const float* route_weights, int32_t top_k, float routed_scale, float shared_scale, float* h_out,
                                 const float* norm_weight, float eps, float* normed, int64_t n, int32_t H, const int32_t* slots,
                                 int32_t slots_per_row, int32_t slot_base, uint32_t* stats, void* lm_workspace, void* stream);
+/* The same for a step that wants the logits of some rows only: the planes of rows 0 .. m_rows - 1 (at most 2048) are those of the rows rows[m] of n; neither the residual nor the
+ * normalised rows are stored. */
+int i64h_fused_residual_norm_lm_rows(const float* h, const float* add, const float* moe_rows, const int32_t* moe_inv, const float* moe_shared,
+                                     const float* route_weights, int32_t top_k, float routed_scale, float shared_scale,
+                                     const float* norm_weight, float eps, int64_t n, int32_t H, const int32_t* rows, int64_t m_rows, void* lm_workspace, void* stream);
 /* The same residual update + norm, with the per-call quantization of the Linear calls that read the normalised rows folded in
  * (the rows of DynamicInt8Linear.forward's _quantize_activations, vllm_i64/core/loader.py:57-76, for every call fed by this
  * norm): one launch of co-resident workgroups with a grid barrier between "ranges of all rows known" and "rows quantized", so

@@ -58,6 +58,7 @@ SIGNATURES: Dict[str, str] = {
     "i64h_rmsnorm": "ppplifp",
     "i64h_fused_residual_norm": "ppppppiffppfplipiipp",
     "i64h_fused_residual_norm_lm": "ppppppiffppfplipiippp",
+    "i64h_fused_residual_norm_lm_rows": "ppppppiffpfliplpp",
     "i64h_lm_head_planes": "ppplii" + "p",
     "i64h_fused_residual_norm_fp8": "ppppppiffppfplippp",
     "i64h_fused_residual_norm_quant": "ppppppiffppflipiippppipppip",

@@ -100,7 +100,8 @@ __global__ __launch_bounds__(256) void fused_residual_norm_kernel(const float* _
                                                                   MoeCombine mc, int n, int rpb, float* __restrict__ h_out,
                                                                   const float* __restrict__ w, float eps, float* __restrict__ normed,
                                                                   int H, const int32_t* __restrict__ slots, int spr, int slot_base,
-                                                                  uint32_t* __restrict__ stats, uint32_t* __restrict__ lm_planes, int lm_ktp) {
+                                                                  uint32_t* __restrict__ stats, uint32_t* __restrict__ lm_planes, int lm_ktp,
+                                                                  const int32_t* __restrict__ rows, int count) {
     __shared__ float red[8], rlo[4], rhi[4];
     __shared__ float tab_lo[I64H_STAT_TAB], tab_hi[I64H_STAT_TAB];
     // one row per workgroup (decode): the row's few slots are updated directly, without the per-workgroup table
@@ -113,43 +114,44 @@ __global__ __launch_bounds__(256) void fused_residual_norm_kernel(const float* _
     // one row per workgroup: the row's slot ids are fetched now, so that the statistics update at the end does not start
     // with a dependent read
     int early_slot[4] = {0, 0, 0, 0};
-    const bool early = !use_tab && stats != nullptr && slots != nullptr && spr <= 4 && threadIdx.x == 0 && (int64_t)blockIdx.x * rpb < n;
+    const bool early = !use_tab && stats != nullptr && slots != nullptr && spr <= 4 && threadIdx.x == 0 && (int64_t)blockIdx.x * rpb < count;
     if (early) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             if (j < spr) early_slot[j] = slots[(int64_t)blockIdx.x * rpb * spr + j];
     }
     const int64_t t0 = (int64_t)blockIdx.x * rpb;
-    const int64_t t1 = t0 + rpb < n ? t0 + rpb : n;
+    const int64_t t1 = t0 + rpb < count ? t0 + rpb : count;
     // the norm weights are requested together with the first row: behind the barrier they would be a round trip of their own
     float4 gw[FRN_MAXV];
 #pragma unroll
     for (int j = 0; j < FRN_MAXV; ++j) {
         const int i = threadIdx.x + j * 256;
-        gw[j] = (normed && i < nv) ? ((const float4*)w)[i] : make_float4(0, 0, 0, 0);
+        gw[j] = ((normed || lm_planes) && i < nv) ? ((const float4*)w)[i] : make_float4(0, 0, 0, 0);
     }
     for (int64_t t = t0; t < t1; ++t) {
+        const int64_t src = rows ? (int64_t)rows[t] : t;      // (rows: those whose logits are wanted)
         float4 v[FRN_MAXV];
         float ss = 0.0f;
 #pragma unroll
         for (int j = 0; j < FRN_MAXV; ++j) {
             const int i = threadIdx.x + j * 256;
             if (i < nv) {
-                float4 a = h ? ((const float4*)(h + t * H))[i] : make_float4(0, 0, 0, 0);
+                float4 a = h ? ((const float4*)(h + src * H))[i] : make_float4(0, 0, 0, 0);
                 if (add) {
-                    float4 b = ((const float4*)(add + t * H))[i];
+                    float4 b = ((const float4*)(add + src * H))[i];
                     a.x = a.x + b.x; a.y = a.y + b.y; a.z = a.z + b.z; a.w = a.w + b.w;
                 }
                 if (mc.rows) {
-                    float4 r0 = ((const float4*)(mc.rows + (int64_t)(mc.inv ? mc.inv[t] : t) * H))[i];
+                    float4 r0 = ((const float4*)(mc.rows + (int64_t)(mc.inv ? mc.inv[src] : src) * H))[i];
                     float4 o = make_float4(mc.wk[0] * r0.x, mc.wk[0] * r0.y, mc.wk[0] * r0.z, mc.wk[0] * r0.w);
                     for (int k = 1; k < mc.top_k; ++k) {
-                        float4 rk = ((const float4*)(mc.rows + (int64_t)(mc.inv ? mc.inv[(int64_t)k * n + t] : (int64_t)k * n + t) * H))[i];
+                        float4 rk = ((const float4*)(mc.rows + (int64_t)(mc.inv ? mc.inv[(int64_t)k * n + src] : (int64_t)k * n + src) * H))[i];
                         o.x = o.x + mc.wk[k] * rk.x; o.y = o.y + mc.wk[k] * rk.y;
                         o.z = o.z + mc.wk[k] * rk.z; o.w = o.w + mc.wk[k] * rk.w;
                     }
                     if (mc.shared) {
-                        float4 s = ((const float4*)(mc.shared + t * H))[i];
+                        float4 s = ((const float4*)(mc.shared + src * H))[i];
                         o.x = mc.routed_scale * o.x + mc.shared_scale * s.x; o.y = mc.routed_scale * o.y + mc.shared_scale * s.y;
                         o.z = mc.routed_scale * o.z + mc.shared_scale * s.z; o.w = mc.routed_scale * o.w + mc.shared_scale * s.w;
                     } else {
@@ -158,13 +160,13 @@ __global__ __launch_bounds__(256) void fused_residual_norm_kernel(const float* _
                     if (h || add) { a.x = a.x + o.x; a.y = a.y + o.y; a.z = a.z + o.z; a.w = a.w + o.w; }
                     else a = o;  // no residual stream: the bare MoE output
                 }
-                if (h_out) ((float4*)(h_out + t * H))[i] = a;
+                if (h_out) ((float4*)(h_out + src * H))[i] = a;
                 v[j] = a;
                 ss = __builtin_fmaf(a.x, a.x, ss); ss = __builtin_fmaf(a.y, a.y, ss);
                 ss = __builtin_fmaf(a.z, a.z, ss); ss = __builtin_fmaf(a.w, a.w, ss);
             }
         }
-        if (!normed) continue;  // uniform for the whole grid
+        if (!normed && !lm_planes) continue;  // uniform for the whole grid
         ss = wave_sum(ss);
         if ((threadIdx.x & 63) == 0) red[(t & 1) * 4 + (threadIdx.x >> 6)] = ss;  // two sets: the next row's partials never overtake a reader
         __syncthreads();
@@ -178,7 +180,7 @@ __global__ __launch_bounds__(256) void fused_residual_norm_kernel(const float* _
                 const float4 g = gw[j];
                 float4 a = v[j];
                 a.x = a.x * rr * g.x; a.y = a.y * rr * g.y; a.z = a.z * rr * g.z; a.w = a.w * rr * g.w;
-                ((float4*)(normed + t * H))[i] = a;
+                if (normed) ((float4*)(normed + t * H))[i] = a;
                 if (lm_planes) {
                     // the tied lm_head's activation planes of this row, in its fragment order (i64h_lmhead.hip): the four values are the
                     // pairs 2 i and 2 i + 1 of the row, neighbours in a lane's 16 bytes - the row split launch of i64h_lm_head, saved
@@ -871,12 +873,13 @@ int i64h_rmsnorm(const float* x, const float* weight, float* out, int64_t rows, 
 static int frn_launch(const float* h, const float* add, const float* moe_rows, const int32_t* moe_inv, const float* moe_shared,
                              const float* route_weights, int32_t top_k, float routed_scale, float shared_scale, float* h_out,
                              const float* norm_weight, float eps, float* normed, int64_t n, int32_t H, const int32_t* slots,
-                             int32_t slots_per_row, int32_t slot_base, uint32_t* stats, void* stream, uint32_t* lm_planes, int lm_ktp) {
+                             int32_t slots_per_row, int32_t slot_base, uint32_t* stats, void* stream, uint32_t* lm_planes, int lm_ktp, const int32_t* rows = nullptr, int64_t m_rows = 0) {
     I64H_CHECK_ARG(n >= 0 && H > 0 && H % 4 == 0 && H <= 1024 * FRN_MAXV, "fused_residual_norm: H=%d unsupported (multiple of 4, <= %d)", H,
                    1024 * FRN_MAXV);
     I64H_CHECK_ARG(top_k >= 0 && top_k <= 8, "fused_residual_norm: top_k=%d unsupported", top_k);
     I64H_CHECK_ARG(moe_rows == nullptr || (route_weights != nullptr && top_k > 0), "fused_residual_norm: moe args");  // moe_inv NULL: rows already in (route, token) order
-    if (n == 0) return 0;
+    const int64_t count = rows ? m_rows : n;
+    if (n == 0 || count == 0) return 0;
     MoeCombine mc;
     mc.rows = moe_rows;
     mc.inv = moe_inv;
@@ -896,9 +899,9 @@ static int frn_launch(const float* h, const float* add, const float* moe_rows, c
         I64H_CHECK_LAUNCH();
         return 0;
     }
-    const int rpb = n > 2048 ? 8 : 1;  // many rows: fold 8 rows per workgroup before touching the global stat slots
-    hipLaunchKernelGGL(fused_residual_norm_kernel, dim3((unsigned)i64h_cdiv(n, rpb)), dim3(256), 0, (hipStream_t)stream, h, add, mc,
-                       (int)n, rpb, h_out, norm_weight, eps, normed, (int)H, slots, (int)slots_per_row, (int)slot_base, stats, lm_planes, lm_ktp);
+    const int rpb = count > 2048 ? 8 : 1;  // many rows: fold 8 rows per workgroup before touching the global stat slots
+    hipLaunchKernelGGL(fused_residual_norm_kernel, dim3((unsigned)i64h_cdiv(count, rpb)), dim3(256), 0, (hipStream_t)stream, h, add, mc,
+                       (int)n, rpb, h_out, norm_weight, eps, normed, (int)H, slots, (int)slots_per_row, (int)slot_base, stats, lm_planes, lm_ktp, rows, (int)count);
     I64H_CHECK_LAUNCH();
     return 0;
 }
@@ -922,6 +925,17 @@ int i64h_fused_residual_norm_lm(const float* h, const float* add, const float* m
     I64H_CHECK_ARG(H % 32 == 0 && n <= 2048, "fused_residual_norm_lm: H=%d must be a multiple of 32, at most 2048 rows", H);
     return frn_launch(h, add, moe_rows, moe_inv, moe_shared, route_weights, top_k, routed_scale, shared_scale, h_out, norm_weight, eps, normed, n,
                       H, slots, slots_per_row, slot_base, stats, stream, (uint32_t*)lm_workspace, (H + 255) / 256 * 8);
+}
+
+// The final norm of a step that wants the logits of some rows: row m of the planes is the residual update and norm of row rows[m] of n; nothing else is stored.  (16384 rows of which
+// eight are wanted: 90 us with all of them normed and stored, 5 so, and no row split in front of the lm_head.)
+int i64h_fused_residual_norm_lm_rows(const float* h, const float* add, const float* moe_rows, const int32_t* moe_inv, const float* moe_shared,
+                                     const float* route_weights, int32_t top_k, float routed_scale, float shared_scale,
+                                     const float* norm_weight, float eps, int64_t n, int32_t H, const int32_t* rows, int64_t m_rows, void* lm_workspace, void* stream) {
+    I64H_CHECK_ARG(lm_workspace != nullptr && (uintptr_t)lm_workspace % 16 == 0 && rows != nullptr, "fused_residual_norm_lm_rows: workspace (16-byte aligned) and rows are required");
+    I64H_CHECK_ARG(H % 32 == 0 && m_rows >= 0 && m_rows <= 2048, "fused_residual_norm_lm_rows: H=%d must be a multiple of 32, at most 2048 rows", H);
+    return frn_launch(h, add, moe_rows, moe_inv, moe_shared, route_weights, top_k, routed_scale, shared_scale, nullptr, norm_weight, eps, nullptr, n,
+                      H, nullptr, 1, 0, nullptr, stream, (uint32_t*)lm_workspace, (H + 255) / 256 * 8, rows, m_rows);
 }
 
 // Residual update + RMSNorm + the per-token e4m3fn quantization of the normalised rows (i64h_fused_residual_norm followed by

@@ -265,6 +265,20 @@ class I64MoEModel:
                      ops._stream())
         return B.logits
 
+    def _final(self, B: "_Buffers", logit_rows, norm_w, eps: float, record=None, **mk) -> None:
+        """The last residual update, the final norm and the logits.  Where the logits of some rows are wanted, these alone are normed, straight into the lm_head's operands."""
+        M, H = B.logits.shape[0], self.cfg.hidden_size
+        if logit_rows is not None and record is None and self.LM_HEAD_BF16X3 and self.LM_PLANES_FROM_NORM and H % 32 == 0 and 0 < M <= 2048:
+            if B.lm_planes_ws is None:
+                B.lm_planes_ws = torch.zeros(max(16, ops.lm_head_workspace_bytes(M, H)), dtype=torch.uint8, device=self.device)
+            for k in ("h_out", "slot_base"):
+                mk.pop(k, None)
+            ops.fused_residual_norm_lm_rows(B.h, norm_w, eps, logit_rows, B.lm_planes_ws, **mk)
+            ops.lm_head_planes(B.lm_planes_ws, self.embed, B.logits)
+            return
+        ops.fused_residual_norm(B.h, norm_w, eps, normed=B.normed, **mk)
+        self._lm_head(B, logit_rows)
+
     # ---- helpers ----
     # An engine's steps come in many row counts (chunked prefill, mixed batches): the step buffers of the most recently used counts
     # are kept, older sets are dropped (their memory goes back to the allocator, ordered by the stream).  A set whose addresses a
@@ -650,10 +664,12 @@ class I64MoEModel:
                 last = l + 1 == cfg.num_layers
                 mk = dict(moe_rows=moe_rows, moe_inv=moe_inv, moe_shared=B.sh_out if cfg.shared_intermediate_size else None, route_weights=rw,
                           routed_scale=W["routed_scale"], shared_scale=W["shared_scale"], h_out=B.h, slot_base=base + spl)
-                if fq and not last:
+                if last:
+                    self._final(B, logit_rows, nxt, eps, record, **mk)
+                elif fq:
                     ops.fused_residual_norm_quant(B.h, nxt, eps, st, self.dec_sync, B.xa, B.xs, **mk)
                 else:
-                    ops.fused_residual_norm(B.h, nxt, eps, normed=B.normed, stats=None if last else st, **mk)
+                    ops.fused_residual_norm(B.h, nxt, eps, normed=B.normed, stats=st, **mk)
                 if record is not None:
                     record[f"l{l}.out"] = B.h.clone()
             else:
@@ -666,11 +682,12 @@ class I64MoEModel:
                 self._linear(B.d_inter, W["dn"], base + 3, B.da, B.ds, B.d_out)
                 nxt = self.layers[l + 1]["ln1"] if l + 1 < cfg.num_layers else self.final_norm
                 last = l + 1 == cfg.num_layers
-                if fq and not last:
+                if last:
+                    self._final(B, logit_rows, nxt, eps, record, add=B.d_out, h_out=B.h)
+                elif fq:
                     ops.fused_residual_norm_quant(B.h, nxt, eps, st, self.dec_sync, B.xa, B.xs, add=B.d_out, h_out=B.h, slot_base=base + spl)
                 else:
-                    ops.fused_residual_norm(B.h, nxt, eps, add=B.d_out, h_out=B.h, normed=B.normed, slot_base=base + spl,
-                                            stats=None if last else st)
+                    ops.fused_residual_norm(B.h, nxt, eps, add=B.d_out, h_out=B.h, normed=B.normed, slot_base=base + spl, stats=st)
                 if record is not None:
                     record[f"l{l}.out"] = B.h.clone()
             if mu and l + 1 < cfg.num_layers:
@@ -678,7 +695,8 @@ class I64MoEModel:
                 ops.rows_minmax(B.h, st, slot_base=base + self.mu_slot + 1)
                 self._linear(B.h, W["mu_proj"], base + self.mu_slot + 1, B.xa, B.xs, B.mu_out)
                 ops.call("i64h_mu_update", ops.ptr(W["mu"]), ops.ptr(B.mu_out), ops.ptr(B.mu_prev), n, H, ops._stream())
-        self._lm_head(B, logit_rows)
+        if tails is not None:      # (the last one has written the final norm's rows)
+            self._lm_head(B, logit_rows)
         return B.logits
 
     # many-row attention form of the library (16-row tiles, rows of a tile that share a sequence share its K/V tiles): taken for
@@ -810,8 +828,8 @@ class I64MoEModel:
         inner = [cfg.expert_inter] + ([cfg.shared_intermediate_size] if cfg.shared_intermediate_size else []) if cfg.is_moe else [cfg.intermediate_size]
         return all(k > 0 and k % 64 == 0 for k in inner) and all((W["q_norm"] is None) == (W["k_norm"] is None) for W in self.layers)
 
-    def _layers_fp8_tiles(self, B, n, positions, slot_ids, ctx_len, kvc, rows_are_slots, splits) -> None:
-        """The decoder layers of such a step.  B.xa / B.xs hold the first layer's normed rows quantized; leaves B.normed (the final norm's rows)."""
+    def _layers_fp8_tiles(self, B, n, positions, slot_ids, ctx_len, kvc, rows_are_slots, splits, logit_rows) -> None:
+        """The decoder layers of such a step and its logits.  B.xa / B.xs hold the first layer's normed rows quantized."""
         cfg, H, eps = self.cfg, self.cfg.hidden_size, self.cfg.rms_eps
         desc = ops.fp8_codes_desc
         attn2d = B.attn.view(n, H)
@@ -845,7 +863,7 @@ class I64MoEModel:
             if l + 1 < cfg.num_layers:
                 ops.fused_residual_norm_fp8(B.h, nxt, eps, B.xa, B.xs, **mk)
             else:
-                ops.fused_residual_norm(B.h, nxt, eps, normed=B.normed, **mk)
+                self._final(B, logit_rows, nxt, eps, **mk)
 
     def _forward_fp8(self, token_ids, positions, slot_ids, ctx_len, logit_rows, kvc, record, max_ctx_hint, rows_are_slots, tokens_per_seq=None):
         """The forward with every Linear an fp8_linear (vllm_i64/core/fp8.py:137-194, its torch._scaled_mm branch): activations are
@@ -898,7 +916,7 @@ class I64MoEModel:
             return ops.gemm_fp8(xq, xs, Wp.w_q, Wp.w_s, out, w_frags=wf, **kw)
 
         if tiles:
-            self._layers_fp8_tiles(B, n, positions, slot_ids, ctx_len, kvc, rows_are_slots, splits)
+            self._layers_fp8_tiles(B, n, positions, slot_ids, ctx_len, kvc, rows_are_slots, splits, logit_rows)
         for l, W in enumerate(self.layers) if not tiles else ():
             if record is not None:
                 record[f"l{l}.in"] = B.h.clone()
@@ -967,7 +985,9 @@ class I64MoEModel:
                         linear(B.sh_inter, B.sha, B.shs, W["sh_dn"], B.sh_out)
                 mk = dict(moe_rows=B.e_out, moe_inv=None, moe_shared=B.sh_out if S else None, route_weights=rw,
                           routed_scale=W["routed_scale"], shared_scale=W["shared_scale"], h_out=B.h)
-                if nq and not last:
+                if last:
+                    self._final(B, logit_rows, nxt, eps, record, **mk)
+                elif nq:
                     ops.fused_residual_norm_fp8(B.h, nxt, eps, B.xa, B.xs, **mk)
                 else:
                     ops.fused_residual_norm(B.h, nxt, eps, normed=B.normed, **mk)
@@ -975,19 +995,20 @@ class I64MoEModel:
                 linear(x_in, B.xa, B.xs, W["gu"], B.d_inter, epilogue=ops.EPI_SWIGLU, **nk)
                 linear(B.d_inter, B.da, B.ds, W["dn"], B.h, c_add=B.h)   # h += down(...); the next norm rides in the next qkv call
                 if last:
-                    ops.fused_residual_norm(B.h, nxt, eps, normed=B.normed)
+                    self._final(B, logit_rows, nxt, eps, record)
                 else:
                     pend = nxt
             else:
                 linear(x_in, B.xa, B.xs, W["gu"], B.d_inter, epilogue=ops.EPI_SWIGLU, **nk)
                 linear(B.d_inter, B.da, B.ds, W["dn"], B.d_out)
-                if nq and not last:
+                if last:
+                    self._final(B, logit_rows, nxt, eps, record, add=B.d_out, h_out=B.h)
+                elif nq:
                     ops.fused_residual_norm_fp8(B.h, nxt, eps, B.xa, B.xs, add=B.d_out, h_out=B.h)
                 else:
                     ops.fused_residual_norm(B.h, nxt, eps, add=B.d_out, h_out=B.h, normed=B.normed)
             if record is not None:
                 record[f"l{l}.out"] = B.h.clone()
-        self._lm_head(B, logit_rows)
         return B.logits
 
     def _moe(self, B: _Buffers, W: dict, l: int, base: int, prequantized: bool = False):

@@ -578,6 +578,20 @@ def fused_residual_norm(h: torch.Tensor, norm_weight: Optional[torch.Tensor], ep
     return h_out, normed
 
 
+def fused_residual_norm_lm_rows(h: torch.Tensor, norm_weight: torch.Tensor, eps: float, rows: torch.Tensor, lm_workspace: torch.Tensor, add: Optional[torch.Tensor] = None,
+                                moe_rows: Optional[torch.Tensor] = None, moe_inv: Optional[torch.Tensor] = None, moe_shared: Optional[torch.Tensor] = None,
+                                route_weights: Sequence[float] = (), routed_scale: float = 1.0, shared_scale: float = 1.0) -> None:
+    """The residual update and norm of the rows `rows` int32 [M] alone, as the activation planes of lm_head_planes (lm_workspace: lm_head_workspace_bytes(M, H) bytes, zeroed once by the
+    caller); h itself stays as it is."""
+    _chk(h, torch.float32, "h"), _chk(rows, torch.int32, "rows")
+    n, H = h.shape
+    if lm_workspace.numel() * lm_workspace.element_size() < lm_head_workspace_bytes(rows.numel(), H):
+        raise _lib.I64HError("fused_residual_norm_lm_rows: workspace smaller than the rows' planes")
+    rw = (ctypes.c_float * 8)(*([float(w) for w in route_weights] + [0.0] * (8 - len(route_weights))))
+    call("i64h_fused_residual_norm_lm_rows", ptr(h), ptr(add), ptr(moe_rows), ptr(moe_inv), ptr(moe_shared), ctypes.addressof(rw), len(route_weights), float(routed_scale),
+         float(shared_scale), ptr(norm_weight), float(eps), n, H, ptr(rows), rows.numel(), ptr(lm_workspace), _stream())
+
+
 def gemm_i8_frags_qkv_rope_kv(a8: torch.Tensor, row_scale: torch.Tensor, w_frags: torch.Tensor, w_scale: torch.Tensor, q_norm_w, k_norm_w,
                               qk_eps: float, rope_tab, positions, slot_ids, block_table, k_cache, v_cache, num_heads: int,
                               num_kv_heads: int, head_dim: int, q_out: Optional[torch.Tensor] = None) -> torch.Tensor:
