@@ -271,3 +271,38 @@ def test_prefill_attention_over_bf16_pages(dev, nh, kvh, block):
     ops.stats_reset(same)
     ops.rows_minmax(out.view(rows, nh * hd).to(dev), same, slots=torch.ones(rows, dtype=torch.int32, device=dev))
     assert torch.equal(ops.qparams(stats, 2)[2][1], ops.qparams(same, 2)[2][1])
+
+
+@pytest.mark.parametrize("step", [7.5, 8.5, 30.0])
+def test_prefill_attention_whose_scores_climb(dev, step):
+    """Scores that rise by ``step`` powers of two from one 64-token tile to the next, in every second row (they fall in the others): the
+    reference of the running sums is kept where a tile lies less than 8 above it and renewed where it lies higher.  A score's sum of at most
+    70 terms is within 16 roundings of the terms' magnitudes (below 4 x step x ln 2 + 8), a weight as much relative to itself, the result
+    twice that times the largest value.  A row's bits do not depend on the rows beside it: the same prompt in two portions gives them too."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(int(step))
+    hd, block, L = 64, 16, 64 * 5 + 7
+    up = torch.zeros(hd)
+    up[5] = 1.0
+    tile = (torch.arange(L) // 64).float().view(L, 1, 1)
+    k = (torch.randn(L, 2, hd, generator=g) * 0.5 + tile * up * 8.0).bfloat16()
+    v = torch.randn(L, 2, hd, generator=g).bfloat16()
+    q = torch.randn(L, 8, hd, generator=g) * 0.5
+    q[:, :, 5] = step * 0.6931472 * (1.0 - 2.0 * (torch.arange(L) % 2).float()).view(L, 1)
+    nb = (L + block - 1) // block
+    pad = lambda x: torch.cat([x, torch.zeros(nb * block - L, 2, hd).bfloat16()]).view(nb, block, 2, hd).to(dev)
+    bt = torch.arange(nb, dtype=torch.int32, device=dev).view(1, nb)
+    kp, vp = pad(k), pad(v)
+
+    def run(lo):
+        n = L - lo
+        return ops.paged_attn(q[lo:].contiguous().to(dev), kp, vp, bt, torch.arange(lo + 1, L + 1, dtype=torch.int32, device=dev),
+                              slot_ids=torch.zeros(n, dtype=torch.int32, device=dev), splits=1).cpu()
+
+    out = run(0)
+    s = torch.einsum("thd,shd->ths", q.double(), k.double().repeat_interleave(4, 1)) / hd ** 0.5
+    s = s.masked_fill(torch.arange(L).view(1, 1, L) > torch.arange(L).view(L, 1, 1), float("-inf"))
+    ref = torch.einsum("ths,shd->thd", torch.softmax(s, -1), v.double().repeat_interleave(4, 1))
+    bound = 2 * 16 * 2.0 ** -24 * (5 * step * 0.6931472 + 8) * float(v.abs().max())
+    assert (out.double() - ref).abs().max() <= bound
+    assert torch.equal(run(37), out[37:])

@@ -677,10 +677,15 @@ __global__ __launch_bounds__(GS * 64, I64H_PF_OCC) void paged_attn_prefill_bf16_
 // registers leave two waves a SIMD.  Here a tile is loaded straight into LDS, 16 bytes a lane, the column that a lane brings chosen so that the piece lands where
 // pb_k / pb_v say, while the tile before it is worked on: one barrier a tile, three waves a SIMD.  A lane looks up the page of one token a tile (every wave all
 // 64) a tile ahead of the loads; a ballot of them says, without LDS, which tokens have a page, and whether a tile needs a mask at all.
-// The operations and their order are the form above's, the results the same bits.  16 heads over 4 KV heads, before and after, us: 8 sequences of 2048 rows
+// A row's reference is not its running maximum but one that a score may exceed by PF_SLACK: the maximum over a row's four lanes, a serial chain of exchanges
+// between the two products of each tile, and the rescaling are left to the tiles that need them (a row's first, and few after it).  With / without, us: 8 sequences of
+// 2048 rows 259 / 269, one of 481 13.6 / 14.1, 1500 + 77 40.7 / 42.7, 12 over 12 114 / 119, 32 over 4 152 / 162, 100 rows behind 900 39.3 / 41.2; the mean error
+// against 64 bits 3.22e-7 / 3.23e-7 (wide scores 7.29e-7 / 7.39e-7).  Started at minus the reference, the sums of the scores need no subtraction (250, 13.1, 39.2),
+// but lie 3 to 15 % further from 64 bits.  The form above against this one before that, 16 heads over 4 KV heads, us: 8 sequences of 2048 rows
 // 291 -> 248, one of 481 17.6 -> 14.1, 1500 + 77 52 -> 42.5; 12 heads over 12, 2 of 2048 204 -> 118; 16 over 8 150 -> 108; 32 over 4 182 -> 160; forty of 16 rows
 // 8.5 -> 8.5.  With three tiles in LDS (and two on their way) 250, 14.1, 43.0, 137, 115, 165: fewer workgroups fit.  Four waves a SIMD spill (309).
 // 8-bit caches stay with the form above, which converts on the way into LDS.
+#define PF_SLACK 8.0f      // how far above its reference a row's score may lie: weights up to 2^8, which 32-bit sums hold as well as those up to one
 template <int GS>
 __global__ __launch_bounds__(GS * 64, 3) void paged_attn_prefill_direct_kernel(const float* __restrict__ q, const __hip_bfloat16* __restrict__ k_cache,
                                                                          const __hip_bfloat16* __restrict__ v_cache, const int32_t* __restrict__ block_table,
@@ -819,20 +824,19 @@ __global__ __launch_bounds__(GS * 64, 3) void paged_attn_prefill_direct_kernel(c
             float mx = -INFINITY;
 #pragma unroll
             for (int t = 0; t < 4; ++t) mx = fmaxf(mx, fmaxf(fmaxf(sc[t][0], sc[t][1]), fmaxf(sc[t][2], sc[t][3])));
-            {  // over the four lanes of a query row (lane ^ 16, lane ^ 32) through register swaps, no LDS round trip
+            if (__ballot(mx > m + PF_SLACK)) {      // some row's first tile, or far above its reference: a new one, what there is rescaled (rare after the first tiles)
+                // over the four lanes of a query row (lane ^ 16, lane ^ 32) through register swaps, no LDS round trip
                 const PairF sr = swap_rows(mx);
                 mx = fmaxf(sr.lo, sr.hi);
                 const PairF sh = swap_halves(mx);
                 mx = fmaxf(sh.lo, sh.hi);
-            }
-            const float mn = fmaxf(m, mx);
-            if (__ballot(mn != m)) {  // some row's running maximum moved: rescale (rare after the first tiles)
+                const float mn = mx > m + PF_SLACK ? mx : m;  // by the row's own scores: its neighbours in the tile change nothing in its result
                 const float alpha = (mn == -INFINITY) ? 1.0f : exp2f(m - mn);
 #pragma unroll
                 for (int j = 0; j < 5; ++j) acc[j] *= alpha;
+                m = mn;
             }
-            m = mn;
-            const float mref = (mn == -INFINITY) ? 0.0f : mn;  // exp2(-inf - 0) = 0 for masked scores, no per-element test
+            const float mref = (m == -INFINITY) ? 0.0f : m;  // exp2(-inf - 0) = 0 for masked scores, no per-element test
 #pragma unroll
             for (int kp = 0; kp < 2; ++kp) {  // 32 tokens per step: the lane's slots are its registers of score tiles 2 kp and 2 kp + 1
                 float pv[8];
