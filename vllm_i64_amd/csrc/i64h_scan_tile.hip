@@ -267,14 +267,26 @@ __global__ __launch_bounds__(256) void scan_pairs_kernel(const i64h_gdn_args p, 
     }
 }
 
+// a descriptor of `bytes` from `base` on (the same in every lane, which the compiler doesn't see where they run along with a loop)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t st_buffer(const float* base, uint32_t bytes) {
+    const uint64_t b = (uint64_t)base;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b), hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(((uint64_t)hi << 32) | lo), 0, (int)__builtin_amdgcn_readfirstlane(bytes), 0x00020000);
+}
+
 // One workgroup per (16 value columns, head, run); wave w holds the key channels [16 BPW w, + 16 BPW) of the state, lane (g, c) of column c the
 // channels 4 g .. 4 g + 3 of every block of 16.  Operands come two tiles ahead, straight into registers.
-// What bounds a long run is a tile's chain - 8 matrix instructions, LDS and a barrier, 4, 8 more: 1.1 us of 16 tokens (token by token 2.5); reading q, k and
-// decays here and taking the products in every workgroup was 2.0 (29 narrow loads a wave are 1550 cycles of address and L1 work, their products 650).
+// What bounds a long run is a tile's chain - 8 matrix instructions, LDS and a barrier, 4, 8 more - and what one wave a SIMD has to issue beside it: 0.88 us of 16
+// tokens of 128 channels (token by token 2.5), of which the 29 matrix instructions are 930 cycles of 2000 and the loads' addresses 350.  Loads through descriptors
+// (no 64-bit address a lane, no branch for rows behind the end) and in four groups that stand between the products, the read-out's products around the exchange,
+// its sums and stores behind the next tile's barrier; before that 1.13 us.  us, before and after: 1531 rows, 16 heads 107 -> 84, five ragged runs 110 -> 89,
+// 8 of 512 over 8 heads 56 -> 48, 32 of 2048 949 -> 796, 64 channels 76 -> 58; linear attention 68 -> 57, 84 -> 61, 38 -> 34, 572 -> 553, 52 -> 37 (64 runs of 256 rows,
+// 16 heads: 294 -> 300).  All of a tile's loads in front of its products: 101 for the first; reloading an operand's registers behind its last product instead of a
+// third set: 85, linear attention 71.  Reading q, k and decays here and taking the products in every workgroup was 2.0 us a tile.
 // The workgroups of a head are a multiple of eight apart where there are eight heads: one die's L2 then serves them all.
 template <int BPW, bool DELTA>
-__global__ __launch_bounds__(256, BPW > 2 ? 1 : 2) void scan_tile_kernel(const i64h_gdn_args p) {
-    constexpr int NP = 64 * BPW, FL = st_floats(NP);
+__global__ __launch_bounds__(256, BPW > 2 && DELTA ? 1 : 2) void scan_tile_kernel(const i64h_gdn_args p) {
+    constexpr int NP = 64 * BPW, FL = st_floats(NP), SETS = 3;
     __shared__ stf4 sX[2][DELTA ? 4 : 1][64], sY[2][4][64];
     const int N = p.dim, P = p.vdim;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -295,80 +307,119 @@ __global__ __launch_bounds__(256, BPW > 2 ? 1 : 2) void scan_tile_kernel(const i
     }
     const int nt = (int)((r1 - r0 + ST_TOK - 1) / ST_TOK);
     const float* tiles = p.work + (st_slot(r0, seg) * p.heads + a) * FL;
-    const float* vbase = p.X + r0 * p.ldx + p.v_off + a * P;
-    const int64_t tstep = (int64_t)p.heads * FL;
-    const uint32_t ldx4 = 4 * (uint32_t)p.ldx, vc = cok ? 4 * col : 0;      // (16 rows span less than 4 GiB: the launch's check)
+    const int64_t tstep = (int64_t)p.heads * FL, vstep = ST_TOK * p.ldx;
     const int rows_last = (int)(r1 - r0) - ST_TOK * (nt - 1);      // of the last tile
+    const float* values = p.X + r0 * p.ldx + p.v_off + a * P;
+    // what a lane reads lies at the same offsets of every tile (16 rows span less than 4 GiB: the launch's check); value rows behind the run's end read as zeros
+    const uint32_t ldx4 = 4 * (uint32_t)p.ldx, at = 4 * (256 * BPW * w + 4 * lane), at_B = 4 * (c * ST_TOK + 4 * g + w), at_T = 4 * (c * ST_TOK + 4 * g);
+    uint32_t at_v[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) at_v[r] = (4 * g + r) * ldx4 + (cok ? 4 * col : 0);
+    auto at4 = [](const __amdgpu_buffer_rsrc_t& m, uint32_t lane_at, uint32_t step) { return __builtin_bit_cast(stf4, __builtin_amdgcn_raw_buffer_load_b128(m, lane_at, step, 0)); };
+    auto at1 = [](const __amdgpu_buffer_rsrc_t& m, uint32_t lane_at, uint32_t step) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(m, lane_at, step, 0)); };
     struct Ops {      // k P and q P (lane: token c, channels 4 g ..), k P_16 / P (tokens 4 g .., channel c), P_16 (channels 4 g ..), values (tokens 4 g ..)
         stf4 qp[BPW], kd[BPW], kp[DELTA ? BPW : 1], tot[BPW], T;
         float v[4], B;
     };
-    auto ld4 = [](const float* base, uint32_t off) { return *(const stf4*)((const char*)base + off); };
-    auto ld1 = [](const float* base, uint32_t off) { return *(const float*)((const char*)base + off); };
-    auto load = [&](int i, Ops& u) {
+    struct Tile {
+        __amdgpu_buffer_rsrc_t m, v;
+    };
+    auto where = [&](int i) {
         i = min(i, nt - 1);      // (past the end: the last tile once more, nobody reads it)
-        const float *m = tiles + i * tstep, *vt = vbase + (int64_t)i * ST_TOK * p.ldx;
-        const uint32_t vl = (i == nt - 1 ? rows_last - 1 : ST_TOK - 1) * ldx4;
-        const uint32_t at = 4 * (256 * BPW * w + 4 * lane);
+        return Tile{st_buffer(tiles + i * tstep, 4 * FL), st_buffer(values + i * vstep, (i < nt - 1 ? ST_TOK - 1 : rows_last - 1) * ldx4 + 4 * (uint32_t)P)};
+    };
+    // a tile's loads in four parts, which stand apart: a wave's sixteen bytes a lane keep the unit that takes them, one for four waves, busy for 16 cycles
+    auto load = [&](const Tile& t, Ops& u, int part) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (part == 0) {
 #pragma unroll
-        for (int b = 0; b < BPW; ++b) {
-            if (DELTA) u.kp[b] = ld4(m + 2 * ST_TOK * NP + 256 * b, at);
-            u.qp[b] = ld4(m + 256 * b, at);
-            u.kd[b] = ld4(m + ST_TOK * NP + 256 * b, at);
-            u.tot[b] = ld4(m + 3 * ST_TOK * NP + 16 * b, 4 * ch0);
+            for (int b = 0; b < BPW; ++b)
+                if (DELTA) u.kp[b] = at4(t.m, at, 4 * (2 * ST_TOK * NP + 256 * b));
+        } else if (part == 1) {
+#pragma unroll
+            for (int b = 0; b < BPW; ++b) u.qp[b] = at4(t.m, at, 4 * 256 * b);
+        } else if (part == 2) {
+#pragma unroll
+            for (int b = 0; b < BPW; ++b) u.tot[b] = at4(t.m, 4 * ch0, 4 * (3 * ST_TOK * NP + 16 * b));
+#pragma unroll
+            for (int r = 0; r < 4; ++r) u.v[r] = at1(t.v, at_v[r], 0);
+            if (DELTA) u.T = at4(t.m, at_T, 4 * (3 * ST_TOK * NP + NP + ST_PAIR));
+        } else {
+#pragma unroll
+            for (int b = 0; b < BPW; ++b) u.kd[b] = at4(t.m, at, 4 * (ST_TOK * NP + 256 * b));
+            u.B = at1(t.m, at_B, 4 * (3 * ST_TOK * NP + NP));
         }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) u.v[r] = ld1(vt, min((4 * g + r) * ldx4, vl) + vc);
-        u.B = ld1(m + 3 * ST_TOK * NP + NP, 4 * (c * ST_TOK + 4 * g + w));
-        if (DELTA) u.T = ld4(m + 3 * ST_TOK * NP + NP + ST_PAIR, 4 * (c * ST_TOK + 4 * g));
+        __builtin_amdgcn_sched_barrier(0);
     };
     // a tile's read-out, once every wave's share lies in LDS: wave w stores the tokens 4 g + w
-    float* obase = p.out + r0 * p.ldo + a * P + col;
-    auto store = [&](int i) {
-        const int t = ST_TOK * i + 4 * g + w;
-        const float* y = (const float*)&sY[i & 1][0][lane] + w;
-        const float o = (y[0] + y[256]) + (y[512] + y[768]);
-        if (cok && t < (int)(r1 - r0)) obase[t * p.ldo] = DELTA ? o : o * p.q_scale;
+    float* o_next = p.out + (r0 + 4 * g + w) * p.ldo + a * P + col;
+    const int64_t ostep = ST_TOK * p.ldo;
+    auto store = [&](const float y[4], int rows) {
+        const float o = (y[0] + y[1]) + (y[2] + y[3]);
+        if (cok && 4 * g + w < rows) *o_next = DELTA ? o : o * p.q_scale;
+        o_next += ostep;
     };
     // M v over the tokens up to and with a row's own, term by term: the terms from `first` on, every `stride`th
     auto below = [&](const float* M, const stf4& v, int first, int stride, stf4 o) {
+        const __amdgpu_buffer_rsrc_t m = st_buffer(M, 4 * ST_PAIR);
+        int g4 = 4 * g;
+        asm volatile("" : "+v"(g4));      // (its addresses are not kept in registers through all tiles)
 #pragma unroll 1
         for (int s = first; s < ST_TOK; s += stride) {
             const float lo = (s & 1) ? v[1] : v[0], hi = (s & 1) ? v[3] : v[2];
             const float vs = __shfl((s & 2) ? hi : lo, 16 * (s >> 2) + c);
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                if (s <= 4 * g + r) o[r] = fmaf(M[(4 * g + r) * ST_TOK + s], vs, o[r]);
+                if (s <= g4 + r) o[r] = fmaf(at1(m, 4 * ((g4 + r) * ST_TOK + s), 0), vs, o[r]);
         }
         return o;
     };
+    // What a tile waits for is its chain, so whatever else there is stands where the chain waits: the read-out's products around the exchange of the shares of
+    // k P S, the sums and stores of the tile before behind the barrier that this exchange needs, the state times P_16 in front of its last products.
+    stf4 O = (stf4)0.0f;      // a wave's share of the read-out of the tile before
     auto tile = [&](int i, const Ops& o, Ops& ahead) {
         const int pb = i & 1;
-        load(i + 2, ahead);
+        const Tile next = where(i + SETS - 1);
         if constexpr (DELTA) {
             stf4 x[2] = {(stf4)0.0f, (stf4)0.0f};
 #pragma unroll
             for (int r = 0; r < 4; ++r)
 #pragma unroll
                 for (int b = 0; b < BPW; ++b) x[b & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kp[b][r], S[b][r], x[b & 1], 0, 0, 0);
-            sX[pb][w][lane] = x[0] + x[1];
-        }
+            sY[pb][w][lane] = O;
+            load(next, ahead, 0);
+            sX[pb][w][lane] = BPW > 1 ? x[0] + x[1] : x[0];
+        } else sY[pb][w][lane] = O;
         stf4 y[2] = {(stf4)0.0f, (stf4)0.0f};
+        auto read_out = [&](int r0, int r1) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+            for (int r = r0; r < r1; ++r)
 #pragma unroll
-            for (int b = 0; b < BPW; ++b) y[b & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.qp[b][r], S[b][r], y[b & 1], 0, 0, 0);
+                for (int b = 0; b < BPW; ++b) y[b & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.qp[b][r], S[b][r], y[b & 1], 0, 0, 0);
+        };
+        read_out(0, 1);
         // one barrier a tile: LDS holds two tiles' shares, and the one that is written again was read in front of it
         __syncthreads();
-        stf4 V, W, U;
+        stf4 xs[4];
+        float ys[4];
+        if constexpr (DELTA) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) V[r] = o.v[r];
-        W = V;
-        if constexpr (DELTA) W = V - ((sX[pb][0][lane] + sX[pb][1][lane]) + (sX[pb][2][lane] + sX[pb][3][lane]));
-        if (i == nt - 1) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) W[r] = 4 * g + r < rows_last ? W[r] : 0.0f;
+            for (int j = 0; j < 4; ++j) xs[j] = sX[pb][j][lane];
         }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) ys[j] = ((const float*)&sY[pb][j][lane])[w];
+        load(next, ahead, 1);
+        read_out(1, 4);
+        load(next, ahead, 2);
+#pragma unroll
+        for (int b = 0; b < BPW; ++b) S[b] = S[b] * o.tot[b];
+        stf4 W, U;      // (rows behind the run's end: no value, no key, no write strength)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) W[r] = o.v[r];
+        if constexpr (DELTA) W = W - ((xs[0] + xs[1]) + (xs[2] + xs[3]));
+        // a sum over all 16 tokens would carry what is no finite number to tokens in front of it, through a zero: such a tile is summed term by term
+        auto odd = [](const stf4& x) { return __ballot(!((fabsf(x[0]) + fabsf(x[1])) + (fabsf(x[2]) + fabsf(x[3])) < INFINITY)) != 0; };
+        const float* pr = tiles + i * tstep + 3 * ST_TOK * NP + NP;
         U = W;
         if constexpr (DELTA) {
             stf4 u0 = (stf4)0.0f, u1 = (stf4)0.0f;
@@ -376,49 +427,43 @@ __global__ __launch_bounds__(256, BPW > 2 ? 1 : 2) void scan_tile_kernel(const i
             u1 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.T[2], W[2], u1, 0, 0, 0);
             u0 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.T[1], W[1], u0, 0, 0, 0);
             u1 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.T[3], W[3], u1, 0, 0, 0);
+            if (odd(W)) u0 = below(pr + ST_PAIR, W, 0, 1, (stf4)0.0f), u1 = (stf4)0.0f;
             U = u0 + u1;
         }
-        // a sum over all 16 tokens would carry what is no finite number to tokens in front of it, through a zero: such a tile is summed term by term
-        float mag = 0.0f;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) mag += DELTA ? fabsf(W[r]) + fabsf(U[r]) : fabsf(U[r]);
-        const bool odd = __ballot(!(mag < INFINITY)) != 0;
-        const float* pr = tiles + i * tstep + 3 * ST_TOK * NP + NP;
-        if (DELTA && odd) U = below(pr + ST_PAIR, W, 0, 1, (stf4)0.0f);
-#pragma unroll
-        for (int b = 0; b < BPW; ++b) S[b] = S[b] * o.tot[b];
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
             for (int b = 0; b < BPW; ++b) S[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kd[b][r], U[r], S[b], 0, 0, 0);
+        load(next, ahead, 3);
+        if (i > 0) store(ys, ST_TOK);
         // a wave's share of the read-out: its channels of the state, and every fourth token's write
-        stf4 O = y[0] + y[1];
-        if (odd) O = below(pr, U, w, 4, O);
+        O = BPW > 1 ? y[0] + y[1] : y[0];
+        if (odd(U)) O = below(pr, U, w, 4, O);
         else O = __builtin_amdgcn_mfma_f32_16x16x4f32(o.B, w == 0 ? U[0] : (w == 1 ? U[1] : (w == 2 ? U[2] : U[3])), O, 0, 0, 0);
-        if (i > 0) store(i - 1);
-        sY[pb][w][lane] = O;
     };
-    Ops A, B, C;
-    // (the sets' loads stay apart: waiting for one must not wait for the next)
-#define ST_APART                       \
-    asm volatile("" ::: "memory");     \
-    __builtin_amdgcn_sched_barrier(0);
-    ST_APART
-    load(0, A);
-    ST_APART
-    load(1, B);
-    ST_APART
-#undef ST_APART
-    int i = 0;
-    for (; i + 3 <= nt; i += 3) {      // (not left in the middle: round the loop every set is as many loads behind the next)
-        tile(i, A, C);
-        tile(i + 1, B, A);
-        tile(i + 2, C, B);
+    Ops u[SETS];
+#pragma unroll
+    for (int j = 0; j < SETS - 1; ++j) {      // (the sets' loads stay apart: waiting for one must not wait for the next)
+        const Tile t = where(j);
+#pragma unroll
+        for (int part = 0; part < 4; ++part) load(t, u[j], part);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
     }
-    if (i < nt) tile(i, A, C);
-    if (i + 1 < nt) tile(i + 1, B, A);
+    int i = 0;
+    for (; i + SETS <= nt; i += SETS) {      // (not left in the middle: round the loop every set is as many loads behind the next)
+#pragma unroll
+        for (int j = 0; j < SETS; ++j) tile(i + j, u[j], u[(j + SETS - 1) % SETS]);
+    }
+#pragma unroll
+    for (int j = 0; j < SETS - 1; ++j)
+        if (i + j < nt) tile(i + j, u[j], u[(j + SETS - 1) % SETS]);
+    sY[nt & 1][w][lane] = O;
     __syncthreads();
-    store(nt - 1);
+    float ys[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) ys[j] = ((const float*)&sY[nt & 1][j][lane])[w];
+    store(ys, rows_last);
 #pragma unroll
     for (int b = 0; b < BPW; ++b)
         if (cok && ch0 + 16 * b < N) *(stf4*)(gS + ch0 + 16 * b) = S[b];
