@@ -511,6 +511,7 @@ typedef struct {
     float q_scale;       /* multiplies the read-out S^T q (scan only) */
     float* work;         /* as in i64h_gdn_args */
     int64_t work_floats;
+    int32_t longest;     /* scan only: rows of the longest run, 0 where the caller does not know it (the form is then chosen by the runs' mean) */
 } i64h_gla_args;
 int i64h_gla_gates(const i64h_gla_args* d, void* stream);
 int i64h_gla_scan(const i64h_gla_args* d, void* stream);
@@ -597,6 +598,7 @@ typedef struct {
     int64_t ldf;
     float* work;         /* scan only, may be NULL: at least i64h_scan_work_floats floats, 16-byte aligned - long runs may then be summed in tiles */
     int64_t work_floats;
+    int32_t longest;     /* scan only: rows of the longest run, 0 where the caller does not know it (the form is then chosen by the runs' mean) */
 } i64h_gdn_args;
 int i64h_gdn_gates(const i64h_gdn_args* d, void* stream);
 int i64h_gdn_scan(const i64h_gdn_args* d, void* stream);
@@ -640,8 +642,10 @@ int i64h_rec_step(const i64h_rec_step_args* d, void* stream);
 int i64h_rec_tiles(const i64h_rec_step_args* d, const i64h_gdn_args* s, void* stream);
 int64_t i64h_scan_work_floats(int64_t n, int32_t nseg, int32_t heads, int32_t dim);
 /* Whether either scan (delta != 0: i64h_gdn_scan, else i64h_gla_scan with keys of its own) of nseg runs of n rows, the longest of `longest` rows, is the
- * faster in tiles, and a caller that knows its runs should give it a workspace.  The launch itself knows n and nseg only. */
+ * faster in tiles, and a caller that knows its runs should give it a workspace. */
 int32_t i64h_scan_in_tiles(int64_t n, int32_t nseg, int32_t longest, int32_t heads, int32_t dim, int32_t vdim, int32_t delta);
+/* The same of i64h_rec_tiles against the launches that it stands for: it has more to save. */
+int32_t i64h_rec_in_tiles(int64_t n, int32_t nseg, int32_t longest, int32_t heads, int32_t dim, int32_t vdim, int32_t delta);
 int i64h_set_gdn_scan_form(int32_t form); /* tuning / test knob: 0 (default) = by the runs' length; 1 = loads straight into registers; 2, 3, 4 = staged
                                              through LDS with 1, 2, 4 value columns per lane (where 16-byte rows allow); same results bit for bit.
                                              5 = tiles of 16 tokens whatever the runs' length (with work, 16-byte rows, keys of their own) */

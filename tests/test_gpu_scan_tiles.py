@@ -139,3 +139,47 @@ def test_the_longest_runs_choose_the_tiles_and_need_their_workspace(dev):
     with pytest.raises(_lib.I64HError):
         D.gdn_scan(X.to(dev), Gt.to(dev), f=F.to(dev), q_off=0, k_off=64, v_off=128, heads=2, kv_heads=2, dim=32, vdim=16, seg_start=r.seg, nseg=r.nseg, positions=r.pos,
                    slot_ids=r.slots, state=S0.to(dev), out=torch.empty(r.n, 32, device=dev), n=r.n, work=torch.empty(16, device=dev))
+
+
+@pytest.mark.parametrize("delta", [True, False])
+@pytest.mark.parametrize("singles,length,form", [(6, 15, 1), (6, 16, 2), (2, 40, 2), (3, 80, 2), (3, 120, 5)])
+def test_single_rows_beside_a_prompt_whose_length_is_told(dev, delta, singles, length, form):
+    """The longest run decides the form where the caller tells it, whatever the mean is: the bits are that form's, and the recurrence's in 64 bits."""
+    from vllm_i64_amd import _lib, ops_dense as D
+    H, d, dv = 4, 128, 16
+    r = Rows(dev, [(1 + i, 9, 1) for i in range(singles)] + [(0, 0, length)])
+    X, Gt, F, _ = inputs((H, H, d, dv), r.n, length, 0.9)
+    S0 = torch.randn(singles + 1, H, dv, d, generator=torch.Generator().manual_seed(1))
+    got = []
+    for forced, longest in ((0, length), (form, 0)):
+        S, O = S0.to(dev).clone(), torch.full((r.n, H * dv), 7.0, device=dev)
+        cols = dict(heads=H, dim=d, vdim=dv, seg_start=r.seg, nseg=r.nseg, positions=r.pos, slot_ids=r.slots, state=S, out=O, n=r.n, longest=longest,
+                    work=torch.full((D.scan_work_floats(r.n, r.nseg, H, d),), float("nan"), device=dev))
+        try:
+            _lib.call_dense("i64h_set_gdn_scan_form", forced)
+            if delta:
+                D.gdn_scan(X.to(dev), Gt.to(dev), f=F.to(dev), q_off=0, k_off=H * d, v_off=2 * H * d, kv_heads=H, **cols)
+            else:
+                D.gla_scan(X.to(dev), f=F.to(dev), q_off=0, k_off=H * d, f_off=0, v_off=2 * H * d, q_scale=0.3, **cols)
+        finally:
+            _lib.call_dense("i64h_set_gdn_scan_form", 0)
+        got.append((O.cpu(), S.cpu()))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    for slot, at, c, fresh in ((0, singles, length, True), (2, 1, 1, False)):
+        x = X[at:at + c].double()
+        o, s = recurrence((1.0 if delta else 0.3) * x[:, :H * d].reshape(c, H, d), x[:, H * d:2 * H * d].reshape(c, H, d), x[:, 2 * H * d:].reshape(c, H, dv),
+                          Gt[at:at + c, :H].double() if delta else None, F[at:at + c].double().reshape(c, H, d), torch.zeros(H, dv, d, dtype=F64) if fresh else S0[slot].double())
+        assert err(got[0][0][at:at + c], o.reshape(c, H * dv)) < TOL and err(got[0][1][slot], s) < TOL
+
+
+def test_the_forms_rules():
+    """Runs are worth tiles from a length on that grows with their number, earlier from the projections; what the rules take they take for longer runs too."""
+    from vllm_i64_amd import ops_dense as D
+    for delta in (True, False):
+        for H, d, dv in ((16, 128, 128), (8, 128, 128), (8, 64, 64), (4, 256, 64), (3, 70, 16)):
+            for singles in (0, 7, 40):
+                took = [(D.scan_in_tiles(singles + L, singles + 1, L, H, d, dv, delta=delta), D.rec_in_tiles(singles + L, singles + 1, L, H, d, dv, delta=delta)) for L in range(1, 1200)]
+                assert all(b or not a for a, b in took)      # (alone: from the projections too)
+                for rule in range(2):
+                    on = [t[rule] for t in took]
+                    assert on == sorted(on) and not on[0] and on[-1] == (d % 4 == 0)

@@ -359,14 +359,14 @@ class Gdn(ctypes.Structure):
     _fields_ = [("X", _P), ("ldx", _L), ("q_off", _I), ("k_off", _I), ("v_off", _I), ("heads", _I), ("kv_heads", _I), ("dim", _I), ("vdim", _I),
                 ("G", _P), ("R", _P), ("ldr", _L), ("b_off", _I), ("a_off", _I), ("A_log", _P), ("dt_bias", _P), ("unit_eps", _F), ("q_scale", _F),
                 ("seg_start", _P), ("nseg", _I), ("positions", _P), ("slot_ids", _P), ("state", _P), ("out", _P), ("ldo", _L), ("n", _L),
-                ("F", _P), ("ldf", _L), ("work", _P), ("work_floats", _L)]
+                ("F", _P), ("ldf", _L), ("work", _P), ("work_floats", _L), ("longest", _I)]
 
 
 class Gla(ctypes.Structure):
     """Mirror of i64h_gla_args (include/i64h_dense.h)."""
     _fields_ = [("P", _P), ("ldp", _L), ("q_off", _I), ("f_off", _I), ("k_off", _I), ("v_off", _I), ("heads", _I), ("dim", _I), ("vdim", _I),
                 ("lower", _P), ("q_act", _I), ("seg_start", _P), ("nseg", _I), ("positions", _P), ("slot_ids", _P), ("state", _P), ("out", _P),
-                ("ldo", _L), ("n", _L), ("F", _P), ("ldf", _L), ("q_scale", _F), ("work", _P), ("work_floats", _L)]
+                ("ldo", _L), ("n", _L), ("F", _P), ("ldf", _L), ("q_scale", _F), ("work", _P), ("work_floats", _L), ("longest", _I)]
 
 
 class RecStep(ctypes.Structure):
@@ -397,7 +397,7 @@ _dense: Optional[ctypes.CDLL] = None
 
 
 def dense_exported_symbols():
-    return ["i64h_last_error", "i64h_version", "i64h_device_check", "i64h_latent_attn_workspace_floats", "i64h_kattn_workspace_floats", "i64h_scan_work_floats", "i64h_scan_in_tiles", "i64h_linear_form", *DENSE_SIGNATURES.keys()]
+    return ["i64h_last_error", "i64h_version", "i64h_device_check", "i64h_latent_attn_workspace_floats", "i64h_kattn_workspace_floats", "i64h_scan_work_floats", "i64h_scan_in_tiles", "i64h_rec_in_tiles", "i64h_linear_form", *DENSE_SIGNATURES.keys()]
 
 
 def load_dense() -> ctypes.CDLL:
@@ -414,8 +414,8 @@ def load_dense() -> ctypes.CDLL:
     lib.i64h_device_check.restype = _I
     lib.i64h_scan_work_floats.restype = _L
     lib.i64h_scan_work_floats.argtypes = [_L, _I, _I, _I]
-    lib.i64h_scan_in_tiles.restype = _I
-    lib.i64h_scan_in_tiles.argtypes = [_L, _I, _I, _I, _I, _I, _I]
+    for f in (lib.i64h_scan_in_tiles, lib.i64h_rec_in_tiles):
+        f.restype, f.argtypes = _I, [_L, _I, _I, _I, _I, _I, _I]
     lib.i64h_linear_form.restype = _I
     lib.i64h_linear_form.argtypes = [_P]
     lib.i64h_latent_attn_workspace_floats.restype = _L

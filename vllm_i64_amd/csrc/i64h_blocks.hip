@@ -634,15 +634,29 @@ int i64h_set_gdn_scan_form(int32_t form) {
 }
 
 // Tiles of 16 tokens on the matrix cores are two launches and a tile costs the same however few rows it holds; token by token a launch takes as long as
-// its longest run.  So it is the longest run that decides.  Microseconds in replayed graphs, token by token | in tiles, delta rule (linear attention), heads
-// of 128: 16 heads, a run of 1531 rows 242 | 130 (218 | 83), of 160 29 | 23 (27 | 17), of 96 18.5 | 18.9 (17 | 14), 30 single rows beside 300 78 | 61 (67 | 44);
-// 8 heads, 8 runs of 512 120 | 82 (100 | 57), 20 single rows beside 128 33 | 35 (27 | 25); 8 heads of 64, 8 runs of 17 5.6 | 11.6 (5.0 | 9.0), 16 of 64
-// 14.7 | 17.8 (12.2 | 13.3), 4 of 96 14.0 | 15.4 (11.4 | 11.8).  Narrow heads in thousands of workgroups are little more than their reads either way (32 heads of 64, 32 runs of
-// 192 rows 172 | 187, 121 | 139), as are many short runs (64 of 17 rows 43 | 62).
+// its longest run.  So it is the longest run that decides, against the number of runs, each a tile at least - unless the runs are long on the average.  Microseconds
+// in replayed graphs, token by token | in tiles, delta rule (linear attention), heads of 128: 16 heads, a run of 1531 rows 242 | 107 (215 | 71), of 160 29 | 21 (27 | 16), of 96
+// 18.8 | 18.0 (16.9 | 14.0), of 64 13.4 | 16.0 (12.3 | 12.7), 30 single rows beside 300 64 | 57 (56 | 46), 40 beside 200 57 | 63 (52 | 51), beside 280 74 | 66 (64 | 54), 20 beside 128
+// 37 | 40 (31 | 32); 8 heads, 8 runs of 512 125 | 77 (99 | 54), 40 single rows beside 200 43 | 43 (40 | 34), 20 beside 128 26 | 28 (24 | 24), 4 runs of 64 14.4 | 16.8 (13.8 | 13.3);
+// 8 heads of 64, 8 runs of 17 5.6 | 11.9 (5.0 | 9.3), 16 of 64 14.6 | 16.6 (11.6 | 12.2), 4 of 96 13.9 | 14.4 (11.3 | 10.9).  Narrow heads in thousands of workgroups are little more than
+// their reads either way (32 heads of 64, 32 runs of 192 rows 193 | 182, 140 | 135), as are many short runs (64 of 17 rows 39 | 53).
 int32_t i64h_scan_in_tiles(int64_t n, int32_t nseg, int32_t longest, int32_t heads, int32_t dim, int32_t vdim, int32_t delta) {
     const int64_t groups = (int64_t)heads * ((vdim + 15) / 16) * nseg;      // workgroups of the second launch
-    return dim % 4 == 0 && dim <= 256 && n >= 96 && n >= 8 * (int64_t)nseg && longest >= (delta ? 144 : 112) && (n >= 32 * (int64_t)nseg || groups < 6144) &&
-           (dim > 64 || groups <= 2048);
+    const int64_t least = delta ? 100 + (int64_t)nseg * heads / 4 : 80 + (int64_t)nseg * heads * 3 / 16;
+    return dim % 4 == 0 && dim <= 256 && n >= 96 && (longest >= least || (n >= 32 * (int64_t)nseg && longest >= (delta ? 144 : 112))) &&
+           (n >= 32 * (int64_t)nseg || groups < 6144) && (dim > 64 || groups <= 2048);
+}
+
+// From the projections three launches stand for four or six that read and write the rows between them, so tiles pay earlier.  Microseconds as above, in launches of their own token
+// by token | in tiles: 16 heads of 128, a run of 32 rows 27 | 26 (14.5 | 17), of 48 31 | 27 (17.4 | 17.6), of 96 45 | 30 (26 | 20), 12 single rows beside 48 38 | 41 (22 | 29), beside 80
+// 48 | 45 (29 | 31), 40 beside 100 71 | 77 (46 | 57), beside 200 95 | 85 (63 | 63), beside 280 118 | 91 (78 | 67), 64 beside 200 103 | 108 (68 | 82), beside 400 149 | 123 (98 | 90), 32 runs of
+// 17 85 | 79 (52 | 56), 64 of 17 128 | 132 (86 | 94), 16 of 24 74 | 56 (41 | 39), 32 of 32 110 | 87 (69 | 59); 8 heads, 40 beside 100 53 | 53 (34 | 38), beside 150 64 | 56 (41 | 40), 12 beside
+// 48 32 | 32 (19 | 23); 32 heads of 64, a run of 32 26 | 22, 40 beside 150 66 | 72, 64 beside 400 113 | 109.
+int32_t i64h_rec_in_tiles(int64_t n, int32_t nseg, int32_t longest, int32_t heads, int32_t dim, int32_t vdim, int32_t delta) {
+    const int64_t groups = (int64_t)heads * ((vdim + 15) / 16) * nseg;
+    const int64_t least = delta ? 28 + (int64_t)nseg * (8 + heads) / 8 : 50 + (int64_t)nseg * heads / 4;
+    return i64h_scan_in_tiles(n, nseg, longest, heads, dim, vdim, delta) ||
+           (dim % 4 == 0 && dim <= 128 && (longest >= least || (n >= 128 && n >= 24 * (int64_t)nseg)) && (dim > 64 || groups <= 2048));
 }
 
 // the recurrence's launch, with the delta rule's correction or (a decay per key channel, every head its own keys) without it
@@ -655,14 +669,18 @@ static int gdn_launch(const i64h_gdn_args& d, void* stream) {
                (!d.F || (d.ldf % 4 == 0 && (uintptr_t)d.F % 16 == 0));
     };
     const int kround = kpt <= 4 ? 4 : (kpt <= 8 ? 8 : 16);
-    const bool tiles = i64h_scan_in_tiles(d.n, d.nseg, INT32_MAX, d.heads, d.dim, d.vdim, RULE == GD_DELTA);
+    // runs nobody measured: the mean says whether one of them may be long
+    const bool several = d.n >= 8 * (int64_t)d.nseg;
+    const bool tiles = (d.longest > 0 || several) && i64h_scan_in_tiles(d.n, d.nseg, d.longest > 0 ? d.longest : INT32_MAX, d.heads, d.dim, d.vdim, RULE == GD_DELTA);
     if (RULE != GD_FORGET && d.work && ((g_gdn_form == 0 && tiles) || g_gdn_form == 5) && vec_ok(4) && (uintptr_t)d.work % 16 == 0 && d.ldx < (1 << 25) &&
         (d.n / 16 + d.nseg) * (int64_t)d.heads < (1ll << 31)) {
         I64H_CHECK_ARG(d.work_floats >= i64h_scan_work_floats(d.n, d.nseg, d.heads, d.dim), "scan: a workspace of %lld floats, %lld needed", (long long)d.work_floats,
                        (long long)i64h_scan_work_floats(d.n, d.nseg, d.heads, d.dim));
         return i64h_scan_tiles(d, RULE == GD_DELTA, stream);
     }
-    if (g_gdn_form != 1 && vec_ok(kround) && (g_gdn_form > 1 || d.n >= 8 * (int64_t)d.nseg)) {
+    // Staged through LDS, 16 tokens at a time, from a mean of eight rows a run or one run of 16 on: 16 heads, linear attention (delta rule), straight into registers | staged, 40 single rows
+    // beside 17 rows 23 | 22 us (24 | 23), beside 100 64 | 35 (75 | 39), beside 280 155 | 64 (184 | 74), 3 beside 20 13.5 | 7.1 (15.8 | 7.7); 32 runs of 7 24 | 25 (26.5 | 27.7), 64 of 3 27 | 32 (28 | 35).
+    if (g_gdn_form != 1 && vec_ok(kround) && (g_gdn_form > 1 || several || d.longest >= 16)) {
         // One value column per lane: a token then takes the longest run least time, and it is the longest run that the launch waits for (16
         // heads of 128, runs of 1531, 257, 64, 3 and 1101 rows: 264 us, two columns 448; 27 single rows beside 229 and 256: 68 and 100).  Two
         // columns (fewer reads of the tile) only where many workgroups wait for a CU and the runs are long (8 runs of 512 rows: 220 and 199 us, 32 of 128
@@ -738,7 +756,7 @@ int i64h_gla_scan(const i64h_gla_args* dp, void* stream) {
     a.X = d.P, a.ldx = d.ldp, a.q_off = d.q_off, a.k_off = d.k_off >= 0 ? d.k_off : 0, a.v_off = d.v_off, a.heads = a.kv_heads = d.heads, a.dim = d.dim, a.vdim = d.vdim;
     a.F = (d.F ? d.F : d.P) + d.f_off, a.ldf = d.F ? d.ldf : d.ldp, a.q_scale = d.q_scale, a.seg_start = d.seg_start, a.nseg = d.nseg;
     a.positions = d.positions, a.slot_ids = d.slot_ids, a.state = d.state, a.out = d.out, a.ldo = d.ldo, a.n = d.n;
-    a.work = d.work, a.work_floats = d.work_floats;
+    a.work = d.work, a.work_floats = d.work_floats, a.longest = d.longest;
     return d.k_off >= 0 ? gdn_launch<GD_KEYS>(a, stream) : gdn_launch<GD_FORGET>(a, stream);
 }
 

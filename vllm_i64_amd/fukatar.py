@@ -147,12 +147,12 @@ class FukatarModel(HybridRunner):
         D.linear(B.h, d["w_in"], P, exact=self.exact)
         self._latent_attention(B, d, d["m"], P, l, n, positions, slot_ids, kvc, runs, ctx_hint, B.y)
 
-    def _parallel(self, B, d, l, n, positions, slot_ids, kvc, seg, nseg, runs, ctx_hint, single, work=NO_WORK) -> None:
+    def _parallel(self, B, d, l, n, positions, slot_ids, kvc, seg, nseg, runs, ctx_hint, single, work=NO_WORK, longest: int = 0) -> None:
         a, r = d["m"].left, d["m"].right
         P = B.p[: n * d["n_in"]].view(n, d["n_in"])
         D.linear(B.h, d["w_in"], P, exact=self.exact)
         self._rotary_attention(B, d, a, P, l, n, positions, slot_ids, kvc, runs, ctx_hint, B.y, nseg=nseg)
-        self._gated_delta(B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, single, B.y2, work)
+        self._gated_delta(B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, single, B.y2, work, longest)
 
     @torch.no_grad()
     def forward(self, token_ids: torch.Tensor, positions: torch.Tensor, slot_ids: torch.Tensor, ctx_len: Optional[torch.Tensor] = None,
@@ -196,7 +196,7 @@ class FukatarModel(HybridRunner):
             elif d["type"] == "attention":
                 self._attention(B, d, l, n, positions, slot_ids, kvc, runs, hint, nseg)
             else:
-                self._parallel(B, d, l, n, positions, slot_ids, kvc, seg, nseg, runs, hint, single, work)
+                self._parallel(B, d, l, n, positions, slot_ids, kvc, seg, nseg, runs, hint, single, work, longest)
                 write.update(y2=B.y2, yn_w=d["out_left"], y2n_w=d["out_right"])
             D.streams_step(B.streams, **write)
             if d["mlp"] is not None:

@@ -201,10 +201,11 @@ class HybridRunner:
         return splits, ws
 
     def _scan_work(self, n: int, nseg: int, longest: int, scans, delta: bool) -> Dict[tuple, torch.Tensor]:
-        """The workspace of a step's scans by (heads, dim, vdim), for those of `scans` whose runs are worth the form that takes one.  The caller holds it for
+        """The workspace of a step's scans by (heads, dim, vdim), for those of `scans` whose runs are worth the form that takes one, alone or from the projections.  The caller holds it for
         the step and no longer: 27 KB a tile of 16 rows and head of 128 would otherwise lie beside every kept buffer set.  Where the card has no room for
         it the scans go token by token: the same values in another order of the sums."""
-        sizes = {s: D.scan_work_floats(n, nseg, s[0], s[1]) for s in scans if D.scan_in_tiles(n, nseg, longest, *s, delta=delta)}
+        worth = D.scan_in_tiles if self.exact else D.rec_in_tiles
+        sizes = {s: D.scan_work_floats(n, nseg, s[0], s[1]) for s in scans if worth(n, nseg, longest, *s, delta=delta)}
         if not sizes:
             return {}
         try:
@@ -341,7 +342,7 @@ class HybridRunner:
         return True
 
     # ---- gated linear attention ----
-    def _gated_linear(self, B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, out, scale: float = 1.0, work=NO_WORK) -> None:
+    def _gated_linear(self, B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, out, scale: float = 1.0, work=NO_WORK, longest: int = 0) -> None:
         """Gated linear attention on the projection rows P (columns d["rq_off"], d["rk_off"], d["rv_off"], d["rg_off"]: queries, keys, values, output
         gates; d["a1_off"]: the low-rank decay map's first factor).  sigmoid(z)^(1 / tau) = exp(-softplus(-z) / tau): the second factor and
         its bias are held negated, the exponent's rate is d["a_rate"]."""
@@ -358,12 +359,12 @@ class HybridRunner:
         D.linear(P, d["a2"], F, m=n, a_off=d["a1_off"], exact=self.exact, bias=d["a2_b"], epilogue=D.EPI_DECAY, e=d["a_rate"])
         D.gla_scan(P, f=F, q_off=d["rq_off"], k_off=d["rk_off"], f_off=0, v_off=d["rv_off"], heads=r.heads, dim=r.dim, vdim=r.vdim, seg_start=seg, nseg=nseg,
                    positions=positions, slot_ids=slot_ids, state=kvc.state[l]["gla"], out=R, n=n, q_scale=r.dim ** -0.5,
-                   work=work.get((r.heads, r.dim, r.vdim)))
+                   work=work.get((r.heads, r.dim, r.vdim)), longest=longest)
         D.gate_norm(R, d["r_norm"], Rn, groups=r.heads, eps=self.cfg.norm_eps, z=P, z_off=d["rg_off"], ldz=P.shape[-1], n=n, gate_after=True, width=rv, out16=Rn16)
         self._out(Rn, d["o_right"], out, scale, Rn16)
 
     # ---- gated delta rule ----
-    def _gated_delta(self, B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, single: bool, out, work=NO_WORK) -> None:
+    def _gated_delta(self, B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, single: bool, out, work=NO_WORK, longest: int = 0) -> None:
         """Gated delta rule on the projection rows P: the convolved parts q | k | v from column d["r_off"] on, the write strength's at
         d["rb_off"].  A decay per head comes from the columns d["ra_off"]; a decay per key channel (r.decay 'channel') and its output gate are
         low-rank maps whose first factors' results lie at d["a1_off"] and d["g1_off"]."""
@@ -393,7 +394,7 @@ class HybridRunner:
             D.linear(P, d["a2"], F, m=n, a_off=d["a1_off"], exact=ex, bias=d["dt_bias"], epilogue=D.EPI_DECAY, e=d["a_rate"])
             D.linear(P, d["g2"], Z, m=n, a_off=d["g1_off"], exact=ex)
         D.gdn_scan(X, G, f=F, seg_start=seg, nseg=nseg, positions=positions, slot_ids=slot_ids, state=st["gdn"], out=R,
-                   work=work.get((r.heads, r.dim, r.vdim)), **cols)
+                   work=work.get((r.heads, r.dim, r.vdim)), longest=longest, **cols)
         D.gate_norm(R, d["r_norm"], Rn, groups=r.heads, eps=self.cfg.norm_eps, z=Z, z_off=z_off, ldz=ldz, n=n, gate_after=True, width=rv, sigmoid=r.gate == "sigmoid", out16=Rn16)
         D.linear(Rn, d["o_right"], out, a16=Rn16, exact=ex)
 

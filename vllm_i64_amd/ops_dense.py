@@ -589,6 +589,11 @@ def scan_in_tiles(n: int, nseg: int, longest: int, heads: int, dim: int, vdim: i
     return bool(_lib.load_dense().i64h_scan_in_tiles(int(n), int(nseg), int(longest), int(heads), int(dim), int(vdim), int(bool(delta))))
 
 
+def rec_in_tiles(n: int, nseg: int, longest: int, heads: int, dim: int, vdim: int, *, delta: bool) -> bool:
+    """Whether rec_tiles over such runs is worth a workspace (see i64h_rec_in_tiles)."""
+    return bool(_lib.load_dense().i64h_rec_in_tiles(int(n), int(nseg), int(longest), int(heads), int(dim), int(vdim), int(bool(delta))))
+
+
 def _scan_work(work: Optional[torch.Tensor]) -> dict:
     if work is None:
         return {}
@@ -598,9 +603,9 @@ def _scan_work(work: Optional[torch.Tensor]) -> dict:
 
 def gdn_scan(x: torch.Tensor, g: torch.Tensor, *, q_off: int, k_off: int, v_off: int, heads: int, kv_heads: int, dim: int, vdim: int, seg_start: torch.Tensor,
              nseg: int, positions: torch.Tensor, slot_ids: torch.Tensor, state: torch.Tensor, out: torch.Tensor, n: int,
-             f: Optional[torch.Tensor] = None, work: Optional[torch.Tensor] = None) -> torch.Tensor:
+             f: Optional[torch.Tensor] = None, work: Optional[torch.Tensor] = None, longest: int = 0) -> torch.Tensor:
     """See i64h_gdn_scan.  state fp32 [slots, heads, vdim, dim]; out fp32 [n, heads * vdim]; f fp32 [n, heads * dim]: a decay per key channel;
-    work fp32 [scan_work_floats]: long runs may be summed in tiles."""
+    work fp32 [scan_work_floats]: long runs may be summed in tiles; longest: the longest run's rows, where they are known."""
     if f is not None:
         _chk(f, torch.float32, "f")
         if f.shape[-1] < heads * dim or f.numel() < n * f.shape[-1]:
@@ -612,7 +617,7 @@ def gdn_scan(x: torch.Tensor, g: torch.Tensor, *, q_off: int, k_off: int, v_off:
         raise _lib.I64HError("gdn_scan: shapes do not fit the sizes")
     d = _gdn_args(x, g, q_off=q_off, k_off=k_off, v_off=v_off, heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, n=n, seg_start=ptr(seg_start), nseg=nseg,
                   positions=ptr(positions), slot_ids=ptr(slot_ids), state=ptr(state), out=ptr(out), ldo=heads * vdim, F=ptr(f),
-                  ldf=f.shape[-1] if f is not None else 0, **_scan_work(work))
+                  ldf=f.shape[-1] if f is not None else 0, longest=longest, **_scan_work(work))
     call_dense("i64h_gdn_scan", _ref(d), _stream())
     return out
 
@@ -646,16 +651,16 @@ def gla_gates(p: torch.Tensor, *, q_off: int, f_off: int, v_off: int, heads: int
 
 def gla_scan(p: torch.Tensor, *, q_off: int, f_off: int, v_off: int, heads: int, dim: int, vdim: int, seg_start: torch.Tensor, nseg: int,
              positions: torch.Tensor, slot_ids: torch.Tensor, state: torch.Tensor, out: torch.Tensor, n: int, k_off: int = -1,
-             f: Optional[torch.Tensor] = None, q_scale: float = 1.0, work: Optional[torch.Tensor] = None) -> torch.Tensor:
+             f: Optional[torch.Tensor] = None, q_scale: float = 1.0, work: Optional[torch.Tensor] = None, longest: int = 0) -> torch.Tensor:
     """See i64h_gla_scan.  state fp32 [slots, heads, vdim, dim]; out fp32 [n, heads * vdim]; k_off < 0: the key is one minus the decay.
-    f fp32 [n, ld]: the decays, where they are no columns of p; q_scale multiplies the read-out; work: see gdn_scan."""
+    f fp32 [n, ld]: the decays, where they are no columns of p; q_scale multiplies the read-out; work, longest: see gdn_scan."""
     _chk(state, torch.float32, "state"), _chk(out, torch.float32, "out")
     _chk(seg_start, torch.int32, "seg_start"), _chk(positions, torch.int32, "positions"), _chk(slot_ids, torch.int32, "slot_ids")
     _rows_ok("gla_scan", n, positions, slot_ids)
     if tuple(state.shape[1:]) != (heads, vdim, dim) or out.numel() < n * heads * vdim or seg_start.numel() < nseg + 1:
         raise _lib.I64HError("gla_scan: shapes do not fit the sizes")
     d = _gla_args(p, q_off=q_off, f_off=f_off, v_off=v_off, heads=heads, dim=dim, vdim=vdim, k_off=k_off, n=n, f=f, q_scale=q_scale, seg_start=ptr(seg_start), nseg=nseg,
-                  positions=ptr(positions), slot_ids=ptr(slot_ids), state=ptr(state), out=ptr(out), ldo=heads * vdim, **_scan_work(work))
+                  positions=ptr(positions), slot_ids=ptr(slot_ids), state=ptr(state), out=ptr(out), ldo=heads * vdim, longest=longest, **_scan_work(work))
     call_dense("i64h_gla_scan", _ref(d), _stream())
     return out
 

@@ -193,7 +193,7 @@ class PukatarModel(HybridRunner):
             if d["type"] == "attention":
                 self._rotary_attention(B, d, d["m"], P, r, n, positions, slot_ids, kvc, runs, hint, B.y, nseg=nseg)
             else:
-                self._gated_delta(B, d, d["m"], P, r, n, positions, slot_ids, kvc, seg, nseg, single, B.y, work)
+                self._gated_delta(B, d, d["m"], P, r, n, positions, slot_ids, kvc, seg, nseg, single, B.y, work, longest)
             write = dict(y=B.y, out_w=self.ones1)
             if d["mlp"] is not None:
                 write.update(ff)

@@ -128,7 +128,7 @@ class VepelixModel(HybridRunner):
         return d
 
     # ---- sublayers: the input is B.h, the result lands in B.y (and B.y2, to be added) ----
-    def _mixer(self, B, d, r, n, positions, slot_ids, kvc, seg, nseg, runs, hint, h16=None, work=NO_WORK) -> dict:
+    def _mixer(self, B, d, r, n, positions, slot_ids, kvc, seg, nseg, runs, hint, h16=None, work=NO_WORK, longest: int = 0) -> dict:
         """Returns the operands of the residual's write.  h16: the input rows in bf16, read in B.h's place."""
         m = d["m"]
         P = B.p[: n * d["ld"]].view(n, d["ld"])
@@ -138,7 +138,7 @@ class VepelixModel(HybridRunner):
             return dict(y=B.y)
         with self._beside(n):      # attention and recurrence share nothing but the projection rows
             self._rotary_attention(B, d, m.left, P, r, n, positions, slot_ids, kvc, runs, hint, B.y, m.left_scale, nseg)
-        self._gated_linear(B, d, m.right, P, r, n, positions, slot_ids, kvc, seg, nseg, B.y2, m.right_scale, work)
+        self._gated_linear(B, d, m.right, P, r, n, positions, slot_ids, kvc, seg, nseg, B.y2, m.right_scale, work, longest)
         self._meet(n)
         return dict(y=B.y, y2=B.y2)
 
@@ -185,7 +185,7 @@ class VepelixModel(HybridRunner):
             elif t:
                 D.streams_step(x, y=B.xe[1], out_w=self.ones1, **normed(d["norm1"]))
             # (elsewhere the launch that wrote the residual has normed it)
-            write = self._mixer(B, d, r, n, positions, slot_ids, kvc, seg, nseg, runs, int(max_ctx_hint), B.h16, work)
+            write = self._mixer(B, d, r, n, positions, slot_ids, kvc, seg, nseg, runs, int(max_ctx_hint), B.h16, work, longest)
             write.update(out_w=self.ones1, y_scale=d["ls1"])
             if d["mlp"] is not None:
                 D.streams_step(x, **write, **(normed(d["norm2"]) if d["mlp"].kind == "dense" else read(d["norm2"], **self._moe_read(B, d, n, B.h, B.h16))))

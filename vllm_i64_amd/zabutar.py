@@ -133,7 +133,7 @@ class ZabutarModel(HybridRunner):
         return d
 
     # ---- mixers and feed-forwards: the sublayer input is B.hc; the result lands in B.y ----
-    def _hgrn2(self, B, d, l, n, positions, slot_ids, kvc, seg, nseg) -> None:
+    def _hgrn2(self, B, d, l, n, positions, slot_ids, kvc, seg, nseg, longest: int = 0) -> None:
         m, ex = d["m"], self.exact
         nk, nv = m.heads * m.dim, m.heads * m.vdim
         P = B.p[: n * d["n_in"]].view(n, d["n_in"])
@@ -141,7 +141,7 @@ class ZabutarModel(HybridRunner):
         cols = dict(q_off=0, f_off=nk, v_off=2 * nk, heads=m.heads, dim=m.dim, vdim=m.vdim, n=n)
         D.gla_gates(P, lower=d["lower"], q_act=True, **cols)
         O = B.a[: n * nv].view(n, nv)
-        D.gla_scan(P, seg_start=seg, nseg=nseg, positions=positions, slot_ids=slot_ids, state=kvc.state[l]["gla"], out=O, **cols)
+        D.gla_scan(P, seg_start=seg, nseg=nseg, positions=positions, slot_ids=slot_ids, state=kvc.state[l]["gla"], out=O, longest=longest, **cols)
         G = B.b[: n * nv].view(n, nv)
         D.gate_norm(O, d["norm"], G, groups=m.heads, eps=self.cfg.norm_eps, n=n)
         D.linear(G, d["o"], B.y, exact=ex)
@@ -183,7 +183,7 @@ class ZabutarModel(HybridRunner):
         if n == 0:
             return B.logits
         eps = cfg.norm_eps
-        seg, nseg, _ = self._runs(n, slot_ids, tokens_per_seq, rows_are_slots)
+        seg, nseg, longest = self._runs(n, slot_ids, tokens_per_seq, rows_are_slots)
         if tokens_per_seq is not None:
             runs = attention_segments(tokens_per_seq, n, self.ATTN_MAX_SEGMENTS)
         else:
@@ -203,7 +203,7 @@ class ZabutarModel(HybridRunner):
             elif q == 2:
                 self._moe_ff(B, d, n, B.hc, B.y, B.y2, record, f"l{l}")
             elif d["type"] == "hgrn2":
-                self._hgrn2(B, d, l, n, positions, slot_ids, kvc, seg, nseg)
+                self._hgrn2(B, d, l, n, positions, slot_ids, kvc, seg, nseg, longest)
             else:
                 self._attention(B, d, l, n, positions, slot_ids, kvc, runs, int(max_ctx_hint))
             write = dict(y=B.y, yn_w=d[f"norm{q}b"], y_eps=eps, out_w=self.ones1)
