@@ -227,7 +227,7 @@ __global__ __launch_bounds__(256) void gdn_tile_kernel(const i64h_gdn_args p, co
     const int N = p.dim, P = p.vdim;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int nlane = lane & 15, cl = lane >> 4;
-    const int a = blockIdx.x / ctiles, seg = blockIdx.y;
+    const int a = blockIdx.x / ctiles, seg = gd_run(p.seg_start, p.nseg, blockIdx.y);
     const int kh = a / (p.heads / p.kv_heads);
     const int wg0 = (blockIdx.x % ctiles) * WC, cw = (w * 4 + cl) * CPT, cbase = wg0 + cw;
     const int64_t r0 = p.seg_start[seg], r1 = p.seg_start[seg + 1];
@@ -634,29 +634,29 @@ int i64h_set_gdn_scan_form(int32_t form) {
 }
 
 // Tiles of 16 tokens on the matrix cores are two launches and a tile costs the same however few rows it holds; token by token a launch takes as long as
-// its longest run.  So it is the longest run that decides, against the number of runs, each a tile at least - unless the runs are long on the average.  Microseconds
-// in replayed graphs, token by token | in tiles, delta rule (linear attention), heads of 128: 16 heads, a run of 1531 rows 242 | 107 (215 | 71), of 160 29 | 21 (27 | 16), of 96
-// 18.8 | 18.0 (16.9 | 14.0), of 64 13.4 | 16.0 (12.3 | 12.7), 30 single rows beside 300 64 | 57 (56 | 46), 40 beside 200 57 | 63 (52 | 51), beside 280 74 | 66 (64 | 54), 20 beside 128
-// 37 | 40 (31 | 32); 8 heads, 8 runs of 512 125 | 77 (99 | 54), 40 single rows beside 200 43 | 43 (40 | 34), 20 beside 128 26 | 28 (24 | 24), 4 runs of 64 14.4 | 16.8 (13.8 | 13.3);
-// 8 heads of 64, 8 runs of 17 5.6 | 11.9 (5.0 | 9.3), 16 of 64 14.6 | 16.6 (11.6 | 12.2), 4 of 96 13.9 | 14.4 (11.3 | 10.9).  Narrow heads in thousands of workgroups are little more than
-// their reads either way (32 heads of 64, 32 runs of 192 rows 193 | 182, 140 | 135), as are many short runs (64 of 17 rows 39 | 53).
+// its longest run.  So it is the longest run that decides, against the number of runs, each a tile at least (in workgroups of the second launch) - unless the runs are long on the
+// average.  Microseconds in replayed graphs, token by token | in tiles, delta rule (linear attention), heads of 128: 16 heads, a run of 1531 rows 242 | 106 (215 | 71), of 160 28 | 21
+// (27 | 15), of 96 17.9 | 17.5 (17.1 | 13.0), of 64 13.5 | 15.7 (12.5 | 11.8), 40 single rows beside 200 39 | 44 (33 | 33), beside 280 51 | 46 (45 | 34), 20 beside 128 26 | 30 (23 | 22), 64 beside
+// 400 69 | 70 (60 | 48), 16 runs of 24 30 | 31 (27 | 22), 4 of 64 22 | 22 (19 | 15); 8 heads, 8 runs of 512 125 | 77 (96 | 52), 40 single rows beside 150 30 | 29 (26 | 21), 20 beside 128
+// 25 | 22 (22 | 17), 4 runs of 64 14.8 | 16.6 (13.9 | 12.6); 8 heads of 64, 8 runs of 17 5.6 | 11.9 (5.0 | 9.3), 16 of 64 14.6 | 16.6 (11.6 | 12.2), 4 of 96 13.9 | 14.4 (11.3 | 10.9).  Narrow
+// heads in thousands of workgroups are little more than their reads either way (32 heads of 64, 32 runs of 192 rows 193 | 182, 140 | 135; 40 single rows beside 280 38 | 36), as are many
+// short runs nobody measured (64 of 17 rows, delta rule 41 | 48).
 int32_t i64h_scan_in_tiles(int64_t n, int32_t nseg, int32_t longest, int32_t heads, int32_t dim, int32_t vdim, int32_t delta) {
     const int64_t groups = (int64_t)heads * ((vdim + 15) / 16) * nseg;      // workgroups of the second launch
-    const int64_t least = delta ? 100 + (int64_t)nseg * heads / 4 : 80 + (int64_t)nseg * heads * 3 / 16;
-    return dim % 4 == 0 && dim <= 256 && n >= 96 && (longest >= least || (n >= 32 * (int64_t)nseg && longest >= (delta ? 144 : 112))) &&
-           (n >= 32 * (int64_t)nseg || groups < 6144) && (dim > 64 || groups <= 2048);
+    const bool even = n >= 32 * (int64_t)nseg, known = longest < INT32_MAX;
+    const bool worth = longest >= (delta ? 92 + groups / 30 : 60 + groups / 38) || (even && longest >= (delta ? 144 : 112)) || (!delta && dim > 64 && known && n >= 128 && n >= 24 * (int64_t)nseg);
+    return dim % 4 == 0 && dim <= 256 && n >= (known ? 64 : 96) && worth && (known || even || groups < 6144) && (dim > 64 || groups <= 2048);
 }
 
 // From the projections three launches stand for four or six that read and write the rows between them, so tiles pay earlier.  Microseconds as above, in launches of their own token
-// by token | in tiles: 16 heads of 128, a run of 32 rows 27 | 26 (14.5 | 17), of 48 31 | 27 (17.4 | 17.6), of 96 45 | 30 (26 | 20), 12 single rows beside 48 38 | 41 (22 | 29), beside 80
-// 48 | 45 (29 | 31), 40 beside 100 71 | 77 (46 | 57), beside 200 95 | 85 (63 | 63), beside 280 118 | 91 (78 | 67), 64 beside 200 103 | 108 (68 | 82), beside 400 149 | 123 (98 | 90), 32 runs of
-// 17 85 | 79 (52 | 56), 64 of 17 128 | 132 (86 | 94), 16 of 24 74 | 56 (41 | 39), 32 of 32 110 | 87 (69 | 59); 8 heads, 40 beside 100 53 | 53 (34 | 38), beside 150 64 | 56 (41 | 40), 12 beside
-// 48 32 | 32 (19 | 23); 32 heads of 64, a run of 32 26 | 22, 40 beside 150 66 | 72, 64 beside 400 113 | 109.
+// by token | in tiles: 16 heads of 128, a run of 32 rows 27 | 26 (14.6 | 16.3), of 64 36 | 28 (20 | 17), of 96 44 | 29 (26 | 19), 8 single rows beside 40 33 | 32 (18 | 20), beside 60 39 | 33 (22 | 21),
+// 20 beside 64 42 | 44 (24 | 28), beside 100 51 | 45 (29 | 29), 40 beside 100 58 | 61 (36 | 40), beside 150 65 | 64 (39 | 43), beside 200 75 | 66 (45 | 44), 64 beside 200 82 | 86 (53 | 59), beside 400
+// 114 | 95 (73 | 62), 32 runs of 17 85 | 73 (53 | 48), 16 of 24 73 | 52 (41 | 34); 8 heads, 40 beside 48 38 | 43 (22 | 27), beside 100 47 | 43 (28 | 27), 20 beside 64 36 | 32 (21 | 21);
+// 32 heads of 64, a run of 32 26 | 22, 40 beside 100 52 | 53, 20 beside 64 37 | 36.
 int32_t i64h_rec_in_tiles(int64_t n, int32_t nseg, int32_t longest, int32_t heads, int32_t dim, int32_t vdim, int32_t delta) {
     const int64_t groups = (int64_t)heads * ((vdim + 15) / 16) * nseg;
-    const int64_t least = delta ? 28 + (int64_t)nseg * (8 + heads) / 8 : 50 + (int64_t)nseg * heads / 4;
     return i64h_scan_in_tiles(n, nseg, longest, heads, dim, vdim, delta) ||
-           (dim % 4 == 0 && dim <= 128 && (longest >= least || (n >= 128 && n >= 24 * (int64_t)nseg)) && (dim > 64 || groups <= 2048));
+           (dim % 4 == 0 && dim <= 128 && (longest >= (delta ? 28 + groups / 48 : 44 + groups / 36) || (n >= 128 && n >= 16 * (int64_t)nseg)) && (dim > 64 || groups <= 2048));
 }
 
 // the recurrence's launch, with the delta rule's correction or (a decay per key channel, every head its own keys) without it
@@ -679,7 +679,7 @@ static int gdn_launch(const i64h_gdn_args& d, void* stream) {
         return i64h_scan_tiles(d, RULE == GD_DELTA, stream);
     }
     // Staged through LDS, 16 tokens at a time, from a mean of eight rows a run or one run of 16 on: 16 heads, linear attention (delta rule), straight into registers | staged, 40 single rows
-    // beside 17 rows 23 | 22 us (24 | 23), beside 100 64 | 35 (75 | 39), beside 280 155 | 64 (184 | 74), 3 beside 20 13.5 | 7.1 (15.8 | 7.7); 32 runs of 7 24 | 25 (26.5 | 27.7), 64 of 3 27 | 32 (28 | 35).
+    // beside 17 rows 23 | 23 us (24 | 23), beside 100 64 | 25 (75 | 27), beside 280 155 | 45 (184 | 51), 3 beside 20 13.5 | 7.1 (15.8 | 7.7); 32 runs of 7 24 | 27 (26.5 | 28), 64 of 3 27 | 32 (28 | 35).
     if (g_gdn_form != 1 && vec_ok(kround) && (g_gdn_form > 1 || several || d.longest >= 16)) {
         // One value column per lane: a token then takes the longest run least time, and it is the longest run that the launch waits for (16
         // heads of 128, runs of 1531, 257, 64, 3 and 1101 rows: 264 us, two columns 448; 27 single rows beside 229 and 256: 68 and 100).  Two

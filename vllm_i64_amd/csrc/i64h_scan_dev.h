@@ -4,6 +4,33 @@
 #include "i64h_common.h"
 
 enum { GD_DELTA = 0, GD_KEYS = 1, GD_FORGET = 2 };
+// The y-th run to be started (the same for the whole workgroup), those of more than 16 rows before the others: workgroups start in their order, and a launch that came to
+// its long runs behind many single rows would wait for them alone.  Delta rule, 16 heads of 128, token by token: 27 single rows in front of 229 and 256
+// 67 -> 50 us, 40 in front of 100 39 -> 27, 8 heads, 20 in front of 128 26.4 -> 24.6; 64 runs of 17 in any order 39.4 -> 40.7.
+// (Beyond 256 runs finding out would cost more than it gives: as they lie.)
+__device__ __forceinline__ int gd_run(const int32_t* __restrict__ seg_start, int nseg, int y) {
+    if (nseg == 1 || nseg > 256) return y;
+    const int lane = threadIdx.x & 63;
+    unsigned long long is[4];
+    int longs = 0;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        const int s = min(64 * b + lane, nseg - 1);
+        is[b] = 64 * b < nseg ? __ballot(seg_start[s + 1] - seg_start[s] > 16 && 64 * b + lane < nseg) : 0;
+        longs += __popcll(is[b]);
+    }
+    int k = y < longs ? y : y - longs, run = y;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        const int have = min(64, max(0, nseg - 64 * b));
+        const unsigned long long all = have == 64 ? ~0ull : (1ull << have) - 1, m = y < longs ? is[b] : ~is[b] & all;
+        const int c = __popcll(m);
+        if (k >= 0 && k < c)      // the k-th of these
+            run = 64 * b + __ffsll(__ballot(((m >> lane) & 1) && __popcll(m & ((1ull << lane) - 1)) == k)) - 1;
+        k -= c;
+    }
+    return __builtin_amdgcn_readfirstlane(run);
+}
 // A lane's KPT channels: four neighbours in every stripe of 64 (so that 16 lanes read 256 consecutive bytes at a time).
 template <int KPT>
 __device__ __forceinline__ int gd_channel(int nlane, int k) {

@@ -11,6 +11,7 @@
 #include <type_traits>
 
 #include "i64h_dense_dev.h"
+#include "i64h_scan_dev.h"
 
 typedef float stf4 __attribute__((ext_vector_type(4)));
 enum { ST_TOK = 16, ST_PAIR = ST_TOK * ST_TOK };
@@ -279,19 +280,20 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t st_buffer(const float* base, u
 // What bounds a long run is a tile's chain - 8 matrix instructions, LDS and a barrier, 4, 8 more - and what one wave a SIMD has to issue beside it: 0.88 us of 16
 // tokens of 128 channels (token by token 2.5), of which the 29 matrix instructions are 930 cycles of 2000 and the loads' addresses 350.  Loads through descriptors
 // (no 64-bit address a lane, no branch for rows behind the end) and in four groups that stand between the products, the read-out's products around the exchange,
-// its sums and stores behind the next tile's barrier; before that 1.13 us.  us, before and after: 1531 rows, 16 heads 107 -> 84, five ragged runs 110 -> 89,
-// 8 of 512 over 8 heads 56 -> 48, 32 of 2048 949 -> 796, 64 channels 76 -> 58; linear attention 68 -> 57, 84 -> 61, 38 -> 34, 572 -> 553, 52 -> 37 (64 runs of 256 rows,
-// 16 heads: 294 -> 300).  All of a tile's loads in front of its products: 101 for the first; reloading an operand's registers behind its last product instead of a
-// third set: 85, linear attention 71.  Reading q, k and decays here and taking the products in every workgroup was 2.0 us a tile.
+// its sums and stores behind the next tile's barrier; before that 1.13 us.  Tiles that load nothing more (a run's last ones) are code of their own, and a run of one or two
+// tiles asks for no more than it has: three sets of operands then take 168 registers where they took 254.  us, before and after: 1531 rows, 16 heads 107 -> 84, five ragged runs
+// 110 -> 89, 8 of 512 over 8 heads 56 -> 49, 32 of 2048 949 -> 759, 64 of 256 over 16 heads 532 -> 438, 27 single rows beside 229 and 256 52 -> 31, 64 channels 76 -> 57; linear
+// attention 68 -> 55, 84 -> 59, 38 -> 34, 572 -> 530, 294 -> 289, 45 -> 21, 52 -> 37.  All of a tile's loads in front of its products: 101 for the first; reloading an operand's registers
+// behind its last product instead of a third set: 85, linear attention 71.  Reading q, k and decays here and taking the products in every workgroup was 2.0 us a tile.
 // The workgroups of a head are a multiple of eight apart where there are eight heads: one die's L2 then serves them all.
 template <int BPW, bool DELTA>
-__global__ __launch_bounds__(256, BPW > 2 && DELTA ? 1 : 2) void scan_tile_kernel(const i64h_gdn_args p) {
+__global__ __launch_bounds__(256, BPW > 2 ? (DELTA ? 1 : 2) : 3) void scan_tile_kernel(const i64h_gdn_args p) {
     constexpr int NP = 64 * BPW, FL = st_floats(NP), SETS = 3;
     __shared__ stf4 sX[2][DELTA ? 4 : 1][64], sY[2][4][64];
     const int N = p.dim, P = p.vdim;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, g = lane >> 4;
-    const int a = blockIdx.x % p.heads, seg = blockIdx.y;
+    const int a = blockIdx.x % p.heads, seg = gd_run(p.seg_start, p.nseg, blockIdx.y);
     const int col = blockIdx.x / p.heads * 16 + c;
     const bool cok = col < P;
     const int64_t r0 = p.seg_start[seg], r1 = p.seg_start[seg + 1];
@@ -377,9 +379,10 @@ __global__ __launch_bounds__(256, BPW > 2 && DELTA ? 1 : 2) void scan_tile_kerne
     // What a tile waits for is its chain, so whatever else there is stands where the chain waits: the read-out's products around the exchange of the shares of
     // k P S, the sums and stores of the tile before behind the barrier that this exchange needs, the state times P_16 in front of its last products.
     stf4 O = (stf4)0.0f;      // a wave's share of the read-out of the tile before
-    auto tile = [&](int i, const Ops& o, Ops& ahead) {
+    auto tile = [&](int i, const Ops& o, Ops& ahead, auto more) {      // more: a tile's operands are loaded meanwhile
         const int pb = i & 1;
-        const Tile next = where(i + SETS - 1);
+        constexpr bool LOAD = decltype(more)::value;
+        const Tile next = LOAD ? where(i + SETS - 1) : Tile{};
         if constexpr (DELTA) {
             stf4 x[2] = {(stf4)0.0f, (stf4)0.0f};
 #pragma unroll
@@ -387,7 +390,7 @@ __global__ __launch_bounds__(256, BPW > 2 && DELTA ? 1 : 2) void scan_tile_kerne
 #pragma unroll
                 for (int b = 0; b < BPW; ++b) x[b & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kp[b][r], S[b][r], x[b & 1], 0, 0, 0);
             sY[pb][w][lane] = O;
-            load(next, ahead, 0);
+            if constexpr (LOAD) load(next, ahead, 0);
             sX[pb][w][lane] = BPW > 1 ? x[0] + x[1] : x[0];
         } else sY[pb][w][lane] = O;
         stf4 y[2] = {(stf4)0.0f, (stf4)0.0f};
@@ -408,9 +411,9 @@ __global__ __launch_bounds__(256, BPW > 2 && DELTA ? 1 : 2) void scan_tile_kerne
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) ys[j] = ((const float*)&sY[pb][j][lane])[w];
-        load(next, ahead, 1);
+        if constexpr (LOAD) load(next, ahead, 1);
         read_out(1, 4);
-        load(next, ahead, 2);
+        if constexpr (LOAD) load(next, ahead, 2);
 #pragma unroll
         for (int b = 0; b < BPW; ++b) S[b] = S[b] * o.tot[b];
         stf4 W, U;      // (rows behind the run's end: no value, no key, no write strength)
@@ -434,7 +437,7 @@ __global__ __launch_bounds__(256, BPW > 2 && DELTA ? 1 : 2) void scan_tile_kerne
         for (int r = 0; r < 4; ++r)
 #pragma unroll
             for (int b = 0; b < BPW; ++b) S[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kd[b][r], U[r], S[b], 0, 0, 0);
-        load(next, ahead, 3);
+        if constexpr (LOAD) load(next, ahead, 3);
         if (i > 0) store(ys, ST_TOK);
         // a wave's share of the read-out: its channels of the state, and every fourth token's write
         O = BPW > 1 ? y[0] + y[1] : y[0];
@@ -442,22 +445,33 @@ __global__ __launch_bounds__(256, BPW > 2 && DELTA ? 1 : 2) void scan_tile_kerne
         else O = __builtin_amdgcn_mfma_f32_16x16x4f32(o.B, w == 0 ? U[0] : (w == 1 ? U[1] : (w == 2 ? U[2] : U[3])), O, 0, 0, 0);
     };
     Ops u[SETS];
+    auto whole = [&](int i, Ops& o) {
+        const Tile t = where(i);
 #pragma unroll
-    for (int j = 0; j < SETS - 1; ++j) {      // (the sets' loads stay apart: waiting for one must not wait for the next)
-        const Tile t = where(j);
+        for (int part = 0; part < 4; ++part) load(t, o, part);
+    };
+    constexpr std::false_type none{};
+    if (nt < SETS) {      // (a run of a tile or two loads no more than it has: beside a prompt most of a step's runs are single rows)
+        whole(0, u[0]);
+        if (nt > 1) whole(1, u[1]);
+        tile(0, u[0], u[0], none);
+        if (nt > 1) tile(1, u[1], u[1], none);
+    } else {
 #pragma unroll
-        for (int part = 0; part < 4; ++part) load(t, u[j], part);
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
+        for (int j = 0; j < SETS - 1; ++j) {      // (the sets' loads stay apart: waiting for one must not wait for the next)
+            whole(j, u[j]);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        int i = 0;
+        for (; i + SETS <= nt; i += SETS) {      // (not left in the middle: round the loop every set is as many loads behind the next)
+#pragma unroll
+            for (int j = 0; j < SETS; ++j) tile(i + j, u[j], u[(j + SETS - 1) % SETS], std::true_type{});
+        }
+#pragma unroll
+        for (int j = 0; j < SETS - 1; ++j)
+            if (i + j < nt) tile(i + j, u[j], u[j], none);
     }
-    int i = 0;
-    for (; i + SETS <= nt; i += SETS) {      // (not left in the middle: round the loop every set is as many loads behind the next)
-#pragma unroll
-        for (int j = 0; j < SETS; ++j) tile(i + j, u[j], u[(j + SETS - 1) % SETS]);
-    }
-#pragma unroll
-    for (int j = 0; j < SETS - 1; ++j)
-        if (i + j < nt) tile(i + j, u[j], u[(j + SETS - 1) % SETS]);
     sY[nt & 1][w][lane] = O;
     __syncthreads();
     float ys[4];
