@@ -142,7 +142,7 @@ def test_the_longest_runs_choose_the_tiles_and_need_their_workspace(dev):
 
 
 @pytest.mark.parametrize("delta", [True, False])
-@pytest.mark.parametrize("singles,length,form", [(6, 15, 1), (6, 16, 2), (2, 40, 2), (3, 59, 2), (3, 120, 5)])
+@pytest.mark.parametrize("singles,length,form", [(6, 15, 1), (6, 16, 2), (2, 40, 2), (3, 100, 2), (3, 150, 5)])
 def test_single_rows_beside_a_prompt_whose_length_is_told(dev, delta, singles, length, form):
     """The longest run decides the form where the caller tells it, whatever the mean is: the bits are that form's, and the recurrence's in 64 bits."""
     from vllm_i64_amd import _lib, ops_dense as D

@@ -634,21 +634,19 @@ int i64h_set_gdn_scan_form(int32_t form) {
 }
 
 // Tiles of 16 tokens on the matrix cores are two launches and a tile costs the same however few rows it holds; token by token a launch takes as long as
-// its longest run.  So it is the longest run that decides, against the number of runs, each a tile at least (in workgroups of the second launch) - unless the runs are long on the
-// average.  Microseconds in replayed graphs, token by token | in tiles, delta rule (linear attention), heads of 128: 16 heads, a run of 1531 rows 242 | 106 (215 | 71), of 160 28 | 21
-// (27 | 15), of 96 17.9 | 17.5 (17.1 | 13.0), of 64 13.5 | 15.7 (12.5 | 11.8), 40 single rows beside 200 39 | 44 (33 | 33), beside 280 51 | 46 (45 | 34), 20 beside 128 26 | 30 (23 | 22), 64 beside
-// 400 69 | 70 (60 | 48), 16 runs of 24 30 | 31 (27 | 22), 4 of 64 22 | 22 (19 | 15); 8 heads, 8 runs of 512 125 | 77 (96 | 52), 40 single rows beside 150 30 | 29 (26 | 21), 20 beside 128
-// 25 | 22 (22 | 17), 4 runs of 64 14.8 | 16.6 (13.9 | 12.6); 8 heads of 64, 8 runs of 17 5.6 | 11.9 (5.0 | 9.3), 16 of 64 14.6 | 16.6 (11.6 | 12.2), 4 of 96 13.9 | 14.4 (11.3 | 10.9).  Narrow
-// heads in thousands of workgroups are little more than their reads either way (32 heads of 64, 32 runs of 192 rows 193 | 182, 140 | 135; 40 single rows beside 280 38 | 36), as are many
-// short runs nobody measured (64 of 17 rows, delta rule 41 | 48).
+// its longest run.  So it is the longest run that decides.  Microseconds in replayed graphs, token by token | in tiles, delta rule (linear attention), heads
+// of 128: 16 heads, a run of 1531 rows 242 | 106 (215 | 71), of 160 28 | 21 (27 | 15), of 96 17.9 | 17.5 (17.1 | 13.0: too little for a workspace of 27 KB a tile and head), 40 single rows beside 200
+// 39 | 44 (33 | 33), beside 280 51 | 46 (45 | 34), 20 beside 128 26 | 30 (23 | 22), 16 runs of 24 30 | 31 (27 | 22), 4 of 64 22 | 22 (19 | 15); 8 heads, 8 runs of 512 125 | 77 (96 | 52), 20 single rows
+// beside 128 25 | 22 (22 | 17); 8 heads of 64, 8 runs of 17 5.6 | 11.9 (5.0 | 9.3), 16 of 64 14.6 | 16.6 (11.6 | 12.2), 4 of 96 13.9 | 14.4 (11.3 | 10.9).  Narrow heads in thousands of workgroups
+// are little more than their reads either way (32 heads of 64, 32 runs of 192 rows 193 | 182, 140 | 135), as are many short runs (64 of 17 rows, delta rule 41 | 48).
 int32_t i64h_scan_in_tiles(int64_t n, int32_t nseg, int32_t longest, int32_t heads, int32_t dim, int32_t vdim, int32_t delta) {
     const int64_t groups = (int64_t)heads * ((vdim + 15) / 16) * nseg;      // workgroups of the second launch
-    const bool even = n >= 32 * (int64_t)nseg, known = longest < INT32_MAX;
-    const bool worth = longest >= (delta ? 92 + groups / 30 : 60 + groups / 38) || (even && longest >= (delta ? 144 : 112)) || (!delta && dim > 64 && known && n >= 128 && n >= 24 * (int64_t)nseg);
-    return dim % 4 == 0 && dim <= 256 && n >= (known ? 64 : 96) && worth && (known || even || groups < 6144) && (dim > 64 || groups <= 2048);
+    return dim % 4 == 0 && dim <= 256 && n >= 96 && n >= 8 * (int64_t)nseg && longest >= (delta ? 144 : 112) && (n >= 32 * (int64_t)nseg || groups < 6144) &&
+           (dim > 64 || groups <= 2048);
 }
 
-// From the projections three launches stand for four or six that read and write the rows between them, so tiles pay earlier.  Microseconds as above, in launches of their own token
+// From the projections three launches stand for four or six that read and write the rows between them, so tiles pay earlier, against the number of runs, each a tile at least (in workgroups
+// of the second launch).  Microseconds as above, in launches of their own token
 // by token | in tiles: 16 heads of 128, a run of 32 rows 27 | 26 (14.6 | 16.3), of 64 36 | 28 (20 | 17), of 96 44 | 29 (26 | 19), 8 single rows beside 40 33 | 32 (18 | 20), beside 60 39 | 33 (22 | 21),
 // 20 beside 64 42 | 44 (24 | 28), beside 100 51 | 45 (29 | 29), 40 beside 100 58 | 61 (36 | 40), beside 150 65 | 64 (39 | 43), beside 200 75 | 66 (45 | 44), 64 beside 200 82 | 86 (53 | 59), beside 400
 // 114 | 95 (73 | 62), 32 runs of 17 85 | 73 (53 | 48), 16 of 24 73 | 52 (41 | 34); 8 heads, 40 beside 48 38 | 43 (22 | 27), beside 100 47 | 43 (28 | 27), 20 beside 64 36 | 32 (21 | 21);
@@ -671,7 +669,7 @@ static int gdn_launch(const i64h_gdn_args& d, void* stream) {
     const int kround = kpt <= 4 ? 4 : (kpt <= 8 ? 8 : 16);
     // runs nobody measured: the mean says whether one of them may be long
     const bool several = d.n >= 8 * (int64_t)d.nseg;
-    const bool tiles = (d.longest > 0 || several) && i64h_scan_in_tiles(d.n, d.nseg, d.longest > 0 ? d.longest : INT32_MAX, d.heads, d.dim, d.vdim, RULE == GD_DELTA);
+    const bool tiles = i64h_scan_in_tiles(d.n, d.nseg, d.longest > 0 ? d.longest : INT32_MAX, d.heads, d.dim, d.vdim, RULE == GD_DELTA);
     if (RULE != GD_FORGET && d.work && ((g_gdn_form == 0 && tiles) || g_gdn_form == 5) && vec_ok(4) && (uintptr_t)d.work % 16 == 0 && d.ldx < (1 << 25) &&
         (d.n / 16 + d.nseg) * (int64_t)d.heads < (1ll << 31)) {
         I64H_CHECK_ARG(d.work_floats >= i64h_scan_work_floats(d.n, d.nseg, d.heads, d.dim), "scan: a workspace of %lld floats, %lld needed", (long long)d.work_floats,

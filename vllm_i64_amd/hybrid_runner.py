@@ -200,11 +200,11 @@ class HybridRunner:
             ws = B.attn_ws[key] = torch.empty(max(1, floats(splits)), dtype=torch.float32, device=self.device)
         return splits, ws
 
-    def _scan_work(self, n: int, nseg: int, longest: int, scans, delta: bool) -> Dict[tuple, torch.Tensor]:
-        """The workspace of a step's scans by (heads, dim, vdim), for those of `scans` whose runs are worth the form that takes one, alone or from the projections.  The caller holds it for
+    def _scan_work(self, n: int, nseg: int, longest: int, scans, delta: bool, rec: bool = False) -> Dict[tuple, torch.Tensor]:
+        """The workspace of a step's scans by (heads, dim, vdim), for those of `scans` whose runs are worth the form that takes one, alone or (rec) from the projections.  The caller holds it for
         the step and no longer: 27 KB a tile of 16 rows and head of 128 would otherwise lie beside every kept buffer set.  Where the card has no room for
         it the scans go token by token: the same values in another order of the sums."""
-        worth = D.scan_in_tiles if self.exact else D.rec_in_tiles
+        worth = D.rec_in_tiles if rec else D.scan_in_tiles
         sizes = {s: D.scan_work_floats(n, nseg, s[0], s[1]) for s in scans if worth(n, nseg, longest, *s, delta=delta)}
         if not sizes:
             return {}

@@ -160,7 +160,7 @@ class PukatarModel(HybridRunner):
             return B.logits
         eps, ex, hint = cfg.norm_eps, self.exact, int(max_ctx_hint)
         seg, nseg, longest = self._runs(n, slot_ids, tokens_per_seq, rows_are_slots)
-        work = self._scan_work(n, nseg, longest, self.scans, delta=True)
+        work = self._scan_work(n, nseg, longest, self.scans, delta=True, rec=not self.exact)
         if tokens_per_seq is not None:
             runs = attention_segments(tokens_per_seq, n, self.ATTN_MAX_SEGMENTS)
         else:

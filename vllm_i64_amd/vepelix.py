@@ -168,7 +168,7 @@ class VepelixModel(HybridRunner):
         if n == 0:
             return B.logits
         seg, nseg, longest = self._runs(n, slot_ids, tokens_per_seq, rows_are_slots)
-        work = self._scan_work(n, nseg, longest, self.scans, delta=False)
+        work = self._scan_work(n, nseg, longest, self.scans, delta=False, rec=not self.exact)
         if tokens_per_seq is not None:
             runs = attention_segments(tokens_per_seq, n, self.ATTN_MAX_SEGMENTS)
         else:
