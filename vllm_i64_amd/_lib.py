@@ -6,6 +6,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 from typing import Dict, Optional
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -428,6 +429,15 @@ def load_dense() -> ctypes.CDLL:
         fn.argtypes = [_KIND[c] for c in sig]
     _dense = lib
     return lib
+
+
+def packer(mirror):
+    """Packs all fields of a descriptor in their order into the bytes that the C struct is: one call where a ctypes structure takes one assignment a field (in an eager
+    step of 10 read-outs and 25 Linears: 11.0 and 7.5 us a call for 13.7 and 8.8)."""
+    code = {_P: "P", _L: "q", _I: "i", _F: "f"}
+    st = struct.Struct("@" + "".join(code[t] for _, t in mirror._fields_) + "0P")
+    assert st.size == ctypes.sizeof(mirror)
+    return st.pack
 
 
 def call_dense(name: str, *args):

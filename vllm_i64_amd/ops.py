@@ -18,13 +18,14 @@ EPI_STORE, EPI_SWIGLU = 0, 1
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)      # (whoever holds a GPU tensor has initialised the GPU)
 
 
 def _stream() -> int:
     """The current stream's handle.  Asked once per launch: through the raw accessor where this torch has it (the Stream object
     route takes ~8 us of host time, a quarter of an eager decode step's launch loop)."""
     if _raw_stream is not None:
-        return _raw_stream(torch.cuda.current_device())
+        return _raw_stream(_device())
     return torch.cuda.current_stream().cuda_stream
 
 

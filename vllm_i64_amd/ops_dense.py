@@ -17,8 +17,18 @@ _DUAL = (EPI_GELU_MUL, EPI_SILU_MUL, EPI_CLAMP_GLU)
 CACHE_DTYPE_CODE = {torch.float32: 0, torch.bfloat16: 2}
 
 
+_pack_linear, _pack_streams = _lib.packer(_lib.Linear), _lib.packer(_lib.Streams)
+
+
 def _ref(s):
     return ctypes.addressof(s)
+
+
+def _at(t: torch.Tensor, dtype: torch.dtype, name: str) -> int:
+    """The address of a contiguous tensor of this type on the GPU; an error for any other."""
+    if not (t.is_cuda and t.dtype == dtype and t.is_contiguous()):
+        _chk(t, dtype, name)
+    return t.data_ptr()
 
 
 def linear(a: Optional[torch.Tensor], w: torch.Tensor, out: Optional[torch.Tensor], *, m: Optional[int] = None, n: Optional[int] = None, k: Optional[int] = None,
@@ -38,82 +48,61 @@ def linear(a: Optional[torch.Tensor], w: torch.Tensor, out: Optional[torch.Tenso
     in_norm_w fp32 [k] with in_eps: the input rows are RMS-normed first (plain result: the epilogue is then EPI_IN_NORM).
     a16 bf16 (k a multiple of 64; the plain, scaled, adding, row-gated and gate / up epilogues): the rows of a, rounded by whoever wrote them, in a's place.
     out16 bf16 (with a16): receives the result rounded, beside out or (out None) in its place."""
+    pa = pa16 = pc = pc16 = 0
     if a16 is None:
         if a is None or out is None or out16 is not None:
             raise _lib.I64HError("linear: no input rows, or a result in bf16 without input rows in bf16")
-        _chk(a, torch.float32, "a"), _chk(w, torch.bfloat16, "w"), _chk(out, torch.float32, "out")
-        o = out
+        pa, pc, o = _at(a, torch.float32, "a") + 4 * a_off, _at(out, torch.float32, "out") + 4 * c_off, out
     else:
-        _chk(a16, torch.bfloat16, "a16"), _chk(w, torch.bfloat16, "w")
-        a, o = a16, out if out is not None else out16
+        pa16, a, o = _at(a16, torch.bfloat16, "a16") + 2 * a_off, a16, out if out is not None else out16
         if out is not None:
-            _chk(out, torch.float32, "out")
+            pc = _at(out, torch.float32, "out") + 4 * c_off
         if out16 is not None:
-            _chk(out16, torch.bfloat16, "out16")
+            pc16 = _at(out16, torch.bfloat16, "out16") + 2 * c_off
             if out is not None and (out16.numel() != out.numel() or out16.shape[-1] != out.shape[-1]):
                 raise _lib.I64HError("linear: out16 is not laid out as out")
-    if a_rows is not None:
-        _chk(a_rows, torch.int32, "a_rows")
-    N = int(n if n is not None else w.shape[-2] // (2 if epilogue in _DUAL else 1))
-    K = int(k if k is not None else w.shape[-1])
-    M = int(m if m is not None else (a_rows.numel() if a_rows is not None else a.shape[0]))
-    lda = int(lda if lda is not None else a.shape[-1])
-    ldc = int(ldc if ldc is not None else o.shape[-1])
-    if w.shape[-1] != K or a_off + (batch - 1) * a_batch + K > lda or c_off + (batch - 1) * c_batch + N > ldc:
+    pw = _at(w, torch.bfloat16, "w")
+    pr = _at(a_rows, torch.int32, "a_rows") if a_rows is not None else 0
+    dual, wk = 2 if epilogue in _DUAL else 1, w.size(-1)
+    N = int(n if n is not None else w.size(-2) // dual)
+    K = int(k if k is not None else wk)
+    M = int(m if m is not None else (a_rows.numel() if a_rows is not None else a.size(0)))
+    lda = int(lda if lda is not None else a.size(-1))
+    ldc = int(ldc if ldc is not None else o.size(-1))
+    if wk != K or a_off + (batch - 1) * a_batch + K > lda or c_off + (batch - 1) * c_batch + N > ldc:
         raise _lib.I64HError(f"linear: K {K} / N {N} do not fit a (row stride {lda}), w {tuple(w.shape)} or out (row stride {ldc})")
     if o.numel() < (M - 1) * ldc + c_off + (batch - 1) * c_batch + N or (a_rows is None and a.numel() < (M - 1) * lda + a_off + (batch - 1) * a_batch + K):
         raise _lib.I64HError("linear: operand smaller than the launch reads or writes")
-    if w.numel() < (batch - 1) * w_batch + N * K * (2 if epilogue in _DUAL else 1):
+    if w.numel() < (batch - 1) * w_batch + N * K * dual:
         raise _lib.I64HError("linear: weight smaller than the launch reads")
+    pe = pb = prs = pn = pg = total = 0
     if e is not None:
-        _chk(e, torch.float32, "e")
+        pe = _at(e, torch.float32, "e") + 4 * e_off
         if e.numel() < (M - 1) * lde + e_off + (batch - 1) * e_batch + (1 if epilogue == EPI_ROW_SIGMOID else N):
             raise _lib.I64HError("linear: gate operand smaller than the launch reads")
     if bias is not None:
-        _chk(bias, torch.float32, "bias")
+        pb = _at(bias, torch.float32, "bias")
         if bias.numel() < (batch - 1) * bias_batch + N:
             raise _lib.I64HError("linear: bias smaller than the launch reads")
     if in_norm_w is not None:
-        _chk(in_norm_w, torch.float32, "in_norm_w")
+        pn = _at(in_norm_w, torch.float32, "in_norm_w")
         if epilogue != EPI_STORE or in_norm_w.numel() != K:
             raise _lib.I64HError("linear: the input norm's weights are not [k], or another epilogue is asked for beside it")
         epilogue = EPI_IN_NORM
     if row_scale is not None:
-        _chk(row_scale, torch.float32, "row_scale")
+        prs = _at(row_scale, torch.float32, "row_scale")
         if row_scale.numel() < M:
             raise _lib.I64HError("linear: fewer row factors than rows")
     if group_off is not None:
-        _chk(group_off, torch.int32, "group_off")
+        pg = _at(group_off, torch.int32, "group_off")
         if group_off.numel() < batch + 1:
             raise _lib.I64HError("linear: group_off needs batch + 1 entries")
-    # (a step makes a few dozen of these: only what is not zero is put in)
-    d = _lib.Linear(lda=lda, W=ptr(w), ldc=ldc, M=M, N=N, K=K, batch=batch, exact=int(exact), epilogue=epilogue, scale=scale)
-    if a16 is None:
-        d.A = ptr(a) + 4 * a_off
-    else:
-        d.A16 = ptr(a16) + 2 * a_off
-    if out is not None:
-        d.C = ptr(out) + 4 * c_off
-    if out16 is not None:
-        d.C16 = ptr(out16) + 2 * c_off
-    if a_batch or w_batch or c_batch:
-        d.a_batch, d.w_batch, d.c_batch = a_batch, w_batch, c_batch
-    if e is not None:
-        d.E, d.lde, d.e_batch = ptr(e) + 4 * e_off, lde, e_batch
-    if bias is not None:
-        d.bias, d.bias_batch = ptr(bias), int(bias_batch)
-    if a_rows is not None:
-        d.a_rows, d.a_height = ptr(a_rows), -(-a.numel() // lda)
-    if group_off is not None:
-        d.group_off, d.rows_total = ptr(group_off), min((a_rows.numel() if a_rows is not None else a.numel() // lda), o.numel() // ldc)
-    if row_scale is not None:
-        d.row_scale = ptr(row_scale)
-    if in_norm_w is not None:
-        d.in_norm_w, d.in_eps = ptr(in_norm_w), in_eps
-    if epilogue == EPI_SOFTCAP:
-        d.softcap = softcap
-    elif epilogue == EPI_CLAMP_GLU or epilogue == EPI_XIELU:
-        d.act_a, d.act_b = act_a, act_b
+        total = min((a_rows.numel() if a_rows is not None else a.numel() // lda), o.numel() // ldc)
+    acts = epilogue == EPI_CLAMP_GLU or epilogue == EPI_XIELU
+    d = _lib.Linear.from_buffer_copy(_pack_linear(
+        pa, lda, pr, pw, pc, ldc, M, N, K, batch, a_batch, w_batch, c_batch, int(exact), epilogue, pe, lde if pe else 0, e_batch if pe else 0,
+        softcap if epilogue == EPI_SOFTCAP else 0.0, pb, int(bias_batch) if pb else 0, scale, act_a if acts else 0.0, act_b if acts else 0.0, pg, prs, pn,
+        in_eps if pn else 0.0, total, -(-a.numel() // lda) if pr else 0, pa16, pc16))
     call_dense("i64h_linear_run", _ref(d), _stream())
     return o
 
@@ -265,40 +254,45 @@ def streams_step(streams: torch.Tensor, *, y: Optional[torch.Tensor] = None, y2:
     h16 bf16 [n, W]: the rows of h rounded, beside h or (h None) in its place.  moe (one stream, no result norms): the arguments of moe_combine but `out`, whose
     result stands for y or is added to it.  route: the arguments of route_topk but logits and h, the choice on the rows of h in the same launch (see i64h_streams_route); plan: those of
     moe_plan but idx, n and top, for at most PLAN_ROWS rows, with sync int32 [32 * 17], zeros between launches."""
-    _chk(streams, torch.float32, "streams")
+    F32 = torch.float32
+    ps = _at(streams, F32, "streams")
     S, n, W = streams.shape
-    for t, name in ((y, "y"), (y2, "y2"), (yn_w, "yn_w"), (y2n_w, "y2n_w"), (mix, "mix"), (out_w, "out_w"), (in_w, "in_w"), (norm_w, "norm_w"), (h, "h"),
-                    (post_w, "post_w"), (norm_b, "norm_b"), (y_scale, "y_scale")):
-        if t is not None:
-            _chk(t, torch.float32, name)
-    for t, name in ((y, "y"), (y2, "y2")):
-        if t is not None and (t.shape[-1] != W or t.numel() < n * W):
-            raise _lib.I64HError(f"streams_step: {name} is not [n, W]")
+    py = _at(y, F32, "y") if y is not None else 0
+    py2 = _at(y2, F32, "y2") if y2 is not None else 0
+    if (y is not None and (y.size(-1) != W or y.numel() < n * W)) or (y2 is not None and (y2.size(-1) != W or y2.numel() < n * W)):
+        raise _lib.I64HError("streams_step: y or y2 is not [n, W]")
+    pmix = _at(mix, F32, "mix") if mix is not None else 0
+    pow_ = _at(out_w, F32, "out_w") if out_w is not None else 0
+    piw = _at(in_w, F32, "in_w") if in_w is not None else 0
     if (mix is not None and mix.numel() != S * S) or (out_w is not None and out_w.numel() != S) or (in_w is not None and in_w.numel() != S):
         raise _lib.I64HError("streams_step: stream weights do not fit the number of streams")
+    pyn = _at(yn_w, F32, "yn_w") if yn_w is not None else 0
+    py2n = _at(y2n_w, F32, "y2n_w") if y2n_w is not None else 0
+    ppost = _at(post_w, F32, "post_w") if post_w is not None else 0
     if (yn_w is not None and yn_w.numel() != W) or (y2n_w is not None and y2n_w.numel() != W) or (post_w is not None and post_w.numel() != W):
         raise _lib.I64HError("streams_step: result norm weights are not [W]")
+    pnb = _at(norm_b, F32, "norm_b") if norm_b is not None else 0
+    pys = _at(y_scale, F32, "y_scale") if y_scale is not None else 0
     if (norm_b is not None and norm_b.numel() != W) or (y_scale is not None and y_scale.numel() != W):
         raise _lib.I64HError("streams_step: the norm's offsets or the result's factors are not [W]")
-    m_rows = n
+    pnw = _at(norm_w, F32, "norm_w") if norm_w is not None else 0
+    m_rows, prows, ph, ph16 = n, 0, 0, 0
     if rows is not None:
-        _chk(rows, torch.int32, "rows")
-        m_rows = rows.numel()
-    if h is not None and h.numel() < m_rows * W:
-        raise _lib.I64HError("streams_step: h smaller than the rows it receives")
+        prows, m_rows = _at(rows, torch.int32, "rows"), rows.numel()
+    if h is not None:
+        ph = _at(h, F32, "h")
+        if h.numel() < m_rows * W:
+            raise _lib.I64HError("streams_step: h smaller than the rows it receives")
     if h16 is not None:
-        _chk(h16, torch.bfloat16, "h16")
+        ph16 = _at(h16, torch.bfloat16, "h16")
         if h16.numel() < m_rows * W:
             raise _lib.I64HError("streams_step: h16 smaller than the rows it receives")
-    mk = {}
+    mk = (0, 0, 0, 0, 0, 0, 0)
     if moe is not None:
         _moe_ok(moe["y"], moe["pair_row"], moe["wgt"], moe["h"], moe["shared"], n, moe["top"], W, moe.get("shared_gate"), "streams_step")
-        mk = dict(moe_y=ptr(moe["y"]), moe_row=ptr(moe["pair_row"]), moe_wgt=ptr(moe["wgt"]), moe_h=ptr(moe["h"]), moe_shared=ptr(moe["shared"]),
-                  moe_gate=ptr(moe.get("shared_gate")), moe_top=moe["top"])
-    d = _lib.Streams(streams=ptr(streams), S=S, n=n, W=W, y=ptr(y), ldy=W, y2=ptr(y2), ldy2=W, yn_w=ptr(yn_w), y2n_w=ptr(y2n_w), y_eps=float(y_eps),
-                     mix=ptr(mix), out_w=ptr(out_w), in_w=ptr(in_w), norm_w=ptr(norm_w), norm_w_len=norm_w.numel() if norm_w is not None else 0,
-                     eps=float(eps), h=ptr(h), rows=ptr(rows), m_rows=m_rows, post_w=ptr(post_w), post_center=int(bool(post_center)), h_center=int(bool(h_center)),
-                     norm_b=ptr(norm_b), y_scale=ptr(y_scale), h16=ptr(h16), **mk)
+        mk = (ptr(moe["y"]), ptr(moe["pair_row"]), ptr(moe["wgt"]), ptr(moe["h"]), ptr(moe["shared"]), ptr(moe.get("shared_gate")), moe["top"])
+    d = _lib.Streams.from_buffer_copy(_pack_streams(ps, S, n, W, py, W, py2, W, pyn, py2n, y_eps, pmix, pow_, piw, pnw, norm_w.numel() if norm_w is not None else 0, eps, ph, prows, m_rows, ppost, int(bool(post_center)),
+                      int(bool(h_center)), pnb, pys, ph16, *mk))
     if route is None:
         call_dense("i64h_streams_step", _ref(d), _stream())
         return h
