@@ -306,3 +306,16 @@ def test_prefill_attention_whose_scores_climb(dev, step):
     bound = 2 * 16 * 2.0 ** -24 * (5 * step * 0.6931472 + 8) * float(v.abs().max())
     assert (out.double() - ref).abs().max() <= bound
     assert torch.equal(run(37), out[37:])
+
+
+@pytest.mark.parametrize("rows,buckets", [(513, 1), (640, 3), (641, 16), (1023, 17), (4097, 200), (9000, 256), (70001, 64)])
+def test_stable_buckets_of_many_rows(dev, rows, buckets):
+    """Rows at the edges of a wave's share, bucket counts that divide the scan's threads or not, empty buckets: a stable sort by bucket, whole numbers exactly."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(rows)
+    key = torch.randint(0, buckets, (rows,), generator=g, dtype=torch.int32) // 3 * 3 % buckets
+    off, perm, inv, _ = ops.bucketize(key.to(dev), buckets)
+    want = torch.sort(key, stable=True)[1]
+    assert torch.equal(perm.cpu().long(), want)
+    assert torch.equal(off.cpu().long(), torch.cat([torch.zeros(1, dtype=torch.long), torch.bincount(key.long(), minlength=buckets).cumsum(0)]))
+    assert torch.equal(inv.cpu().long(), torch.argsort(want))

@@ -7,7 +7,9 @@
 // source order, which is what a boolean-mask gather produces on the CPU.
 #include "i64h_common.h"
 
-#define ROWS_PER_WAVE 512
+#define ROWS_PER_WAVE 128   // of the three launches: what a wave does is a chain of loads and exchanges, so many waves of few rows (32768 rows of 16 buckets, two layers: 512 a wave 11 + 15 + 14 us, 128 a wave
+                            // 4.9 + 5.9 + 5.2, the scan over the waves dealt to all threads of its workgroup)
+#define SMALL_ROWS 512      // up to here one workgroup does all three phases
 #define PLAN_THREADS 256
 #define MAX_BUCKETS 256
 
@@ -45,27 +47,39 @@ __global__ __launch_bounds__(PLAN_THREADS) void bucket_hist_kernel(
     const int64_t R = (int64_t)n * top_k;
     for (int b = lane; b < nb; b += 64) hist[wib][b] = 0;
     __syncthreads();
-    if (gw < num_waves) {
+    if (gw < num_waves && R > 0) {
         int64_t s0 = (int64_t)gw * ROWS_PER_WAVE;
         int64_t s1 = s0 + ROWS_PER_WAVE < R ? s0 + ROWS_PER_WAVE : R;
-        for (int64_t s = s0 + lane; s < s1; s += 64) {
-            int key;
+        constexpr int RPL = ROWS_PER_WAVE / 64;      // a lane's rows: their ids are asked for together, then their table entries
+        int64_t e[RPL];
+        int k[RPL];
+#pragma unroll
+        for (int i = 0; i < RPL; ++i) {
+            const int64_t s = min(s0 + lane + 64 * i, s1 - 1);
+            k[i] = TABLE ? (int)(s / n) : 0;
+            e[i] = TABLE ? ids[s - (int64_t)k[i] * n] : keys_in[s];
+        }
+        if (TABLE) {
+#pragma unroll
+            for (int i = 0; i < RPL; ++i) {
+                const int64_t id = e[i] < 0 ? 0 : (e[i] >= V ? V - 1 : e[i]);
+                e[i] = tables[(int64_t)l * table_layer_stride + (int64_t)k[i] * V + id];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < RPL; ++i) {
+            const int64_t s = s0 + lane + 64 * i;
+            if (s >= s1) continue;
+            int key = (int)e[i];
             if (TABLE) {
-                int k = (int)(s / n);
-                int64_t t = s - (int64_t)k * n;
-                int64_t id = ids[t];
-                id = id < 0 ? 0 : (id >= V ? V - 1 : id);
-                int64_t e = tables[(int64_t)l * table_layer_stride + (int64_t)k * V + id];
-                if (routes) routes[(int64_t)l * R + s] = e;
-                key = (int)e * top_k + k;
+                if (routes) routes[(int64_t)l * R + s] = e[i];
+                key = (int)e[i] * top_k + k[i];
                 key = key < 0 ? 0 : (key >= nb ? nb - 1 : key);
                 if (tok_slots) {  // per token: [0] = the call over all tokens, [1+k] = 1 + bucket of route k
-                    int32_t* ts = tok_slots + ((int64_t)l * n + t) * (1 + top_k);
-                    ts[1 + k] = 1 + key;
-                    if (k == 0) ts[0] = 0;
+                    int32_t* ts = tok_slots + ((int64_t)l * n + (s - (int64_t)k[i] * n)) * (1 + top_k);
+                    ts[1 + k[i]] = 1 + key;
+                    if (k[i] == 0) ts[0] = 0;
                 }
-            } else {
-                key = keys_in[s];
             }
             key = key < 0 ? 0 : (key >= nb ? nb - 1 : key);  // memory safety only; valid inputs never clamp
             keys[(int64_t)l * R + s] = key;
@@ -80,20 +94,34 @@ __global__ __launch_bounds__(PLAN_THREADS) void bucket_hist_kernel(
 // ---- phase B: exclusive scan over waves per bucket, then bucket offsets --------------------------------
 __global__ __launch_bounds__(MAX_BUCKETS) void bucket_scan_kernel(int32_t* __restrict__ wave_counts, int32_t* __restrict__ offsets,
                                                                   int32_t* __restrict__ group_offsets, int group, int nb, int num_waves) {
-    __shared__ int tot[MAX_BUCKETS];
-    const int l = blockIdx.x, b = threadIdx.x;
+    // the waves of a bucket are dealt to as many threads as there are (its count, then its running offsets: two rounds of loads that wait for nothing)
+    __shared__ int tot[MAX_BUCKETS], part[MAX_BUCKETS];
+    const int l = blockIdx.x, nbp = nb <= 1 ? 1 : 1 << (32 - __clz(nb - 1)), parts = MAX_BUCKETS / nbp;
+    const int b = threadIdx.x & (nbp - 1), mine = threadIdx.x / nbp, per = (num_waves + parts - 1) / parts;
+    const int w0 = min(num_waves, mine * per), w1 = min(num_waves, w0 + per);
+    int32_t* p = wave_counts + (int64_t)l * num_waves * nb + min(b, nb - 1);
+    int sum = 0;
+#pragma unroll 8
+    for (int w = w0; w < w1; ++w) sum += p[(int64_t)w * nb];
+    part[threadIdx.x] = sum;
+    __syncthreads();
+    int run = 0;
+    for (int j = 0; j < mine; ++j) run += part[j * nbp + b];
     if (b < nb) {
-        int run = 0;
-        int32_t* p = wave_counts + (int64_t)l * num_waves * nb + b;
-        for (int w = 0; w < num_waves; ++w) {
-            int c = p[(int64_t)w * nb];
-            p[(int64_t)w * nb] = run;
-            run += c;
+        if (mine == parts - 1) tot[b] = run + sum;
+        for (int w = w0; w < w1; w += 8) {
+            int c[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) c[j] = w + j < w1 ? p[(int64_t)(w + j) * nb] : 0;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                if (w + j < w1) p[(int64_t)(w + j) * nb] = run;
+                run += c[j];
+            }
         }
-        tot[b] = run;
     }
     __syncthreads();
-    if (b == 0) {
+    if (threadIdx.x == 0) {
         int run = 0;
         int32_t* o = offsets + (int64_t)l * (nb + 1);
         for (int i = 0; i < nb; ++i) {
@@ -158,7 +186,7 @@ struct PlanEmbed {
     int H, layers;
 };
 
-// ---- all three phases in one launch when one wave covers the rows (decode-sized steps: R <= ROWS_PER_WAVE) -----------------
+// ---- all three phases in one launch when one wave covers the rows (decode-sized steps: R <= SMALL_ROWS) -----------------
 // One workgroup per layer; wave 0 runs phases A and C exactly as the kernels above do for their single wave, the scan of phase B
 // degenerates to the bucket offsets.  Same keys, offsets, permutation: the results are identical to the three-launch path.
 template <bool TABLE>
@@ -168,7 +196,7 @@ __global__ __launch_bounds__(MAX_BUCKETS) void bucket_plan_small_kernel(
     int32_t* __restrict__ wave_counts, int32_t* __restrict__ offsets, int32_t* __restrict__ group_offsets, int32_t* __restrict__ perm,
     int32_t* __restrict__ inv, int32_t* __restrict__ sorted_bucket, int n, int top_k, int64_t V, int nb, PlanEmbed em) {
     __shared__ int hist[MAX_BUCKETS], cursor[MAX_BUCKETS];
-    __shared__ int skey[ROWS_PER_WAVE];
+    __shared__ int skey[SMALL_ROWS];
     if ((int)blockIdx.x >= em.layers) {
         // riders of the plan launch: the embedding rows of the same token ids and the start-of-forward reset of the stat slots
         // (both depend on nothing but the ids; as a launch of their own they cost a dispatch and ~4.6 us in front of layer 0)
@@ -321,7 +349,7 @@ static int bucketize_common(bool table, const int64_t* ids, const int64_t* table
     I64H_CHECK_ARG(R < (1ll << 31), "bucketize: too many rows");
     int num_waves = (int)((R + ROWS_PER_WAVE - 1) / ROWS_PER_WAVE);
     if (num_waves < 1) num_waves = 1;
-    if (R > 0 && R <= ROWS_PER_WAVE) {  // one wave covers the rows: the three phases in one launch
+    if (R > 0 && R <= SMALL_ROWS) {  // one wave covers the rows: the three phases in one launch
         PlanEmbed em = {nullptr, nullptr, nullptr, 0, 0, 0, L};
         if (riders && table) {
             em = *riders;
