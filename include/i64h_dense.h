@@ -28,7 +28,8 @@ int i64h_device_check(void);
  *   row(m) = a_rows ? a_rows[m] : m;  W bf16 [N, K] row-major, batch stride w_batch elements;  C fp32, row stride ldc,
  *   batch stride c_batch.
  * exact = 0: A is rounded to bf16 (nearest even) while it is staged, products on v_mfma_f32_16x16x32_bf16, fp32 sums.
- * exact = 1: W is widened to fp32 while it is staged, products on v_mfma_f32_16x16x4_f32: true 32-bit arithmetic.
+ * exact = 1: products of fp32 rows, sums in fp32.  K of 64 and more: a row's value in three bf16 parts that hold all of it, each times the bf16 weight, on
+ *   v_mfma_f32_16x16x32_bf16; a shorter K: W widened to fp32 while it is staged, v_mfma_f32_16x16x4_f32.
  * epilogue: I64H_EPI_STORE; I64H_EPI_GELU_MUL: gelu_tanh(A W^T) * (A W2^T) with W2 = W + N * K (gate rows, then up rows);
  *   I64H_EPI_MUL_SIGMOID: * sigmoid(E[b][m, n]) (E fp32, row stride lde, batch stride e_batch);
  *   I64H_EPI_SOFTCAP: cap * tanh(. / cap);  I64H_EPI_GELU_ERF: 0.5 v (1 + erf(v / sqrt 2));  I64H_EPI_SCALE: v * scale;
