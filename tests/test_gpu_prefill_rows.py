@@ -308,7 +308,7 @@ def test_prefill_attention_whose_scores_climb(dev, step):
     assert torch.equal(run(37), out[37:])
 
 
-@pytest.mark.parametrize("rows,buckets", [(513, 1), (640, 3), (641, 16), (1023, 17), (4097, 200), (9000, 256), (70001, 64)])
+@pytest.mark.parametrize("rows,buckets", [(1, 5), (65, 1), (512, 256), (513, 1), (640, 3), (641, 16), (1023, 17), (2049, 130), (4000, 256), (4096, 17), (4097, 200), (9000, 256), (70001, 64)])
 def test_stable_buckets_of_many_rows(dev, rows, buckets):
     """Rows at the edges of a wave's share, bucket counts that divide the scan's threads or not, empty buckets: a stable sort by bucket, whole numbers exactly."""
     ops = _ops()

@@ -7,9 +7,11 @@
 // source order, which is what a boolean-mask gather produces on the CPU.
 #include "i64h_common.h"
 
-#define ROWS_PER_WAVE 128   // of the three launches: what a wave does is a chain of loads and exchanges, so many waves of few rows (32768 rows of 16 buckets, two layers: 512 a wave 11 + 15 + 14 us, 128 a wave
-                            // 4.9 + 5.9 + 5.2, the scan over the waves dealt to all threads of its workgroup)
-#define SMALL_ROWS 512      // up to here one workgroup does all three phases
+// Rows a wave of the three launches: what it does is a chain of loads and exchanges, so many waves of few rows, the scan over the waves dealt to all threads of its workgroup, a row's place from
+// ballots.  32768 rows, two layers, replayed: 16 buckets 31.7 -> 11.7 us, 128 buckets 71 -> 31 (512 rows a wave, one thread a bucket in the scan, a walk over the buckets before).
+#define ROWS_PER_WAVE 128
+#define SMALL_ROWS 512      // up to here a workgroup of 256 threads does all three phases, up to MID_ROWS one of 1024
+#define MID_ROWS 4096
 #define PLAN_THREADS 256
 #define MAX_BUCKETS 256
 
@@ -136,6 +138,16 @@ __global__ __launch_bounds__(MAX_BUCKETS) void bucket_scan_kernel(int32_t* __res
     }
 }
 
+// The lanes whose bucket is this lane's, of those in `valid`: a ballot a bit of the bucket
+__device__ __forceinline__ uint64_t same_bucket(int key, uint64_t valid, int bits) {
+    uint64_t m = valid;
+    for (int i = 0; i < bits; ++i) {
+        const uint64_t on = __ballot((key >> i) & 1);
+        m &= ((key >> i) & 1) ? on : ~on;
+    }
+    return m;
+}
+
 // ---- phase C: stable placement ---------------------------------------------------------------------
 __global__ __launch_bounds__(PLAN_THREADS) void bucket_place_kernel(
     const int32_t* __restrict__ keys, const int32_t* __restrict__ wave_counts, const int32_t* __restrict__ offsets,
@@ -152,23 +164,16 @@ __global__ __launch_bounds__(PLAN_THREADS) void bucket_place_kernel(
     const int64_t s0 = (int64_t)gw * ROWS_PER_WAVE;
     const int64_t s1 = s0 + ROWS_PER_WAVE < R ? s0 + ROWS_PER_WAVE : R;
     const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    const int bits = nb <= 1 ? 0 : 32 - __clz(nb - 1);
     for (int64_t base = s0; base < s1; base += 64) {
         const int64_t s = base + lane;
         const bool valid = s < s1;
-        const int key = valid ? keys[(int64_t)l * R + s] : -1;
-        uint64_t todo = __ballot(valid);
-        int pos = 0;
-        while (todo) {  // one iteration per distinct bucket among these 64 rows
-            const int leader = __ffsll((unsigned long long)todo) - 1;
-            const int b = __shfl(key, leader);
-            const uint64_t m = __ballot(valid && key == b);
-            const int start = cursor[wib][b];
-            if (key == b) pos = start + __popcll(m & lt);
-            __builtin_amdgcn_wave_barrier();
-            if (lane == leader) cursor[wib][b] = start + __popcll(m);
-            __builtin_amdgcn_wave_barrier();
-            todo &= ~m;
-        }
+        const int key = valid ? keys[(int64_t)l * R + s] : 0;
+        const uint64_t m = same_bucket(key, __ballot(valid), bits);
+        const int start = cursor[wib][key], rank = __popcll(m & lt), pos = start + rank;
+        __builtin_amdgcn_wave_barrier();
+        if (valid && rank == 0) cursor[wib][key] = start + __popcll(m);
+        __builtin_amdgcn_wave_barrier();
         if (valid) {
             perm[(int64_t)l * R + pos] = (int32_t)s;
             inv[(int64_t)l * R + s] = pos;
@@ -186,99 +191,105 @@ struct PlanEmbed {
     int H, layers;
 };
 
-// ---- all three phases in one launch when one wave covers the rows (decode-sized steps: R <= SMALL_ROWS) -----------------
-// One workgroup per layer; wave 0 runs phases A and C exactly as the kernels above do for their single wave, the scan of phase B
-// degenerates to the bucket offsets.  Same keys, offsets, permutation: the results are identical to the three-launch path.
-template <bool TABLE>
-__global__ __launch_bounds__(MAX_BUCKETS) void bucket_plan_small_kernel(
+// ---- all three phases in one launch for steps whose rows one workgroup covers, RPT rows a thread ------------------------------------------------
+// One workgroup per layer; 64 rows are a group, whose counts by bucket lie in LDS.  A row's place among its group comes from ballots; as one wave's walk over the buckets that its 64 rows
+// have, a dependent LDS read each, and in three launches from 513 rows on, two layers, replayed, before and after, us: 16 buckets, 2 rows 4.5 -> 4.2, 128 rows 6.4 -> 4.5, 512 14.0 -> 4.7, 1024
+// 18.9 -> 6.9, 4096 20.5 -> 11.1 (1024 in the three launches as they are here: 4.0 + 4.0 + 5.1); 128 buckets, 128 rows 20 -> 5.4, 1024 56 -> 8.4.  Same keys, offsets, permutation: the results are identical to the three-launch path.
+template <bool TABLE, int NT, int RPT>
+__global__ __launch_bounds__(NT) void bucket_plan_small_kernel(
     const int64_t* __restrict__ ids, const int64_t* __restrict__ tables, int64_t table_layer_stride,
     const int32_t* __restrict__ keys_in, int32_t* __restrict__ keys, int64_t* __restrict__ routes, int32_t* __restrict__ tok_slots,
-    int32_t* __restrict__ wave_counts, int32_t* __restrict__ offsets, int32_t* __restrict__ group_offsets, int32_t* __restrict__ perm,
+    int32_t* __restrict__ offsets, int32_t* __restrict__ group_offsets, int32_t* __restrict__ perm,
     int32_t* __restrict__ inv, int32_t* __restrict__ sorted_bucket, int n, int top_k, int64_t V, int nb, PlanEmbed em) {
-    __shared__ int hist[MAX_BUCKETS], cursor[MAX_BUCKETS];
-    __shared__ int skey[SMALL_ROWS];
+    extern __shared__ int cnt[];      // [groups][nb]
+    __shared__ int tot[MAX_BUCKETS], first[MAX_BUCKETS + 1];
+    const int tid = threadIdx.x;
     if ((int)blockIdx.x >= em.layers) {
         // riders of the plan launch: the embedding rows of the same token ids and the start-of-forward reset of the stat slots
         // (both depend on nothing but the ids; as a launch of their own they cost a dispatch and ~4.6 us in front of layer 0)
-        const int t = blockIdx.x - em.layers;
-        for (int64_t i = (int64_t)t * MAX_BUCKETS + threadIdx.x; i < em.stat_words; i += (int64_t)n * MAX_BUCKETS) em.stats[i] = I64H_ORDERED_ZERO;
+        const int at = blockIdx.x - em.layers, t = at * (NT / MAX_BUCKETS) + tid / MAX_BUCKETS;
+        for (int64_t i = (int64_t)at * NT + tid; i < em.stat_words; i += (int64_t)(gridDim.x - em.layers) * NT) em.stats[i] = I64H_ORDERED_ZERO;
+        if (t >= n) return;
         int64_t id = ids[t];
         id = id < 0 ? 0 : (id >= em.emb_vocab ? em.emb_vocab - 1 : id);
         const float4* src = (const float4*)(em.table + id * em.H);
         float4* dst = (float4*)(em.out + (int64_t)t * em.H);
-        for (int i = threadIdx.x; i < em.H / 4; i += MAX_BUCKETS) dst[i] = src[i];
+        for (int i = tid % MAX_BUCKETS; i < em.H / 4; i += MAX_BUCKETS) dst[i] = src[i];
         return;
     }
-    const int l = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
-    const int R = n * top_k;
-    if (tid < nb) hist[tid] = 0;
-    __syncthreads();
-    if (tid < 64) {
-        for (int s = lane; s < R; s += 64) {
-            int key;
-            if (TABLE) {
-                const int k = s / n, t = s - k * n;
-                int64_t id = ids[t];
-                id = id < 0 ? 0 : (id >= V ? V - 1 : id);
-                const int64_t e = tables[(int64_t)l * table_layer_stride + (int64_t)k * V + id];
-                if (routes) routes[(int64_t)l * R + s] = e;
-                key = (int)e * top_k + k;
-                key = key < 0 ? 0 : (key >= nb ? nb - 1 : key);
-                if (tok_slots) {
-                    int32_t* ts = tok_slots + ((int64_t)l * n + t) * (1 + top_k);
-                    ts[1 + k] = 1 + key;
-                    if (k == 0) ts[0] = 0;
-                }
-            } else {
-                key = keys_in[s];
-            }
-            key = key < 0 ? 0 : (key >= nb ? nb - 1 : key);
-            keys[(int64_t)l * R + s] = key;
-            skey[s] = key;
-            atomicAdd(&hist[key], 1);
+    const int l = blockIdx.x, lane = tid & 63, g0 = (tid >> 6) * RPT;
+    const int R = n * top_k, groups = (R + 63) / 64, bits = nb <= 1 ? 0 : 32 - __clz(nb - 1);
+    for (int i = tid; i < groups * nb; i += NT) cnt[i] = 0;
+    int64_t e[RPT];
+    int k[RPT], key[RPT], rank[RPT];
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+        const int s = min(64 * (g0 + j) + lane, R - 1);
+        k[j] = TABLE ? s / n : 0;
+        e[j] = TABLE ? ids[s - k[j] * n] : keys_in[s];
+    }
+    if (TABLE) {
+#pragma unroll
+        for (int j = 0; j < RPT; ++j) {
+            const int64_t id = e[j] < 0 ? 0 : (e[j] >= V ? V - 1 : e[j]);
+            e[j] = tables[(int64_t)l * table_layer_stride + (int64_t)k[j] * V + id];
         }
     }
     __syncthreads();
-    if (tid == 0) {
-        int run = 0;
-        int32_t* o = offsets + (int64_t)l * (nb + 1);
-        for (int i = 0; i < nb; ++i) {
-            o[i] = run;
-            cursor[i] = run;
-            run += hist[i];
-        }
-        o[nb] = run;
-        if (group_offsets) {
-            int32_t* go = group_offsets + (int64_t)l * (nb / top_k + 1);
-            for (int i = 0; i <= nb / top_k; ++i) go[i] = o[i * top_k];
-        }
-    }
-    if (tid < nb) wave_counts[(int64_t)l * nb + tid] = 0;  // what phase B leaves behind for a single wave
-    __syncthreads();
-    if (tid >= 64) return;  // wave-uniform
     const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    for (int base = 0; base < R; base += 64) {
-        const int s = base + lane;
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+        const int s = 64 * (g0 + j) + lane;
         const bool valid = s < R;
-        const int key = valid ? skey[s] : -1;
-        uint64_t todo = __ballot(valid);
-        int pos = 0;
-        while (todo) {
-            const int leader = __ffsll((unsigned long long)todo) - 1;
-            const int b = __shfl(key, leader);
-            const uint64_t m = __ballot(valid && key == b);
-            const int start = cursor[b];
-            if (key == b) pos = start + __popcll(m & lt);
-            __builtin_amdgcn_wave_barrier();
-            if (lane == leader) cursor[b] = start + __popcll(m);
-            __builtin_amdgcn_wave_barrier();
-            todo &= ~m;
+        key[j] = TABLE ? (int)e[j] * top_k + k[j] : (int)e[j];
+        key[j] = key[j] < 0 ? 0 : (key[j] >= nb ? nb - 1 : key[j]);
+        const uint64_t m = same_bucket(key[j], __ballot(valid), bits);
+        rank[j] = __popcll(m & lt);
+        if (!valid) continue;
+        if (rank[j] == 0) cnt[(g0 + j) * nb + key[j]] = __popcll(m);
+        keys[(int64_t)l * R + s] = key[j];
+        if (TABLE) {
+            if (routes) routes[(int64_t)l * R + s] = e[j];
+            if (tok_slots) {
+                int32_t* ts = tok_slots + ((int64_t)l * n + (s - k[j] * n)) * (1 + top_k);
+                ts[1 + k[j]] = 1 + key[j];
+                if (k[j] == 0) ts[0] = 0;
+            }
         }
-        if (valid) {
-            perm[(int64_t)l * R + pos] = (int32_t)s;
-            inv[(int64_t)l * R + s] = pos;
-            if (sorted_bucket) sorted_bucket[(int64_t)l * R + pos] = key;
+    }
+    __syncthreads();
+    if (tid < nb) {      // the rows of a bucket in front of every group
+        int run = 0;
+        for (int g = 0; g < groups; g += 8) {
+            int c[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) c[j] = g + j < groups ? cnt[(g + j) * nb + tid] : 0;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                if (g + j < groups) cnt[(g + j) * nb + tid] = run;
+                run += c[j];
+            }
         }
+        tot[tid] = run;
+    }
+    __syncthreads();
+    for (int b = tid; b <= nb; b += NT) {
+        int run = 0;
+#pragma unroll 8
+        for (int i = 0; i < b; ++i) run += tot[i];
+        first[b] = run;
+        offsets[(int64_t)l * (nb + 1) + b] = run;
+        if (group_offsets && b % top_k == 0) group_offsets[(int64_t)l * (nb / top_k + 1) + b / top_k] = run;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+        const int s = 64 * (g0 + j) + lane;
+        if (s >= R) continue;
+        const int pos = first[key[j]] + cnt[(g0 + j) * nb + key[j]] + rank[j];
+        perm[(int64_t)l * R + pos] = (int32_t)s;
+        inv[(int64_t)l * R + s] = pos;
+        if (sorted_bucket) sorted_bucket[(int64_t)l * R + pos] = key[j];
     }
 }
 
@@ -349,20 +360,21 @@ static int bucketize_common(bool table, const int64_t* ids, const int64_t* table
     I64H_CHECK_ARG(R < (1ll << 31), "bucketize: too many rows");
     int num_waves = (int)((R + ROWS_PER_WAVE - 1) / ROWS_PER_WAVE);
     if (num_waves < 1) num_waves = 1;
-    if (R > 0 && R <= SMALL_ROWS) {  // one wave covers the rows: the three phases in one launch
+    const int64_t lds = (R + 63) / 64 * nb * 4;
+    if (R > 0 && R <= MID_ROWS && lds <= 32768) {  // one workgroup covers the rows: the three phases in one launch
         PlanEmbed em = {nullptr, nullptr, nullptr, 0, 0, 0, L};
         if (riders && table) {
             em = *riders;
             em.layers = L;
             *riders_done = true;
         }
-        const int extra = em.table ? n : 0;
-        if (table)
-            hipLaunchKernelGGL(bucket_plan_small_kernel<true>, dim3(L + extra), dim3(MAX_BUCKETS), 0, st, ids, tables, layer_stride, keys_in, keys,
-                               routes, tok_slots, workspace, offsets, group_offsets, perm, inv, sorted_bucket, n, top_k, V, nb, em);
-        else
-            hipLaunchKernelGGL(bucket_plan_small_kernel<false>, dim3(L), dim3(MAX_BUCKETS), 0, st, ids, tables, layer_stride, keys_in, keys,
-                               routes, tok_slots, workspace, offsets, group_offsets, perm, inv, sorted_bucket, n, top_k, V, nb, em);
+        auto launch = [&](auto kern, int threads) {
+            const int extra = em.table ? (int)i64h_cdiv(n, threads / MAX_BUCKETS) : 0;
+            hipLaunchKernelGGL(kern, dim3(L + extra), dim3(threads), (size_t)lds, st, ids, tables, layer_stride, keys_in, keys, routes, tok_slots, offsets, group_offsets, perm, inv,
+                               sorted_bucket, n, top_k, V, nb, em);
+        };
+        if (R <= SMALL_ROWS) table ? launch(bucket_plan_small_kernel<true, 256, 2>, 256) : launch(bucket_plan_small_kernel<false, 256, 2>, 256);
+        else table ? launch(bucket_plan_small_kernel<true, 1024, 4>, 1024) : launch(bucket_plan_small_kernel<false, 1024, 4>, 1024);
         I64H_CHECK_LAUNCH();
         return 0;
     }
