@@ -704,7 +704,7 @@ typedef struct {
 int i64h_moe_plan(const i64h_moe_plan_args* d, void* stream);
 /* i64h_streams_step with i64h_route_topk on the rows of h behind it (r: W, K = the rows' width, at most 17 rows of W, no groups; r->h is not read, and d may leave h and h16 away), and
  * for n <= 128 i64h_moe_plan on that choice (m may be NULL), all in one launch.  sync int32 [32 * 17] (with m): zeros before the first launch, zeros again behind every one; launches that share it
- * follow each other. */
+ * follow each other.  With a mixture's sum in d: the weights, indexes and gates that r writes lie apart from those that d reads, or at the same place with as many choices a row. */
 int i64h_streams_route(const i64h_streams_args* d, const i64h_route_args* r, const i64h_moe_plan_args* m, int32_t* sync, void* stream);
 typedef struct {
     const float* Y;

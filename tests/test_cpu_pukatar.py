@@ -147,3 +147,32 @@ def test_oracle_runs_every_shape():
         layers = []
         z = R.forward(config_of(name), make_weights(name), tokens(name, 12, 1), layers)
         assert z.shape == (12, SHAPES[name]["vocab"]) and bool(torch.isfinite(z).all()) and len(layers) == len(R.layer_runs(config_of(name)))
+
+
+@pytest.mark.parametrize("n", [5, 300])
+def test_a_mixtures_weights_outlive_the_choice_of_the_next(monkeypatch, n):
+    """The launch that sums one mixture also chooses the next one's experts, rows in any order: unless both choose as many, the two choices' weights lie apart."""
+    from vllm_i64_amd import hybrid_runner, ops_dense, pukatar
+    from vllm_i64_amd.config import PukatarConfig
+    steps, launches = [], ("linear", "embed_scaled", "streams_step", "rot_prep", "kattn", "rot_post", "route_topk", "moe_plan", "moe_combine", "causal_conv", "gdn_gates", "gdn_scan", "gate_norm",
+                           "rec_step", "rec_tiles")
+
+    class Recorder:
+        def __getattr__(self, name):
+            if name not in launches:
+                return getattr(ops_dense, name)
+            return lambda *a, **kw: steps.append(kw) if name == "streams_step" else None
+
+    monkeypatch.setattr(pukatar, "D", Recorder())
+    monkeypatch.setattr(hybrid_runner, "D", Recorder())
+    monkeypatch.setattr(hybrid_runner, "upload", lambda v, dtype, device: torch.tensor(v, dtype=dtype, device=device))
+    model = pukatar.PukatarModel(PukatarConfig.from_dict(config_of("plain")), make_weights("plain"), device="cpu", dtype="float32", max_seqs=1, num_kv_blocks=32, kv_block=16)
+    for _ in range(2):
+        i = torch.arange(n)
+        model.forward(i % 64, i.to(torch.int32), torch.zeros(n, dtype=torch.int32), tokens_per_seq=[n])
+    both = [kw for kw in steps if kw.get("moe") is not None and kw.get("route") is not None]
+    assert len(both) == 2
+    for kw in both:
+        old, new = kw["moe"]["wgt"], kw["route"]["wgt"]
+        assert kw["moe"]["top"] != kw["route"]["top"]
+        assert old.data_ptr() + 4 * n * kw["moe"]["top"] <= new.data_ptr() or new.data_ptr() + 4 * n * kw["route"]["top"] <= old.data_ptr()

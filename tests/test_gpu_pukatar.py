@@ -534,3 +534,14 @@ def test_trace_command_on_a_checkpoint_folder(dev, tmp_path):
     c = torch.from_numpy(np.fromfile(out / "2.f32", dtype="<f4").reshape(-1, V))
     assert not (out / "1.f32").exists()
     assert agrees(a, want[[0, 9]], "float32") and agrees(c, torch.stack([want[20], want[2]]), "float32")
+
+
+@pytest.mark.parametrize("tops,n", [((1, 2, 3), 70), ((3, 1, 2), 70), ((2, 2, 2), 300), ((1, 2), 4200)])
+def test_mixtures_one_behind_the_other_choose_as_many_experts_as_each_has(dev, monkeypatch, tops, n):
+    """Prompts with and without the plan in the norm's launch, of more rows than the card holds workgroups, against the oracle."""
+    monkeypatch.setitem(SHAPES, "row", {"architecture": "Pukatar", "vocab": 64, "width": 64, "norm": {"eps": 1e-6},
+                                        "layers": [{"type": "attention", "mixer": {"heads": 2, "dim": 16, "vdim": 8, "scale": 0.25, "mask": {"size": 9}},
+                                                    "mlp": {"kind": "moe", "expert": {"ff": 24, "limit": 2.0}, "router": {"experts": 4, "top": t}, "shared": {"ff": 24, "limit": 2.0}}} for t in tops],
+                                        "ranks": {}})
+    model = make_model("row", "float32", dev, max_tokens=n)
+    whole_prompt(model, "row", tokens("row", n, 3), "float32", layers_too=True)

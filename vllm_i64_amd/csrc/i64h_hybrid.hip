@@ -1167,6 +1167,16 @@ int i64h_streams_route(const i64h_streams_args* dp, const i64h_route_args* rp, c
     I64H_CHECK_ARG(r.E > 0 && r.E + (r.gate_out ? 1 : 0) <= RT_NORM_ENTRIES && r.top > 0 && r.top <= r.E && r.groups <= 1, "streams_route: %d entries in %d groups, top %d (one group of at most %d with a gate's row)",
                    r.E, r.groups, r.top, RT_NORM_ENTRIES);
     I64H_CHECK_ARG(r.W && (uintptr_t)r.W % 8 == 0 && r.K == d.W && !d.rows && r.n == d.n && r.idx && r.wgt && !(r.sigmoid_scores && r.chosen_softmax), "streams_route: the router does not fit the rows");
+    // A row's workgroup reads the weights and rows of the mixture that it sums when it starts and writes its choice when it ends, and rows wait for nobody: what one reads must not be what another writes.
+    if (d.moe_y) {
+        const struct { const void* at; int32_t row; } in[] = {{d.moe_wgt, d.moe_top}, {d.moe_row, d.moe_top}, {d.moe_gate, 1}}, out[] = {{r.wgt, r.top}, {r.idx, r.top}, {r.gate_out, 1}};
+        for (const auto& i : in)
+            for (const auto& o : out) {
+                const uintptr_t a = (uintptr_t)i.at, b = (uintptr_t)o.at;
+                I64H_CHECK_ARG(!a || !b || (a == b && i.row == o.row) || a + 4 * (uintptr_t)d.n * i.row <= b || b + 4 * (uintptr_t)d.n * o.row <= a,
+                               "streams_route: the choice lies over what other rows of the mixture in front still read");
+            }
+    }
     if (pp) {
         const i64h_moe_plan_args& m = *pp;
         I64H_CHECK_ARG(sync && d.n <= RT_PLAN_ROWS, "streams_route: a plan of %lld rows (at most %d), with counters", (long long)d.n, RT_PLAN_ROWS);

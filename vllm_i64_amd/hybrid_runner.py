@@ -433,7 +433,7 @@ class HybridRunner:
         B.act = torch.empty(n * max(act, 1), **f32)
         B.ey = torch.empty(n * g, model.cfg.width, **f32) if t else None   # the outputs, grouped by expert
         B.idx = torch.empty(n * max(t, 1), **i32)
-        B.wgt = torch.empty(n * max(t, 1), **f32)
+        B.wgt, B.wgt_next = torch.empty(n * max(t, 1), **f32), torch.empty(n * max(t, 1), **f32)      # the choice's weights, and those of the one that follows (_moe_read)
         B.pair_token = torch.empty(n * max(g, 1), **i32)
         B.pair_row = torch.empty(n * max(t, 1), **i32)
         B.pair_wgt = torch.empty(n * max(g, 1), **f32)
@@ -524,10 +524,12 @@ class HybridRunner:
         return f.entries + int(bool(f.shared_ff and f.shared_gate)) <= D.ROUTE_ENTRIES and f.groups <= 1 and self._moe_merges()
 
     def _moe_read(self, B, d, n, h, h16) -> dict:
-        """What the launch that norms a mixture's input is to write and choose: h stays away where everybody behind it reads rows in bf16."""
+        """What the launch that norms a mixture's input is to write and choose: h stays away where everybody behind it reads rows in bf16.  The launch may also sum the mixture in front,
+        whose weights another row's workgroup still reads when this choice is written (they lie apart by rows only where both choose as many experts): two sets take turns."""
         f = d["mlp"]
         if not self._routes_in_norm(f):
             return dict(h=h, h16=h16)
+        B.wgt, B.wgt_next = B.wgt_next, B.wgt
         bare = h16 is not None and f.entries == f.experts and self._experts_read16(d, n, d["merged"] and B.joined)
         return dict(h=None if bare else h, h16=h16, route=self._route(B, d), **(dict(plan=self._plan(B, d), sync=B.sync) if n <= D.PLAN_ROWS else {}))
 
