@@ -308,6 +308,54 @@ def test_prefill_attention_whose_scores_climb(dev, step):
     assert torch.equal(run(37), out[37:])
 
 
+@pytest.mark.parametrize("heads,block", [(8, 16), (3, 24)])
+def test_prefill_attention_keeps_values_near_the_end_of_the_range(dev, heads, block):
+    """Values of 2^120 under scores that climb to 2^7.5 above a row's reference: the sums of weights up to 2^8 would leave 32 bits, those of weights up to one, which are at most 2^120 x 5 x 64,
+    do not.  Some sequences of a tile have such values and some have not (theirs are the bits they have without); one has an infinity, and what it reaches is no finite number."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(block)
+    hd, kvh, lens = 64, heads if heads == 3 else 2, [7, 64 * 2 + 5, 64 * 2 + 5, 90, 130]
+    big, infinite = (1, 3), 4
+    nb = [(L + block - 1) // block for L in lens]
+    bt = torch.full((len(lens), max(nb)), -1, dtype=torch.int32)
+    k, v = torch.zeros(sum(nb), block, kvh, hd).bfloat16(), torch.zeros(sum(nb), block, kvh, hd).bfloat16()
+    qs, refs, at = [], [], 0
+    for i, L in enumerate(lens):
+        ks = torch.randn(L, kvh, hd, generator=g) * 0.5
+        ks[:, :, 5] = (torch.arange(L) // 64).float().clamp(max=1).view(L, 1) * 8.0
+        vs = torch.randn(L, kvh, hd, generator=g).clamp(-4, 4) * (2.0 ** 120 if i in big else 1.0)
+        if i == infinite:
+            vs[64, 0, 3] = float("inf")
+        ks, vs = ks.bfloat16(), vs.bfloat16()
+        q = torch.randn(L, heads, hd, generator=g) * 0.5
+        q[:, :, 5] = 7.5 * 0.6931472
+        s = torch.einsum("thd,shd->ths", q.double(), ks.double().repeat_interleave(heads // kvh, 1)) / hd ** 0.5
+        w = torch.softmax(s.masked_fill(torch.arange(L).view(1, 1, L) > torch.arange(L).view(L, 1, 1), float("-inf")), -1)
+        refs.append(torch.einsum("ths,shd->thd", w, vs.double().nan_to_num(posinf=0.0).repeat_interleave(heads // kvh, 1)))
+        qs.append(q)
+        bt[i, :nb[i]] = torch.arange(at, at + nb[i], dtype=torch.int32)
+        k[at:at + nb[i]].view(-1, kvh, hd)[:L], v[at:at + nb[i]].view(-1, kvh, hd)[:L] = ks, vs
+        at += nb[i]
+
+    def run(v):
+        ctx = torch.cat([torch.arange(1, L + 1) for L in lens]).to(torch.int32).to(dev)
+        slot = torch.cat([torch.full((L,), i) for i, L in enumerate(lens)]).to(torch.int32).to(dev)
+        return ops.paged_attn(torch.cat(qs).to(dev), k.to(dev), v.to(dev), bt.to(dev), ctx, slot_ids=slot, splits=1).cpu().split(lens)
+
+    together = run(v)
+    alone = run(torch.where(v.float().abs() > 100.0, 0.0, v.float()).bfloat16())
+    for i, (got, want) in enumerate(zip(together, refs)):
+        if i == infinite:
+            reached = torch.zeros(lens[i], heads, hd, dtype=torch.bool)
+            reached[64:, :heads // kvh, 3] = True
+            assert (~torch.isfinite(got[reached])).all()
+            reached[49:64, :heads // kvh, 3] = True      # (rows of a tile of 16 that sees it may meet it with a weight of zero)
+            got, want = got[~reached], want[~reached]
+        # (a score's sum within 16 roundings of magnitudes below 15, a weight as much relative to itself, the result twice that)
+        assert torch.isfinite(got).all() and (got.double() - want).abs().max() <= 2 * 16 * 2.0 ** -24 * 15 * 4 * (2.0 ** 120 if i in big else 1.0), i
+        assert i in big or i == infinite or torch.equal(alone[i], together[i])
+
+
 @pytest.mark.parametrize("rows,buckets", [(1, 5), (65, 1), (512, 256), (513, 1), (640, 3), (641, 16), (1023, 17), (2049, 130), (4000, 256), (4096, 17), (4097, 200), (9000, 256), (70001, 64)])
 def test_stable_buckets_of_many_rows(dev, rows, buckets):
     """Rows at the edges of a wave's share, bucket counts that divide the scan's threads or not, empty buckets: a stable sort by bucket, whole numbers exactly."""

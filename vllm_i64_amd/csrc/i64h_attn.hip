@@ -685,7 +685,7 @@ __global__ __launch_bounds__(GS * 64, I64H_PF_OCC) void paged_attn_prefill_bf16_
 // 291 -> 248, one of 481 17.6 -> 14.1, 1500 + 77 52 -> 42.5; 12 heads over 12, 2 of 2048 204 -> 118; 16 over 8 150 -> 108; 32 over 4 182 -> 160; forty of 16 rows
 // 8.5 -> 8.5.  With three tiles in LDS (and two on their way) 250, 14.1, 43.0, 137, 115, 165: fewer workgroups fit.  Four waves a SIMD spill (309).
 // 8-bit caches stay with the form above, which converts on the way into LDS.
-#define PF_SLACK 8.0f      // how far above its reference a row's score may lie: weights up to 2^8, which 32-bit sums hold as well as those up to one
+#define PF_SLACK 8.0f      // how far above its reference a row's score may lie: weights up to 2^8, which 32-bit sums hold as well as those up to one (of values to 1e36; beyond, a row may go round again)
 template <int GS>
 __global__ __launch_bounds__(GS * 64, 3) void paged_attn_prefill_direct_kernel(const float* __restrict__ q, const __hip_bfloat16* __restrict__ k_cache,
                                                                          const __hip_bfloat16* __restrict__ v_cache, const int32_t* __restrict__ block_table,
@@ -703,6 +703,7 @@ __global__ __launch_bounds__(GS * 64, 3) void paged_attn_prefill_direct_kernel(c
     const int my_slot = valid ? (slot_ids ? slot_ids[r] : r) : -1;
     const int my_ctx = valid ? ctx_len[r] : 0;
     bool done = !valid;
+    float slack = PF_SLACK;      // this lane's row's
     float olo = 0.0f, ohi = 0.0f;  // range of the rows this lane stores (with zero, as the quantizer's range has it)
     const int bshift = (block & (block - 1)) == 0 ? __builtin_ctz(block) : -1;
 
@@ -824,13 +825,13 @@ __global__ __launch_bounds__(GS * 64, 3) void paged_attn_prefill_direct_kernel(c
             float mx = -INFINITY;
 #pragma unroll
             for (int t = 0; t < 4; ++t) mx = fmaxf(mx, fmaxf(fmaxf(sc[t][0], sc[t][1]), fmaxf(sc[t][2], sc[t][3])));
-            if (__ballot(mx > m + PF_SLACK)) {      // some row's first tile, or far above its reference: a new one, what there is rescaled (rare after the first tiles)
+            if (__ballot(mx > m + slack)) {      // some row's first tile, or far above its reference: a new one, what there is rescaled (rare after the first tiles)
                 // over the four lanes of a query row (lane ^ 16, lane ^ 32) through register swaps, no LDS round trip
                 const PairF sr = swap_rows(mx);
                 mx = fmaxf(sr.lo, sr.hi);
                 const PairF sh = swap_halves(mx);
                 mx = fmaxf(sh.lo, sh.hi);
-                const float mn = mx > m + PF_SLACK ? mx : m;  // by the row's own scores: its neighbours in the tile change nothing in its result
+                const float mn = mx > m + slack ? mx : m;  // by the row's own scores: its neighbours in the tile change nothing in its result
                 const float alpha = (mn == -INFINITY) ? 1.0f : exp2f(m - mn);
 #pragma unroll
                 for (int j = 0; j < 5; ++j) acc[j] *= alpha;
@@ -884,6 +885,25 @@ __global__ __launch_bounds__(GS * 64, 3) void paged_attn_prefill_direct_kernel(c
             }
             if (tile < tiles) step(tile, S0, S1);
             __builtin_amdgcn_s_waitcnt(0x0f70);      // (nothing is on its way into LDS when a pass ends)
+        }
+        // Sums over weights up to 2^PF_SLACK may leave the range where those over weights up to one stay in it: such rows are taken again, under their
+        // running maximum (every wave goes round with them).  Finding out costs nothing to 2 us: 8 of 2048 255 | 255, one of 481 14.0 | 13.7, 1500 + 77 40.8 | 41.7, 2 of 2048 of 16 over 8 103 | 105.
+        float none = 0.0f;      // (0 where all sums are finite)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) none = fmaf(acc[j][e], 0.0f, none);
+        const unsigned long long odd = __ballot(active && slack > 0.0f && none != 0.0f);
+        bool round = odd != 0;
+        if constexpr (GS > 1) {      // (words of the tiles, which nobody reads or loads any more: fewer workgroups would fit with LDS of its own)
+            __syncthreads();
+            if (lane == 0) ((int*)s0)[wid] = round;
+            __syncthreads();
+            round = __ballot(lane < GS && ((const int*)s0)[lane & (GS - 1)]) != 0;
+        }
+        if (round) {
+            if ((odd | odd >> 16 | odd >> 32 | odd >> 48) >> c & 1) slack = 0.0f;
+            continue;
         }
         const float lsum = acc[4][0];  // every row of the ones fragment carries the normaliser of query row c
         if (active) {
