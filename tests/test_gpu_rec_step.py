@@ -141,3 +141,117 @@ def test_tiles_from_the_projections(H, d, dv, ranks, taps, runs, delta):
     idle = torch.ones(slots, dtype=torch.bool, device=DEV)
     idle[own] = False
     assert torch.equal(s2[idle], state[idle])
+
+
+class Layer:
+    """A recurrence's operands for runs of rows, and the same in 64 bits on the CPU."""
+    def __init__(self, H, d, dv, ranks, taps, runs, delta):
+        self.H, self.d, self.dv, self.taps, self.runs, self.delta = H, d, dv, taps, runs, delta
+        g = torch.Generator().manual_seed(H * d + dv + len(runs))
+        r = lambda *s, std=1.0: torch.randn(*s, generator=g) * std
+        n, nd, rv = sum(runs), H * d, H * dv
+        C, slots = 2 * nd + rv, len(runs) + 2
+        pad4 = lambda x: (x + 3) // 4 * 4
+        self.a_off = pad4(C)
+        self.z_off = self.a_off + pad4(ranks[0])
+        self.b_off = self.z_off + max(pad4(ranks[1]), pad4(rv))
+        self.P = r(n, pad4(self.b_off + H))
+        self.a, self.bias, self.rate = r(nd, ranks[0], std=ranks[0] ** -0.5).bfloat16(), r(nd), torch.rand(nd, generator=g) + 0.1
+        self.z, self.norm_w = r(rv, ranks[1], std=ranks[1] ** -0.5).bfloat16(), r(dv)
+        self.conv_w, self.conv, self.state = r(C, taps, std=0.5), r(slots, taps - 1, C), r(slots, H, dv, d, std=0.3)
+        self.own = torch.randperm(slots, generator=g)[:len(runs)]
+        self.first = [(0, 700, 1, 2, 3)[i % 5] for i in range(len(runs))]
+
+    def launch(self, P):
+        n, nseg, rv, nd = len(P), len(self.runs), self.H * self.dv, self.H * self.d
+        gpu = lambda t: t.to(DEV).clone()
+        pos = torch.cat([torch.arange(m) + p for m, p in zip(self.runs, self.first)]).to(torch.int32).to(DEV)
+        slot = torch.cat([s.repeat(m) for m, s in zip(self.runs, self.own)]).to(torch.int32).to(DEV)
+        state, conv, out = gpu(self.state), gpu(self.conv), torch.full((n, rv), float("nan"), device=DEV)
+        kw = dict(heads=self.H, dim=self.d, vdim=self.dv, a=gpu(self.a), a_off=self.a_off, a_bias=gpu(self.bias), a_rate=gpu(self.rate), norm_w=gpu(self.norm_w), eps=1e-6, positions=pos,
+                  slot_ids=slot, state=state, n=n, out=out, q_scale=self.d ** -0.5, q_off=0, z_off=self.z_off)
+        kw.update(dict(conv_w=gpu(self.conv_w), conv=conv, b_off=self.b_off, unit_eps=1e-6, z=gpu(self.z), sigmoid=True) if self.delta else dict(k_off=nd, v_off=2 * nd))
+        if max(self.runs) == 1:
+            D.rec_step(gpu(P), **kw)
+        else:
+            seg = torch.tensor([0, *torch.tensor(self.runs).cumsum(0).tolist()], dtype=torch.int32, device=DEV)
+            room = lambda: torch.full((n, rv), float("nan"), device=DEV)
+            D.rec_tiles(gpu(P), seg_start=seg, nseg=nseg, work=torch.full((D.scan_work_floats(n, nseg, self.H, self.d),), float("nan"), device=DEV), r=room(), x=room(), **kw)
+        return out.cpu(), state.cpu()[self.own]
+
+    def exact(self, P):
+        H, d, dv, nd = self.H, self.d, self.dv, self.H * self.d
+        outs, states, at = [], [], 0
+        map_ = lambda x, w: (x.bfloat16().double()[:, None, :] * w.double()[None]).sum(-1)
+        for m, slot, pos in zip(self.runs, self.own, self.first):
+            p = P[at:at + m].double()
+            at += m
+            f = torch.exp(-self.rate.double() * torch.logaddexp(torch.zeros(1).double(), map_(p[:, self.a_off:self.a_off + self.a.shape[1]].float(), self.a) + self.bias.double())).view(m, H, d)
+            x = p[:, :2 * nd + H * dv]
+            if self.delta:
+                back = self.conv[slot].double().clone()
+                back[:max(0, self.taps - 1 - pos)] = 0      # (before the sequence's first token)
+                rows = torch.cat([back, x])
+                x = sum(rows[k:k + m] * self.conv_w[:, k].double() for k in range(self.taps))
+                x = x * torch.sigmoid(x)
+            q, k, v = x[:, :nd].view(m, H, d), x[:, nd:2 * nd].view(m, H, d), x[:, 2 * nd:].view(m, H, dv)
+            if self.delta:
+                unit = lambda t: t / torch.sqrt((t * t).sum(-1, keepdim=True) + 1e-6)
+                q, k, beta = unit(q), unit(k), torch.sigmoid(p[:, self.b_off:self.b_off + H])
+                gate = torch.sigmoid(map_(p[:, self.z_off:self.z_off + self.z.shape[1]].float(), self.z))
+            else:
+                zc = p[:, self.z_off:self.z_off + H * dv]
+                gate = zc * torch.sigmoid(zc)
+            S, o = self.state[slot].double() * (pos != 0), torch.zeros(m, H, dv).double()
+            for t in range(m):
+                S = S * f[t][:, None, :]
+                u = beta[t][:, None] * (v[t] - (S * k[t][:, None, :]).sum(-1)) if self.delta else v[t]
+                S = S + u[:, :, None] * k[t][:, None, :]
+                o[t] = (S * q[t][:, None, :]).sum(-1) * d ** -0.5
+            outs.append((o / torch.sqrt((o * o).mean(-1, keepdim=True) + 1e-6) * self.norm_w.double()).view(m, H * dv) * gate)
+            states.append(S)
+        return torch.cat(outs), torch.stack(states), o
+
+
+LAYERS = [(3, 64, 64, (8, 136), 3, (17, 3, 40)), (2, 68, 60, (40, 72), 2, (31, 1, 48)), (2, 128, 128, (136, 40), 4, (50, 1, 20)), (2, 64, 68, (40, 8), 8, (1,) * 5), (3, 128, 64, (136, 72), 4, (1,) * 7)]
+
+
+def _near(got, want):
+    """32-bit sums of some hundred terms through up to 50 steps and a division by a row's root mean square, against 64 bits: 1e-4 of the largest value."""
+    ok = torch.isfinite(want)
+    assert torch.equal(torch.isfinite(got), ok)
+    assert (got[ok].double() - want[ok]).abs().max() <= 1e-4 * want[ok].abs().max()
+
+
+@pytest.mark.parametrize("delta", [True, False])
+@pytest.mark.parametrize("H,d,dv,ranks,taps,runs", LAYERS)
+def test_infinite_weights_of_the_maps(H, d, dv, ranks, taps, runs, delta):
+    """A decay of an infinite sum is zero or one and a gate too: ranks that are no whole steps of the products meet nothing but their own values."""
+    L = Layer(H, d, dv, ranks, taps, runs, delta)
+    _near(L.launch(L.P)[0], L.exact(L.P)[0])
+    inf = float("inf")
+    L.a[1, 0], L.a[d, ranks[0] - 1], L.a[H * d - 1, ranks[0] - 6] = inf, -inf, inf
+    L.z[0, 1], L.z[dv, ranks[1] - 8] = inf, -inf
+    got, want = L.launch(L.P), L.exact(L.P)
+    assert torch.isfinite(want[0]).all()
+    _near(got[0], want[0]), _near(got[1], want[1])
+
+
+@pytest.mark.parametrize("what", ["q", "k", "v", "decay", "strength", "gate"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), 3e38])
+@pytest.mark.parametrize("delta", [True, False])
+@pytest.mark.parametrize("H,d,dv,ranks,taps,runs", LAYERS)
+def test_a_row_that_is_no_number(H, d, dv, ranks, taps, runs, delta, what, value):
+    """... reaches what 64 bits say it reaches: its own columns, its head or its sequence, from its token on, and no other run's bits."""
+    L = Layer(H, d, dv, ranks, taps, runs, delta)
+    P, row = L.P.clone(), sum(runs[:-1]) + runs[-1] * 2 // 3
+    P[row, {"q": d + 1, "k": H * d + d + 2, "v": 2 * H * d + 3, "decay": L.a_off + ranks[0] - 2, "strength": L.b_off + 1, "gate": L.z_off + min(ranks[1], dv) - 1}[what]] = value
+    (got, gs), (want, ws, _), (clean, cs) = L.launch(P), L.exact(P), L.launch(L.P)
+    first = sum(runs[:-1])
+    assert torch.equal(got[:first], clean[:first]) and torch.equal(gs[:-1], cs[:-1])
+    assert torch.isfinite(got[first:row]).all()
+    if value != 3e38:
+        if what == "v":      # (an infinite value's sums over channels and over tokens are an infinity here and none there: a head's norm makes zeros of its row or nothing)
+            assert (~torch.isfinite(got[row:, 3])).all()
+            got[row:, :dv], want[row:, :dv] = 0, 0
+        _near(got, want), _near(gs, ws)

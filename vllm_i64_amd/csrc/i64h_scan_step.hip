@@ -189,7 +189,7 @@ __global__ __launch_bounds__(256) void gate_map_kernel(const i64h_rec_step_args 
         v[b] = acc[b] = dn_v4f{0, 0, 0, 0};
         if (ok && col < V) v[b] = *(const dn_v4f*)(y + t * ldy + a * V + col);
     }
-    for (int k0 = 0; k0 < p.z_rank; k0 += 128) {      // (four steps' loads together, none behind a branch: past the rank the rows' values are zeros, past the last column nobody uses the sum)
+    for (int k0 = 0; k0 < p.z_rank; k0 += 128) {      // (four steps' loads together, none behind a branch: past the rank both factors are zeros, past the last column nobody uses the sum)
         dn_v4f u[4][2];
         dn_v4u m[4][NV];
 #pragma unroll
@@ -203,7 +203,11 @@ __global__ __launch_bounds__(256) void gate_map_kernel(const i64h_rec_step_args 
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             dn_v4u x{dn_bf16_pair(u[s][0][0], u[s][0][1]), dn_bf16_pair(u[s][0][2], u[s][0][3]), dn_bf16_pair(u[s][1][0], u[s][1][1]), dn_bf16_pair(u[s][1][2], u[s][1][3])};
-            if (k0 + 32 * s + 8 * g >= p.z_rank) x = dn_v4u{0, 0, 0, 0};
+            if (k0 + 32 * s + 8 * g >= p.z_rank) {
+                x = dn_v4u{0, 0, 0, 0};
+#pragma unroll
+                for (int b = 0; b < NV; ++b) m[s][b] = dn_v4u{0, 0, 0, 0};
+            }
 #pragma unroll
             for (int b = 0; b < NV; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_v8bf, m[s][b]), __builtin_bit_cast(dn_v8bf, x), acc[b], 0, 0, 0);
         }

@@ -65,15 +65,17 @@ __device__ __forceinline__ void st_raw(const i64h_gdn_args& p, const i64h_rec_st
         for (int b = 0; b < NP / 64; ++b) acc[b] = dn_v4f{0, 0, 0, 0};
 #pragma unroll 4
         for (int k0 = 0; k0 < r.a_rank; k0 += 32) {
-            // (no branch at a load: past the rank the rows' values are zeros, past the last channel nobody uses the sum; four steps' loads asked for together take 139 registers for 79 and
-            // longer, 70 us for 58)
+            // (no branch at a load: past the rank both factors are zeros - an infinite weight times a zero would be no number -, past the last channel nobody uses the sum; four steps' loads
+            // asked for together take 139 registers for 79 and longer, 70 us for 58)
             const int k = min(k0 + 8 * g, r.a_rank - 8);
+            const bool past = k != k0 + 8 * g;
             const dn_v4f u = *(const dn_v4f*)(arow + k), v = *(const dn_v4f*)(arow + k + 4);
             dn_v4u x{dn_bf16_pair(u[0], u[1]), dn_bf16_pair(u[2], u[3]), dn_bf16_pair(v[0], v[1]), dn_bf16_pair(v[2], v[3])};
-            if (k != k0 + 8 * g) x = dn_v4u{0, 0, 0, 0};
+            if (past) x = dn_v4u{0, 0, 0, 0};
 #pragma unroll
             for (int b = 0; b < NP / 64; ++b) {
-                const dn_v4u m = *(const dn_v4u*)(map + (int64_t)min(16 * (w + 4 * b) + c, N - 1) * r.a_rank + k);
+                dn_v4u m = *(const dn_v4u*)(map + (int64_t)min(16 * (w + 4 * b) + c, N - 1) * r.a_rank + k);
+                if (past) m = dn_v4u{0, 0, 0, 0};
                 acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_v8bf, m), __builtin_bit_cast(dn_v8bf, x), acc[b], 0, 0, 0);
             }
         }
