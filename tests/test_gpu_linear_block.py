@@ -238,3 +238,28 @@ def test_parts_of_32_bit_rows(dev, use_form, form):
     want = (z * torch.sigmoid(z) * up.double()).float()
     ok = torch.isfinite(ref) & torch.isfinite(up)
     assert torch.equal(out.cpu()[ok].isnan(), want[ok].isnan()) and out.cpu()[(ref.isnan() | up.isnan())].isnan().all()
+
+
+def test_a_row_of_nan_among_32_bit_rows_takes_no_longer(dev):
+    """Sums that are no number are taken again term by term, up to the first term that makes them none: a sequence that is lost does not hold up the step's others (15 times as long if
+    every term is taken; the smallest of some times each, and a bound far from both)."""
+    from vllm_i64_amd import ops_dense as D
+    g = torch.Generator().manual_seed(1)
+    a, w, out = torch.randn(376, 1024, generator=g).to(dev), bf16(torch.randn(5760, 1024, generator=g)).to(dev), torch.empty(376, 5760, device=dev)
+
+    def fastest():
+        best = float("inf")
+        for _ in range(8):
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            e[0].record()
+            for _ in range(5):
+                D.linear(a, w, out, exact=True)
+            e[1].record()
+            torch.cuda.synchronize()
+            best = min(best, e[0].elapsed_time(e[1]))
+        return best
+
+    numbers = fastest()
+    a[3] = float("nan")
+    assert fastest() < 4 * numbers
+    assert out[3].isnan().all() and int(out.isnan().sum()) == 5760
