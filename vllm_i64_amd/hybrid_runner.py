@@ -200,12 +200,11 @@ class HybridRunner:
             ws = B.attn_ws[key] = torch.empty(max(1, floats(splits)), dtype=torch.float32, device=self.device)
         return splits, ws
 
-    def _scan_work(self, n: int, nseg: int, longest: int, scans, delta: bool, rec: bool = False) -> Dict[tuple, torch.Tensor]:
-        """The workspace of a step's scans by (heads, dim, vdim), for those of `scans` whose runs are worth the form that takes one, alone or (rec) from the projections.  The caller holds it for
+    def _scan_work(self, n: int, nseg: int, longest: int, scans, delta: bool, recs=()) -> Dict[tuple, torch.Tensor]:
+        """The workspace of a step's scans by (heads, dim, vdim), for those of `scans` whose runs are worth the form that takes one, alone or (recs) from the projections.  The caller holds it for
         the step and no longer: 27 KB a tile of 16 rows and head of 128 would otherwise lie beside every kept buffer set.  Where the card has no room for
         it the scans go token by token: the same values in another order of the sums."""
-        worth = D.rec_in_tiles if rec else D.scan_in_tiles
-        sizes = {s: D.scan_work_floats(n, nseg, s[0], s[1]) for s in scans if worth(n, nseg, longest, *s, delta=delta)}
+        sizes = {s: D.scan_work_floats(n, nseg, s[0], s[1]) for s in scans if (D.rec_in_tiles if s in recs else D.scan_in_tiles)(n, nseg, longest, *s, delta=delta)}
         if not sizes:
             return {}
         try:
@@ -334,12 +333,21 @@ class HybridRunner:
         if nseg == n and taps <= D.REC_STEP_TAPS:
             D.rec_step(P, heads=r.heads, dim=r.dim, vdim=r.vdim, n=n, exact=self.exact, **own)
             return True
-        # (linear attention in narrow heads has nothing to save but the decays' way through memory: 32 heads of 64, runs of 700 and 300, 55.6 us in launches of its own, 56.2 here; of 128, 16
-        # heads, 2956 rows 145 and 131; the delta rule 104 and 90, 270 and 191)
-        if ws is None or self.exact or r.vdim % 4 or taps > D.REC_TILE_TAPS or (taps == 0 and r.dim <= 64):
+        if ws is None or not self._rec_tiles_take(r, taps):
             return False
         D.rec_tiles(P, seg_start=seg, nseg=nseg, work=ws, r=R, x=X, heads=r.heads, dim=r.dim, vdim=r.vdim, n=n, **own)
         return True
+
+    def _rec_tiles_take(self, r, taps: int) -> bool:
+        """Whether prompts of a recurrence may go from the projections in tiles (taps of its convolution, 0: linear attention)."""
+        # (linear attention in narrow heads has nothing to save but the decays' way through memory: 32 heads of 64, runs of 700 and 300, 55.6 us in launches of its own, 56.2 here; of 128, 16
+        # heads, 2956 rows 145 and 131; the delta rule 104 and 90, 270 and 191)
+        return not self.exact and max(r.dim, r.vdim) <= D.REC_DIM and r.dim % 4 == 0 and r.vdim % 4 == 0 and taps <= D.REC_TILE_TAPS and (taps > 0 or r.dim > 64)
+
+    @staticmethod
+    def _delta_recurs(r) -> bool:
+        """Whether a delta rule has the form of one that goes from its projections: a decay per key channel, every head its own keys, a convolution."""
+        return r.decay == "channel" and r.kv_heads == r.heads and r.conv > 1
 
     # ---- gated linear attention ----
     def _gated_linear(self, B, d, r, P, l, n, positions, slot_ids, kvc, seg, nseg, out, scale: float = 1.0, work=NO_WORK, longest: int = 0) -> None:
@@ -375,7 +383,7 @@ class HybridRunner:
         wide = self._rounded(n, rv)
         Rn, Rn16 = None if wide else B.c[: n * rv].view(n, rv), self._as16(B.c16, n, rv) if wide else None
         R = B.b[: n * rv].view(n, rv)
-        if channel and r.kv_heads == r.heads and "conv" in st and \
+        if self._delta_recurs(r) and \
                 self._recurs(r, P, n, seg, nseg, work, R, B.a[: n * rv], r.conv, q_off=d["r_off"], a=d["a2"], a_off=d["a1_off"], a_bias=d["dt_bias"], a_rate=d["a_rate"], z=d["g2"],
                              z_off=d["g1_off"], norm_w=d["r_norm"], eps=self.cfg.norm_eps, positions=positions, slot_ids=slot_ids, state=st["gdn"], out=Rn, out16=Rn16, conv_w=d["conv_w"],
                              conv=st["conv"], b_off=d["rb_off"], unit_eps=UNIT_EPS, q_scale=r.dim ** -0.5, sigmoid=r.gate == "sigmoid"):

@@ -95,6 +95,7 @@ class PukatarModel(HybridRunner):
         self.max_rv = max([m.heads * m.vdim for m in deltas] or [0])
         self.max_delta_heads = max([m.heads for m in deltas] or [0])
         self.scans = {(m.heads, m.dim, m.vdim) for m in deltas}
+        self.recs = {(m.heads, m.dim, m.vdim) for m in deltas if self._delta_recurs(m) and self._rec_tiles_take(m, m.conv)}
         self._moe_sizes([l.mlp for l in cfg.layers])
         if cache_dtype is None:
             cache_dtype = torch.float32 if self.exact else torch.bfloat16
@@ -160,7 +161,7 @@ class PukatarModel(HybridRunner):
             return B.logits
         eps, ex, hint = cfg.norm_eps, self.exact, int(max_ctx_hint)
         seg, nseg, longest = self._runs(n, slot_ids, tokens_per_seq, rows_are_slots)
-        work = self._scan_work(n, nseg, longest, self.scans, delta=True, rec=not self.exact)
+        work = self._scan_work(n, nseg, longest, self.scans, delta=True, recs=self.recs)
         if tokens_per_seq is not None:
             runs = attention_segments(tokens_per_seq, n, self.ATTN_MAX_SEGMENTS)
         else:

@@ -89,6 +89,7 @@ class VepelixModel(HybridRunner):
         self.max_rk = max([r.heads * r.dim for r in rights] or [0])
         self.max_rv = max([r.heads * r.vdim for r in rights] or [0])
         self.scans = {(r.heads, r.dim, r.vdim) for r in rights}
+        self.recs = {(r.heads, r.dim, r.vdim) for r in rights if self._rec_tiles_take(r, 0)}
         self._moe_sizes([l.mlp for l in cfg.layers])
         if cache_dtype is None:
             cache_dtype = torch.float32 if self.exact else torch.bfloat16
@@ -168,7 +169,7 @@ class VepelixModel(HybridRunner):
         if n == 0:
             return B.logits
         seg, nseg, longest = self._runs(n, slot_ids, tokens_per_seq, rows_are_slots)
-        work = self._scan_work(n, nseg, longest, self.scans, delta=False, rec=not self.exact)
+        work = self._scan_work(n, nseg, longest, self.scans, delta=False, recs=self.recs)
         if tokens_per_seq is not None:
             runs = attention_segments(tokens_per_seq, n, self.ATTN_MAX_SEGMENTS)
         else:
