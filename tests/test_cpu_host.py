@@ -160,3 +160,14 @@ def test_linear_takes_numbers_of_any_kind(monkeypatch):
     for exact, apart, scale in ((True, 8, 2.5), (np.bool_(True), np.int64(8), np.float32(2.5)), (1.0, 8.0, torch.tensor(2.5))):
         D.linear(a, w, out, n=8, batch=2, w_batch=256, c_batch=8, bias=torch.zeros(2, 8), bias_batch=apart, exact=exact, epilogue=D.EPI_SCALE, scale=scale)
         assert (seen[-1].exact, seen[-1].bias_batch, seen[-1].scale) == (1, 8, 2.5)
+
+
+@pytest.mark.parametrize("top_k,experts,hidden,inter,shared,rows", [(2, 8, 1024, 512, 512, 362), (1, 256, 16, 16, 0, 42532), (2, 128, 64, 16, 0, 9551), (8, 32, 32, 16, 16, 3421), (2, 4, 128, 64, 64, 2843),
+                                                                    (1, 64, 256, 128, 0, 4278)])
+def test_rows_that_fit_the_library_s_own_scratch(top_k, experts, hidden, inter, shared, rows):
+    """The entry point that allocates nothing takes so many rows of these layers, however many rows a wave of its plan counts."""
+    import ctypes
+    from vllm_i64_amd import _lib
+    lib = _lib.load()
+    L = _lib.MoeLayer(top_k=top_k, num_experts=experts, hidden=hidden, expert_inter=inter, shared_inter=shared)
+    assert 0 < lib.i64h_moe_forward_workspace_bytes(rows, ctypes.addressof(L)) <= lib.i64h_moe_forward_static_max_bytes()

@@ -240,6 +240,17 @@ def test_moe_forward_c_entry_matches_oracle_both_paths(dev):
         assert np.abs(y - ref).mean() <= 1e-5, (n, np.abs(y - ref).mean())
 
 
+def test_moe_forward_of_many_rows(dev):
+    """Rows whose plan is three launches over counts that lie where the inner rows are written afterwards: against the oracle, to the bar of the test above."""
+    ocfg, w = M.named_config("tiny-moe"), M.make_weights(M.named_config("tiny-moe"), seed=0)
+    layer, bank = _tiny_moe_layer(dev, w)[1], M.LinearBank(w, "int8")
+    g = torch.Generator().manual_seed(5)
+    x, ids = torch.randn(2500, ocfg.hidden_size, generator=g) * 0.7, torch.randint(0, ocfg.vocab_size, (2500,), generator=g)
+    ref = M.moe_forward(ocfg, bank, 1, x, ids)
+    for _ in range(2):
+        assert (layer(x.to(dev), ids.to(dev)).cpu() - ref).abs().max().item() <= 1e-2
+
+
 def test_moe_forward_without_token_ids_routes_cyclic(dev):
     """token_ids=None: every token goes to experts (0 + k) % E (token_routed_mlp.py:120-130)."""
     ocfg = M.named_config("tiny-moe")

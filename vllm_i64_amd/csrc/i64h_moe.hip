@@ -50,9 +50,11 @@ MoeScratch carve(void* ws, int64_t n, const i64h_moe_layer* L) {
     s.perm = c.take<int32_t>(R);
     s.inv = c.take<int32_t>(R);
     s.sorted_bucket = c.take<int32_t>(R);
-    s.plan_ws = c.take<int32_t>(i64h_bucketize_workspace_bytes(R, nb, 1) / 4 + 1);
     s.stats = c.take<uint32_t>((int64_t)(4 + 2 * nb) * i64h_stats_words_per_slot());
-    s.e_inter = c.take<float>(R * L->expert_inter);
+    // (the plan's counts are read for the last time before the inner rows are written: one place for both, and what fits a given workspace doesn't hang on how many rows a wave of the plan counts)
+    const int64_t plan = i64h_bucketize_workspace_bytes(R, nb, 1) / 4 + 1, inner = R * L->expert_inter;
+    s.e_inter = c.take<float>(plan > inner ? plan : inner);
+    s.plan_ws = (int32_t*)s.e_inter;
     s.e_out = c.take<float>(R * L->hidden);
     s.sh_inter = c.take<float>(L->shared_inter > 0 ? n * L->shared_inter : 0);
     s.sh_out = c.take<float>(L->shared_inter > 0 ? n * L->hidden : 0);
