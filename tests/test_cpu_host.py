@@ -171,3 +171,23 @@ def test_rows_that_fit_the_library_s_own_scratch(top_k, experts, hidden, inter, 
     lib = _lib.load()
     L = _lib.MoeLayer(top_k=top_k, num_experts=experts, hidden=hidden, expert_inter=inter, shared_inter=shared)
     assert 0 < lib.i64h_moe_forward_workspace_bytes(rows, ctypes.addressof(L)) <= lib.i64h_moe_forward_static_max_bytes()
+
+
+def test_operands_that_a_launch_would_read_or_write_out_of_bounds_are_refused():
+    """C entries called past the Python checks: the refusal comes before anything is launched (addresses that are none)."""
+    import ctypes
+    from vllm_i64_amd import _lib
+    at, lib, dense = 1 << 20, _lib.load(), _lib.load_dense()
+    w8 = (ctypes.c_float * 8)()
+    assert lib.i64h_fused_residual_norm_lm_rows(at, 0, 0, 0, 0, ctypes.addressof(w8), 0, 1.0, 1.0, 0, 1e-6, 4, 64, at, 2, at, 0) != 0
+    assert b"norm's weights" in lib.i64h_last_error()
+    base = dict(P=at, ldp=2048, heads=2, dim=64, vdim=64, a_off=384, a_rank=8, A=at, a_bias=at, a_rate=at, norm_w=at, positions=at, slot_ids=at, state=at, out=at, ldo=128, n=3, z_off=512)
+    linear, delta = dict(base, k_off=128, v_off=256), dict(base, conv_w=at, conv=at, taps=4, Z=at, z_rank=8, b_off=600)
+    for args in (dict(linear, ldo=127), dict(linear, k_off=2000), dict(linear, v_off=1924), dict(linear, z_off=1924), dict(linear, a_off=2044), dict(delta, q_off=1668), dict(delta, b_off=2047),
+                 dict(delta, z_off=2044)):
+        d = _lib.RecStep(**args)
+        assert dense.i64h_rec_step(ctypes.addressof(d), 0) != 0 and b"behind the row's end" in dense.i64h_last_error(), args
+    d = _lib.RecStep(**delta)
+    for x in (dict(ldx=127), dict(ldx=128, v_off=4), dict(ldx=256, v_off=-4)):
+        s = _lib.Gdn(**{**dict(X=at, seg_start=at, nseg=1, out=at, ldo=128, work=at, work_floats=1 << 40), **x})
+        assert dense.i64h_rec_tiles(ctypes.addressof(d), ctypes.addressof(s), 0) != 0 and b"rows for the read-out" in dense.i64h_last_error(), x

@@ -932,7 +932,8 @@ int i64h_fused_residual_norm_lm(const float* h, const float* add, const float* m
 int i64h_fused_residual_norm_lm_rows(const float* h, const float* add, const float* moe_rows, const int32_t* moe_inv, const float* moe_shared,
                                      const float* route_weights, int32_t top_k, float routed_scale, float shared_scale,
                                      const float* norm_weight, float eps, int64_t n, int32_t H, const int32_t* rows, int64_t m_rows, void* lm_workspace, void* stream) {
-    I64H_CHECK_ARG(lm_workspace != nullptr && (uintptr_t)lm_workspace % 16 == 0 && rows != nullptr, "fused_residual_norm_lm_rows: workspace (16-byte aligned) and rows are required");
+    I64H_CHECK_ARG(lm_workspace != nullptr && (uintptr_t)lm_workspace % 16 == 0 && rows != nullptr && norm_weight != nullptr,
+                   "fused_residual_norm_lm_rows: workspace (16-byte aligned), rows and the norm's weights are required");
     I64H_CHECK_ARG(H % 32 == 0 && m_rows >= 0 && m_rows <= 2048, "fused_residual_norm_lm_rows: H=%d must be a multiple of 32, at most 2048 rows", H);
     return frn_launch(h, add, moe_rows, moe_inv, moe_shared, route_weights, top_k, routed_scale, shared_scale, nullptr, norm_weight, eps, nullptr, n,
                       H, nullptr, 1, 0, nullptr, stream, (uint32_t*)lm_workspace, (H + 255) / 256 * 8, rows, m_rows);

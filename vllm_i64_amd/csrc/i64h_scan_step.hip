@@ -245,6 +245,10 @@ static int rec_check(const i64h_rec_step_args& d, const char* what) {
     I64H_CHECK_ARG((((uintptr_t)d.P | (uintptr_t)d.A | (uintptr_t)d.Z | (uintptr_t)d.state) & 15) == 0 && d.ldp % 4 == 0 && d.a_off % 4 == 0 &&
                    (delta ? d.z_off % 4 == 0 : d.q_off % 4 == 0 && d.k_off % 4 == 0), "%s: rows and states are read 16 bytes at a time", what);
     I64H_CHECK_ARG(d.n * d.heads < (1ll << 31), "%s: %lld rows of %d heads", what, (long long)d.n, d.heads);
+    const int64_t nd = (int64_t)d.heads * d.dim, rv = (int64_t)d.heads * d.vdim;
+    auto inside = [&](int64_t off, int64_t width) { return off + width <= d.ldp; };
+    I64H_CHECK_ARG(d.ldo >= rv && inside(d.a_off, d.a_rank) && (delta ? inside(d.q_off, 2 * nd + rv) && inside(d.b_off, d.heads) && inside(d.z_off, d.z_rank)
+                                                                   : inside(d.q_off, nd) && inside(d.k_off, nd) && inside(d.v_off, rv) && inside(d.z_off, rv)), "%s: columns behind the row's end", what);
     return 0;
 }
 
@@ -275,7 +279,7 @@ int i64h_rec_tiles(const i64h_rec_step_args* dp, const i64h_gdn_args* sp, void* 
     if (rec_check(d, "rec_tiles")) return 1;
     I64H_CHECK_ARG(!d.exact && d.dim % 4 == 0 && d.vdim % 4 == 0 && (!delta || d.taps <= 4), "rec_tiles: products of bf16 values, columns in fours, at most 4 taps");
     i64h_gdn_args a = *sp;
-    I64H_CHECK_ARG(a.seg_start && a.nseg > 0 && a.nseg <= 65535 && a.out && a.ldo >= (int64_t)d.heads * d.vdim && (!delta || a.X) && a.work && a.work_floats >= i64h_scan_work_floats(d.n, a.nseg, d.heads, d.dim),
+    I64H_CHECK_ARG(a.seg_start && a.nseg > 0 && a.nseg <= 65535 && a.out && a.ldo >= (int64_t)d.heads * d.vdim && (!delta || (a.X && a.v_off >= 0 && a.ldx >= a.v_off + (int64_t)d.heads * d.vdim)) && a.work && a.work_floats >= i64h_scan_work_floats(d.n, a.nseg, d.heads, d.dim),
                    "rec_tiles: runs, a workspace and rows for the read-out");
     I64H_CHECK_ARG((((uintptr_t)a.work | (uintptr_t)a.out | (uintptr_t)d.norm_w | (uintptr_t)d.a_rate | (uintptr_t)d.a_bias | (uintptr_t)d.out | (uintptr_t)d.out16) & 15) == 0 && a.ldo % 4 == 0 && d.ldo % 4 == 0 &&
                    d.ldp < (1 << 25) && a.ldx < (1 << 25) && (d.n / 16 + a.nseg) * (int64_t)d.heads < (1ll << 31), "rec_tiles: rows are read 16 bytes at a time");
