@@ -724,10 +724,11 @@ def test_fused_qkv_rope_kv_equals_two_kernel_path(dev):
         assert outs[1][0].abs().sum() > 0
 
 
-@pytest.mark.parametrize("n", [1, 64, 200, 300])
+@pytest.mark.parametrize("n", [1, 64, 200, 300, 301, 2047, 2048, 2049, 5000])
 def test_plan_with_embedding_rows_equals_the_two_launches(n):
     """i64h_moe_plan_embedding against i64h_moe_plan + i64h_embedding_stats_reset: every plan output, the embedding rows and the reset
-    stat slots identical (one launch up to 512 (route, token) rows, the separate launches beyond - n = 300 at top-2)."""
+    stat slots identical, and the plan a stable sort's (one launch of 256 threads up to 512 (route, token) rows, of 1024 threads and four
+    embedding rows a workgroup up to 4096 - n = 2048 at top-2 -, the separate launches beyond)."""
     from vllm_i64_amd import ops
     dev = torch.device("cuda:0")
     g = torch.Generator().manual_seed(n)
@@ -747,6 +748,15 @@ def test_plan_with_embedding_rows_equals_the_two_launches(n):
     for name in ("routes", "keys", "offsets", "perm", "inv", "sorted_bucket", "expert_offsets", "tok_slots"):
         assert torch.equal(getattr(a, name), getattr(b, name)), name
     assert torch.equal(h_a, h_b) and torch.equal(st_a, st_b)
+    at = ids.cpu().clamp(max=V - 1)
+    assert torch.equal(h_b.cpu(), embed.cpu()[at])
+    for l in range(L):
+        key = (tables.cpu()[l, :, :][:, at] * top_k + torch.arange(top_k).view(-1, 1)).reshape(-1)
+        perm = torch.sort(key, stable=True)[1]
+        assert torch.equal(b.keys[l].cpu().long(), key) and torch.equal(b.perm[l].cpu().long(), perm) and torch.equal(b.inv[l].cpu().long(), torch.argsort(perm))
+        assert torch.equal(b.sorted_bucket[l].cpu().long(), key[perm])
+        first = torch.cat([torch.zeros(1, dtype=torch.long), torch.bincount(key, minlength=E * top_k).cumsum(0)])
+        assert torch.equal(b.offsets[l].cpu().long(), first) and torch.equal(b.expert_offsets[l].cpu().long(), first[::top_k])
     assert not torch.isnan(h_b).any() and int((st_b == 12345).sum()) == 0
 
 
