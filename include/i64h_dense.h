@@ -28,8 +28,9 @@ int i64h_device_check(void);
  *   row(m) = a_rows ? a_rows[m] : m;  W bf16 [N, K] row-major, batch stride w_batch elements;  C fp32, row stride ldc,
  *   batch stride c_batch.
  * exact = 0: A is rounded to bf16 (nearest even) while it is staged, products on v_mfma_f32_16x16x32_bf16, fp32 sums.
- * exact = 1: products of fp32 rows, sums in fp32.  K of 64 and more: a row's value in three bf16 parts that hold all of it, each times the bf16 weight, on
- *   v_mfma_f32_16x16x32_bf16; a shorter K: W widened to fp32 while it is staged, v_mfma_f32_16x16x4_f32.
+ * exact = 1: products of fp32 rows, sums in fp32.  K of 64 and more, or a gate / up pair, over operands that are read 16 bytes at a time (A, W and in_norm_w aligned, lda and a_batch
+ *   multiples of four, K and w_batch of eight) and lie within 32-bit offsets: a row's value in three bf16 parts that hold all of it, each times the bf16 weight, on
+ *   v_mfma_f32_16x16x32_bf16.  All else: W widened to fp32 while it is staged, v_mfma_f32_16x16x4_f32.  (Other bits, both from true 32-bit products.)
  * epilogue: I64H_EPI_STORE; I64H_EPI_GELU_MUL: gelu_tanh(A W^T) * (A W2^T) with W2 = W + N * K (gate rows, then up rows);
  *   I64H_EPI_MUL_SIGMOID: * sigmoid(E[b][m, n]) (E fp32, row stride lde, batch stride e_batch);
  *   I64H_EPI_SOFTCAP: cap * tanh(. / cap);  I64H_EPI_GELU_ERF: 0.5 v (1 + erf(v / sqrt 2));  I64H_EPI_SCALE: v * scale;

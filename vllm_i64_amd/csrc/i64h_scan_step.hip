@@ -3,7 +3,7 @@
 // in one workgroup, so that a layer waits for one launch in the place of six (linear attention: three).
 // What bounds it: few rows the chain inside a workgroup (loads of the sequence's slot, of the state behind it, sums, norm), many rows the state's way from memory and
 // back; the low-rank maps' 64 KB a head come from L2.  7 rows of 8 heads of 128 in a graph: six launches of the delta rule 23 us, this one 9, a step of eight such layers 510 -> 404; 64 rows
-// of 16 heads, linear attention beside an attention over 134 MB: 16 + 45 + 6 -> 42 (134 MB of state at the copy rate: 28), a step 1524 -> 1508.
+// of 16 heads, linear attention: 37 -> 24 alone; beside an attention over 134 MB the launch takes 59 and the attention 58 where it took 37, together 268 MB at the copy rate, a step 1524 -> 1508.
 #include "i64h_dense_dev.h"
 #include "i64h_scan_dev.h"
 
