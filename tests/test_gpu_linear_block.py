@@ -241,8 +241,8 @@ def test_parts_of_32_bit_rows(dev, use_form, form):
 
 
 def test_a_row_of_nan_among_32_bit_rows_takes_no_longer(dev):
-    """Sums that are no number are taken again term by term, up to the first term that makes them none: a sequence that is lost does not hold up the step's others (15 times as long if
-    every term is taken; the smallest of some times each, and a bound far from both)."""
+    """Sums that are no number are taken again term by term only where the row itself holds numbers: a sequence that is lost does not hold up the step's others (15 times as long if
+    every sum is taken again; the smallest of some times each, and a bound far from both)."""
     from vllm_i64_amd import ops_dense as D
     g = torch.Generator().manual_seed(1)
     a, w, out = torch.randn(376, 1024, generator=g).to(dev), bf16(torch.randn(5760, 1024, generator=g)).to(dev), torch.empty(376, 5760, device=dev)
@@ -260,6 +260,10 @@ def test_a_row_of_nan_among_32_bit_rows_takes_no_longer(dev):
         return best
 
     numbers = fastest()
-    a[3] = float("nan")
-    assert fastest() < 4 * numbers
+    for lost in (slice(None), slice(1023, None)):
+        a[3, lost] = float("nan")
+        assert fastest() < 4 * numbers
+        a[3] = 0
+    a[3, 1023] = float("nan")
+    D.linear(a, w, out, exact=True)
     assert out[3].isnan().all() and int(out.isnan().sum()) == 5760

@@ -218,14 +218,14 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
         }
     }
     // the weights are the left operand: a lane holds four neighbouring columns of a row
-    // (376 x 5760 x 1024, us: 31; a row of NaN 32, one at the end of a row 208, an infinite weight 51)
-    if constexpr (EX) {      // an infinite weight makes no number of a part that is zero: such sums are taken again term by term
-        auto again = [&](float v, int64_t rl, int c) {
-            if (v == v) return v;
-            const float* x = p.A + b * p.a_batch + (p.a_rows ? (int64_t)p.a_rows[m0 + rl] : m0 + rl) * p.lda;
+    // An infinite weight makes no number of a part that is zero: such sums are taken again term by term, unless the row itself holds what is no number.  376 x 5760 x 1024, us: 31; a row of NaN 30,
+    // one at the end of a row 56, an infinite weight 85 (every such sum taken term by term 475, 476, 140).
+    if constexpr (EX) {
+        auto row = [&](int64_t rl) { return p.A + b * p.a_batch + (p.a_rows ? (int64_t)p.a_rows[m0 + rl] : m0 + rl) * p.lda; };
+        auto again = [&](const float* x, int c) {      // (K is a multiple of eight)
             const uint16_t* w = (const uint16_t*)p.W + b * p.w_batch + (int64_t)c * K;
-            v = 0.0f;
-            for (int k = 0; k < K && v == v; k += 8)      // (what is no number stays so: a row of NaN ends here at once; K is a multiple of eight)
+            float v = 0.0f;
+            for (int k = 0; k < K && v == v; k += 8)
 #pragma unroll
                 for (int i = 0; i < 8; ++i) v = fmaf(INN ? x[k + i] * p.in_norm_w[k + i] : x[k + i], dn_bf16_to_f32(w[k + i]), v);
             return v;
@@ -233,13 +233,24 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : KG) void linear_block_kerne
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
             const int rl = wm * WM + i * 16 + fr;
-            if (rl >= M) continue;
+            bool odd = false;
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) odd |= acc[i][j][g] != acc[i][j][g];
+            if (rl >= M || !odd) continue;
+            const float* x = row(rl);
+            bool lost = false;
+            for (int k = 0; k < K && !lost; k += 8)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) lost |= x[k + e] != x[k + e];
+            if (lost) continue;
 #pragma unroll
             for (int j = 0; j < FN; ++j) {
                 const int c = n0 + wn * (COLS / NWN) + (DUAL ? j % (FN / 2) : j) * 16 + fk * 4;
 #pragma unroll
                 for (int g = 0; g < 4; ++g)
-                    if (c + g < N) acc[i][j][g] = again(acc[i][j][g], rl, c + g + (DUAL && j >= FN / 2 ? N : 0));
+                    if (c + g < N && acc[i][j][g] != acc[i][j][g]) acc[i][j][g] = again(x, c + g + (DUAL && j >= FN / 2 ? N : 0));
             }
         }
     }
